@@ -32,6 +32,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
 // Two shapes of workgroup: 8 waves = 256 query rows with an 8-stage tile ring (one workgroup holds a compute unit:
@@ -258,19 +259,22 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.0f;
-  float m_run = -INFINITY;  // running row max (log2 domain) of query l32
-  // Row sums come from the matrix pipe too: an all-ones A operand (e4m3 1.0 = 0x38) makes every
-  // row of `lacc` the sum over keys of the SAME e4m3-rounded P the numerator uses.  Only
-  // register 0 is read (all 16 hold the same value), so only it is rescaled.
-  v16f lacc;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) lacc[r] = 0.0f;
-  // eight registers on purpose: left as one constant the compiler keeps a single copy and rebuilds
+  // reference point of query l32 in the log2 domain (its "running maximum"), and what the steps read it as: the
+  // exponent's constant part and the score above which the point has to move
+  float m_run = -INFINITY, x_base = INFINITY, x_limit = -INFINITY;
+  // Row sums come from the matrix pipe too, of the SAME e4m3-rounded P the numerator uses.  The 16x16x128 instruction
+  // takes half the matrix cycles of the 32x32x64 one and a quarter of its accumulators; its B operand is P's register
+  // block read as 16 columns with four groups of 16 lanes stacked along the contraction: groups 0 and 2 hold the two
+  // halves of query (lane % 16)'s keys, groups 1 and 3 those of query 16 + (lane % 16).  A therefore carries ones
+  // (e4m3 1.0 = 0x38) where output row 4 g' .. 4 g' + 3 and group g agree in parity and zeros elsewhere: the lanes of
+  // group g' then find the sum of their own query in all four registers.  Only register 0 is read and rescaled.
+  v4f lacc = {0.0f, 0.0f, 0.0f, 0.0f};
+  // eight registers on purpose: left as one value the compiler keeps a single copy and rebuilds
   // the 8-register operand with seven moves in every step
   v8i ones;
 #pragma unroll
   for (int r = 0; r < 8; ++r) {
-    int one4 = 0x38383838;
+    int one4 = ((lane >> 2) & 1) == ((lane >> 4) & 1) ? 0x38383838 : 0;
     pin(one4);
     ones[r] = one4;
   }
@@ -555,9 +559,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   auto lane_max = [&](const v16i (&blk)[2]) {
     return max(max(max8(blk[0], 0), max8(blk[0], 8)), max(max8(blk[1], 0), max8(blk[1], 8)));
   };
-  // new running max of query l32 given this lane's tile maximum; returns 2^(old max - new max)
-  bool tile_is_nothing = false;  // set by update_max, per lane
-  auto update_max = [&](int imax, float sc, float mneg) -> float {
+  constexpr float kShift = kPwlExp ? kPShiftPwl : kPShift, kLazy = kPwlExp ? kLazyMaxPwl : kLazyMax;
+  // Moves query l32's reference point where this tile's maximum asks for it (imax: this lane's maximum, over half the
+  // query's keys) and returns 2^(old point - new point), exactly 1 where the point stays.
+  auto move_point = [&](int imax, float sc, float mneg) -> float {
     {
       // the other half of query l32's keys lives in lane l32 + 32
       int other = imax;
@@ -566,13 +571,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     }
     // the accumulator read as fp32 is magic + dot, so one fma gives sc * dot (mneg = -magic * sc)
     const float m_tile = __builtin_fmaf(__int_as_float(imax), sc, mneg);
-    const float m_new = m_tile > m_run + (kPwlExp ? kLazyMaxPwl : kLazyMax) ? m_tile : m_run;  // -inf at the first tile: always taken
-    const float alpha = fast_exp2(m_run - m_new);                     // exactly 1 where the reference point stays
+    const float m_new = m_tile > x_limit ? m_tile : m_run;  // the limit is -inf at the first tile: always taken
+    const float alpha = fast_exp2(m_run - m_new);
     m_run = m_new;
-    // Every probability of this row in this tile is below 2^(m_tile - m_run + shift).  Under 2^-10 (half the smallest
-    // e4m3 subnormal; a tie goes to the even code, zero) each one converts to the zero code - taken with a margin of
-    // one octave for the exponent's few units of rounding.
-    tile_is_nothing = m_tile < m_run - (kPShift + 11.0f);
+    x_limit = m_new + kLazy;
+    x_base = kShift - m_new;
     return alpha;
   };
   // p = exp2(sc*dot - m_run + shift); the magic is folded into the constant c, which is off by
@@ -614,21 +617,58 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // two rings: step 0 requests K tile kStages into the slot of K tile 0, which every wave must have read by then
   if constexpr (Shape::kTwoRings) __builtin_amdgcn_s_barrier();
   if (diag_at(0)) causal_scores(s_a);
-  int mx_cur = lane_max(s_a);  // this lane's maximum of the tile whose probabilities come next
-  float ks_cur = s_ks[0];
+
+  // What a step needs to know about its tile before the first probability: the scale, the exponent's constant and
+  // whether a reference point moves.  Worked out at the end of the step before, so that its chain of dependent
+  // operations runs under that step's last matrix instruction and the wait at the barrier.  Points move in few steps
+  // (11 % of a wave's on outlier-ridden scores, 3 % on flat ones): a lane compares its own half's maximum with the
+  // limit, and only when some lane of the wave exceeds it are the halves joined and points, factors and constants
+  // formed anew (one wave-uniform branch instead of eight vector operations and a transcendental in every step).
+  // With the 16x16 row sums, same bits: 10.60 -> 10.35 ms at B=1 H=40 L=32760 with outliers, 11.44 -> 11.05 without
+  // (2045 cycles per step, from 2073; the chip runs at its power limit there, and fewer operations raise its clock too).
+  float sc = 0.0f, xc = 0.0f;           // scale of the coming tile, its exponent constant
+  float alpha_next = 1.0f;              // factor the coming tile's point move puts on everything before it
+  bool moved_next = false;              // (wave-uniform) whether it is other than 1
+  bool nothing = false;                 // (wave-uniform) every probability of the coming tile converts to zero
+  auto look_ahead = [&](int jn, int mx, float ks) {
+    sc = qs * ks;
+    const float mneg = -kMagicVal * sc;
+    const float m_half = __builtin_fmaf(__int_as_float(mx), sc, mneg);
+    moved_next = false;
+    if (__any(m_half > x_limit)) {
+      // (a tile this wave's mask row does not ask for, or that is not this loop's, leaves the points alone)
+      if (jn < n_main && mine_at(jn)) {
+        alpha_next = move_point(mx, sc, mneg);
+        moved_next = true;
+      }
+    }
+    // exponent of key r: x = sc*dot - m_run + shift, with the magic folded into the constant
+    // (which is therefore off by at most ~1.5 integer steps of the dot product)
+    xc = x_base + mneg;
+    // Every probability of a row in this tile is below 2^(m_tile - m_run + shift).  Under 2^-10 (half the smallest
+    // e4m3 subnormal; a tie goes to the even code, zero) each one converts to the zero code - taken with a margin of
+    // one octave for the exponent's few units of rounding.  With every row of the wave that far down, the wave writes
+    // the zeros directly and leaves out the 64 exponentials and 32 conversions per lane (every chunk below tests this
+    // one scalar); the matrix work that concerns the neighbouring tiles stays.  Same bits either way - the
+    // pvthreshold idea of the reference's sparse kernel (sage_sla.py:237-253) with a threshold at which nothing changes.
+    if constexpr (kTileSkip) nothing = __all(m_half < m_run - (kPShift + 11.0f));
+  };
+  look_ahead(0, lane_max(s_a), s_ks[0]);
+  moved_next = false;  // nothing has been accumulated yet
 
   // Software pipeline, one key tile per step.  While this tile's probabilities are computed on
   // the VALU, the matrix pipe runs the S^T MFMAs of the NEXT tile and the PV MFMAs of the
   // PREVIOUS tile: every MFMA below is followed by the VALU work that hides it, LDS operands are
   // requested three MFMAs ahead, and sched_barrier pins that order.  The max reduction of the
-  // next tile rides in the PV chunks, so a step starts with only the short finalisation.
+  // next tile rides in the PV chunks.
   // Because PV lags one tile, so does the rescaling of O:
-  //   at step j   O holds tiles <= j-2 relative to max m(j-2); alpha_prev = 2^(m(j-2) - m(j-1))
-  //   step j      O *= alpha_prev (rare branch), then O += P(j-1) V(j-1), both relative to m(j-1)
+  //   at step j   O holds tiles <= j-2 relative to point m(j-2); alpha = 2^(m(j-2) - m(j-1)), alpha_next = 2^(m(j-1) - m(j))
+  //   step j      O *= alpha (rare branch), then O += P(j-1) V(j-1), both relative to m(j-1)
   // LDS ring of 8 stages: tile j-1 (V), j (V next step), j+1 (K), j+2 .. j+4 (arriving).
   // probabilities of the previous and of the current tile swap registers every step, like s_a / s_b
   v8i pf_x = {0, 0, 0, 0, 0, 0, 0, 0}, pf_y = {0, 0, 0, 0, 0, 0, 0, 0};
-  float alpha_prev = 1.0f;
+  float alpha = 1.0f;
+  bool moved = false;
   auto tile_step = [&](int j, v16i (&s_cur)[2], v16i (&s_nxt)[2], const v8i& pf_prev, v8i& pf) {
     const uint8_t* kst = k_slot(j + 1);
     const uint8_t* vst = v_slot(j - 1);
@@ -640,37 +680,22 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     };
     v4i kf[4];
     v8i vf[4];
-    // operands of the first three S^T MFMAs and the next tile's K scale: requested before the
-    // dependent scalar work below, so their LDS latency is hidden behind it
+    // operands of the first three S^T MFMAs and the next tile's K scale
     kf[0] = k_frag(0);
     kf[1] = k_frag(1);
     kf[2] = k_frag(2);  // (kG >= 2: chunks 0 .. 3 always exist)
     const float ks_nxt = s_ks[min(j + 1, n_tiles - 1)];
     int entering = 0;  // the list entry the next step's window gains; it arrives with the operands above
     if constexpr (kSparse) entering = s_list[min(j + 1 + Shape::kAheadK, n_tiles - 1)];
-    const bool mine = mine_at(j);
     issue_copy(j);
-    if (__any(alpha_prev < 1.0f)) scale_o(alpha_prev);
-    // row sums of tile j-1: 64 matrix cycles that run under the max finalisation below
-    lacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones, pf_prev, lacc, 0, 0, 0, 0, 0, 0);
-    const float sc = qs * ks_cur;
-    const float mneg = -kMagicVal * sc;
-    // a tile this wave's mask row does not ask for leaves the running maximum alone (wave-uniform
-    // branch); its probabilities are zeroed where they are packed
-    alpha_prev = mine ? update_max(mx_cur, sc, mneg) : 1.0f;
-    // exponent of key r: x = sc*dot - m_run + shift, with the magic folded into the constant
-    // (which is therefore off by at most ~1.5 integer steps of the dot product)
-    const float c = ((kPwlExp ? kPShiftPwl : kPShift) - m_run) + mneg;
+    if (moved) scale_o(alpha);  // wave-uniform
+    alpha = alpha_next;
+    moved = moved_next;
+    // row sums of tile j-1: they cover the latency of the operands just requested
+    lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_prev, lacc, 0, 0, 0, 0, 0, 0);
     const float scp = kPwlExp ? 8.0f * sc : sc;
-    const float cp = kPwlExp ? __builtin_fmaf(8.0f, c, 55.5f) : c;
-    int pm[4];
-    // A tile whose scores lie more than 17 octaves under the reference point of every one of the wave's 32 rows: each
-    // probability byte would be the zero code.  The wave then writes the zeros directly and leaves out the 64
-    // exponentials and 32 conversions per lane (every chunk below tests this one scalar); the matrix work that
-    // concerns the neighbouring tiles stays.  Same bits either way - the pvthreshold idea of the reference's sparse
-    // kernel (sage_sla.py:237-253) with a threshold at which nothing changes.
-    bool nothing = false;  // wave-uniform
-    if constexpr (kTileSkip) nothing = mine && __all(tile_is_nothing);
+    const float cp = kPwlExp ? __builtin_fmaf(8.0f, xc, 55.5f) : xc;
+    const bool skip = nothing;
     // The S^T chunks are short (a 32-cycle MFMA each): a wave inside them goes ahead of the SIMD's other
     // wave, which is usually in its PV chunks and has 64-cycle MFMAs to hide behind (measured: -1.3 %).
     __builtin_amdgcn_s_setprio(1);
@@ -692,7 +717,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         int wi = (int)w;
         if (i & 1) pin(wi);
         pf[i >> 1] = wi;
-      } else if (!nothing) {
+      } else if (!skip) {
         const float e0 = p_of(s_cur[0][2 * i], scp, cp), e1 = p_of(s_cur[0][2 * i + 1], scp, cp);
         if (i & 1) {
           int w = __builtin_amdgcn_cvt_pk_fp8_f32(e0, e1, pf[i >> 1], true);
@@ -712,30 +737,36 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     __builtin_amdgcn_s_setprio(0);
     // 4 x [PV MFMA of tile j-1 (64 matrix cycles) | 4 probabilities of tile j | a quarter of
     // the max reduction of tile j+1, whose S^T MFMAs were issued at least one chunk ago]
+    int mx = 0;
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) {
       if (dt == 0 && kG == 4) vf[3] = v_frag(3);
       if (dt < kG) oacc[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf[dt], pf_prev, oacc[dt], 0, 0, 0, 0, 0, 0);
       int w = 0;
-      if (!nothing) w = pack4(s_cur[1][4 * dt], s_cur[1][4 * dt + 1], s_cur[1][4 * dt + 2], s_cur[1][4 * dt + 3], scp, cp);
+      if (!skip) w = pack4(s_cur[1][4 * dt], s_cur[1][4 * dt + 1], s_cur[1][4 * dt + 2], s_cur[1][4 * dt + 3], scp, cp);
       pin(w);
       pf[4 + dt] = w;
-      pm[dt] = max8(s_nxt[dt >> 1], (dt & 1) * 8);
-      pin(pm[dt]);
+      // one chain over the 32 scores, two per instruction
+      const v16i& blk = s_nxt[dt >> 1];
+      const int r0 = (dt & 1) * 8;
+      mx = dt == 0 ? max(blk[0], blk[1]) : max(max(mx, blk[r0]), blk[r0 + 1]);
+      mx = max(max(mx, blk[r0 + 2]), blk[r0 + 3]);
+      mx = max(max(mx, blk[r0 + 4]), blk[r0 + 5]);
+      mx = max(max(mx, blk[r0 + 6]), blk[r0 + 7]);
+      pin(mx);
       __builtin_amdgcn_sched_barrier(0);
     }
-    mx_cur = max(max(pm[0], pm[1]), max(pm[2], pm[3]));
-    ks_cur = ks_nxt;
     if constexpr (kSparse) {
 #pragma unroll
       for (int i = 0; i + 1 < kWindow; ++i) ahead[i] = ahead[i + 1];
       ahead[kWindow - 1] = __builtin_amdgcn_readfirstlane(entering) & 0xffff;
-      if (!mine) {  // wave-uniform and rare: a tile this wave's row does not take part in contributes nothing
+      if (!mine_at(j)) {  // wave-uniform and rare: a tile this wave's row does not take part in contributes nothing
 #pragma unroll
         for (int i = 0; i < 8; ++i) pf[i] = 0;
       }
       if (diag_at(j)) causal_probs(pf);
     }
+    look_ahead(j + 1, mx, ks_nxt);
     // after this barrier: tile j+2 is visible to every wave, and nobody reads tile j-1 any more
     tile_barrier();
   };
@@ -755,12 +786,12 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if (has_tail) __builtin_amdgcn_s_barrier();
   }
   if (n_main > 0) {  // drain: PV of the last pipelined tile
-    scale_o(alpha_prev);
+    if (moved) scale_o(alpha);
     const uint8_t* vst = v_slot(n_main - 1);
     const v8i pf_last = (n_main & 1) ? pf_y : pf_x;  // written by the last step
 #pragma unroll
     for (int dt = 0; dt < kG; ++dt) pv_slice(vst, dt, pf_last);
-    lacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones, pf_last, lacc, 0, 0, 0, 0, 0, 0);
+    lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_last, lacc, 0, 0, 0, 0, 0, 0);
   }
   if (has_tail && mine_at(n_tiles - 1)) {  // ragged last tile, not pipelined: mask keys >= lk
     const int j = nkb - 1, jj = n_tiles - 1;
@@ -774,8 +805,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       }
     const float sc = qs * s_ks[jj];
     const float mneg = -kMagicVal * sc;
-    scale_o(update_max(lane_max(s_cur), sc, mneg));
-    const float c = ((kPwlExp ? kPShiftPwl : kPShift) - m_run) + mneg;
+    scale_o(move_point(lane_max(s_cur), sc, mneg));
+    const float c = x_base + mneg;
     const float scp = kPwlExp ? 8.0f * sc : sc;
     const float cp = kPwlExp ? __builtin_fmaf(8.0f, c, 55.5f) : c;
     v8i pf;
@@ -797,7 +828,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     const uint8_t* vst = v_slot(jj);
 #pragma unroll
     for (int dt = 0; dt < kG; ++dt) pv_slice(vst, dt, pf);
-    lacc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones, pf, lacc, 0, 0, 0, 0, 0, 0);
+    lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, lacc, 0, 0, 0, 0, 0, 0);
   }
 
   if constexpr (kSplit) {

@@ -1,0 +1,54 @@
+"""The attention kernel's own branches at the sizes where they can go wrong, against the tile-by-tile emulation fed with
+the operands the GPU quantized.
+
+Tolerance of every comparison: kernel and emulation do the same fp32 operations up to summation order and up to an
+exponential that may differ in its last place, so a probability lands on another e4m3 code only within an ulp of a
+rounding boundary (6 % of one probability); everything else is the final rounding to the output type, 2^-9 relative."""
+
+import pytest
+import torch
+
+from ksanadit_amd import sage_ops
+from ksanadit_amd.layout import untile_k, untile_v
+from oracle.sage_emul_ref import sage_emul_from_quant
+
+pytestmark = pytest.mark.gpu
+
+
+def _emul(ws, Lq, Lk, dtype, **kw):
+    return sage_emul_from_quant(
+        ws.q_i8.cpu()[:, :, :Lq], ws.q_scale.cpu()[:, :, :Lq], untile_k(ws.k_tiles.cpu(), Lk), ws.k_scale.cpu(),
+        untile_v(ws.v_tiles.cpu(), Lk).view(torch.float8_e4m3fn), ws.v_scale.cpu(), dtype, **kw)
+
+
+def _close(out, want):
+    out, want = out.float(), want.float()
+    scale = max(float(want.abs().max()), 1e-3)
+    diff = (out - want).abs()
+    assert torch.isfinite(out).all()
+    assert float(diff.max()) <= 2e-2 * scale
+    assert float((diff > 5e-3 * scale).float().mean()) <= 1e-3
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("Lk", [64, 128, 192, 448, 470])
+@pytest.mark.parametrize("lift", [0.5, 6.0], ids=["below_the_limit", "above_the_limit"])
+def test_reference_points_move_at_any_tile(hip_device, waves, Lk, lift):
+    """Each key tile in turn outdoes every tile before it, for some query rows only: the reference point of those rows
+    moves at the first, a middle, the last full and the ragged tile (or stays, where the step is small)."""
+    Lq, H = 160, 1
+    print(f"case waves={waves} Lk={Lk} lift={lift}", flush=True)
+    g = torch.Generator().manual_seed(Lk)
+    q, k, v = (torch.randn((1, n, H, 128), generator=g) for n in (Lq, Lk, Lk))
+    direction = torch.randn(128, generator=g)
+    direction /= direction.norm()
+    # key tile t leans towards the direction by t steps, query row i towards it or away: scores rise (or fall) tile by tile
+    step = torch.arange(Lk) // 64
+    k = k * 0.2 + (step[None, :, None, None] * lift) * direction
+    q = q * 0.2 + (torch.where(torch.arange(Lq) % 3 == 0, -4.0, 4.0)[None, :, None, None]) * direction
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    qd, kd, vd = (t.to(hip_device) for t in (q, k, v))
+    ws = sage_ops.workspace_for(qd, kd)
+    sage_ops.quant_q(qd, ws, 128**-0.5), sage_ops.quant_k(kd, ws, True), sage_ops.quant_v(vd, ws)
+    out = sage_ops.attn_fwd(ws, torch.empty_like(qd), wg_waves=waves).cpu()
+    _close(out, _emul(ws, Lq, Lk, q.dtype))
