@@ -183,9 +183,18 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     // Consecutive workgroup ids land on consecutive XCDs (8 per chip, one L2 each).  Give every
     // XCD a contiguous run of (head, query block) pairs so the workgroups that stream the same
     // K/V tiles share one L2.
-    const int xcd = blockIdx.x & 7;
-    wg = xcd * wg_per_xcd + (blockIdx.x >> 3);
-    if (wg >= n_wg) return;
+    const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+    if (p.batch_run == 0) {
+      wg = xcd * wg_per_xcd + at;
+      if (wg >= n_wg) return;
+    } else {
+      // batch entries of unequal length: an eighth of every entry's workgroups to every XCD.  One run across the entries
+      // would leave the XCDs that drew the short ones idle (B=3, 24 heads, lengths 100 / 72 / 45 % of 4099: 265 -> 177 us).
+      const int b = at / p.batch_run, n_batch = p.Hq * n_qwg;
+      const int in_batch = xcd * p.batch_run + (at - b * p.batch_run);
+      wg = b * n_batch + in_batch;
+      if (in_batch >= n_batch || wg >= n_wg) return;
+    }
   }
   const int bh = wg / n_qwg;
   int qwg = wg - bh * n_qwg;
@@ -1038,7 +1047,16 @@ static int pick_wg_waves(const AttnParams& p) {
   return dense_in_four_waves(n_wg8, p.nkb) ? 4 : 8;
 }
 
-hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t s) {
+// Grid of a launch whose workgroups are numbered in runs per XCD (see the kernel's first lines), and the run's length.
+// Per-entry counts live in device memory, so entries of a batch that has any are taken to be unequal.
+static dim3 xcd_grid(AttnParams* p, int n_qwg, int n_wg, int* wg_per_xcd) {
+  p->batch_run = p->B > 1 && (p->k_lens != nullptr || p->q_lens != nullptr) ? (p->Hq * n_qwg + 7) / 8 : 0;
+  *wg_per_xcd = p->batch_run != 0 ? p->batch_run * p->B : (n_wg + 7) / 8;
+  return dim3(*wg_per_xcd * 8);
+}
+
+hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
+  AttnParams p = params;
   if (p.nkb > kMaxKeyTiles) return hipErrorInvalidValue;
   const bool sparse = p.block_mask != nullptr || p.causal;
   if (sparse && p.nkb > kSparseMaxKeyTiles) return hipErrorInvalidValue;
@@ -1047,8 +1065,8 @@ hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t s) {
   if (waves == 4) {
     const int n_qwg = (p.Lq + WgShape<4>::kRows - 1) / WgShape<4>::kRows;
     const int n_wg = p.B * p.Hq * n_qwg;
-    const int wg_per_xcd = (n_wg + 7) / 8;
-    const dim3 grid(wg_per_xcd * 8);
+    int wg_per_xcd = 0;
+    const dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
     if (sparse)
       return p.causal ? launch_shape<true, false, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
                       : launch_shape<true, false, 4, false>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s);
@@ -1057,8 +1075,8 @@ hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t s) {
   }
   const int n_qwg = (p.Lq + kAttnQPerWg - 1) / kAttnQPerWg;
   const int n_wg = p.B * p.Hq * n_qwg;
-  const int wg_per_xcd = (n_wg + 7) / 8;
-  const dim3 grid(wg_per_xcd * 8);
+  int wg_per_xcd = 0;
+  const dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
   // (tile lists in 256-row workgroups, by flag only: one instantiation serves causal and plain calls)
   if (sparse) return launch_shape<true, false, 8, true>(p, grid, max_lds<true, 8>(), n_qwg, n_wg, wg_per_xcd, s);
   // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
@@ -1071,8 +1089,9 @@ hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t s) {
   if (n_split == 0) return launch_shape<false, false, 8>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
   const int rest = n_wg - n_full;
   if (n_full > 0) {
-    const int per_xcd = (n_full + 7) / 8;
-    const hipError_t e = launch_shape<false, false, 8>(p, dim3(per_xcd * 8), lds, n_qwg, n_full, per_xcd, s);
+    int per_xcd = 0;
+    const dim3 grid_full = xcd_grid(&p, n_qwg, n_full, &per_xcd);
+    const hipError_t e = launch_shape<false, false, 8>(p, grid_full, lds, n_qwg, n_full, per_xcd, s);
     if (e != hipSuccess) return e;
   }
   AttnParams ps = p;
