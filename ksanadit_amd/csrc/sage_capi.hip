@@ -746,6 +746,41 @@ int ksana_sage_forward_masked(const void* q, const void* k, const void* v, void*
 }  // extern "C"
 
 namespace {
+// All three quantizers of a call whose arguments have been validated
+int quant_qkv(const void* q, const void* k, const void* v, int dtype, const int64_t q_st[4], const int64_t k_st[4],
+              const int64_t v_st[4], const ksana_sage_shape* s, const ksana_sage_prep* prep, float sm_scale, int smooth_k,
+              int smooth_v, void* ws, void* stream) {
+  if (!smooth_v) {
+    const StageRange range("ksana_sage.quant_qkv");
+    ksana_sage_ws_layout l;
+    ksana_sage_workspace_layout(s, &l);
+    ksana_sage::PrepParams pq, pk;
+    const ksana_sage::PrepParams *ppq = nullptr, *ppk = nullptr;
+    if (int rc = make_prep(prep, prep ? prep->q_norm_weight : nullptr, "q", q_st, s->B, s->Lq, s->D, ws_at<float>(ws, l.q_rms), &pq, &ppq))
+      return rc;
+    if (int rc = make_prep(prep, prep ? prep->k_norm_weight : nullptr, "k", k_st, s->B, s->Lk, s->D, ws_at<float>(ws, l.k_rms), &pk, &ppk))
+      return rc;
+    ksana_sage::QkvCall c{};
+    c.q = in_tensor(q, dtype, q_st, s->D), c.k = in_tensor(k, dtype, k_st, s->D), c.v = in_tensor(v, dtype, v_st, s->D);
+    c.B = s->B, c.Hq = s->Hq, c.Hkv = s->Hkv, c.Lq = s->Lq, c.Lk = s->Lk, c.lq_pad = l.lq_pad, c.nkb = l.nkb, c.nch = l.nch;
+    c.premul = (sm_scale * 1.4426950408889634f) * 0.0078125f;  // (as in quant_q_impl)
+    c.smooth_k = smooth_k ? 1 : 0;
+    c.q_i8 = ws_at<int8_t>(ws, l.q_i8), c.q_scale = ws_at<float>(ws, l.q_scale);
+    c.k_part = ws_at<float>(ws, l.k_part), c.k_mean = ws_at<float>(ws, l.k_mean);
+    c.k_tiles = ws_at<int8_t>(ws, l.k_i8), c.k_scale = ws_at<float>(ws, l.k_scale);
+    c.v_part = ws_at<float>(ws, l.v_part), c.v_scale = ws_at<float>(ws, l.v_scale), c.v_inv = ws_at<float>(ws, l.v_inv);
+    c.v_mean = ws_at<float>(ws, l.v_mean), c.v_tiles = ws_at<uint8_t>(ws, l.v_fp8);
+    const int bhk = s->B * s->Hkv;
+    c.sync = sync_at(ws_at<int>(ws, l.k_sync), ws_at<int>(ws, l.v_sync), bhk);
+    bool used = false;
+    const hipError_t e = ksana_sage::launch_quant_qkv(c, ppq, ppk, static_cast<hipStream_t>(stream), &used);
+    if (e != hipSuccess) return hip_fail(e, "q, k, v quantizer launch");
+    if (used) return 0;
+  }
+  if (int rc = ksana_sage_quant_qk_prep(q, k, dtype, q_st, k_st, s, prep, sm_scale, smooth_k, ws, stream)) return rc;
+  return ksana_sage_quant_v_smooth(v, dtype, v_st, s, smooth_v, ws, stream);
+}
+
 int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype, const int64_t q_st[4],
                  const int64_t k_st[4], const int64_t v_st[4], const int64_t o_st[4], const ksana_sage_shape* s,
                  const ksana_sage_prep* prep, const int8_t* block_mask, const int64_t mask_st[2],
@@ -772,8 +807,8 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
     if (int rc = make_prep(prep, prep ? prep->k_norm_weight : nullptr, "k", k_st, s->B, s->Lk, s->D, &dummy, &pp, &ppp))
       return rc;
   }
-  if (int rc = ksana_sage_quant_qk_prep(q, k, dtype, q_st, k_st, s, prep, sm_scale, smooth_k, ws, stream)) return rc;
-  if (int rc = ksana_sage_quant_v_smooth(v, dtype, v_st, s, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws, stream)) return rc;
+  if (int rc = quant_qkv(q, k, v, dtype, q_st, k_st, v_st, s, prep, sm_scale, smooth_k, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws, stream))
+    return rc;
   return ksana_sage_attn_fwd_masked(ws, o, dtype, o_st, s, block_mask, mask_st, k_lens, causal,
                                     flags & ~KSANA_SAGE_FLAG_SMOOTH_V, stream);
 }

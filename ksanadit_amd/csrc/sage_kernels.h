@@ -128,6 +128,25 @@ bool one_read_demoted(bool may_allocate = true);
 // resident-workgroup counts (a host-side self-check; touches no device)
 int selftest_occupancy_cache();
 
+// Q, K and V of one call (no V smoothing), see quant_qkv_stage1_kernel.  *used == false: the shape or the folded step does
+// not suit it and nothing was launched.  pq / pk: nullptr, or the step folded into q / k (kind 2 only).
+struct QkvCall {
+  InTensor q, k, v;
+  int B, Hq, Hkv, Lq, Lk, lq_pad, nkb, nch;
+  float premul;
+  int smooth_k;
+  int8_t* q_i8;
+  float* q_scale;
+  float *k_part, *k_mean;
+  int8_t* k_tiles;
+  float* k_scale;
+  float *v_part, *v_scale, *v_inv, *v_mean;
+  uint8_t* v_tiles;
+  QuantSync sync;  // (the areas of K and V follow each other)
+  int tiles_per_wg;  // filled in by the launcher
+};
+hipError_t launch_quant_qkv(const QkvCall& call, const PrepParams* pq, const PrepParams* pk, hipStream_t s, bool* used);
+
 // One-read quantizers: *used == false means the shape does not suit them and nothing was launched.
 // `may_allocate`: see one_read_demoted.
 hipError_t launch_quant_k_fused(const InTensor& k, int B, int H, int L, int nkb, int nch, int smooth, float* part,
@@ -136,6 +155,7 @@ hipError_t launch_quant_k_fused(const InTensor& k, int B, int H, int L, int nkb,
 hipError_t launch_quant_v_fused(const InTensor& v, int B, int H, int L, int nkb, int nch, float* part, float* v_scale,
                                 float* v_inv, float* v_mean, uint8_t* v_tiles, const QuantSync& sync, hipStream_t s,
                                 bool* used);
+
 
 // out[b, h, blk, :] = mean of the rows of block blk (rows per block: a multiple of 32, at most 256) of x[b, :, h, :],
 // of round_to_half(x - centre[b, h, :]) when centre != nullptr; out is [B, H, ceil(L / rows), 128] in x's half type

@@ -371,31 +371,38 @@ __global__ __launch_bounds__(kThreads) void row_inv_rms_kernel(const uint16_t* _
 // centre is the channel mean).  grid = (nch, H, B).
 // ---------------------------------------------------------------------------------------
 template <int DT, int OP, int PRE>
-__global__ __launch_bounds__(kThreads) void col_partial_kernel(const uint16_t* __restrict__ x, int64_t sB, int64_t sL,
-                                                               int64_t sH, int H, int L_all, int d_in, float* __restrict__ part,
-                                                               int nch, const PrepParams pp,
-                                                               const float* __restrict__ centre) {
+__device__ __forceinline__ void col_partial_chunk(int ch, int h, int b, const uint16_t* __restrict__ x, int64_t sB, int64_t sL,
+                                                  int64_t sH, int H, int L_all, int d_in, float* __restrict__ part, int nch,
+                                                  const PrepParams& pp, const float* __restrict__ centre) {
   constexpr bool kSum = OP == 0;
-  const int ch = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
   const int L = c16 * 16 < d_in ? L_all : 0;  // channels at or past d_in (head size 64) read as zero padding
   const uint16_t* base = x + b * sB + h * sH + c16 * 16;
   const RopeLds rl = maybe_stage_rope<PRE>(pp, b, ch * kMeanChunk, kMeanChunk);
   float acc[16];
   if constexpr (PRE) {
-    float rows[kMeanChunk / kSlots][16];
+    // all loads first, then the rows one after the other as they arrive (as in quant_k_chunk)
+    uint4 raw[kMeanChunk / kSlots][2];
 #pragma unroll
     for (int i = 0; i < kMeanChunk / kSlots; ++i) {
       const int row = ch * kMeanChunk + i * kSlots + slot;
-      load_row16<DT>(base + (int64_t)row * sL, row < L, rows[i]);
-      if (row < L) prep16<DT, PRE>(rows[i], pp, rl, b, row, h, c16);
+      fetch_row16(base + (int64_t)row * sL, row < L, raw[i]);
     }
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = kSum ? rows[0][e] : fabsf(rows[0][e]);
+    for (int i = 0; i < kMeanChunk / kSlots; ++i) {
+      const int row = ch * kMeanChunk + i * kSlots + slot;
+      float x[16];
+      widen8<DT>(raw[i][0], x);
+      widen8<DT>(raw[i][1], x + 8);
+      if (row < L) prep16<DT, PRE>(x, pp, rl, b, row, h, c16);
 #pragma unroll
-    for (int i = 1; i < kMeanChunk / kSlots; ++i) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[e] = kSum ? acc[e] + rows[i][e] : fmaxf(acc[e], fabsf(rows[i][e]));
+      for (int e = 0; e < 16; ++e) {
+        if (i == 0)
+          acc[e] = kSum ? x[e] : fabsf(x[e]);
+        else
+          acc[e] = kSum ? acc[e] + x[e] : fmaxf(acc[e], fabsf(x[e]));
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
   } else {
     // all sixteen loads of the lane are issued first and stay in flight as 16-bit values; they are widened and
@@ -457,6 +464,14 @@ __global__ __launch_bounds__(kThreads) void col_partial_kernel(const uint16_t* _
     const float hi = kSum ? s_w[2][t] + s_w[3][t] : fmaxf(s_w[2][t], s_w[3][t]);
     part[(((int64_t)b * H + h) * nch + ch) * kD + t] = kSum ? lo + hi : fmaxf(lo, hi);
   }
+}
+
+template <int DT, int OP, int PRE>
+__global__ __launch_bounds__(kThreads) void col_partial_kernel(const uint16_t* __restrict__ x, int64_t sB, int64_t sL,
+                                                               int64_t sH, int H, int L_all, int d_in, float* __restrict__ part,
+                                                               int nch, const PrepParams pp,
+                                                               const float* __restrict__ centre) {
+  col_partial_chunk<DT, OP, PRE>(blockIdx.x, blockIdx.y, blockIdx.z, x, sB, sL, sH, H, L_all, d_in, part, nch, pp, centre);
 }
 
 // Finalisation of the column reductions.  grid = B*H, 1024 threads.  All chunk partials of the
@@ -701,13 +716,12 @@ __device__ __forceinline__ void store_block_mean(float (&acc)[16], int t, float 
 // ---------------------------------------------------------------------------------------
 // POOL: the workgroup's 128 rows are one block of the sparse-linear backend's block map; their average (of the input
 // as it is) goes to pooled[b, h, blk, :] - what block_mean_kernel would read q a second time for.
-template <int DT, int PRE, bool POOL = false>
-__global__ __launch_bounds__(kThreads) void quant_q_kernel(const uint16_t* __restrict__ q, int64_t sB, int64_t sL,
-                                                           int64_t sH, int H, int L_all, int d_in, int lq_pad, float premul,
-                                                           int8_t* __restrict__ q_i8, float* __restrict__ q_scale,
-                                                           const PrepParams pp, uint16_t* __restrict__ pooled = nullptr) {
+template <int DT, int PRE, bool POOL>
+__device__ __forceinline__ void quant_q_block(int blk, int h, int b, const uint16_t* __restrict__ q, int64_t sB, int64_t sL,
+                                              int64_t sH, int H, int L_all, int d_in, int lq_pad, float premul,
+                                              int8_t* __restrict__ q_i8, float* __restrict__ q_scale, const PrepParams& pp,
+                                              uint16_t* __restrict__ pooled) {
   static_assert(!(POOL && PRE), "block averages are taken of the tensor as it is");
-  const int blk = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
   const int L = c16 * 16 < d_in ? L_all : 0;  // channels at or past d_in (head size 64) read as zero padding
   const uint16_t* base = q + b * sB + h * sH + c16 * 16;
@@ -762,11 +776,20 @@ __global__ __launch_bounds__(kThreads) void quant_q_kernel(const uint16_t* __res
       static_assert(R == 4, "four rows per slot");
       __shared__ float s_w[4][kD];
       store_block_mean<DT>(acc, t, (float)min(kRowsPerWg, L_all - blk * kRowsPerWg),
-                           pooled + (bh * gridDim.x + blk) * kD, s_w);
+                           pooled + (bh * (lq_pad / kRowsPerWg) + blk) * kD, s_w);
     }
 #pragma unroll
     for (int i = 0; i < R; ++i) finish_row(x[i], blk * kRowsPerWg + i * kSlots + slot);
   }
+}
+
+template <int DT, int PRE, bool POOL = false>
+__global__ __launch_bounds__(kThreads) void quant_q_kernel(const uint16_t* __restrict__ q, int64_t sB, int64_t sL,
+                                                           int64_t sH, int H, int L_all, int d_in, int lq_pad, float premul,
+                                                           int8_t* __restrict__ q_i8, float* __restrict__ q_scale,
+                                                           const PrepParams pp, uint16_t* __restrict__ pooled = nullptr) {
+  quant_q_block<DT, PRE, POOL>(blockIdx.x, blockIdx.y, blockIdx.z, q, sB, sL, sH, H, L_all, d_in, lq_pad, premul, q_i8, q_scale,
+                               pp, pooled);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -920,24 +943,29 @@ __global__ __launch_bounds__(kThreads) void quant_q_rows_kernel(const uint16_t* 
 // POOL: the workgroup's 64 rows are one key block of the sparse-linear backend's block map; the average of
 // k - mean(k), each difference rounded to the tensor's half type first as the reference forms it, goes to
 // pooled[b, h, blk, :] - what block_mean_kernel would read k a third time for.
-template <int DT, int PRE, bool POOL = false>
-__global__ __launch_bounds__(kThreads) void quant_k_kernel(const uint16_t* __restrict__ k, int64_t sB, int64_t sL,
-                                                           int64_t sH, int H, int L_all, int d_in, int nkb,
-                                                           const float* __restrict__ k_mean,
-                                                           int8_t* __restrict__ k_tiles, float* __restrict__ k_scale,
-                                                           const PrepParams pp, uint16_t* __restrict__ pooled = nullptr) {
+// `mean`: where the head's channel means are found (128 floats, global memory or LDS) - called once the rows are on
+// their way.
+template <int DT, int PRE, bool POOL, typename Mean>
+__device__ __forceinline__ void quant_k_block(int blk, int h, int b, const uint16_t* __restrict__ k, int64_t sB, int64_t sL,
+                                              int64_t sH, int H, int L_all, int d_in, int nkb, Mean&& mean,
+                                              int8_t* __restrict__ k_tiles, float* __restrict__ k_scale, const PrepParams& pp,
+                                              uint16_t* __restrict__ pooled) {
   static_assert(!(POOL && PRE), "block averages are taken of the tensor as it is");
-  // Heads and batch entries from the last one down: this pass follows the column-sum pass over the same tensor, which
-  // went upwards, so what that pass touched last - and the last-level cache may still hold - is read first.
-  const int blk = blockIdx.x, h = (int)gridDim.y - 1 - (int)blockIdx.y, b = (int)gridDim.z - 1 - (int)blockIdx.z;
   const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
   const int L = c16 * 16 < d_in ? L_all : 0;  // channels at or past d_in (head size 64) read as zero padding
   const int64_t bh = (int64_t)b * H + h;
   const uint16_t* base = k + b * sB + h * sH + c16 * 16;
+  constexpr int R = kBlkK / kSlots;
+  uint4 raw[R][2];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int row = blk * kBlkK + i * kSlots + slot;
+    fetch_row16(base + (int64_t)row * sL, row < L, raw[i]);
+  }
+  const float* k_mean = mean();
   float km[16];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) km[e] = k_mean[bh * kD + c16 * 16 + e];
-  constexpr int R = kBlkK / kSlots;
+  for (int e = 0; e < 16; ++e) km[e] = k_mean[c16 * 16 + e];
   const RopeLds rl = maybe_stage_rope<PRE>(pp, b, blk * kBlkK, kBlkK);
   float x[R][16];
   float amax = 0.0f;
@@ -946,7 +974,8 @@ __global__ __launch_bounds__(kThreads) void quant_k_kernel(const uint16_t* __res
   for (int i = 0; i < R; ++i) {
     const int row = blk * kBlkK + i * kSlots + slot;
     const bool valid = row < L;
-    load_row16<DT>(base + (int64_t)row * sL, valid, x[i]);
+    widen8<DT>(raw[i][0], x[i]);
+    widen8<DT>(raw[i][1], x[i] + 8);
     if constexpr (PRE) {
       if (valid) prep16<DT, PRE>(x[i], pp, rl, b, row, h, c16);
     }
@@ -984,29 +1013,46 @@ __global__ __launch_bounds__(kThreads) void quant_k_kernel(const uint16_t* __res
   }
 }
 
+template <int DT, int PRE, bool POOL = false>
+__global__ __launch_bounds__(kThreads) void quant_k_kernel(const uint16_t* __restrict__ k, int64_t sB, int64_t sL,
+                                                           int64_t sH, int H, int L_all, int d_in, int nkb,
+                                                           const float* __restrict__ k_mean,
+                                                           int8_t* __restrict__ k_tiles, float* __restrict__ k_scale,
+                                                           const PrepParams pp, uint16_t* __restrict__ pooled = nullptr) {
+  // Heads and batch entries from the last one down: this pass follows the column-sum pass over the same tensor, which
+  // went upwards, so what that pass touched last - and the last-level cache may still hold - is read first.
+  const int h = (int)gridDim.y - 1 - (int)blockIdx.y, b = (int)gridDim.z - 1 - (int)blockIdx.z;
+  quant_k_block<DT, PRE, POOL>(blockIdx.x, h, b, k, sB, sL, sH, H, L_all, d_in, nkb,
+                               [&] { return k_mean + ((int64_t)b * H + h) * kD; }, k_tiles, k_scale, pp, pooled);
+}
+
 // ---------------------------------------------------------------------------------------
 // V: one workgroup per 64-row block.  grid = (nkb, H, B).  Scales with 448/amax[d], converts
 // to e4m3fn, transposes through LDS and writes the V^T tile in the order the fp8 MFMA
 // consumes it: chunk (dt = d/32, tt = half of the 64 rows) is 64 lanes x 16 bytes,
 // lane = 32*hh + d%32, byte r <-> row 32*tt + 8*(r/4) + 4*hh + r%4.
 // ---------------------------------------------------------------------------------------
-template <int DT, bool CENTRE>
-__global__ __launch_bounds__(kThreads) void quant_v_kernel(const uint16_t* __restrict__ v, int64_t sB, int64_t sL,
-                                                           int64_t sH, int H, int L_all, int d_in, int nkb,
-                                                           const float* __restrict__ v_inv,
-                                                           const float* __restrict__ v_mean,
-                                                           uint8_t* __restrict__ v_tiles) {
-  // (heads and batch entries from the last one down, like quant_k_kernel: the abs-max pass went upwards)
-  const int blk = blockIdx.x, h = (int)gridDim.y - 1 - (int)blockIdx.y, b = (int)gridDim.z - 1 - (int)blockIdx.z;
+// `factors`: where the head's 128 factors 448 / amax are found - called once the rows are on their way.
+template <int DT, bool CENTRE, typename Factors>
+__device__ __forceinline__ void quant_v_block(int blk, int h, int b, const uint16_t* __restrict__ v, int64_t sB, int64_t sL,
+                                              int64_t sH, int H, int L_all, int d_in, int nkb, Factors&& factors,
+                                              const float* __restrict__ v_mean, uint8_t* __restrict__ v_tiles) {
   const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
   const int L = c16 * 16 < d_in ? L_all : 0;  // channels at or past d_in (head size 64) read as zero padding
   const int64_t bh = (int64_t)b * H + h;
   const uint16_t* base = v + b * sB + h * sH + c16 * 16;
   constexpr int kStride = kD + 16;  // LDS row pitch in bytes
   __shared__ __attribute__((aligned(16))) uint8_t s_v[kBlkK * kStride];
+  uint4 raw[kBlkK / kSlots][2];
+#pragma unroll
+  for (int i = 0; i < kBlkK / kSlots; ++i) {
+    const int row = blk * kBlkK + i * kSlots + slot;
+    fetch_row16(base + (int64_t)row * sL, row < L, raw[i]);
+  }
+  const float* v_inv = factors();
   float inv[16];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) inv[e] = v_inv[bh * kD + c16 * 16 + e];
+  for (int e = 0; e < 16; ++e) inv[e] = v_inv[c16 * 16 + e];
   float mean[16];
   if constexpr (CENTRE) {
 #pragma unroll
@@ -1015,9 +1061,10 @@ __global__ __launch_bounds__(kThreads) void quant_v_kernel(const uint16_t* __res
 #pragma unroll
   for (int i = 0; i < kBlkK / kSlots; ++i) {
     const int r = i * kSlots + slot;
-    const int row = blk * kBlkK + r;
+    [[maybe_unused]] const int row = blk * kBlkK + r;
     float x[16];
-    load_row16<DT>(base + (int64_t)row * sL, row < L, x);
+    widen8<DT>(raw[i][0], x);
+    widen8<DT>(raw[i][1], x + 8);
     if constexpr (CENTRE) {  // rows past the end stay zero
       if (row < L) {
 #pragma unroll
@@ -1059,6 +1106,17 @@ __global__ __launch_bounds__(kThreads) void quant_v_kernel(const uint16_t* __res
   }
 }
 
+template <int DT, bool CENTRE>
+__global__ __launch_bounds__(kThreads) void quant_v_kernel(const uint16_t* __restrict__ v, int64_t sB, int64_t sL,
+                                                           int64_t sH, int H, int L_all, int d_in, int nkb,
+                                                           const float* __restrict__ v_inv,
+                                                           const float* __restrict__ v_mean,
+                                                           uint8_t* __restrict__ v_tiles) {
+  // (heads and batch entries from the last one down, like quant_k_kernel: the abs-max pass went upwards)
+  const int h = (int)gridDim.y - 1 - (int)blockIdx.y, b = (int)gridDim.z - 1 - (int)blockIdx.z;
+  quant_v_block<DT, CENTRE>(blockIdx.x, h, b, v, sB, sL, sH, H, L_all, d_in, nkb,
+                            [&] { return v_inv + ((int64_t)b * H + h) * kD; }, v_mean, v_tiles);
+}
 
 // ---------------------------------------------------------------------------------------
 // One-read quantizers for K and V.
@@ -1185,17 +1243,13 @@ __device__ __forceinline__ void stage_partials(const float (&v)[kFinLoads], floa
   for (int j = 0; j < kFinLoads; ++j) s_part[(int)threadIdx.x + kThreads * j] = v[j];
 }
 
-// With the Wan step folded in the kernel is asked to fit three waves per SIMD (168 registers; it spills ten of them):
-// a workgroup idles while it waits for its head's mean, and with two workgroups per compute unit instead of three
-// the kernel measured 23 % slower.
-template <int DT, int PRE>
-__global__ __launch_bounds__(kThreads, PRE == 1 ? 3 : 1) void quant_k_fused_kernel(const uint16_t* __restrict__ k, int64_t sB, int64_t sL,
-                                                                 int64_t sH, int H, int L_all, int d_in, int nkb, int nch,
-                                                                 float* __restrict__ part, float* k_mean, int dtype,
-                                                                 int smooth, int8_t* __restrict__ k_tiles,
-                                                                 float* __restrict__ k_scale, const PrepParams pp,
-                                                                 const HeadSync sy) {
-  const int bh = blockIdx.x / nch, ch = blockIdx.x - bh * nch;
+// SOLO: the head is this one chunk (at most 256 rows), so its sums are the head's and nobody is waited for.
+template <int DT, int PRE, bool SOLO>
+__device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __restrict__ k, int64_t sB, int64_t sL,
+                                              int64_t sH, int H, int L_all, int d_in, int nkb, int nch,
+                                              float* __restrict__ part, float* k_mean, int dtype, int smooth,
+                                              int8_t* __restrict__ k_tiles, float* __restrict__ k_scale,
+                                              const PrepParams& pp, const HeadSync& sy) {
   const int b = bh / H, h = bh - b * H;
   const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
   const int L = c16 * 16 < d_in ? L_all : 0;  // channels at or past d_in (head size 64) read as zero padding
@@ -1255,6 +1309,14 @@ __global__ __launch_bounds__(kThreads, PRE == 1 ? 3 : 1) void quant_k_fused_kern
     for (int e = 0; e < 16; ++e) s_w[wave][c16 * 16 + e] = acc[e];
   }
   __syncthreads();
+  if constexpr (SOLO) {
+    if (t < kD) {
+      const float mean = round_to_half_dtype(__fdiv_rn((s_w[0][t] + s_w[1][t]) + (s_w[2][t] + s_w[3][t]), (float)L_all), dtype);
+      s_mean[t] = mean;
+      k_mean[bh * kD + t] = mean;
+    }
+    __syncthreads();
+  } else {
   if (t < kD) {
     publish_f32(part + ((int64_t)bh * nch + ch) * kD + t, (s_w[0][t] + s_w[1][t]) + (s_w[2][t] + s_w[3][t]));
     complete_accesses();  // the partial result is visible chip-wide before this chunk is counted in
@@ -1343,6 +1405,7 @@ __global__ __launch_bounds__(kThreads, PRE == 1 ? 3 : 1) void quant_k_fused_kern
     }
   }
   }
+  }
   // ---- 4. quantize the four 64-row tiles of the chunk from registers -----------------------------
 #pragma unroll
   for (int tt = 0; tt < kMeanChunk / kBlkK; ++tt) {
@@ -1380,16 +1443,29 @@ __global__ __launch_bounds__(kThreads, PRE == 1 ? 3 : 1) void quant_k_fused_kern
   }
 }
 
+// With the Wan step folded in the kernel is asked to fit three waves per SIMD (168 registers; it spills ten of them):
+// a workgroup idles while it waits for its head's mean, and with two workgroups per compute unit instead of three
+// the kernel measured 23 % slower.
+template <int DT, int PRE>
+__global__ __launch_bounds__(kThreads, PRE == 1 ? 3 : 1) void quant_k_fused_kernel(const uint16_t* __restrict__ k, int64_t sB, int64_t sL,
+                                                                 int64_t sH, int H, int L_all, int d_in, int nkb, int nch,
+                                                                 float* __restrict__ part, float* k_mean, int dtype,
+                                                                 int smooth, int8_t* __restrict__ k_tiles,
+                                                                 float* __restrict__ k_scale, const PrepParams pp,
+                                                                 const HeadSync sy) {
+  const int bh = blockIdx.x / nch;
+  quant_k_chunk<DT, PRE, false>(bh, blockIdx.x - bh * nch, k, sB, sL, sH, H, L_all, d_in, nkb, nch, part, k_mean, dtype, smooth,
+                                k_tiles, k_scale, pp, sy);
+}
+
 // V: column abs-max of the whole sequence (the last workgroup of a head to arrive takes the maximum over the
 // chunks' maxima - no order to respect - and publishes the scales), then per-channel e4m3 in the transposed tile
 // order of quant_v_kernel.
-template <int DT>
-__global__ __launch_bounds__(kThreads) void quant_v_fused_kernel(const uint16_t* __restrict__ v, int64_t sB, int64_t sL,
-                                                                 int64_t sH, int H, int L_all, int d_in, int nkb, int nch,
-                                                                 float* __restrict__ part, float* v_scale, float* v_inv,
-                                                                 float* __restrict__ v_mean,
-                                                                 uint8_t* __restrict__ v_tiles, const HeadSync sy) {
-  const int bh = blockIdx.x / nch, ch = blockIdx.x - bh * nch;
+template <int DT, bool SOLO>
+__device__ __forceinline__ void quant_v_chunk(int bh, int ch, const uint16_t* __restrict__ v, int64_t sB, int64_t sL,
+                                              int64_t sH, int H, int L_all, int d_in, int nkb, int nch,
+                                              float* __restrict__ part, float* v_scale, float* v_inv,
+                                              float* __restrict__ v_mean, uint8_t* __restrict__ v_tiles, const HeadSync& sy) {
   const int b = bh / H, h = bh - b * H;
   const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
   const int L = c16 * 16 < d_in ? L_all : 0;  // channels at or past d_in (head size 64) read as zero padding
@@ -1428,6 +1504,18 @@ __global__ __launch_bounds__(kThreads) void quant_v_fused_kernel(const uint16_t*
     for (int e = 0; e < 16; ++e) s_w[wave][c16 * 16 + e] = acc[e];
   }
   __syncthreads();
+  if constexpr (SOLO) {
+    if (t < kD) {
+      const float amax = fmaxf(fmaxf(s_w[0][t], s_w[1][t]), fmaxf(s_w[2][t], s_w[3][t]));
+      const bool nz = amax > 0.0f;
+      const float inv = nz ? __fdiv_rn(448.0f, amax) : 0.0f;
+      s_inv[t] = inv;
+      v_inv[bh * kD + t] = inv;
+      v_scale[bh * kD + t] = nz ? __fdiv_rn(amax, 448.0f) : 0.0f;
+      v_mean[bh * kD + t] = 0.0f;
+    }
+    __syncthreads();
+  } else {
   if (t < kD) {
     publish_f32(part + ((int64_t)bh * nch + ch) * kD + t, fmaxf(fmaxf(s_w[0][t], s_w[1][t]), fmaxf(s_w[2][t], s_w[3][t])));
     complete_accesses();  // visible chip-wide before this chunk is counted in
@@ -1500,6 +1588,7 @@ __global__ __launch_bounds__(kThreads) void quant_v_fused_kernel(const uint16_t*
       __syncthreads();
     }
   }
+  }
   float inv[16];
 #pragma unroll
   for (int e = 0; e < 16; ++e) inv[e] = s_inv[c16 * 16 + e];
@@ -1548,6 +1637,184 @@ __global__ __launch_bounds__(kThreads) void quant_v_fused_kernel(const uint16_t*
       store_out16(tile + oc * 16, make_uint4(w[0], w[1], w[2], w[3]));
     }
   }
+}
+
+template <int DT>
+__global__ __launch_bounds__(kThreads) void quant_v_fused_kernel(const uint16_t* __restrict__ v, int64_t sB, int64_t sL,
+                                                                 int64_t sH, int H, int L_all, int d_in, int nkb, int nch,
+                                                                 float* __restrict__ part, float* v_scale, float* v_inv,
+                                                                 float* __restrict__ v_mean,
+                                                                 uint8_t* __restrict__ v_tiles, const HeadSync sy) {
+  const int bh = blockIdx.x / nch;
+  quant_v_chunk<DT, false>(bh, blockIdx.x - bh * nch, v, sB, sL, sH, H, L_all, d_in, nkb, nch, part, v_scale, v_inv, v_mean, v_tiles,
+                           sy);
+}
+
+// ---------------------------------------------------------------------------------------
+// Q, K and V of one call together, in one or two launches.
+//
+// Separate quantizers are six launches, and below a few thousand tokens each of them is bound by being one: 4-5 us from
+// the end of a kernel to the end of the next however little the next does.  Three forms (launch_quant_qkv picks):
+//
+//   small    at most 256 keys, one chunk per head: the K and V workgroups hold their whole head, one launch does all.
+//   stages   stage 1 takes the chunk sums of K, the chunk maxima of V and quantizes Q; stage 2 quantizes K and V, every
+//            workgroup forming its head's statistic from the chunks' by itself (the same operations in the same order as
+//            the finalisation kernels).  Stage 2 reads its inputs a second time - out of the caches while K and V fit
+//            them - and nch * 512 bytes of partial results per workgroup.
+//   meet     one launch, every input read once: K's and V's chunks meet per head as in the one-read kernels above.
+//
+// Measured, all quantizer launches of a call, us (separate quantizers / this):  B=2, 64 heads, 32 tokens 27 / 8 small;
+// 40 heads, 1560 tokens 43 / 22 stages; 9000 tokens 107 stages, 113 meet; 14000 tokens 201 stages, 169 meet; 32760
+// tokens 398 / 383 meet (HBM-bound: 9 bytes per element at 4 TB/s).
+// ---------------------------------------------------------------------------------------
+template <int OP>  // 0: K's mean (ordered sum), 1: V's factor 448 / amax
+__device__ __forceinline__ void head_statistic(const QkvCall& c, int bh, bool publish, float (*s_stat)[kD]) {
+  const int t = threadIdx.x, d = t & (kD - 1);
+  const float* hp = (OP == 0 ? c.k_part : c.v_part) + (int64_t)bh * c.nch * kD + d;
+  if constexpr (OP == 0) {
+    if (t < kD) {
+      float tot = 0.0f;
+      if (c.smooth_k) {
+        for (int c0 = 0; c0 < c.nch; c0 += 16) {  // 16 loads in flight; added in chunk order
+          float v[16];
+#pragma unroll
+          for (int j = 0; j < 16; ++j) v[j] = hp[min(c0 + j, c.nch - 1) * kD];
+#pragma unroll
+          for (int j = 0; j < 16; ++j)
+            if (c0 + j < c.nch) tot = c0 + j == 0 ? v[0] : tot + v[j];
+        }
+      }
+      const float mean = c.smooth_k ? round_to_half_dtype(__fdiv_rn(tot, (float)c.Lk), c.k.dtype) : 0.0f;
+      s_stat[0][d] = mean;
+      if (publish) c.k_mean[bh * kD + d] = mean;
+    }
+    __syncthreads();
+  } else {
+    float m = 0.0f;  // a maximum needs no order: the two halves of the workgroup take the even and the odd chunks
+    for (int c0 = t >> 7; c0 < c.nch; c0 += 32) {
+      float v[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[j] = hp[min(c0 + 2 * j, c.nch - 1) * kD];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) m = fmaxf(m, v[j]);  // (a chunk taken twice changes no maximum)
+    }
+    s_stat[t >> 7][d] = m;
+    __syncthreads();
+    const float amax = fmaxf(s_stat[0][d], s_stat[1][d]);
+    const bool nz = amax > 0.0f;
+    const float inv = nz ? __fdiv_rn(448.0f, amax) : 0.0f;
+    __syncthreads();
+    if (t < kD) {
+      s_stat[0][d] = inv;
+      if (publish) {
+        c.v_inv[bh * kD + d] = inv;
+        c.v_scale[bh * kD + d] = nz ? __fdiv_rn(amax, 448.0f) : 0.0f;
+        c.v_mean[bh * kD + d] = 0.0f;  // the attention adds whatever the slot holds
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// (this form has no wait that could expire)
+__device__ __forceinline__ void clear_status(const QkvCall& c) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *c.sync.k_status = 0, *c.sync.v_status = 0;
+}
+
+template <int DT, int KIND>
+__device__ __forceinline__ void quant_q_item(int item, const QkvCall& c, const PrepParams& pp) {
+  const int nqb = c.lq_pad / kQPad, bh = item / nqb;
+  quant_q_block<DT, KIND, false>(item - bh * nqb, bh % c.Hq, bh / c.Hq, c.q.ptr, c.q.sB, c.q.sL, c.q.sH, c.Hq, c.Lq, c.q.D, c.lq_pad,
+                                 c.premul, c.q_i8, c.q_scale, pp, nullptr);
+}
+
+template <int DT, int KIND>
+__global__ __launch_bounds__(kThreads, KIND == 0 ? 5 : 4) void quant_qkv_stage1_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
+  clear_status(c);
+  const int n_v = c.B * c.Hkv * c.nch, n_k = c.smooth_k ? n_v : 0;
+  int item = blockIdx.x;
+  if (item < n_k) {
+    const int bh = item / c.nch;
+    col_partial_chunk<DT, 0, KIND>(item - bh * c.nch, bh % c.Hkv, bh / c.Hkv, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D,
+                                   c.k_part, c.nch, pk, nullptr);
+    return;
+  }
+  item -= n_k;
+  if (item < n_v) {
+    const int bh = item / c.nch;
+    col_partial_chunk<DT, 1, 0>(item - bh * c.nch, bh % c.Hkv, bh / c.Hkv, c.v.ptr, c.v.sB, c.v.sL, c.v.sH, c.Hkv, c.Lk, c.v.D, c.v_part,
+                                c.nch, pk, nullptr);
+    return;
+  }
+  quant_q_item<DT, KIND>(item - n_v, c, pq);
+}
+
+template <int DT, int KIND>
+__global__ __launch_bounds__(kThreads, KIND == 0 ? 6 : 5) void quant_qkv_stage2_kernel(const QkvCall c, const PrepParams pk) {
+  __shared__ float s_stat[2][kD];
+  const int per_head = (c.nkb + c.tiles_per_wg - 1) / c.tiles_per_wg, n = c.B * c.Hkv * per_head;
+  const bool is_v = (int)blockIdx.x >= n;
+  const int item = is_v ? blockIdx.x - n : blockIdx.x;
+  const int bh = item / per_head, run = item - bh * per_head, b = bh / c.Hkv, h = bh - b * c.Hkv;
+  const int first = run * c.tiles_per_wg, last = min(c.nkb, first + c.tiles_per_wg);
+  auto stat = [&]() -> const float* { return s_stat[0]; };
+  if (is_v) {
+    head_statistic<1>(c, bh, run == 0, s_stat);
+    for (int blk = first; blk < last; ++blk) {
+      quant_v_block<DT, false>(blk, h, b, c.v.ptr, c.v.sB, c.v.sL, c.v.sH, c.Hkv, c.Lk, c.v.D, c.nkb, stat, nullptr, c.v_tiles);
+      __syncthreads();  // the tile has been read out of LDS
+    }
+  } else {
+    head_statistic<0>(c, bh, run == 0, s_stat);
+    for (int blk = first; blk < last; ++blk) {
+      quant_k_block<DT, KIND, false>(blk, h, b, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.nkb, stat, c.k_tiles, c.k_scale,
+                                     pk, nullptr);
+      __syncthreads();
+    }
+  }
+}
+
+// One launch over inputs that are read once: the chunks of K and V meet per head as in the one-read kernels above, and
+// the items of a head - its K chunks, its V chunks, the Q blocks of its query heads - are neighbours in the grid, so the
+// Q blocks (which wait for nobody) and the V chunks work while K's chunks wait for their mean.
+template <int DT, int KIND>
+__global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk,
+                                                                     const HeadSync sk, const HeadSync sv) {
+  const int nqb = c.lq_pad / kQPad, group = c.Hq / c.Hkv, per_head = 2 * c.nch + group * nqb;
+  const int bh = blockIdx.x / per_head;
+  int item = blockIdx.x - bh * per_head;
+  if (item < c.nch) {
+    quant_k_chunk<DT, KIND, false>(bh, item, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.nkb, c.nch, c.k_part, c.k_mean,
+                                   c.k.dtype, c.smooth_k, c.k_tiles, c.k_scale, pk, sk);
+    return;
+  }
+  item -= c.nch;
+  if (item < c.nch) {
+    quant_v_chunk<DT, false>(bh, item, c.v.ptr, c.v.sB, c.v.sL, c.v.sH, c.Hkv, c.Lk, c.v.D, c.nkb, c.nch, c.v_part, c.v_scale, c.v_inv,
+                             c.v_mean, c.v_tiles, sv);
+    return;
+  }
+  item -= c.nch;
+  const int b = bh / c.Hkv, hk = bh - b * c.Hkv;
+  const int hq = hk * group + item / nqb;
+  quant_q_item<DT, KIND>((b * c.Hq + hq) * nqb + item % nqb, c, pq);
+}
+
+// at most 256 keys: one launch
+template <int DT, int KIND>
+__global__ __launch_bounds__(kThreads, 4) void quant_qkv_small_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
+  clear_status(c);
+  const int n = c.B * c.Hkv;
+  const int item = blockIdx.x;
+  const HeadSync nobody{};
+  if (item < n)
+    quant_k_chunk<DT, KIND, true>(item, 0, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.nkb, 1, c.k_part, c.k_mean, c.k.dtype,
+                                  c.smooth_k, c.k_tiles, c.k_scale, pk, nobody);
+  else if (item < 2 * n)
+    quant_v_chunk<DT, true>(item - n, 0, c.v.ptr, c.v.sB, c.v.sL, c.v.sH, c.Hkv, c.Lk, c.v.D, c.nkb, 1, c.v_part, c.v_scale, c.v_inv,
+                            c.v_mean, c.v_tiles, nobody);
+  else
+    quant_q_item<DT, KIND>(item - 2 * n, c, pq);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1962,6 +2229,62 @@ hipError_t launch_quant_v_fused(const InTensor& v, int B, int H, int L, int nkb,
     }
   });
   if (*used) e = hipGetLastError();
+  return e;
+}
+
+// Two stages while a head's partial results stay small next to the rows a workgroup of stage 2 quantizes (64 chunks are
+// 32 KiB, the rows 16-64 KiB) and the second reading of K and V comes from the last-level cache (256 MB): 40 heads of
+// 9000 tokens (184 MB of K and V) take 107 us in two stages and 113 in one meeting launch, 14000 tokens 201 and 169.
+constexpr int kStageMaxChunks = 64;
+constexpr int64_t kStageMaxBytes = 192ll << 20;
+// Beyond this many chunks a head's first workgroups wait for its last ones longer than a second pass takes (296 chunks:
+// the separate quantizers are 3 % faster).
+constexpr int kMeetMaxChunks = 160;
+
+template <int DT, int KIND>
+static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepParams& pk, hipStream_t s, bool* used) {
+  const dim3 block(kThreads);
+  const int64_t n_q = (int64_t)c.B * c.Hq * (c.lq_pad / kQPad), n_chunks = (int64_t)c.B * c.Hkv * c.nch;
+  if (c.nch == 1) {
+    quant_qkv_small_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, pq, pk);
+    *used = true;
+  } else if (c.nch <= kStageMaxChunks && 4 * (int64_t)c.B * c.Hkv * c.Lk * c.k.D <= kStageMaxBytes) {
+    // about four workgroups per compute unit before a workgroup is given more than one tile per statistic
+    const int64_t tiles = 2 * (int64_t)c.B * c.Hkv * c.nkb;
+    c.tiles_per_wg = tiles >= 4096 ? 4 : (tiles >= 2048 ? 2 : 1);
+    const int64_t n2 = 2 * (int64_t)c.B * c.Hkv * ((c.nkb + c.tiles_per_wg - 1) / c.tiles_per_wg);
+    quant_qkv_stage1_kernel<DT, KIND><<<dim3((unsigned)(n_q + (c.smooth_k ? 2 : 1) * n_chunks)), block, 0, s>>>(c, pq, pk);
+    quant_qkv_stage2_kernel<DT, KIND><<<dim3((unsigned)n2), block, 0, s>>>(c, pk);
+    *used = true;
+  } else if (c.nch <= kMeetMaxChunks) {
+    const QuantOptions opt = quant_options();
+    // (V's one-read setting stands for both: K's concerns its separate kernel, which nothing shares the chip with)
+    if (!opt.one_read_v || one_read_demoted()) return hipSuccess;
+    if (2 * c.nch > resident_workgroups(quant_qkv_meet_kernel<DT, KIND>, 0)) return hipSuccess;
+    int* host = host_word(false).dev;
+    const QuantSync& y = c.sync;
+    const int n_words = (int)(y.v_status - y.k_counter) + kSyncStride;
+    const hipError_t e = launch_clear_ints(y.k_counter, n_words, s);
+    if (e != hipSuccess) return e;
+    const HeadSync sk{y.k_counter, y.k_ready, y.k_status, opt.wait_ticks, host}, sv{y.v_counter, y.v_ready, y.v_status, opt.wait_ticks, host};
+    quant_qkv_meet_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, pq, pk, sk, sv);
+    *used = true;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_quant_qkv(const QkvCall& call, const PrepParams* pq, const PrepParams* pk, hipStream_t s, bool* used) {
+  *used = false;
+  QkvCall c = call;
+  const int kind = pq != nullptr ? pq->kind : (pk != nullptr ? pk->kind : 0);
+  if (kind != 0 && kind != 2) return hipSuccess;
+  if ((int64_t)c.B * c.Hq * (c.lq_pad / kQPad) + 2 * (int64_t)c.B * c.Hkv * c.nkb > INT32_MAX) return hipSuccess;
+  // (a side without anything to apply runs with every step of its parameters switched off)
+  PrepParams off{};
+  off.kind = kind;
+  const PrepParams &a = pq != nullptr ? *pq : off, &b = pk != nullptr ? *pk : off;
+  hipError_t e = hipSuccess;
+  KSANA_DISPATCH_DT(c.q.dtype, { e = kind == 0 ? launch_qkv_kind<DT, 0>(c, a, b, s, used) : launch_qkv_kind<DT, 2>(c, a, b, s, used); });
   return e;
 }
 

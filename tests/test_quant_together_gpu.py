@@ -1,0 +1,57 @@
+"""Q, K and V quantized together (the first launches of a whole call) against the separate quantizers, which are pinned
+to the oracle bit for bit in test_quant_gpu.py and test_prep_gpu.py: the same bits in every area of the workspace."""
+
+import pytest
+import torch
+
+from ksanadit_amd import sage_ops
+
+pytestmark = pytest.mark.gpu
+
+AREAS = ("q_i8", "q_scale", "k_tiles", "k_scale", "k_mean", "v_tiles", "v_scale", "v_mean")
+
+
+def _compare(hip_device, B, Lq, Lk, Hq, Hkv, D, dtype, smooth_k=True, prep=None, strided=False):
+    g = torch.Generator(device=hip_device).manual_seed(Lq + 7 * Lk + D)
+
+    def draw(L, H):
+        x = torch.randn((B, L, H + (1 if strided else 0), D), generator=g, device=hip_device)
+        x = x + 2.0 * torch.randn((H + (1 if strided else 0), D), generator=g, device=hip_device)
+        return x.to(dtype)[:, :, :H]
+
+    q, k, v = draw(Lq, Hq), draw(Lk, Hkv), draw(Lk, Hkv)
+    v[:, :, 0, 3] = 0  # a channel that is zero throughout
+    k[:, : min(64, Lk), 0] = 0
+    ws, want = sage_ops.workspace_for(q, k), sage_ops.workspace_for(q, k)
+    ws.blob.fill_(0x7F), want.blob.fill_(0x7F)
+    out = sage_ops.sageattn(q, k, v, workspace=ws, smooth_k=smooth_k, prep=prep)
+    sage_ops.quant_qk(q, k, want, D**-0.5, smooth_k, prep=prep)
+    sage_ops.quant_v(v, want)
+    for name in AREAS:
+        assert torch.equal(getattr(ws, name).view(torch.uint8), getattr(want, name).view(torch.uint8)), name
+    assert sage_ops.quant_status(ws) == (0, 0)
+    assert torch.equal(out, sage_ops.attn_fwd(want, torch.empty_like(out)))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Lq,Lk,Hq,Hkv,D,smooth_k", [
+    (2, 32, 32, 4, 4, 128, True), (1, 1, 1, 1, 1, 128, True), (1, 300, 256, 2, 1, 128, True), (1, 40, 256, 2, 2, 64, False),
+    (1, 129, 257, 3, 3, 128, True), (2, 513, 1560, 4, 2, 128, True), (1, 100, 640, 2, 2, 64, True), (1, 64, 700, 2, 2, 128, False),
+    (1, 200, 16384, 2, 2, 128, True), (1, 64, 16385, 1, 1, 128, True), (1, 128, 8300, 16, 16, 128, True),
+    (1, 128, 20000, 24, 12, 128, True), (1, 128, 17000, 1, 1, 64, False)])
+def test_together_gives_the_separate_quantizers_bits(hip_device, B, Lq, Lk, Hq, Hkv, D, smooth_k, dtype):
+    print(f"case B={B} Lq={Lq} Lk={Lk} Hq={Hq} Hkv={Hkv} D={D} smooth_k={smooth_k} {dtype}", flush=True)
+    _compare(hip_device, B, Lq, Lk, Hq, Hkv, D, dtype, smooth_k)
+    _compare(hip_device, B, Lq, Lk, Hq, Hkv, D, dtype, smooth_k, strided=True)
+
+
+@pytest.mark.parametrize("txt,img,weights,tables", [(5, 60, True, True), (256, 1000, True, True), (300, 400, False, True), (13, 3000, True, False)])
+def test_together_with_the_joint_block_step(hip_device, txt, img, weights, tables):
+    print(f"case txt={txt} img={img} weights={weights} tables={tables}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(txt)
+    ws = [1.0 + 0.2 * torch.randn(128, generator=g, device=hip_device) if weights else None for _ in range(4)]
+    ang = torch.rand((txt + img, 64), generator=g, device=hip_device) * 6.0
+    tab = torch.polar(torch.ones_like(ang), ang) if tables else None
+    prep = sage_ops.QwenPrep(txt, *ws, 1e-6, img_freqs=None if tab is None else tab[:img].contiguous(),
+                             txt_freqs=None if tab is None else tab[img:].contiguous())
+    _compare(hip_device, 2, txt + img, txt + img, 3, 3, 128, torch.bfloat16, True, prep)
