@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define KSANA_SAGE_ABI_VERSION 20
+#define KSANA_SAGE_ABI_VERSION 21
 
 /* element types of q/k/v/o */
 #define KSANA_SAGE_BF16 0
@@ -380,6 +380,15 @@ int ksana_sage_forward_masked(const void* q, const void* k, const void* v, void*
                               const int64_t o_strides[4], const ksana_sage_shape* shape, const int8_t* block_mask,
                               const int64_t mask_strides[2], const int32_t* k_lens, float sm_scale, int smooth_k,
                               int causal, int flags, void* workspace, void* stream);
+
+/* The three calls above in their general form: any of `prep`, `block_mask`, `q_lens` (see ksana_sage_attn_fwd_varlen) and
+ * `k_lens` may be NULL, and the result is written in `o_dtype`. */
+int ksana_sage_forward_varlen(const void* q, const void* k, const void* v, void* o, int dtype, int o_dtype,
+                              const int64_t q_strides[4], const int64_t k_strides[4], const int64_t v_strides[4],
+                              const int64_t o_strides[4], const ksana_sage_shape* shape, const ksana_sage_prep* prep,
+                              const int8_t* block_mask, const int64_t mask_strides[2], const int32_t* q_lens,
+                              const int32_t* k_lens, float sm_scale, int smooth_k, int causal, int flags,
+                              void* workspace, void* stream);
 
 #ifdef __cplusplus
 }

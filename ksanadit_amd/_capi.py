@@ -11,7 +11,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libksana_sage_hip.so"
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 BF16, FP16 = 0, 1
 OK, EINVAL, ENOTSUP, EHIP = 0, -1, -2, -3
@@ -52,6 +52,7 @@ EXPORTS = (
     "ksana_sage_attn_fwd_masked",
     "ksana_sage_attn_fwd_varlen",
     "ksana_sage_forward_masked",
+    "ksana_sage_forward_varlen",
 )
 
 
@@ -144,6 +145,10 @@ def _declare(lib):
     lib.ksana_sage_attn_fwd_varlen.restype = i
     lib.ksana_sage_forward_masked.argtypes = [vp, vp, vp, vp, i, st, st, st, st, sp, vp, ms, vp, f, i, i, i, vp, vp]
     lib.ksana_sage_forward_masked.restype = i
+    # (structures by address: a caller that keeps them from call to call hands over plain integers, which ctypes
+    # converts in a fraction of the time its pointer objects take)
+    lib.ksana_sage_forward_varlen.argtypes = [vp, vp, vp, vp, i, i, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, f, i, i, i, vp, vp]
+    lib.ksana_sage_forward_varlen.restype = i
 
 
 def library_present() -> bool:

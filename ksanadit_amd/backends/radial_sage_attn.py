@@ -81,9 +81,10 @@ class RadialSageAttentionImpl(KsanaAttentionBackendImpl):
                 latent_shape: list[int] | None = None, **kwargs) -> torch.Tensor:
         if dense_only or step_iter < self.dense_attn_steps or block_id < self.dense_blocks_num:
             return self.dense_attn(query, key, value, **kwargs)
-        if k_lens is None or not bool((k_lens == k_lens[0]).all()):
+        lens = [] if k_lens is None else k_lens.tolist()  # (one copy to the host when it lives on the GPU)
+        if not lens or any(n != lens[0] for n in lens):
             raise ValueError("k_lens must be the same for all tokens")
-        video_token_num = int(k_lens[0])
+        video_token_num = int(lens[0])
         _, _, num_frame, l_h, l_w = latent_shape
         if l_h % (self.block_size // 8) != 0 or l_w % (self.block_size // 8) != 0:
             raise ValueError(f"output's width and height must be divisible by block size {self.block_size}")

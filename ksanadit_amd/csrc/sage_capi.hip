@@ -194,9 +194,9 @@ int check_causal(const ksana_sage_shape* s, int causal) {
   return 0;
 }
 
-int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype, const int64_t q_st[4],
+int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype, int o_dtype, const int64_t q_st[4],
                  const int64_t k_st[4], const int64_t v_st[4], const int64_t o_st[4], const ksana_sage_shape* s,
-                 const ksana_sage_prep* prep, const int8_t* block_mask, const int64_t mask_st[2],
+                 const ksana_sage_prep* prep, const int8_t* block_mask, const int64_t mask_st[2], const int32_t* q_lens,
                  const int32_t* k_lens, float sm_scale, int smooth_k, int causal, int flags, void* ws, void* stream);
 
 // Validates `prep` for one tensor (`weight` is that tensor's norm weight) and fills the kernel-side
@@ -730,8 +730,8 @@ int ksana_sage_forward_prep(const void* q, const void* k, const void* v, void* o
                             const int64_t k_st[4], const int64_t v_st[4], const int64_t o_st[4],
                             const ksana_sage_shape* s, const ksana_sage_prep* prep, const int32_t* k_lens,
                             float sm_scale, int smooth_k, int causal, int flags, void* ws, void* stream) {
-  return forward_impl(q, k, v, o, dtype, q_st, k_st, v_st, o_st, s, prep, nullptr, nullptr, k_lens, sm_scale, smooth_k,
-                      causal, flags, ws, stream);
+  return forward_impl(q, k, v, o, dtype, dtype, q_st, k_st, v_st, o_st, s, prep, nullptr, nullptr, nullptr, k_lens, sm_scale,
+                      smooth_k, causal, flags, ws, stream);
 }
 
 int ksana_sage_forward_masked(const void* q, const void* k, const void* v, void* o, int dtype, const int64_t q_st[4],
@@ -739,7 +739,17 @@ int ksana_sage_forward_masked(const void* q, const void* k, const void* v, void*
                               const ksana_sage_shape* s, const int8_t* block_mask, const int64_t mask_st[2],
                               const int32_t* k_lens, float sm_scale, int smooth_k, int causal, int flags, void* ws,
                               void* stream) {
-  return forward_impl(q, k, v, o, dtype, q_st, k_st, v_st, o_st, s, nullptr, block_mask, mask_st, k_lens, sm_scale,
+  return forward_impl(q, k, v, o, dtype, dtype, q_st, k_st, v_st, o_st, s, nullptr, block_mask, mask_st, nullptr, k_lens, sm_scale,
+                      smooth_k, causal, flags, ws, stream);
+}
+
+int ksana_sage_forward_varlen(const void* q, const void* k, const void* v, void* o, int dtype, int o_dtype,
+                              const int64_t q_st[4], const int64_t k_st[4], const int64_t v_st[4],
+                              const int64_t o_st[4], const ksana_sage_shape* s, const ksana_sage_prep* prep,
+                              const int8_t* block_mask, const int64_t mask_st[2], const int32_t* q_lens,
+                              const int32_t* k_lens, float sm_scale, int smooth_k, int causal, int flags, void* ws,
+                              void* stream) {
+  return forward_impl(q, k, v, o, dtype, o_dtype, q_st, k_st, v_st, o_st, s, prep, block_mask, mask_st, q_lens, k_lens, sm_scale,
                       smooth_k, causal, flags, ws, stream);
 }
 
@@ -781,9 +791,9 @@ int quant_qkv(const void* q, const void* k, const void* v, int dtype, const int6
   return ksana_sage_quant_v_smooth(v, dtype, v_st, s, smooth_v, ws, stream);
 }
 
-int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype, const int64_t q_st[4],
+int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype, int o_dtype, const int64_t q_st[4],
                  const int64_t k_st[4], const int64_t v_st[4], const int64_t o_st[4], const ksana_sage_shape* s,
-                 const ksana_sage_prep* prep, const int8_t* block_mask, const int64_t mask_st[2],
+                 const ksana_sage_prep* prep, const int8_t* block_mask, const int64_t mask_st[2], const int32_t* q_lens,
                  const int32_t* k_lens, float sm_scale, int smooth_k, int causal, int flags, void* ws, void* stream) {
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_mask(s, block_mask, mask_st)) return rc;
@@ -792,12 +802,15 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
   if (int rc = check_tensor("q", q, dtype, q_st, s->B, s->Lq, s->Hq)) return rc;
   if (int rc = check_tensor("k", k, dtype, k_st, s->B, s->Lk, s->Hkv)) return rc;
   if (int rc = check_tensor("v", v, dtype, v_st, s->B, s->Lk, s->Hkv)) return rc;
-  if (int rc = check_tensor("o", o, dtype, o_st, s->B, s->Lq, s->Hq)) return rc;
+  if (int rc = check_tensor("o", o, o_dtype, o_st, s->B, s->Lq, s->Hq)) return rc;
   if (int rc = check_ws(ws)) return rc;
   if (flags & ~(KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_SMOOTH_V | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES |
                 KSANA_SAGE_FLAG_TILE_SKIP))
     return fail(KSANA_SAGE_EINVAL, "unknown flag bits 0x%x", flags);
+  if ((flags & KSANA_SAGE_FLAG_TILE_SKIP) && (flags & KSANA_SAGE_FLAG_PWL_EXP2))
+    return fail(KSANA_SAGE_EINVAL, "KSANA_SAGE_FLAG_TILE_SKIP goes with the exact exponential only, not with KSANA_SAGE_FLAG_PWL_EXP2");
   if (reinterpret_cast<uintptr_t>(k_lens) & 3) return fail(KSANA_SAGE_EINVAL, "k_lens is not 4-byte aligned");
+  if (reinterpret_cast<uintptr_t>(q_lens) & 3) return fail(KSANA_SAGE_EINVAL, "q_lens is not 4-byte aligned");
   {
     ksana_sage::PrepParams pp;
     const ksana_sage::PrepParams* ppp = nullptr;
@@ -809,7 +822,7 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
   }
   if (int rc = quant_qkv(q, k, v, dtype, q_st, k_st, v_st, s, prep, sm_scale, smooth_k, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws, stream))
     return rc;
-  return ksana_sage_attn_fwd_masked(ws, o, dtype, o_st, s, block_mask, mask_st, k_lens, causal,
+  return ksana_sage_attn_fwd_varlen(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal,
                                     flags & ~KSANA_SAGE_FLAG_SMOOTH_V, stream);
 }
 }  // namespace

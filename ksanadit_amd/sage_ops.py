@@ -74,8 +74,10 @@ def _prep_operand(t: torch.Tensor, device, dtype) -> torch.Tensor:
     return conv
 
 
-def _stream_ptr(device) -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream_ptr(device) -> int:
+    """torch's current stream on ``device`` as the library takes it (the raw handle: building a ``torch.cuda.Stream``
+    around it first costs 2 us a call)."""
+    return torch._C._cuda_getCurrentRawStream(device.index if device.index is not None else torch.cuda.current_device())
 
 
 def _require_hip(*tensors: torch.Tensor) -> None:
@@ -533,7 +535,7 @@ _demotion_logged = False
 def _log_demotion_once() -> None:
     """Debug aid of the op path: say once that the library fell back to its two-pass quantizers on this GPU."""
     global _demotion_logged
-    if _demotion_logged or not log.isEnabledFor(10):  # logging.DEBUG
+    if _demotion_logged:
         return
     if one_read_state()["demoted"]:
         _demotion_logged = True
@@ -620,6 +622,57 @@ def attn_fwd(ws: SageWorkspace, out: torch.Tensor, causal: bool = False, pwl_exp
     return out
 
 
+class _CallPlan:
+    """What ``sageattn`` works out from the shapes, strides, dtypes and devices of q, k, v: whether the kernels can take
+    them, the C structures the library reads and the workspace's size.  A model repeats a handful of shapes thousands of
+    times; worked out anew in every call this was half of a small call's host time (25 us at B=2 L=32 H=64, 14 with it)."""
+
+    __slots__ = ("runs", "out_shape", "device", "dtype", "dtype_code", "shape", "shape_ptr", "ws_bytes", "q_st", "k_st", "v_st", "o_st",
+                 "_strides")
+
+    def __init__(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor):
+        """``q``, ``k``, ``v``: ``[B, L, H, D]`` as the kernels will read them."""
+        self.out_shape, self.device, self.dtype, self.dtype_code = tuple(q.shape), q.device, q.dtype, _DTYPES[q.dtype]
+        self.runs = q.numel() != 0
+        if not self.runs:
+            return
+        B, Lq, Hq, D = q.shape
+        self.shape, layout = _capi.workspace_layout(B, Hq, k.shape[2], Lq, k.shape[1], D)
+        self.shape_ptr, self.ws_bytes = C.addressof(self.shape), layout.total_bytes
+        out_strides = (Lq * Hq * D, Hq * D, D, 1)
+        self._strides = [_strides(q), _strides(k), _strides(v), _capi.Strides(*out_strides)]  # (kept alive: addresses below)
+        self.q_st, self.k_st, self.v_st, self.o_st = (C.addressof(x) for x in self._strides)
+
+
+# Bounded: a full table is started over (the plans are cheap, a few hundred bytes each).  One dict operation per call,
+# so threads need no lock; two that meet a new shape at the same time both work it out.
+_plans: dict = {}
+_MAX_PLANS = 512
+
+
+def _make_plan(q, k, v, tensor_layout: str, with_prep: bool, key):
+    """Checks q, k, v, makes those the kernels cannot read contiguous, and returns ``[B, L, H, D]`` tensors with their plan -
+    remembered under ``key`` when nothing had to be copied."""
+    if tensor_layout not in ("NHD", "HND"):
+        raise ValueError(f"tensor_layout {tensor_layout!r} unknown")
+    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
+        raise ValueError("sageattn expects 4-D tensors")
+    if tensor_layout == "HND":
+        if with_prep:
+            raise ValueError("prep needs the NHD layout (a token row must be contiguous)")
+        q, k, v = (t.transpose(1, 2) for t in (q, k, v))
+    _require_hip(q, k, v)
+    if k.shape != v.shape or q.shape[0] != k.shape[0] or q.shape[3] != k.shape[3]:
+        raise ValueError(f"incompatible shapes q{tuple(q.shape)} k{tuple(k.shape)} v{tuple(v.shape)}")
+    usable = [_usable(t) for t in (q, k, v)]
+    plan = _CallPlan(*usable)
+    if all(a is b for a, b in zip(usable, (q, k, v))):
+        if len(_plans) >= _MAX_PLANS:
+            _plans.clear()
+        _plans[key] = plan
+    return (*usable, plan)
+
+
 def sageattn(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -658,65 +711,56 @@ def sageattn(
     ``tile_skip=True`` (exact exponential only): see ``attn_fwd``; same bits, faster on sharply peaked attention."""
     if tile_skip and pwl_exp2:
         raise ValueError("tile_skip goes with the exact exponential only")
-    if tensor_layout not in ("NHD", "HND"):
-        raise ValueError(f"tensor_layout {tensor_layout!r} unknown")
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
-        raise ValueError("sageattn expects 4-D tensors")
-    if tensor_layout == "HND":
-        if prep is not None:
-            raise ValueError("prep needs the NHD layout (a token row must be contiguous)")
-        q, k, v = (t.transpose(1, 2) for t in (q, k, v))
-    _require_hip(q, k, v)
-    if k.shape != v.shape or q.shape[0] != k.shape[0] or q.shape[3] != k.shape[3]:
-        raise ValueError(f"incompatible shapes q{tuple(q.shape)} k{tuple(k.shape)} v{tuple(v.shape)}")
-    q, k, v = _usable(q), _usable(k), _usable(v)
-    B, Lq, Hq, D = q.shape
-    if q.numel() == 0:  # nothing to attend from: same empty result SDPA gives
-        out = torch.empty((B, Lq, Hq, D), dtype=q.dtype, device=q.device)
-        return out.transpose(1, 2) if tensor_layout == "HND" else out
-    sm_scale = D**-0.5 if sm_scale is None else float(sm_scale)
-    ws = workspace_for(q, k) if workspace is None else workspace
-    ws.require(q.device, B=B, Hq=Hq, Hkv=k.shape[2], Lq=Lq, Lk=k.shape[1], D=D)
-    lib = _capi.load()
-    _log_demotion_once()
-    kl = _k_lens_arg(k_lens, B, q.device)
-    flags = (_capi.FLAG_PWL_EXP2 if pwl_exp2 else 0) | (_capi.FLAG_SMOOTH_V if smooth_v else 0)
-    flags |= _capi.FLAG_TILE_SKIP if tile_skip else 0
-    if prep is not None:
-        _check_qwen_rows(prep, Lq)
-        _check_qwen_rows(prep, k.shape[1])
-    result_dtype = q.dtype if out_dtype is None else out_dtype
+    key = (q.shape, q.stride(), k.shape, k.stride(), v.shape, v.stride(), q.dtype, k.dtype, v.dtype,
+           q.get_device(), k.get_device(), v.get_device(), tensor_layout)
+    plan = _plans.get(key)
+    q_ptr, k_ptr, v_ptr = q.data_ptr(), k.data_ptr(), v.data_ptr()
+    if plan is None or (q_ptr | k_ptr | v_ptr) & 15:
+        q, k, v, plan = _make_plan(q, k, v, tensor_layout, prep is not None, key)
+        q_ptr, k_ptr, v_ptr = q.data_ptr(), k.data_ptr(), v.data_ptr()
+    hnd = tensor_layout == "HND"
+    if hnd and prep is not None:
+        raise ValueError("prep needs the NHD layout (a token row must be contiguous)")
+    B, Lq, Hq, D = plan.out_shape
+    device = plan.device
+    result_dtype = plan.dtype if out_dtype is None else out_dtype
     if result_dtype not in _DTYPES:
         raise ValueError(f"out_dtype must be float16 or bfloat16, got {out_dtype}")
-    out = torch.empty((B, Lq, Hq, D), dtype=result_dtype, device=q.device)
-    if q_lens is not None or result_dtype != q.dtype:
-        # the one-call entry points take neither q_lens nor a result dtype of their own: quantize (the quantized
-        # operands carry no dtype), then the attention entry point that takes both
-        quant_qk(q, k, ws, sm_scale, smooth_k, prep=prep)
-        quant_v(v, ws, smooth_v)
-        attn_fwd(ws, out, causal=is_causal, pwl_exp2=pwl_exp2, k_lens=kl, block_mask=block_mask, q_lens=q_lens)
-        return out.transpose(1, 2) if tensor_layout == "HND" else out
-    if block_mask is not None:
-        if prep is not None:
+    out = torch.empty(plan.out_shape, dtype=result_dtype, device=device)
+    if not plan.runs:  # nothing to attend from: same empty result SDPA gives
+        return out.transpose(1, 2) if hnd else out
+    sm_scale = D**-0.5 if sm_scale is None else float(sm_scale)
+    if workspace is None:
+        blob = torch.empty(plan.ws_bytes, dtype=torch.uint8, device=device)  # (torch's blocks start at multiples of 512)
+    else:
+        s = plan.shape
+        workspace.require(device, B=s.B, Hq=s.Hq, Hkv=s.Hkv, Lq=s.Lq, Lk=s.Lk, D=s.D)
+        blob = workspace.blob
+    lib = _capi.load()
+    if log.isEnabledFor(10):  # logging.DEBUG
+        _log_demotion_once()
+    kl = None if k_lens is None else _k_lens_arg(k_lens, B, device)
+    ql = None if q_lens is None else _k_lens_arg(q_lens, B, device, "q_lens")
+    flags = (_capi.FLAG_PWL_EXP2 if pwl_exp2 else 0) | (_capi.FLAG_SMOOTH_V if smooth_v else 0)
+    flags |= _capi.FLAG_TILE_SKIP if tile_skip else 0
+    prep_ptr = mask_ptr = mask_st = None
+    if prep is not None:
+        if block_mask is not None and q_lens is None and result_dtype == plan.dtype:
             raise ValueError("block_mask and prep cannot be combined in one call; quantize with prep, then attn_fwd")
-        mask, mask_st = _block_mask_arg(block_mask, B, Hq, Lq, k.shape[1], q.device)
-        rc = lib.ksana_sage_forward_masked(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _DTYPES[q.dtype],
-            _strides(q), _strides(k), _strides(v), _strides(out), C.byref(ws.shape), mask.data_ptr(), mask_st,
-            None if kl is None else kl.data_ptr(), sm_scale, int(smooth_k), int(is_causal), flags, ws.ptr,
-            _stream_ptr(q.device),
-        )
-        _capi.check(rc, "ksana_sage_forward_masked")
-        return out.transpose(1, 2) if tensor_layout == "HND" else out
-    c_prep, _keep = (None, None) if prep is None else prep.to_c(q.device)
-    rc = lib.ksana_sage_forward_prep(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _DTYPES[q.dtype],
-        _strides(q), _strides(k), _strides(v), _strides(out), C.byref(ws.shape),
-        None if c_prep is None else C.byref(c_prep), None if kl is None else kl.data_ptr(), sm_scale, int(smooth_k),
-        int(is_causal), flags, ws.ptr, _stream_ptr(q.device),
-    )
-    _capi.check(rc, "ksana_sage_forward_prep" if prep is not None else "ksana_sage_forward")
-    return out.transpose(1, 2) if tensor_layout == "HND" else out
+        _check_qwen_rows(prep, Lq)
+        _check_qwen_rows(prep, plan.shape.Lk)
+        c_prep, _keep = prep.to_c(device)
+        prep_ptr = C.addressof(c_prep)
+    if block_mask is not None:
+        mask, mask_st = _block_mask_arg(block_mask, B, Hq, Lq, plan.shape.Lk, device)
+        mask_ptr = mask.data_ptr()
+    rc = lib.ksana_sage_forward_varlen(
+        q_ptr, k_ptr, v_ptr, out.data_ptr(), plan.dtype_code, _DTYPES[result_dtype], plan.q_st, plan.k_st, plan.v_st, plan.o_st,
+        plan.shape_ptr, prep_ptr, mask_ptr, mask_st, None if ql is None else ql.data_ptr(), None if kl is None else kl.data_ptr(),
+        sm_scale, int(smooth_k), int(is_causal), flags, blob.data_ptr(), _stream_ptr(device))
+    if rc != _capi.OK:
+        _capi.check(rc, "ksana_sage_forward")
+    return out.transpose(1, 2) if hnd else out
 
 
 def wan_self_attention(q_proj: torch.Tensor, k_proj: torch.Tensor, v_proj: torch.Tensor, num_heads: int,
