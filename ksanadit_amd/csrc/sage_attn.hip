@@ -104,6 +104,16 @@ __device__ __forceinline__ void lds_copy16(const void* gbase, unsigned lane_off,
                : "s"(lds_off), "v"(lane_off), "s"(gbase)
                : "memory", "m0");
 }
+// The same through a buffer descriptor: 16 bytes per lane from (base + src_off + lane_off) to `lds_base + kSlot`.  One scalar
+// offset serves every buffer whose tiles have the same number, and a slot known at compile time rides in the
+// instruction that writes M0 - two scalar instructions per copy where the 64-bit form above takes six.
+template <int kSlot>
+__device__ __forceinline__ void lds_copy16_at(const v4i& buffer, unsigned lane_off, unsigned src_off, unsigned lds_base) {
+  asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
+               :
+               : "s"(lds_base), "n"(kSlot), "v"(lane_off), "s"(buffer), "s"(src_off)
+               : "memory", "m0", "scc");
+}
 #pragma clang diagnostic pop
 
 // Opaque use+def at this program point: keeps the optimizer from sinking the computation of
@@ -172,6 +182,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   constexpr int kListMax = kW == 8 ? kSparseMaxKeyTiles : kSparseMaxKeyTiles4;
   static_assert(!(kTileSkip && kPwlExp), "the piecewise-linear code formula has its own zero point: no tiles are skipped there");
   static_assert(kG == 4 || kG == 2, "128 channels, or 64 zero-extended");
+  constexpr bool kUnrolled = !kPwlExp && !kTileSkip;  // the variants calls take by default
   constexpr int kMagicBits = kG == 4 ? kMagicI : kMagicI2;
   constexpr float kMagicVal = kG == 4 ? kMagicF : kMagicF2;
   int wg, split = 0;
@@ -495,6 +506,38 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
     for (int i = 0; i < kWindow; ++i) ahead[i] = tile_of(min(kAhead + i, n_tiles - 1));
   }
+  // The key loop's own copies: descriptors over this workgroup's tiles, the lane's offset in a tile, the offset of the
+  // tiles the next copies take (past the last tile it stays there, as above)
+  auto tiles_from = [&](const void* base) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32) & 0xffff, (p.nkb - tile0) * kTileBytes, 0x00020000};
+  };
+  const v4i k_buf = tiles_from(k_src), v_buf = tiles_from(v_src);
+  const unsigned lane_off = (unsigned)(wave * 64 + lane) * 16;
+  const unsigned lds_base = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)smem + (unsigned)wave * 1024;
+  const int off_last = (n_tiles - 1) * kTileBytes;
+  int off_v = min(kAhead, n_tiles - 1) * kTileBytes, off_k = min(Shape::kAheadK, n_tiles - 1) * kTileBytes;
+  auto copy_to = [&](auto slot, const v4i& buffer, int off) {
+    constexpr int kSlot = decltype(slot)::value;
+    lds_copy16_at<kSlot>(buffer, lane_off, off, lds_base);
+    if constexpr (kW == 4) lds_copy16_at<kSlot + 4096>(buffer, lane_off + 4096, off, lds_base);
+  };
+  // the copies of loop step j at ring position kAt (= j modulo kStages)
+  auto issue_copy_at = [&](auto at) {
+    constexpr int kAt = decltype(at)::value;
+    constexpr int kVs = (kAt + kAhead) & (kStages - 1), kKs = (kAt + Shape::kAheadK) & (kStages - 1);
+    using VSlot = std::integral_constant<int, Shape::kTwoRings ? (kStages + kVs) * kTileBytes : kVs * kStageBytes + kTileBytes>;
+    using KSlot = std::integral_constant<int, Shape::kTwoRings ? kKs * kTileBytes : kKs * kStageBytes>;
+    if constexpr (kSparse) {
+      copy_to(VSlot{}, v_buf, ahead[0] * kTileBytes);
+      copy_to(KSlot{}, k_buf, ahead[kWindow - 1] * kTileBytes);
+    } else {
+      copy_to(VSlot{}, v_buf, off_v);  // first: it is awaited first
+      copy_to(KSlot{}, k_buf, kAhead == Shape::kAheadK ? off_v : off_k);
+      off_v = min(off_v + kTileBytes, off_last);
+      off_k = min(off_k + kTileBytes, off_last);
+    }
+  };
   // the copies of loop step j (step -1: nothing; the prologue below brings the first tiles in)
   auto issue_copy = [&](int j) {
     if constexpr (kSparse) {
@@ -636,19 +679,22 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // With the 16x16 row sums, same bits: 10.60 -> 10.35 ms at B=1 H=40 L=32760 with outliers, 11.44 -> 11.05 without
   // (2045 cycles per step, from 2073; the chip runs at its power limit there, and fewer operations raise its clock too).
   float sc = 0.0f, xc = 0.0f;           // scale of the coming tile, its exponent constant
-  float alpha_next = 1.0f;              // factor the coming tile's point move puts on everything before it
-  bool moved_next = false;              // (wave-uniform) whether it is other than 1
+  // factor a tile's point move puts on everything before it, and (wave-uniform) whether there is one: of even tiles and
+  // of odd ones (step j applies tile j-1's and then finds tile j+1's)
+  float alpha_even = 1.0f, alpha_odd = 1.0f;
+  int moved_even = 0, moved_odd = 0;
   bool nothing = false;                 // (wave-uniform) every probability of the coming tile converts to zero
-  auto look_ahead = [&](int jn, int mx, float ks) {
+  auto look_ahead = [&](int jn, int mx, float ks, float& alpha, int& moved) {
     sc = qs * ks;
     const float mneg = -kMagicVal * sc;
     const float m_half = __builtin_fmaf(__int_as_float(mx), sc, mneg);
-    moved_next = false;
-    if (__any(m_half > x_limit)) {
+    moved = 0;
+    if (__ballot(m_half > x_limit) != 0) {
+      asm volatile("");  // (two branches on purpose: merged into one condition, the second is computed in every step)
       // (a tile this wave's mask row does not ask for, or that is not this loop's, leaves the points alone)
       if (jn < n_main && mine_at(jn)) {
-        alpha_next = move_point(mx, sc, mneg);
-        moved_next = true;
+        alpha = move_point(mx, sc, mneg);
+        moved = 1;
       }
     }
     // exponent of key r: x = sc*dot - m_run + shift, with the magic folded into the constant
@@ -662,8 +708,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     // pvthreshold idea of the reference's sparse kernel (sage_sla.py:237-253) with a threshold at which nothing changes.
     if constexpr (kTileSkip) nothing = __all(m_half < m_run - (kPShift + 11.0f));
   };
-  look_ahead(0, lane_max(s_a), s_ks[0]);
-  moved_next = false;  // nothing has been accumulated yet
+  look_ahead(0, lane_max(s_a), s_ks[0], alpha_even, moved_even);
+  moved_even = 0;  // nothing has been accumulated yet
 
   // Software pipeline, one key tile per step.  While this tile's probabilities are computed on
   // the VALU, the matrix pipe runs the S^T MFMAs of the NEXT tile and the PV MFMAs of the
@@ -671,16 +717,20 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // requested three MFMAs ahead, and sched_barrier pins that order.  The max reduction of the
   // next tile rides in the PV chunks.
   // Because PV lags one tile, so does the rescaling of O:
-  //   at step j   O holds tiles <= j-2 relative to point m(j-2); alpha = 2^(m(j-2) - m(j-1)), alpha_next = 2^(m(j-1) - m(j))
+  //   at step j   O holds tiles <= j-2 relative to point m(j-2); alpha = 2^(m(j-2) - m(j-1)), tile j-1's
   //   step j      O *= alpha (rare branch), then O += P(j-1) V(j-1), both relative to m(j-1)
   // LDS ring of 8 stages: tile j-1 (V), j (V next step), j+1 (K), j+2 .. j+4 (arriving).
   // probabilities of the previous and of the current tile swap registers every step, like s_a / s_b
   v8i pf_x = {0, 0, 0, 0, 0, 0, 0, 0}, pf_y = {0, 0, 0, 0, 0, 0, 0, 0};
-  float alpha = 1.0f;
-  bool moved = false;
-  auto tile_step = [&](int j, v16i (&s_cur)[2], v16i (&s_nxt)[2], const v8i& pf_prev, v8i& pf) {
-    const uint8_t* kst = k_slot(j + 1);
-    const uint8_t* vst = v_slot(j - 1);
+  // `at`: the step's position in the tile ring (j modulo kStages) where the loop is unrolled over the ring, so that every
+  // LDS address is a constant; -1 in the loop over what remains.
+  // byte offset into LDS of the next tile's K scale (a vector register on purpose: as a scalar it is moved to one at every use)
+  int ks_off = (int)(reinterpret_cast<const uint8_t*>(s_ks) - smem) + 4;
+  pin(ks_off);
+  auto tile_step = [&](auto at, int j, v16i (&s_cur)[2], v16i (&s_nxt)[2], const v8i& pf_prev, v8i& pf, float& alpha, int& moved) {
+    constexpr int kAt = decltype(at)::value;
+    const uint8_t* kst = k_slot(kAt >= 0 ? kAt + 1 : j + 1);
+    const uint8_t* vst = v_slot(kAt >= 0 ? kAt - 1 : j - 1);
     auto k_frag = [&](int i) { return *reinterpret_cast<const v4i*>(kst + (((i & 1) * 4 + (i >> 1)) * 64 + lane) * 16); };
     auto v_frag = [&](int dt) {
       const v4i lo = *reinterpret_cast<const v4i*>(vst + ((dt * 2 + 0) * 64 + lane) * 16);
@@ -693,13 +743,14 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     kf[0] = k_frag(0);
     kf[1] = k_frag(1);
     kf[2] = k_frag(2);  // (kG >= 2: chunks 0 .. 3 always exist)
-    const float ks_nxt = s_ks[min(j + 1, n_tiles - 1)];
+    // (one past the last tile's reads whatever follows the scales in LDS: a value nothing uses)
+    const float ks_nxt = *reinterpret_cast<const float*>(smem + ks_off + (kAt >= 0 ? 4 * kAt : 0));
+    if constexpr (kAt < 0) ks_off += 4;
     int entering = 0;  // the list entry the next step's window gains; it arrives with the operands above
     if constexpr (kSparse) entering = s_list[min(j + 1 + Shape::kAheadK, n_tiles - 1)];
-    issue_copy(j);
-    if (moved) scale_o(alpha);  // wave-uniform
-    alpha = alpha_next;
-    moved = moved_next;
+    if constexpr (kAt >= 0) issue_copy_at(at);
+    else issue_copy(j);
+    if (moved != 0) scale_o(alpha);  // wave-uniform
     // row sums of tile j-1: they cover the latency of the operands just requested
     lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_prev, lacc, 0, 0, 0, 0, 0, 0);
     const float scp = kPwlExp ? 8.0f * sc : sc;
@@ -775,18 +826,35 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       }
       if (diag_at(j)) causal_probs(pf);
     }
-    look_ahead(j + 1, mx, ks_nxt);
+    look_ahead(j + 1, mx, ks_nxt, alpha, moved);
     // after this barrier: tile j+2 is visible to every wave, and nobody reads tile j-1 any more
     tile_barrier();
   };
 
   {
     int j = 0;
-    for (; j + 2 <= n_main; j += 2) {
-      tile_step(j, s_a, s_b, pf_x, pf_y);
-      tile_step(j + 1, s_b, s_a, pf_y, pf_x);
+    using Anywhere = std::integral_constant<int, -1>;
+    if constexpr (kUnrolled) {
+      auto two = [&](auto at) {
+        constexpr int kAt = decltype(at)::value;
+        tile_step(std::integral_constant<int, kAt>{}, j + kAt, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
+        tile_step(std::integral_constant<int, kAt + 1>{}, j + kAt + 1, s_b, s_a, pf_y, pf_x, alpha_even, moved_even);
+      };
+      for (; j + kStages <= n_main; j += kStages) {
+        two(std::integral_constant<int, 0>{});
+        two(std::integral_constant<int, 2>{});
+        if constexpr (kStages == 8) {
+          two(std::integral_constant<int, 4>{});
+          two(std::integral_constant<int, 6>{});
+        }
+        ks_off += 4 * kStages;
+      }
     }
-    if (j < n_main) tile_step(j, s_a, s_b, pf_x, pf_y);
+    for (; j + 2 <= n_main; j += 2) {
+      tile_step(Anywhere{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
+      tile_step(Anywhere{}, j + 1, s_b, s_a, pf_y, pf_x, alpha_even, moved_even);
+    }
+    if (j < n_main) tile_step(Anywhere{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may outlive the workgroup's LDS
   if constexpr (Shape::kTwoRings) {
@@ -795,7 +863,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if (has_tail) __builtin_amdgcn_s_barrier();
   }
   if (n_main > 0) {  // drain: PV of the last pipelined tile
-    if (moved) scale_o(alpha);
+    if ((n_main & 1) != 0) {
+      if (moved_even != 0) scale_o(alpha_even);
+    } else {
+      if (moved_odd != 0) scale_o(alpha_odd);
+    }
     const uint8_t* vst = v_slot(n_main - 1);
     const v8i pf_last = (n_main & 1) ? pf_y : pf_x;  // written by the last step
 #pragma unroll
@@ -952,7 +1024,7 @@ __global__ __launch_bounds__(256) void sage_attn_merge_kernel(const AttnParams p
 template <bool kSparse, int kW>
 constexpr size_t max_lds() {
   return kSparse ? WgShape<kW>::kRingBytes + 1024 + (kW == 8 ? kSparseMaxKeyTiles * 8 : kSparseMaxKeyTiles4 * 6) + 1024
-                 : WgShape<kW>::kRingBytes + 1024 + (kW == 8 ? kMaxKeyTiles : kShortMaxKeyTiles) * 4;
+                 : WgShape<kW>::kRingBytes + 2048 + (kW == 8 ? kMaxKeyTiles : kShortMaxKeyTiles) * 4;
 }
 
 template <int DT, bool kPwlExp, bool kSparse, bool kSplit, int kW, bool kCausal, bool kTileSkip = false, int kG = 4>
@@ -1070,7 +1142,7 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
     if (sparse)
       return p.causal ? launch_shape<true, false, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
                       : launch_shape<true, false, 4, false>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s);
-    const size_t lds = WgShape<4>::kRingBytes + 1024 + (((size_t)p.nkb * 4 + 1023) & ~size_t(1023));
+    const size_t lds = WgShape<4>::kRingBytes + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
     return launch_shape<false, false, 4>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
   }
   const int n_qwg = (p.Lq + kAttnQPerWg - 1) / kAttnQPerWg;
@@ -1080,7 +1152,7 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   // (tile lists in 256-row workgroups, by flag only: one instantiation serves causal and plain calls)
   if (sparse) return launch_shape<true, false, 8, true>(p, grid, max_lds<true, 8>(), n_qwg, n_wg, wg_per_xcd, s);
   // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
-  const size_t lds = WgShape<8>::kRingBytes + 1024 + (((size_t)p.nkb * 4 + 1023) & ~size_t(1023));
+  const size_t lds = WgShape<8>::kRingBytes + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
   // The workgroups beyond the last full round of the chip (one workgroup per compute unit) would hold it for a
   // whole round alone.  When they are few, each is cut into runs of key tiles that together fill a round, and a
   // small kernel merges the runs: 2568 workgroups are then 10 rounds and a bit instead of 11, 280 are 1.1 instead of 2.
