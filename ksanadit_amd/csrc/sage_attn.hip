@@ -45,7 +45,7 @@ struct WgShape {
   static constexpr int kThreads = kW * 64;
   static constexpr int kRows = kW * 32;                // query rows per workgroup
   static constexpr int kStages = kW == 8 ? 8 : 4;      // LDS ring (power of two): tiles j-1 .. j+kAhead live at step j
-  static constexpr int kAhead = kW == 8 ? 4 : 2;       // global -> LDS copies are issued this many tiles ahead
+  static constexpr int kAhead = kW == 8 ? 5 : 2;       // global -> LDS copies are issued this many tiles ahead
   static constexpr int kCopies = 2 * (8 / kW);         // 1 KiB copy instructions per wave and tile (K and V^T halves)
   static constexpr int kRingBytes = kStages * 2 * kTileBytes;
   // The 4-wave shape keeps K tiles and V^T tiles in two rings of kStages slots each (same memory).  A K tile is
@@ -58,6 +58,12 @@ struct WgShape {
   // copies that may still be in flight at the barrier that ends a step: those of the newest (kAhead - 2) tiles in
   // one ring; with two rings everything issued in this step and the one before
   static constexpr int kInFlight = kTwoRings ? 2 * kCopies : kCopies * (kAhead - 2);
+  // The eight-stage ring has room for waves a step apart: in the loop that is unrolled over it the waves meet after
+  // every second step only (a step j and its successor read tiles j-1 .. j+2 and bring in j+5 and j+6, whose slots held
+  // j-3 and j-2), so a wave that rescales its rows holds up the others half as often: 2616 -> 2571 us at 40 heads of
+  // 16384 tokens, 2477 -> 2446 with outliers.  What may be in flight there is what the two steps have issued.
+  static constexpr bool kPairs = kW == 8;
+  static constexpr int kInFlightPairs = 2 * kCopies;
 };
 constexpr int kMagicI = 0x4B400000;       // bits of 12582912.0f = 1.5 * 2^23: fp32 values are 1 apart there
 constexpr float kMagicF = 12582912.0f;
@@ -553,6 +559,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   auto tile_barrier = [&]() {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(Shape::kInFlight) : "memory");
   };
+  // the same after the second step of a pair (Shape::kPairs); steps [0, n_paired) run in pairs
+  auto pair_barrier = [&]() {
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(Shape::kInFlightPairs) : "memory");
+  };
+  const int n_paired = kUnrolled && Shape::kPairs ? n_main / kStages * kStages : 0;
 
   // The compiler does not see the asynchronous copies in the memory-operation counter it models.  Every ordinary global
   // load of the set-up (Q fragments, scales) must therefore be known to have returned before the key loop starts:
@@ -586,7 +597,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       // (looks the tiles up where they are needed: a wave without rows has nothing an LDS wait could hold up)
       copy_half(v_src, j + kAhead, v_slot(j + kAhead));
       copy_half(k_src, j + Shape::kAheadK, k_slot(j + Shape::kAheadK));
-      tile_barrier();
+      if (j >= n_paired) tile_barrier();
+      else if ((j & 1) != 0) pair_barrier();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if constexpr (!kSplit) write_zero_rows();  // rows in [lq, Lq), if any (the merge kernel writes them for cut blocks)
@@ -719,7 +731,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // Because PV lags one tile, so does the rescaling of O:
   //   at step j   O holds tiles <= j-2 relative to point m(j-2); alpha = 2^(m(j-2) - m(j-1)), tile j-1's
   //   step j      O *= alpha (rare branch), then O += P(j-1) V(j-1), both relative to m(j-1)
-  // LDS ring of 8 stages: tile j-1 (V), j (V next step), j+1 (K), j+2 .. j+4 (arriving).
+  // LDS ring of 8 stages: tile j-1 (V), j (V next step), j+1 (K), j+2 .. j+5 (arriving).
   // probabilities of the previous and of the current tile swap registers every step, like s_a / s_b
   v8i pf_x = {0, 0, 0, 0, 0, 0, 0, 0}, pf_y = {0, 0, 0, 0, 0, 0, 0, 0};
   // `at`: the step's position in the tile ring (j modulo kStages) where the loop is unrolled over the ring, so that every
@@ -748,8 +760,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if constexpr (kAt < 0) ks_off += 4;
     int entering = 0;  // the list entry the next step's window gains; it arrives with the operands above
     if constexpr (kSparse) entering = s_list[min(j + 1 + Shape::kAheadK, n_tiles - 1)];
-    if constexpr (kAt >= 0) issue_copy_at(at);
-    else issue_copy(j);
     if (moved != 0) scale_o(alpha);  // wave-uniform
     // row sums of tile j-1: they cover the latency of the operands just requested
     lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_prev, lacc, 0, 0, 0, 0, 0, 0);
@@ -768,6 +778,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         if (has_qk(i + 3)) kf[(i + 3) & 3] = k_frag(i + 3);
       } else if (i + 3 - 8 < kG) {
         vf[i + 3 - 8] = v_frag(i + 3 - 8);
+      }
+      // the copies, clear of the step's first operand reads and of the barrier (-1 % against issuing them at the head)
+      if (i == 4) {
+        if constexpr (kAt >= 0) issue_copy_at(at);
+        else issue_copy(j);
       }
       if (has_qk(i)) s_nxt[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[i & 3], qf[s], s == 0 ? magic : s_nxt[t], 0, 0, 0);
       if constexpr (kPwlExp) {
@@ -828,7 +843,12 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     }
     look_ahead(j + 1, mx, ks_nxt, alpha, moved);
     // after this barrier: tile j+2 is visible to every wave, and nobody reads tile j-1 any more
-    tile_barrier();
+    // (after a pair's: tiles up to j+4, the ones the next pair reads)
+    if constexpr (Shape::kPairs && kAt >= 0) {
+      if constexpr ((kAt & 1) != 0) pair_barrier();
+    } else {
+      tile_barrier();
+    }
   };
 
   {
