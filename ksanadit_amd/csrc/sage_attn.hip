@@ -44,26 +44,24 @@ struct WgShape {
   static_assert(kW == 8 || kW == 4, "workgroups of 8 or 4 waves");
   static constexpr int kThreads = kW * 64;
   static constexpr int kRows = kW * 32;                // query rows per workgroup
-  static constexpr int kStages = kW == 8 ? 8 : 4;      // LDS ring (power of two): tiles j-1 .. j+kAhead live at step j
-  static constexpr int kAhead = kW == 8 ? 5 : 2;       // global -> LDS copies are issued this many tiles ahead
-  static constexpr int kCopies = 2 * (8 / kW);         // 1 KiB copy instructions per wave and tile (K and V^T halves)
+  // K tiles and V^T tiles have a ring of kStages slots each.  A K tile is read one step BEFORE the step of its
+  // probabilities and its V^T tile one step AFTER, so in one ring of whole tiles two K halves would always be dead; in a
+  // ring of its own K can be requested further ahead.
+  static constexpr int kStages = kW == 8 ? 8 : 4;
   static constexpr int kRingBytes = kStages * 2 * kTileBytes;
-  // The 4-wave shape keeps K tiles and V^T tiles in two rings of kStages slots each (same memory).  A K tile is
-  // read one step BEFORE the step of its probabilities and its V^T tile one step AFTER, so in one ring of whole
-  // tiles two K halves are always dead; in its own ring K can be requested kStages tiles ahead instead of two.
-  // That matters where tiles miss the L2 (block masks): with two tiles ahead and every copy awaited at the end of the
-  // step it was issued in, a copy has one step (about a microsecond) to arrive; now it has three.
-  static constexpr bool kTwoRings = kW == 4;
-  static constexpr int kAheadK = kTwoRings ? kStages : kAhead;
-  // copies that may still be in flight at the barrier that ends a step: those of the newest (kAhead - 2) tiles in
-  // one ring; with two rings everything issued in this step and the one before
-  static constexpr int kInFlight = kTwoRings ? 2 * kCopies : kCopies * (kAhead - 2);
-  // The eight-stage ring has room for waves a step apart: in the loop that is unrolled over it the waves meet after
-  // every second step only (a step j and its successor read tiles j-1 .. j+2 and bring in j+5 and j+6, whose slots held
-  // j-3 and j-2), so a wave that rescales its rows holds up the others half as often: 2616 -> 2571 us at 40 heads of
-  // 16384 tokens, 2477 -> 2446 with outliers.  What may be in flight there is what the two steps have issued.
-  static constexpr bool kPairs = kW == 8;
-  static constexpr int kInFlightPairs = 2 * kCopies;
+  static constexpr int kCopies = 2 * (8 / kW);         // 1 KiB copy instructions per wave and tile (K and V^T halves)
+  // How many tiles ahead step j requests the V^T and the K tile.  4 waves: K into the slot of tile j, which every wave
+  // has read; a copy then has three steps (about three microseconds) to arrive, which matters where tiles miss the L2
+  // (block masks).  8 waves: what the groups of four steps below allow.
+  static constexpr int kAhead = kW == 8 ? 3 : 2, kAheadK = kW == 8 ? 5 : 4;
+  // copies that may still be in flight at the barrier that ends a step: those of this step and of the one before
+  static constexpr int kInFlight = 2 * kCopies;
+  // The 8-wave shape's rings have room for waves that are steps apart: in the loop unrolled over them the waves meet after
+  // every fourth step only, so that a wave which rescales its rows holds up the others less often.  The copies of a
+  // group's four steps (g .. g+3: V^T tiles g+3 .. g+6, K tiles g+5 .. g+8, into slots last read before the group) go out
+  // in its first two steps and have landed when it ends.  Us at 40 heads of 16384 tokens, a barrier after every step /
+  // every second / every fourth: 2616 / 2571 / GROUPFIG (with outliers 2477 / 2446 / GROUPFIGO).
+  static constexpr int kGroup = kW == 8 ? 4 : 1;
 };
 constexpr int kMagicI = 0x4B400000;       // bits of 12582912.0f = 1.5 * 2^23: fp32 values are 1 apart there
 constexpr float kMagicF = 12582912.0f;
@@ -84,7 +82,6 @@ constexpr float kMagicF2 = 25165824.0f;
 // for the subnormal codes (it fades them linearly), which must stay 2^-14 below the true maximum to be harmless.
 constexpr float kPShift = 6.0f, kPShiftPwl = 8.0f;
 constexpr float kLazyMax = 2.7f, kLazyMaxPwl = 0.0f;
-constexpr int kStageBytes = 2 * kTileBytes;  // K tile + V tile
 constexpr int kSparseMaxKeyTiles4 = 2048;    // 4-wave workgroups keep their tile list as 16-bit entries so that two fit a compute unit
 constexpr int kMaxKeyTiles = 4096;           // K scales of one head are kept in LDS: Lk <= 262144
 constexpr int kShortKeyTiles = 16;           // dense calls with at most this many key tiles (Lk <= 1024) take 4-wave workgroups
@@ -188,7 +185,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   constexpr int kListMax = kW == 8 ? kSparseMaxKeyTiles : kSparseMaxKeyTiles4;
   static_assert(!(kTileSkip && kPwlExp), "the piecewise-linear code formula has its own zero point: no tiles are skipped there");
   static_assert(kG == 4 || kG == 2, "128 channels, or 64 zero-extended");
-  constexpr bool kUnrolled = !kPwlExp && !kTileSkip;  // the variants calls take by default
+  constexpr bool kUnrolled = !kPwlExp && !kTileSkip && !(kSparse && kW == 8);  // the variants calls take by default
   constexpr int kMagicBits = kG == 4 ? kMagicI : kMagicI2;
   constexpr float kMagicVal = kG == 4 ? kMagicF : kMagicF2;
   int wg, split = 0;
@@ -322,7 +319,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // K scales live in LDS behind the ring: a per-tile global load would share the in-order
   // vmcnt queue with the tile copies and stall on all of them
   // behind the ring: the head's V scales and V means (2 x 128 floats, read by the epilogue), then its K scales
-  float* s_vs = reinterpret_cast<float*>(smem + kStages * kStageBytes);
+  float* s_vs = reinterpret_cast<float*>(smem + Shape::kRingBytes);
   float* s_ks = s_vs + 2 * kD;
 
   // ---- block mask: the workgroup's list of key tiles ---------------------------------------
@@ -482,14 +479,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   const bool has_tail = (lk & (kBlkK - 1)) != 0 && tile_of(n_tiles - 1) == nkb - 1;
   const int n_main = has_tail ? n_tiles - 1 : n_tiles;  // entries handled by the pipelined loop
   // LDS slot of a tile's K half / V^T half
-  auto k_slot = [&](int tile) -> uint8_t* {
-    if constexpr (Shape::kTwoRings) return smem + (tile & (kStages - 1)) * kTileBytes;
-    return smem + (tile & (kStages - 1)) * kStageBytes;
-  };
-  auto v_slot = [&](int tile) -> uint8_t* {
-    if constexpr (Shape::kTwoRings) return smem + (kStages + (tile & (kStages - 1))) * kTileBytes;
-    return smem + (tile & (kStages - 1)) * kStageBytes + kTileBytes;
-  };
+  auto k_slot = [&](int tile) -> uint8_t* { return smem + (tile & (kStages - 1)) * kTileBytes; };
+  auto v_slot = [&](int tile) -> uint8_t* { return smem + (kStages + (tile & (kStages - 1))) * kTileBytes; };
   // clamped: past the end the last tile is copied again into a slot nobody reads any more,
   // which keeps the loop free of branches and the outstanding-copy count constant
   auto copy_tile_half = [&](const uint8_t* src, int jl, uint8_t* dst) {  // jl: key tile number, wave-uniform
@@ -528,20 +519,29 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     lds_copy16_at<kSlot>(buffer, lane_off, off, lds_base);
     if constexpr (kW == 4) lds_copy16_at<kSlot + 4096>(buffer, lane_off + 4096, off, lds_base);
   };
-  // the copies of loop step j at ring position kAt (= j modulo kStages)
-  auto issue_copy_at = [&](auto at) {
-    constexpr int kAt = decltype(at)::value;
-    constexpr int kVs = (kAt + kAhead) & (kStages - 1), kKs = (kAt + Shape::kAheadK) & (kStages - 1);
-    using VSlot = std::integral_constant<int, Shape::kTwoRings ? (kStages + kVs) * kTileBytes : kVs * kStageBytes + kTileBytes>;
-    using KSlot = std::integral_constant<int, Shape::kTwoRings ? kKs * kTileBytes : kKs * kStageBytes>;
+  // the V^T and K tile that tile number kTile (modulo kStages) would request in a loop of single steps
+  auto copies_of = [&](auto tile) {
+    constexpr int kTile = decltype(tile)::value;
+    using VSlot = std::integral_constant<int, (kStages + ((kTile + kAhead) & (kStages - 1))) * kTileBytes>;
+    using KSlot = std::integral_constant<int, ((kTile + Shape::kAheadK) & (kStages - 1)) * kTileBytes>;
     if constexpr (kSparse) {
       copy_to(VSlot{}, v_buf, ahead[0] * kTileBytes);
       copy_to(KSlot{}, k_buf, ahead[kWindow - 1] * kTileBytes);
     } else {
       copy_to(VSlot{}, v_buf, off_v);  // first: it is awaited first
-      copy_to(KSlot{}, k_buf, kAhead == Shape::kAheadK ? off_v : off_k);
+      copy_to(KSlot{}, k_buf, off_k);
       off_v = min(off_v + kTileBytes, off_last);
       off_k = min(off_k + kTileBytes, off_last);
+    }
+  };
+  // the copies of loop step j at ring position kAt (= j modulo kStages)
+  auto issue_copy_at = [&](auto at) {
+    constexpr int kAt = decltype(at)::value, kIn = kAt & (Shape::kGroup - 1);  // position in the group of steps
+    if constexpr (Shape::kGroup == 1) {
+      copies_of(at);
+    } else if constexpr (kIn < 2) {
+      copies_of(std::integral_constant<int, kAt + kIn>{});
+      copies_of(std::integral_constant<int, kAt + kIn + 1>{});
     }
   };
   // the copies of loop step j (step -1: nothing; the prologue below brings the first tiles in)
@@ -559,11 +559,9 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   auto tile_barrier = [&]() {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(Shape::kInFlight) : "memory");
   };
-  // the same after the second step of a pair (Shape::kPairs); steps [0, n_paired) run in pairs
-  auto pair_barrier = [&]() {
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(Shape::kInFlightPairs) : "memory");
-  };
-  const int n_paired = kUnrolled && Shape::kPairs ? n_main / kStages * kStages : 0;
+  // the same after the last step of a group (Shape::kGroup): everything has landed.  Steps [0, n_grouped) run in groups.
+  auto group_barrier = [&]() { asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); };
+  const int n_grouped = kUnrolled && Shape::kGroup > 1 ? n_main / kStages * kStages : 0;
 
   // The compiler does not see the asynchronous copies in the memory-operation counter it models.  Every ordinary global
   // load of the set-up (Q fragments, scales) must therefore be known to have returned before the key loop starts:
@@ -574,31 +572,23 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
   for (int c = 0; c < 8 / kW; ++c)
     *reinterpret_cast<uint4*>(v_slot(-1) + (c * kThreadsAttn + tid) * 16) = make_uint4(0, 0, 0, 0);
-  if constexpr (Shape::kTwoRings) {
 #pragma unroll
-    for (int t = 0; t < kAhead; ++t) copy_half(v_src, t, v_slot(t));
+  for (int t = 0; t < kAhead; ++t) copy_half(v_src, t, v_slot(t));
 #pragma unroll
-    for (int t = 0; t < Shape::kAheadK; ++t) copy_half(k_src, t, k_slot(t));
-  } else {
-#pragma unroll
-    for (int t = 0; t < kAhead; ++t) {  // tile by tile: the oldest copies are the ones awaited
-      copy_half(k_src, t, k_slot(t));
-      copy_half(v_src, t, v_slot(t));
-    }
-  }
+  for (int t = 0; t < Shape::kAheadK; ++t) copy_half(k_src, t, k_slot(t));
   fill_scales();
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the set-up's loads and, older than some of them, the copies
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
   if (!active) {
     // same copy / barrier sequence as the active waves
-    if constexpr (Shape::kTwoRings) __builtin_amdgcn_s_barrier();
+    if constexpr (Shape::kAheadK == kStages) __builtin_amdgcn_s_barrier();
     for (int j = 0; j < n_main; ++j) {
       // (looks the tiles up where they are needed: a wave without rows has nothing an LDS wait could hold up)
       copy_half(v_src, j + kAhead, v_slot(j + kAhead));
       copy_half(k_src, j + Shape::kAheadK, k_slot(j + Shape::kAheadK));
-      if (j >= n_paired) tile_barrier();
-      else if ((j & 1) != 0) pair_barrier();
+      if (j >= n_grouped) tile_barrier();
+      else if ((j & (Shape::kGroup - 1)) == Shape::kGroup - 1) group_barrier();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if constexpr (!kSplit) write_zero_rows();  // rows in [lq, Lq), if any (the merge kernel writes them for cut blocks)
@@ -678,8 +668,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 
   v16i s_a[2], s_b[2];
   qk_tile<kG>(k_slot(0), lane, qf, magic, s_a);
-  // two rings: step 0 requests K tile kStages into the slot of K tile 0, which every wave must have read by then
-  if constexpr (Shape::kTwoRings) __builtin_amdgcn_s_barrier();
+  // where step 0 requests K tile kStages: into the slot of K tile 0, which every wave must have read by then
+  if constexpr (Shape::kAheadK == kStages) __builtin_amdgcn_s_barrier();
   if (diag_at(0)) causal_scores(s_a);
 
   // What a step needs to know about its tile before the first probability: the scale, the exponent's constant and
@@ -731,7 +721,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // Because PV lags one tile, so does the rescaling of O:
   //   at step j   O holds tiles <= j-2 relative to point m(j-2); alpha = 2^(m(j-2) - m(j-1)), tile j-1's
   //   step j      O *= alpha (rare branch), then O += P(j-1) V(j-1), both relative to m(j-1)
-  // LDS ring of 8 stages: tile j-1 (V), j (V next step), j+1 (K), j+2 .. j+5 (arriving).
   // probabilities of the previous and of the current tile swap registers every step, like s_a / s_b
   v8i pf_x = {0, 0, 0, 0, 0, 0, 0, 0}, pf_y = {0, 0, 0, 0, 0, 0, 0, 0};
   // `at`: the step's position in the tile ring (j modulo kStages) where the loop is unrolled over the ring, so that every
@@ -842,13 +831,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       if (diag_at(j)) causal_probs(pf);
     }
     look_ahead(j + 1, mx, ks_nxt, alpha, moved);
-    // after this barrier: tile j+2 is visible to every wave, and nobody reads tile j-1 any more
-    // (after a pair's: tiles up to j+4, the ones the next pair reads)
-    if constexpr (Shape::kPairs && kAt >= 0) {
-      if constexpr ((kAt & 1) != 0) pair_barrier();
-    } else {
-      tile_barrier();
-    }
+    // after this barrier: K tile j+2 and V^T tile j are visible to every wave, and nobody reads their predecessors any
+    // more (after a group's: K tiles up to j+5, V^T tiles up to j+3, the ones the next group reads)
+    if constexpr (kAt < 0 || Shape::kGroup == 1) tile_barrier();
+    else if constexpr ((kAt & (Shape::kGroup - 1)) == Shape::kGroup - 1) group_barrier();
   };
 
   {
@@ -877,11 +863,9 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if (j < n_main) tile_step(Anywhere{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may outlive the workgroup's LDS
-  if constexpr (Shape::kTwoRings) {
-    // the peeled last tile's V^T half was requested two steps ago; the loop's last barrier vouches only for copies
-    // three steps old, so the waves meet once more after each has seen its own copies land (uniform condition)
-    if (has_tail) __builtin_amdgcn_s_barrier();
-  }
+  // The loop's last barrier vouches only for copies a few steps old: before the peeled last tile's V^T half is read, the
+  // waves meet once more after each has seen its own copies land (uniform condition).
+  if (has_tail) __builtin_amdgcn_s_barrier();
   if (n_main > 0) {  // drain: PV of the last pipelined tile
     if ((n_main & 1) != 0) {
       if (moved_even != 0) scale_o(alpha_even);
