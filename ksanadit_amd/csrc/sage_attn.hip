@@ -59,8 +59,9 @@ struct WgShape {
   // The 8-wave shape's rings have room for waves that are steps apart: in the loop unrolled over them the waves meet after
   // every fourth step only, so that a wave which rescales its rows holds up the others less often.  The copies of a
   // group's four steps (g .. g+3: V^T tiles g+3 .. g+6, K tiles g+5 .. g+8, into slots last read before the group) go out
-  // in its first two steps and have landed when it ends.  Us at 40 heads of 16384 tokens, a barrier after every step /
-  // every second / every fourth: 2616 / 2571 / GROUPFIG (with outliers 2477 / 2446 / GROUPFIGO).
+  // in its first two steps and have landed when it ends.  A barrier after every second step instead of every step:
+  // 2616 -> 2571 us at 40 heads of 16384 tokens (2477 -> 2446 with outliers); after every fourth: 0-0.4 % more, and
+  // 515 -> 501 us at B=2, 16 heads of 64 channels, 9001 tokens.
   static constexpr int kGroup = kW == 8 ? 4 : 1;
 };
 constexpr int kMagicI = 0x4B400000;       // bits of 12582912.0f = 1.5 * 2^23: fp32 values are 1 apart there
@@ -572,13 +573,25 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
   for (int c = 0; c < 8 / kW; ++c)
     *reinterpret_cast<uint4*>(v_slot(-1) + (c * kThreadsAttn + tid) * 16) = make_uint4(0, 0, 0, 0);
+  // Awaited here is what must be there before the first barrier of the loop: in single steps (4 waves) K tiles 0 and 1; the
+  // rest goes out after the wait as the copies of "steps -2 and -1" and is awaited by the loop's own count (8 key
+  // tiles, 32760 queries, 40 heads: -1.2 %).
+  constexpr bool kLateCopies = Shape::kGroup == 1;
 #pragma unroll
-  for (int t = 0; t < kAhead; ++t) copy_half(v_src, t, v_slot(t));
+  for (int t = 0; t < (kLateCopies ? 0 : kAhead); ++t) copy_half(v_src, t, v_slot(t));
 #pragma unroll
-  for (int t = 0; t < Shape::kAheadK; ++t) copy_half(k_src, t, k_slot(t));
+  for (int t = 0; t < (kLateCopies ? 2 : Shape::kAheadK); ++t) copy_half(k_src, t, k_slot(t));
   fill_scales();
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the set-up's loads and, older than some of them, the copies
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (kLateCopies) {
+    static_assert(Shape::kAheadK == kAhead + 2, "V^T tiles 0, 1 with K tiles 2, 3");
+#pragma unroll
+    for (int t = 0; t < kAhead; ++t) {
+      copy_half(v_src, t, v_slot(t));
+      copy_half(k_src, t + 2, k_slot(t + 2));
+    }
+  }
 
   if (!active) {
     // same copy / barrier sequence as the active waves

@@ -52,3 +52,26 @@ def test_reference_points_move_at_any_tile(hip_device, waves, Lk, lift):
     sage_ops.quant_q(qd, ws, 128**-0.5), sage_ops.quant_k(kd, ws, True), sage_ops.quant_v(vd, ws)
     out = sage_ops.attn_fwd(ws, torch.empty_like(qd), wg_waves=waves).cpu()
     _close(out, _emul(ws, Lq, Lk, q.dtype))
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("tiles,tail", [(1, 0), (3, 5), (4, 0), (7, 0), (8, 0), (8, 1), (9, 63), (15, 2), (16, 0), (17, 0), (21, 7)])
+@pytest.mark.parametrize("mode", ["dense", "causal", "masked"])
+def test_key_loop_around_its_unrolled_groups(hip_device, waves, tiles, tail, mode):
+    """Numbers of key tiles around the unrolled loop's length (8, or 4), with and without a ragged last tile, with waves
+    that have no query rows (they only take part in the copies and barriers) and a last wave of a few rows."""
+    Lq, Lk, H = 300, 64 * tiles + tail, 1
+    print(f"case waves={waves} Lk={Lk} {mode}", flush=True)
+    g = torch.Generator().manual_seed(Lk)
+    q, k, v = (torch.randn((1, n, H, 128), generator=g).to(torch.bfloat16) for n in (Lq, Lk, Lk))
+    qd, kd, vd = (t.to(hip_device) for t in (q, k, v))
+    ws = sage_ops.workspace_for(qd, kd)
+    sage_ops.quant_q(qd, ws, 128**-0.5), sage_ops.quant_k(kd, ws, True), sage_ops.quant_v(vd, ws)
+    kw = {}
+    if mode == "causal":
+        kw["causal"] = True
+    if mode == "masked":
+        kw["block_mask"] = (torch.rand((1, H, 3, -(-Lk // 64)), generator=g) < 0.7).to(torch.int8)
+    out = sage_ops.attn_fwd(ws, torch.empty_like(qd), wg_waves=waves, **kw).cpu()
+    split = sage_ops.key_split_plan(ws) if mode == "dense" and waves == 8 else None
+    _close(out, _emul(ws, Lq, Lk, q.dtype, key_split=split, **kw))
