@@ -85,8 +85,7 @@ constexpr float kPShift = 6.0f, kPShiftPwl = 8.0f;
 constexpr float kLazyMax = 2.7f, kLazyMaxPwl = 0.0f;
 constexpr int kSparseMaxKeyTiles4 = 2048;    // 4-wave workgroups keep their tile list as 16-bit entries so that two fit a compute unit
 constexpr int kMaxKeyTiles = 4096;           // K scales of one head are kept in LDS: Lk <= 262144
-constexpr int kShortKeyTiles = 16;           // dense calls with at most this many key tiles (Lk <= 1024) take 4-wave workgroups
-constexpr int kMidKeyTiles = 96;             // ... and up to this many (Lk <= 6144) when their 256-row grid fills the chip at least once
+constexpr int kShortKeyTiles = 16;           // calls with at most this many key tiles (Lk <= 1024) are never cut into runs of keys
 constexpr int kShortMaxKeyTiles = 2048;      // the most key tiles a dense 4-wave workgroup can hold scales for
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -165,22 +164,23 @@ __device__ __forceinline__ void qk_tile(const uint8_t* k_stage, int lane, const 
   }
 }
 
-// kSplit: the workgroup takes one of `p.n_split` equal runs of key tiles of its (head, query block) and leaves
-// unnormalised accumulators, running maxima and row sums in the workspace for sage_attn_merge_kernel.  Used for
-// the workgroups beyond the last full round of the chip, which would otherwise hold it for a whole round alone.
+// Dense 8-wave calls can hold two kinds of workgroup in one grid: blocks below p.split_first_block walk all key tiles of
+// their (head, query block); each of the blocks from there on takes one of `p.n_split` equal runs of key tiles and leaves
+// unnormalised accumulators, running maxima and row sums in the workspace for sage_attn_merge_kernel.  The runs stand
+// for the query blocks beyond the last full round of the chip, which would otherwise hold it for a whole round alone; in
+// the same grid they start as the last whole blocks finish.
 // kG: 32-channel groups the matrix instructions cover - 4, or 2 when the head size is 64 (rows run zero-extended to
 // 128 channels and the operands keep their layout; see kMagicI2 for what is left out and why nothing is lost; the
 // result equals the full-width code's up to the rounding of one constant in the exponent).
-template <int DT, bool kPwlExp, bool kSparse, bool kSplit, int kW, bool kTileSkip, int kG, bool kCausal>
+template <int DT, bool kPwlExp, bool kSparse, int kW, bool kTileSkip, int kG, bool kCausal>
 __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel(const AttnParams p, int n_qwg,
                                                                                    int n_wg, int wg_per_xcd) {
-  static_assert(!(kSparse && kSplit), "the key split is built for the dense loop only");
+  constexpr bool kCanSplit = !kSparse && kW == 8;
   static_assert(kSparse || !kCausal, "causal calls run through the tile list");
   // kCausal == false: the caller vouches that p.causal is 0, and everything that serves the diagonal (the per-wave
   // last tile, 32 lane masks held in scalar registers, the selects that blank a wave's probabilities past its rows)
   // is compiled out of the key loop
   const bool causal = kCausal && p.causal;
-  static_assert(!kSplit || kW == 8, "the key split is built for 256-row workgroups");
   using Shape = WgShape<kW>;
   constexpr int kThreadsAttn = Shape::kThreads, kRowsWg = Shape::kRows, kStages = Shape::kStages, kAhead = Shape::kAhead;
   constexpr int kListMax = kW == 8 ? kSparseMaxKeyTiles : kSparseMaxKeyTiles4;
@@ -189,11 +189,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   constexpr bool kUnrolled = !kPwlExp && !kTileSkip && !(kSparse && kW == 8);  // the variants calls take by default
   constexpr int kMagicBits = kG == 4 ? kMagicI : kMagicI2;
   constexpr float kMagicVal = kG == 4 ? kMagicF : kMagicF2;
-  int wg, split = 0;
-  if constexpr (kSplit) {
-    const int item = blockIdx.x / p.n_split;
-    split = blockIdx.x - item * p.n_split;
-    wg = p.split_first_wg + item;
+  int wg;
+  const bool is_run = kCanSplit && (int)blockIdx.x >= p.split_first_block;  // uniform
+  const int run_id = is_run ? (int)blockIdx.x - p.split_first_block : 0;    // the partial result's place in the workspace
+  if (is_run) {
+    wg = p.split_first_wg + run_id / p.n_split;
   } else {
     // Consecutive workgroup ids land on consecutive XCDs (8 per chip, one L2 each).  Give every
     // XCD a contiguous run of (head, query block) pairs so the workgroups that stream the same
@@ -240,7 +240,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     }
   };
   int tile0 = 0;  // first key tile of this workgroup's run
-  if constexpr (kSplit) {
+  if (is_run) {
+    const int split = run_id % p.n_split;
     const int tiles = (lk + kBlkK - 1) / kBlkK;
     const int per = (tiles + p.n_split - 1) / p.n_split;
     tile0 = split * per;
@@ -248,10 +249,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if (tile0 >= tile1 || qwg * kRowsWg >= lq) {  // nothing in this run (few tiles, a batch entry without keys, or no query row): an empty partial
       if (active) {
         const int row = wave * 32 + l32;
-        float* po = p.split_o + ((int64_t)blockIdx.x * kAttnQPerWg + row) * kD + 64 * hh;
+        float* po = p.split_o + ((int64_t)run_id * kAttnQPerWg + row) * kD + 64 * hh;
 #pragma unroll
         for (int i = 0; i < 16; ++i) reinterpret_cast<float4*>(po)[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (hh == 0) reinterpret_cast<float2*>(p.split_ml)[(int64_t)blockIdx.x * kAttnQPerWg + row] = make_float2(-INFINITY, 0.f);
+        if (hh == 0) reinterpret_cast<float2*>(p.split_ml)[(int64_t)run_id * kAttnQPerWg + row] = make_float2(-INFINITY, 0.f);
       }
       return;
     }
@@ -604,7 +605,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       else if ((j & (Shape::kGroup - 1)) == Shape::kGroup - 1) group_barrier();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if constexpr (!kSplit) write_zero_rows();  // rows in [lq, Lq), if any (the merge kernel writes them for cut blocks)
+    if (!is_run) write_zero_rows();  // rows in [lq, Lq), if any (the merge kernel writes them for cut blocks)
     return;
   }
 
@@ -929,17 +930,17 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, lacc, 0, 0, 0, 0, 0, 0);
   }
 
-  if constexpr (kSplit) {
+  if (is_run) {
     // partial result of this run of keys: O^T and the row sum relative to the run's own maximum
     const int row = wave * 32 + l32;
-    float* po = p.split_o + ((int64_t)blockIdx.x * kAttnQPerWg + row) * kD;
+    float* po = p.split_o + ((int64_t)run_id * kAttnQPerWg + row) * kD;
 #pragma unroll
     for (int dt = 0; dt < kG; ++dt)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         *reinterpret_cast<float4*>(po + 32 * dt + 8 * g + 4 * hh) =
             make_float4(oacc[dt][4 * g + 0], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]);
-    if (hh == 0) reinterpret_cast<float2*>(p.split_ml)[(int64_t)blockIdx.x * kAttnQPerWg + row] = make_float2(m_run, lacc[0]);
+    if (hh == 0) reinterpret_cast<float2*>(p.split_ml)[(int64_t)run_id * kAttnQPerWg + row] = make_float2(m_run, lacc[0]);
     return;
   }
   // ---- epilogue: O = O^T / rowsum * v_scale (+ the V mean), written [B, Lq, H, D] ---------------
@@ -1017,17 +1018,35 @@ __global__ __launch_bounds__(256) void sage_attn_merge_kernel(const AttnParams p
   }
   const float2* ml = reinterpret_cast<const float2*>(p.split_ml) + (int64_t)item * p.n_split * kAttnQPerWg + row;
   const float* po = p.split_o + ((int64_t)item * p.n_split * kAttnQPerWg + row) * kD + d;
+  // Eight runs at a time, their loads in flight together: one run after the other, a row waits for as many memory
+  // latencies as it has runs (8 query blocks of 32 runs: 29.5 us, 10.5 like this).
+  constexpr int kAtOnce = 8;
   float m = -INFINITY;
-  for (int s = 0; s < p.n_split; ++s) m = fmaxf(m, ml[(int64_t)s * kAttnQPerWg].x);
+  for (int s0 = 0; s0 < p.n_split; s0 += kAtOnce) {
+    float mm[kAtOnce];
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i) mm[i] = ml[(int64_t)min(s0 + i, p.n_split - 1) * kAttnQPerWg].x;
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i) m = fmaxf(m, mm[i]);
+  }
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   float l = 0.0f;
-  for (int s = 0; s < p.n_split; ++s) {
-    const float2 e = ml[(int64_t)s * kAttnQPerWg];
-    if (e.y == 0.0f) continue;  // an empty run (its maximum is -inf)
-    const float w = fast_exp2(e.x - m);
-    const float4 o = *reinterpret_cast<const float4*>(po + (int64_t)s * kAttnQPerWg * kD);
-    acc.x += o.x * w, acc.y += o.y * w, acc.z += o.z * w, acc.w += o.w * w;
-    l += e.y * w;
+  for (int s0 = 0; s0 < p.n_split; s0 += kAtOnce) {
+    float2 e[kAtOnce];
+    float4 o[kAtOnce];
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i) {
+      const int64_t at = min(s0 + i, p.n_split - 1);
+      e[i] = ml[at * kAttnQPerWg];
+      o[i] = *reinterpret_cast<const float4*>(po + at * (kAttnQPerWg * kD));
+    }
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i) {
+      if (s0 + i >= p.n_split || e[i].y == 0.0f) continue;  // (no such run, or an empty one, whose maximum is -inf)
+      const float w = fast_exp2(e[i].x - m);
+      acc.x += o[i].x * w, acc.y += o[i].y * w, acc.z += o[i].z * w, acc.w += o[i].w * w;
+      l += e[i].y * w;
+    }
   }
   const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
   const float keep_mean = l > 0.0f ? 1.0f : 0.0f;
@@ -1044,7 +1063,7 @@ constexpr size_t max_lds() {
                  : WgShape<kW>::kRingBytes + 2048 + (kW == 8 ? kMaxKeyTiles : kShortMaxKeyTiles) * 4;
 }
 
-template <int DT, bool kPwlExp, bool kSparse, bool kSplit, int kW, bool kCausal, bool kTileSkip = false, int kG = 4>
+template <int DT, bool kPwlExp, bool kSparse, int kW, bool kCausal, bool kTileSkip = false, int kG = 4>
 hipError_t launch_variant(const AttnParams& p, dim3 grid, size_t lds, int n_qwg, int n_wg, int wg_per_xcd,
                           hipStream_t s) {
   // more than 64 KiB of dynamic LDS has to be requested per kernel, once per device
@@ -1055,32 +1074,32 @@ hipError_t launch_variant(const AttnParams& p, dim3 grid, size_t lds, int n_qwg,
   if (e != hipSuccess) return e;
   if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
   if (!requested[dev].load(std::memory_order_acquire)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kSplit, kW, kTileSkip, kG, kCausal>),
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds<kSparse, kW>());
     if (e != hipSuccess) return e;
     requested[dev].store(true, std::memory_order_release);
   }
-  sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kSplit, kW, kTileSkip, kG, kCausal><<<grid, dim3(kW * 64), lds, s>>>(p, n_qwg, n_wg, wg_per_xcd);
+  sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal><<<grid, dim3(kW * 64), lds, s>>>(p, n_qwg, n_wg, wg_per_xcd);
   return hipGetLastError();
 }
 
-// the (dtype, exp2 form, tile skip) instantiations behind one (mask, split, workgroup shape) choice
-template <bool kSparse, bool kSplit, int kW, bool kCausal = false>
+// the (dtype, exp2 form, tile skip) instantiations behind one (mask, workgroup shape) choice
+template <bool kSparse, int kW, bool kCausal = false>
 hipError_t launch_shape(const AttnParams& p, dim3 grid, size_t lds, int n_qwg, int n_wg, int wg_per_xcd, hipStream_t s) {
   const bool bf16 = p.o.dtype == KSANA_SAGE_BF16;
   // head size 64: the matrix instructions on the zero halves are left out (plain exact-exponential calls; the other
   // variants run the full-width code on the same operands, which gives the same bits)
   if (p.exact_exp2 && !p.tile_skip && p.d_out <= 64)
-    return bf16 ? launch_variant<KSANA_SAGE_BF16, false, kSparse, kSplit, kW, kCausal, false, 2>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
-                : launch_variant<KSANA_SAGE_FP16, false, kSparse, kSplit, kW, kCausal, false, 2>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+    return bf16 ? launch_variant<KSANA_SAGE_BF16, false, kSparse, kW, kCausal, false, 2>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
+                : launch_variant<KSANA_SAGE_FP16, false, kSparse, kW, kCausal, false, 2>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
   if (p.exact_exp2 && p.tile_skip)
-    return bf16 ? launch_variant<KSANA_SAGE_BF16, false, kSparse, kSplit, kW, kCausal, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
-                : launch_variant<KSANA_SAGE_FP16, false, kSparse, kSplit, kW, kCausal, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+    return bf16 ? launch_variant<KSANA_SAGE_BF16, false, kSparse, kW, kCausal, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
+                : launch_variant<KSANA_SAGE_FP16, false, kSparse, kW, kCausal, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
   if (p.exact_exp2)
-    return bf16 ? launch_variant<KSANA_SAGE_BF16, false, kSparse, kSplit, kW, kCausal>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
-                : launch_variant<KSANA_SAGE_FP16, false, kSparse, kSplit, kW, kCausal>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
-  return bf16 ? launch_variant<KSANA_SAGE_BF16, true, kSparse, kSplit, kW, kCausal>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
-              : launch_variant<KSANA_SAGE_FP16, true, kSparse, kSplit, kW, kCausal>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+    return bf16 ? launch_variant<KSANA_SAGE_BF16, false, kSparse, kW, kCausal>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
+                : launch_variant<KSANA_SAGE_FP16, false, kSparse, kW, kCausal>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+  return bf16 ? launch_variant<KSANA_SAGE_BF16, true, kSparse, kW, kCausal>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
+              : launch_variant<KSANA_SAGE_FP16, true, kSparse, kW, kCausal>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
 }
 
 // compute units of the current device (the size of one round of workgroups: one workgroup per unit)
@@ -1099,41 +1118,62 @@ int compute_units() {
 
 }  // namespace
 
-// Dense calls that take 4-wave workgroups (n_wg8: their grid in 256-row workgroups): short key loops, where a
-// workgroup's fixed costs weigh as much as its loop and hide under the compute unit's other workgroup - measured at
-// B * H = 40 and 48: 32 tiles 14-19 % faster than 256-row workgroups, 64-68 tiles 2-6 %, 128 tiles 1-3 % slower.
-// Beyond kShortKeyTiles only when the chip is full anyway: a grid of a few workgroups is better off cut into runs of
-// keys, which only the 256-row shape does.
-static bool dense_in_four_waves(int n_wg8, int nkb) {
-  return nkb <= kShortKeyTiles || (nkb <= kMidKeyTiles && n_wg8 >= compute_units());
+// How a dense call is laid out: workgroups of 4 or 8 waves, and (8 waves) the first workgroup that is cut into runs of
+// key tiles, and into how many (0: none).
+struct DensePlan {
+  int waves, first_cut, runs;
+};
+
+// n_wg: the grid in 256-row workgroups, nkb: key tiles.  The choice is between
+//   8 waves        one workgroup per compute unit: the lowest time per tile, but the workgroups beyond the last full round
+//                  of the chip take most of a round however few they are (alone, they run a third faster),
+//   8 waves, cut   those workgroups as runs of keys that fill the chip: a short round, then the merge kernel,
+//   4 waves        two workgroups per compute unit, which hide each other's set-up and epilogue; in an incomplete round
+//                  one alone on its unit takes half the time.
+// Estimates in units of one tile of an 8-wave workgroup (about a microsecond), fitted to measurements of grids of 0.03 ..
+// 4.5 rounds and 8 .. 200 tiles: a full round of T tiles takes 1.005 T + 5.5 (8 waves) or 1.05 T + 4.5 (4 waves).  An
+// incomplete one takes at least 0.75 of that in 8 waves; in 4 waves 0.5 up to half full and its own filling and 0.1 more
+// from there (0.55 and 0.17 more where it is the only round).  Runs of keys take their own tiles, and writing and merging
+// up to 256 partial results of 128 KiB costs 5 .. 15.
+// Examples, us, 4 waves / 8 waves cut: 2.25 rounds of 96 tiles 258 / 242, 1.1 of 68 tiles 114 / 97, 3.1 of 80 tiles
+// 312 / 282; but a quarter of a round of 20 tiles 17 / 28, of 32 tiles 24 / 32.
+static DensePlan plan_dense(int n_wg, int nkb) {
+  const int cus = compute_units();
+  const int rounds = n_wg / cus, rest = n_wg % cus;
+  int runs = 0;
+  if (rest != 0 && 2 * rest <= cus && nkb > kShortKeyTiles) {
+    runs = min(min(cus / rest, kMaxSplitPartials / rest), nkb / kMinTilesPerSplit);
+    if (runs < 2) runs = 0;
+  }
+  if (n_wg <= cus / 16 && runs != 0) return DensePlan{8, 0, runs};  // a handful of workgroups: as many runs as there are
+  const float part = (float)rest / (float)cus, alone = rounds == 0 ? 1.0f : 0.0f;
+  const float round8 = 1.005f * (float)nkb + 5.5f, round4 = 1.05f * (float)nkb + 4.5f;
+  const float whole8 = ((float)rounds + (rest == 0 ? 0.0f : fmaxf(0.75f, part))) * round8 + 4.0f * alone;
+  const float cut8 = runs == 0 ? INFINITY
+                               : (float)rounds * round8 + 0.9f * ((float)((nkb + runs - 1) / runs) + 5.5f) + 5.0f +
+                                     10.0f * (float)(rest * runs) / (float)cus;
+  const float part4 = rest == 0         ? 0.0f
+                      : 2 * rest <= cus ? 0.5f + 0.045f * alone
+                                        : fminf(1.0f, part + 0.1f + 0.07f * alone);
+  const float whole4 = nkb > kShortMaxKeyTiles ? INFINITY : ((float)rounds + part4) * round4 + 3.6f * alone;
+  if (whole4 < fminf(whole8, cut8)) return DensePlan{4, n_wg, 0};
+  if (cut8 < whole8) return DensePlan{8, n_wg - rest, runs};
+  return DensePlan{8, n_wg, 0};
 }
 
 void plan_key_split(int n_wg, int nkb, int* first_wg, int* runs) {
-  if (dense_in_four_waves(n_wg, nkb)) {  // these shapes run in 4-wave workgroups, which are never cut
-    *first_wg = n_wg, *runs = 0;
-    return;
-  }
-  const int cus = compute_units();
-  const int rest = n_wg % cus;
-  int n_split = 0;
-  if (rest != 0 && 2 * rest <= cus) {
-    n_split = min(min(cus / rest, kMaxSplitPartials / rest), nkb / kMinTilesPerSplit);
-    if (n_split < 2) n_split = 0;
-  }
-  *first_wg = n_split ? n_wg - rest : n_wg;
-  *runs = n_split;
+  const DensePlan plan = plan_dense(n_wg, nkb);
+  *first_wg = plan.first_cut, *runs = plan.runs;
 }
 
 // Workgroup shape for a call: 4-wave workgroups (two per compute unit) when a block mask or causal masking is
 // involved (a workgroup is then one 128-row mask row, so no wave multiplies a tile only the neighbouring mask row
-// asked for) and for short key sequences (dense_in_four_waves); 8-wave workgroups otherwise, which copy
-// every K/V tile once per 256 rows instead of once per 128.  p.wg_waves (4 or 8) overrides the choice.
+// asked for), plan_dense's choice otherwise.  p.wg_waves (4 or 8) overrides the choice.
 static int pick_wg_waves(const AttnParams& p) {
   if (p.wg_waves == 4 || p.wg_waves == 8) return p.wg_waves;
   const bool sparse = p.block_mask != nullptr || p.causal;
   if (sparse) return p.nkb <= kSparseMaxKeyTiles4 ? 4 : 8;
-  const int n_wg8 = p.B * p.Hq * ((p.Lq + kAttnQPerWg - 1) / kAttnQPerWg);
-  return dense_in_four_waves(n_wg8, p.nkb) ? 4 : 8;
+  return plan_dense(p.B * p.Hq * ((p.Lq + kAttnQPerWg - 1) / kAttnQPerWg), p.nkb).waves;
 }
 
 // Grid of a launch whose workgroups are numbered in runs per XCD (see the kernel's first lines), and the run's length.
@@ -1146,6 +1186,7 @@ static dim3 xcd_grid(AttnParams* p, int n_qwg, int n_wg, int* wg_per_xcd) {
 
 hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   AttnParams p = params;
+  p.split_first_block = INT32_MAX;
   if (p.nkb > kMaxKeyTiles) return hipErrorInvalidValue;
   const bool sparse = p.block_mask != nullptr || p.causal;
   if (sparse && p.nkb > kSparseMaxKeyTiles) return hipErrorInvalidValue;
@@ -1157,17 +1198,17 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
     int wg_per_xcd = 0;
     const dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
     if (sparse)
-      return p.causal ? launch_shape<true, false, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
-                      : launch_shape<true, false, 4, false>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s);
+      return p.causal ? launch_shape<true, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
+                      : launch_shape<true, 4, false>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s);
     const size_t lds = WgShape<4>::kRingBytes + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
-    return launch_shape<false, false, 4>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+    return launch_shape<false, 4>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
   }
   const int n_qwg = (p.Lq + kAttnQPerWg - 1) / kAttnQPerWg;
   const int n_wg = p.B * p.Hq * n_qwg;
   int wg_per_xcd = 0;
   const dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
   // (tile lists in 256-row workgroups, by flag only: one instantiation serves causal and plain calls)
-  if (sparse) return launch_shape<true, false, 8, true>(p, grid, max_lds<true, 8>(), n_qwg, n_wg, wg_per_xcd, s);
+  if (sparse) return launch_shape<true, 8, true>(p, grid, max_lds<true, 8>(), n_qwg, n_wg, wg_per_xcd, s);
   // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
   const size_t lds = WgShape<8>::kRingBytes + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
   // The workgroups beyond the last full round of the chip (one workgroup per compute unit) would hold it for a
@@ -1175,23 +1216,18 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   // small kernel merges the runs: 2568 workgroups are then 10 rounds and a bit instead of 11, 280 are 1.1 instead of 2.
   int n_full = n_wg, n_split = 0;
   if (p.split_o != nullptr) plan_key_split(n_wg, p.nkb, &n_full, &n_split);
-  if (n_split == 0) return launch_shape<false, false, 8>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+  if (n_split == 0) return launch_shape<false, 8>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
   const int rest = n_wg - n_full;
-  if (n_full > 0) {
-    int per_xcd = 0;
-    const dim3 grid_full = xcd_grid(&p, n_qwg, n_full, &per_xcd);
-    const hipError_t e = launch_shape<false, false, 8>(p, grid_full, lds, n_qwg, n_full, per_xcd, s);
-    if (e != hipSuccess) return e;
-  }
-  AttnParams ps = p;
-  ps.split_first_wg = n_full;
-  ps.n_split = n_split;
-  const hipError_t e = launch_shape<false, true, 8>(ps, dim3(rest * n_split), lds, n_qwg, n_wg, 0, s);
+  const dim3 grid_full = n_full > 0 ? xcd_grid(&p, n_qwg, n_full, &wg_per_xcd) : dim3(0);
+  p.split_first_block = (int)grid_full.x;
+  p.split_first_wg = n_full;
+  p.n_split = n_split;
+  const hipError_t e = launch_shape<false, 8>(p, dim3(grid_full.x + rest * n_split), lds, n_qwg, n_full, wg_per_xcd, s);
   if (e != hipSuccess) return e;
   if (p.o.dtype == KSANA_SAGE_BF16)
-    sage_attn_merge_kernel<KSANA_SAGE_BF16><<<dim3(rest, kAttnQPerWg / 8), dim3(256), 0, s>>>(ps, n_qwg);
+    sage_attn_merge_kernel<KSANA_SAGE_BF16><<<dim3(rest, kAttnQPerWg / 8), dim3(256), 0, s>>>(p, n_qwg);
   else
-    sage_attn_merge_kernel<KSANA_SAGE_FP16><<<dim3(rest, kAttnQPerWg / 8), dim3(256), 0, s>>>(ps, n_qwg);
+    sage_attn_merge_kernel<KSANA_SAGE_FP16><<<dim3(rest, kAttnQPerWg / 8), dim3(256), 0, s>>>(p, n_qwg);
   return hipGetLastError();
 }
 

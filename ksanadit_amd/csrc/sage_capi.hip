@@ -700,7 +700,6 @@ int ksana_sage_attn_fwd_varlen(void* ws, void* o, int dtype, const int64_t o_st[
   p.v_mean = ws_at<float>(ws, l.v_mean);
   p.split_o = ws_at<float>(ws, l.split_o);
   p.split_ml = ws_at<float>(ws, l.split_ml);
-  p.split_first_wg = 0, p.n_split = 0;
   p.wg_waves = (flags & KSANA_SAGE_FLAG_WG_4_WAVES) ? 4 : ((flags & KSANA_SAGE_FLAG_WG_8_WAVES) ? 8 : 0);
   p.o = ksana_sage::OutTensor{static_cast<uint16_t*>(o), o_st[0], o_st[1], o_st[2], dtype};
   p.B = s->B, p.Hq = s->Hq, p.Hkv = s->Hkv, p.Lq = s->Lq, p.Lk = s->Lk;

@@ -198,7 +198,7 @@ struct AttnParams {
   // accumulators, and per row its running maximum and row sum; room for kMaxSplitPartials partials
   float* split_o;
   float* split_ml;
-  int split_first_wg, n_split;  // filled in by the launcher
+  int split_first_block = 0, split_first_wg = 0, n_split = 0;  // filled in by the launcher
   int batch_run = 0;  // filled in by the launcher: 0, or the workgroups of one batch entry that go to one XCD
   int wg_waves;  // 0: the launcher picks the workgroup shape; 4 or 8: forced (for measurements and tests)
   int d_out;     // channels of an output row that exist: 128, or 64 (head size 64 runs zero-padded to 128)

@@ -75,3 +75,26 @@ def test_key_loop_around_its_unrolled_groups(hip_device, waves, tiles, tail, mod
     out = sage_ops.attn_fwd(ws, torch.empty_like(qd), wg_waves=waves, **kw).cpu()
     split = sage_ops.key_split_plan(ws) if mode == "dense" and waves == 8 else None
     _close(out, _emul(ws, Lq, Lk, q.dtype, key_split=split, **kw))
+
+
+@pytest.mark.parametrize("Lk", [64 * 33, 64 * 40 + 1])
+def test_whole_and_cut_query_blocks_in_one_grid(hip_device, Lk):
+    """65 heads of 4 query blocks: one full round of whole blocks and 4 blocks cut into runs of keys.  The last head holds
+    the cut ones (ragged rows in the last), the head before it whole ones."""
+    Lq, H, at = 1000, 65, 63
+    print(f"case Lk={Lk}", flush=True)
+    g = torch.Generator().manual_seed(Lk)
+    q, k, v = (torch.randn((1, n, H, 128), generator=g).to(torch.bfloat16) for n in (Lq, Lk, Lk))
+    qd, kd, vd = (t.to(hip_device) for t in (q, k, v))
+    ws = sage_ops.workspace_for(qd, kd)
+    plan = sage_ops.key_split_plan(ws)
+    if torch.cuda.get_device_properties(hip_device).multi_processor_count == 256:
+        assert plan is not None and plan[0] == 256 and plan[1] >= 2, plan
+    out = sage_ops.sageattn(qd, kd, vd, workspace=ws)[:, :, at:].cpu()
+    heads = slice(at, H)
+    split = None if plan is None else (max(plan[0] - 4 * at, 0), plan[1])
+    want = sage_emul_from_quant(
+        ws.q_i8.cpu()[:, heads, :Lq], ws.q_scale.cpu()[:, heads, :Lq], untile_k(ws.k_tiles.cpu()[:, heads], Lk),
+        ws.k_scale.cpu()[:, heads], untile_v(ws.v_tiles.cpu()[:, heads], Lk).view(torch.float8_e4m3fn),
+        ws.v_scale.cpu()[:, heads], q.dtype, key_split=split)
+    _close(out, want)
