@@ -563,6 +563,9 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   };
   // the same after the last step of a group (Shape::kGroup): everything has landed.  Steps [0, n_grouped) run in groups.
   auto group_barrier = [&]() { asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); };
+  // K tile kStages goes into the slot of K tile 0, which every wave must have read by then - in the set-up, and a single
+  // step requests tiles kAheadK ahead, the first group of steps all up to kStages, before the loop's first barrier.
+  constexpr bool kSlotZeroSoon = Shape::kAheadK == kStages || (kUnrolled && Shape::kGroup > 1);
   const int n_grouped = kUnrolled && Shape::kGroup > 1 ? n_main / kStages * kStages : 0;
 
   // The compiler does not see the asynchronous copies in the memory-operation counter it models.  Every ordinary global
@@ -596,7 +599,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 
   if (!active) {
     // same copy / barrier sequence as the active waves
-    if constexpr (Shape::kAheadK == kStages) __builtin_amdgcn_s_barrier();
+    if constexpr (kSlotZeroSoon) __builtin_amdgcn_s_barrier();
     for (int j = 0; j < n_main; ++j) {
       // (looks the tiles up where they are needed: a wave without rows has nothing an LDS wait could hold up)
       copy_half(v_src, j + kAhead, v_slot(j + kAhead));
@@ -682,8 +685,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 
   v16i s_a[2], s_b[2];
   qk_tile<kG>(k_slot(0), lane, qf, magic, s_a);
-  // where step 0 requests K tile kStages: into the slot of K tile 0, which every wave must have read by then
-  if constexpr (Shape::kAheadK == kStages) __builtin_amdgcn_s_barrier();
+  if constexpr (kSlotZeroSoon) __builtin_amdgcn_s_barrier();
   if (diag_at(0)) causal_scores(s_a);
 
   // What a step needs to know about its tile before the first probability: the scale, the exponent's constant and

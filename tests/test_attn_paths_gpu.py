@@ -98,3 +98,18 @@ def test_whole_and_cut_query_blocks_in_one_grid(hip_device, Lk):
         ws.k_scale.cpu()[:, heads], untile_v(ws.v_tiles.cpu()[:, heads], Lk).view(torch.float8_e4m3fn),
         ws.v_scale.cpu()[:, heads], q.dtype, key_split=split)
     _close(out, want)
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("Lk", [64 * 8, 64 * 9, 64 * 17 + 3])
+def test_repeated_calls_give_the_same_bits(hip_device, waves, Lk):
+    """The waves of a workgroup share the tile ring and meet seldom: whatever their pace, no tile is replaced before all have
+    read it."""
+    print(f"case waves={waves} Lk={Lk}", flush=True)
+    g = torch.Generator().manual_seed(Lk)
+    q, k, v = (torch.randn((1, n, 16, 128), generator=g).to(torch.float16).to(hip_device) for n in (512, Lk, Lk))
+    ws = sage_ops.workspace_for(q, k)
+    sage_ops.quant_q(q, ws, 128**-0.5), sage_ops.quant_k(k, ws, True), sage_ops.quant_v(v, ws)
+    first = sage_ops.attn_fwd(ws, torch.empty_like(q), wg_waves=waves)
+    for _ in range(40):
+        assert torch.equal(sage_ops.attn_fwd(ws, torch.empty_like(q), wg_waves=waves), first)
