@@ -286,13 +286,16 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.0f;
   // reference point of query l32 in the log2 domain (its "running maximum"), and what the steps read it as: the
   // exponent's constant part and the score above which the point has to move
-  float m_run = -INFINITY, x_base = INFINITY, x_limit = -INFINITY;
+  // (base -inf: the probabilities of a row without a point are zeros)
+  float m_run = -INFINITY, x_base = -INFINITY, x_limit = -INFINITY;
   // Row sums come from the matrix pipe too, of the SAME e4m3-rounded P the numerator uses.  The 16x16x128 instruction
   // takes half the matrix cycles of the 32x32x64 one and a quarter of its accumulators; its B operand is P's register
   // block read as 16 columns with four groups of 16 lanes stacked along the contraction: groups 0 and 2 hold the two
   // halves of query (lane % 16)'s keys, groups 1 and 3 those of query 16 + (lane % 16).  A therefore carries ones
   // (e4m3 1.0 = 0x38) where output row 4 g' .. 4 g' + 3 and group g agree in parity and zeros elsewhere: the lanes of
   // group g' then find the sum of their own query in all four registers.  Only register 0 is read and rescaled.
+  // A zero of A meets the probabilities of the query 16 further, and zero times NaN is NaN: no probability may be one
+  // (move_point sees to it).
   v4f lacc = {0.0f, 0.0f, 0.0f, 0.0f};
   // eight registers on purpose: left as one value the compiler keeps a single copy and rebuilds
   // the 8-register operand with seven moves in every step
@@ -633,7 +636,9 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   constexpr float kShift = kPwlExp ? kPShiftPwl : kPShift, kLazy = kPwlExp ? kLazyMaxPwl : kLazyMax;
   // Moves query l32's reference point where this tile's maximum asks for it (imax: this lane's maximum, over half the
   // query's keys) and returns 2^(old point - new point), exactly 1 where the point stays.
-  auto move_point = [&](int imax, float sc, float mneg) -> float {
+  // A row whose scores are not numbers (an infinity in its q, or in a key) gets the factor NaN, which makes its
+  // accumulators and sums NaN, and goes on with zero scores: its probabilities must stay numbers, see lacc.
+  auto move_point = [&](int imax, float& sc, float& mneg) -> float {
     {
       // the other half of query l32's keys lives in lane l32 + 32
       int other = imax;
@@ -642,8 +647,12 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     }
     // the accumulator read as fp32 is magic + dot, so one fma gives sc * dot (mneg = -magic * sc)
     const float m_tile = __builtin_fmaf(__int_as_float(imax), sc, mneg);
-    const float m_new = m_tile > x_limit ? m_tile : m_run;  // the limit is -inf at the first tile: always taken
-    const float alpha = fast_exp2(m_run - m_new);
+    const bool nan = m_tile != m_tile;
+    const float m_new = nan ? 0.0f : (m_tile > x_limit ? m_tile : m_run);  // the limit is -inf at the first tile: always taken
+    const float alpha = fast_exp2((nan ? m_tile : m_run) - m_new);
+    sc = nan ? 0.0f : sc;
+    mneg = nan ? 0.0f : mneg;
+    qs = nan ? 0.0f : qs;
     m_run = m_new;
     x_limit = m_new + kLazy;
     x_base = kShift - m_new;
@@ -704,10 +713,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   bool nothing = false;                 // (wave-uniform) every probability of the coming tile converts to zero
   auto look_ahead = [&](int jn, int mx, float ks, float& alpha, int& moved) {
     sc = qs * ks;
-    const float mneg = -kMagicVal * sc;
+    float mneg = -kMagicVal * sc;
     const float m_half = __builtin_fmaf(__int_as_float(mx), sc, mneg);
     moved = 0;
-    if (__ballot(m_half > x_limit) != 0) {
+    if (__ballot(!(m_half <= x_limit)) != 0) {  // (NaN counts as above)
       asm volatile("");  // (two branches on purpose: merged into one condition, the second is computed in every step)
       // (a tile this wave's mask row does not ask for, or that is not this loop's, leaves the points alone)
       if (jn < n_main && mine_at(jn)) {
@@ -727,7 +736,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if constexpr (kTileSkip) nothing = __all(m_half < m_run - (kPShift + 11.0f));
   };
   look_ahead(0, lane_max(s_a), s_ks[0], alpha_even, moved_even);
-  moved_even = 0;  // nothing has been accumulated yet
+  moved_even = __any(alpha_even != alpha_even);  // nothing has been accumulated yet: only a NaN has anything to say
 
   // Software pipeline, one key tile per step.  While this tile's probabilities are computed on
   // the VALU, the matrix pipe runs the S^T MFMAs of the NEXT tile and the PV MFMAs of the
@@ -904,8 +913,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         const int key = j * kBlkK + 32 * t + 8 * (r >> 2) + 4 * hh + (r & 3);
         if (key >= lk) s_cur[t][r] = kMagicBits - (1 << 22);  // below every real score
       }
-    const float sc = qs * s_ks[jj];
-    const float mneg = -kMagicVal * sc;
+    float sc = qs * s_ks[jj];
+    float mneg = -kMagicVal * sc;
     scale_o(move_point(lane_max(s_cur), sc, mneg));
     const float c = x_base + mneg;
     const float scp = kPwlExp ? 8.0f * sc : sc;

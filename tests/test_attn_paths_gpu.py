@@ -113,3 +113,25 @@ def test_repeated_calls_give_the_same_bits(hip_device, waves, Lk):
     first = sage_ops.attn_fwd(ws, torch.empty_like(q), wg_waves=waves)
     for _ in range(40):
         assert torch.equal(sage_ops.attn_fwd(ws, torch.empty_like(q), wg_waves=waves), first)
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("Lk", [30, 64, 200, 64 * 12])
+@pytest.mark.parametrize("mode", ["exact", "pwl", "skip", "causal"])
+def test_query_rows_that_are_not_finite_stay_on_their_own(hip_device, waves, Lk, mode):
+    """Rows of q with an infinity in them (padding rows may hold anything) give NaN and leave every other row's bits alone."""
+    print(f"case waves={waves} Lk={Lk} {mode}", flush=True)
+    g = torch.Generator().manual_seed(Lk)
+    q, k, v = (torch.randn((1, n, 1, 128), generator=g).to(torch.bfloat16) for n in (100, Lk, Lk))
+    bad = torch.zeros(100, dtype=torch.bool)
+    bad[[0, 5, 37, 40, 99]] = True
+    outs = []
+    for value in (0.0, float("inf")):
+        q[0, bad, 0, 9] = value
+        qd, kd, vd = (t.to(hip_device) for t in (q, k, v))
+        ws = sage_ops.workspace_for(qd, kd)
+        sage_ops.quant_q(qd, ws, 128**-0.5), sage_ops.quant_k(kd, ws, True), sage_ops.quant_v(vd, ws)
+        outs.append(sage_ops.attn_fwd(ws, torch.empty_like(qd), wg_waves=waves, pwl_exp2=mode == "pwl", tile_skip=mode == "skip",
+                                      causal=mode == "causal").cpu()[0])
+    assert torch.isnan(outs[1][bad]).all()
+    assert torch.isfinite(outs[1][~bad]).all() and torch.equal(outs[0][~bad], outs[1][~bad])
