@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define KSANA_SAGE_ABI_VERSION 21
+#define KSANA_SAGE_ABI_VERSION 22
 
 /* element types of q/k/v/o */
 #define KSANA_SAGE_BF16 0
@@ -69,6 +69,11 @@ extern "C" {
                                      /* the reference passes 1e6, i.e. "never"), at a threshold where nothing changes.    */
                                      /* Off by default: the test per tile costs ~7 % where no tile qualifies (flat         */
                                      /* attention); it pays where attention is peaked.                                     */
+
+#define KSANA_SAGE_FLAG_Q_UNSTORED 32 /* ksana_sage_forward* only: the caller does not read q_i8 and q_scale from the       */
+                                      /* workspace afterwards and o does not overlap q.  Without a block mask and a step   */
+                                      /* folded into q, where o has its type and the sizes make it pay, the attention      */
+                                      /* kernel then quantizes Q itself and the two areas stay unwritten.  Same bits.      */
 
 typedef struct ksana_sage_shape {
   int32_t B;   /* batch                                                     */

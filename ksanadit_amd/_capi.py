@@ -11,7 +11,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libksana_sage_hip.so"
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 BF16, FP16 = 0, 1
 OK, EINVAL, ENOTSUP, EHIP = 0, -1, -2, -3
@@ -20,6 +20,7 @@ FLAG_SMOOTH_V = 2
 FLAG_WG_4_WAVES = 4
 FLAG_WG_8_WAVES = 8
 FLAG_TILE_SKIP = 16
+FLAG_Q_UNSTORED = 32
 PREP_WAN, PREP_WAN_COMFY, PREP_QWEN = 0, 1, 2
 KEEP = -(2**63)  # KSANA_SAGE_KEEP
 

@@ -81,7 +81,7 @@ class RadialSageAttentionImpl(KsanaAttentionBackendImpl):
                 latent_shape: list[int] | None = None, **kwargs) -> torch.Tensor:
         if dense_only or step_iter < self.dense_attn_steps or block_id < self.dense_blocks_num:
             return self.dense_attn(query, key, value, **kwargs)
-        lens = [] if k_lens is None else k_lens.tolist()  # (one copy to the host when it lives on the GPU)
+        lens = [] if k_lens is None else k_lens.reshape(len(k_lens)).tolist()  # (one copy to the host when it lives on the GPU)
         if not lens or any(n != lens[0] for n in lens):
             raise ValueError("k_lens must be the same for all tokens")
         video_token_num = int(lens[0])

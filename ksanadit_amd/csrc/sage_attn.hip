@@ -19,6 +19,7 @@
 // The int32 accumulators start at the bit pattern of 1.5 * 2^23 ("magic"): the result read
 // as fp32 IS 12582912 + dot exactly (|dot| <= 127*127*128 < 2^22), which removes the
 // int->float conversion from the softmax: p = exp2(fma(acc_as_float, sc, c)).
+#include "sage_device.h"
 #include "sage_kernels.h"
 
 #include <atomic>
@@ -164,6 +165,69 @@ __device__ __forceinline__ void qk_tile(const uint8_t* k_stage, int lane, const 
   }
 }
 
+// Q quantized where it is used.  Lane l of a wave holds the channels 32 s + 16 (l / 32) + 0 .. 15, s < kG, of the wave's row
+// l % 32 - those of its matrix operand - so the row's transform is strides 1 .. 8 inside sixteen channels, 16 between lanes
+// l and l ^ 32, 32 and 64 between the groups: the order, the roundings and therefore the bits of the separate quantizer
+// (fwht128, pack_int8x16).  Head size 64 (kG == 2): the upper half of an extended row repeats the lower, so stride 64 and
+// the row's other half change nothing.  Bound by its latency in the set-up (two or three waves' worth of instructions per
+// SIMD, all at once); what it saves is the quantizer's pass over Q, which is HBM-bound.  Whole calls, us, before / with it:
+// 32760 queries on 512 keys, 40 heads 373 / 336; padded batch (B=3, 24 heads, 3001 x 4099) 210 / 202; causal 8191, 32 heads
+// 352 / 345; 9001 tokens of 64 channels, B=2, 16 heads 563 / 557.  Which calls take it: q_in_attention_pays.
+template <int DT, int kG>
+__device__ __forceinline__ void quant_q_rows(const uint4 (&raw)[8], float premul, v4i (&qf)[4], float& qs) {
+  float x[kG][16];
+#pragma unroll
+  for (int s = 0; s < kG; ++s) {
+    widen8<DT>(raw[2 * s], x[s]);
+    widen8<DT>(raw[2 * s + 1], x[s] + 8);
+#pragma unroll
+    for (int st = 1; st < 16; st <<= 1)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if ((i & st) == 0) {
+          const float a = x[s][i], b = x[s][i + st];
+          x[s][i] = a + b;
+          x[s][i + st] = a - b;
+        }
+    // two values at a time: the first swap gives the lower lanes both ends of the first value's butterfly and the upper
+    // lanes both ends of the second's, the second swap takes the results home
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) {
+      const auto ab = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[s][i]), __float_as_uint(x[s][i + 1]), false, false);
+      const float a = __uint_as_float(ab[0]), b = __uint_as_float(ab[1]);
+      const auto home = __builtin_amdgcn_permlane32_swap(__float_as_uint(a + b), __float_as_uint(a - b), false, false);
+      x[s][i] = __uint_as_float(home[0]);
+      x[s][i + 1] = __uint_as_float(home[1]);
+    }
+  }
+#pragma unroll
+  for (int st = 1; st < kG; st <<= 1)
+#pragma unroll
+    for (int s = 0; s < kG; ++s)
+      if ((s & st) == 0)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float a = x[s][i], b = x[s + st][i];
+          x[s][i] = a + b;
+          x[s + st][i] = a - b;
+        }
+  float amax = 0.0f;
+#pragma unroll
+  for (int s = 0; s < kG; ++s)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      x[s][i] = x[s][i] * premul;
+      amax = fmaxf(amax, fabsf(x[s][i]));
+    }
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
+  amax = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+  const bool nz = amax > 0.0f;
+  const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
+  qs = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+#pragma unroll
+  for (int s = 0; s < kG; ++s) qf[s] = __builtin_bit_cast(v4i, pack_int8x16(x[s], inv));
+}
+
 // Dense 8-wave calls can hold two kinds of workgroup in one grid: blocks below p.split_first_block walk all key tiles of
 // their (head, query block); each of the blocks from there on takes one of `p.n_split` equal runs of key tiles and leaves
 // unnormalised accumulators, running maxima and row sums in the workspace for sage_attn_merge_kernel.  The runs stand
@@ -269,14 +333,29 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // ---- Q fragments (B operand), 4 channel steps --------------------------------------
   v4i qf[4];
   float qs = 0.0f;
-  if (active) {
+  uint4 q_raw[8];
+  // (not with a block mask: there such calls' key loops ran 1 % slower for the code being there)
+  constexpr bool kOwnQ = !kSparse || kCausal;
+  const bool own_q = kOwnQ && active && p.q_rows.ptr != nullptr;  // uniform per wave
+#pragma unroll
+  for (int s = 0; s < 4; ++s) qf[s] = v4i{0, 0, 0, 0};
+  if (own_q) {
+    // requested here, quantized once the first tiles are on their way
+    const int row = q0 + l32;
+    const uint16_t* qrow = p.q_rows.ptr + b * p.q_rows.sB + (int64_t)row * p.q_rows.sL + h * p.q_rows.sH + 16 * hh;
+#pragma unroll
+    for (int s = 0; s < kG; ++s) {
+      q_raw[2 * s] = q_raw[2 * s + 1] = make_uint4(0, 0, 0, 0);
+      if (row < p.Lq && 32 * s < p.q_rows.D) {
+        q_raw[2 * s] = *reinterpret_cast<const uint4*>(qrow + 32 * s);
+        q_raw[2 * s + 1] = *reinterpret_cast<const uint4*>(qrow + 32 * s + 8);
+      }
+    }
+  } else if (active) {
     const int8_t* qrow = p.q_i8 + ((int64_t)bh * p.lq_pad + q0 + l32) * kD + 16 * hh;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) qf[s] = s < kG ? *reinterpret_cast<const v4i*>(qrow + 32 * s) : v4i{0, 0, 0, 0};
+    for (int s = 0; s < kG; ++s) qf[s] = *reinterpret_cast<const v4i*>(qrow + 32 * s);
     qs = p.q_scale[(int64_t)bh * p.lq_pad + q0 + l32];  // one scale per query row = per lane
-  } else {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) qf[s] = v4i{0, 0, 0, 0};
   }
 
   v16f oacc[4];
@@ -589,6 +668,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
   for (int t = 0; t < (kLateCopies ? 2 : Shape::kAheadK); ++t) copy_half(k_src, t, k_slot(t));
   fill_scales();
+  if (own_q) quant_q_rows<DT, kG>(q_raw, p.q_premul, qf, qs);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the set-up's loads and, older than some of them, the copies
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if constexpr (kLateCopies) {
@@ -1176,6 +1256,17 @@ void plan_key_split(int n_wg, int nkb, int* first_wg, int* runs) {
   const DensePlan plan = plan_dense(n_wg, nkb);
   *first_wg = plan.first_cut, *runs = plan.runs;
 }
+
+// Quantized in the attention kernel, Q is read once (2 bytes per channel where the quantizer's pass moves 4 with its reading
+// back), for about 800 vector instructions per wave that its set-up then waits for, 2-3 us.  That pays
+//   from one full round of the chip: below it every workgroup's set-up is exposed, and the quantizer's Q blocks ride in
+//     the launches of K and V (us through memory / in the kernel: 256 blocks, 32 tiles 58.3 / 56.6; 128 blocks 41.0 / 42.1;
+//     16 blocks 32.2 / 34.8);
+//   beyond 256 keys: up to there all quantizers are one launch (256 blocks, 2 tiles 23.0 / 24.1; 8 tiles 33.1 / 30.0);
+//   up to 256 tiles: there the gain is half a per cent (2560 blocks: 8 tiles 195 / 178, 32 tiles 452 / 438, 128 tiles
+//     1477 / 1455, 256 tiles 2801 / 2786), and on chips at their power limit the instructions cost the key loop as much
+//     (512 tiles: 10337 / 10365).
+bool q_in_attention_pays(int n_wg, int nkb) { return n_wg >= compute_units() && nkb * kBlkK > kMeanChunk && nkb <= 256; }
 
 // Workgroup shape for a call: 4-wave workgroups (two per compute unit) when a block mask or causal masking is
 // involved (a workgroup is then one 128-row mask row, so no wave multiplies a tile only the neighbouring mask row

@@ -194,6 +194,13 @@ int check_causal(const ksana_sage_shape* s, int causal) {
   return 0;
 }
 
+// the factor a transformed row of Q takes before it is rounded to int8
+float q_premul_of(float sm_scale) { return (sm_scale * 1.4426950408889634f) * 0.0078125f; }
+
+int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
+              const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags,
+              const ksana_sage::InTensor* q_rows, float q_premul, void* stream);
+
 int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype, int o_dtype, const int64_t q_st[4],
                  const int64_t k_st[4], const int64_t v_st[4], const int64_t o_st[4], const ksana_sage_shape* s,
                  const ksana_sage_prep* prep, const int8_t* block_mask, const int64_t mask_st[2], const int32_t* q_lens,
@@ -372,7 +379,7 @@ static int quant_q_impl(const void* q, int dtype, const int64_t st[4], const ksa
     return rc;
   // one fp32 product, then an exact power of two (1/128 undoes the unnormalised Hadamard
   // transforms of Q and K): part of the quantizer specification
-  const float premul = (sm_scale * 1.4426950408889634f) * 0.0078125f;
+  const float premul = q_premul_of(sm_scale);
   if (ppp && ppp->inv_rms) {
     // a norm over the token row: statistic and quantization in one kernel that takes whole rows
     const bool take_k = k != nullptr && prep->k_norm_weight != nullptr && k_st[2] == ksana_sage::kD;
@@ -676,45 +683,7 @@ int ksana_sage_attn_fwd_masked(void* ws, void* o, int dtype, const int64_t o_st[
 int ksana_sage_attn_fwd_varlen(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s,
                                const int8_t* block_mask, const int64_t mask_st[2], const int32_t* q_lens,
                                const int32_t* k_lens, int causal, int flags, void* stream) {
-  const StageRange range("ksana_sage.attention");
-  if (int rc = check_shape(s)) return rc;
-  if (int rc = check_mask(s, block_mask, mask_st)) return rc;
-  if (int rc = check_causal(s, causal)) return rc;
-  if (flags & ~(KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES | KSANA_SAGE_FLAG_TILE_SKIP))
-    return fail(KSANA_SAGE_EINVAL, "unknown flag bits 0x%x", flags);
-  if ((flags & KSANA_SAGE_FLAG_TILE_SKIP) && (flags & KSANA_SAGE_FLAG_PWL_EXP2))
-    return fail(KSANA_SAGE_EINVAL, "KSANA_SAGE_FLAG_TILE_SKIP goes with the exact exponential only, not with KSANA_SAGE_FLAG_PWL_EXP2");
-  if (int rc = check_tensor("o", o, dtype, o_st, s->B, s->Lq, s->Hq)) return rc;
-  if (int rc = check_ws(ws)) return rc;
-  if (reinterpret_cast<uintptr_t>(k_lens) & 3) return fail(KSANA_SAGE_EINVAL, "k_lens is not 4-byte aligned");
-  if (reinterpret_cast<uintptr_t>(q_lens) & 3) return fail(KSANA_SAGE_EINVAL, "q_lens is not 4-byte aligned");
-  ksana_sage_ws_layout l;
-  ksana_sage_workspace_layout(s, &l);
-  ksana_sage::AttnParams p;
-  p.q_i8 = ws_at<int8_t>(ws, l.q_i8);
-  p.q_scale = ws_at<float>(ws, l.q_scale);
-  p.k_tiles = ws_at<int8_t>(ws, l.k_i8);
-  p.k_scale = ws_at<float>(ws, l.k_scale);
-  p.v_tiles = ws_at<uint8_t>(ws, l.v_fp8);
-  p.v_scale = ws_at<float>(ws, l.v_scale);
-  p.v_mean = ws_at<float>(ws, l.v_mean);
-  p.split_o = ws_at<float>(ws, l.split_o);
-  p.split_ml = ws_at<float>(ws, l.split_ml);
-  p.wg_waves = (flags & KSANA_SAGE_FLAG_WG_4_WAVES) ? 4 : ((flags & KSANA_SAGE_FLAG_WG_8_WAVES) ? 8 : 0);
-  p.o = ksana_sage::OutTensor{static_cast<uint16_t*>(o), o_st[0], o_st[1], o_st[2], dtype};
-  p.B = s->B, p.Hq = s->Hq, p.Hkv = s->Hkv, p.Lq = s->Lq, p.Lk = s->Lk;
-  p.lq_pad = l.lq_pad, p.nkb = l.nkb;
-  p.exact_exp2 = (flags & KSANA_SAGE_FLAG_PWL_EXP2) ? 0 : 1;
-  p.k_lens = k_lens;
-  p.q_lens = q_lens;
-  p.block_mask = block_mask;
-  p.mask_sB = block_mask ? mask_st[0] : 0;
-  p.mask_sH = block_mask ? mask_st[1] : 0;
-  p.causal = causal ? 1 : 0;
-  p.d_out = s->D;
-  p.tile_skip = (flags & KSANA_SAGE_FLAG_TILE_SKIP) ? 1 : 0;
-  hipError_t e = ksana_sage::launch_attn_fwd(p, static_cast<hipStream_t>(stream));
-  return e == hipSuccess ? 0 : hip_fail(e, "attention launch");
+  return attn_impl(ws, o, dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, flags, nullptr, 0.0f, stream);
 }
 
 int ksana_sage_forward(const void* q, const void* k, const void* v, void* o, int dtype, const int64_t q_st[4],
@@ -755,8 +724,54 @@ int ksana_sage_forward_varlen(const void* q, const void* k, const void* v, void*
 }  // extern "C"
 
 namespace {
-// All three quantizers of a call whose arguments have been validated
-int quant_qkv(const void* q, const void* k, const void* v, int dtype, const int64_t q_st[4], const int64_t k_st[4],
+// q_rows: nullptr, or Q as the caller has it (validated, of the result's dtype) for the kernel to quantize
+int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
+              const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags,
+              const ksana_sage::InTensor* q_rows, float q_premul, void* stream) {
+  const StageRange range("ksana_sage.attention");
+  if (int rc = check_shape(s)) return rc;
+  if (int rc = check_mask(s, block_mask, mask_st)) return rc;
+  if (int rc = check_causal(s, causal)) return rc;
+  if (flags & ~(KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES | KSANA_SAGE_FLAG_TILE_SKIP))
+    return fail(KSANA_SAGE_EINVAL, "unknown flag bits 0x%x", flags);
+  if ((flags & KSANA_SAGE_FLAG_TILE_SKIP) && (flags & KSANA_SAGE_FLAG_PWL_EXP2))
+    return fail(KSANA_SAGE_EINVAL, "KSANA_SAGE_FLAG_TILE_SKIP goes with the exact exponential only, not with KSANA_SAGE_FLAG_PWL_EXP2");
+  if (int rc = check_tensor("o", o, dtype, o_st, s->B, s->Lq, s->Hq)) return rc;
+  if (int rc = check_ws(ws)) return rc;
+  if (reinterpret_cast<uintptr_t>(k_lens) & 3) return fail(KSANA_SAGE_EINVAL, "k_lens is not 4-byte aligned");
+  if (reinterpret_cast<uintptr_t>(q_lens) & 3) return fail(KSANA_SAGE_EINVAL, "q_lens is not 4-byte aligned");
+  ksana_sage_ws_layout l;
+  ksana_sage_workspace_layout(s, &l);
+  ksana_sage::AttnParams p;
+  if (q_rows != nullptr) p.q_rows = *q_rows, p.q_premul = q_premul;
+  p.q_i8 = ws_at<int8_t>(ws, l.q_i8);
+  p.q_scale = ws_at<float>(ws, l.q_scale);
+  p.k_tiles = ws_at<int8_t>(ws, l.k_i8);
+  p.k_scale = ws_at<float>(ws, l.k_scale);
+  p.v_tiles = ws_at<uint8_t>(ws, l.v_fp8);
+  p.v_scale = ws_at<float>(ws, l.v_scale);
+  p.v_mean = ws_at<float>(ws, l.v_mean);
+  p.split_o = ws_at<float>(ws, l.split_o);
+  p.split_ml = ws_at<float>(ws, l.split_ml);
+  p.wg_waves = (flags & KSANA_SAGE_FLAG_WG_4_WAVES) ? 4 : ((flags & KSANA_SAGE_FLAG_WG_8_WAVES) ? 8 : 0);
+  p.o = ksana_sage::OutTensor{static_cast<uint16_t*>(o), o_st[0], o_st[1], o_st[2], dtype};
+  p.B = s->B, p.Hq = s->Hq, p.Hkv = s->Hkv, p.Lq = s->Lq, p.Lk = s->Lk;
+  p.lq_pad = l.lq_pad, p.nkb = l.nkb;
+  p.exact_exp2 = (flags & KSANA_SAGE_FLAG_PWL_EXP2) ? 0 : 1;
+  p.k_lens = k_lens;
+  p.q_lens = q_lens;
+  p.block_mask = block_mask;
+  p.mask_sB = block_mask ? mask_st[0] : 0;
+  p.mask_sH = block_mask ? mask_st[1] : 0;
+  p.causal = causal ? 1 : 0;
+  p.d_out = s->D;
+  p.tile_skip = (flags & KSANA_SAGE_FLAG_TILE_SKIP) ? 1 : 0;
+  hipError_t e = ksana_sage::launch_attn_fwd(p, static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? 0 : hip_fail(e, "attention launch");
+}
+
+// The quantizers of a call whose arguments have been validated: of Q, K and V, or (with_q == false, no prep) of K and V
+int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtype, const int64_t q_st[4], const int64_t k_st[4],
               const int64_t v_st[4], const ksana_sage_shape* s, const ksana_sage_prep* prep, float sm_scale, int smooth_k,
               int smooth_v, void* ws, void* stream) {
   if (!smooth_v) {
@@ -772,7 +787,8 @@ int quant_qkv(const void* q, const void* k, const void* v, int dtype, const int6
     ksana_sage::QkvCall c{};
     c.q = in_tensor(q, dtype, q_st, s->D), c.k = in_tensor(k, dtype, k_st, s->D), c.v = in_tensor(v, dtype, v_st, s->D);
     c.B = s->B, c.Hq = s->Hq, c.Hkv = s->Hkv, c.Lq = s->Lq, c.Lk = s->Lk, c.lq_pad = l.lq_pad, c.nkb = l.nkb, c.nch = l.nch;
-    c.premul = (sm_scale * 1.4426950408889634f) * 0.0078125f;  // (as in quant_q_impl)
+    c.nqb = with_q ? l.lq_pad / ksana_sage::kQPad : 0;
+    c.premul = q_premul_of(sm_scale);
     c.smooth_k = smooth_k ? 1 : 0;
     c.q_i8 = ws_at<int8_t>(ws, l.q_i8), c.q_scale = ws_at<float>(ws, l.q_scale);
     c.k_part = ws_at<float>(ws, l.k_part), c.k_mean = ws_at<float>(ws, l.k_mean);
@@ -786,7 +802,11 @@ int quant_qkv(const void* q, const void* k, const void* v, int dtype, const int6
     if (e != hipSuccess) return hip_fail(e, "q, k, v quantizer launch");
     if (used) return 0;
   }
-  if (int rc = ksana_sage_quant_qk_prep(q, k, dtype, q_st, k_st, s, prep, sm_scale, smooth_k, ws, stream)) return rc;
+  if (!with_q) {
+    if (int rc = ksana_sage_quant_k(k, dtype, k_st, s, smooth_k, ws, stream)) return rc;
+  } else if (int rc = ksana_sage_quant_qk_prep(q, k, dtype, q_st, k_st, s, prep, sm_scale, smooth_k, ws, stream)) {
+    return rc;
+  }
   return ksana_sage_quant_v_smooth(v, dtype, v_st, s, smooth_v, ws, stream);
 }
 
@@ -804,7 +824,7 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
   if (int rc = check_tensor("o", o, o_dtype, o_st, s->B, s->Lq, s->Hq)) return rc;
   if (int rc = check_ws(ws)) return rc;
   if (flags & ~(KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_SMOOTH_V | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES |
-                KSANA_SAGE_FLAG_TILE_SKIP))
+                KSANA_SAGE_FLAG_TILE_SKIP | KSANA_SAGE_FLAG_Q_UNSTORED))
     return fail(KSANA_SAGE_EINVAL, "unknown flag bits 0x%x", flags);
   if ((flags & KSANA_SAGE_FLAG_TILE_SKIP) && (flags & KSANA_SAGE_FLAG_PWL_EXP2))
     return fail(KSANA_SAGE_EINVAL, "KSANA_SAGE_FLAG_TILE_SKIP goes with the exact exponential only, not with KSANA_SAGE_FLAG_PWL_EXP2");
@@ -819,9 +839,15 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
     if (int rc = make_prep(prep, prep ? prep->k_norm_weight : nullptr, "k", k_st, s->B, s->Lk, s->D, &dummy, &pp, &ppp))
       return rc;
   }
-  if (int rc = quant_qkv(q, k, v, dtype, q_st, k_st, v_st, s, prep, sm_scale, smooth_k, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws, stream))
+  const int n_wg = s->B * s->Hq * ((s->Lq + ksana_sage::kAttnQPerWg - 1) / ksana_sage::kAttnQPerWg);
+  const bool own_q = (flags & KSANA_SAGE_FLAG_Q_UNSTORED) && prep == nullptr && block_mask == nullptr && o_dtype == dtype &&
+                     ksana_sage::q_in_attention_pays(n_wg, (s->Lk + ksana_sage::kBlkK - 1) / ksana_sage::kBlkK);
+  if (int rc = quant_qkv(!own_q, q, k, v, dtype, q_st, k_st, v_st, s, prep, sm_scale, smooth_k, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws,
+                         stream))
     return rc;
-  return ksana_sage_attn_fwd_varlen(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal,
-                                    flags & ~KSANA_SAGE_FLAG_SMOOTH_V, stream);
+  const ksana_sage::InTensor q_rows = in_tensor(q, dtype, q_st, s->D);
+  return attn_impl(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal,
+                   flags & ~(KSANA_SAGE_FLAG_SMOOTH_V | KSANA_SAGE_FLAG_Q_UNSTORED), own_q ? &q_rows : nullptr, q_premul_of(sm_scale),
+                   stream);
 }
 }  // namespace

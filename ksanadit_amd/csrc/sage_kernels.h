@@ -133,6 +133,7 @@ int selftest_occupancy_cache();
 struct QkvCall {
   InTensor q, k, v;
   int B, Hq, Hkv, Lq, Lk, lq_pad, nkb, nch;
+  int nqb;  // blocks of kQPad query rows per head, or 0: the attention kernel quantizes Q (AttnParams::q_rows)
   float premul;
   int smooth_k;
   int8_t* q_i8;
@@ -177,6 +178,10 @@ hipError_t launch_sla_block_map(const uint16_t* pooled_q, const uint16_t* pooled
                                 int8_t* block_map, hipStream_t s);
 
 struct AttnParams {
+  // q_rows.ptr != nullptr: Q as the caller has it (of the result's dtype); every wave quantizes its own rows, q_i8 and q_scale
+  // are not read
+  InTensor q_rows{};
+  float q_premul = 0.0f;
   const int8_t* q_i8;
   const float* q_scale;
   const int8_t* k_tiles;
@@ -213,5 +218,7 @@ hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t s);
 // Which of `n_wg` dense workgroups the launcher cuts into runs of key tiles on the current device, and into how
 // many: workgroups [*first_wg, n_wg) into *runs each; *runs == 0 means none.
 void plan_key_split(int n_wg, int nkb, int* first_wg, int* runs);
+// Is a call with `n_wg` 256-row query blocks and `nkb` key tiles faster when the attention kernel quantizes Q itself?
+bool q_in_attention_pays(int n_wg, int nkb);
 
 }  // namespace ksana_sage

@@ -6,6 +6,7 @@
 //
 // The arithmetic is fixed to the last bit (it is compared bit-exactly with a PyTorch
 // specification): plain IEEE fp32 add / sub / mul / div, round-half-even, no contraction.
+#include "sage_device.h"
 #include "sage_kernels.h"
 
 #include <cstdlib>
@@ -19,23 +20,6 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kSlots = 32;  // row slots per workgroup
-
-template <int DT>
-__device__ __forceinline__ void widen8(const uint4& raw, float* out) {
-  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if constexpr (DT == KSANA_SAGE_BF16) {
-      out[2 * i] = __uint_as_float(w[i] << 16);
-      out[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
-    } else {
-      typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-      h2 p = __builtin_bit_cast(h2, w[i]);
-      out[2 * i] = (float)p[0];
-      out[2 * i + 1] = (float)p[1];
-    }
-  }
-}
 
 // 16 channels of one row; rows at or beyond L read as zero.
 template <int DT>
@@ -657,24 +641,6 @@ __device__ __forceinline__ float block_max(float v, float* s_red) {
   if ((threadIdx.x & 63) == 0) s_red[wave] = v;
   __syncthreads();
   return fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-}
-
-// rne(x * inv) as int8, sixteen at a time, the product exact: one fused multiply-add onto 1.5 * 2^23, where the fp32
-// grid is the integers, rounds the exact sum to nearest, ties to even, and leaves the two's-complement int8 in the low
-// byte.  No clamp: |x| <= amax and inv = fl(127 / amax) keep |x * inv| below 127.5.  One instruction per value plus
-// three byte-gathers per four.
-__device__ __forceinline__ uint4 pack_int8x16(const float* x, float inv) {
-  uint32_t w[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    uint32_t z[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) z[j] = __float_as_uint(__fmaf_rn(x[4 * i + j], inv, 12582912.0f));
-    const uint32_t lo = __builtin_amdgcn_perm(z[1], z[0], 0x0c0c0400u);  // bytes 0, 1 <- low bytes of z0, z1
-    const uint32_t hi = __builtin_amdgcn_perm(z[3], z[2], 0x04000c0cu);  // bytes 2, 3 <- low bytes of z2, z3
-    w[i] = lo | hi;
-  }
-  return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
 // Block mean from per-thread partial sums (thread = row slot x 16 channels; a slot has added its rows in increasing
@@ -1723,8 +1689,8 @@ __device__ __forceinline__ void clear_status(const QkvCall& c) {
 
 template <int DT, int KIND>
 __device__ __forceinline__ void quant_q_item(int item, const QkvCall& c, const PrepParams& pp) {
-  const int nqb = c.lq_pad / kQPad, bh = item / nqb;
-  quant_q_block<DT, KIND, false>(item - bh * nqb, bh % c.Hq, bh / c.Hq, c.q.ptr, c.q.sB, c.q.sL, c.q.sH, c.Hq, c.Lq, c.q.D, c.lq_pad,
+  const int bh = item / c.nqb;
+  quant_q_block<DT, KIND, false>(item - bh * c.nqb, bh % c.Hq, bh / c.Hq, c.q.ptr, c.q.sB, c.q.sL, c.q.sH, c.Hq, c.Lq, c.q.D, c.lq_pad,
                                  c.premul, c.q_i8, c.q_scale, pp, nullptr);
 }
 
@@ -1780,7 +1746,7 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 6 : 5) void quant_qkv_stage2_
 template <int DT, int KIND>
 __global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk,
                                                                      const HeadSync sk, const HeadSync sv) {
-  const int nqb = c.lq_pad / kQPad, group = c.Hq / c.Hkv, per_head = 2 * c.nch + group * nqb;
+  const int group = c.Hq / c.Hkv, per_head = 2 * c.nch + group * c.nqb;
   const int bh = blockIdx.x / per_head;
   int item = blockIdx.x - bh * per_head;
   if (item < c.nch) {
@@ -1796,8 +1762,8 @@ __global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCa
   }
   item -= c.nch;
   const int b = bh / c.Hkv, hk = bh - b * c.Hkv;
-  const int hq = hk * group + item / nqb;
-  quant_q_item<DT, KIND>((b * c.Hq + hq) * nqb + item % nqb, c, pq);
+  const int hq = hk * group + item / c.nqb;
+  quant_q_item<DT, KIND>((b * c.Hq + hq) * c.nqb + item % c.nqb, c, pq);
 }
 
 // at most 256 keys: one launch
@@ -2244,7 +2210,7 @@ constexpr int kMeetMaxChunks = 160;
 template <int DT, int KIND>
 static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepParams& pk, hipStream_t s, bool* used) {
   const dim3 block(kThreads);
-  const int64_t n_q = (int64_t)c.B * c.Hq * (c.lq_pad / kQPad), n_chunks = (int64_t)c.B * c.Hkv * c.nch;
+  const int64_t n_q = (int64_t)c.B * c.Hq * c.nqb, n_chunks = (int64_t)c.B * c.Hkv * c.nch;
   if (c.nch == 1) {
     quant_qkv_small_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, pq, pk);
     *used = true;
@@ -2278,7 +2244,7 @@ hipError_t launch_quant_qkv(const QkvCall& call, const PrepParams* pq, const Pre
   QkvCall c = call;
   const int kind = pq != nullptr ? pq->kind : (pk != nullptr ? pk->kind : 0);
   if (kind != 0 && kind != 2) return hipSuccess;
-  if ((int64_t)c.B * c.Hq * (c.lq_pad / kQPad) + 2 * (int64_t)c.B * c.Hkv * c.nkb > INT32_MAX) return hipSuccess;
+  if ((int64_t)c.B * c.Hq * c.nqb + 2 * (int64_t)c.B * c.Hkv * c.nkb > INT32_MAX) return hipSuccess;
   // (a side without anything to apply runs with every step of its parameters switched off)
   PrepParams off{};
   off.kind = kind;

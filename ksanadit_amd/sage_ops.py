@@ -723,12 +723,13 @@ def sageattn(
         raise ValueError("prep needs the NHD layout (a token row must be contiguous)")
     B, Lq, Hq, D = plan.out_shape
     device = plan.device
+    if not plan.runs:  # nothing to attend from: same empty result SDPA gives
+        out = torch.empty(plan.out_shape, dtype=plan.dtype, device=device)
+        return out.transpose(1, 2) if hnd else out
     result_dtype = plan.dtype if out_dtype is None else out_dtype
     if result_dtype not in _DTYPES:
         raise ValueError(f"out_dtype must be float16 or bfloat16, got {out_dtype}")
     out = torch.empty(plan.out_shape, dtype=result_dtype, device=device)
-    if not plan.runs:  # nothing to attend from: same empty result SDPA gives
-        return out.transpose(1, 2) if hnd else out
     sm_scale = D**-0.5 if sm_scale is None else float(sm_scale)
     if workspace is None:
         blob = torch.empty(plan.ws_bytes, dtype=torch.uint8, device=device)  # (torch's blocks start at multiples of 512)
@@ -743,6 +744,7 @@ def sageattn(
     ql = None if q_lens is None else _k_lens_arg(q_lens, B, device, "q_lens")
     flags = (_capi.FLAG_PWL_EXP2 if pwl_exp2 else 0) | (_capi.FLAG_SMOOTH_V if smooth_v else 0)
     flags |= _capi.FLAG_TILE_SKIP if tile_skip else 0
+    flags |= _capi.FLAG_Q_UNSTORED if workspace is None else 0  # nobody sees the workspace after the call
     prep_ptr = mask_ptr = mask_st = None
     if prep is not None:
         if block_mask is not None and q_lens is None and result_dtype == plan.dtype:
