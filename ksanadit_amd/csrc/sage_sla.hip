@@ -234,18 +234,38 @@ __global__ __launch_bounds__(kSlaThreads) void sla_kv_finalize_kernel(const floa
                                                                       uint16_t* __restrict__ m_frag,
                                                                       float* __restrict__ ksum) {
   const int bh = blockIdx.y, d0 = blockIdx.x * kFinRows, t = threadIdx.x;
-  __shared__ float s_kv[kFinRows * kD];
+  __shared__ __attribute__((aligned(16))) float s_kv[kFinRows * kD];
   const float* p = part + (int64_t)bh * runs * kSlaPartFloats;
-  for (int idx = t; idx < kFinRows * kD; idx += kSlaThreads) {
-    float a = 0.0f;
-    for (int r = 0; r < runs; ++r) a = r == 0 ? p[d0 * kD + idx] : a + p[(int64_t)r * kSlaPartFloats + d0 * kD + idx];
-    s_kv[idx] = round_half<DT>(a);
+  // Bound by latency: the runs are added in order, but read four at a time, both of the thread's quadruples together (one
+  // value of one run at a time, 12 runs were 96 memory latencies one after the other: 40 heads 39 -> 16 us).
+  constexpr int kQuads = kFinRows * kD / 4 / kSlaThreads, kAtOnce = 4;
+  float4 sum[kQuads];
+#pragma unroll
+  for (int i = 0; i < kQuads; ++i) sum[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  float sum1 = 0.0f;
+  for (int r0 = 0; r0 < runs; r0 += kAtOnce) {
+    float4 x[kAtOnce][kQuads];
+    float y[kAtOnce];
+#pragma unroll
+    for (int c = 0; c < kAtOnce; ++c) {
+      const float* pr = p + (int64_t)min(r0 + c, runs - 1) * kSlaPartFloats;
+#pragma unroll
+      for (int i = 0; i < kQuads; ++i) x[c][i] = *reinterpret_cast<const float4*>(pr + d0 * kD + 4 * (i * kSlaThreads + t));
+      y[c] = pr[kD * kD + d0 + (t & (kFinRows - 1))];
+    }
+#pragma unroll
+    for (int c = 0; c < kAtOnce; ++c) {
+      if (r0 + c >= runs) break;  // uniform
+#pragma unroll
+      for (int i = 0; i < kQuads; ++i) sum[i].x += x[c][i].x, sum[i].y += x[c][i].y, sum[i].z += x[c][i].z, sum[i].w += x[c][i].w;
+      sum1 += y[c];
+    }
   }
-  if (t < kFinRows) {
-    float a = 0.0f;
-    for (int r = 0; r < runs; ++r) a = r == 0 ? p[kD * kD + d0 + t] : a + p[(int64_t)r * kSlaPartFloats + kD * kD + d0 + t];
-    ksum[bh * kD + d0 + t] = round_half<DT>(a);
-  }
+#pragma unroll
+  for (int i = 0; i < kQuads; ++i)
+    *reinterpret_cast<float4*>(s_kv + 4 * (i * kSlaThreads + t)) =
+        make_float4(round_half<DT>(sum[i].x), round_half<DT>(sum[i].y), round_half<DT>(sum[i].z), round_half<DT>(sum[i].w));
+  if (t < kFinRows) ksum[bh * kD + d0 + t] = round_half<DT>(sum1);
   __syncthreads();
   // thread t: output column n = t % 128 for the rows d0 + (t / 128), d0 + (t / 128) + 2, ...
   const int n = t & (kD - 1);
@@ -254,6 +274,7 @@ __global__ __launch_bounds__(kSlaThreads) void sla_kv_finalize_kernel(const floa
 #pragma unroll
     for (int i = 0; i < kFinRows / 2; ++i) m[i] = 0.0f;
     const float4* wr = reinterpret_cast<const float4*>(proj_w + n * kD);  // W[n][c]
+#pragma unroll 8
     for (int c4 = 0; c4 < kD / 4; ++c4) {
       const float4 wv = wr[c4];
 #pragma unroll
@@ -419,18 +440,23 @@ __global__ __launch_bounds__(kSlaThreads, 2) void sla_apply_kernel(const uint16_
 // The block map from the pooled blocks (get_block_map, sage_sla.py:83-90): score = pooled_q pooled_k^T as a tensor of
 // the half type (fp32 accumulation, one rounding), then for every query block the `keep` key blocks with the largest
 // scores get a one, the others a zero; of equal scores the lower index wins (what a stable descending sort gives;
-// torch.topk leaves it open).  grid = (ceil(nq / 32), B * H), 256 threads; dynamic LDS 32 * nk_pad * 2 bytes.
+// torch.topk leaves it open).  grid = (ceil(nq / 32), B * H), 1024 threads; dynamic LDS 32 * nk_pad * 2 bytes.
+//
+// Bound by the length of the selection, a chain of counts: hence sixteen waves with two query blocks each, not four with
+// eight, and registers for 512 key blocks where there are no more (40 heads of 256 x 512 blocks: 59 -> 37 us).
 //
 // Scores: 32 query blocks x 32 key blocks per 32x32x16 matrix instruction, contraction over the 128 channels - both
-// operands are 16-byte pieces of pooled rows as they lie in memory; wave w takes the key tiles w, w + 4, ...  Each
-// score goes to LDS as a 16-bit key whose unsigned order is the order of the values.  Selection, one wave per 8 query
+// operands are 16-byte pieces of pooled rows as they lie in memory; wave w takes the key tiles w, w + 16, ...  Each
+// score goes to LDS as a 16-bit key whose unsigned order is the order of the values.  Selection, one wave per 2 query
 // blocks: the keep-th largest key by bisection over its 16 bits (count of keys >= candidate by ballots), then ones for
 // the keys above it and for as many of its equals, lowest index first, as are still missing.
 // ---------------------------------------------------------------------------------------------------------------
 constexpr int kMapMaxKeyBlocks = 1024;
+constexpr int kMapThreads = 1024, kMapWaves = kMapThreads / 64;
 
-template <int DT>
-__global__ __launch_bounds__(kSlaThreads) void sla_block_map_kernel(const uint16_t* __restrict__ pooled_q,
+// kPerLane: 64 * kPerLane key blocks at most
+template <int DT, int kPerLane>
+__global__ __launch_bounds__(kMapThreads) void sla_block_map_kernel(const uint16_t* __restrict__ pooled_q,
                                                                     const uint16_t* __restrict__ pooled_k, int nq, int nk,
                                                                     int nk_pad, int keep, int8_t* __restrict__ block_map) {
   extern __shared__ __attribute__((aligned(16))) uint8_t s_dyn[];
@@ -444,7 +470,7 @@ __global__ __launch_bounds__(kSlaThreads) void sla_block_map_kernel(const uint16
   uint4 a[8];
 #pragma unroll
   for (int s = 0; s < 8; ++s) a[s] = q0 + l32 < nq ? *reinterpret_cast<const uint4*>(pq + 16 * s) : make_uint4(0, 0, 0, 0);
-  for (int nt = w; nt * 32 < nk_pad; nt += 4) {
+  for (int nt = w; nt * 32 < nk_pad; nt += kMapWaves) {
     const int kb = nt * 32 + l32;
     uint4 b[8];
 #pragma unroll
@@ -469,9 +495,9 @@ __global__ __launch_bounds__(kSlaThreads) void sla_block_map_kernel(const uint16
   }
   __syncthreads();
   // a row's keys in registers: lane holds the keys lane + 64 i (0, the padding value, beyond nk)
-  constexpr int kPerLane = kMapMaxKeyBlocks / 64;
-  for (int mi = 0; mi < 8; ++mi) {
-    const int m = 8 * w + mi;
+  constexpr int kRowsPerWave = 32 / kMapWaves;
+  for (int mi = 0; mi < kRowsPerWave; ++mi) {
+    const int m = kRowsPerWave * w + mi;
     if (q0 + m >= nq) break;  // wave-uniform
     const uint16_t* row = s_key + m * nk_pad;
     int8_t* out = block_map + ((int64_t)bh * nq + q0 + m) * nk;
@@ -569,12 +595,20 @@ hipError_t launch_sla_block_map(const uint16_t* pooled_q, const uint16_t* pooled
                                 int8_t* block_map, hipStream_t s) {
   if (nk > kMapMaxKeyBlocks) return hipErrorInvalidValue;
   const int nk_pad = (nk + 31) / 32 * 32;
-  const dim3 grid((nq + 31) / 32, BH), block(kSlaThreads);
+  const dim3 grid((nq + 31) / 32, BH), block(kMapThreads);
   const size_t lds = (size_t)32 * nk_pad * 2;
-  if (dtype == KSANA_SAGE_BF16)
-    sla_block_map_kernel<KSANA_SAGE_BF16><<<grid, block, lds, s>>>(pooled_q, pooled_k, nq, nk, nk_pad, keep, block_map);
-  else
-    sla_block_map_kernel<KSANA_SAGE_FP16><<<grid, block, lds, s>>>(pooled_q, pooled_k, nq, nk, nk_pad, keep, block_map);
+  const bool bf16 = dtype == KSANA_SAGE_BF16;
+  constexpr int kAll = kMapMaxKeyBlocks / 64;
+  if (nk <= 512) {
+    if (bf16)
+      sla_block_map_kernel<KSANA_SAGE_BF16, 8><<<grid, block, lds, s>>>(pooled_q, pooled_k, nq, nk, nk_pad, keep, block_map);
+    else
+      sla_block_map_kernel<KSANA_SAGE_FP16, 8><<<grid, block, lds, s>>>(pooled_q, pooled_k, nq, nk, nk_pad, keep, block_map);
+  } else if (bf16) {
+    sla_block_map_kernel<KSANA_SAGE_BF16, kAll><<<grid, block, lds, s>>>(pooled_q, pooled_k, nq, nk, nk_pad, keep, block_map);
+  } else {
+    sla_block_map_kernel<KSANA_SAGE_FP16, kAll><<<grid, block, lds, s>>>(pooled_q, pooled_k, nq, nk, nk_pad, keep, block_map);
+  }
   return hipGetLastError();
 }
 }  // namespace ksana_sage
