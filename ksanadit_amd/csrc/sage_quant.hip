@@ -1627,11 +1627,12 @@ __global__ __launch_bounds__(kThreads) void quant_v_fused_kernel(const uint16_t*
 //            workgroup forming its head's statistic from the chunks' by itself (the same operations in the same order as
 //            the finalisation kernels).  Stage 2 reads its inputs a second time - out of the caches while K and V fit
 //            them - and nch * 512 bytes of partial results per workgroup.
-//   meet     one launch, every input read once: K's and V's chunks meet per head as in the one-read kernels above.
+//   meet     one launch, every input read once: K's and V's chunks meet per head as in the one-read kernels above.  Calls
+//            with a step folded in do not take it (see launch_qkv_kind).
 //
 // Measured, all quantizer launches of a call, us (separate quantizers / this):  B=2, 64 heads, 32 tokens 27 / 8 small;
-// 40 heads, 1560 tokens 43 / 22 stages; 9000 tokens 107 stages, 113 meet; 14000 tokens 201 stages, 169 meet; 32760
-// tokens 398 / 383 meet (HBM-bound: 9 bytes per element at 4 TB/s).
+// 40 heads, 1560 tokens 43 / 22 stages; 9000 tokens 120 / 106 stages; 14000 tokens 184 / 158 meet; 32760 tokens 392 / 369
+// meet (HBM-bound: 9 bytes per element at 4 TB/s).
 // ---------------------------------------------------------------------------------------
 template <int OP>  // 0: K's mean (ordered sum), 1: V's factor 448 / amax
 __device__ __forceinline__ void head_statistic(const QkvCall& c, int bh, bool publish, float (*s_stat)[kD]) {
@@ -1743,15 +1744,15 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 6 : 5) void quant_qkv_stage2_
 // One launch over inputs that are read once: the chunks of K and V meet per head as in the one-read kernels above, and
 // the items of a head - its K chunks, its V chunks, the Q blocks of its query heads - are neighbours in the grid, so the
 // Q blocks (which wait for nobody) and the V chunks work while K's chunks wait for their mean.
-template <int DT, int KIND>
-__global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk,
-                                                                     const HeadSync sk, const HeadSync sv) {
+template <int DT>
+__global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCall c, const HeadSync sk, const HeadSync sv) {
+  const PrepParams none{};
   const int group = c.Hq / c.Hkv, per_head = 2 * c.nch + group * c.nqb;
   const int bh = blockIdx.x / per_head;
   int item = blockIdx.x - bh * per_head;
   if (item < c.nch) {
-    quant_k_chunk<DT, KIND, false>(bh, item, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.nkb, c.nch, c.k_part, c.k_mean,
-                                   c.k.dtype, c.smooth_k, c.k_tiles, c.k_scale, pk, sk);
+    quant_k_chunk<DT, 0, false>(bh, item, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.nkb, c.nch, c.k_part, c.k_mean,
+                                c.k.dtype, c.smooth_k, c.k_tiles, c.k_scale, none, sk);
     return;
   }
   item -= c.nch;
@@ -1763,7 +1764,7 @@ __global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCa
   item -= c.nch;
   const int b = bh / c.Hkv, hk = bh - b * c.Hkv;
   const int hq = hk * group + item / c.nqb;
-  quant_q_item<DT, KIND>((b * c.Hq + hq) * c.nqb + item % c.nqb, c, pq);
+  quant_q_item<DT, 0>((b * c.Hq + hq) * c.nqb + item % c.nqb, c, none);
 }
 
 // at most 256 keys: one launch
@@ -2199,22 +2200,32 @@ hipError_t launch_quant_v_fused(const InTensor& v, int B, int H, int L, int nkb,
 }
 
 // Two stages while a head's partial results stay small next to the rows a workgroup of stage 2 quantizes (64 chunks are
-// 32 KiB, the rows 16-64 KiB) and the second reading of K and V comes from the last-level cache (256 MB): 40 heads of
-// 9000 tokens (184 MB of K and V) take 107 us in two stages and 113 in one meeting launch, 14000 tokens 201 and 169.
+// 32 KiB, the rows 16-64 KiB) and the second reading of K and V comes from the last-level cache (256 MB).  Beyond that
+// calls without a folded step take the meeting launch.  us, stages / meeting / separate kernels:
+//   40 heads of 9000 tokens (176 MB of K and V) 106 / 108 / 120; 24 heads of 17000 (199 MB) 125 / 122 / 135, two entries of
+//   8500 122 / 117 / 131; 40 heads of 14000 (273 MB) 192 / 158 / 184; 8 heads of 20000 (78 MB, 79 chunks) 46 / 49 / 56.
 constexpr int kStageMaxChunks = 64;
 constexpr int64_t kStageMaxBytes = 192ll << 20;
+// With the joint block's step stage 2 norms and rotates K once more, and loses its lead earlier; beyond the limit these calls
+// take the separate kernels (K from one read, the step done once).  24 heads, us, stages / separate: one entry of 13000
+// tokens (152 MB) 166 / 175, of 14000 (164 MB) 190 / 186, of 16000 (188 MB) 225 / 205; two of 6500 (152 MB) 159 / 169, of
+// 7000 (164 MB) 183 / 176, of 8056 (189 MB) 210 / 190; four of 3500 (164 MB) 177 / 173.  A meeting launch with the step in it
+// is no gain over them: meeting / separate 188 / 186 and 212 / 205 for the 14000 and 16000 tokens, two entries of 10256 263 /
+// 253, of 16896 414 / 411, one of 16896 219 / 229, of 20512 269 / 270, of 30512 392 / 371, of 40512 512 / 539.
+constexpr int64_t kStageMaxBytesJoint = 160ll << 20;
 // Beyond this many chunks a head's first workgroups wait for its last ones longer than a second pass takes (296 chunks:
 // the separate quantizers are 3 % faster).
 constexpr int kMeetMaxChunks = 160;
 
 template <int DT, int KIND>
 static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepParams& pk, hipStream_t s, bool* used) {
+  static_assert(KIND == 0 || KIND == 2, "nothing folded in, or the joint block's step");
   const dim3 block(kThreads);
   const int64_t n_q = (int64_t)c.B * c.Hq * c.nqb, n_chunks = (int64_t)c.B * c.Hkv * c.nch;
   if (c.nch == 1) {
     quant_qkv_small_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, pq, pk);
     *used = true;
-  } else if (c.nch <= kStageMaxChunks && 4 * (int64_t)c.B * c.Hkv * c.Lk * c.k.D <= kStageMaxBytes) {
+  } else if (c.nch <= kStageMaxChunks && 4 * (int64_t)c.B * c.Hkv * c.Lk * c.k.D <= (KIND == 0 ? kStageMaxBytes : kStageMaxBytesJoint)) {
     // about four workgroups per compute unit before a workgroup is given more than one tile per statistic
     const int64_t tiles = 2 * (int64_t)c.B * c.Hkv * c.nkb;
     c.tiles_per_wg = tiles >= 4096 ? 4 : (tiles >= 2048 ? 2 : 1);
@@ -2222,18 +2233,18 @@ static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepPa
     quant_qkv_stage1_kernel<DT, KIND><<<dim3((unsigned)(n_q + (c.smooth_k ? 2 : 1) * n_chunks)), block, 0, s>>>(c, pq, pk);
     quant_qkv_stage2_kernel<DT, KIND><<<dim3((unsigned)n2), block, 0, s>>>(c, pk);
     *used = true;
-  } else if (c.nch <= kMeetMaxChunks) {
+  } else if (KIND == 0 && c.nch <= kMeetMaxChunks) {
     const QuantOptions opt = quant_options();
     // (V's one-read setting stands for both: K's concerns its separate kernel, which nothing shares the chip with)
     if (!opt.one_read_v || one_read_demoted()) return hipSuccess;
-    if (2 * c.nch > resident_workgroups(quant_qkv_meet_kernel<DT, KIND>, 0)) return hipSuccess;
+    if (2 * c.nch > resident_workgroups(quant_qkv_meet_kernel<DT>, 0)) return hipSuccess;
     int* host = host_word(false).dev;
     const QuantSync& y = c.sync;
     const int n_words = (int)(y.v_status - y.k_counter) + kSyncStride;
     const hipError_t e = launch_clear_ints(y.k_counter, n_words, s);
     if (e != hipSuccess) return e;
     const HeadSync sk{y.k_counter, y.k_ready, y.k_status, opt.wait_ticks, host}, sv{y.v_counter, y.v_ready, y.v_status, opt.wait_ticks, host};
-    quant_qkv_meet_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, pq, pk, sk, sv);
+    quant_qkv_meet_kernel<DT><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, sk, sv);
     *used = true;
   }
   return hipGetLastError();

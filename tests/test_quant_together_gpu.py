@@ -55,3 +55,16 @@ def test_together_with_the_joint_block_step(hip_device, txt, img, weights, table
     prep = sage_ops.QwenPrep(txt, *ws, 1e-6, img_freqs=None if tab is None else tab[:img].contiguous(),
                              txt_freqs=None if tab is None else tab[img:].contiguous())
     _compare(hip_device, 2, txt + img, txt + img, 3, 3, 128, torch.bfloat16, True, prep)
+
+
+@pytest.mark.parametrize("B,txt,img,H", [
+    (1, 56, 13576, 24), (1, 56, 13676, 24),    # 159.75 and 160.9 MB of K and V: the last size in two stages, separate kernels
+    (1, 100, 16284, 1), (1, 100, 16285, 1)])   # 64 chunks of keys, and one row more
+def test_together_with_the_joint_block_step_at_its_limits(hip_device, B, txt, img, H):
+    print(f"case B={B} txt={txt} img={img} H={H}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(img)
+    ws = [1.0 + 0.2 * torch.randn(128, generator=g, device=hip_device) for _ in range(4)]
+    ang = torch.rand((txt + img, 64), generator=g, device=hip_device) * 6.0
+    tab = torch.polar(torch.ones_like(ang), ang)
+    prep = sage_ops.QwenPrep(txt, *ws, 1e-6, img_freqs=tab[:img].contiguous(), txt_freqs=tab[img:].contiguous())
+    _compare(hip_device, B, txt + img, txt + img, H, H, 128, torch.bfloat16, True, prep)
