@@ -2200,7 +2200,7 @@ hipError_t launch_quant_v_fused(const InTensor& v, int B, int H, int L, int nkb,
 }
 
 // Two stages while a head's partial results stay small next to the rows a workgroup of stage 2 quantizes (64 chunks are
-// 32 KiB, the rows 16-64 KiB) and the second reading of K and V comes from the last-level cache (256 MB).  Beyond that
+// 32 KiB, the rows 16-32 KiB) and the second reading of K and V comes from the last-level cache (256 MB).  Beyond that
 // calls without a folded step take the meeting launch.  us, stages / meeting / separate kernels:
 //   40 heads of 9000 tokens (176 MB of K and V) 106 / 108 / 120; 24 heads of 17000 (199 MB) 125 / 122 / 135, two entries of
 //   8500 122 / 117 / 131; 40 heads of 14000 (273 MB) 192 / 158 / 184; 8 heads of 20000 (78 MB, 79 chunks) 46 / 49 / 56.
@@ -2216,6 +2216,11 @@ constexpr int64_t kStageMaxBytesJoint = 160ll << 20;
 // Beyond this many chunks a head's first workgroups wait for its last ones longer than a second pass takes (296 chunks:
 // the separate quantizers are 3 % faster).
 constexpr int kMeetMaxChunks = 160;
+// From here on stage 2 has workgroups enough to give each two tiles per statistic it forms.  us, with 1 / 2 / 4 tiles (an
+// attention launch without rows, 10-35 us, in each figure): plain, 1024 tiles 18.5 / 20.1 / 20.7, 2048 33.1 / 33.5 / 33.9,
+// 3264 45.8 / 45.2 / 46.4, 6528 86.0 / 83.3 / 83.9, 11280 143.0 / 140.1 / 141.0; joint block, 1024 32.2 / 35.2 / 38.5, 3264
+// 68.6 / 71.0 / 73.6, 5120 92.6 / 91.3 / 96.7, 6528 125.4 / 124.3 / 127.2.
+constexpr int kTwoTilesFrom = 2048, kTwoTilesFromJoint = 4096;
 
 template <int DT, int KIND>
 static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepParams& pk, hipStream_t s, bool* used) {
@@ -2226,9 +2231,8 @@ static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepPa
     quant_qkv_small_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, pq, pk);
     *used = true;
   } else if (c.nch <= kStageMaxChunks && 4 * (int64_t)c.B * c.Hkv * c.Lk * c.k.D <= (KIND == 0 ? kStageMaxBytes : kStageMaxBytesJoint)) {
-    // about four workgroups per compute unit before a workgroup is given more than one tile per statistic
     const int64_t tiles = 2 * (int64_t)c.B * c.Hkv * c.nkb;
-    c.tiles_per_wg = tiles >= 4096 ? 4 : (tiles >= 2048 ? 2 : 1);
+    c.tiles_per_wg = tiles >= (KIND == 0 ? kTwoTilesFrom : kTwoTilesFromJoint) ? 2 : 1;
     const int64_t n2 = 2 * (int64_t)c.B * c.Hkv * ((c.nkb + c.tiles_per_wg - 1) / c.tiles_per_wg);
     quant_qkv_stage1_kernel<DT, KIND><<<dim3((unsigned)(n_q + (c.smooth_k ? 2 : 1) * n_chunks)), block, 0, s>>>(c, pq, pk);
     quant_qkv_stage2_kernel<DT, KIND><<<dim3((unsigned)n2), block, 0, s>>>(c, pk);

@@ -38,7 +38,8 @@ def _compare(hip_device, B, Lq, Lk, Hq, Hkv, D, dtype, smooth_k=True, prep=None,
     (2, 32, 32, 4, 4, 128, True), (1, 1, 1, 1, 1, 128, True), (1, 300, 256, 2, 1, 128, True), (1, 40, 256, 2, 2, 64, False),
     (1, 129, 257, 3, 3, 128, True), (2, 513, 1560, 4, 2, 128, True), (1, 100, 640, 2, 2, 64, True), (1, 64, 700, 2, 2, 128, False),
     (1, 200, 16384, 2, 2, 128, True), (1, 64, 16385, 1, 1, 128, True), (1, 128, 8300, 16, 16, 128, True),
-    (1, 128, 20000, 24, 12, 128, True), (1, 128, 17000, 1, 1, 64, False)])
+    (1, 128, 20000, 24, 12, 128, True), (1, 128, 17000, 1, 1, 64, False),
+    (1, 128, 4096 - 64, 16, 16, 128, True), (1, 128, 4096 + 64, 16, 16, 128, True)])  # 2016 and 2080 tiles: one and two a workgroup
 def test_together_gives_the_separate_quantizers_bits(hip_device, B, Lq, Lk, Hq, Hkv, D, smooth_k, dtype):
     print(f"case B={B} Lq={Lq} Lk={Lk} Hq={Hq} Hkv={Hkv} D={D} smooth_k={smooth_k} {dtype}", flush=True)
     _compare(hip_device, B, Lq, Lk, Hq, Hkv, D, dtype, smooth_k)
@@ -59,7 +60,8 @@ def test_together_with_the_joint_block_step(hip_device, txt, img, weights, table
 
 @pytest.mark.parametrize("B,txt,img,H", [
     (1, 56, 13576, 24), (1, 56, 13676, 24),    # 159.75 and 160.9 MB of K and V: the last size in two stages, separate kernels
-    (1, 100, 16284, 1), (1, 100, 16285, 1)])   # 64 chunks of keys, and one row more
+    (1, 100, 16284, 1), (1, 100, 16285, 1),    # 64 chunks of keys, and one row more
+    (1, 100, 5340, 24), (1, 100, 5468, 24)])   # 4080 and (an odd number a head) 4176 tiles: one and two a workgroup of stage 2
 def test_together_with_the_joint_block_step_at_its_limits(hip_device, B, txt, img, H):
     print(f"case B={B} txt={txt} img={img} H={H}", flush=True)
     g = torch.Generator(device=hip_device).manual_seed(img)
