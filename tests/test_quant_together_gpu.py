@@ -70,3 +70,59 @@ def test_together_with_the_joint_block_step_at_its_limits(hip_device, B, txt, im
     tab = torch.polar(torch.ones_like(ang), ang)
     prep = sage_ops.QwenPrep(txt, *ws, 1e-6, img_freqs=tab[:img].contiguous(), txt_freqs=tab[img:].contiguous())
     _compare(hip_device, B, txt + img, txt + img, H, H, 128, torch.bfloat16, True, prep)
+
+
+def _inputs(hip_device, B, Lk, Hq, Hkv, D, dtype):
+    g = torch.Generator(device=hip_device).manual_seed(Lk + D)
+    k = torch.randn((B, Lk, Hkv, D), generator=g, device=hip_device) + 2.0 * torch.randn((Hkv, D), generator=g, device=hip_device)
+    q, v = (torch.randn((B, n, h, D), generator=g, device=hip_device) for n, h in ((128, Hq), (Lk, Hkv)))
+    return q.to(dtype), k.to(dtype), v.to(dtype)
+
+
+def _same_areas(ws, want):
+    for name in AREAS:
+        assert torch.equal(getattr(ws, name).view(torch.uint8), getattr(want, name).view(torch.uint8)), name
+
+
+@pytest.mark.parametrize("B,Lk,Hq,Hkv,D,dtype,smooth_k", [
+    (1, 16385, 1, 1, 128, torch.bfloat16, True), (2, 17000, 4, 2, 128, torch.float16, True), (1, 16641, 2, 2, 64, torch.bfloat16, True),
+    (2, 8500, 24, 24, 128, torch.bfloat16, True), (1, 20000, 2, 2, 128, torch.bfloat16, False)])
+def test_the_meeting_launch_stays_exact_when_its_waits_run_out(hip_device, quant_settings, B, Lk, Hq, Hkv, D, dtype, smooth_k):
+    """K's and V's chunks share one launch and one area of counters; with a negative bound every workgroup but the last
+    arrivers of its head's K and V takes the statistic from the input."""
+    print(f"case B={B} Lk={Lk} Hq={Hq} Hkv={Hkv} D={D} {dtype} smooth_k={smooth_k}", flush=True)
+    q, k, v = _inputs(hip_device, B, Lk, Hq, Hkv, D, dtype)
+    ws, want = sage_ops.workspace_for(q, k), sage_ops.workspace_for(q, k)
+    ws.blob.fill_(0x7F), want.blob.fill_(0x7F)
+    sage_ops.quant_qk(q, k, want, D**-0.5, smooth_k)
+    sage_ops.quant_v(v, want)
+    for bound in (-1, 0):  # 0: which workgroups give up depends on timing
+        quant_settings(wait_ticks=bound)
+        sage_ops.sageattn(q, k, v, workspace=ws, smooth_k=smooth_k)
+        status = sage_ops.quant_status(ws)
+        if bound < 0:
+            assert status == (1 if smooth_k else 0, 1)  # without a mean to take off K waits for nobody
+        _same_areas(ws, want)
+        assert not sage_ops.one_read_state()["demoted"]  # test-mode bounds switch nothing off
+    quant_settings(wait_ticks=200000)
+    sage_ops.sageattn(q, k, v, workspace=ws, smooth_k=smooth_k)
+    assert sage_ops.quant_status(ws) == (0, 0)
+    _same_areas(ws, want)
+
+
+def test_an_expired_bound_of_the_meeting_launch_switches_it_off(hip_device, quant_settings):
+    print("case expired bound, whole call", flush=True)
+    q, k, v = _inputs(hip_device, 1, 20000, 8, 8, 128, torch.bfloat16)
+    ws, want = sage_ops.workspace_for(q, k), sage_ops.workspace_for(q, k)
+    sage_ops.quant_qk(q, k, want, 128**-0.5)
+    sage_ops.quant_v(v, want)
+    quant_settings(wait_ticks=1)  # 10 ns: any workgroup that finds its head's flag down twice gives up
+    sage_ops.sageattn(q, k, v, workspace=ws)
+    _same_areas(ws, want)
+    if sage_ops.quant_status(ws) == (0, 0):
+        pytest.skip("no workgroup had to wait for its head in this run")
+    assert sage_ops.one_read_state()["demoted"]
+    ws.blob.fill_(0x7F)
+    sage_ops.sageattn(q, k, v, workspace=ws)  # the separate two-pass kernels: nobody waits
+    assert sage_ops.quant_status(ws) == (0, 0)
+    _same_areas(ws, want)
