@@ -2239,7 +2239,7 @@ static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepPa
     *used = true;
   } else if (KIND == 0 && c.nch <= kMeetMaxChunks) {
     const QuantOptions opt = quant_options();
-    // (V's one-read setting stands for both: K's concerns its separate kernel, which nothing shares the chip with)
+    // (V's one-read setting stands for both here: K's letter concerns its separate kernel, see ksana_sage_configure)
     if (!opt.one_read_v || one_read_demoted()) return hipSuccess;
     if (2 * c.nch > resident_workgroups(quant_qkv_meet_kernel<DT>, 0)) return hipSuccess;
     int* host = host_word(false).dev;

@@ -512,7 +512,8 @@ def quant_status(ws: SageWorkspace) -> tuple[int, int]:
 
 def configure(one_read: str | None = None, wait_ticks: int | None = None) -> None:
     """Process-wide settings of the one-read K / V quantizers (``ksana_sage_configure``): ``one_read`` is a string of
-    the letters ``k`` and ``v`` (the stages that read their input once when the shape allows), ``wait_ticks`` the bound
+    the letters ``k`` and ``v`` (the stages that read their input once when the shape allows; in whole calls of 65 to 160
+    chunks of 256 keys, or more than 192 MB of K and V, ``v`` selects one launch that reads K once too), ``wait_ticks`` the bound
     on a workgroup's wait for its head's statistic in 10 ns ticks (0 / negative: test modes, see the header).
     ``None`` leaves a setting as it is.  Every call re-arms the one-read kernels on all GPUs."""
     rc = _capi.load().ksana_sage_configure(None if one_read is None else one_read.encode(),

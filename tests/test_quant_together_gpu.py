@@ -126,3 +126,26 @@ def test_an_expired_bound_of_the_meeting_launch_switches_it_off(hip_device, quan
     sage_ops.sageattn(q, k, v, workspace=ws)  # the separate two-pass kernels: nobody waits
     assert sage_ops.quant_status(ws) == (0, 0)
     _same_areas(ws, want)
+
+
+@pytest.mark.parametrize("Lk,qwen,smooth_v,waits", [
+    (16384, False, False, {"v": (0, 0), "": (0, 0), "k": (0, 0), "kv": (0, 0)}),   # two stages: nobody waits
+    (16385, False, False, {"v": (1, 1), "": (0, 0), "k": (1, 0), "kv": (1, 1)}),   # one launch with "v", separate kernels without
+    (41000, False, False, {"v": (0, 1), "": (0, 0), "k": (1, 0), "kv": (1, 1)}),   # more than 160 chunks: separate kernels
+    (16385, True, False, {"v": (1, 1), "": (1, 0), "k": (1, 0), "kv": (1, 1)}),    # with a folded step K tries to read once
+    (3000, False, True, {"v": (0, 0), "": (0, 0), "k": (1, 0), "kv": (1, 0)})])    # V smoothing: separate kernels, V in passes
+def test_which_settings_make_whole_calls_wait(hip_device, quant_settings, Lk, qwen, smooth_v, waits):
+    """The routes of ``ksana_sage_configure``'s letters, seen through the status words of calls whose workgroups never look at
+    a flag: 1 where a stage's workgroups meet."""
+    q, k, v = _inputs(hip_device, 1, Lk, 1, 1, 128, torch.bfloat16)
+    prep = None
+    if qwen:
+        q, w = k.flip(1), torch.ones(128, device=hip_device)
+        prep = sage_ops.QwenPrep(5, w, w, w, w, 1e-6)
+    ws = sage_ops.workspace_for(q, k)
+    for letters, status in waits.items():
+        print(f"case Lk={Lk} qwen={qwen} smooth_v={smooth_v} letters={letters!r}", flush=True)
+        quant_settings(one_read=letters, wait_ticks=-1)
+        ws.blob.fill_(0x7F)
+        sage_ops.sageattn(q, k, v, workspace=ws, prep=prep, smooth_v=smooth_v)
+        assert sage_ops.quant_status(ws) == status, letters
