@@ -222,7 +222,7 @@ def other_workloads(sage_ops, dev, pwl, iters=7):
                                      "kept_pair_rate_vs_dense": round((w.L + 1) / (2.0 * w.L) * ms / t_causal, 3)}
         del q, k, v, ws, out
         torch.cuda.empty_cache()
-    # Head size 64 (no BASELINE model has it; the backend interface serves it): the headline shape's token count
+    # Head size 64 (no measured model has it; the backend interface serves it): the headline shape's token count
     d64 = Workload("wan14b_480p_head_size_64", 1008, 1, 40, 32760)
     q, k, v = device_inputs(d64, dev)
     q, k, v = (t[..., :64].contiguous() for t in (q, k, v))

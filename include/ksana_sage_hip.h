@@ -39,21 +39,22 @@ extern "C" {
 /* error codes */
 #define KSANA_SAGE_OK 0
 #define KSANA_SAGE_EINVAL (-1)   /* bad shape, stride, alignment, dtype or null pointer      */
-#define KSANA_SAGE_ENOTSUP (-2)  /* valid request this build does not implement (D != 128, sizes beyond its limits) */
+#define KSANA_SAGE_ENOTSUP (-2)  /* valid request the library does not implement (a head size other than 64 and 128, sizes beyond its limits) */
 #define KSANA_SAGE_EHIP (-3)     /* the HIP runtime reported an error at launch               */
 
 /* flags of the attention entry points */
 #define KSANA_SAGE_FLAG_PWL_EXP2 1 /* Default (flag clear): P = exp2(x) on the transcendental unit, then the  */
                                    /* hardware e4m3 cast.  Flag set: the e4m3 CODE of P is computed directly  */
                                    /* as rne(8*x + 55.5), i.e. exp2 with a piecewise-linear 3-bit mantissa:   */
-                                   /* ~35 % fewer vector-ALU slots (about 1.2x faster), cos-sim to SDPA lower */
+                                   /* ~35 % fewer vector-ALU slots (1.06-1.12x at 27 000 keys and more of 128 */
+                                   /* channels, nothing at 4 400 and below, 0.82x at 64), cos-sim to SDPA lower */
                                    /* by ~1.5e-4 and the worst element about 2x further out.                  */
 #define KSANA_SAGE_FLAG_SMOOTH_V 2 /* ksana_sage_forward* only: quantize V with its channel means taken off   */
                                    /* (see ksana_sage_quant_v_smooth).                                        */
 
 #define KSANA_SAGE_FLAG_WG_4_WAVES 4 /* attention entry points: force workgroups of 4 waves (128 query rows, two per   */
 #define KSANA_SAGE_FLAG_WG_8_WAVES 8 /* compute unit) / of 8 waves (256 rows, one per unit) instead of the library's   */
-                                     /* own choice (4 with a block mask, causal masking or Lk <= 1024).  Same results  */
+                                     /* own choice (4 with a block mask or causal masking, else by estimated time).  Same results */
                                      /* up to the rounding of the key-run merge; for measurements.                     */
 
 /* rows per int8 scale: Q per token, K per 64 keys (sage_sla.py:190,204 uses (128, 64) off-Hopper;
@@ -67,8 +68,8 @@ extern "C" {
                                      /* probability byte of such a tile is the zero code, so the result is the same bits  */
                                      /* - the pvthreshold argument of the reference's sparse kernel (sage_sla.py:237-253; */
                                      /* the reference passes 1e6, i.e. "never"), at a threshold where nothing changes.    */
-                                     /* Off by default: the test per tile costs ~7 % where no tile qualifies (flat         */
-                                     /* attention); it pays where attention is peaked.                                     */
+                                     /* Off by default: its loop is 7-13 % slower than the default one where no tile       */
+                                     /* qualifies; it gains up to 7 % where attention is sharply peaked.                   */
 
 #define KSANA_SAGE_FLAG_Q_UNSTORED 32 /* ksana_sage_forward* only: the caller does not read q_i8 and q_scale from the       */
                                       /* workspace afterwards and o does not overlap q.  Without a block mask and a step   */
@@ -318,8 +319,10 @@ int ksana_sage_quant_status(const void* workspace, const ksana_sage_shape* shape
  * call (sage_sla.py:237-253, dense form).  flags: KSANA_SAGE_FLAG_*.
  * When the number of 256-row query blocks times heads leaves a small remainder against the number of compute units,
  * the workgroups of that remainder are cut into runs of key tiles that fill the chip together, and a second small
- * kernel merges the runs (dense, non-causal calls only); the result is the same attention within rounding, and
- * repeated calls give identical bits.  The quantized operands in the workspace are only read; the runs' scratch
+ * kernel merges the runs (dense, non-causal calls of more than 16 key tiles only); the result is the same attention within
+ * rounding, and repeated calls give identical bits.  A run keeps reference points of its own, so a row's probabilities are
+ * rounded to e4m3 against other points in a cut block than in a whole one: the bits of a row (not their error, which is the
+ * same to 0.5 % of itself) depend on how many query blocks and heads the call has; ksana_sage_attn_key_split tells.  The quantized operands in the workspace are only read; the runs' scratch
  * (split_o, split_ml) is the one part of it this call writes.
  * causal: non-zero lets query row i attend to keys [0, i] only (the is_causal of sage_attn.py:75-81 and of
  * sdpa.py:62-79), on top of k_lens and the block mask; for Lq != Lk the triangle is anchored at the top left corner,

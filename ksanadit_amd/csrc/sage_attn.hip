@@ -268,7 +268,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       if (wg >= n_wg) return;
     } else {
       // batch entries of unequal length: an eighth of every entry's workgroups to every XCD.  One run across the entries
-      // would leave the XCDs that drew the short ones idle (B=3, 24 heads, lengths 100 / 72 / 45 % of 4099: 265 -> 177 us).
+      // would leave the XCDs that drew the short ones idle.  The entries run in the order of their index, longest first or
+      // not: the order that ends with the longest one costs up to 5-8 % in grids of two rounds, nothing in long ones.  us,
+      // one run across the entries / this, for lengths falling, rising, the longest last but one: B=3, 24 heads, 100 / 72 /
+      // 45 % of 3001 x 4099 265 / 165, 273 / 173, 273 / 178; B=2, 40 heads of 16384 5560 / 3280, 5530 / 3272, 5600 / 3270.
       const int b = at / p.batch_run, n_batch = p.Hq * n_qwg;
       const int in_batch = xcd * p.batch_run + (at - b * p.batch_run);
       wg = b * n_batch + in_batch;
@@ -785,7 +788,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // limit, and only when some lane of the wave exceeds it are the halves joined and points, factors and constants
   // formed anew (one wave-uniform branch instead of eight vector operations and a transcendental in every step).
   // With the 16x16 row sums, same bits: 10.60 -> 10.35 ms at B=1 H=40 L=32760 with outliers, 11.44 -> 11.05 without
-  // (2045 cycles per step, from 2073; the chip runs at its power limit there, and fewer operations raise its clock too).
+  // (2045 cycles per step, from 2073, and 1843 with the loop unrolled and grouped; the chip runs at its power limit there,
+  // and fewer operations raise its clock too).
   float sc = 0.0f, xc = 0.0f;           // scale of the coming tile, its exponent constant
   // factor a tile's point move puts on everything before it, and (wave-uniform) whether there is one: of even tiles and
   // of odd ones (step j applies tile j-1's and then finds tile j+1's)

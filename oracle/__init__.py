@@ -1,7 +1,7 @@
 """CPU oracle for the quantized (Sage-style) attention path.  TEST INFRASTRUCTURE ONLY.
 
 Nothing here is product code: only ``tests/``, ``__graft_entry__.smoke()`` and the
-``cpu_baseline`` leg of ``bench.py`` may import this package, and only as the checker.
+``cpu_baseline`` leg of ``bench.py`` may import this package, and only to compare with.
 The product path (``ksanadit_amd``) never imports it and has no CPU fallback.
 
 Functions and what pins each of them:

@@ -299,7 +299,7 @@ def test_sdpa_backend_on_cpu_matches_oracle_and_reference_checks():
 
 
 def test_cpu_plumbing_workload_through_the_op():
-    """the CPU-runnable case goes through this package's SDPA backend."""
+    """The CPU-runnable case (1 560 tokens) goes through this package's SDPA backend."""
     q, k, v = make_inputs("cpu_plumbing", heads=2)
     assert q.shape == (1, 1560, 2, 128) and q.dtype == torch.bfloat16
     attn = pick_attn_op(KsanaAttentionConfig(backend="torch_sdpa"))(num_heads=2, head_size=128)
