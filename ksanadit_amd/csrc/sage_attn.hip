@@ -240,11 +240,11 @@ template <int DT, bool kPwlExp, bool kSparse, int kW, bool kTileSkip, int kG, bo
 __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel(const AttnParams p, int n_qwg,
                                                                                    int n_wg, int wg_per_xcd) {
   constexpr bool kCanSplit = !kSparse && kW == 8;
-  static_assert(kSparse || !kCausal, "causal calls run through the tile list");
+  static_assert(kSparse || !kCausal || (kW == 4 && !kPwlExp && !kTileSkip), "causal without a list: the default variant in 4 waves");
   // kCausal == false: the caller vouches that p.causal is 0, and everything that serves the diagonal (the per-wave
   // last tile, 32 lane masks held in scalar registers, the selects that blank a wave's probabilities past its rows)
   // is compiled out of the key loop
-  const bool causal = kCausal && p.causal;
+  const bool causal = kCausal && (!kSparse || p.causal);
   using Shape = WgShape<kW>;
   constexpr int kThreadsAttn = Shape::kThreads, kRowsWg = Shape::kRows, kStages = Shape::kStages, kAhead = Shape::kAhead;
   constexpr int kListMax = kW == 8 ? kSparseMaxKeyTiles : kSparseMaxKeyTiles4;
@@ -253,35 +253,63 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   constexpr bool kUnrolled = !kPwlExp && !kTileSkip && !(kSparse && kW == 8);  // the variants calls take by default
   constexpr int kMagicBits = kG == 4 ? kMagicI : kMagicI2;
   constexpr float kMagicVal = kG == 4 ? kMagicF : kMagicF2;
-  int wg;
+  int bh, qwg;  // (batch, head) pair and query block
   const bool is_run = kCanSplit && (int)blockIdx.x >= p.split_first_block;  // uniform
   const int run_id = is_run ? (int)blockIdx.x - p.split_first_block : 0;    // the partial result's place in the workspace
-  if (is_run) {
-    wg = p.split_first_wg + run_id / p.n_split;
-  } else {
-    // Consecutive workgroup ids land on consecutive XCDs (8 per chip, one L2 each).  Give every
-    // XCD a contiguous run of (head, query block) pairs so the workgroups that stream the same
-    // K/V tiles share one L2.
-    const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
-    if (p.batch_run == 0) {
-      wg = xcd * wg_per_xcd + at;
-      if (wg >= n_wg) return;
+  if (kCausal && p.causal_group != 0) {
+    // The later a query block, the more key tiles it walks: every XCD starts its long blocks first (causal_grid).
+    const int xcd = blockIdx.x & 7;
+    int at = blockIdx.x >> 3;
+    const int shared = (p.causal_rest * n_qwg - xcd + 7) >> 3;  // this XCD's eighth of the pairs left over
+    if (at < shared) {
+      const int i = at * 8 + xcd, blk = i / p.causal_rest;
+      bh = 8 * p.causal_own + i - blk * p.causal_rest;
+      qwg = n_qwg - 1 - blk;
     } else {
-      // batch entries of unequal length: an eighth of every entry's workgroups to every XCD.  One run across the entries
-      // would leave the XCDs that drew the short ones idle.  The entries run in the order of their index, longest first or
-      // not: the order that ends with the longest one costs up to 5-8 % in grids of two rounds, nothing in long ones.  us,
-      // one run across the entries / this, for lengths falling, rising, the longest last but one: B=3, 24 heads, 100 / 72 /
-      // 45 % of 3001 x 4099 265 / 165, 273 / 173, 273 / 178; B=2, 40 heads of 16384 5560 / 3280, 5530 / 3272, 5600 / 3270.
-      const int b = at / p.batch_run, n_batch = p.Hq * n_qwg;
-      const int in_batch = xcd * p.batch_run + (at - b * p.batch_run);
-      wg = b * n_batch + in_batch;
-      if (in_batch >= n_batch || wg >= n_wg) return;
+      at -= shared;
+      if (at >= p.causal_own * n_qwg) return;
+      // groups of causal_group pairs, the first one with what does not divide evenly
+      const int n_groups = p.causal_own / p.causal_group;
+      int first = 0, size = p.causal_own - (n_groups - 1) * p.causal_group;
+      if (at >= size * n_qwg) {
+        at -= size * n_qwg;
+        const int g = at / (p.causal_group * n_qwg);
+        at -= g * p.causal_group * n_qwg;
+        first = size + g * p.causal_group;
+        size = p.causal_group;
+      }
+      const int blk = at / size;
+      bh = xcd * p.causal_own + first + at - blk * size;
+      qwg = n_qwg - 1 - blk;
     }
+  } else {
+    int wg;
+    if (is_run) {
+      wg = p.split_first_wg + run_id / p.n_split;
+    } else {
+      // Consecutive workgroup ids land on consecutive XCDs (8 per chip, one L2 each).  Give every
+      // XCD a contiguous run of (head, query block) pairs so the workgroups that stream the same
+      // K/V tiles share one L2.
+      const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+      if (p.batch_run == 0) {
+        wg = xcd * wg_per_xcd + at;
+        if (wg >= n_wg) return;
+      } else {
+        // batch entries of unequal length: an eighth of every entry's workgroups to every XCD.  One run across the entries
+        // would leave the XCDs that drew the short ones idle.  The entries run in the order of their index, longest first or
+        // not: the order that ends with the longest one costs up to 5-8 % in grids of two rounds, nothing in long ones.  us,
+        // one run across the entries / this, for lengths falling, rising, the longest last but one: B=3, 24 heads, 100 / 72 /
+        // 45 % of 3001 x 4099 265 / 165, 273 / 173, 273 / 178; B=2, 40 heads of 16384 5560 / 3280, 5530 / 3272, 5600 / 3270.
+        const int b = at / p.batch_run, n_batch = p.Hq * n_qwg;
+        const int in_batch = xcd * p.batch_run + (at - b * p.batch_run);
+        wg = b * n_batch + in_batch;
+        if (in_batch >= n_batch || wg >= n_wg) return;
+      }
+    }
+    bh = wg / n_qwg;
+    qwg = wg - bh * n_qwg;
+    if (causal) qwg = n_qwg - 1 - qwg;  // the long ones first, as above
   }
-  const int bh = wg / n_qwg;
-  int qwg = wg - bh * n_qwg;
-  // causal: the later a query block, the more key tiles it walks - start the long ones first
-  if (kSparse && causal) qwg = n_qwg - 1 - qwg;
   const int b = bh / p.Hq, h = bh - b * p.Hq;
   const int bhk = b * p.Hkv + h / (p.Hq / p.Hkv);
 
@@ -416,17 +444,19 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // << 16 | row-1 flag << 17.  The loop below then walks list positions instead of tile
   // numbers; a wave whose row does not ask for a tile zeroes its probabilities for it and
   // leaves its running maximum alone, so the result is exactly the masked softmax.
-  // Causal attention (key <= query row) runs through the same list: the workgroup lists the tiles up
-  // to the one holding its last row, a wave leaves alone the tiles past its own last row, and the one
+  // Causal attention (key <= query row) on top of a mask runs through the same list, and without one over the tile
+  // numbers themselves: the workgroup takes the tiles up to the one holding its last row, a wave leaves alone the tiles past its own last row, and the one
   // tile that straddles its rows' diagonal is masked element by element.
   // (one mask row per 4-wave workgroup: an entry is the tile number and fits 16 bits; with two mask rows per
   // workgroup it carries their two flags above the number)
   using ListEntry = typename std::conditional<kW == 4, uint16_t, int>::type;
   ListEntry* s_list = reinterpret_cast<ListEntry*>(s_ks + kListMax);
   int* s_count = reinterpret_cast<int*>(s_list + kListMax);
-  int n_tiles = nkb;  // loop length: list entries with a mask, key tiles without
+  // loop length: list entries with a mask, key tiles without (causal: up to the one holding the workgroup's last row)
+  const int wg_tiles = causal ? min(nkb, ((qwg * kRowsWg + kRowsWg - 1) >> 6) + 1) : nkb;
+  int n_tiles = wg_tiles;
   // a wave's 32 rows start at a multiple of 32, so exactly one 64-key tile holds their diagonal
-  const int my_last = (kSparse && causal) ? (q0 >> 6) : 0x7fffffff;
+  const int my_last = causal ? (q0 >> 6) : 0x7ffffffe;
   if constexpr (kSparse) {
     if (wave == 0) {
       const int nqm = (p.Lq + kMaskBlkQ - 1) / kMaskBlkQ;
@@ -434,7 +464,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       constexpr int kMaskRows = kRowsWg / kMaskBlkQ;  // mask rows a workgroup covers: 2 or 1
       const int8_t* m0 = masked ? p.block_mask + b * p.mask_sB + h * p.mask_sH + (int64_t)(kMaskRows * qwg) * p.nkb : nullptr;
       const bool two = kMaskRows == 2 && 2 * qwg + 1 < nqm;
-      const int wg_tiles = causal ? min(nkb, ((qwg * kRowsWg + kRowsWg - 1) >> 6) + 1) : nkb;
       int base = 0;
       // eight chunks of 64 tiles at a time: their mask bytes are requested together, so a list of 512 tiles costs
       // one memory latency instead of eight
@@ -484,7 +513,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if constexpr (kSparse) {
       for (int i = tid; i < n_tiles; i += kThreadsAttn) s_ks[i] = ks_ptr[s_list[i] & 0xffff];
     } else {
-      for (int i = tid; i < nkb; i += kThreadsAttn) s_ks[i] = ks_ptr[i];
+      for (int i = tid; i < n_tiles; i += kThreadsAttn) s_ks[i] = ks_ptr[i];
     }
     if (tid < 2 * kD) s_vs[tid] = vsm;
   };
@@ -492,6 +521,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // are the first n_mine, and the diagonal tile, if listed, is the last of them.  Both are found once here; the key
   // loop then compares loop positions instead of looking list entries up.
   int n_mine = n_tiles, jdiag = -1;  // wave-uniform
+  if constexpr (kCausal && !kSparse) {
+    n_mine = min(n_tiles, my_last + 1);
+    if (my_last < n_tiles) jdiag = my_last;
+  }
   if constexpr (kSparse) {
     if (causal) {
       if (p.block_mask == nullptr) {  // the list is 0, 1, 2, ...
@@ -520,11 +553,12 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       const int e = __builtin_amdgcn_readfirstlane(s_list[jj]);
       return ((e >> (16 + (wave >> 2))) & 1) != 0 && jj < n_mine;
     }
+    if constexpr (kCausal) return jj < n_mine;
     return true;
   };
-  // causal only: list position jj holds the tile on this wave's diagonal
+  // causal only: loop position jj holds the tile on this wave's diagonal
   auto diag_at = [&](int jj) -> bool {
-    if constexpr (kSparse && kCausal) return jj == jdiag;
+    if constexpr (kCausal) return jj == jdiag;
     return false;
   };
   // scores of keys beyond the row's own position drop below every real score ...
@@ -652,7 +686,12 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // K tile kStages goes into the slot of K tile 0, which every wave must have read by then - in the set-up, and a single
   // step requests tiles kAheadK ahead, the first group of steps all up to kStages, before the loop's first barrier.
   constexpr bool kSlotZeroSoon = Shape::kAheadK == kStages || (kUnrolled && Shape::kGroup > 1);
-  const int n_grouped = kUnrolled && Shape::kGroup > 1 ? n_main / kStages * kStages : 0;
+  // Without a list, the steps before any of the workgroup's waves meets its diagonal tile know nothing of it: they are the
+  // dense loop's (with the diagonal's code in every unrolled step to be jumped over,
+  // 8 191 tokens of 32 heads took 334 us instead of 323).
+  constexpr bool kDiagApart = kCausal && !kSparse && kUnrolled;
+  const int n_plain = kDiagApart ? min(n_main, max(0, ((qwg * kRowsWg) >> 6) - 1)) : n_main;
+  const int n_grouped = kUnrolled && Shape::kGroup > 1 ? n_plain / kStages * kStages : 0;
 
   // The compiler does not see the asynchronous copies in the memory-operation counter it models.  Every ordinary global
   // load of the set-up (Q fragments, scales) must therefore be known to have returned before the key loop starts:
@@ -905,7 +944,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (kSparse) {  // rare, wave-uniform: the next tile is the one on this wave's diagonal
+    if constexpr (kCausal && !(kDiagApart && kAt >= 0)) {  // rare, wave-uniform: the next tile is the one on this wave's diagonal
       if (j + 1 < n_tiles && diag_at(j + 1)) causal_scores(s_nxt);
     }
     __builtin_amdgcn_s_setprio(0);
@@ -934,6 +973,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
       for (int i = 0; i + 1 < kWindow; ++i) ahead[i] = ahead[i + 1];
       ahead[kWindow - 1] = __builtin_amdgcn_readfirstlane(entering) & 0xffff;
+    }
+    if constexpr (kSparse || (kCausal && !(kDiagApart && kAt >= 0))) {
       if (!mine_at(j)) {  // wave-uniform and rare: a tile this wave's row does not take part in contributes nothing
 #pragma unroll
         for (int i = 0; i < 8; ++i) pf[i] = 0;
@@ -956,7 +997,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         tile_step(std::integral_constant<int, kAt>{}, j + kAt, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
         tile_step(std::integral_constant<int, kAt + 1>{}, j + kAt + 1, s_b, s_a, pf_y, pf_x, alpha_even, moved_even);
       };
-      for (; j + kStages <= n_main; j += kStages) {
+      for (; j + kStages <= n_plain; j += kStages) {
         two(std::integral_constant<int, 0>{});
         two(std::integral_constant<int, 2>{});
         if constexpr (kStages == 8) {
@@ -1045,7 +1086,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // past its last tile) and leave as whole 256-byte rows, 16 bytes per lane.
   const int q = q0 + l32;
   // zero for a mask row that allows none of its keys (an empty sum, not 0/0) and for rows at or beyond lq
-  const float inv_l = ((!kSparse || lacc[0] > 0.0f) && q < lq) ? 1.0f / lacc[0] : 0.0f;
+  const float inv_l = ((!(kSparse || kCausal) || lacc[0] > 0.0f) && q < lq) ? 1.0f / lacc[0] : 0.0f;
   // the channel means the V quantizer took off come back here (rows of P sum to one); they are zeros without V
   // smoothing, and a row that saw no key stays zero
   const float keep_mean = inv_l != 0.0f ? 1.0f : 0.0f;
@@ -1179,6 +1220,19 @@ hipError_t launch_variant(const AttnParams& p, dim3 grid, size_t lds, int n_qwg,
   return hipGetLastError();
 }
 
+// Causal calls without a block mask, in the default variant: key tiles are walked without a list, and the steps before the
+// diagonal are the dense loop's.  us per call, tile list / this: 8 191 tokens of 32 heads (8 of keys) 350 / 323, 12 x 7 411
+// 151 / 142, 40 x 32 760 6 285 / 5 820, 20 000 tokens of one head 239 / 207, 40 x 1 024 36.9 / 35.3.  (8 waves: 2 % faster from
+// eight rounds of 90 blocks per head, 5 - 30 % slower in short grids; not built.)
+hipError_t launch_causal(const AttnParams& p, dim3 grid, size_t lds, int n_qwg, int n_wg, int wg_per_xcd, hipStream_t s) {
+  const bool bf16 = p.o.dtype == KSANA_SAGE_BF16;
+  if (p.d_out <= 64)
+    return bf16 ? launch_variant<KSANA_SAGE_BF16, false, false, 4, true, false, 2>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
+                : launch_variant<KSANA_SAGE_FP16, false, false, 4, true, false, 2>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+  return bf16 ? launch_variant<KSANA_SAGE_BF16, false, false, 4, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
+              : launch_variant<KSANA_SAGE_FP16, false, false, 4, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+}
+
 // the (dtype, exp2 form, tile skip) instantiations behind one (mask, workgroup shape) choice
 template <bool kSparse, int kW, bool kCausal = false>
 hipError_t launch_shape(const AttnParams& p, dim3 grid, size_t lds, int n_qwg, int n_wg, int wg_per_xcd, hipStream_t s) {
@@ -1291,33 +1345,47 @@ static dim3 xcd_grid(AttnParams* p, int n_qwg, int n_wg, int* wg_per_xcd) {
   return dim3(*wg_per_xcd * 8);
 }
 
+// The numbering of a causal launch (the kernel's first lines): every XCD takes B * Hq / 8 (batch, head) pairs of its own and
+// an eighth of the query blocks of the pairs left over - one run of blocks per XCD gives some of them a pair's long half and
+// others its short one.  Blocks go out from the last one down, through a group of pairs together: one pair after the other,
+// the last pair's long blocks start when little is left to run beside them.  A group has six blocks for each of an XCD's
+// workgroup places; larger ones only share the L2 between more heads.  us per call, one run and one pair after the other /
+// groups of 2 / of 6 blocks per place / all pairs together: 8 191 tokens of 32 heads 361 / 356 / 350 / 350, 2 x 3 000 of 64 heads
+// 254 / 240 / 236 / 236, 24 x 2 048 55 / 50 / 50 / 50; without the tile list 40 x 32 760 5 990 in groups of 6, 6 285 all together.
+constexpr int kPlacesPerXcd = 64;  // 4-wave workgroups: two on each of 32 compute units
+static void causal_grid(AttnParams* p, int n_qwg) {
+  const int pairs = p->B * p->Hq;
+  p->causal_own = pairs / 8;
+  p->causal_rest = pairs - 8 * p->causal_own;
+  p->causal_group = min((6 * kPlacesPerXcd + n_qwg - 1) / n_qwg, max(p->causal_own, 1));
+}
+
 hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   AttnParams p = params;
   p.split_first_block = INT32_MAX;
   if (p.nkb > kMaxKeyTiles) return hipErrorInvalidValue;
   const bool sparse = p.block_mask != nullptr || p.causal;
   if (sparse && p.nkb > kSparseMaxKeyTiles) return hipErrorInvalidValue;
+  const bool plain_causal = p.causal && p.block_mask == nullptr && p.exact_exp2 && !p.tile_skip;  // no tile list
   int waves = pick_wg_waves(p);
   if (waves == 4 && p.nkb > (sparse ? kSparseMaxKeyTiles4 : kShortMaxKeyTiles)) waves = 8;
-  if (waves == 4) {
-    const int n_qwg = (p.Lq + WgShape<4>::kRows - 1) / WgShape<4>::kRows;
-    const int n_wg = p.B * p.Hq * n_qwg;
-    int wg_per_xcd = 0;
-    const dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
-    if (sparse)
-      return p.causal ? launch_shape<true, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
-                      : launch_shape<true, 4, false>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s);
-    const size_t lds = WgShape<4>::kRingBytes + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
-    return launch_shape<false, 4>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
-  }
-  const int n_qwg = (p.Lq + kAttnQPerWg - 1) / kAttnQPerWg;
+  const int rows = 32 * waves;
+  const int n_qwg = (p.Lq + rows - 1) / rows;
   const int n_wg = p.B * p.Hq * n_qwg;
   int wg_per_xcd = 0;
   const dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
+  if (p.causal && p.batch_run == 0) causal_grid(&p, n_qwg);  // (the same number of workgroups)
+  // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
+  const size_t lds = (waves == 4 ? WgShape<4>::kRingBytes : WgShape<8>::kRingBytes) + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
+  if (waves == 4) {
+    if (plain_causal) return launch_causal(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+    if (sparse)
+      return p.causal ? launch_shape<true, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
+                      : launch_shape<true, 4, false>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s);
+    return launch_shape<false, 4>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+  }
   // (tile lists in 256-row workgroups, by flag only: one instantiation serves causal and plain calls)
   if (sparse) return launch_shape<true, 8, true>(p, grid, max_lds<true, 8>(), n_qwg, n_wg, wg_per_xcd, s);
-  // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
-  const size_t lds = WgShape<8>::kRingBytes + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
   // The workgroups beyond the last full round of the chip (one workgroup per compute unit) would hold it for a
   // whole round alone.  When they are few, each is cut into runs of key tiles that together fill a round, and a
   // small kernel merges the runs: 2568 workgroups are then 10 rounds and a bit instead of 11, 280 are 1.1 instead of 2.

@@ -100,6 +100,21 @@ def test_whole_and_cut_query_blocks_in_one_grid(hip_device, Lk):
     _close(out, want)
 
 
+@pytest.mark.parametrize("B,H", [(1, 1), (1, 3), (1, 8), (3, 5), (1, 17), (2, 24)])
+@pytest.mark.parametrize("L", [100, 128, 640, 1300])
+def test_causal_blocks_are_shared_out_over_the_chip(hip_device, B, H, L):
+    """Every (batch, head, query block) is computed once, whether its pair belongs to one XCD or to all of them and
+    whatever group of pairs it is walked through with; one block ahead of the diagonal, on it, and several."""
+    print(f"case B={B} H={H} L={L}", flush=True)
+    g = torch.Generator().manual_seed(100 * L + 10 * B + H)
+    q, k, v = (torch.randn((B, L, H, 128), generator=g).to(torch.bfloat16) for _ in range(3))
+    qd, kd, vd = (t.to(hip_device) for t in (q, k, v))
+    ws = sage_ops.workspace_for(qd, kd)
+    sage_ops.quant_q(qd, ws, 128**-0.5), sage_ops.quant_k(kd, ws, True), sage_ops.quant_v(vd, ws)
+    out = sage_ops.attn_fwd(ws, torch.full_like(qd, float("nan")), causal=True).cpu()
+    _close(out, _emul(ws, L, L, q.dtype, causal=True))
+
+
 @pytest.mark.parametrize("waves", [4, 8])
 @pytest.mark.parametrize("Lk", [64 * 8, 64 * 9, 64 * 17 + 3])
 def test_repeated_calls_give_the_same_bits(hip_device, waves, Lk):
