@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define KSANA_SAGE_ABI_VERSION 22
+#define KSANA_SAGE_ABI_VERSION 23
 
 /* element types of q/k/v/o */
 #define KSANA_SAGE_BF16 0
@@ -75,6 +75,11 @@ extern "C" {
                                       /* workspace afterwards and o does not overlap q.  Without a block mask and a step   */
                                       /* folded into q, where o has its type and the sizes make it pay, the attention      */
                                       /* kernel then quantizes Q itself and the two areas stay unwritten.  Same bits.      */
+
+#define KSANA_SAGE_FLAG_WS_UNSTORED 64 /* ksana_sage_forward* only, with KSANA_SAGE_FLAG_Q_UNSTORED: the caller reads nothing  */
+                                       /* from the workspace afterwards and o overlaps none of q, k, v.  A call that          */
+                                       /* ksana_sage_forward_scratch gives no bytes for then runs in one launch that touches  */
+                                       /* no workspace.  Same bits.                                                           */
 
 typedef struct ksana_sage_shape {
   int32_t B;   /* batch                                                     */
@@ -386,6 +391,11 @@ int ksana_sage_forward_prep(const void* q, const void* k, const void* v, void* o
                             const int64_t o_strides[4], const ksana_sage_shape* shape, const ksana_sage_prep* prep,
                             const int32_t* k_lens, float sm_scale, int smooth_k, int causal, int flags,
                             void* workspace, void* stream);
+
+/* *bytes = the workspace a ksana_sage_forward* call needs: the layout's total_bytes, or 0 for a call without `prep` and block
+ * mask, with o of the inputs' type and KSANA_SAGE_FLAG_Q_UNSTORED | KSANA_SAGE_FLAG_WS_UNSTORED as its only flags, that is
+ * short enough for one launch (its workspace may then be NULL).  No counterpart in the reference. */
+int ksana_sage_forward_scratch(const ksana_sage_shape* shape, int flags, uint64_t* bytes);
 
 /* ksana_sage_forward with the block mask of ksana_sage_attn_fwd_masked. */
 int ksana_sage_forward_masked(const void* q, const void* k, const void* v, void* o, int dtype,

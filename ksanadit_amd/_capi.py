@@ -11,7 +11,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libksana_sage_hip.so"
-ABI_VERSION = 22
+ABI_VERSION = 23
 
 BF16, FP16 = 0, 1
 OK, EINVAL, ENOTSUP, EHIP = 0, -1, -2, -3
@@ -21,6 +21,7 @@ FLAG_WG_4_WAVES = 4
 FLAG_WG_8_WAVES = 8
 FLAG_TILE_SKIP = 16
 FLAG_Q_UNSTORED = 32
+FLAG_WS_UNSTORED = 64
 PREP_WAN, PREP_WAN_COMFY, PREP_QWEN = 0, 1, 2
 KEEP = -(2**63)  # KSANA_SAGE_KEEP
 
@@ -54,6 +55,7 @@ EXPORTS = (
     "ksana_sage_attn_fwd_varlen",
     "ksana_sage_forward_masked",
     "ksana_sage_forward_varlen",
+    "ksana_sage_forward_scratch",
 )
 
 
@@ -111,6 +113,7 @@ def _declare(lib):
     lib.ksana_sage_one_read_state.argtypes = [C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int64), C.POINTER(C.c_int)]
     lib.ksana_sage_one_read_state.restype = i
     lib.ksana_sage_selftest.argtypes, lib.ksana_sage_selftest.restype = [], i
+    lib.ksana_sage_forward_scratch.argtypes, lib.ksana_sage_forward_scratch.restype = [sp, i, C.POINTER(C.c_uint64)], i
     lib.ksana_sage_quant_q.argtypes, lib.ksana_sage_quant_q.restype = [vp, i, st, sp, f, vp, vp], i
     lib.ksana_sage_quant_k.argtypes, lib.ksana_sage_quant_k.restype = [vp, i, st, sp, i, vp, vp], i
     lib.ksana_sage_quant_k_static.argtypes, lib.ksana_sage_quant_k_static.restype = [vp, i, st, sp, i, vp, vp], i

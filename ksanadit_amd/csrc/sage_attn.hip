@@ -19,8 +19,7 @@
 // The int32 accumulators start at the bit pattern of 1.5 * 2^23 ("magic"): the result read
 // as fp32 IS 12582912 + dot exactly (|dot| <= 127*127*128 < 2^22), which removes the
 // int->float conversion from the softmax: p = exp2(fma(acc_as_float, sc, c)).
-#include "sage_device.h"
-#include "sage_kernels.h"
+#include "sage_attn_device.h"
 
 #include <atomic>
 #include <type_traits>
@@ -29,12 +28,6 @@
 
 namespace ksana_sage {
 namespace {
-
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 // Two shapes of workgroup: 8 waves = 256 query rows with an 8-stage tile ring (one workgroup holds a compute unit:
 // every K/V tile copied serves 256 rows), and 4 waves = 128 query rows with a 4-stage ring, two of which share a
@@ -65,31 +58,10 @@ struct WgShape {
   // 515 -> 501 us at B=2, 16 heads of 64 channels, 9001 tokens.
   static constexpr int kGroup = kW == 8 ? 4 : 1;
 };
-constexpr int kMagicI = 0x4B400000;       // bits of 12582912.0f = 1.5 * 2^23: fp32 values are 1 apart there
-constexpr float kMagicF = 12582912.0f;
-// Head size 64 runs on rows whose upper 64 channels are zeros before the Hadamard transform - and a copy of the lower
-// 64 after it (H128 [x; 0] = [H64 x; H64 x]): the dot product over 128 channels is twice the one over the lower 64.
-// The kernel then multiplies the lower half only and starts its accumulators at 1.5 * 2^24, where fp32 values are 2
-// apart: the bits read as fp32 are 25165824 + 2 * dot, the full product, with no instruction spent on the doubling
-// (|dot| <= 127 * 127 * 64 < 2^21).
-constexpr int kMagicI2 = 0x4BC00000;      // bits of 25165824.0f = 1.5 * 2^24
-constexpr float kMagicF2 = 25165824.0f;
-// P is scaled by 2^6 before the e4m3 cast, and the reference point of a row (its "running maximum") is moved only when
-// a tile's maximum exceeds it by more than kLazyMax octaves: probabilities then reach 2^(6 + 2.7) = 416 < 448, the
-// largest e4m3 value, and the accumulators are rescaled in a few per cent of the steps instead of up to half of them
-// (rows of flat attention set a new maximum every few tiles, by small amounts).  An e4m3 rounding does not depend on
-// the power of two in front, so the result differs only where probabilities fall off the subnormal end, 2^-15 of the
-// reference point.
-// The piecewise-linear path keeps 2^8 and moves the reference point at every new maximum: its code formula is wrong
-// for the subnormal codes (it fades them linearly), which must stay 2^-14 below the true maximum to be harmless.
-constexpr float kPShift = 6.0f, kPShiftPwl = 8.0f;
-constexpr float kLazyMax = 2.7f, kLazyMaxPwl = 0.0f;
 constexpr int kSparseMaxKeyTiles4 = 2048;    // 4-wave workgroups keep their tile list as 16-bit entries so that two fit a compute unit
 constexpr int kMaxKeyTiles = 4096;           // K scales of one head are kept in LDS: Lk <= 262144
 constexpr int kShortKeyTiles = 16;           // calls with at most this many key tiles (Lk <= 1024) are never cut into runs of keys
 constexpr int kShortMaxKeyTiles = 2048;      // the most key tiles a dense 4-wave workgroup can hold scales for
-
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // 16 bytes per lane from global memory straight into LDS at `lds_dst + 16 * lane` (lds_dst is
 // wave-uniform).  Written as inline assembly on purpose: the compiler's wait-count model treats
@@ -120,114 +92,6 @@ __device__ __forceinline__ void lds_copy16_at(const v4i& buffer, unsigned lane_o
 }
 #pragma clang diagnostic pop
 
-// Opaque use+def at this program point: keeps the optimizer from sinking the computation of
-// `x` into a later basic block (it emits no instruction).
-template <typename T>
-__device__ __forceinline__ void pin(T& x) {
-  asm volatile("" : "+v"(x));
-}
-
-template <int DT>
-__device__ __forceinline__ uint2 half4(float a, float b, float c, float d) {
-  uint32_t lo, hi;
-  if constexpr (DT == KSANA_SAGE_BF16) {
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    b2 x = {(__bf16)a, (__bf16)b}, y = {(__bf16)c, (__bf16)d};
-    lo = __builtin_bit_cast(uint32_t, x);
-    hi = __builtin_bit_cast(uint32_t, y);
-  } else {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    h2 x = {(_Float16)a, (_Float16)b}, y = {(_Float16)c, (_Float16)d};
-    lo = __builtin_bit_cast(uint32_t, x);
-    hi = __builtin_bit_cast(uint32_t, y);
-  }
-  return make_uint2(lo, hi);
-}
-template <int DT>
-__device__ __forceinline__ void store4(uint16_t* dst, float a, float b, float c, float d) {
-  *reinterpret_cast<uint2*>(dst) = half4<DT>(a, b, c, d);
-}
-
-// S^T tile (64 keys x 32 queries) of one wave: two 32-key sub-tiles, kG 32-channel steps (the channel groups that
-// hold data: 4, or 2 for head size 64, whose upper 64 channels are zeros on both sides).
-template <int kG>
-__device__ __forceinline__ void qk_tile(const uint8_t* k_stage, int lane, const v4i (&qf)[4], const v16i& magic,
-                                        v16i (&acc)[2]) {
-  acc[0] = magic;
-  acc[1] = magic;
-#pragma unroll
-  for (int s = 0; s < kG; ++s) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const v4i kf = *reinterpret_cast<const v4i*>(k_stage + ((t * 4 + s) * 64 + lane) * 16);
-      acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[s], acc[t], 0, 0, 0);
-    }
-  }
-}
-
-// Q quantized where it is used.  Lane l of a wave holds the channels 32 s + 16 (l / 32) + 0 .. 15, s < kG, of the wave's row
-// l % 32 - those of its matrix operand - so the row's transform is strides 1 .. 8 inside sixteen channels, 16 between lanes
-// l and l ^ 32, 32 and 64 between the groups: the order, the roundings and therefore the bits of the separate quantizer
-// (fwht128, pack_int8x16).  Head size 64 (kG == 2): the upper half of an extended row repeats the lower, so stride 64 and
-// the row's other half change nothing.  Bound by its latency in the set-up (two or three waves' worth of instructions per
-// SIMD, all at once); what it saves is the quantizer's pass over Q, which is HBM-bound.  Whole calls, us, before / with it:
-// 32760 queries on 512 keys, 40 heads 373 / 336; padded batch (B=3, 24 heads, 3001 x 4099) 210 / 202; causal 8191, 32 heads
-// 352 / 345; 9001 tokens of 64 channels, B=2, 16 heads 563 / 557.  Which calls take it: q_in_attention_pays.
-template <int DT, int kG>
-__device__ __forceinline__ void quant_q_rows(const uint4 (&raw)[8], float premul, v4i (&qf)[4], float& qs) {
-  float x[kG][16];
-#pragma unroll
-  for (int s = 0; s < kG; ++s) {
-    widen8<DT>(raw[2 * s], x[s]);
-    widen8<DT>(raw[2 * s + 1], x[s] + 8);
-#pragma unroll
-    for (int st = 1; st < 16; st <<= 1)
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
-        if ((i & st) == 0) {
-          const float a = x[s][i], b = x[s][i + st];
-          x[s][i] = a + b;
-          x[s][i + st] = a - b;
-        }
-    // two values at a time: the first swap gives the lower lanes both ends of the first value's butterfly and the upper
-    // lanes both ends of the second's, the second swap takes the results home
-#pragma unroll
-    for (int i = 0; i < 16; i += 2) {
-      const auto ab = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[s][i]), __float_as_uint(x[s][i + 1]), false, false);
-      const float a = __uint_as_float(ab[0]), b = __uint_as_float(ab[1]);
-      const auto home = __builtin_amdgcn_permlane32_swap(__float_as_uint(a + b), __float_as_uint(a - b), false, false);
-      x[s][i] = __uint_as_float(home[0]);
-      x[s][i + 1] = __uint_as_float(home[1]);
-    }
-  }
-#pragma unroll
-  for (int st = 1; st < kG; st <<= 1)
-#pragma unroll
-    for (int s = 0; s < kG; ++s)
-      if ((s & st) == 0)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const float a = x[s][i], b = x[s + st][i];
-          x[s][i] = a + b;
-          x[s + st][i] = a - b;
-        }
-  float amax = 0.0f;
-#pragma unroll
-  for (int s = 0; s < kG; ++s)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      x[s][i] = x[s][i] * premul;
-      amax = fmaxf(amax, fabsf(x[s][i]));
-    }
-  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
-  amax = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
-  const bool nz = amax > 0.0f;
-  const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
-  qs = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
-#pragma unroll
-  for (int s = 0; s < kG; ++s) qf[s] = __builtin_bit_cast(v4i, pack_int8x16(x[s], inv));
-}
-
 // Dense 8-wave calls can hold two kinds of workgroup in one grid: blocks below p.split_first_block walk all key tiles of
 // their (head, query block); each of the blocks from there on takes one of `p.n_split` equal runs of key tiles and leaves
 // unnormalised accumulators, running maxima and row sums in the workspace for sage_attn_merge_kernel.  The runs stand
@@ -239,6 +103,7 @@ __device__ __forceinline__ void quant_q_rows(const uint4 (&raw)[8], float premul
 template <int DT, bool kPwlExp, bool kSparse, int kW, bool kTileSkip, int kG, bool kCausal>
 __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel(const AttnParams p, int n_qwg,
                                                                                    int n_wg, int wg_per_xcd) {
+  want(p.q_rows.ptr, p.k_tiles, p.o.sH, p.block_mask, n_qwg);
   constexpr bool kCanSplit = !kSparse && kW == 8;
   static_assert(kSparse || !kCausal || (kW == 4 && !kPwlExp && !kTileSkip), "causal without a list: the default variant in 4 waves");
   // kCausal == false: the caller vouches that p.causal is 0, and everything that serves the diagonal (the per-wave

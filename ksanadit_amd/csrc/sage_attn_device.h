@@ -1,0 +1,146 @@
+// What the attention kernels share: matrix operand types, the constants of the softmax, the S^T product of a tile and Q
+// quantized in the layout its matrix operand wants.
+#pragma once
+
+#include "sage_device.h"
+#include "sage_kernels.h"
+
+namespace ksana_sage {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+constexpr int kMagicI = 0x4B400000;       // bits of 12582912.0f = 1.5 * 2^23: fp32 values are 1 apart there
+constexpr float kMagicF = 12582912.0f;
+// Head size 64 runs on rows whose upper 64 channels are zeros before the Hadamard transform - and a copy of the lower
+// 64 after it (H128 [x; 0] = [H64 x; H64 x]): the dot product over 128 channels is twice the one over the lower 64.
+// The kernel then multiplies the lower half only and starts its accumulators at 1.5 * 2^24, where fp32 values are 2
+// apart: the bits read as fp32 are 25165824 + 2 * dot, the full product, with no instruction spent on the doubling
+// (|dot| <= 127 * 127 * 64 < 2^21).
+constexpr int kMagicI2 = 0x4BC00000;      // bits of 25165824.0f = 1.5 * 2^24
+constexpr float kMagicF2 = 25165824.0f;
+// P is scaled by 2^6 before the e4m3 cast, and the reference point of a row (its "running maximum") is moved only when
+// a tile's maximum exceeds it by more than kLazyMax octaves: probabilities then reach 2^(6 + 2.7) = 416 < 448, the
+// largest e4m3 value, and the accumulators are rescaled in a few per cent of the steps instead of up to half of them
+// (rows of flat attention set a new maximum every few tiles, by small amounts).  An e4m3 rounding does not depend on
+// the power of two in front, so the result differs only where probabilities fall off the subnormal end, 2^-15 of the
+// reference point.
+// The piecewise-linear path keeps 2^8 and moves the reference point at every new maximum: its code formula is wrong
+// for the subnormal codes (it fades them linearly), which must stay 2^-14 below the true maximum to be harmless.
+constexpr float kPShift = 6.0f, kPShiftPwl = 8.0f;
+constexpr float kLazyMax = 2.7f, kLazyMaxPwl = 0.0f;
+
+__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// Opaque use+def at this program point: keeps the optimizer from sinking the computation of
+// `x` into a later basic block (it emits no instruction).
+template <typename T>
+__device__ __forceinline__ void pin(T& x) {
+  asm volatile("" : "+v"(x));
+}
+
+template <int DT>
+__device__ __forceinline__ uint2 half4(float a, float b, float c, float d) {
+  uint32_t lo, hi;
+  if constexpr (DT == KSANA_SAGE_BF16) {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    b2 x = {(__bf16)a, (__bf16)b}, y = {(__bf16)c, (__bf16)d};
+    lo = __builtin_bit_cast(uint32_t, x);
+    hi = __builtin_bit_cast(uint32_t, y);
+  } else {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    h2 x = {(_Float16)a, (_Float16)b}, y = {(_Float16)c, (_Float16)d};
+    lo = __builtin_bit_cast(uint32_t, x);
+    hi = __builtin_bit_cast(uint32_t, y);
+  }
+  return make_uint2(lo, hi);
+}
+template <int DT>
+__device__ __forceinline__ void store4(uint16_t* dst, float a, float b, float c, float d) {
+  *reinterpret_cast<uint2*>(dst) = half4<DT>(a, b, c, d);
+}
+
+// S^T tile (64 keys x 32 queries) of one wave: two 32-key sub-tiles, kG 32-channel steps (the channel groups that
+// hold data: 4, or 2 for head size 64, whose upper 64 channels are zeros on both sides).
+template <int kG>
+__device__ __forceinline__ void qk_tile(const uint8_t* k_stage, int lane, const v4i (&qf)[4], const v16i& magic,
+                                        v16i (&acc)[2]) {
+  acc[0] = magic;
+  acc[1] = magic;
+#pragma unroll
+  for (int s = 0; s < kG; ++s) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const v4i kf = *reinterpret_cast<const v4i*>(k_stage + ((t * 4 + s) * 64 + lane) * 16);
+      acc[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf, qf[s], acc[t], 0, 0, 0);
+    }
+  }
+}
+
+// Q quantized where it is used.  Lane l of a wave holds the channels 32 s + 16 (l / 32) + 0 .. 15, s < kG, of the wave's row
+// l % 32 - those of its matrix operand - so the row's transform is strides 1 .. 8 inside sixteen channels, 16 between lanes
+// l and l ^ 32, 32 and 64 between the groups: the order, the roundings and therefore the bits of the separate quantizer
+// (fwht128, pack_int8x16).  Head size 64 (kG == 2): the upper half of an extended row repeats the lower, so stride 64 and
+// the row's other half change nothing.  Bound by its latency in the set-up (two or three waves' worth of instructions per
+// SIMD, all at once); what it saves is the quantizer's pass over Q, which is HBM-bound.  Whole calls, us, before / with it:
+// 32760 queries on 512 keys, 40 heads 373 / 336; padded batch (B=3, 24 heads, 3001 x 4099) 210 / 202; causal 8191, 32 heads
+// 352 / 345; 9001 tokens of 64 channels, B=2, 16 heads 563 / 557.  Which calls take it: q_in_attention_pays.
+template <int DT, int kG>
+__device__ __forceinline__ void quant_q_rows(const uint4 (&raw)[8], float premul, v4i (&qf)[4], float& qs) {
+  float x[kG][16];
+#pragma unroll
+  for (int s = 0; s < kG; ++s) {
+    widen8<DT>(raw[2 * s], x[s]);
+    widen8<DT>(raw[2 * s + 1], x[s] + 8);
+#pragma unroll
+    for (int st = 1; st < 16; st <<= 1)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if ((i & st) == 0) {
+          const float a = x[s][i], b = x[s][i + st];
+          x[s][i] = a + b;
+          x[s][i + st] = a - b;
+        }
+    // two values at a time: the first swap gives the lower lanes both ends of the first value's butterfly and the upper
+    // lanes both ends of the second's, the second swap takes the results home
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) {
+      const auto ab = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[s][i]), __float_as_uint(x[s][i + 1]), false, false);
+      const float a = __uint_as_float(ab[0]), b = __uint_as_float(ab[1]);
+      const auto home = __builtin_amdgcn_permlane32_swap(__float_as_uint(a + b), __float_as_uint(a - b), false, false);
+      x[s][i] = __uint_as_float(home[0]);
+      x[s][i + 1] = __uint_as_float(home[1]);
+    }
+  }
+#pragma unroll
+  for (int st = 1; st < kG; st <<= 1)
+#pragma unroll
+    for (int s = 0; s < kG; ++s)
+      if ((s & st) == 0)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float a = x[s][i], b = x[s + st][i];
+          x[s][i] = a + b;
+          x[s + st][i] = a - b;
+        }
+  float amax = 0.0f;
+#pragma unroll
+  for (int s = 0; s < kG; ++s)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      x[s][i] = x[s][i] * premul;
+      amax = fmaxf(amax, fabsf(x[s][i]));
+    }
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
+  amax = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+  const bool nz = amax > 0.0f;
+  const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
+  qs = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+#pragma unroll
+  for (int s = 0; s < kG; ++s) qf[s] = __builtin_bit_cast(v4i, pack_int8x16(x[s], inv));
+}
+
+}  // namespace ksana_sage

@@ -194,6 +194,11 @@ int check_causal(const ksana_sage_shape* s, int causal) {
   return 0;
 }
 
+// Does a call without a folded step and a block mask, of one type throughout, run in one launch without a workspace?
+bool in_one_launch(const ksana_sage_shape* s, int flags) {
+  return flags == (KSANA_SAGE_FLAG_Q_UNSTORED | KSANA_SAGE_FLAG_WS_UNSTORED) && ksana_sage::small_call_suits(s->B, s->Hq, s->Lq, s->Lk);
+}
+
 // the factor a transformed row of Q takes before it is rounded to int8
 float q_premul_of(float sm_scale) { return (sm_scale * 1.4426950408889634f) * 0.0078125f; }
 
@@ -352,6 +357,15 @@ int ksana_sage_workspace_layout(const ksana_sage_shape* s, ksana_sage_ws_layout*
   l.v_sync = take((uint64_t)sync_words((int)bhk) * 4);
   l.total_bytes = off;
   *out = l;
+  return 0;
+}
+
+int ksana_sage_forward_scratch(const ksana_sage_shape* s, int flags, uint64_t* bytes) {
+  if (int rc = check_shape(s)) return rc;
+  if (!bytes) return fail(KSANA_SAGE_EINVAL, "out-pointer is null");
+  ksana_sage_ws_layout l;
+  ksana_sage_workspace_layout(s, &l);
+  *bytes = in_one_launch(s, flags) ? 0 : l.total_bytes;
   return 0;
 }
 
@@ -822,14 +836,25 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
   if (int rc = check_tensor("k", k, dtype, k_st, s->B, s->Lk, s->Hkv)) return rc;
   if (int rc = check_tensor("v", v, dtype, v_st, s->B, s->Lk, s->Hkv)) return rc;
   if (int rc = check_tensor("o", o, o_dtype, o_st, s->B, s->Lq, s->Hq)) return rc;
-  if (int rc = check_ws(ws)) return rc;
+  const bool small = prep == nullptr && block_mask == nullptr && o_dtype == dtype && in_one_launch(s, flags);
+  if (!small)
+    if (int rc = check_ws(ws)) return rc;
   if (flags & ~(KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_SMOOTH_V | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES |
-                KSANA_SAGE_FLAG_TILE_SKIP | KSANA_SAGE_FLAG_Q_UNSTORED))
+                KSANA_SAGE_FLAG_TILE_SKIP | KSANA_SAGE_FLAG_Q_UNSTORED | KSANA_SAGE_FLAG_WS_UNSTORED))
     return fail(KSANA_SAGE_EINVAL, "unknown flag bits 0x%x", flags);
   if ((flags & KSANA_SAGE_FLAG_TILE_SKIP) && (flags & KSANA_SAGE_FLAG_PWL_EXP2))
     return fail(KSANA_SAGE_EINVAL, "KSANA_SAGE_FLAG_TILE_SKIP goes with the exact exponential only, not with KSANA_SAGE_FLAG_PWL_EXP2");
   if (reinterpret_cast<uintptr_t>(k_lens) & 3) return fail(KSANA_SAGE_EINVAL, "k_lens is not 4-byte aligned");
   if (reinterpret_cast<uintptr_t>(q_lens) & 3) return fail(KSANA_SAGE_EINVAL, "q_lens is not 4-byte aligned");
+  if (small) {
+    const StageRange range("ksana_sage.small");
+    const ksana_sage::SmallCall c{in_tensor(q, dtype, q_st, s->D), in_tensor(k, dtype, k_st, s->D), in_tensor(v, dtype, v_st, s->D),
+                                  ksana_sage::OutTensor{static_cast<uint16_t*>(o), o_st[0], o_st[1], o_st[2], o_dtype},
+                                  s->B, s->Hq, s->Hkv, s->Lq, s->Lk, q_premul_of(sm_scale), smooth_k ? 1 : 0, causal ? 1 : 0, s->D,
+                                  q_lens, k_lens};
+    const hipError_t e = ksana_sage::launch_small(c, static_cast<hipStream_t>(stream));
+    return e == hipSuccess ? 0 : hip_fail(e, "one-launch attention");
+  }
   {
     ksana_sage::PrepParams pp;
     const ksana_sage::PrepParams* ppp = nullptr;
@@ -847,7 +872,7 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
     return rc;
   const ksana_sage::InTensor q_rows = in_tensor(q, dtype, q_st, s->D);
   return attn_impl(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal,
-                   flags & ~(KSANA_SAGE_FLAG_SMOOTH_V | KSANA_SAGE_FLAG_Q_UNSTORED), own_q ? &q_rows : nullptr, q_premul_of(sm_scale),
+                   flags & ~(KSANA_SAGE_FLAG_SMOOTH_V | KSANA_SAGE_FLAG_Q_UNSTORED | KSANA_SAGE_FLAG_WS_UNSTORED), own_q ? &q_rows : nullptr, q_premul_of(sm_scale),
                    stream);
 }
 }  // namespace

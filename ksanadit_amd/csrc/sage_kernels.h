@@ -205,13 +205,13 @@ struct AttnParams {
   float* split_ml;
   int split_first_block = 0, split_first_wg = 0, n_split = 0;  // filled in by the launcher
   int batch_run = 0;  // filled in by the launcher: 0, or the workgroups of one batch entry that go to one XCD
-  // filled in by the launcher for causal calls: (batch, head) pairs an XCD has to itself, the pairs left over, and how many
-  // of its own it walks through together (0: not a causal call, or one numbered by batch_run)
-  int causal_own = 0, causal_rest = 0, causal_group = 0;
   int wg_waves;  // 0: the launcher picks the workgroup shape; 4 or 8: forced (for measurements and tests)
   int d_out;     // channels of an output row that exist: 128, or 64 (head size 64 runs zero-padded to 128)
   int tile_skip; // 1: a wave leaves out the exponentials of a key tile whose probabilities would all be the zero code
                  // (same bits; pays on sharply peaked attention, costs 7-13 % where no tile qualifies); 0: every tile in full
+  // filled in by the launcher for causal calls: (batch, head) pairs an XCD has to itself, the pairs left over, and how many
+  // of its own it walks through together (0: not a causal call, or one numbered by batch_run)
+  int causal_own = 0, causal_rest = 0, causal_group = 0;
 };
 constexpr int kMaxSplitPartials = 256;  // (workgroups beyond the last full round) x (runs each) never exceeds this
 constexpr int kMinTilesPerSplit = 8;    // a run shorter than this does not repay its prologue
@@ -223,5 +223,17 @@ hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t s);
 void plan_key_split(int n_wg, int nkb, int* first_wg, int* runs);
 // Is a call with `n_wg` 256-row query blocks and `nkb` key tiles faster when the attention kernel quantizes Q itself?
 bool q_in_attention_pays(int n_wg, int nkb);
+
+// A whole call of at most kMeanChunk keys in one launch (sage_small.hip): q, k and v as the caller has them, o of their type.
+struct SmallCall {
+  InTensor q, k, v;
+  OutTensor o;
+  int B, Hq, Hkv, Lq, Lk;
+  float premul;
+  int smooth_k, causal, d_out;
+  const int32_t *q_lens, *k_lens;  // as in AttnParams
+};
+bool small_call_suits(int B, int Hq, int Lq, int Lk);
+hipError_t launch_small(const SmallCall& c, hipStream_t s);
 
 }  // namespace ksana_sage

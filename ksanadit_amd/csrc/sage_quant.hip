@@ -42,21 +42,6 @@ __device__ __forceinline__ void store_out16(void* p, uint4 v) {
   __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(p));
 }
 
-// The same row as it sits in memory (two 16-byte loads), for code that wants the next row in flight while it works
-// on the current one.
-__device__ __forceinline__ void fetch_row16(const uint16_t* row_ptr, bool valid, uint4 (&raw)[2]) {
-  raw[0] = raw[1] = make_uint4(0, 0, 0, 0);
-  if (valid) {
-    raw[0] = *reinterpret_cast<const uint4*>(row_ptr);
-    raw[1] = *reinterpret_cast<const uint4*>(row_ptr + 8);
-  }
-}
-
-__device__ __forceinline__ float round_to_half_dtype(float x, int dtype) {
-  if (dtype == KSANA_SAGE_BF16) return (float)(__bf16)x;
-  return (float)(_Float16)x;
-}
-
 // ---------------------------------------------------------------------------------------
 // The step before attention, on the 16 channels [16*c16, 16*c16+16) of head h, token `row`:
 //   y = half( (x * inv_rms[row]) * weight[ch] )                         RMSNorm, fp32, in this order
@@ -157,8 +142,6 @@ __device__ __forceinline__ int small_div(int n, int d, int* rem) {
   return q;
 }
 
-template <int M>
-__device__ __forceinline__ float lane_xor(float v);
 
 // The Qwen-Image block's step before attention on the 16 channels [16*c16, 16*c16+16) of one head of token `row`
 // (the 8 lanes c16 = 0..7 of the row are adjacent):
@@ -533,104 +516,6 @@ __global__ __launch_bounds__(kFinThreads) void v_scale_finalize_kernel(const flo
     v_inv[bh * kD + threadIdx.x] = nz ? __fdiv_rn(448.0f, amax) : 0.0f;
     if (zero_mean != nullptr) zero_mean[bh * kD + threadIdx.x] = 0.0f;
   }
-}
-
-// Value of lane (id ^ M) for M = 1, 2, 4, through DPP (the exchange then rides on the consuming
-// VALU instruction instead of a round trip through the LDS crossbar).
-//   quad_perm [1,0,3,2] = id ^ 1;  quad_perm [2,3,0,1] = id ^ 2;
-//   row_half_mirror (id -> 7 - id within 8 lanes) followed by quad_perm [3,2,1,0] (id ^ 3) = id ^ 4.
-template <int M>
-__device__ __forceinline__ float lane_xor(float v) {
-  static_assert(M == 1 || M == 2 || M == 4, "only within groups of 8 lanes");
-  const int iv = __float_as_int(v);
-  if constexpr (M == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(iv, 0xB1, 0xF, 0xF, true));
-  if constexpr (M == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(iv, 0x4E, 0xF, 0xF, true));
-  const int t = __builtin_amdgcn_mov_dpp(iv, 0x141, 0xF, 0xF, true);
-  return __int_as_float(__builtin_amdgcn_mov_dpp(t, 0x1B, 0xF, 0xF, true));
-}
-
-// One butterfly stage across lanes c16 and c16 ^ M: every lane takes `own + sign * other` with sign = -1 on the lane
-// that holds the "b" half of a pair.  That lane ought to take `other - own`: it ends up with the negative of its
-// value, exactly (a sum and its mirror image round alike).  Both lanes of any LATER stage's pair agree in bit M of
-// c16, so they carry the same factor and the later butterfly is the mirror image of the right one as a whole: after
-// the three stages a lane holds its transform times (-1)^popcount(c16), which the caller folds into the factor it
-// multiplies with next (fwht_lane_sign).  Written this way the stage is one multiply-add per value whose first
-// operand arrives through DPP - no separate sign flip, and no register written just ahead of the DPP read.
-// The instruction is written out: the compiler keeps the DPP move and the multiply-add apart (two instructions per
-// value).  Eight values per statement; `s_nop 1` in front gives the two wait states a DPP read needs after a
-// vector-ALU write of the same register, whatever instruction the compiler placed just before; inside a statement
-// every register is read at least eight instructions after it was written.
-#define KSANA_FMAC_DPP8(CTRL)                                                                                      \
-  "v_fmac_f32_dpp %0, %0, %8 " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"                                 \
-  "v_fmac_f32_dpp %1, %1, %8 " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"                                 \
-  "v_fmac_f32_dpp %2, %2, %8 " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"                                 \
-  "v_fmac_f32_dpp %3, %3, %8 " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"                                 \
-  "v_fmac_f32_dpp %4, %4, %8 " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"                                 \
-  "v_fmac_f32_dpp %5, %5, %8 " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"                                 \
-  "v_fmac_f32_dpp %6, %6, %8 " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"                                 \
-  "v_fmac_f32_dpp %7, %7, %8 " CTRL " row_mask:0xf bank_mask:0xf bound_ctrl:1"
-template <int M>
-__device__ __forceinline__ void fwht_cross_stage(float* x, int c16) {
-  const float sign = (c16 & M) ? -1.0f : 1.0f;
-#pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    float* y = x + 8 * g;
-    if constexpr (M == 1) {
-      asm volatile("s_nop 1\n\t" KSANA_FMAC_DPP8("quad_perm:[1,0,3,2]")
-                   : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]), "+v"(y[4]), "+v"(y[5]), "+v"(y[6]), "+v"(y[7])
-                   : "v"(sign));
-    } else if constexpr (M == 2) {
-      asm volatile("s_nop 1\n\t" KSANA_FMAC_DPP8("quad_perm:[2,3,0,1]")
-                   : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]), "+v"(y[4]), "+v"(y[5]), "+v"(y[6]), "+v"(y[7])
-                   : "v"(sign));
-    } else {
-      // lane ^ 4 within 8 = row_half_mirror (lane -> 7 - lane) followed by quad_perm [3,2,1,0] (lane ^ 3)
-      float t[8];
-      asm volatile("s_nop 1\n\t"
-                   "v_mov_b32_dpp %8, %0 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_mov_b32_dpp %9, %1 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_mov_b32_dpp %10, %2 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_mov_b32_dpp %11, %3 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_mov_b32_dpp %12, %4 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_mov_b32_dpp %13, %5 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_mov_b32_dpp %14, %6 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_mov_b32_dpp %15, %7 row_half_mirror row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_fmac_f32_dpp %0, %8, %16 quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_fmac_f32_dpp %1, %9, %16 quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_fmac_f32_dpp %2, %10, %16 quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_fmac_f32_dpp %3, %11, %16 quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_fmac_f32_dpp %4, %12, %16 quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_fmac_f32_dpp %5, %13, %16 quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_fmac_f32_dpp %6, %14, %16 quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
-                   "v_fmac_f32_dpp %7, %15, %16 quad_perm:[3,2,1,0] row_mask:0xf bank_mask:0xf bound_ctrl:1"
-                   : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]), "+v"(y[3]), "+v"(y[4]), "+v"(y[5]), "+v"(y[6]), "+v"(y[7]),
-                     "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2]), "=&v"(t[3]), "=&v"(t[4]), "=&v"(t[5]), "=&v"(t[6]), "=&v"(t[7])
-                   : "v"(sign));
-    }
-  }
-}
-
-// The factor fwht128 leaves on the values of lane c16 (see fwht_cross_stage).
-__device__ __forceinline__ float fwht_lane_sign(int c16) { return (__popc(c16 & 7) & 1) ? -1.0f : 1.0f; }
-
-// Unnormalised Walsh-Hadamard transform of one 128-channel row held by 8 adjacent lanes x 16
-// values (channel = 16*c16 + e), TIMES fwht_lane_sign(c16).  Butterflies (a, b) -> (a + b, a - b) with stride 1, 2,
-// 4, 8 inside the lane, then 16, 32, 64 across lanes c16 ^ 1, ^ 2, ^ 4 - in exactly that order.
-__device__ __forceinline__ void fwht128(float* x, int c16) {
-#pragma unroll
-  for (int s = 1; s < 16; s <<= 1) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      if ((i & s) == 0) {
-        const float a = x[i], b = x[i + s];
-        x[i] = a + b;
-        x[i + s] = a - b;
-      }
-    }
-  }
-  fwht_cross_stage<1>(x, c16);
-  fwht_cross_stage<2>(x, c16);
-  fwht_cross_stage<4>(x, c16);
 }
 
 // max over the workgroup of a non-negative per-thread value
@@ -1697,6 +1582,7 @@ __device__ __forceinline__ void quant_q_item(int item, const QkvCall& c, const P
 
 template <int DT, int KIND>
 __global__ __launch_bounds__(kThreads, KIND == 0 ? 5 : 4) void quant_qkv_stage1_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
+  want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   clear_status(c);
   const int n_v = c.B * c.Hkv * c.nch, n_k = c.smooth_k ? n_v : 0;
   int item = blockIdx.x;
@@ -1718,6 +1604,7 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 5 : 4) void quant_qkv_stage1_
 
 template <int DT, int KIND>
 __global__ __launch_bounds__(kThreads, KIND == 0 ? 6 : 5) void quant_qkv_stage2_kernel(const QkvCall c, const PrepParams pk) {
+  want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   __shared__ float s_stat[2][kD];
   const int per_head = (c.nkb + c.tiles_per_wg - 1) / c.tiles_per_wg, n = c.B * c.Hkv * per_head;
   const bool is_v = (int)blockIdx.x >= n;
@@ -1770,6 +1657,7 @@ __global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCa
 // at most 256 keys: one launch
 template <int DT, int KIND>
 __global__ __launch_bounds__(kThreads, 4) void quant_qkv_small_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
+  want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   clear_status(c);
   const int n = c.B * c.Hkv;
   const int item = blockIdx.x;

@@ -623,12 +623,15 @@ def attn_fwd(ws: SageWorkspace, out: torch.Tensor, causal: bool = False, pwl_exp
     return out
 
 
+_UNSTORED = _capi.FLAG_Q_UNSTORED | _capi.FLAG_WS_UNSTORED  # nobody sees the workspace after the call
+
+
 class _CallPlan:
     """What ``sageattn`` works out from the shapes, strides, dtypes and devices of q, k, v: whether the kernels can take
     them, the C structures the library reads and the workspace's size.  A model repeats a handful of shapes thousands of
     times; worked out anew in every call this was half of a small call's host time (25 us at B=2 L=32 H=64, 14 with it)."""
 
-    __slots__ = ("runs", "out_shape", "device", "dtype", "dtype_code", "shape", "shape_ptr", "ws_bytes", "q_st", "k_st", "v_st", "o_st",
+    __slots__ = ("runs", "out_shape", "device", "dtype", "dtype_code", "shape", "shape_ptr", "ws_bytes", "one_launch", "q_st", "k_st", "v_st", "o_st",
                  "_strides")
 
     def __init__(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor):
@@ -640,6 +643,9 @@ class _CallPlan:
         B, Lq, Hq, D = q.shape
         self.shape, layout = _capi.workspace_layout(B, Hq, k.shape[2], Lq, k.shape[1], D)
         self.shape_ptr, self.ws_bytes = C.addressof(self.shape), layout.total_bytes
+        scratch = C.c_uint64(0)
+        _capi.check(_capi.load().ksana_sage_forward_scratch(C.byref(self.shape), _UNSTORED, C.byref(scratch)), "ksana_sage_forward_scratch")
+        self.one_launch = scratch.value == 0  # (a call without options)
         out_strides = (Lq * Hq * D, Hq * D, D, 1)
         self._strides = [_strides(q), _strides(k), _strides(v), _capi.Strides(*out_strides)]  # (kept alive: addresses below)
         self.q_st, self.k_st, self.v_st, self.o_st = (C.addressof(x) for x in self._strides)
@@ -733,8 +739,14 @@ def sageattn(
         raise ValueError(f"out_dtype must be float16 or bfloat16, got {out_dtype}")
     out = torch.empty(plan.out_shape, dtype=result_dtype, device=device)
     sm_scale = D**-0.5 if sm_scale is None else float(sm_scale)
+    flags = (_capi.FLAG_PWL_EXP2 if pwl_exp2 else 0) | (_capi.FLAG_SMOOTH_V if smooth_v else 0)
+    flags |= _capi.FLAG_TILE_SKIP if tile_skip else 0
     if workspace is None:
-        blob = torch.empty(plan.ws_bytes, dtype=torch.uint8, device=device)  # (torch's blocks start at multiples of 512)
+        if plan.one_launch and flags == 0 and prep is None and block_mask is None and result_dtype == plan.dtype:
+            blob = None  # short calls leave nothing in memory but their result
+        else:
+            blob = torch.empty(plan.ws_bytes, dtype=torch.uint8, device=device)  # (torch's blocks start at multiples of 512)
+        flags |= _UNSTORED
     else:
         s = plan.shape
         workspace.require(device, B=s.B, Hq=s.Hq, Hkv=s.Hkv, Lq=s.Lq, Lk=s.Lk, D=s.D)
@@ -744,9 +756,6 @@ def sageattn(
         _log_demotion_once()
     kl = None if k_lens is None else _k_lens_arg(k_lens, B, device)
     ql = None if q_lens is None else _k_lens_arg(q_lens, B, device, "q_lens")
-    flags = (_capi.FLAG_PWL_EXP2 if pwl_exp2 else 0) | (_capi.FLAG_SMOOTH_V if smooth_v else 0)
-    flags |= _capi.FLAG_TILE_SKIP if tile_skip else 0
-    flags |= _capi.FLAG_Q_UNSTORED if workspace is None else 0  # nobody sees the workspace after the call
     prep_ptr = mask_ptr = mask_st = None
     if prep is not None:
         if block_mask is not None and q_lens is None and result_dtype == plan.dtype:
@@ -761,7 +770,7 @@ def sageattn(
     rc = lib.ksana_sage_forward_varlen(
         q_ptr, k_ptr, v_ptr, out.data_ptr(), plan.dtype_code, _DTYPES[result_dtype], plan.q_st, plan.k_st, plan.v_st, plan.o_st,
         plan.shape_ptr, prep_ptr, mask_ptr, mask_st, None if ql is None else ql.data_ptr(), None if kl is None else kl.data_ptr(),
-        sm_scale, int(smooth_k), int(is_causal), flags, blob.data_ptr(), _stream_ptr(device))
+        sm_scale, int(smooth_k), int(is_causal), flags, None if blob is None else blob.data_ptr(), _stream_ptr(device))
     if rc != _capi.OK:
         _capi.check(rc, "ksana_sage_forward")
     return out.transpose(1, 2) if hnd else out
