@@ -369,6 +369,18 @@ int ksana_sage_attn_fwd_varlen(void* workspace, void* o, int dtype, const int64_
  * emulation does); no counterpart in the reference. */
 int ksana_sage_attn_key_split(const ksana_sage_shape* shape, int* first_workgroup, int* runs);
 
+/* The sparse-linear backend's whole call (sage_sla.py:100-292): quantize q, k and v, the block map that keeps the `keep` key
+ * blocks of largest pooled score per 128 query rows, attention over the kept blocks, and the linear branch with the block's
+ * layer - o = sparse + (phi(q) kv) W^T / (1e-5 + phi(q) . sum phi(k)) + bias - in five launches.  The same results as
+ * ksana_sage_quant_qk_pooled, ksana_sage_quant_v, ksana_sage_sla_block_map, ksana_sage_attn_fwd_masked and
+ * ksana_sage_sla_linear in turn, the linear branch's row sums up to their order.  Head size 128, Hq == Hkv, Lq == Lk <= 65536, o
+ * overlaps none of q, k, v; proj_weight (fp32 [128][128], out x in) and proj_bias (fp32 [128]) may be NULL. */
+int ksana_sage_sla_forward_bytes(const ksana_sage_shape* shape, uint64_t* bytes);
+int ksana_sage_sla_forward(const void* q, const void* k, const void* v, void* o, int dtype, const int64_t q_strides[4],
+                           const int64_t k_strides[4], const int64_t v_strides[4], const int64_t o_strides[4],
+                           const ksana_sage_shape* shape, float sm_scale, int keep, const float* proj_weight,
+                           const float* proj_bias, void* workspace, void* stream);
+
 /* Measurement aid, no counterpart in the reference: launches `workgroups` workgroups of 8 waves that each issue, `steps`
  * times, the attention kernel's matrix instructions per key tile (8 INT8 + 5 FP8 MFMAs) on register operands and
  * nothing else.  `scratch` receives workgroups * 512 floats (so the work is not optimised away); *ops_per_launch is the

@@ -56,6 +56,8 @@ EXPORTS = (
     "ksana_sage_forward_masked",
     "ksana_sage_forward_varlen",
     "ksana_sage_forward_scratch",
+    "ksana_sage_sla_forward_bytes",
+    "ksana_sage_sla_forward",
 )
 
 
@@ -132,6 +134,10 @@ def _declare(lib):
     lib.ksana_sage_sla_linear.argtypes = [vp, vp, vp, i, st, st, st, i, i, i, vp, vp, vp, st, vp, st, vp, vp]
     lib.ksana_sage_sla_linear.restype = i
     lib.ksana_sage_sla_block_map.argtypes, lib.ksana_sage_sla_block_map.restype = [vp, vp, i, i, i, i, i, i, vp, vp], i
+    lib.ksana_sage_sla_forward_bytes.argtypes = [sp, C.POINTER(C.c_uint64)]
+    lib.ksana_sage_sla_forward_bytes.restype = i
+    lib.ksana_sage_sla_forward.argtypes = [vp, vp, vp, vp, i, st, st, st, st, sp, f, i, vp, vp, vp, vp]
+    lib.ksana_sage_sla_forward.restype = i
     lib.ksana_sage_mfma_probe.argtypes = [vp, C.c_uint64, i, i, vp, C.POINTER(C.c_double)]
     lib.ksana_sage_mfma_probe.restype = i
     lib.ksana_sage_forward.argtypes = [vp, vp, vp, vp, i, st, st, st, st, sp, vp, f, i, i, i, vp, vp]

@@ -13,6 +13,9 @@ Drop-in for ksana/operations/attention/backends/sage_sla.py:100-292.  Per call (
    to the sparse result (sage_sla.py:273-287) - the HIP kernels behind ``ksana_sage_sla_linear``: one pass over k and
    v, one over q, with ``proj_l`` (when it is a plain ``torch.nn.Linear``) and the final sum folded in.
 
+With a plain linear ``proj_l`` and at most 65536 tokens of q, k, v of one shape, all of it is one library call
+(``ksana_sage_sla_forward``), in which the linear branch's pass over k and v takes the statistics of their quantizers along.
+
 The product of the block averages and the top-k selection are one HIP kernel (``ksana_sage_sla_block_map``; of two key
 blocks with equal products the lower index makes the cut - ``torch.topk``, which the reference calls, leaves that open).
 """
@@ -102,6 +105,12 @@ class SageSLAAttentionImpl(KsanaAttentionBackendImpl):
         dtype = query.dtype
         if dtype not in (torch.float16, torch.bfloat16):
             query, key, value = (t.to(torch.bfloat16) for t in (query, key, value))
+        nk = -(-key.shape[1] // MASK_BLKK)
+        if (isinstance(proj_l, torch.nn.Linear) and tuple(proj_l.weight.shape) == (query.shape[-1],) * 2 and query.numel() != 0
+                and query.shape == key.shape == value.shape and nk <= 1024):
+            keep = min(nk, int(self.topk * nk))
+            out = sage_ops.sla_forward(query, key, value, keep, proj_l.weight, proj_l.bias).to(dtype)
+            return (out, keep / nk) if return_sparsity else out
         # quantize once; the block map is built next to the quantized operands and drives the attention over them
         ws = sage_ops.workspace_for(query, key)
         pooled_q, pooled_k = sage_ops.quant_qk_pooled(query, key, ws, query.shape[-1] ** -0.5)  # averages ride along

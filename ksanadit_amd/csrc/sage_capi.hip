@@ -202,6 +202,24 @@ bool in_one_launch(const ksana_sage_shape* s, int flags) {
 // the factor a transformed row of Q takes before it is rounded to int8
 float q_premul_of(float sm_scale) { return (sm_scale * 1.4426950408889634f) * 0.0078125f; }
 
+// q, k and v of a call and where its workspace keeps what the quantizers make of them
+ksana_sage::QkvCall qkv_call(bool with_q, const ksana_sage::InTensor& q, const ksana_sage::InTensor& k, const ksana_sage::InTensor& v,
+                             const ksana_sage_shape* s, const ksana_sage_ws_layout& l, float sm_scale, int smooth_k, void* ws) {
+  ksana_sage::QkvCall c{};
+  c.q = q, c.k = k, c.v = v;
+  c.B = s->B, c.Hq = s->Hq, c.Hkv = s->Hkv, c.Lq = s->Lq, c.Lk = s->Lk, c.lq_pad = l.lq_pad, c.nkb = l.nkb, c.nch = l.nch;
+  c.nqb = with_q ? l.lq_pad / ksana_sage::kQPad : 0;
+  c.premul = q_premul_of(sm_scale);
+  c.smooth_k = smooth_k ? 1 : 0;
+  c.q_i8 = ws_at<int8_t>(ws, l.q_i8), c.q_scale = ws_at<float>(ws, l.q_scale);
+  c.k_part = ws_at<float>(ws, l.k_part), c.k_mean = ws_at<float>(ws, l.k_mean);
+  c.k_tiles = ws_at<int8_t>(ws, l.k_i8), c.k_scale = ws_at<float>(ws, l.k_scale);
+  c.v_part = ws_at<float>(ws, l.v_part), c.v_scale = ws_at<float>(ws, l.v_scale), c.v_inv = ws_at<float>(ws, l.v_inv);
+  c.v_mean = ws_at<float>(ws, l.v_mean), c.v_tiles = ws_at<uint8_t>(ws, l.v_fp8);
+  c.sync = sync_at(ws_at<int>(ws, l.k_sync), ws_at<int>(ws, l.v_sync), s->B * s->Hkv);
+  return c;
+}
+
 int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
               const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags,
               const ksana_sage::InTensor* q_rows, float q_premul, void* stream);
@@ -674,6 +692,79 @@ int ksana_sage_sla_block_map(const void* pooled_q, const void* pooled_k, int dty
   return e == hipSuccess ? 0 : hip_fail(e, "block map launch");
 }
 
+// Workspace of ksana_sage_sla_forward: the general layout, then the block averages, the map and the linear branch's areas
+struct SlaForwardLayout {
+  ksana_sage_ws_layout ws;
+  uint64_t pooled_q, pooled_k, map, part, m_frag, ksum, total;
+  int nq, nk;
+};
+static int sla_forward_layout(const ksana_sage_shape* s, SlaForwardLayout* out) {
+  if (int rc = check_shape(s)) return rc;
+  if (s->D != ksana_sage::kD || s->Hq != s->Hkv || s->Lq != s->Lk)
+    return fail(KSANA_SAGE_ENOTSUP, "the sparse-linear call needs head size 128, Hq == Hkv and Lq == Lk");
+  SlaForwardLayout l{};
+  ksana_sage_workspace_layout(s, &l.ws);
+  l.nq = (s->Lq + ksana_sage::kQPad - 1) / ksana_sage::kQPad, l.nk = l.ws.nkb;
+  if (l.nk > 1024) return fail(KSANA_SAGE_ENOTSUP, "Lk=%d: %d key blocks exceed 1024 (a group's scores are kept in LDS)", s->Lk, l.nk);
+  if ((int64_t)s->B * s->Hq > 65535) return fail(KSANA_SAGE_EINVAL, "B * H = %lld exceeds 65535", (long long)s->B * s->Hq);
+  const uint64_t bh = (uint64_t)s->B * s->Hq;
+  uint64_t part = 0, frag = 0, ksum = 0, sla = 0, off = align256(l.ws.total_bytes);
+  if (int rc = sla_layout(s->B, s->Hq, s->Lk, &part, &frag, &ksum, &sla)) return rc;
+  l.pooled_q = off, off = align256(off + bh * l.nq * ksana_sage::kD * 2);
+  l.pooled_k = off, off = align256(off + bh * l.nk * ksana_sage::kD * 2);
+  l.map = off, off = align256(off + bh * l.nq * l.nk);
+  l.part = off + part, l.m_frag = off + frag, l.ksum = off + ksum, l.total = off + sla;
+  *out = l;
+  return 0;
+}
+
+int ksana_sage_sla_forward_bytes(const ksana_sage_shape* s, uint64_t* bytes) {
+  if (!bytes) return fail(KSANA_SAGE_EINVAL, "out-pointer is null");
+  SlaForwardLayout l;
+  if (int rc = sla_forward_layout(s, &l)) return rc;
+  *bytes = l.total;
+  return 0;
+}
+
+int ksana_sage_sla_forward(const void* q, const void* k, const void* v, void* o, int dtype, const int64_t q_st[4], const int64_t k_st[4],
+                           const int64_t v_st[4], const int64_t o_st[4], const ksana_sage_shape* s, float sm_scale, int keep,
+                           const float* proj_weight, const float* proj_bias, void* ws, void* stream) {
+  SlaForwardLayout l;
+  if (int rc = sla_forward_layout(s, &l)) return rc;
+  if (int rc = check_tensor("q", q, dtype, q_st, s->B, s->Lq, s->Hq)) return rc;
+  if (int rc = check_tensor("k", k, dtype, k_st, s->B, s->Lk, s->Hkv)) return rc;
+  if (int rc = check_tensor("v", v, dtype, v_st, s->B, s->Lk, s->Hkv)) return rc;
+  if (int rc = check_tensor("o", o, dtype, o_st, s->B, s->Lq, s->Hq)) return rc;
+  if (int rc = check_ws(ws)) return rc;
+  if ((reinterpret_cast<uintptr_t>(proj_weight) | reinterpret_cast<uintptr_t>(proj_bias)) & 15u)
+    return fail(KSANA_SAGE_EINVAL, "projection weight / bias not 16-byte aligned");
+  hipStream_t hs = static_cast<hipStream_t>(stream);
+  const ksana_sage::InTensor qt = in_tensor(q, dtype, q_st), kt = in_tensor(k, dtype, k_st), vt = in_tensor(v, dtype, v_st);
+  float *part = ws_at<float>(ws, l.part), *ksum = ws_at<float>(ws, l.ksum);
+  uint16_t* frag = ws_at<uint16_t>(ws, l.m_frag);
+  uint16_t *pooled_q = ws_at<uint16_t>(ws, l.pooled_q), *pooled_k = ws_at<uint16_t>(ws, l.pooled_k);
+  int8_t* map = ws_at<int8_t>(ws, l.map);
+  const int64_t map_st[2] = {(int64_t)s->Hq * l.nq * l.nk, (int64_t)l.nq * l.nk};
+  {
+    const StageRange range("ksana_sage.quant_qkv");
+    const ksana_sage::QkvCall c = qkv_call(true, qt, kt, vt, s, l.ws, sm_scale, 1, ws);
+    hipError_t e = ksana_sage::launch_sla_kv_stats(kt, vt, s->B, s->Hkv, s->Lk, part, c.k_part, c.v_part, c.nch, hs);
+    if (e != hipSuccess) return hip_fail(e, "sparse-linear statistics launch");
+    int runs = 1, rows_per_run = s->Lk;
+    ksana_sage::plan_sla_runs(s->B, s->Hkv, s->Lk, &runs, &rows_per_run);
+    e = ksana_sage::launch_quant_sla(c, ksana_sage::SlaFinal{part, runs, proj_weight, frag, ksum, pooled_q, pooled_k}, hs);
+    if (e != hipSuccess) return hip_fail(e, "sparse-linear quantizer launch");
+  }
+  if (int rc = ksana_sage_sla_block_map(pooled_q, pooled_k, dtype, s->B, s->Hq, l.nq, l.nk, keep, map, stream)) return rc;
+  if (int rc = attn_impl(ws, o, dtype, o_st, s, map, map_st, nullptr, nullptr, 0, 0, nullptr, 0.0f, stream)) return rc;
+  const StageRange range("ksana_sage.sla_linear");
+  const ksana_sage::InTensor add = in_tensor(o, dtype, o_st);
+  const hipError_t e = ksana_sage::launch_sla_apply(qt, s->B, s->Hq, s->Lq, proj_bias, &add,
+                                                    ksana_sage::OutTensor{static_cast<uint16_t*>(o), o_st[0], o_st[1], o_st[2], dtype}, frag,
+                                                    ksum, hs);
+  return e == hipSuccess ? 0 : hip_fail(e, "sparse-linear second pass launch");
+}
+
 int ksana_sage_attn_key_split(const ksana_sage_shape* s, int* first_workgroup, int* runs) {
   if (int rc = check_shape(s)) return rc;
   if (!first_workgroup || !runs) return fail(KSANA_SAGE_EINVAL, "out-pointer is null");
@@ -798,19 +889,8 @@ int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtyp
       return rc;
     if (int rc = make_prep(prep, prep ? prep->k_norm_weight : nullptr, "k", k_st, s->B, s->Lk, s->D, ws_at<float>(ws, l.k_rms), &pk, &ppk))
       return rc;
-    ksana_sage::QkvCall c{};
-    c.q = in_tensor(q, dtype, q_st, s->D), c.k = in_tensor(k, dtype, k_st, s->D), c.v = in_tensor(v, dtype, v_st, s->D);
-    c.B = s->B, c.Hq = s->Hq, c.Hkv = s->Hkv, c.Lq = s->Lq, c.Lk = s->Lk, c.lq_pad = l.lq_pad, c.nkb = l.nkb, c.nch = l.nch;
-    c.nqb = with_q ? l.lq_pad / ksana_sage::kQPad : 0;
-    c.premul = q_premul_of(sm_scale);
-    c.smooth_k = smooth_k ? 1 : 0;
-    c.q_i8 = ws_at<int8_t>(ws, l.q_i8), c.q_scale = ws_at<float>(ws, l.q_scale);
-    c.k_part = ws_at<float>(ws, l.k_part), c.k_mean = ws_at<float>(ws, l.k_mean);
-    c.k_tiles = ws_at<int8_t>(ws, l.k_i8), c.k_scale = ws_at<float>(ws, l.k_scale);
-    c.v_part = ws_at<float>(ws, l.v_part), c.v_scale = ws_at<float>(ws, l.v_scale), c.v_inv = ws_at<float>(ws, l.v_inv);
-    c.v_mean = ws_at<float>(ws, l.v_mean), c.v_tiles = ws_at<uint8_t>(ws, l.v_fp8);
-    const int bhk = s->B * s->Hkv;
-    c.sync = sync_at(ws_at<int>(ws, l.k_sync), ws_at<int>(ws, l.v_sync), bhk);
+    const ksana_sage::QkvCall c = qkv_call(with_q, in_tensor(q, dtype, q_st, s->D), in_tensor(k, dtype, k_st, s->D),
+                                           in_tensor(v, dtype, v_st, s->D), s, l, sm_scale, smooth_k, ws);
     bool used = false;
     const hipError_t e = ksana_sage::launch_quant_qkv(c, ppq, ppk, static_cast<hipStream_t>(stream), &used);
     if (e != hipSuccess) return hip_fail(e, "q, k, v quantizer launch");

@@ -172,6 +172,24 @@ hipError_t launch_sla_linear(const InTensor& q, const InTensor& k, const InTenso
                              const float* proj_w, const float* proj_b, const InTensor* add, const OutTensor& out,
                              float* part, uint16_t* m_frag, float* ksum, hipStream_t s);
 
+// The first pass alone, with the chunk sums of K and the chunk maxima of |V| the quantizers start from (smooth_k), and the second.
+hipError_t launch_sla_kv_stats(const InTensor& k, const InTensor& v, int B, int H, int L, float* part, float* k_part, float* v_part, int nch,
+                               hipStream_t s);
+hipError_t launch_sla_apply(const InTensor& q, int B, int H, int L, const float* proj_b, const InTensor* add, const OutTensor& out,
+                            const uint16_t* m_frag, const float* ksum, hipStream_t s);
+// What launch_sla_kv_stats left, finished while Q, K and V are quantized, the block averages of Q and K taken along: one launch
+// (c.nqb > 0, head size 128, Hq == Hkv)
+struct SlaFinal {
+  const float* part;
+  int runs;
+  const float* proj_w;
+  uint16_t* m_frag;
+  float* ksum;
+  uint16_t *pooled_q, *pooled_k;
+};
+struct QkvCall;
+hipError_t launch_quant_sla(const QkvCall& call, const SlaFinal& f, hipStream_t s);
+
 // int8 block_map[BH][nq][nk]: per query block ones at the `keep` key blocks with the largest pooled_q . pooled_k (half
 // tensors [BH][n][128], contiguous); nk <= 1024
 hipError_t launch_sla_block_map(const uint16_t* pooled_q, const uint16_t* pooled_k, int dtype, int BH, int nq, int nk, int keep,

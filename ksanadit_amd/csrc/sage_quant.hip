@@ -8,6 +8,7 @@
 // specification): plain IEEE fp32 add / sub / mul / div, round-half-even, no contraction.
 #include "sage_device.h"
 #include "sage_kernels.h"
+#include "sage_sla_device.h"
 
 #include <cstdlib>
 #include <cstring>
@@ -1672,6 +1673,72 @@ __global__ __launch_bounds__(kThreads, 4) void quant_qkv_small_kernel(const QkvC
     quant_q_item<DT, KIND>(item - 2 * n, c, pq);
 }
 
+// The sparse-linear backend's second launch: the statistics have come with the linear branch's pass over K and V, so K and V are
+// quantized (from the last head down: what that pass read last is read first), Q with them, the block averages of Q and K
+// are taken along, and the linear branch's matrices are finished.  With the first launch it replaces seven (Q, K's sums, their
+// finalisation, K, V with its counters, the linear branch's finalisation) and a third reading of K and a second of V: HBM-bound.
+// kReady: a launch in between (sla_finalize_kernel) has finished the heads' statistics and the linear branch's matrices - from
+// kSlaReadyChunks on, where the chunk results every workgroup would add up are no longer small next to its rows.
+template <int DT, bool kReady>
+__global__ __launch_bounds__(kThreads, 4) void quant_sla_kernel(const QkvCall c, const SlaFinal f) {
+  __shared__ float s_stat[2][kD];
+  int item = blockIdx.x;
+  const int n_bh = c.B * c.Hkv;
+  if constexpr (!kReady) {
+    clear_status(c);
+    const int n_fin = n_bh * (kD / kFinRows);
+    if (item < n_fin) {
+      sla_kv_finalize<DT>(item % (kD / kFinRows), item / (kD / kFinRows), f.part, f.runs, f.proj_w, f.m_frag, f.ksum);
+      return;
+    }
+    item -= n_fin;
+  }
+  const int per_head = (c.nkb + c.tiles_per_wg - 1) / c.tiles_per_wg;
+  if (item < 2 * n_bh * per_head) {
+    const int up = item / (2 * per_head), bh = n_bh - 1 - up, b = bh / c.Hkv, h = bh - b * c.Hkv;
+    int run = item - up * (2 * per_head);
+    const bool is_v = run >= per_head;
+    if (is_v) run -= per_head;
+    const int first = run * c.tiles_per_wg, last = min(c.nkb, first + c.tiles_per_wg);
+    auto stat = [&]() -> const float* { return kReady ? (is_v ? c.v_inv : c.k_mean) + bh * kD : s_stat[0]; };
+    const PrepParams none{};
+    if (is_v) {
+      if constexpr (!kReady) head_statistic<1>(c, bh, run == 0, s_stat);
+      for (int blk = first; blk < last; ++blk) {
+        quant_v_block<DT, false>(blk, h, b, c.v.ptr, c.v.sB, c.v.sL, c.v.sH, c.Hkv, c.Lk, c.v.D, c.nkb, stat, nullptr, c.v_tiles);
+        __syncthreads();  // the tile has been read out of LDS
+      }
+    } else {
+      if constexpr (!kReady) head_statistic<0>(c, bh, run == 0, s_stat);
+      for (int blk = first; blk < last; ++blk) {
+        quant_k_block<DT, 0, true>(blk, h, b, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.nkb, stat, c.k_tiles, c.k_scale,
+                                   none, f.pooled_k);
+        __syncthreads();
+      }
+    }
+    return;
+  }
+  item -= 2 * n_bh * per_head;
+  const PrepParams none{};
+  const int bh = item / c.nqb;
+  quant_q_block<DT, 0, true>(item - bh * c.nqb, bh % c.Hq, bh / c.Hq, c.q.ptr, c.q.sB, c.q.sL, c.q.sH, c.Hq, c.Lq, c.q.D, c.lq_pad,
+                             c.premul, c.q_i8, c.q_scale, none, f.pooled_q);
+}
+
+// the heads' statistics and the linear branch's matrices: grid = B * H * (8 + 2)
+template <int DT>
+__global__ __launch_bounds__(kThreads) void sla_finalize_kernel(const QkvCall c, const SlaFinal f) {
+  __shared__ float s_stat[2][kD];
+  clear_status(c);
+  const int n_bh = c.B * c.Hkv, n_fin = n_bh * (kD / kFinRows), item = blockIdx.x;
+  if (item < n_bh)
+    head_statistic<0>(c, item, true, s_stat);
+  else if (item < 2 * n_bh)
+    head_statistic<1>(c, item - n_bh, true, s_stat);
+  else if (item < 2 * n_bh + n_fin)
+    sla_kv_finalize<DT>((item - 2 * n_bh) % (kD / kFinRows), (item - 2 * n_bh) / (kD / kFinRows), f.part, f.runs, f.proj_w, f.m_frag, f.ksum);
+}
+
 // ---------------------------------------------------------------------------------------
 // Block means: out[b, h, blk, d] = mean over the rows [blk * rows, min((blk + 1) * rows, L)) of x[b, :, h, d],
 // optionally of x - centre[b, h, d] with each difference rounded to the tensor's half type first (the reference
@@ -2155,6 +2222,31 @@ hipError_t launch_quant_qkv(const QkvCall& call, const PrepParams* pq, const Pre
   hipError_t e = hipSuccess;
   KSANA_DISPATCH_DT(c.q.dtype, { e = kind == 0 ? launch_qkv_kind<DT, 0>(c, a, b, s, used) : launch_qkv_kind<DT, 2>(c, a, b, s, used); });
   return e;
+}
+
+// us per call, every workgroup by itself / a launch in between: 40 heads of 3000 tokens (12 chunks) 122 / 131, of 6867 (27) 272 / 281, of
+// 12000 (47) 483 / 486, of 32760 (128) 2006 / 1938; 12 heads of 16000 (63) 234 / 247.
+constexpr int kSlaReadyChunks = 64;
+
+hipError_t launch_quant_sla(const QkvCall& call, const SlaFinal& f, hipStream_t s) {
+  QkvCall c = call;
+  c.tiles_per_wg = 2 * (int64_t)c.B * c.Hkv * c.nkb >= kTwoTilesFrom ? 2 : 1;
+  const bool ready = c.nch >= kSlaReadyChunks;
+  if (ready) c.tiles_per_wg = 1;
+  const int64_t n_bh = (int64_t)c.B * c.Hkv;
+  const int64_t n = 2 * n_bh * ((c.nkb + c.tiles_per_wg - 1) / c.tiles_per_wg) + (int64_t)c.B * c.Hq * c.nqb;
+  const int64_t n_fin = n_bh * (kD / kFinRows);
+  if (n + n_fin > INT32_MAX) return hipErrorInvalidValue;
+  const dim3 block(kThreads);
+  KSANA_DISPATCH_DT(c.q.dtype, {
+    if (ready) {
+      sla_finalize_kernel<DT><<<dim3((unsigned)(2 * n_bh + n_fin)), block, 0, s>>>(c, f);
+      quant_sla_kernel<DT, true><<<dim3((unsigned)n), block, 0, s>>>(c, f);
+    } else {
+      quant_sla_kernel<DT, false><<<dim3((unsigned)(n_fin + n)), block, 0, s>>>(c, f);
+    }
+  });
+  return hipGetLastError();
 }
 
 hipError_t launch_quant_v(const InTensor& v, int B, int H, int L, int nkb, const float* v_inv, const float* v_mean,

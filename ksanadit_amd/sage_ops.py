@@ -476,14 +476,7 @@ def sla_linear(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, proj_weight: t
             add = _usable(add)
     w = b = None
     if proj_weight is not None:
-        if tuple(proj_weight.shape) != (D, D):
-            raise ValueError(f"proj_weight must be [{D}, {D}]")
-        # the layer runs in the tensors' dtype under autocast: the weight is rounded to it first
-        w = _prep_operand(_prep_operand(proj_weight, q.device, q.dtype), q.device, torch.float32)
-        if proj_bias is not None:
-            if proj_bias.numel() != D:
-                raise ValueError(f"proj_bias must hold {D} values")
-            b = _prep_operand(_prep_operand(proj_bias, q.device, q.dtype), q.device, torch.float32)
+        w, b = _proj_operands(proj_weight, proj_bias, q.device, q.dtype)
     elif proj_bias is not None:
         raise ValueError("proj_bias given without proj_weight")
     lib = _capi.load()
@@ -496,6 +489,46 @@ def sla_linear(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, proj_weight: t
                                    None if add is None else _strides(add), out.data_ptr(), _strides(out),
                                    scratch.data_ptr(), _stream_ptr(q.device))
     _capi.check(rc, "ksana_sage_sla_linear")
+    return out
+
+
+def _proj_operands(proj_weight: torch.Tensor, proj_bias: torch.Tensor | None, device, dtype):
+    """The block's layer as the kernels read it: fp32, its values rounded to ``dtype`` first (the layer runs in the tensors'
+    dtype under autocast)."""
+    D = 128
+    if tuple(proj_weight.shape) != (D, D):
+        raise ValueError(f"proj_weight must be [{D}, {D}]")
+    w = _prep_operand(_prep_operand(proj_weight, device, dtype), device, torch.float32)
+    if proj_bias is None:
+        return w, None
+    if proj_bias.numel() != D:
+        raise ValueError(f"proj_bias must hold {D} values")
+    return w, _prep_operand(_prep_operand(proj_bias, device, dtype), device, torch.float32)
+
+
+def sla_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, keep: int, proj_weight: torch.Tensor,
+                proj_bias: torch.Tensor | None = None) -> torch.Tensor:
+    """The sparse-linear backend's whole call on ``[B, L, H, 128]`` tensors of one shape (``ksana_sage_sla_forward``): block
+    map with ``keep`` key blocks per query block, block-sparse attention, linear branch through the block's layer, their
+    sum.  At most 65536 tokens."""
+    _require_hip(q, k, v)
+    if q.dim() != 4 or q.shape[3] != 128 or k.shape != q.shape or v.shape != q.shape:
+        raise ValueError("sla_forward expects q, k, v of one shape [B, L, H, 128]")
+    w, b = _proj_operands(proj_weight, proj_bias, q.device, q.dtype)
+    out = torch.empty_like(q)
+    q, k, v = _usable(q), _usable(k), _usable(v)
+    if _usable(out) is not out:
+        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    B, L, H, D = q.shape
+    shape, _ = _capi.workspace_layout(B, H, H, L, L, D)
+    lib = _capi.load()
+    nbytes = C.c_uint64(0)
+    _capi.check(lib.ksana_sage_sla_forward_bytes(C.byref(shape), C.byref(nbytes)), "ksana_sage_sla_forward_bytes")
+    blob = torch.empty(nbytes.value, dtype=torch.uint8, device=q.device)  # (torch's blocks start at multiples of 512)
+    rc = lib.ksana_sage_sla_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _DTYPES[q.dtype], _strides(q), _strides(k),
+                                    _strides(v), _strides(out), C.byref(shape), D**-0.5, int(keep), w.data_ptr(),
+                                    None if b is None else b.data_ptr(), blob.data_ptr(), _stream_ptr(q.device))
+    _capi.check(rc, "ksana_sage_sla_forward")
     return out
 
 
