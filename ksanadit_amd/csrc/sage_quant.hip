@@ -150,22 +150,38 @@ __device__ __forceinline__ int small_div(int n, int d, int* rem) {
 //       mean: every lane adds its 16 squares in channel order, the 8 lane sums meet in an adjacent-pair tree
 //   (y[2i], y[2i+1]) -> half( (y[2i] + i*y[2i+1]) * freqs[row, i] )    complex64: four products, one subtraction and
 //       one addition, each rounded to fp32
-template <int DT>
-__device__ __forceinline__ void prep16_qwen(float* x, const PrepParams& pp, int row, int c16) {
+//
+// What a row's lane reads besides the row, the same for all heads: where its 16 norm weights are, and 8 rotation factors.
+struct QwenRow {
+  const float4* w;  // nullptr: no norm
+  bool rotate;
+  float4 cs[4];  // two factors each, (re, im), (re, im)
+};
+__device__ __forceinline__ void qwen_row(QwenRow& f, const PrepParams& pp, int row, int c16) {
   const bool txt = row < pp.txt_len;
   const float* w = txt ? pp.weight_txt : pp.weight_img;
-  if (w != nullptr) {
+  const float2* tab = txt ? pp.freqs_txt : pp.freqs_img;
+  f.w = w != nullptr ? reinterpret_cast<const float4*>(w + c16 * 16) : nullptr;
+  f.rotate = tab != nullptr;
+  if (f.rotate) {
+    const float4* t4 = reinterpret_cast<const float4*>(tab + (int64_t)(txt ? row : row - pp.txt_len) * (kD / 2) + c16 * 8);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f.cs[j] = t4[j];
+  }
+}
+template <int DT>
+__device__ __forceinline__ void prep16_qwen(float* x, const QwenRow& f, float eps) {
+  if (f.w != nullptr) {
     float ss = 0.0f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) ss = e == 0 ? x[0] * x[0] : ss + x[e] * x[e];  // squares of half values are exact
     ss = ss + lane_xor<1>(ss);
     ss = ss + lane_xor<2>(ss);
     ss = ss + lane_xor<4>(ss);
-    const float r = __fdiv_rn(1.0f, sqrtf(__fdiv_rn(ss, (float)kD) + pp.eps));
-    const float4* w4 = reinterpret_cast<const float4*>(w + c16 * 16);
+    const float r = __fdiv_rn(1.0f, sqrtf(__fdiv_rn(ss, (float)kD) + eps));
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float4 wj = w4[j];
+      const float4 wj = f.w[j];
       x[4 * j + 0] = (x[4 * j + 0] * r) * wj.x;
       x[4 * j + 1] = (x[4 * j + 1] * r) * wj.y;
       x[4 * j + 2] = (x[4 * j + 2] * r) * wj.z;
@@ -174,12 +190,10 @@ __device__ __forceinline__ void prep16_qwen(float* x, const PrepParams& pp, int 
       through_half2<DT>(x[4 * j + 2], x[4 * j + 3]);
     }
   }
-  const float2* tab = txt ? pp.freqs_txt : pp.freqs_img;
-  if (tab != nullptr) {
-    const float4* t4 = reinterpret_cast<const float4*>(tab + (int64_t)(txt ? row : row - pp.txt_len) * (kD / 2) + c16 * 8);
+  if (f.rotate) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float4 cs = t4[j];  // two factors: (re, im), (re, im)
+      const float4 cs = f.cs[j];
       const float a0 = x[4 * j], b0 = x[4 * j + 1], a1 = x[4 * j + 2], b1 = x[4 * j + 3];
       x[4 * j + 0] = a0 * cs.x - b0 * cs.y;
       x[4 * j + 1] = a0 * cs.y + b0 * cs.x;
@@ -189,6 +203,13 @@ __device__ __forceinline__ void prep16_qwen(float* x, const PrepParams& pp, int 
       through_half2<DT>(x[4 * j + 2], x[4 * j + 3]);
     }
   }
+}
+
+template <int DT>
+__device__ __forceinline__ void prep16_qwen(float* x, const PrepParams& pp, int row, int c16) {
+  QwenRow f;
+  qwen_row(f, pp, row, c16);
+  prep16_qwen<DT>(x, f, pp.eps);
 }
 
 // The pieces of the Wan step on the 16 channels of a lane.
@@ -561,6 +582,24 @@ __device__ __forceinline__ void store_block_mean(float (&acc)[16], int t, float 
   }
 }
 
+// a row of Q from its lanes' channels: transform, premul_lane = premul * fwht_lane_sign(c16), scale and codes
+__device__ __forceinline__ void quant_q_row(float* x, int c16, float premul_lane, float* scale, int8_t* codes) {
+  fwht128(x, c16);
+  float amax = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    x[e] = x[e] * premul_lane;
+    amax = fmaxf(amax, fabsf(x[e]));
+  }
+  amax = fmaxf(amax, lane_xor<1>(amax));
+  amax = fmaxf(amax, lane_xor<2>(amax));
+  amax = fmaxf(amax, lane_xor<4>(amax));
+  const bool nz = amax > 0.0f;
+  const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
+  if (c16 == 0) *scale = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+  store_out16(codes + c16 * 16, pack_int8x16(x, inv));
+}
+
 // ---------------------------------------------------------------------------------------
 // Q: Hadamard transform, fold sm_scale*log2(e)/128, one int8 scale per query row.  One
 // workgroup handles 128 rows (4 per row slot).  grid = (lq_pad/128, H, B).  Output row-major
@@ -582,20 +621,7 @@ __device__ __forceinline__ void quant_q_block(int blk, int h, int b, const uint1
   const RopeLds rl = maybe_stage_rope<PRE>(pp, b, blk * kRowsPerWg, kRowsPerWg);
   const float premul_lane = premul * fwht_lane_sign(c16);
   auto finish_row = [&](float* xr, int row) {
-    fwht128(xr, c16);
-    float amax = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      xr[e] = xr[e] * premul_lane;
-      amax = fmaxf(amax, fabsf(xr[e]));
-    }
-    amax = fmaxf(amax, lane_xor<1>(amax));
-    amax = fmaxf(amax, lane_xor<2>(amax));
-    amax = fmaxf(amax, lane_xor<4>(amax));
-    const bool nz = amax > 0.0f;
-    const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
-    if (c16 == 0) q_scale[bh * lq_pad + row] = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
-    store_out16(q_i8 + (bh * lq_pad + row) * kD + c16 * 16, pack_int8x16(xr, inv));
+    quant_q_row(xr, c16, premul_lane, q_scale + bh * lq_pad + row, q_i8 + (bh * lq_pad + row) * kD);
   };
   if constexpr (PRE) {
     // The norm and the rotation are arithmetic-heavy (vector fp64): one row at a time with only the next row's two
@@ -1520,27 +1546,31 @@ __global__ __launch_bounds__(kThreads) void quant_v_fused_kernel(const uint16_t*
 // 40 heads, 1560 tokens 43 / 22 stages; 9000 tokens 120 / 106 stages; 14000 tokens 184 / 158 meet; 32760 tokens 392 / 369
 // meet (HBM-bound: 9 bytes per element at 4 TB/s).
 // ---------------------------------------------------------------------------------------
+// channel d's mean of a head of K
+__device__ __forceinline__ float head_mean(const QkvCall& c, int bh, int d, bool publish) {
+  const float* hp = c.k_part + (int64_t)bh * c.nch * kD + d;
+  float tot = 0.0f;
+  if (c.smooth_k) {
+    for (int c0 = 0; c0 < c.nch; c0 += 16) {  // 16 loads in flight; added in chunk order
+      float v[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v[j] = hp[min(c0 + j, c.nch - 1) * kD];
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        if (c0 + j < c.nch) tot = c0 + j == 0 ? v[0] : tot + v[j];
+    }
+  }
+  const float mean = c.smooth_k ? round_to_half_dtype(__fdiv_rn(tot, (float)c.Lk), c.k.dtype) : 0.0f;
+  if (publish) c.k_mean[bh * kD + d] = mean;
+  return mean;
+}
+
 template <int OP>  // 0: K's mean (ordered sum), 1: V's factor 448 / amax
 __device__ __forceinline__ void head_statistic(const QkvCall& c, int bh, bool publish, float (*s_stat)[kD]) {
   const int t = threadIdx.x, d = t & (kD - 1);
   const float* hp = (OP == 0 ? c.k_part : c.v_part) + (int64_t)bh * c.nch * kD + d;
   if constexpr (OP == 0) {
-    if (t < kD) {
-      float tot = 0.0f;
-      if (c.smooth_k) {
-        for (int c0 = 0; c0 < c.nch; c0 += 16) {  // 16 loads in flight; added in chunk order
-          float v[16];
-#pragma unroll
-          for (int j = 0; j < 16; ++j) v[j] = hp[min(c0 + j, c.nch - 1) * kD];
-#pragma unroll
-          for (int j = 0; j < 16; ++j)
-            if (c0 + j < c.nch) tot = c0 + j == 0 ? v[0] : tot + v[j];
-        }
-      }
-      const float mean = c.smooth_k ? round_to_half_dtype(__fdiv_rn(tot, (float)c.Lk), c.k.dtype) : 0.0f;
-      s_stat[0][d] = mean;
-      if (publish) c.k_mean[bh * kD + d] = mean;
-    }
+    if (t < kD) s_stat[0][d] = head_mean(c, bh, d, publish);
     __syncthreads();
   } else {
     float m = 0.0f;  // a maximum needs no order: the two halves of the workgroup take the even and the odd chunks
@@ -1581,16 +1611,184 @@ __device__ __forceinline__ void quant_q_item(int item, const QkvCall& c, const P
                                  c.premul, c.q_i8, c.q_scale, pp, nullptr);
 }
 
-template <int DT, int KIND>
+// The joint block's items take several heads of the same rows: a lane's norm weights and rotation factors are read once for all of
+// them (a row's factors are twice its own bytes, and came out of the L2 for every head).  Bound by vector work, 54-62 % busy:
+// 2 x 4352 tokens of 24 heads, stage 1 70 -> 61 us, stage 2 47 -> 45.
+constexpr int kJointHeadsQ = 4, kJointHeadsK = 2;
+
+// 32 query rows of kJointHeadsQ heads
+template <int DT>
+__device__ __forceinline__ void joint_q_item(int item, const QkvCall& c, const PrepParams& pp) {
+  const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
+  const int blocks = c.lq_pad / kSlots, groups = (c.Hq + kJointHeadsQ - 1) / kJointHeadsQ;
+  const int bg = item / blocks, row = (item - bg * blocks) * kSlots + slot, b = bg / groups, h0 = (bg - b * groups) * kJointHeadsQ;
+  const bool valid = row < c.Lq;
+  const uint16_t* base = c.q.ptr + b * c.q.sB + (int64_t)row * c.q.sL + c16 * 16;
+  const int n = min(kJointHeadsQ, c.Hq - h0);
+  uint4 next[2];
+  fetch_row16(base + h0 * c.q.sH, valid, next);
+  QwenRow f{};
+  if (valid) qwen_row(f, pp, row, c16);
+  const float premul_lane = c.premul * fwht_lane_sign(c16);
+#pragma unroll 1  // (unrolled, the heads' work is pulled together and spills)
+  for (int i = 0; i < n; ++i) {
+    float x[16];
+    widen8<DT>(next[0], x);
+    widen8<DT>(next[1], x + 8);
+    if (i + 1 < n) fetch_row16(base + (h0 + i + 1) * c.q.sH, valid, next);
+    if (valid) prep16_qwen<DT>(x, f, pp.eps);
+    const int64_t at = ((int64_t)b * c.Hq + h0 + i) * c.lq_pad + row;
+    quant_q_row(x, c16, premul_lane, c.q_scale + at, c.q_i8 + at * kD);
+  }
+}
+
+// the column sums of one chunk of K for kJointHeadsK heads, in the order of col_partial_chunk
+template <int DT>
+__device__ __forceinline__ void joint_k_sums(int item, const QkvCall& c, const PrepParams& pp) {
+  const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
+  const int groups = (c.Hkv + kJointHeadsK - 1) / kJointHeadsK;
+  const int bg = item / c.nch, ch = item - bg * c.nch, b = bg / groups, h0 = (bg - b * groups) * kJointHeadsK;
+  const uint16_t* base = c.k.ptr + b * c.k.sB + h0 * c.k.sH + c16 * 16;
+  float acc[kJointHeadsK][16];
+  uint4 next[kJointHeadsK][2];
+  auto fetch = [&](int i) {
+    const int row = ch * kMeanChunk + i * kSlots + slot;
+#pragma unroll
+    for (int hh = 0; hh < kJointHeadsK; ++hh) {
+      next[hh][0] = next[hh][1] = make_uint4(0, 0, 0, 0);
+      if (h0 + hh < c.Hkv) fetch_row16(base + (int64_t)row * c.k.sL + hh * c.k.sH, row < c.Lk, next[hh]);
+    }
+  };
+  auto add_row = [&](int i, bool first) {
+    const int row = ch * kMeanChunk + i * kSlots + slot;
+    uint4 raw[kJointHeadsK][2];
+#pragma unroll
+    for (int hh = 0; hh < kJointHeadsK; ++hh) raw[hh][0] = next[hh][0], raw[hh][1] = next[hh][1];
+    QwenRow f{};
+    if (row < c.Lk) qwen_row(f, pp, row, c16);
+    if (i + 1 < kMeanChunk / kSlots) fetch(i + 1);
+#pragma unroll
+    for (int hh = 0; hh < kJointHeadsK; ++hh) {
+      float x[16];
+      widen8<DT>(raw[hh][0], x);
+      widen8<DT>(raw[hh][1], x + 8);
+      if (row < c.Lk) prep16_qwen<DT>(x, f, pp.eps);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[hh][e] = first ? x[e] : acc[hh][e] + x[e];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  fetch(0);
+  add_row(0, true);
+#pragma unroll 1  // (unrolled, the rows' work is pulled together and spills)
+  for (int i = 1; i < kMeanChunk / kSlots; ++i) add_row(i, false);
+  __shared__ float s_w[kJointHeadsK][4][kD];
+  const int wave = t >> 6, lane = t & 63;
+#pragma unroll
+  for (int hh = 0; hh < kJointHeadsK; ++hh) {
+#pragma unroll
+    for (int m = 8; m <= 32; m <<= 1) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[hh][e] = acc[hh][e] + __shfl_xor(acc[hh][e], m);
+    }
+    if (lane < 8) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s_w[hh][wave][c16 * 16 + e] = acc[hh][e];
+    }
+  }
+  __syncthreads();
+  static_assert(kJointHeadsK * kD == kThreads, "a thread per head and channel");
+  const int hh = t >> 7, d = t & (kD - 1);
+  if (h0 + hh < c.Hkv)
+    c.k_part[(((int64_t)b * c.Hkv + h0 + hh) * c.nch + ch) * kD + d] =
+        (s_w[hh][0][d] + s_w[hh][1][d]) + (s_w[hh][2][d] + s_w[hh][3][d]);
+}
+
+// one tile of K for kJointHeadsK heads; the heads' means from the chunk sums
+template <int DT>
+__device__ __forceinline__ void joint_k_item(int item, const QkvCall& c, const PrepParams& pp) {
+  const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
+  const int groups = (c.Hkv + kJointHeadsK - 1) / kJointHeadsK;
+  const int bg = item / c.nkb, blk = item - bg * c.nkb, b = bg / groups, h0 = (bg - b * groups) * kJointHeadsK;
+  const uint16_t* base = c.k.ptr + b * c.k.sB + h0 * c.k.sH + c16 * 16;
+  __shared__ float s_mean[kJointHeadsK][kD];
+  __shared__ float s_red[kJointHeadsK][4];
+  constexpr int R = kBlkK / kSlots;
+  uint4 next[R][2];
+  QwenRow f[R]{};
+  auto fetch = [&](int hh) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int row = blk * kBlkK + i * kSlots + slot;
+      fetch_row16(base + (int64_t)row * c.k.sL + hh * c.k.sH, row < c.Lk, next[i]);
+    }
+  };
+  fetch(0);
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int row = blk * kBlkK + i * kSlots + slot;
+    if (row < c.Lk) qwen_row(f[i], pp, row, c16);
+  }
+  {
+    const int hh = t >> 7, d = t & (kD - 1), bh = b * c.Hkv + h0 + hh;
+    if (h0 + hh < c.Hkv) s_mean[hh][d] = head_mean(c, bh, d, blk == 0);
+  }
+  __syncthreads();
+  const int wave = t >> 6;
+  const int n = min(kJointHeadsK, c.Hkv - h0);
+#pragma unroll 1
+  for (int hh = 0; hh < n; ++hh) {
+    float x[R][16], amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      widen8<DT>(next[i][0], x[i]);
+      widen8<DT>(next[i][1], x[i] + 8);
+    }
+    if (hh + 1 < n) fetch(hh + 1);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const bool valid = blk * kBlkK + i * kSlots + slot < c.Lk;
+      if (valid) prep16_qwen<DT>(x[i], f[i], pp.eps);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) x[i][e] = valid ? x[i][e] - s_mean[hh][c16 * 16 + e] : 0.0f;
+      fwht128(x[i], c16);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(x[i][e]));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int m = 1; m <= 32; m <<= 1) amax = fmaxf(amax, __shfl_xor(amax, m));
+    if ((t & 63) == 0) s_red[hh][wave] = amax;
+    __syncthreads();
+    amax = fmaxf(fmaxf(s_red[hh][0], s_red[hh][1]), fmaxf(s_red[hh][2], s_red[hh][3]));
+    const bool nz = amax > 0.0f;
+    const float inv_lane = (nz ? __fdiv_rn(127.0f, amax) : 0.0f) * fwht_lane_sign(c16);
+    const int64_t at = ((int64_t)b * c.Hkv + h0 + hh) * c.nkb + blk;
+    if (t == 0) c.k_scale[at] = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int frag = i * 4 + (c16 >> 1), ln = (c16 & 1) * 32 + slot;
+      store_out16(c.k_tiles + at * kTileBytes + (frag * 64 + ln) * 16, pack_int8x16(x[i], inv_lane));
+    }
+  }
+}
+
+// kHeads: the joint block's step with several heads per item (launch_qkv_kind)
+template <int DT, int KIND, bool kHeads>
 __global__ __launch_bounds__(kThreads, KIND == 0 ? 5 : 4) void quant_qkv_stage1_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
   want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   clear_status(c);
-  const int n_v = c.B * c.Hkv * c.nch, n_k = c.smooth_k ? n_v : 0;
+  const int n_v = c.B * c.Hkv * c.nch;
+  const int n_k = !c.smooth_k ? 0 : (!kHeads ? n_v : c.B * ((c.Hkv + kJointHeadsK - 1) / kJointHeadsK) * c.nch);
   int item = blockIdx.x;
   if (item < n_k) {
-    const int bh = item / c.nch;
-    col_partial_chunk<DT, 0, KIND>(item - bh * c.nch, bh % c.Hkv, bh / c.Hkv, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D,
-                                   c.k_part, c.nch, pk, nullptr);
+    if constexpr (kHeads) {
+      joint_k_sums<DT>(item, c, pk);
+    } else {
+      const int bh = item / c.nch;
+      col_partial_chunk<DT, 0, KIND>(item - bh * c.nch, bh % c.Hkv, bh / c.Hkv, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.k_part,
+                                  c.nch, pk, nullptr);
+    }
     return;
   }
   item -= n_k;
@@ -1600,16 +1798,26 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 5 : 4) void quant_qkv_stage1_
                                 c.nch, pk, nullptr);
     return;
   }
-  quant_q_item<DT, KIND>(item - n_v, c, pq);
+  if constexpr (kHeads)
+    joint_q_item<DT>(item - n_v, c, pq);
+  else
+    quant_q_item<DT, KIND>(item - n_v, c, pq);
 }
 
-template <int DT, int KIND>
-__global__ __launch_bounds__(kThreads, KIND == 0 ? 6 : 5) void quant_qkv_stage2_kernel(const QkvCall c, const PrepParams pk) {
+template <int DT, int KIND, bool kHeads>
+__global__ __launch_bounds__(kThreads, KIND == 0 ? 6 : (kHeads ? 4 : 5)) void quant_qkv_stage2_kernel(const QkvCall c, const PrepParams pk) {
   want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   __shared__ float s_stat[2][kD];
   const int per_head = (c.nkb + c.tiles_per_wg - 1) / c.tiles_per_wg, n = c.B * c.Hkv * per_head;
-  const bool is_v = (int)blockIdx.x >= n;
-  const int item = is_v ? blockIdx.x - n : blockIdx.x;
+  const int n_k = !kHeads ? n : c.B * ((c.Hkv + kJointHeadsK - 1) / kJointHeadsK) * c.nkb;
+  const bool is_v = (int)blockIdx.x >= n_k;
+  if constexpr (kHeads) {
+    if (!is_v) {
+      joint_k_item<DT>(blockIdx.x, c, pk);
+      return;
+    }
+  }
+  const int item = is_v ? blockIdx.x - n_k : blockIdx.x;
   const int bh = item / per_head, run = item - bh * per_head, b = bh / c.Hkv, h = bh - b * c.Hkv;
   const int first = run * c.tiles_per_wg, last = min(c.nkb, first + c.tiles_per_wg);
   auto stat = [&]() -> const float* { return s_stat[0]; };
@@ -2161,13 +2369,14 @@ hipError_t launch_quant_v_fused(const InTensor& v, int B, int H, int L, int nkb,
 //   8500 122 / 117 / 131; 40 heads of 14000 (273 MB) 192 / 158 / 184; 8 heads of 20000 (78 MB, 79 chunks) 46 / 49 / 56.
 constexpr int kStageMaxChunks = 64;
 constexpr int64_t kStageMaxBytes = 192ll << 20;
-// With the joint block's step stage 2 norms and rotates K once more, and loses its lead earlier; beyond the limit these calls
-// take the separate kernels (K from one read, the step done once).  24 heads, us, stages / separate: one entry of 13000
-// tokens (152 MB) 166 / 175, of 14000 (164 MB) 190 / 186, of 16000 (188 MB) 225 / 205; two of 6500 (152 MB) 159 / 169, of
-// 7000 (164 MB) 183 / 176, of 8056 (189 MB) 210 / 190; four of 3500 (164 MB) 177 / 173.  A meeting launch with the step in it
-// is no gain over them: meeting / separate 188 / 186 and 212 / 205 for the 14000 and 16000 tokens, two entries of 10256 263 /
-// 253, of 16896 414 / 411, one of 16896 219 / 229, of 20512 269 / 270, of 30512 392 / 371, of 40512 512 / 539.
-constexpr int64_t kStageMaxBytesJoint = 160ll << 20;
+// The joint block's calls beyond it take the separate kernels (K from one read, the step done once): stages / separate, whole
+// calls of 24 heads, one entry of 15512 tokens (191 MB) 1604 / 1608, four of 3856 (190 MB) 572.5 / 574.5, of 7056 (347 MB) 1552 /
+// 1533, one of 16256 (200 MB) 1708 / 1700, two of 10512 (258 MB) 1578 / 1567.  A meeting launch with the step in it is no gain over them.
+// Joint block, several heads per item or one: from this many workgroups (of one head, Q's blocks and K's and V's chunks) on the
+// items of several heads still fill the chip.  Whole calls, us, one / several: 24 heads of 1024 tokens 42.2 / 48.3, of 2560 (960
+// workgroups) 82.2 / 84.8, of 4512 203 / 196; two entries of 1024 54.2 / 58.9, of 1328 (1104) 84.7 / 83.9, of 2056 133 / 128, of
+// 4352 360 / 347.5, of 6512 689 / 664.
+constexpr int kJointHeadsFrom = 1104;
 // Beyond this many chunks a head's first workgroups wait for its last ones longer than a second pass takes (296 chunks:
 // the separate quantizers are 3 % faster).
 constexpr int kMeetMaxChunks = 160;
@@ -2185,12 +2394,19 @@ static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepPa
   if (c.nch == 1) {
     quant_qkv_small_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, pq, pk);
     *used = true;
-  } else if (c.nch <= kStageMaxChunks && 4 * (int64_t)c.B * c.Hkv * c.Lk * c.k.D <= (KIND == 0 ? kStageMaxBytes : kStageMaxBytesJoint)) {
+  } else if (c.nch <= kStageMaxChunks && 4 * (int64_t)c.B * c.Hkv * c.Lk * c.k.D <= kStageMaxBytes) {
     const int64_t tiles = 2 * (int64_t)c.B * c.Hkv * c.nkb;
     c.tiles_per_wg = tiles >= (KIND == 0 ? kTwoTilesFrom : kTwoTilesFromJoint) ? 2 : 1;
-    const int64_t n2 = 2 * (int64_t)c.B * c.Hkv * ((c.nkb + c.tiles_per_wg - 1) / c.tiles_per_wg);
-    quant_qkv_stage1_kernel<DT, KIND><<<dim3((unsigned)(n_q + (c.smooth_k ? 2 : 1) * n_chunks)), block, 0, s>>>(c, pq, pk);
-    quant_qkv_stage2_kernel<DT, KIND><<<dim3((unsigned)n2), block, 0, s>>>(c, pk);
+    const int64_t n_v2 = (int64_t)c.B * c.Hkv * ((c.nkb + c.tiles_per_wg - 1) / c.tiles_per_wg);
+    if (KIND == 2 && n_q + 2 * n_chunks >= kJointHeadsFrom) {
+      const int64_t k_groups = (int64_t)c.B * ((c.Hkv + kJointHeadsK - 1) / kJointHeadsK);
+      const int64_t n_rows = c.nqb == 0 ? 0 : (int64_t)c.B * ((c.Hq + kJointHeadsQ - 1) / kJointHeadsQ) * (c.lq_pad / kSlots);
+      quant_qkv_stage1_kernel<DT, 2, true><<<dim3((unsigned)(n_rows + n_chunks + (c.smooth_k ? k_groups * c.nch : 0))), block, 0, s>>>(c, pq, pk);
+      quant_qkv_stage2_kernel<DT, 2, true><<<dim3((unsigned)(k_groups * c.nkb + n_v2)), block, 0, s>>>(c, pk);
+    } else {
+      quant_qkv_stage1_kernel<DT, KIND, false><<<dim3((unsigned)(n_q + (c.smooth_k ? 2 : 1) * n_chunks)), block, 0, s>>>(c, pq, pk);
+      quant_qkv_stage2_kernel<DT, KIND, false><<<dim3((unsigned)(2 * n_v2)), block, 0, s>>>(c, pk);
+    }
     *used = true;
   } else if (KIND == 0 && c.nch <= kMeetMaxChunks) {
     const QuantOptions opt = quant_options();

@@ -59,7 +59,8 @@ def test_together_with_the_joint_block_step(hip_device, txt, img, weights, table
 
 
 @pytest.mark.parametrize("B,txt,img,H", [
-    (1, 56, 13576, 24), (1, 56, 13676, 24),    # 159.75 and 160.9 MB of K and V: the last size in two stages, separate kernels
+    (1, 56, 13576, 24), (1, 56, 13676, 24),
+    (2, 56, 8136, 24), (2, 56, 8137, 24),      # 192 MB of K and V: the last size in two stages, and separate kernels
     (1, 100, 16284, 1), (1, 100, 16285, 1),    # 64 chunks of keys, and one row more
     (1, 100, 5340, 24), (1, 100, 5468, 24)])   # 4080 and (an odd number a head) 4176 tiles: one and two a workgroup of stage 2
 def test_together_with_the_joint_block_step_at_its_limits(hip_device, B, txt, img, H):
@@ -70,6 +71,21 @@ def test_together_with_the_joint_block_step_at_its_limits(hip_device, B, txt, im
     tab = torch.polar(torch.ones_like(ang), ang)
     prep = sage_ops.QwenPrep(txt, *ws, 1e-6, img_freqs=tab[:img].contiguous(), txt_freqs=tab[img:].contiguous())
     _compare(hip_device, B, txt + img, txt + img, H, H, 128, torch.bfloat16, True, prep)
+
+
+@pytest.mark.parametrize("B,txt,img,Hq,Hkv,weights,tables,dtype", [
+    (2, 52, 1284, 24, 24, True, True, torch.bfloat16), (2, 52, 1228, 24, 24, True, True, torch.bfloat16),  # 1104 and 1008 workgroups: several heads, one
+    (2, 13, 1401, 27, 27, True, True, torch.float16),      # heads that leave both groups incomplete, ragged lengths
+    (3, 200, 1700, 18, 9, False, True, torch.bfloat16), (2, 0, 2500, 21, 21, True, False, torch.bfloat16)])
+def test_the_joint_block_step_on_several_heads_per_item(hip_device, B, txt, img, Hq, Hkv, weights, tables, dtype):
+    print(f"case B={B} txt={txt} img={img} Hq={Hq} Hkv={Hkv} weights={weights} tables={tables} {dtype}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(img)
+    ws = [1.0 + 0.2 * torch.randn(128, generator=g, device=hip_device) if weights else None for _ in range(4)]
+    ang = torch.rand((txt + img, 64), generator=g, device=hip_device) * 6.0
+    tab = torch.polar(torch.ones_like(ang), ang) if tables else None
+    prep = sage_ops.QwenPrep(txt, *ws, 1e-6, img_freqs=None if tab is None else tab[:img].contiguous(),
+                             txt_freqs=None if tab is None or txt == 0 else tab[img:].contiguous())
+    _compare(hip_device, B, txt + img, txt + img, Hq, Hkv, 128, dtype, True, prep)
 
 
 def _inputs(hip_device, B, Lk, Hq, Hkv, D, dtype):
