@@ -59,8 +59,7 @@ def test_together_with_the_joint_block_step(hip_device, txt, img, weights, table
 
 
 @pytest.mark.parametrize("B,txt,img,H", [
-    (1, 56, 13576, 24), (1, 56, 13676, 24),
-    (2, 56, 8136, 24), (2, 56, 8137, 24),      # 192 MB of K and V: the last size in two stages, and separate kernels
+    (1, 56, 13576, 24), (1, 56, 13676, 24),    # 159.75 and 160.9 MB of K and V: the last size in two stages, separate kernels
     (1, 100, 16284, 1), (1, 100, 16285, 1),    # 64 chunks of keys, and one row more
     (1, 100, 5340, 24), (1, 100, 5468, 24)])   # 4080 and (an odd number a head) 4176 tiles: one and two a workgroup of stage 2
 def test_together_with_the_joint_block_step_at_its_limits(hip_device, B, txt, img, H):
@@ -86,6 +85,17 @@ def test_the_joint_block_step_on_several_heads_per_item(hip_device, B, txt, img,
     prep = sage_ops.QwenPrep(txt, *ws, 1e-6, img_freqs=None if tab is None else tab[:img].contiguous(),
                              txt_freqs=None if tab is None or txt == 0 else tab[img:].contiguous())
     _compare(hip_device, B, txt + img, txt + img, Hq, Hkv, 128, dtype, True, prep)
+
+
+@pytest.mark.parametrize("img", [8136, 8137])    # 192 MB of K and V: the last size in two stages, and separate kernels
+def test_together_with_the_joint_block_step_at_192_mb(hip_device, img):
+    print(f"case img={img}", flush=True)
+    B, txt, H = 2, 56, 24
+    assert (2 * B * (txt + img) * H * 128 * 2 <= 192 << 20) == (img == 8136)
+    ang = torch.rand((txt + img, 64), generator=torch.Generator(device=hip_device).manual_seed(img), device=hip_device) * 6.0
+    tab = torch.polar(torch.ones_like(ang), ang)
+    prep = sage_ops.QwenPrep(txt, None, None, None, None, 1e-6, img_freqs=tab[:img].contiguous(), txt_freqs=tab[img:].contiguous())
+    _compare(hip_device, B, txt + img, txt + img, H, H, 128, torch.bfloat16, True, prep)
 
 
 def _inputs(hip_device, B, Lk, Hq, Hkv, D, dtype):
