@@ -20,6 +20,7 @@
 // as fp32 IS 12582912 + dot exactly (|dot| <= 127*127*128 < 2^22), which removes the
 // int->float conversion from the softmax: p = exp2(fma(acc_as_float, sc, c)).
 #include "sage_attn_device.h"
+#include "sage_sla_device.h"
 
 #include <atomic>
 #include <type_traits>
@@ -100,7 +101,8 @@ __device__ __forceinline__ void lds_copy16_at(const v4i& buffer, unsigned lane_o
 // kG: 32-channel groups the matrix instructions cover - 4, or 2 when the head size is 64 (rows run zero-extended to
 // 128 channels and the operands keep their layout; see kMagicI2 for what is left out and why nothing is lost; the
 // result equals the full-width code's up to the rounding of one constant in the exponent).
-template <int DT, bool kPwlExp, bool kSparse, int kW, bool kTileSkip, int kG, bool kCausal>
+// kLinear: the sparse-linear backend's linear branch is added to the result in the epilogue.
+template <int DT, bool kPwlExp, bool kSparse, int kW, bool kTileSkip, int kG, bool kCausal, bool kLinear>
 __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel(const AttnParams p, int n_qwg,
                                                                                    int n_wg, int wg_per_xcd) {
   want(p.q_rows.ptr, p.k_tiles, p.o.sH, p.block_mask, n_qwg);
@@ -115,6 +117,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   constexpr int kListMax = kW == 8 ? kSparseMaxKeyTiles : kSparseMaxKeyTiles4;
   static_assert(!(kTileSkip && kPwlExp), "the piecewise-linear code formula has its own zero point: no tiles are skipped there");
   static_assert(kG == 4 || kG == 2, "128 channels, or 64 zero-extended");
+  static_assert(!kLinear || (kSparse && !kCausal && kW == 4 && kG == 4), "the linear branch goes with a block mask, 128 rows a workgroup");
   constexpr bool kUnrolled = !kPwlExp && !kTileSkip && !(kSparse && kW == 8);  // the variants calls take by default
   constexpr int kMagicBits = kG == 4 ? kMagicI : kMagicI2;
   constexpr float kMagicVal = kG == 4 ? kMagicF : kMagicF2;
@@ -960,35 +963,102 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // free by now); read one quadruple at a time where they are used, every one of the 16 groups below would start
   // with an LDS round trip of its own.  Without V smoothing the means are all zero - seen here by the wave as a
   // whole - and their products and sums are left out (a zero output may then keep a minus sign it used to lose).
+  uint8_t* stage = smem + wave * (32 * kPitch);
   const float4* vs4 = reinterpret_cast<const float4*>(s_vs);
   const float4* vm4 = reinterpret_cast<const float4*>(s_vs + kD);
   float4 s4a[16];
 #pragma unroll
   for (int i = 0; i < 4 * kG; ++i) s4a[i] = vs4[(32 * (i >> 2) + 8 * (i & 3) + 4 * hh) >> 2];
-  const float2 mm = reinterpret_cast<const float2*>(s_vs + kD)[lane];
-  const bool has_mean = __any(mm.x != 0.0f || mm.y != 0.0f);  // wave-uniform
-  __syncthreads();  // waves that ended early (no query rows) do not count
-  uint8_t* stage = smem + wave * (32 * kPitch);
-  if (!has_mean) {
+  if constexpr (kLinear) {
+    // The linear branch of the lane's row, of the row as the caller has it, and the sum of the two results, each rounded to
+    // the half type first - what a pass of its own (sla_apply_kernel) gives, bit for bit.  A lane of that product holds the
+    // same channels of the same row as a lane of O^T, so the sum is taken in registers.  LDS from the ring's start: the
+    // head's matrix, ksum and bias, the staged rows (the V scales have been read; no V means on this path).  The matrix
+    // is on its way while the row's exponentials are taken.
+    // As a pass of its own the branch reads q and the result and writes the result again, 1 GB at 32760 rows of 40 heads,
+    // bound by memory; here its arithmetic runs beside the neighbour workgroup's key loop.  us per call, a tenth of the keys
+    // kept, pass of its own / here: 40 heads of 32760 rows 2000 / 1859, of 6867 272 / 230, 12 of 2000 72 / 52.
+    const uint16_t* lrow = p.q_rows.ptr + b * p.q_rows.sB + (int64_t)min(q, p.Lq - 1) * p.q_rows.sL + h * p.q_rows.sH + 8 * hh;
+    uint4 lraw[8];
 #pragma unroll
-    for (int i = 0; i < 4 * kG; ++i) {
+    for (int s = 0; s < 8; ++s) lraw[s] = *reinterpret_cast<const uint4*>(lrow + 16 * s);
+    const float2 ks2 = reinterpret_cast<const float2*>(p.lin.ksum + (int64_t)bh * kD)[lane];
+    float2 bias2 = make_float2(0.0f, 0.0f);
+    if (p.lin.bias != nullptr) bias2 = reinterpret_cast<const float2*>(p.lin.bias)[lane];
+    uint2 oh[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
       const int dt = i >> 2, g = i & 3;
-      const int d = 32 * dt + 8 * g + 4 * hh;
-      const float4 s4 = s4a[i];
-      *reinterpret_cast<uint2*>(stage + l32 * kPitch + 2 * d) =
-          half4<DT>(oacc[dt][4 * g + 0] * inv_l * s4.x, oacc[dt][4 * g + 1] * inv_l * s4.y,
-                    oacc[dt][4 * g + 2] * inv_l * s4.z, oacc[dt][4 * g + 3] * inv_l * s4.w);
+      float o4[4] = {oacc[dt][4 * g + 0] * inv_l * s4a[i].x, oacc[dt][4 * g + 1] * inv_l * s4a[i].y,
+                     oacc[dt][4 * g + 2] * inv_l * s4a[i].z, oacc[dt][4 * g + 3] * inv_l * s4a[i].w};
+      // (pinned: the product and the conversion may otherwise become one fp16 instruction, with one rounding instead of two)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pin(o4[e]);
+      oh[i] = half4<DT>(o4[0], o4[1], o4[2], o4[3]);
+    }
+    __syncthreads();  // waves that ended early (no query rows) do not count
+    constexpr int kMatBytes = kD * kD * 2;
+    const uint8_t* mat = reinterpret_cast<const uint8_t*>(p.lin.frag + (int64_t)bh * kD * kD);
+    const int n_waves = min(kW, (lq - qwg * kRowsWg + 31) >> 5);  // the waves still here share the copies
+    if (n_waves == kW) {
+#pragma unroll
+      for (int i = 0; i < kMatBytes / 1024 / kW; ++i) lds_copy16(mat, (unsigned)((i * kW + wave) * 64 + lane) * 16, smem + (i * kW + wave) * 1024);
+    } else {
+#pragma unroll 1
+      for (int i = wave; i < kMatBytes / 1024; i += n_waves) lds_copy16(mat, (unsigned)(i * 64 + lane) * 16, smem + i * 1024);
+    }
+    float* s_ksum = reinterpret_cast<float*>(smem + kMatBytes);
+    float* s_bias = s_ksum + kD;
+    if (wave == 0) {
+      reinterpret_cast<float2*>(s_ksum)[lane] = ks2;
+      reinterpret_cast<float2*>(s_bias)[lane] = bias2;
+    }
+    float x[8][8];
+    const float rinv = sla_row_exps<DT>(lraw, x);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    uint4 fq[8];
+    const float scale = sla_row_scale<DT>(x, rinv, s_ksum, hh, fq);
+    stage = smem + kMatBytes + 2 * kD * 4 + wave * (32 * kPitch);
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      const v16f lin = sla_row_product<DT>(reinterpret_cast<const uint4*>(smem), fq, dt, lane);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int d = 32 * dt + 8 * g + 4 * hh;
+        const float4 bs = *reinterpret_cast<const float4*>(s_bias + d);
+        const uint2 lh = half4<DT>(__builtin_fmaf(lin[4 * g + 0], scale, bs.x), __builtin_fmaf(lin[4 * g + 1], scale, bs.y),
+                                   __builtin_fmaf(lin[4 * g + 2], scale, bs.z), __builtin_fmaf(lin[4 * g + 3], scale, bs.w));
+        float a4[8], o4[8];
+        widen8<DT>(make_uint4(lh.x, lh.y, 0, 0), a4);
+        widen8<DT>(make_uint4(oh[4 * dt + g].x, oh[4 * dt + g].y, 0, 0), o4);
+        *reinterpret_cast<uint2*>(stage + l32 * kPitch + 2 * d) = half4<DT>(a4[0] + o4[0], a4[1] + o4[1], a4[2] + o4[2], a4[3] + o4[3]);
+      }
     }
   } else {
+    const float2 mm = reinterpret_cast<const float2*>(s_vs + kD)[lane];
+    const bool has_mean = __any(mm.x != 0.0f || mm.y != 0.0f);  // wave-uniform
+    __syncthreads();  // waves that ended early (no query rows) do not count
+    if (!has_mean) {
 #pragma unroll
-    for (int i = 0; i < 4 * kG; ++i) {
-      const int dt = i >> 2, g = i & 3;
-      const int d = 32 * dt + 8 * g + 4 * hh;
-      const float4 s4 = s4a[i];
-      const float4 m4 = vm4[d >> 2];
-      *reinterpret_cast<uint2*>(stage + l32 * kPitch + 2 * d) =
-          half4<DT>(oacc[dt][4 * g + 0] * inv_l * s4.x + m4.x * keep_mean, oacc[dt][4 * g + 1] * inv_l * s4.y + m4.y * keep_mean,
-                    oacc[dt][4 * g + 2] * inv_l * s4.z + m4.z * keep_mean, oacc[dt][4 * g + 3] * inv_l * s4.w + m4.w * keep_mean);
+      for (int i = 0; i < 4 * kG; ++i) {
+        const int dt = i >> 2, g = i & 3;
+        const int d = 32 * dt + 8 * g + 4 * hh;
+        const float4 s4 = s4a[i];
+        *reinterpret_cast<uint2*>(stage + l32 * kPitch + 2 * d) =
+            half4<DT>(oacc[dt][4 * g + 0] * inv_l * s4.x, oacc[dt][4 * g + 1] * inv_l * s4.y,
+                      oacc[dt][4 * g + 2] * inv_l * s4.z, oacc[dt][4 * g + 3] * inv_l * s4.w);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4 * kG; ++i) {
+        const int dt = i >> 2, g = i & 3;
+        const int d = 32 * dt + 8 * g + 4 * hh;
+        const float4 s4 = s4a[i];
+        const float4 m4 = vm4[d >> 2];
+        *reinterpret_cast<uint2*>(stage + l32 * kPitch + 2 * d) =
+            half4<DT>(oacc[dt][4 * g + 0] * inv_l * s4.x + m4.x * keep_mean, oacc[dt][4 * g + 1] * inv_l * s4.y + m4.y * keep_mean,
+                      oacc[dt][4 * g + 2] * inv_l * s4.z + m4.z * keep_mean, oacc[dt][4 * g + 3] * inv_l * s4.w + m4.w * keep_mean);
+      }
     }
   }
   // LDS serves one wave's accesses in order: the reads below see the writes above
@@ -1065,7 +1135,7 @@ constexpr size_t max_lds() {
                  : WgShape<kW>::kRingBytes + 2048 + (kW == 8 ? kMaxKeyTiles : kShortMaxKeyTiles) * 4;
 }
 
-template <int DT, bool kPwlExp, bool kSparse, int kW, bool kCausal, bool kTileSkip = false, int kG = 4>
+template <int DT, bool kPwlExp, bool kSparse, int kW, bool kCausal, bool kTileSkip = false, int kG = 4, bool kLinear = false>
 hipError_t launch_variant(const AttnParams& p, dim3 grid, size_t lds, int n_qwg, int n_wg, int wg_per_xcd,
                           hipStream_t s) {
   // more than 64 KiB of dynamic LDS has to be requested per kernel, once per device
@@ -1076,12 +1146,12 @@ hipError_t launch_variant(const AttnParams& p, dim3 grid, size_t lds, int n_qwg,
   if (e != hipSuccess) return e;
   if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
   if (!requested[dev].load(std::memory_order_acquire)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal>),
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal, kLinear>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds<kSparse, kW>());
     if (e != hipSuccess) return e;
     requested[dev].store(true, std::memory_order_release);
   }
-  sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal><<<grid, dim3(kW * 64), lds, s>>>(p, n_qwg, n_wg, wg_per_xcd);
+  sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal, kLinear><<<grid, dim3(kW * 64), lds, s>>>(p, n_qwg, n_wg, wg_per_xcd);
   return hipGetLastError();
 }
 
@@ -1242,6 +1312,14 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   if (p.causal && p.batch_run == 0) causal_grid(&p, n_qwg);  // (the same number of workgroups)
   // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
   const size_t lds = (waves == 4 ? WgShape<4>::kRingBytes : WgShape<8>::kRingBytes) + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
+  if (p.lin.frag != nullptr) {
+    if (waves != 4 || p.block_mask == nullptr || p.causal || !p.exact_exp2 || p.tile_skip || p.d_out != kD || p.q_lens != nullptr ||
+        p.k_lens != nullptr)
+      return hipErrorInvalidValue;
+    return p.o.dtype == KSANA_SAGE_BF16
+               ? launch_variant<KSANA_SAGE_BF16, false, true, 4, false, false, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
+               : launch_variant<KSANA_SAGE_FP16, false, true, 4, false, false, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s);
+  }
   if (waves == 4) {
     if (plain_causal) return launch_causal(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
     if (sparse)

@@ -222,7 +222,7 @@ ksana_sage::QkvCall qkv_call(bool with_q, const ksana_sage::InTensor& q, const k
 
 int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
               const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags,
-              const ksana_sage::InTensor* q_rows, float q_premul, void* stream);
+              const ksana_sage::InTensor* q_rows, float q_premul, void* stream, const ksana_sage::AttnLinear* lin = nullptr);
 
 int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype, int o_dtype, const int64_t q_st[4],
                  const int64_t k_st[4], const int64_t v_st[4], const int64_t o_st[4], const ksana_sage_shape* s,
@@ -756,6 +756,11 @@ int ksana_sage_sla_forward(const void* q, const void* k, const void* v, void* o,
     if (e != hipSuccess) return hip_fail(e, "sparse-linear quantizer launch");
   }
   if (int rc = ksana_sage_sla_block_map(pooled_q, pooled_k, dtype, s->B, s->Hq, l.nq, l.nk, keep, map, stream)) return rc;
+  if (keep >= 1) {
+    // Every query block has a key block: the linear branch's second pass rides in the attention kernel's epilogue.
+    const ksana_sage::AttnLinear lin{frag, ksum, proj_bias};
+    return attn_impl(ws, o, dtype, o_st, s, map, map_st, nullptr, nullptr, 0, 0, &qt, 0.0f, stream, &lin);
+  }
   if (int rc = attn_impl(ws, o, dtype, o_st, s, map, map_st, nullptr, nullptr, 0, 0, nullptr, 0.0f, stream)) return rc;
   const StageRange range("ksana_sage.sla_linear");
   const ksana_sage::InTensor add = in_tensor(o, dtype, o_st);
@@ -829,10 +834,11 @@ int ksana_sage_forward_varlen(const void* q, const void* k, const void* v, void*
 }  // extern "C"
 
 namespace {
-// q_rows: nullptr, or Q as the caller has it (validated, of the result's dtype) for the kernel to quantize
+// q_rows: nullptr, or Q as the caller has it (validated, of the result's dtype) for the kernel to quantize - with lin, for
+// the linear branch that the kernel then adds
 int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
               const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags,
-              const ksana_sage::InTensor* q_rows, float q_premul, void* stream) {
+              const ksana_sage::InTensor* q_rows, float q_premul, void* stream, const ksana_sage::AttnLinear* lin) {
   const StageRange range("ksana_sage.attention");
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_mask(s, block_mask, mask_st)) return rc;
@@ -849,6 +855,7 @@ int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_s
   ksana_sage_workspace_layout(s, &l);
   ksana_sage::AttnParams p;
   if (q_rows != nullptr) p.q_rows = *q_rows, p.q_premul = q_premul;
+  if (lin != nullptr) p.lin = *lin;
   p.q_i8 = ws_at<int8_t>(ws, l.q_i8);
   p.q_scale = ws_at<float>(ws, l.q_scale);
   p.k_tiles = ws_at<int8_t>(ws, l.k_i8);

@@ -195,6 +195,12 @@ hipError_t launch_quant_sla(const QkvCall& call, const SlaFinal& f, hipStream_t 
 hipError_t launch_sla_block_map(const uint16_t* pooled_q, const uint16_t* pooled_k, int dtype, int BH, int nq, int nk, int keep,
                                 int8_t* block_map, hipStream_t s);
 
+// The linear branch of the sparse-linear backend as launch_quant_sla leaves it (frag == nullptr: none), the bias or nullptr
+struct AttnLinear {
+  const uint16_t* frag = nullptr;
+  const float *ksum = nullptr, *bias = nullptr;
+};
+
 struct AttnParams {
   // q_rows.ptr != nullptr: Q as the caller has it (of the result's dtype); every wave quantizes its own rows, q_i8 and q_scale
   // are not read
@@ -230,6 +236,9 @@ struct AttnParams {
   // filled in by the launcher for causal calls: (batch, head) pairs an XCD has to itself, the pairs left over, and how many
   // of its own it walks through together (0: not a causal call, or one numbered by batch_run)
   int causal_own = 0, causal_rest = 0, causal_group = 0;
+  // lin.frag != nullptr: that branch is added to every row; q_rows is then Q as the caller has it, for the branch (q_i8 is
+  // read as ever).  With a block mask that gives every query block a key block, head size 128, no counts, default variant.
+  AttnLinear lin{};
 };
 constexpr int kMaxSplitPartials = 256;  // (workgroups beyond the last full round) x (runs each) never exceeds this
 constexpr int kMinTilesPerSplit = 8;    // a run shorter than this does not repay its prologue

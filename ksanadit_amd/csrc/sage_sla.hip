@@ -108,48 +108,12 @@ __global__ __launch_bounds__(kSlaThreads, 2) void sla_apply_kernel(const uint16_
       }
     }
     float x[8][8];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      widen8<DT>(raw[s], x[s]);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, x[s][e]);
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    const float c = -mx * kLog2e;
-    float sum = 0.0f;
-#pragma unroll
-    for (int s = 0; s < 8; ++s)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        x[s][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[s][e], kLog2e, c));
-        sum += x[s][e];
-      }
-    sum += __shfl_xor(sum, 32);
-    const float inv = __builtin_amdgcn_rcpf(sum);
+    const float inv = sla_row_exps<DT>(raw, x);
     uint4 fq[8];
-    float den = 0.0f;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      uint32_t pw[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float f0 = x[s][2 * e] * inv, f1 = x[s][2 * e + 1] * inv;
-        pw[e] = pack2<DT>(f0, f1);
-        den = __builtin_fmaf(f0, s_ks[16 * s + 8 * g + 2 * e], den);
-        den = __builtin_fmaf(f1, s_ks[16 * s + 8 * g + 2 * e + 1], den);
-      }
-      fq[s] = make_uint4(pw[0], pw[1], pw[2], pw[3]);
-    }
-    den += __shfl_xor(den, 32);
-    const float scale = __builtin_amdgcn_rcpf(1e-5f + den);
+    const float scale = sla_row_scale<DT>(x, inv, s_ks, g, fq);
 #pragma unroll
     for (int nt = 0; nt < 4; ++nt) {
-      v16f acc;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-#pragma unroll
-      for (int s = 0; s < 8; ++s) acc = mfma32<DT>(s_m[(nt * 8 + s) * 64 + lane], fq[s], acc);
+      const v16f acc = sla_row_product<DT>(s_m, fq, nt, lane);
       // register r: output channel 32 nt + 8 (r / 4) + 4 g + r % 4 of row l32
 #pragma unroll
       for (int q4 = 0; q4 < 4; ++q4) {

@@ -360,4 +360,61 @@ __device__ __forceinline__ void sla_kv_finalize(int slice, int bh, const float* 
   }
 }
 
+// ---- the second pass, one row per pair of lanes (row = lane % 32 of the wave, g = lane / 32): out = phi(q) M / (1e-5 +
+// phi(q) . ksum) ---------------------------------------------------------------------------------------------------
+// raw[s]: the channels 16 s + 8 g .. + 7 of the lane's row, s = 0 .. 7 - half of the row, and its B operands of the
+// 32x32x16 instruction; the other half sits in lane + 32.  x: the exponentials of its channels; returns 1 / their row sum.
+template <int DT>
+__device__ __forceinline__ float sla_row_exps(const uint4 (&raw)[8], float (&x)[8][8]) {
+  float mx = -INFINITY;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    widen8<DT>(raw[s], x[s]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, x[s][e]);
+  }
+  mx = fmaxf(mx, __shfl_xor(mx, 32));
+  const float c = -mx * kLog2e;
+  float sum = 0.0f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      x[s][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[s][e], kLog2e, c));
+      sum += x[s][e];
+    }
+  sum += __shfl_xor(sum, 32);
+  return __builtin_amdgcn_rcpf(sum);
+}
+// the operands fq (phi in the half type) and 1 / (1e-5 + phi . ksum); s_ks: ksum of the head, in LDS
+template <int DT>
+__device__ __forceinline__ float sla_row_scale(const float (&x)[8][8], float inv, const float* s_ks, int g, uint4 (&fq)[8]) {
+  float den = 0.0f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    uint32_t pw[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float f0 = x[s][2 * e] * inv, f1 = x[s][2 * e + 1] * inv;
+      pw[e] = pack2<DT>(f0, f1);
+      den = __builtin_fmaf(f0, s_ks[16 * s + 8 * g + 2 * e], den);
+      den = __builtin_fmaf(f1, s_ks[16 * s + 8 * g + 2 * e + 1], den);
+    }
+    fq[s] = make_uint4(pw[0], pw[1], pw[2], pw[3]);
+  }
+  den += __shfl_xor(den, 32);
+  return __builtin_amdgcn_rcpf(1e-5f + den);
+}
+// Output channels 32 nt .. + 31 of the lane's row, transposed (out^T = M^T phi(q)^T): register r is channel
+// 32 nt + 8 (r / 4) + 4 g + r % 4.  s_m: M in operand order, in LDS.
+template <int DT>
+__device__ __forceinline__ v16f sla_row_product(const uint4* s_m, const uint4 (&fq)[8], int nt, int lane) {
+  v16f acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) acc = mfma32<DT>(s_m[(nt * 8 + s) * 64 + lane], fq[s], acc);
+  return acc;
+}
+
 }  // namespace ksana_sage
