@@ -429,45 +429,49 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if constexpr (kCausal) return jj == jdiag;
     return false;
   };
-  // scores of keys beyond the row's own position drop below every real score ...
-  auto causal_half = [&](v16i blk, int t) -> v16i {
-    // (pinned: the comparisons below are the same in every step, and hoisted out of the key loop they would sit in
+  // Tiles of which a lane's query sees the first n keys only - the one on a wave's diagonal (n depends on the lane) and the
+  // head's last one where its keys are no multiple of 64: the scores of the others drop below every real score ...
+  auto blank_half = [&](v16i blk, int t, int n) -> v16i {
+    // (pinned: what follows is the same in every step, and hoisted out of the key loop it would sit in
     // 32 scalar register pairs for a block that runs once per wave)
-    int row_local = (q0 & 63) + l32;
-    pin(row_local);
+    int last = n - 1 - 4 * hh;
+    pin(last);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      // all-ones where the key lies beyond the row
-      const int beyond = (row_local - 4 * hh - (32 * t + 8 * (r >> 2) + (r & 3))) >> 31;
+      const int beyond = (last - (32 * t + 8 * (r >> 2) + (r & 3))) >> 31;  // all-ones where the key is one of those
       blk[r] = (blk[r] & ~beyond) | ((kMagicBits - (1 << 22)) & beyond);
     }
     return blk;
   };
-  auto causal_scores = [&](v16i (&blk)[2]) {
-    blk[0] = causal_half(blk[0], 0);
-    blk[1] = causal_half(blk[1], 1);
+  auto blank_scores = [&](v16i (&blk)[2], int n) {
+    blk[0] = blank_half(blk[0], 0, n);
+    blk[1] = blank_half(blk[1], 1, n);
   };
   // ... and their probability bytes are cleared outright (code 0 is +0.0 in e4m3), so that a row
   // whose scale is zero does not count them either
-  auto causal_probs = [&](v8i& pf) {
-    int row_local = (q0 & 63) + l32;
-    pin(row_local);
+  auto blank_probs = [&](v8i& pf, int n) {
+    int first = n - 4 * hh;
+    pin(first);
 #pragma unroll
     for (int w = 0; w < 8; ++w) {
-      // bytes of the first min(max(n, 0), 4) keys of this dword stay
-      const int n = min(max(row_local - 4 * hh - (32 * (w >> 2) + 8 * (w & 3)) + 1, 0), 4);
-      const unsigned keep = n >= 4 ? 0xffffffffu : ((1u << (8 * n)) - 1u);
+      // bytes of the first min(max(m, 0), 4) keys of this dword stay
+      const int m = min(max(first - (32 * (w >> 2) + 8 * (w & 3)), 0), 4);
+      const unsigned keep = m >= 4 ? 0xffffffffu : ((1u << (8 * m)) - 1u);
       pf[w] &= (int)keep;
     }
   };
+  const int n_diag = (q0 & 63) + l32 + 1;
 
   // ---- asynchronous tile copies: HBM/L2 -> LDS without passing through registers ----------
   // Each wave moves its 1 KiB slice of the K tile and of the V^T tile (lane i -> byte 16*i of
   // the slice).  Copies retire in issue order, so "at most 2*n outstanding" == "all but the
   // newest n tiles have landed".
-  // keys >= lk live only in the last key tile, which (if the list holds it) is the last entry
-  const bool has_tail = (lk & (kBlkK - 1)) != 0 && tile_of(n_tiles - 1) == nkb - 1;
-  const int n_main = has_tail ? n_tiles - 1 : n_tiles;  // entries handled by the pipelined loop
+  // keys >= lk live only in the last key tile, which (if the list holds it) is the last entry; -1: there are none.  That tile
+  // is a step of the loop like the others, blanked as the diagonal's is.  (As a step of its own after the loop, with a branch
+  // per blanked score, one key of 64 in it cost 6 us a workgroup, 63 of them 2: 40 heads of 1536 queries, 512 / 513 / 575 keys
+  // 18.0 / 24.0 / 20.5 us, 18.1 / 18.8 / 19.1 like this.)
+  const int n_last = lk & (kBlkK - 1);
+  const int tail = n_last != 0 && tile_of(n_tiles - 1) == nkb - 1 ? n_tiles - 1 : -1;
   // LDS slot of a tile's K half / V^T half
   auto k_slot = [&](int tile) -> uint8_t* { return smem + (tile & (kStages - 1)) * kTileBytes; };
   auto v_slot = [&](int tile) -> uint8_t* { return smem + (kStages + (tile & (kStages - 1))) * kTileBytes; };
@@ -556,9 +560,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   constexpr bool kSlotZeroSoon = Shape::kAheadK == kStages || (kUnrolled && Shape::kGroup > 1);
   // Without a list, the steps before any of the workgroup's waves meets its diagonal tile know nothing of it: they are the
   // dense loop's (with the diagonal's code in every unrolled step to be jumped over,
-  // 8 191 tokens of 32 heads took 334 us instead of 323).
+  // 8 191 tokens of 32 heads took 334 us instead of 323).  No unrolled step meets the ragged last tile either.
   constexpr bool kDiagApart = kCausal && !kSparse && kUnrolled;
-  const int n_plain = kDiagApart ? min(n_main, max(0, ((qwg * kRowsWg) >> 6) - 1)) : n_main;
+  const int n_whole = tail >= 0 ? max(0, n_tiles - 2) : n_tiles;  // steps that neither form that tile's scores nor its probabilities
+  const int n_plain = kDiagApart ? min(n_whole, max(0, ((qwg * kRowsWg) >> 6) - 1)) : n_whole;
   const int n_grouped = kUnrolled && Shape::kGroup > 1 ? n_plain / kStages * kStages : 0;
 
   // The compiler does not see the asynchronous copies in the memory-operation counter it models.  Every ordinary global
@@ -594,7 +599,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   if (!active) {
     // same copy / barrier sequence as the active waves
     if constexpr (kSlotZeroSoon) __builtin_amdgcn_s_barrier();
-    for (int j = 0; j < n_main; ++j) {
+    for (int j = 0; j < n_tiles; ++j) {
       // (looks the tiles up where they are needed: a wave without rows has nothing an LDS wait could hold up)
       copy_half(v_src, j + kAhead, v_slot(j + kAhead));
       copy_half(k_src, j + Shape::kAheadK, k_slot(j + Shape::kAheadK));
@@ -686,7 +691,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   v16i s_a[2], s_b[2];
   qk_tile<kG>(k_slot(0), lane, qf, magic, s_a);
   if constexpr (kSlotZeroSoon) __builtin_amdgcn_s_barrier();
-  if (diag_at(0)) causal_scores(s_a);
+  if (diag_at(0)) blank_scores(s_a, n_diag);
+  if (tail == 0) blank_scores(s_a, n_last);
 
   // What a step needs to know about its tile before the first probability: the scale, the exponent's constant and
   // whether a reference point moves.  Worked out at the end of the step before, so that its chain of dependent
@@ -711,7 +717,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if (__ballot(!(m_half <= x_limit)) != 0) {  // (NaN counts as above)
       asm volatile("");  // (two branches on purpose: merged into one condition, the second is computed in every step)
       // (a tile this wave's mask row does not ask for, or that is not this loop's, leaves the points alone)
-      if (jn < n_main && mine_at(jn)) {
+      if (jn < n_tiles && mine_at(jn)) {
         alpha = move_point(mx, sc, mneg);
         moved = 1;
       }
@@ -813,7 +819,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (kCausal && !(kDiagApart && kAt >= 0)) {  // rare, wave-uniform: the next tile is the one on this wave's diagonal
-      if (j + 1 < n_tiles && diag_at(j + 1)) causal_scores(s_nxt);
+      if (j + 1 < n_tiles && diag_at(j + 1)) blank_scores(s_nxt, n_diag);
+    }
+    if constexpr (kAt < 0) {
+      if (j + 1 == tail) blank_scores(s_nxt, n_last);
     }
     __builtin_amdgcn_s_setprio(0);
     // 4 x [PV MFMA of tile j-1 (64 matrix cycles) | 4 probabilities of tile j | a quarter of
@@ -847,7 +856,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
         for (int i = 0; i < 8; ++i) pf[i] = 0;
       }
-      if (diag_at(j)) causal_probs(pf);
+      if (diag_at(j)) blank_probs(pf, n_diag);
+    }
+    if constexpr (kAt < 0) {
+      if (j == tail) blank_probs(pf, n_last);
     }
     look_ahead(j + 1, mx, ks_nxt, alpha, moved);
     // after this barrier: K tile j+2 and V^T tile j are visible to every wave, and nobody reads their predecessors any
@@ -875,64 +887,24 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         ks_off += 4 * kStages;
       }
     }
-    for (; j + 2 <= n_main; j += 2) {
+    for (; j + 2 <= n_tiles; j += 2) {
       tile_step(Anywhere{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
       tile_step(Anywhere{}, j + 1, s_b, s_a, pf_y, pf_x, alpha_even, moved_even);
     }
-    if (j < n_main) tile_step(Anywhere{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
+    if (j < n_tiles) tile_step(Anywhere{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may outlive the workgroup's LDS
-  // The loop's last barrier vouches only for copies a few steps old: before the peeled last tile's V^T half is read, the
-  // waves meet once more after each has seen its own copies land (uniform condition).
-  if (has_tail) __builtin_amdgcn_s_barrier();
-  if (n_main > 0) {  // drain: PV of the last pipelined tile
-    if ((n_main & 1) != 0) {
+  {  // drain: PV of the last tile
+    if ((n_tiles & 1) != 0) {
       if (moved_even != 0) scale_o(alpha_even);
     } else {
       if (moved_odd != 0) scale_o(alpha_odd);
     }
-    const uint8_t* vst = v_slot(n_main - 1);
-    const v8i pf_last = (n_main & 1) ? pf_y : pf_x;  // written by the last step
+    const uint8_t* vst = v_slot(n_tiles - 1);
+    const v8i pf_last = (n_tiles & 1) ? pf_y : pf_x;  // written by the last step
 #pragma unroll
     for (int dt = 0; dt < kG; ++dt) pv_slice(vst, dt, pf_last);
     lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_last, lacc, 0, 0, 0, 0, 0, 0);
-  }
-  if (has_tail && mine_at(n_tiles - 1)) {  // ragged last tile, not pipelined: mask keys >= lk
-    const int j = nkb - 1, jj = n_tiles - 1;
-    v16i (&s_cur)[2] = (n_main & 1) ? s_b : s_a;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int key = j * kBlkK + 32 * t + 8 * (r >> 2) + 4 * hh + (r & 3);
-        if (key >= lk) s_cur[t][r] = kMagicBits - (1 << 22);  // below every real score
-      }
-    float sc = qs * s_ks[jj];
-    float mneg = -kMagicVal * sc;
-    scale_o(move_point(lane_max(s_cur), sc, mneg));
-    const float c = x_base + mneg;
-    const float scp = kPwlExp ? 8.0f * sc : sc;
-    const float cp = kPwlExp ? __builtin_fmaf(8.0f, c, 55.5f) : c;
-    v8i pf;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int w = pack4(s_cur[t][4 * g], s_cur[t][4 * g + 1], s_cur[t][4 * g + 2], s_cur[t][4 * g + 3], scp, cp);
-        // zero the bytes of keys at or beyond lk (code 0 is +0.0 in e4m3)
-        unsigned keep = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = j * kBlkK + 32 * t + 8 * g + 4 * hh + i;
-          if (key < lk) keep |= 0xffu << (8 * i);
-        }
-        pf[4 * t + g] = w & (int)keep;
-      }
-    if (diag_at(jj)) causal_probs(pf);
-    const uint8_t* vst = v_slot(jj);
-#pragma unroll
-    for (int dt = 0; dt < kG; ++dt) pv_slice(vst, dt, pf);
-    lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, lacc, 0, 0, 0, 0, 0, 0);
   }
 
   if (is_run) {

@@ -150,3 +150,24 @@ def test_query_rows_that_are_not_finite_stay_on_their_own(hip_device, waves, Lk,
                                       causal=mode == "causal").cpu()[0])
     assert torch.isnan(outs[1][bad]).all()
     assert torch.isfinite(outs[1][~bad]).all() and torch.equal(outs[0][~bad], outs[1][~bad])
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("whole", range(15))
+@pytest.mark.parametrize("rest", [1, 37, 63])
+def test_the_ragged_tile_at_any_place_of_the_ring(hip_device, waves, whole, rest):
+    """The last, ragged key tile is a step of the loop like the others: at every place of the ring and of a group, with few
+    and with all but one of its keys, and the largest score of a row among the ones that exist or just short of them."""
+    Lq, H, Lk = 130, 1, 64 * whole + rest
+    print(f"case waves={waves} Lk={Lk}", flush=True)
+    g = torch.Generator().manual_seed(Lk)
+    q, k, v = (torch.randn((1, n, H, 128), generator=g).to(torch.bfloat16) for n in (Lq, Lk, Lk))
+    k[:, -1] = 3 * q[:, 5]  # row 5 sees little but the very last key
+    qd, kd, vd = (t.to(hip_device) for t in (q, k, v))
+    ws = sage_ops.workspace_for(qd, kd)
+    sage_ops.quant_q(qd, ws, 128**-0.5), sage_ops.quant_k(kd, ws, True), sage_ops.quant_v(vd, ws)
+    out = sage_ops.attn_fwd(ws, torch.empty_like(qd), wg_waves=waves).cpu()
+    _close(out, _emul(ws, Lq, Lk, q.dtype))
+    short = torch.tensor([max(Lk - 1, 1)], dtype=torch.int32, device=hip_device)  # the count a batch entry may have of its own
+    out = sage_ops.attn_fwd(ws, torch.empty_like(qd), wg_waves=waves, k_lens=short).cpu()
+    _close(out, _emul(ws, Lq, Lk, q.dtype, k_lens=short.cpu()))
