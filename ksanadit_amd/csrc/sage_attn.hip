@@ -690,7 +690,9 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 
   v16i s_a[2], s_b[2];
   qk_tile<kG>(k_slot(0), lane, qf, magic, s_a);
-  if constexpr (kSlotZeroSoon) __builtin_amdgcn_s_barrier();
+  // (with the wait: a bare barrier lets the tile's last reads be on their way still when a wave without rows, which has nothing
+  // else to do, requests the tile that goes into their slot)
+  if constexpr (kSlotZeroSoon) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if (diag_at(0)) blank_scores(s_a, n_diag);
   if (tail == 0) blank_scores(s_a, n_last);
 

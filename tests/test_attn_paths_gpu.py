@@ -171,3 +171,20 @@ def test_the_ragged_tile_at_any_place_of_the_ring(hip_device, waves, whole, rest
     short = torch.tensor([max(Lk - 1, 1)], dtype=torch.int32, device=hip_device)  # the count a batch entry may have of its own
     out = sage_ops.attn_fwd(ws, torch.empty_like(qd), wg_waves=waves, k_lens=short).cpu()
     _close(out, _emul(ws, Lq, Lk, q.dtype, k_lens=short.cpu()))
+
+
+@pytest.mark.parametrize("rows", [1, 31, 40, 96])
+@pytest.mark.parametrize("Lk", [77, 128, 300, 448])
+def test_a_workgroup_with_waves_that_have_no_rows(hip_device, rows, Lk):
+    """The last workgroup of a head has one, two or three waves with rows; the others only move tiles and run ahead as far
+    as the barriers let them.  With many heads, in a kernel's first launch after another one: the same bits as in 8 waves."""
+    B, H, Lq = 2, 64, 4096 + rows
+    print(f"case rows={rows} Lk={Lk}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(Lk)
+    q, k, v = (torch.randn((B, n, h, 128), generator=g, device=hip_device).half() for n, h in ((Lq, H), (Lk, 16), (Lk, 16)))
+    ws = sage_ops.workspace_for(q, k)
+    for _ in range(3):
+        sage_ops.quant_q(q, ws, 128**-0.5), sage_ops.quant_k(k, ws, True), sage_ops.quant_v(v, ws)
+        four = sage_ops.attn_fwd(ws, torch.empty_like(q), wg_waves=4)
+        eight = sage_ops.attn_fwd(ws, torch.empty_like(q), wg_waves=8)
+        assert torch.equal(four, eight)
