@@ -64,24 +64,9 @@ constexpr int kMaxKeyTiles = 4096;           // K scales of one head are kept in
 constexpr int kShortKeyTiles = 16;           // calls with at most this many key tiles (Lk <= 1024) are never cut into runs of keys
 constexpr int kShortMaxKeyTiles = 2048;      // the most key tiles a dense 4-wave workgroup can hold scales for
 
-// 16 bytes per lane from global memory straight into LDS at `lds_dst + 16 * lane` (lds_dst is
-// wave-uniform).  Written as inline assembly on purpose: the compiler's wait-count model treats
-// the builtin form as a possible LDS access through the flat path and from then on waits for
-// ALL outstanding LDS reads before every use (lgkmcnt(0)), which serialises the operand
-// prefetch.  The copy is tracked by hand instead (vmcnt, see tile_barrier).
-// The global address is a wave-uniform base (scalar registers) plus a 32-bit per-lane offset.
-// M0 is written and named as clobbered; the compiler remarks that M0 is a register it reserves (it re-materialises
-// M0 before each of its own uses and never keeps a value live in it), which is the behaviour relied on here.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void lds_copy16(const void* gbase, unsigned lane_off, const void* lds_dst) {
-  const unsigned lds_off = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)lds_dst;
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(lds_off), "v"(lane_off), "s"(gbase)
-               : "memory", "m0");
-}
-// The same through a buffer descriptor: 16 bytes per lane from (base + src_off + lane_off) to `lds_base + kSlot`.  One scalar
+// lds_copy16 through a buffer descriptor: 16 bytes per lane from (base + src_off + lane_off) to `lds_base + kSlot`.  One scalar
 // offset serves every buffer whose tiles have the same number, and a slot known at compile time rides in the
 // instruction that writes M0 - two scalar instructions per copy where the 64-bit form above takes six.
 template <int kSlot>
@@ -429,45 +414,14 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if constexpr (kCausal) return jj == jdiag;
     return false;
   };
-  // Tiles of which a lane's query sees the first n keys only - the one on a wave's diagonal (n depends on the lane) and the
-  // head's last one where its keys are no multiple of 64: the scores of the others drop below every real score ...
-  auto blank_half = [&](v16i blk, int t, int n) -> v16i {
-    // (pinned: what follows is the same in every step, and hoisted out of the key loop it would sit in
-    // 32 scalar register pairs for a block that runs once per wave)
-    int last = n - 1 - 4 * hh;
-    pin(last);
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int beyond = (last - (32 * t + 8 * (r >> 2) + (r & 3))) >> 31;  // all-ones where the key is one of those
-      blk[r] = (blk[r] & ~beyond) | ((kMagicBits - (1 << 22)) & beyond);
-    }
-    return blk;
-  };
-  auto blank_scores = [&](v16i (&blk)[2], int n) {
-    blk[0] = blank_half(blk[0], 0, n);
-    blk[1] = blank_half(blk[1], 1, n);
-  };
-  // ... and their probability bytes are cleared outright (code 0 is +0.0 in e4m3), so that a row
-  // whose scale is zero does not count them either
-  auto blank_probs = [&](v8i& pf, int n) {
-    int first = n - 4 * hh;
-    pin(first);
-#pragma unroll
-    for (int w = 0; w < 8; ++w) {
-      // bytes of the first min(max(m, 0), 4) keys of this dword stay
-      const int m = min(max(first - (32 * (w >> 2) + 8 * (w & 3)), 0), 4);
-      const unsigned keep = m >= 4 ? 0xffffffffu : ((1u << (8 * m)) - 1u);
-      pf[w] &= (int)keep;
-    }
-  };
-  const int n_diag = (q0 & 63) + l32 + 1;
+  const int n_diag = (q0 & 63) + l32 + 1;  // keys of its diagonal's tile that a lane's query sees
 
   // ---- asynchronous tile copies: HBM/L2 -> LDS without passing through registers ----------
   // Each wave moves its 1 KiB slice of the K tile and of the V^T tile (lane i -> byte 16*i of
   // the slice).  Copies retire in issue order, so "at most 2*n outstanding" == "all but the
   // newest n tiles have landed".
   // keys >= lk live only in the last key tile, which (if the list holds it) is the last entry; -1: there are none.  That tile
-  // is a step of the loop like the others, blanked as the diagonal's is.  (As a step of its own after the loop, with a branch
+  // is a step of the loop like the others, blanked as the diagonal's is (blank_scores, blank_probs).  (As a step of its own after the loop, with a branch
   // per blanked score, one key of 64 in it cost 6 us a workgroup, 63 of them 2: 40 heads of 1536 queries, 512 / 513 / 575 keys
   // 18.0 / 24.0 / 20.5 us, 18.1 / 18.8 / 19.1 like this.)
   const int n_last = lk & (kBlkK - 1);
@@ -693,8 +647,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // (with the wait: a bare barrier lets the tile's last reads be on their way still when a wave without rows, which has nothing
   // else to do, requests the tile that goes into their slot)
   if constexpr (kSlotZeroSoon) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  if (diag_at(0)) blank_scores(s_a, n_diag);
-  if (tail == 0) blank_scores(s_a, n_last);
+  if (diag_at(0)) blank_scores<kMagicBits>(s_a, hh, n_diag);
+  if (tail == 0) blank_scores<kMagicBits>(s_a, hh, n_last);
 
   // What a step needs to know about its tile before the first probability: the scale, the exponent's constant and
   // whether a reference point moves.  Worked out at the end of the step before, so that its chain of dependent
@@ -821,10 +775,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (kCausal && !(kDiagApart && kAt >= 0)) {  // rare, wave-uniform: the next tile is the one on this wave's diagonal
-      if (j + 1 < n_tiles && diag_at(j + 1)) blank_scores(s_nxt, n_diag);
+      if (j + 1 < n_tiles && diag_at(j + 1)) blank_scores<kMagicBits>(s_nxt, hh, n_diag);
     }
     if constexpr (kAt < 0) {
-      if (j + 1 == tail) blank_scores(s_nxt, n_last);
+      if (j + 1 == tail) blank_scores<kMagicBits>(s_nxt, hh, n_last);
     }
     __builtin_amdgcn_s_setprio(0);
     // 4 x [PV MFMA of tile j-1 (64 matrix cycles) | 4 probabilities of tile j | a quarter of
@@ -858,10 +812,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
         for (int i = 0; i < 8; ++i) pf[i] = 0;
       }
-      if (diag_at(j)) blank_probs(pf, n_diag);
+      if (diag_at(j)) blank_probs(pf, hh, n_diag);
     }
     if constexpr (kAt < 0) {
-      if (j == tail) blank_probs(pf, n_last);
+      if (j == tail) blank_probs(pf, hh, n_last);
     }
     look_ahead(j + 1, mx, ks_nxt, alpha, moved);
     // after this barrier: K tile j+2 and V^T tile j are visible to every wave, and nobody reads their predecessors any
@@ -1275,6 +1229,9 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   if (p.nkb > kMaxKeyTiles) return hipErrorInvalidValue;
   const bool sparse = p.block_mask != nullptr || p.causal;
   if (sparse && p.nkb > kSparseMaxKeyTiles) return hipErrorInvalidValue;
+  if (!sparse && p.q_rows.ptr != nullptr && p.q_lens == nullptr && p.k_lens == nullptr && p.exact_exp2 && !p.tile_skip && p.wg_waves == 0 &&
+      resident_call_suits(p.B, p.Hq, p.Lq, p.Lk))
+    return launch_resident(p, s);
   const bool plain_causal = p.causal && p.block_mask == nullptr && p.exact_exp2 && !p.tile_skip;  // no tile list
   int waves = pick_wg_waves(p);
   if (waves == 4 && p.nkb > (sparse ? kSparseMaxKeyTiles4 : kShortMaxKeyTiles)) waves = 8;

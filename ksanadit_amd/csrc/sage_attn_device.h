@@ -63,6 +63,56 @@ __device__ __forceinline__ void store4(uint16_t* dst, float a, float b, float c,
   *reinterpret_cast<uint2*>(dst) = half4<DT>(a, b, c, d);
 }
 
+// 16 bytes per lane from global memory straight into LDS at `lds_dst + 16 * lane` (lds_dst is
+// wave-uniform).  Written as inline assembly on purpose: the compiler's wait-count model treats
+// the builtin form as a possible LDS access through the flat path and from then on waits for
+// ALL outstanding LDS reads before every use (lgkmcnt(0)), which serialises the operand
+// prefetch.  The copy is tracked by hand instead (vmcnt, see tile_barrier).
+// The global address is a wave-uniform base (scalar registers) plus a 32-bit per-lane offset.
+// M0 is written and named as clobbered; the compiler remarks that M0 is a register it reserves (it re-materialises
+// M0 before each of its own uses and never keeps a value live in it), which is the behaviour relied on here.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void lds_copy16(const void* gbase, unsigned lane_off, const void* lds_dst) {
+  const unsigned lds_off = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)lds_dst;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds_off), "v"(lane_off), "s"(gbase)
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+// Tiles of which a lane's query sees the first n keys only - the one on a wave's diagonal (n depends on the lane) and a
+// head's last one where its keys are no multiple of 64: the scores of the others drop below every real score (hh = lane / 32)
+template <int kMagicBits>
+__device__ __forceinline__ void blank_scores(v16i (&blk)[2], int hh, int n) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    // (pinned: what follows is the same in every step, and hoisted out of the key loop it would sit in
+    // 32 scalar register pairs for a block that runs once per wave)
+    int last = n - 1 - 4 * hh;
+    pin(last);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int beyond = (last - (32 * t + 8 * (r >> 2) + (r & 3))) >> 31;  // all-ones where the key is one of those
+      blk[t][r] = (blk[t][r] & ~beyond) | ((kMagicBits - (1 << 22)) & beyond);
+    }
+  }
+}
+// ... and their probability bytes are cleared outright (code 0 is +0.0 in e4m3), so that a row
+// whose scale is zero does not count them either
+__device__ __forceinline__ void blank_probs(v8i& pf, int hh, int n) {
+  int first = n - 4 * hh;
+  pin(first);
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    // bytes of the first min(max(m, 0), 4) keys of this dword stay
+    const int m = min(max(first - (32 * (w >> 2) + 8 * (w & 3)), 0), 4);
+    const unsigned keep = m >= 4 ? 0xffffffffu : ((1u << (8 * m)) - 1u);
+    pf[w] &= (int)keep;
+  }
+}
+
 // S^T tile (64 keys x 32 queries) of one wave: two 32-key sub-tiles, kG 32-channel steps (the channel groups that
 // hold data: 4, or 2 for head size 64, whose upper 64 channels are zeros on both sides).
 template <int kG>

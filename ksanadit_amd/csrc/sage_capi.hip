@@ -953,7 +953,10 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
   }
   const int n_wg = s->B * s->Hq * ((s->Lq + ksana_sage::kAttnQPerWg - 1) / ksana_sage::kAttnQPerWg);
   const bool own_q = (flags & KSANA_SAGE_FLAG_Q_UNSTORED) && prep == nullptr && block_mask == nullptr && o_dtype == dtype &&
-                     ksana_sage::q_in_attention_pays(n_wg, (s->Lk + ksana_sage::kBlkK - 1) / ksana_sage::kBlkK);
+                     (ksana_sage::q_in_attention_pays(n_wg, (s->Lk + ksana_sage::kBlkK - 1) / ksana_sage::kBlkK) ||
+                      (!causal && q_lens == nullptr && k_lens == nullptr &&
+                       !(flags & (KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_TILE_SKIP | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES)) &&
+                       ksana_sage::resident_call_suits(s->B, s->Hq, s->Lq, s->Lk)));
   if (int rc = quant_qkv(!own_q, q, k, v, dtype, q_st, k_st, v_st, s, prep, sm_scale, smooth_k, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws,
                          stream))
     return rc;
