@@ -882,10 +882,11 @@ int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_s
   return e == hipSuccess ? 0 : hip_fail(e, "attention launch");
 }
 
-// The quantizers of a call whose arguments have been validated: of Q, K and V, or (with_q == false, no prep) of K and V
+// The quantizers of a call whose arguments have been validated: of Q, K and V, or (with_q == false, no prep) of K and V.
+// q_lens, k_lens: see QkvCall
 int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtype, const int64_t q_st[4], const int64_t k_st[4],
               const int64_t v_st[4], const ksana_sage_shape* s, const ksana_sage_prep* prep, float sm_scale, int smooth_k,
-              int smooth_v, void* ws, void* stream) {
+              int smooth_v, void* ws, void* stream, const int32_t* q_lens, const int32_t* k_lens) {
   if (!smooth_v) {
     const StageRange range("ksana_sage.quant_qkv");
     ksana_sage_ws_layout l;
@@ -896,8 +897,9 @@ int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtyp
       return rc;
     if (int rc = make_prep(prep, prep ? prep->k_norm_weight : nullptr, "k", k_st, s->B, s->Lk, s->D, ws_at<float>(ws, l.k_rms), &pk, &ppk))
       return rc;
-    const ksana_sage::QkvCall c = qkv_call(with_q, in_tensor(q, dtype, q_st, s->D), in_tensor(k, dtype, k_st, s->D),
-                                           in_tensor(v, dtype, v_st, s->D), s, l, sm_scale, smooth_k, ws);
+    ksana_sage::QkvCall c = qkv_call(with_q, in_tensor(q, dtype, q_st, s->D), in_tensor(k, dtype, k_st, s->D),
+                                     in_tensor(v, dtype, v_st, s->D), s, l, sm_scale, smooth_k, ws);
+    c.q_lens = q_lens, c.k_lens = k_lens;
     bool used = false;
     const hipError_t e = ksana_sage::launch_quant_qkv(c, ppq, ppk, static_cast<hipStream_t>(stream), &used);
     if (e != hipSuccess) return hip_fail(e, "q, k, v quantizer launch");
@@ -957,8 +959,9 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
                       (!causal && q_lens == nullptr && k_lens == nullptr &&
                        !(flags & (KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_TILE_SKIP | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES)) &&
                        ksana_sage::resident_call_suits(s->B, s->Hq, s->Lq, s->Lk)));
+  const bool trim = (flags & KSANA_SAGE_FLAG_WS_UNSTORED) && prep == nullptr;  // what no row or key that takes part needs
   if (int rc = quant_qkv(!own_q, q, k, v, dtype, q_st, k_st, v_st, s, prep, sm_scale, smooth_k, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws,
-                         stream))
+                         stream, trim ? q_lens : nullptr, trim ? k_lens : nullptr))
     return rc;
   const ksana_sage::InTensor q_rows = in_tensor(q, dtype, q_st, s->D);
   return attn_impl(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal,

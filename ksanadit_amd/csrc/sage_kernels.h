@@ -145,6 +145,9 @@ struct QkvCall {
   uint8_t* v_tiles;
   QuantSync sync;  // (the areas of K and V follow each other)
   int tiles_per_wg;  // filled in by the launcher
+  // nullptr, or (no folded step) the counts of the attention that follows and nobody else sees the codes: keys and query
+  // rows that take no part count for the statistics as ever, but blocks made of them alone are not quantized
+  const int32_t *q_lens, *k_lens;
 };
 hipError_t launch_quant_qkv(const QkvCall& call, const PrepParams* pq, const PrepParams* pk, hipStream_t s, bool* used);
 
