@@ -393,10 +393,10 @@ int ksana_sage_quant_q(const void* q, int dtype, const int64_t st[4], const ksan
 }
 
 // `k` != nullptr (the caller has checked k as a tensor): when q's path takes whole token rows anyway (a norm over the
-// row), the row statistic of k is taken along and *k_rms_done says so
+// row), the row statistic of k is taken along and *k_rms_done says so; so are n_clear words cleared that a later launch counts in
 static int quant_q_impl(const void* q, int dtype, const int64_t st[4], const ksana_sage_shape* s,
                         const ksana_sage_prep* prep, float sm_scale, void* ws, void* stream, const void* k,
-                        const int64_t k_st[4], bool* k_rms_done, uint16_t* pooled = nullptr) {
+                        const int64_t k_st[4], bool* k_rms_done, uint16_t* pooled = nullptr, int* clear = nullptr, int n_clear = 0) {
   const StageRange range("ksana_sage.quant_q");
   if (k_rms_done) *k_rms_done = false;
   if (int rc = check_shape(s)) return rc;
@@ -419,7 +419,7 @@ static int quant_q_impl(const void* q, int dtype, const int64_t st[4], const ksa
     hipError_t e = ksana_sage::launch_quant_q_rows(in_tensor(q, dtype, st, s->D), s->B, s->Hq, s->Lq, l.lq_pad, premul,
                                                    prep->norm_eps, ws_at<int8_t>(ws, l.q_i8), ws_at<float>(ws, l.q_scale),
                                                    static_cast<hipStream_t>(stream), *ppp, take_k ? &kt : nullptr,
-                                                   s->Hkv, s->Lk, ws_at<float>(ws, l.k_rms));
+                                                   s->Hkv, s->Lk, ws_at<float>(ws, l.k_rms), clear, take_k ? n_clear : 0);
     if (e != hipSuccess) return hip_fail(e, "quant_q (whole rows) launch");
     if (k_rms_done) *k_rms_done = take_k;
     return 0;
@@ -441,10 +441,12 @@ int ksana_sage_quant_k(const void* k, int dtype, const int64_t st[4], const ksan
 }
 
 // `part` == nullptr: the chunk sums and the counters go to the workspace's own k_part / k_sync areas
-// `rms_done`: the row statistic of k (k_rms area) has been taken by the call before (quant_q_impl)
+// `rms_done`: the row statistic of k (k_rms area) has been taken by the call before (quant_q_impl); `cleared`: and so have the
+// counters been cleared
 static int quant_k_impl(const void* k, int dtype, const int64_t st[4], const ksana_sage_shape* s,
                         const ksana_sage_prep* prep, int smooth_k, void* ws, float* part, int* sync_words,
-                        void* stream, bool rms_done = false, bool may_allocate = true, uint16_t* pooled = nullptr) {
+                        void* stream, bool rms_done = false, bool may_allocate = true, uint16_t* pooled = nullptr,
+                        bool cleared = false) {
   const StageRange range("ksana_sage.quant_k");
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_tensor("k", k, dtype, st, s->B, s->Lk, s->Hkv)) return rc;
@@ -469,7 +471,7 @@ static int quant_k_impl(const void* k, int dtype, const int64_t st[4], const ksa
   if ((one_read('k') || ppp != nullptr) && pooled == nullptr) {  // (block averages ride in the two-pass kernel)
     // one read of K: chunk sums, the head's mean and the quantization in one kernel, when the shape suits it (always
     // tried when the step before attention is applied on the way in: the rotation is then done once, not twice)
-    e = ksana_sage::launch_clear_ints(sync_words, ksana_sage::sync_words(bhk), hs);
+    if (!cleared) e = ksana_sage::launch_clear_ints(sync_words, ksana_sage::sync_words(bhk), hs);
     if (e != hipSuccess) return hip_fail(e, "k counter clear launch");
     bool used = false;
     e = ksana_sage::launch_quant_k_fused(kt, s->B, s->Hkv, s->Lk, l.nkb, l.nch, smooth_k ? 1 : 0, part,
@@ -557,8 +559,17 @@ int ksana_sage_quant_v(const void* v, int dtype, const int64_t st[4], const ksan
   return ksana_sage_quant_v_smooth(v, dtype, st, s, 0, ws, stream);
 }
 
+static int quant_v_impl(const void* v, int dtype, const int64_t st[4], const ksana_sage_shape* s, int smooth_v,
+                        void* ws, void* stream, bool cleared);
+
 int ksana_sage_quant_v_smooth(const void* v, int dtype, const int64_t st[4], const ksana_sage_shape* s, int smooth_v,
                               void* ws, void* stream) {
+  return quant_v_impl(v, dtype, st, s, smooth_v, ws, stream, false);
+}
+
+// `cleared`: the counters are zero
+static int quant_v_impl(const void* v, int dtype, const int64_t st[4], const ksana_sage_shape* s, int smooth_v,
+                        void* ws, void* stream, bool cleared) {
   const StageRange range("ksana_sage.quant_v");
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_tensor("v", v, dtype, st, s->B, s->Lk, s->Hkv)) return rc;
@@ -573,7 +584,7 @@ int ksana_sage_quant_v_smooth(const void* v, int dtype, const int64_t st[4], con
   if (!smooth_v && one_read('v')) {
     // one read of V: column maxima, scales and the quantization in one kernel, when the shape suits it
     int* words = ws_at<int>(ws, l.v_sync);
-    e = ksana_sage::launch_clear_ints(words, ksana_sage::sync_words(bhk), hs);
+    if (!cleared) e = ksana_sage::launch_clear_ints(words, ksana_sage::sync_words(bhk), hs);
     if (e != hipSuccess) return hip_fail(e, "v counter clear launch");
     bool used = false;
     e = ksana_sage::launch_quant_v_fused(vt, s->B, s->Hkv, s->Lk, l.nkb, l.nch, ws_at<float>(ws, l.v_part),
@@ -904,6 +915,29 @@ int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtyp
     const hipError_t e = ksana_sage::launch_quant_qkv(c, ppq, ppk, static_cast<hipStream_t>(stream), &used);
     if (e != hipSuccess) return hip_fail(e, "q, k, v quantizer launch");
     if (used) return 0;
+  }
+  if (with_q && prep != nullptr && !smooth_v && one_read('v')) {
+    // a norm over the token row folded in: Q's kernel takes K's row statistic along and clears the counters of K's and V's
+    ksana_sage_ws_layout l;
+    ksana_sage_workspace_layout(s, &l);
+    const ksana_sage::QkvCall c = qkv_call(true, in_tensor(q, dtype, q_st, s->D), in_tensor(k, dtype, k_st, s->D),
+                                           in_tensor(v, dtype, v_st, s->D), s, l, sm_scale, smooth_k, ws);
+    bool k_rms_done = false, used = false;
+    if (int rc = quant_q_impl(q, dtype, q_st, s, prep, sm_scale, ws, stream, k, k_st, &k_rms_done, nullptr, c.sync.k_counter,
+                              (int)(c.sync.v_status - c.sync.k_counter) + ksana_sage::kSyncStride))
+      return rc;
+    if (k_rms_done) {
+      const StageRange range("ksana_sage.quant_kv");
+      ksana_sage::PrepParams pk;
+      const ksana_sage::PrepParams* ppk = nullptr;
+      if (int rc = make_prep(prep, prep->k_norm_weight, "k", k_st, s->B, s->Lk, s->D, ws_at<float>(ws, l.k_rms), &pk, &ppk)) return rc;
+      const hipError_t e = ksana_sage::launch_quant_kv_meet(c, *ppk, static_cast<hipStream_t>(stream), &used);
+      if (e != hipSuccess) return hip_fail(e, "k, v quantizer launch");
+    }
+    if (used) return 0;
+    if (int rc = quant_k_impl(k, dtype, k_st, s, prep, smooth_k, ws, nullptr, nullptr, stream, k_rms_done, true, nullptr, k_rms_done))
+      return rc;
+    return quant_v_impl(v, dtype, v_st, s, 0, ws, stream, k_rms_done);
   }
   if (!with_q) {
     if (int rc = ksana_sage_quant_k(k, dtype, k_st, s, smooth_k, ws, stream)) return rc;

@@ -78,11 +78,12 @@ hipError_t launch_v_scale_finalize(const float* part, int BH, int nch, float* v_
 hipError_t launch_quant_q(const InTensor& q, int B, int H, int L, int lq_pad, float premul, int8_t* q_i8,
                           float* q_scale, hipStream_t s, const PrepParams* prep = nullptr, uint16_t* pooled = nullptr);
 // Q with a token-row norm (prep.inv_rms, prep.weight set; kinds 1 and 3): statistic and quantization from one pass over
-// HBM, 32 whole token rows per workgroup; writes prep.inv_rms as launch_row_inv_rms would.  k_rows != nullptr: the
-// statistic of rows [0, k_L) of that tensor (k_H heads of 128 channels, contiguous per row) goes to k_rms on the way.
+// HBM, whole token rows; writes prep.inv_rms as launch_row_inv_rms would.  k_rows != nullptr: the statistic of rows
+// [0, k_L) of that tensor (k_H heads of 128 channels, contiguous per row) goes to k_rms on the way.  n_clear words at
+// `clear` are set to zero.
 hipError_t launch_quant_q_rows(const InTensor& q, int B, int H, int L, int lq_pad, float premul, float eps,
                                int8_t* q_i8, float* q_scale, hipStream_t s, const PrepParams& prep,
-                               const InTensor* k_rows, int k_H, int k_L, float* k_rms);
+                               const InTensor* k_rows, int k_H, int k_L, float* k_rms, int* clear, int n_clear);
 hipError_t launch_quant_k(const InTensor& k, int B, int H, int L, int nkb, const float* k_mean, int8_t* k_tiles,
                           float* k_scale, hipStream_t s, const PrepParams* prep = nullptr, uint16_t* pooled = nullptr);
 // v_mean: nullptr, or the channel means taken off before scaling (V smoothing)
@@ -150,6 +151,9 @@ struct QkvCall {
   const int32_t *q_lens, *k_lens;
 };
 hipError_t launch_quant_qkv(const QkvCall& call, const PrepParams* pq, const PrepParams* pk, hipStream_t s, bool* used);
+
+// K with a step of kind 1 or 3 and V, both from one read, in one launch; c.sync is all zero before it
+hipError_t launch_quant_kv_meet(const QkvCall& c, const PrepParams& prep, hipStream_t s, bool* used);
 
 // One-read quantizers: *used == false means the shape does not suit them and nothing was launched.
 // `may_allocate`: see one_read_demoted.

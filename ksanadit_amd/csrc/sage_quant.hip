@@ -696,9 +696,12 @@ __global__ __launch_bounds__(kThreads) void quant_q_rows_kernel(const uint16_t* 
                                                                 int64_t sH, int H, int L, int lq_pad, float premul,
                                                                 float eps, int8_t* __restrict__ q_i8,
                                                                 float* __restrict__ q_scale, const PrepParams pp,
-                                                                float* __restrict__ rms_out, const RowStatOf ks) {
+                                                                float* __restrict__ rms_out, const RowStatOf ks,
+                                                                int* __restrict__ clear, int n_clear) {
   const int r0 = blockIdx.x * kRowsQ, b = blockIdx.y;
   const int t = threadIdx.x, slot = t >> 3, c16 = t & 7;
+  if (b == 0)  // the counters of the launch that follows
+    for (int i = blockIdx.x * kThreads + t; i < n_clear; i += gridDim.x * kThreads) clear[i] = 0;
   const int wave = t >> 6, lane = t & 63;
   __shared__ float s_rms[kRowsQ];
   // ---- the rows' statistics: wave w takes rows 2 w and 2 w + 1 together (every row's sum adds its groups of 8
@@ -1121,9 +1124,18 @@ __device__ __forceinline__ void stage_partials(const float (&v)[kFinLoads], floa
   for (int j = 0; j < kFinLoads; ++j) s_part[(int)threadIdx.x + kThreads * j] = v[j];
 }
 
+// The large LDS buffer of a chunk, one for K's and V's code where a kernel holds both (and asks for the same size)
+constexpr int kChunkLdsK = kFinStage * kD * 4, kChunkLdsV = 2 * kBlkK * (kD + 16);
+static_assert(kChunkLdsV >= kChunkLdsK, "V's is the size for both");
+template <int kBytes>
+__device__ __forceinline__ uint8_t* chunk_lds() {
+  __shared__ __attribute__((aligned(16))) uint8_t s[kBytes];
+  return s;
+}
+
 // SOLO: the head is this one chunk (at most 256 rows), so its sums are the head's and nobody is waited for.
 // n_use: the head's tiles that are wanted, at most nkb; a chunk without any leaves once its sums are counted in.
-template <int DT, int PRE, bool SOLO>
+template <int DT, int PRE, bool SOLO, int kBytes = kChunkLdsV>
 __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __restrict__ k, int64_t sB, int64_t sL,
                                               int64_t sH, int H, int L_all, int d_in, int nkb, int nch,
                                               float* __restrict__ part, float* k_mean, int dtype, int smooth,
@@ -1139,7 +1151,7 @@ __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __
   __shared__ float s_mean[kD];
   __shared__ float s_red[4][4];
   __shared__ int s_last;
-  __shared__ float s_part[kFinStage * kD];
+  float* s_part = reinterpret_cast<float*>(chunk_lds<kBytes>());
 
   // ---- 1. the chunk, and its column sums in the specified order -------------------------------
   // every load of the chunk goes out first (the rows stay in registers as 16-bit values until the end anyway): 16 KiB
@@ -1334,7 +1346,7 @@ __global__ __launch_bounds__(kThreads, PRE == 1 ? 3 : 1) void quant_k_fused_kern
                                                                  float* __restrict__ k_scale, const PrepParams pp,
                                                                  const HeadSync sy) {
   const int bh = blockIdx.x / nch;
-  quant_k_chunk<DT, PRE, false>(bh, blockIdx.x - bh * nch, k, sB, sL, sH, H, L_all, d_in, nkb, nch, part, k_mean, dtype, smooth,
+  quant_k_chunk<DT, PRE, false, kChunkLdsK>(bh, blockIdx.x - bh * nch, k, sB, sL, sH, H, L_all, d_in, nkb, nch, part, k_mean, dtype, smooth,
                                 k_tiles, k_scale, pp, sy, nkb);
 }
 
@@ -1356,7 +1368,7 @@ __device__ __forceinline__ void quant_v_chunk(int bh, int ch, const uint16_t* __
   __shared__ float s_inv[kD];
   __shared__ int s_last;
   constexpr int kStride = kD + 16;  // LDS row pitch in bytes
-  __shared__ __attribute__((aligned(16))) uint8_t s_v[2][kBlkK * kStride];
+  uint8_t(*s_v)[kBlkK * kStride] = reinterpret_cast<uint8_t(*)[kBlkK * kStride]>(chunk_lds<kChunkLdsV>());
 
   uint4 raw[kChunkRowsPerSlot][2];
   float acc[16];
@@ -1530,6 +1542,19 @@ __global__ __launch_bounds__(kThreads) void quant_v_fused_kernel(const uint16_t*
   const int bh = blockIdx.x / nch;
   quant_v_chunk<DT, false>(bh, blockIdx.x - bh * nch, v, sB, sL, sH, H, L_all, d_in, nkb, nch, part, v_scale, v_inv, v_mean, v_tiles,
                            sy, nkb);
+}
+
+// K with a step folded in and V in one launch: a head's V chunks are neighbours of its K chunks.  What that saves is a launch;
+// the two do not run faster together (see kKvMeetMax).
+template <int DT, int PRE>
+__global__ __launch_bounds__(kThreads, 3) void quant_kv_meet_kernel(const QkvCall c, const PrepParams pp, const HeadSync sk, const HeadSync sv) {
+  const int bh = blockIdx.x / (2 * c.nch), item = blockIdx.x - bh * 2 * c.nch;
+  if (item < c.nch)
+    quant_k_chunk<DT, PRE, false>(bh, item, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.nkb, c.nch, c.k_part, c.k_mean,
+                                  c.k.dtype, c.smooth_k, c.k_tiles, c.k_scale, pp, sk, c.nkb);
+  else
+    quant_v_chunk<DT, false>(bh, item - c.nch, c.v.ptr, c.v.sB, c.v.sL, c.v.sH, c.Hkv, c.Lk, c.v.D, c.nkb, c.nch, c.v_part, c.v_scale,
+                             c.v_inv, c.v_mean, c.v_tiles, sv, c.nkb);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2113,7 +2138,7 @@ hipError_t launch_quant_q(const InTensor& q, int B, int H, int L, int lq_pad, fl
 
 hipError_t launch_quant_q_rows(const InTensor& q, int B, int H, int L, int lq_pad, float premul, float eps,
                                int8_t* q_i8, float* q_scale, hipStream_t s, const PrepParams& prep,
-                               const InTensor* k_rows, int k_H, int k_L, float* k_rms) {
+                               const InTensor* k_rows, int k_H, int k_L, float* k_rms, int* clear, int n_clear) {
   RowStatOf ks{};
   if (k_rows != nullptr)
     ks = RowStatOf{k_rows->ptr, k_rows->sB, k_rows->sL, k_L, k_H * (kD / 8), (float)(k_H * kD), k_rms};
@@ -2124,9 +2149,9 @@ hipError_t launch_quant_q_rows(const InTensor& q, int B, int H, int L, int lq_pa
   const size_t lds = 0;  // the rotation factors of a token are held in registers across its heads: nothing is staged
   KSANA_DISPATCH_DT(q.dtype, {
     if (pp.kind == 3)
-      quant_q_rows_kernel<DT, 3><<<grid, block, lds, s>>>(q.ptr, q.sB, q.sL, q.sH, H, L, lq_pad, premul, eps, q_i8, q_scale, pp, rms_out, ks);
+      quant_q_rows_kernel<DT, 3><<<grid, block, lds, s>>>(q.ptr, q.sB, q.sL, q.sH, H, L, lq_pad, premul, eps, q_i8, q_scale, pp, rms_out, ks, clear, n_clear);
     else
-      quant_q_rows_kernel<DT, 1><<<grid, block, lds, s>>>(q.ptr, q.sB, q.sL, q.sH, H, L, lq_pad, premul, eps, q_i8, q_scale, pp, rms_out, ks);
+      quant_q_rows_kernel<DT, 1><<<grid, block, lds, s>>>(q.ptr, q.sB, q.sL, q.sH, H, L, lq_pad, premul, eps, q_i8, q_scale, pp, rms_out, ks, clear, n_clear);
   });
   return hipGetLastError();
 }
@@ -2352,6 +2377,32 @@ hipError_t launch_quant_k_fused(const InTensor& k, int B, int H, int L, int nkb,
   });
   if (*used) e = hipGetLastError();
   return e;
+}
+
+// us, K's and V's launch / one for both, up to here: 12 heads of 9792 tokens 51 / 48, 2 x 24 of 7200 122 / 121, 24 of 27280 (5136
+// workgroups) 251 / 249, and the gap between two launches, 3 us; beyond: 12 heads of 74400 380 / 390, 40 of 32760 413 / 428.
+constexpr int64_t kKvMeetMax = 5200;
+
+hipError_t launch_quant_kv_meet(const QkvCall& c, const PrepParams& prep, hipStream_t s, bool* used) {
+  *used = false;
+  const int64_t grid = 2 * (int64_t)c.B * c.Hkv * c.nch;
+  if (grid > kKvMeetMax || (prep.kind != 1 && prep.kind != 3) || one_read_demoted()) return hipSuccess;
+  const QuantSync& y = c.sync;
+  const long long ticks = quant_options().wait_ticks;
+  int* host = host_word(false).dev;
+  const HeadSync sk{y.k_counter, y.k_ready, y.k_status, ticks, host}, sv{y.v_counter, y.v_ready, y.v_status, ticks, host};
+  PrepParams pp = prep;
+  const size_t lds = plan_rope_lds(&pp, c.B, kMeanChunk);
+  auto go = [&](auto kernel) {
+    if (2 * c.nch > resident_workgroups(kernel, lds)) return;
+    kernel<<<dim3((unsigned)grid), dim3(kThreads), lds, s>>>(c, pp, sk, sv);
+    *used = true;
+  };
+  KSANA_DISPATCH_DT(c.k.dtype, {
+    if (pp.kind == 1) go(quant_kv_meet_kernel<DT, 1>);
+    else go(quant_kv_meet_kernel<DT, 3>);
+  });
+  return *used ? hipGetLastError() : hipSuccess;
 }
 
 hipError_t launch_quant_v_fused(const InTensor& v, int B, int H, int L, int nkb, int nch, float* part, float* v_scale,

@@ -98,6 +98,24 @@ def test_together_with_the_joint_block_step_at_192_mb(hip_device, img):
     _compare(hip_device, B, txt + img, txt + img, H, H, 128, torch.bfloat16, True, prep)
 
 
+# K and V in one launch, K of several chunks and of one, other numbers of keys and heads; 5760 workgroups: a launch each, their
+# counters cleared by Q's; no norm of k or of q: K's statistic is not there yet, or Q's kernel is another one
+@pytest.mark.parametrize("B,Lq,Lk,Hq,Hkv,norm,rotation", [
+    (1, 300, 300, 12, 12, "qk", "wan"), (2, 1000, 1000, 3, 3, "qk", "comfy"), (2, 200, 520, 4, 4, "qk", None), (1, 520, 70, 8, 4, "qk", None),
+    (1, 15360, 15360, 48, 48, "qk", "wan"), (1, 640, 640, 4, 4, "q", "wan"), (1, 640, 640, 4, 4, "k", "wan")])
+def test_the_row_norm_step_in_whole_calls(hip_device, B, Lq, Lk, Hq, Hkv, norm, rotation):
+    print(f"case B={B} Lq={Lq} Lk={Lk} Hq={Hq} Hkv={Hkv} {norm} {rotation}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(Lk)
+    wq, wk = (1.0 + 0.2 * torch.randn(h * 128, generator=g, device=hip_device) if n in norm else None for n, h in (("q", Hq), ("k", Hkv)))
+    kw = {}
+    if rotation == "wan":
+        ang = torch.rand((1024, 64), generator=g, device=hip_device, dtype=torch.float64) * 6.0
+        kw = dict(freqs=torch.polar(torch.ones_like(ang), ang), grid_sizes=[(Lq // 20, 4, 5)] * B)
+    if rotation == "comfy":
+        kw = dict(comfy_freqs=torch.randn((Lq - 7, 64, 2, 2), generator=g, device=hip_device))
+    _compare(hip_device, B, Lq, Lk, Hq, Hkv, 128, torch.bfloat16, True, sage_ops.WanPrep(wq, wk, 1e-6, **kw))
+
+
 def _inputs(hip_device, B, Lk, Hq, Hkv, D, dtype):
     g = torch.Generator(device=hip_device).manual_seed(Lk + D)
     k = torch.randn((B, Lk, Hkv, D), generator=g, device=hip_device) + 2.0 * torch.randn((Hkv, D), generator=g, device=hip_device)
