@@ -61,7 +61,7 @@ struct WgShape {
 };
 constexpr int kSparseMaxKeyTiles4 = 2048;    // 4-wave workgroups keep their tile list as 16-bit entries so that two fit a compute unit
 constexpr int kMaxKeyTiles = 4096;           // K scales of one head are kept in LDS: Lk <= 262144
-constexpr int kShortKeyTiles = 16;           // calls with at most this many key tiles (Lk <= 1024) are never cut into runs of keys
+constexpr int kShortKeyTiles = 16;           // with at most this many key tiles (Lk <= 1024) nobody's keys are cut into runs
 constexpr int kShortMaxKeyTiles = 2048;      // the most key tiles a dense 4-wave workgroup can hold scales for
 
 #pragma clang diagnostic push
@@ -169,16 +169,21 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform by construction: keep it scalar
   const int l32 = lane & 31, hh = lane >> 5;
-  const int q0 = qwg * kRowsWg + wave * 32;
   // query rows [0, lq) of this batch take part: all of them, or the caller's per-batch count; the rows from lq up
   // to Lq exist in the output and are written as zeros
   int lq = p.Lq;
   if (p.q_lens != nullptr) lq = min(max(p.q_lens[b], 0), p.Lq);  // uniform: a scalar load
-  const bool active = q0 < lq;  // wave-uniform; inactive waves only help move tiles
-
   // keys [0, lk) of this batch take part: all of them, or the caller's per-batch count
   int lk = p.Lk;
   if (p.k_lens != nullptr) lk = min(max(p.k_lens[b], 0), p.Lk);  // uniform: a scalar load
+  // A last block of at most 32 rows has work for one wave.  Alone on its unit that wave takes half a microsecond a step, next to
+  // another workgroup as long as the whole blocks do; so its four waves share the keys out instead (see below).
+  constexpr bool kCanShare = !kSparse && !kCausal && kW == 4 && !kPwlExp && !kTileSkip;
+  const bool shared =
+      kCanShare && __builtin_amdgcn_readfirstlane(p.wg_waves == 0 && lq > qwg * kRowsWg && lq - qwg * kRowsWg <= 32 &&
+                                                  lk > kShortKeyTiles * kBlkK) != 0;
+  const int q0 = qwg * kRowsWg + (shared ? 0 : wave * 32);
+  const bool active = q0 < lq;  // wave-uniform; inactive waves only help move tiles
   auto write_zero_rows = [&]() {  // softmax over no key: the output rows are defined as zeros
     const int q = q0 + l32;
     if (q < p.Lq && 64 * hh < p.d_out) {
@@ -221,7 +226,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // (not with a block mask: there such calls' key loops ran 1 % slower for the code being there; and out of the way of the
   // calls that do not take it: 12 workgroups of 10 tiles 23.9 us with it in line, 23.0 without)
   constexpr bool kOwnQ = !kSparse || kCausal;
-  const bool own_q = __builtin_expect(kOwnQ && active && p.q_rows.ptr != nullptr, 0);  // uniform per wave
+  const bool own_q = __builtin_expect(kOwnQ && active && !shared && p.q_rows.ptr != nullptr, 0);  // uniform per wave
 #pragma unroll
   for (int s = 0; s < 4; ++s) qf[s] = v4i{0, 0, 0, 0};
   if (own_q) {
@@ -236,7 +241,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         q_raw[2 * s + 1] = *reinterpret_cast<const uint4*>(qrow + 32 * s + 8);
       }
     }
-  } else if (active) {
+  } else if (active && !(shared && p.q_rows.ptr != nullptr)) {
     const int8_t* qrow = p.q_i8 + ((int64_t)bh * p.lq_pad + q0 + l32) * kD + 16 * hh;
 #pragma unroll
     for (int s = 0; s < kG; ++s) qf[s] = *reinterpret_cast<const v4i*>(qrow + 32 * s);
@@ -370,6 +375,148 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     }
     if (tid < 2 * kD) s_vs[tid] = vsm;
   };
+  if constexpr (kCanShare) {
+    if (shared) {
+      // Wave w takes the w-th run of ceil(tiles / 4) key tiles, its operands straight from the L2 into registers (V under
+      // the softmax, the next tile's K under the product with V), with reference points of its own; the four results are put together as the merge kernel does it, through LDS.  Bound by its chain of steps, a
+      // quarter as long.  us per call, whole / shared: 40 heads of 1560 tokens, where eight of the 520 workgroups start when the
+      // others end, 67.9 / 56.8.  Errors against 64 bits are those of whole rows or below: 0.0383 / 0.0388 at N(0, 1),
+      // 0.0289 / 0.0295 with outliers.
+      if (p.q_rows.ptr != nullptr) {
+        uint4 raw[8];
+        const uint16_t* qrow = p.q_rows.ptr + b * p.q_rows.sB + (int64_t)min(q0 + l32, p.Lq - 1) * p.q_rows.sL + h * p.q_rows.sH + 16 * hh;
+#pragma unroll
+        for (int i = 0; i < 2 * kG; ++i) {
+          raw[i] = *reinterpret_cast<const uint4*>(qrow + 32 * (i >> 1) + 8 * (i & 1));
+          if (q0 + l32 >= lq) raw[i] = make_uint4(0, 0, 0, 0);
+        }
+        quant_q_rows<DT, kG>(raw, p.q_premul, qf, qs);
+      }
+      fill_scales();
+      __syncthreads();
+      const int per = (nkb + kW - 1) / kW, j0 = min(wave * per, nkb), j1 = min(j0 + per, nkb);
+      const uint8_t* kt = k_src + lane * 16;
+      const uint8_t* vt = v_src + lane * 16;
+      v4i kf[2 * kG];  // (sub-tile t, channel step s) at t * kG + s
+      auto fetch_k = [&](int j) {
+#pragma unroll
+        for (int i = 0; i < 2 * kG; ++i)
+          kf[i] = *reinterpret_cast<const v4i*>(kt + (int64_t)j * kTileBytes + ((i / kG) * 4 + i % kG) * 1024);
+      };
+      if (j0 < j1) fetch_k(j0);
+#pragma unroll 1
+      for (int j = j0; j < j1; ++j) {
+        v16i s[2] = {magic, magic};
+#pragma unroll
+        for (int c = 0; c < kG; ++c)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) s[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[u * kG + c], qf[c], s[u], 0, 0, 0);
+        v8i vf[kG];
+#pragma unroll
+        for (int dt = 0; dt < kG; ++dt) {
+          const v4i lo = *reinterpret_cast<const v4i*>(vt + (int64_t)j * kTileBytes + (2 * dt + 0) * 1024);
+          const v4i hi = *reinterpret_cast<const v4i*>(vt + (int64_t)j * kTileBytes + (2 * dt + 1) * 1024);
+          vf[dt] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        }
+        const int n_last = j == nkb - 1 ? lk & (kBlkK - 1) : 0;  // (uniform) keys of a ragged tile
+        if (n_last != 0) blank_scores<kMagicBits>(s, hh, n_last);
+        int top = max(s[0][0], s[1][0]);
+#pragma unroll
+        for (int r = 1; r < 16; ++r) top = max(max(top, s[0][r]), s[1][r]);
+        const auto sw = __builtin_amdgcn_permlane32_swap(top, top, false, false);
+        top = max((int)sw[0], (int)sw[1]);
+        float sc = qs * s_ks[j], mneg = -kMagicVal * sc;
+        const float m_tile = __builtin_fmaf(__int_as_float(top), sc, mneg);
+        const bool nan = m_tile != m_tile;  // a row whose scores are not numbers becomes NaN and goes on with zero scores
+        const float m_new = nan ? 0.0f : (m_tile > x_limit ? m_tile : m_run);
+        const float alpha = fast_exp2((nan ? m_tile : m_run) - m_new);
+        sc = nan ? 0.0f : sc;
+        mneg = nan ? 0.0f : mneg;
+        qs = nan ? 0.0f : qs;
+        m_run = m_new;
+        x_limit = m_new + kLazyMax;
+        x_base = kPShift - m_new;
+        if (j == j0 ? __any(alpha != alpha) : __any(alpha != 1.0f)) {
+#pragma unroll
+          for (int dt = 0; dt < kG; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
+          lacc[0] *= alpha;
+        }
+        const float xc = x_base + mneg;
+        v8i pf;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+          float e[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) e[i] = fast_exp2(__builtin_fmaf(__int_as_float(s[w >> 2][4 * (w & 3) + i]), sc, xc));
+          int code = __builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], __float_as_int(e[0]), false);
+          pf[w] = __builtin_amdgcn_cvt_pk_fp8_f32(e[2], e[3], code, true);
+        }
+        if (n_last != 0) blank_probs(pf, hh, n_last);
+        fetch_k(min(j + 1, nkb - 1));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int dt = 0; dt < kG; ++dt) oacc[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf[dt], pf, oacc[dt], 0, 0, 0, 0, 0, 0);
+        lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, lacc, 0, 0, 0, 0, 0, 0);
+      }
+      // every wave's accumulators in the ring, points and sums where the K scales were; wave w then finishes channels 32 w ..
+      float* s_o = reinterpret_cast<float*>(smem);
+      float2* s_ml = reinterpret_cast<float2*>(s_ks);
+      __syncthreads();
+#pragma unroll
+      for (int dt = 0; dt < kG; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s_o[((wave * 4 + dt) * 16 + r) * 64 + lane] = oacc[dt][r];
+      if (hh == 0) s_ml[wave * 32 + l32] = make_float2(m_run, lacc[0]);
+      __syncthreads();
+      if (wave >= kG) __builtin_amdgcn_endpgm();
+      float2 ml[kW];
+      float m = -INFINITY, l = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kW; ++i) {
+        ml[i] = s_ml[i * 32 + l32];
+        m = fmaxf(m, ml[i].x);
+      }
+      float o[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[r] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kW; ++i) {
+        if (i * per >= nkb) continue;  // (uniform) a run without tiles
+        const float w = fast_exp2(ml[i].x - m);
+        l += ml[i].y * w;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[r] += s_o[((i * 4 + wave) * 16 + r) * 64 + lane] * w;
+      }
+      const int row = q0 + l32;
+      const float inv_l = row < lq ? 1.0f / l : 0.0f, keep_mean = inv_l != 0.0f ? 1.0f : 0.0f;
+      uint16_t* orow = p.o.ptr + b * p.o.sB + (int64_t)row * p.o.sL + h * p.o.sH + 32 * wave + 8 * hh;
+#pragma unroll
+      for (int g = 0; g < 4; g += 2) {
+        uint2 w[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int r = 4 * (g + e), d = 32 * wave + 8 * (g + e) + 4 * hh;
+          const float4 s4 = *reinterpret_cast<const float4*>(s_vs + d), m4 = *reinterpret_cast<const float4*>(s_vs + kD + d);
+          w[e] = half4<DT>(o[r] * inv_l * s4.x + m4.x * keep_mean, o[r + 1] * inv_l * s4.y + m4.y * keep_mean,
+                           o[r + 2] * inv_l * s4.z + m4.z * keep_mean, o[r + 3] * inv_l * s4.w + m4.w * keep_mean);
+        }
+        // lanes l and l + 32 trade every second four channels, so that each stores eight in a row
+        const auto x = __builtin_amdgcn_permlane32_swap(w[0].x, w[1].x, false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(w[0].y, w[1].y, false, false);
+        if (row < p.Lq) *reinterpret_cast<uint4*>(orow + 8 * g) = make_uint4(x[0], y[0], x[1], y[1]);
+      }
+      // rows [lq, Lq) of the block's other three quarters, if any, are zeros
+#pragma unroll
+      for (int i = 1; i < kW; ++i)
+        if (row + 32 * i < p.Lq) {
+          uint4* z = reinterpret_cast<uint4*>(p.o.ptr + b * p.o.sB + (int64_t)(row + 32 * i) * p.o.sL + h * p.o.sH + 32 * wave + 16 * hh);
+          z[0] = z[1] = make_uint4(0, 0, 0, 0);
+        }
+      __builtin_amdgcn_endpgm();
+    }
+  }
   // Causal calls: the list is in key order, so the entries this wave takes part in (tile <= the one on its diagonal)
   // are the first n_mine, and the diagonal tile, if listed, is the last of them.  Both are found once here; the key
   // loop then compares loop positions instead of looking list entries up.

@@ -188,3 +188,30 @@ def test_a_workgroup_with_waves_that_have_no_rows(hip_device, rows, Lk):
         four = sage_ops.attn_fwd(ws, torch.empty_like(q), wg_waves=4)
         eight = sage_ops.attn_fwd(ws, torch.empty_like(q), wg_waves=8)
         assert torch.equal(four, eight)
+
+
+@pytest.mark.parametrize("rows,Lk,D,dtype", [(1, 1025, 128, torch.bfloat16), (24, 1560, 128, torch.float16), (32, 64 * 20, 128, torch.bfloat16),
+                                             (17, 1100, 64, torch.float16), (32, 64 * 17, 64, torch.bfloat16), (9, 2049, 128, torch.bfloat16)])
+@pytest.mark.parametrize("whole_call", [False, True])
+def test_a_last_block_whose_waves_share_the_keys(hip_device, rows, Lk, D, dtype, whole_call):
+    """A last block of up to 32 rows: its four waves take a quarter of the key tiles each, like key runs; the blocks before
+    it are whole.  Numbers of tiles that four does and does not divide, ragged last tiles, the first tile of a run the ragged one."""
+    H, Lq = 60, 128 * 2 + rows  # 120 blocks of 256 rows: the plan takes 4-wave workgroups
+    print(f"case rows={rows} Lk={Lk} D={D} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(Lk)
+    q, k, v = (torch.randn((1, n, H, D), generator=g).to(dtype) for n in (Lq, Lk, Lk))
+    q[0, -1, 1] = float("inf")
+    qd, kd, vd = (t.to(hip_device) for t in (q, k, v))
+    ws = sage_ops.workspace_for(qd, kd)
+    assert sage_ops.key_split_plan(ws) is None
+    sage_ops.quant_q(qd, ws, D**-0.5), sage_ops.quant_k(kd, ws, True), sage_ops.quant_v(vd, ws)
+    out = (sage_ops.sageattn(qd, kd, vd) if whole_call else sage_ops.attn_fwd(ws, torch.empty_like(qd))).cpu()
+    four = sage_ops.attn_fwd(ws, torch.empty_like(qd), wg_waves=4).cpu()
+    assert torch.equal(out[:, :-rows], four[:, :-rows])
+    assert torch.equal(out.isnan(), four.isnan()) and out[0, -1, 1].isnan().any()
+    heads, last = slice(2, 4), slice(Lq - rows, Lq)
+    magic = {} if D == 128 else {"magic": 25165824.0}
+    want = sage_emul_from_quant(
+        ws.q_i8.cpu()[:, heads, last], ws.q_scale.cpu()[:, heads, last], untile_k(ws.k_tiles.cpu()[:, heads], Lk), ws.k_scale.cpu()[:, heads],
+        untile_v(ws.v_tiles.cpu()[:, heads], Lk).view(torch.float8_e4m3fn), ws.v_scale.cpu()[:, heads], dtype, key_split=(0, 4), **magic)
+    _close(out[:, last, heads], want[..., :D])
