@@ -176,13 +176,15 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // keys [0, lk) of this batch take part: all of them, or the caller's per-batch count
   int lk = p.Lk;
   if (p.k_lens != nullptr) lk = min(max(p.k_lens[b], 0), p.Lk);  // uniform: a scalar load
-  // A last block of at most 32 rows has work for one wave.  Alone on its unit that wave takes half a microsecond a step, next to
-  // another workgroup as long as the whole blocks do; so its four waves share the keys out instead (see below).
+  // A last block of at most 64 rows has work for one or two waves.  Alone on its unit such a workgroup takes half a microsecond a
+  // step, next to another one as long as the whole blocks do; so its four waves share the keys out instead (see below).
   constexpr bool kCanShare = !kSparse && !kCausal && kW == 4 && !kPwlExp && !kTileSkip;
-  const bool shared =
-      kCanShare && __builtin_amdgcn_readfirstlane(p.wg_waves == 0 && lq > qwg * kRowsWg && lq - qwg * kRowsWg <= 32 &&
-                                                  lk > kShortKeyTiles * kBlkK) != 0;
-  const int q0 = qwg * kRowsWg + (shared ? 0 : wave * 32);
+  // (by the rows the tensor has: a row's bits do not depend on its batch entry's count)
+  const int rows_here = p.Lq - qwg * kRowsWg;
+  const bool shared = kCanShare && __builtin_amdgcn_readfirstlane(p.wg_waves == 0 && rows_here <= 64 && lq > qwg * kRowsWg &&
+                                                                  lk > kShortKeyTiles * kBlkK) != 0;
+  const int sharers = rows_here > 32 ? 2 : 4;  // waves per 32 rows
+  const int q0 = qwg * kRowsWg + 32 * (shared ? wave / sharers : wave);
   const bool active = q0 < lq;  // wave-uniform; inactive waves only help move tiles
   auto write_zero_rows = [&]() {  // softmax over no key: the output rows are defined as zeros
     const int q = q0 + l32;
@@ -377,7 +379,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   };
   if constexpr (kCanShare) {
     if (shared) {
-      // Wave w takes the w-th run of ceil(tiles / 4) key tiles, its operands straight from the L2 into registers (V under
+      // A wave takes a run of ceil(tiles / sharers) key tiles, its operands straight from the L2 into registers (V under
       // the softmax, the next tile's K under the product with V), with reference points of its own; the four results are put together as the merge kernel does it, through LDS.  Bound by its chain of steps, a
       // quarter as long.  us per call, whole / shared: 40 heads of 1560 tokens, where eight of the 520 workgroups start when the
       // others end, 67.9 / 56.8.  Errors against 64 bits are those of whole rows or below: 0.0383 / 0.0388 at N(0, 1),
@@ -394,7 +396,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       }
       fill_scales();
       __syncthreads();
-      const int per = (nkb + kW - 1) / kW, j0 = min(wave * per, nkb), j1 = min(j0 + per, nkb);
+      const int per = (nkb + sharers - 1) / sharers, run = wave & (sharers - 1), j0 = min(run * per, nkb), j1 = min(j0 + per, nkb);
       const uint8_t* kt = k_src + lane * 16;
       const uint8_t* vt = v_src + lane * 16;
       v4i kf[2 * kG];  // (sub-tile t, channel step s) at t * kG + s
@@ -460,7 +462,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         for (int dt = 0; dt < kG; ++dt) oacc[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf[dt], pf, oacc[dt], 0, 0, 0, 0, 0, 0);
         lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, lacc, 0, 0, 0, 0, 0, 0);
       }
-      // every wave's accumulators in the ring, points and sums where the K scales were; wave w then finishes channels 32 w ..
+      // every wave's accumulators in the ring, points and sums where the K scales were; then the waves of a row group finish a
+      // quarter or half of its channels each
       float* s_o = reinterpret_cast<float*>(smem);
       float2* s_ml = reinterpret_cast<float2*>(s_ks);
       __syncthreads();
@@ -470,50 +473,52 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         for (int r = 0; r < 16; ++r) s_o[((wave * 4 + dt) * 16 + r) * 64 + lane] = oacc[dt][r];
       if (hh == 0) s_ml[wave * 32 + l32] = make_float2(m_run, lacc[0]);
       __syncthreads();
-      if (wave >= kG) __builtin_amdgcn_endpgm();
-      float2 ml[kW];
+      const int first = wave - run;  // the row group's first wave
+      float weight[kW];
       float m = -INFINITY, l = 0.0f;
 #pragma unroll
-      for (int i = 0; i < kW; ++i) {
-        ml[i] = s_ml[i * 32 + l32];
-        m = fmaxf(m, ml[i].x);
-      }
-      float o[16];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[r] = 0.0f;
+      for (int i = 0; i < kW; ++i)
+        if (i < sharers) m = fmaxf(m, s_ml[(first + i) * 32 + l32].x);
 #pragma unroll
       for (int i = 0; i < kW; ++i) {
-        if (i * per >= nkb) continue;  // (uniform) a run without tiles
-        const float w = fast_exp2(ml[i].x - m);
-        l += ml[i].y * w;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[r] += s_o[((i * 4 + wave) * 16 + r) * 64 + lane] * w;
+        weight[i] = 0.0f;
+        if (i < sharers && i * per < nkb) {  // (uniform) a run with tiles
+          const float2 ml = s_ml[(first + i) * 32 + l32];
+          weight[i] = fast_exp2(ml.x - m);
+          l += ml.y * weight[i];
+        }
       }
       const int row = q0 + l32;
-      const float inv_l = row < lq ? 1.0f / l : 0.0f, keep_mean = inv_l != 0.0f ? 1.0f : 0.0f;
-      uint16_t* orow = p.o.ptr + b * p.o.sB + (int64_t)row * p.o.sL + h * p.o.sH + 32 * wave + 8 * hh;
+      const float inv_l = 1.0f / l, keep_mean = inv_l != 0.0f ? 1.0f : 0.0f;
+#pragma unroll 1
+      for (int cg = run; cg < kG; cg += sharers) {
+        float o[16];
 #pragma unroll
-      for (int g = 0; g < 4; g += 2) {
-        uint2 w[2];
+        for (int r = 0; r < 16; ++r) o[r] = 0.0f;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const int r = 4 * (g + e), d = 32 * wave + 8 * (g + e) + 4 * hh;
-          const float4 s4 = *reinterpret_cast<const float4*>(s_vs + d), m4 = *reinterpret_cast<const float4*>(s_vs + kD + d);
-          w[e] = half4<DT>(o[r] * inv_l * s4.x + m4.x * keep_mean, o[r + 1] * inv_l * s4.y + m4.y * keep_mean,
-                           o[r + 2] * inv_l * s4.z + m4.z * keep_mean, o[r + 3] * inv_l * s4.w + m4.w * keep_mean);
+        for (int i = 0; i < kW; ++i) {
+          if (i >= sharers || i * per >= nkb) continue;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[r] += s_o[(((first + i) * 4 + cg) * 16 + r) * 64 + lane] * weight[i];
         }
-        // lanes l and l + 32 trade every second four channels, so that each stores eight in a row
-        const auto x = __builtin_amdgcn_permlane32_swap(w[0].x, w[1].x, false, false);
-        const auto y = __builtin_amdgcn_permlane32_swap(w[0].y, w[1].y, false, false);
-        if (row < p.Lq) *reinterpret_cast<uint4*>(orow + 8 * g) = make_uint4(x[0], y[0], x[1], y[1]);
+        uint16_t* orow = p.o.ptr + b * p.o.sB + (int64_t)row * p.o.sL + h * p.o.sH + 32 * cg + 8 * hh;
+#pragma unroll
+        for (int g = 0; g < 4; g += 2) {
+          uint2 w[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const int r = 4 * (g + e), d = 32 * cg + 8 * (g + e) + 4 * hh;
+            const float4 s4 = *reinterpret_cast<const float4*>(s_vs + d), m4 = *reinterpret_cast<const float4*>(s_vs + kD + d);
+            w[e] = half4<DT>(o[r] * inv_l * s4.x + m4.x * keep_mean, o[r + 1] * inv_l * s4.y + m4.y * keep_mean,
+                             o[r + 2] * inv_l * s4.z + m4.z * keep_mean, o[r + 3] * inv_l * s4.w + m4.w * keep_mean);
+            if (row >= lq) w[e] = make_uint2(0, 0);
+          }
+          // lanes l and l + 32 trade every second four channels, so that each stores eight in a row
+          const auto x = __builtin_amdgcn_permlane32_swap(w[0].x, w[1].x, false, false);
+          const auto y = __builtin_amdgcn_permlane32_swap(w[0].y, w[1].y, false, false);
+          if (row < p.Lq) *reinterpret_cast<uint4*>(orow + 8 * g) = make_uint4(x[0], y[0], x[1], y[1]);
+        }
       }
-      // rows [lq, Lq) of the block's other three quarters, if any, are zeros
-#pragma unroll
-      for (int i = 1; i < kW; ++i)
-        if (row + 32 * i < p.Lq) {
-          uint4* z = reinterpret_cast<uint4*>(p.o.ptr + b * p.o.sB + (int64_t)(row + 32 * i) * p.o.sL + h * p.o.sH + 32 * wave + 16 * hh);
-          z[0] = z[1] = make_uint4(0, 0, 0, 0);
-        }
       __builtin_amdgcn_endpgm();
     }
   }

@@ -191,11 +191,12 @@ def test_a_workgroup_with_waves_that_have_no_rows(hip_device, rows, Lk):
 
 
 @pytest.mark.parametrize("rows,Lk,D,dtype", [(1, 1025, 128, torch.bfloat16), (24, 1560, 128, torch.float16), (32, 64 * 20, 128, torch.bfloat16),
-                                             (17, 1100, 64, torch.float16), (32, 64 * 17, 64, torch.bfloat16), (9, 2049, 128, torch.bfloat16)])
+                                             (17, 1100, 64, torch.float16), (32, 64 * 17, 64, torch.bfloat16), (9, 2049, 128, torch.bfloat16),
+                                             (33, 1025, 128, torch.float16), (57, 64 * 18, 128, torch.bfloat16), (64, 1300, 64, torch.bfloat16)])
 @pytest.mark.parametrize("whole_call", [False, True])
 def test_a_last_block_whose_waves_share_the_keys(hip_device, rows, Lk, D, dtype, whole_call):
-    """A last block of up to 32 rows: its four waves take a quarter of the key tiles each, like key runs; the blocks before
-    it are whole.  Numbers of tiles that four does and does not divide, ragged last tiles, the first tile of a run the ragged one."""
+    """A last block of up to 32 or 64 rows: its waves take a quarter or half of the key tiles each, like key runs; the blocks
+    before it are whole.  Numbers of tiles that divide and do not, ragged last tiles, the first tile of a run the ragged one."""
     H, Lq = 60, 128 * 2 + rows  # 120 blocks of 256 rows: the plan takes 4-wave workgroups
     print(f"case rows={rows} Lk={Lk} D={D} {dtype}", flush=True)
     g = torch.Generator().manual_seed(Lk)
@@ -213,5 +214,25 @@ def test_a_last_block_whose_waves_share_the_keys(hip_device, rows, Lk, D, dtype,
     magic = {} if D == 128 else {"magic": 25165824.0}
     want = sage_emul_from_quant(
         ws.q_i8.cpu()[:, heads, last], ws.q_scale.cpu()[:, heads, last], untile_k(ws.k_tiles.cpu()[:, heads], Lk), ws.k_scale.cpu()[:, heads],
-        untile_v(ws.v_tiles.cpu()[:, heads], Lk).view(torch.float8_e4m3fn), ws.v_scale.cpu()[:, heads], dtype, key_split=(0, 4), **magic)
+        untile_v(ws.v_tiles.cpu()[:, heads], Lk).view(torch.float8_e4m3fn), ws.v_scale.cpu()[:, heads], dtype, key_split=(0, 4 if rows <= 32 else 2), **magic)
     _close(out[:, last, heads], want[..., :D])
+
+
+@pytest.mark.parametrize("k_len", [1100, 900])
+@pytest.mark.parametrize("rows", [57, 20])
+def test_a_shared_last_block_in_batches_with_lengths(hip_device, k_len, rows):
+    """Entries that end before, inside and with a last block whose waves share the keys (1100 of them; not 900): rows that
+    count have the bits they have without counts of rows, the others are zeros."""
+    B, H, Lq, Lk = 5, 16, 256 + rows, 1100
+    g = torch.Generator(device=hip_device).manual_seed(k_len)
+    q, k, v = (torch.randn((B, n, H, 128), generator=g, device=hip_device).half() for n in (Lq, Lk, Lk))
+    k_lens = torch.tensor([Lk, k_len, k_len, k_len, Lk], dtype=torch.int32, device=hip_device)
+    q_lens = [Lq, 257, 256 + rows // 2, 192, 0]
+    q[4, :] = float("nan")
+    for call in (lambda **kw: sage_ops.sageattn(q, k, v, k_lens=k_lens, **kw),
+                 lambda **kw: sage_ops.attn_fwd(ws, torch.empty_like(q).fill_(float("nan")), k_lens=k_lens, **kw)):
+        ws = sage_ops.workspace_for(q, k)
+        sage_ops.quant_q(q, ws, 128**-0.5), sage_ops.quant_k(k, ws, True), sage_ops.quant_v(v, ws)
+        out, full = call(q_lens=torch.tensor(q_lens, dtype=torch.int32, device=hip_device)), call()
+        for b, n in enumerate(q_lens):
+            assert torch.equal(out[b, :n], full[b, :n]) and not out[b, n:].isnan().any() and not out[b, n:].any(), b
