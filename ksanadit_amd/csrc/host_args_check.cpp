@@ -9,6 +9,15 @@
 #include <vector>
 
 #include "../../include/ksana_sage_hip.h"
+#include "sage_kernels.h"
+
+// Counts of batch entries are any int32, clamped to the tensor before anything is added to them.  As constant expressions: an
+// overflow on the way is an error of the build.
+static_assert(ksana_sage::tiles_counted(INT32_MAX, 5) == 5 && ksana_sage::tiles_counted(INT32_MAX - 63, 5) == 5);
+static_assert(ksana_sage::tiles_counted(321, 5) == 5 && ksana_sage::tiles_counted(257, 5) == 5 && ksana_sage::tiles_counted(256, 5) == 4);
+static_assert(ksana_sage::tiles_counted(1, 5) == 1 && ksana_sage::tiles_counted(0, 5) == 0);
+static_assert(ksana_sage::tiles_counted(-1, 5) == 0 && ksana_sage::tiles_counted(INT32_MIN, 5) == 0);
+static_assert(ksana_sage::rows_counted(INT32_MAX, 300) == 300 && ksana_sage::rows_counted(299, 300) == 299 && ksana_sage::rows_counted(INT32_MIN, 300) == 0);
 
 static int g_failed = 0;
 #define EXPECT(call, want)                                                                        \

@@ -172,10 +172,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // query rows [0, lq) of this batch take part: all of them, or the caller's per-batch count; the rows from lq up
   // to Lq exist in the output and are written as zeros
   int lq = p.Lq;
-  if (p.q_lens != nullptr) lq = min(max(p.q_lens[b], 0), p.Lq);  // uniform: a scalar load
+  if (p.q_lens != nullptr) lq = rows_counted(p.q_lens[b], p.Lq);  // uniform: a scalar load
   // keys [0, lk) of this batch take part: all of them, or the caller's per-batch count
   int lk = p.Lk;
-  if (p.k_lens != nullptr) lk = min(max(p.k_lens[b], 0), p.Lk);  // uniform: a scalar load
+  if (p.k_lens != nullptr) lk = rows_counted(p.k_lens[b], p.Lk);  // uniform: a scalar load
   // A last block of at most 64 rows has work for one or two waves.  Alone on its unit such a workgroup takes half a microsecond a
   // step, next to another one as long as the whole blocks do; so its four waves share the keys out instead (see below).
   constexpr bool kCanShare = !kSparse && !kCausal && kW == 4 && !kPwlExp && !kTileSkip;
@@ -1164,7 +1164,7 @@ __global__ __launch_bounds__(256) void sage_attn_merge_kernel(const AttnParams p
   const int q = qwg * kAttnQPerWg + row;
   if (q >= p.Lq || d >= p.d_out) return;
   uint16_t* orow = p.o.ptr + b * p.o.sB + (int64_t)q * p.o.sL + h * p.o.sH;
-  if (p.q_lens != nullptr && q >= min(max(p.q_lens[b], 0), p.Lq)) {  // a row that does not take part: zeros
+  if (p.q_lens != nullptr && q >= rows_counted(p.q_lens[b], p.Lq)) {  // a row that does not take part: zeros
     *reinterpret_cast<uint2*>(orow + d) = make_uint2(0, 0);
     return;
   }

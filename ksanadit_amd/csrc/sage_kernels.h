@@ -16,6 +16,17 @@ constexpr int kMeanChunk = 256;  // rows per partial column sum
 constexpr int kTileBytes = kBlkK * kD;  // one K (int8) or V^T (fp8) tile: 8192 bytes
 constexpr int kAttnQPerWg = 256; // query rows per attention workgroup (8 waves x 32)
 
+// The rows (or keys) that a caller's count of a batch entry stands for, of the `most` that the tensor has.  Any int32 may come
+// in: it is clamped before anything is added to it.
+__host__ __device__ constexpr int rows_counted(int count, int most) {
+  const int some = count < 0 ? 0 : count;
+  return some < most ? some : most;
+}
+// .. and the key tiles that hold them, of the tensor's
+__host__ __device__ constexpr int tiles_counted(int count, int tiles) {
+  return (int)(((unsigned)rows_counted(count, tiles * kBlkK) + kBlkK - 1) / kBlkK);
+}
+
 struct InTensor {
   const uint16_t* ptr;
   int64_t sB, sL, sH;  // element strides of [B, L, H, D]; D stride is 1

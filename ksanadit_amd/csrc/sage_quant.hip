@@ -1637,7 +1637,7 @@ __device__ __forceinline__ void clear_status(const QkvCall& c) {
 // falling off to 45 %: 6 x 24 heads of 520 rows on 10561 keys 456 / 420, of 16 of 1111 on 4311 190 / 178, 3 x 24 of 3001 on
 // 4099 195.4 / 193.1); their statistics are not, so the codes that are read stay the same.
 __device__ __forceinline__ int tiles_in_use(const QkvCall& c, int b) {
-  return c.k_lens == nullptr ? c.nkb : min(c.nkb, (max(c.k_lens[b], 0) + kBlkK - 1) / kBlkK);
+  return c.k_lens == nullptr ? c.nkb : tiles_counted(c.k_lens[b], c.nkb);
 }
 
 template <int DT, int KIND>

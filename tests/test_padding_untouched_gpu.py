@@ -26,3 +26,27 @@ def test_same_bits_as_with_everything_quantized(hip_device, B, Hq, Hkv, Lq, Lk, 
         got = sage_ops.sageattn(q, k, v, **kw)
         torch.empty_like(got).fill_(float("nan"))  # what the allocator hands out next is not a finished result
         assert torch.equal(got, sage_ops.attn_fwd(ws, torch.empty_like(q), **kw)), (k_lens, q_lens)
+
+
+INT_MAX, INT_MIN = 2**31 - 1, -(2**31)
+
+
+# (.. and the calls of one launch, and K and V of less than a tile)
+@pytest.mark.parametrize("B,Hq,Hkv,Lq,Lk", [(5, 4, 4, 100, 37), (5, 8, 4, 300, 230), (5, 64, 32, 900, 230), (5, 4, 2, 700, 1500), (5, 8, 8, 200, 17000)])
+def test_counts_of_any_value_are_clamped(hip_device, B, Hq, Hkv, Lq, Lk):
+    """A count is clamped to the tensor before anything is added to it: negative ones are none, those beyond the tensor all."""
+    print(f"case B={B} Hq={Hq} Lq={Lq} Lk={Lk}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(Lk)
+    q, k, v = (torch.randn((B, n, h, 128), generator=g, device=hip_device).bfloat16() for n, h in ((Lq, Hq), (Lk, Hkv), (Lk, Hkv)))
+    ws = sage_ops.workspace_for(q, k)
+    sage_ops.quant_q(q, ws, 128**-0.5), sage_ops.quant_k(k, ws, True), sage_ops.quant_v(v, ws)
+    for k_lens, q_lens in (([INT_MAX, INT_MAX - 62, INT_MAX - 63, Lk + 1, Lk - 1], [INT_MAX, Lq + 1, Lq - 1, INT_MAX - 62, 1]),
+                           ([-1, INT_MIN, -Lk, 1, INT_MAX], [Lq, Lq, Lq, INT_MIN, -1])):
+        within = [[max(0, min(n, most)) for n in lens] for lens, most in ((k_lens, Lk), (q_lens, Lq))]
+        as_given, clamped = ([torch.tensor(x, dtype=torch.int32, device=hip_device) for x in pair] for pair in ((k_lens, q_lens), within))
+        want = sage_ops.attn_fwd(ws, torch.empty_like(q), k_lens=clamped[0], q_lens=clamped[1])
+        for lens in (as_given, clamped):
+            assert torch.equal(sage_ops.sageattn(q, k, v, k_lens=lens[0], q_lens=lens[1]), want), (k_lens, q_lens)
+        assert torch.equal(sage_ops.attn_fwd(ws, torch.empty_like(q), k_lens=as_given[0], q_lens=as_given[1]), want), (k_lens, q_lens)
+        for b, (n_k, n_q) in enumerate(zip(*within)):
+            assert (want[b, n_q:] == 0).all() and (n_k > 0 or (want[b] == 0).all())
