@@ -1032,9 +1032,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // A lane holds its query row in pieces of four channels; stored as they are, every store instruction would
   // touch 32 rows with 16 bytes each.  The rows go through LDS instead (the tile ring is free once every wave is
   // past its last tile) and leave as whole 256-byte rows, 16 bytes per lane.
-  const int q = q0 + l32;
-  // zero for a mask row that allows none of its keys (an empty sum, not 0/0) and for rows at or beyond lq
-  const float inv_l = ((!(kSparse || kCausal) || lacc[0] > 0.0f) && q < lq) ? 1.0f / lacc[0] : 0.0f;
+  // zero for a mask row that allows none of its keys (an empty sum, not 0/0)
+  const float inv_l = !(kSparse || kCausal) || lacc[0] > 0.0f ? 1.0f / lacc[0] : 0.0f;
   // the channel means the V quantizer took off come back here (rows of P sum to one); they are zeros without V
   // smoothing, and a row that saw no key stays zero
   const float keep_mean = inv_l != 0.0f ? 1.0f : 0.0f;
@@ -1058,7 +1057,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     // As a pass of its own the branch reads q and the result and writes the result again, 1 GB at 32760 rows of 40 heads,
     // bound by memory; here its arithmetic runs beside the neighbour workgroup's key loop.  us per call, a tenth of the keys
     // kept, pass of its own / here: 40 heads of 32760 rows 2000 / 1859, of 6867 272 / 230, 12 of 2000 72 / 52.
-    const uint16_t* lrow = p.q_rows.ptr + b * p.q_rows.sB + (int64_t)min(q, p.Lq - 1) * p.q_rows.sL + h * p.q_rows.sH + 8 * hh;
+    const uint16_t* lrow = p.q_rows.ptr + b * p.q_rows.sB + (int64_t)min(q0 + l32, p.Lq - 1) * p.q_rows.sL + h * p.q_rows.sH + 8 * hh;
     uint4 lraw[8];
 #pragma unroll
     for (int s = 0; s < 8; ++s) lraw[s] = *reinterpret_cast<const uint4*>(lrow + 16 * s);
@@ -1139,6 +1138,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
             half4<DT>(oacc[dt][4 * g + 0] * inv_l * s4.x + m4.x * keep_mean, oacc[dt][4 * g + 1] * inv_l * s4.y + m4.y * keep_mean,
                       oacc[dt][4 * g + 2] * inv_l * s4.z + m4.z * keep_mean, oacc[dt][4 * g + 3] * inv_l * s4.w + m4.w * keep_mean);
       }
+    }
+    // rows at or beyond lq (zeros put in their place and not a factor of zero: what q holds there, or v, need not be finite)
+    if (q0 + 32 > lq && q0 + l32 >= lq) {
+#pragma unroll
+      for (int i = 0; i < 2 * kG; ++i) *reinterpret_cast<uint4*>(stage + l32 * kPitch + 32 * i + 16 * hh) = make_uint4(0, 0, 0, 0);
     }
   }
   // LDS serves one wave's accesses in order: the reads below see the writes above

@@ -338,7 +338,7 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c,
 
   // ---- O = O^T / rowsum * v_scale, whole rows out through LDS -----------------------------------------
   // (a dense row always has a sum; causal rows: as the general kernel has it)
-  const float inv_l = ((!c.causal || lacc[0] > 0.0f) && row < lq) ? 1.0f / lacc[0] : 0.0f;
+  const float inv_l = !c.causal || lacc[0] > 0.0f ? 1.0f / lacc[0] : 0.0f;
   float4 s4[16];
 #pragma unroll
   for (int i = 0; i < 4 * kG; ++i) s4[i] = reinterpret_cast<const float4*>(s_vs)[(32 * (i >> 2) + 8 * (i & 3) + 4 * hh) >> 2];
@@ -357,6 +357,16 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c,
     const int idx = i * 64 + lane, r = idx >> 4, piece = idx & 15;
     const uint4 w = *reinterpret_cast<const uint4*>(stage + r * kOutPitch + 16 * piece);
     if (q0 + r < c.Lq && 8 * piece < c.d_out && 8 * piece < 32 * kG) *reinterpret_cast<uint4*>(obase + (int64_t)(q0 + r) * c.o.sL + 8 * piece) = w;
+  }
+  // Rows that do not count become zeros, whatever their q, or v, holds.  (By the threads that have just written them and not
+  // in their stead: a branch ahead of the stores holds up the last instructions of every call, 9.9 -> 10.1 us at 32 tokens.)
+  if (q0 + 32 > lq) {
+#pragma unroll 1
+    for (int i = 0; i < 8; ++i) {
+      const int idx = i * 64 + lane, r = idx >> 4, piece = idx & 15;
+      if (q0 + r >= lq && q0 + r < c.Lq && 8 * piece < c.d_out)
+        *reinterpret_cast<uint4*>(obase + (int64_t)(q0 + r) * c.o.sL + 8 * piece) = make_uint4(0, 0, 0, 0);
+    }
   }
 }
 

@@ -1,4 +1,4 @@
-"""Batches with lengths of their own, workspace unseen: blocks of rows or keys that take no part are not quantized.  Against the
+"""Batches with lengths of their own: what takes no part.  Workspace unseen, blocks of such rows or keys are not quantized; against the
 stage-wise entry points, which quantize everything: the statistics are the same, so the results are the same bits."""
 
 import pytest
@@ -50,3 +50,40 @@ def test_counts_of_any_value_are_clamped(hip_device, B, Hq, Hkv, Lq, Lk):
         assert torch.equal(sage_ops.attn_fwd(ws, torch.empty_like(q), k_lens=as_given[0], q_lens=as_given[1]), want), (k_lens, q_lens)
         for b, (n_k, n_q) in enumerate(zip(*within)):
             assert (want[b, n_q:] == 0).all() and (n_k > 0 or (want[b] == 0).all())
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(is_causal=True), dict(mask=True), dict(mask=True, is_causal=True), dict(mask=True, wg_waves=8), dict(wg_waves=4),
+                                dict(wg_waves=8), dict(smooth_v=True), dict(pwl_exp2=True), dict(tile_skip=True)], ids=lambda kw: "-".join(map(str, kw)) or "plain")
+# (one launch; the attention kernel quantizes Q; Q quantized apart, keys in runs; a last block whose waves share the keys)
+@pytest.mark.parametrize("H,Lq,Lk,D", [(4, 100, 200, 128), (4, 100, 200, 64), (64, 400, 600, 128), (64, 400, 600, 64), (2, 600, 1100, 128), (16, 300, 1100, 128)])
+def test_rows_that_do_not_count_are_zeros_whatever_they_hold(hip_device, H, Lq, Lk, D, kw):
+    """Infinities and NaN in the padding rows of q, and infinite values: the rows that do not count are written as zeros, the
+    others as ever."""
+    print(f"case H={H} Lq={Lq} Lk={Lk} D={D} {kw}", flush=True)
+    kw = dict(kw)
+    g = torch.Generator(device=hip_device).manual_seed(Lq + D)
+    q, k, v = (torch.randn((3, n, H, D), generator=g, device=hip_device).bfloat16() for n in (Lq, Lk, Lk))
+    if kw.pop("mask", False):
+        kw["block_mask"] = (torch.rand((-(-Lq // 128), -(-Lk // 64)), generator=g, device=hip_device) < 0.6).to(torch.int8)
+        kw["block_mask"][:, 0] = 1
+    q_lens = [Lq, Lq - 5, 33]
+    kw["q_lens"] = torch.tensor(q_lens, dtype=torch.int32, device=hip_device)
+
+    def call():
+        if "wg_waves" not in kw:
+            return sage_ops.sageattn(q, k, v, **kw)
+        ws = sage_ops.workspace_for(q, k)
+        sage_ops.quant_q(q, ws, D**-0.5), sage_ops.quant_k(k, ws, True), sage_ops.quant_v(v, ws)
+        return sage_ops.attn_fwd(ws, torch.full_like(q, float("nan")), **kw)
+
+    want = call()
+    for b, n in enumerate(q_lens):
+        q[b, n:, 0], q[b, n:, 1, 3] = float("inf"), float("-inf")
+        q[b, n + 1 :: 3] = float("nan")
+    for _ in range(2):
+        got = call()
+        for b, n in enumerate(q_lens):
+            assert (got[b, n:] == 0).all(), f"entry {b}: {int((got[b, n:] != 0).sum())} values of the padding are not zero"
+            if want is not None:
+                assert torch.equal(got[b, :n], want[b, :n]), f"entry {b}: rows that count have changed"
+        v[:, Lk // 2, 0, 1], want = float("inf"), None
