@@ -182,8 +182,8 @@ const char* ksana_sage_last_error(void);
  *     to 64 chunks of 256 keys and 192 MB of K and V two launches read K and V twice whatever is set here, and nobody
  *     waits.  Beyond that, up to 160 chunks and without a folded step, "v" also selects one launch in which K's and
  *     V's chunks meet: both are then read once, with or without a "k".  With the Wan step and its norms of q and k,
- *     "v" also selects one launch for K's and V's one-read kernels up to 5200 chunks of 256 keys (K's and V's of all
- *     heads), and a launch each beyond.  Without "v", and for all other whole calls, the letters select the separate
+ *     "v" also selects one launch for K's and V's one-read kernels where the chip works through the chunks of 256 keys
+ *     (K's and V's of all heads) in less than 1.5 or in 2 to 7 rounds, and a launch each otherwise.  Without "v", and for all other whole calls, the letters select the separate
  *     kernels as for the stage-wise entry points.
  *   wait_ticks: KSANA_SAGE_KEEP = leave as it is; otherwise the bound, in 10 ns ticks, on a workgroup's wait for its
  *     head's statistic.  First value: KSANA_SAGE_WAIT_TICKS, default 200000 (2 ms; the kernels run 0.1 - 0.5 ms).

@@ -1545,7 +1545,7 @@ __global__ __launch_bounds__(kThreads) void quant_v_fused_kernel(const uint16_t*
 }
 
 // K with a step folded in and V in one launch: a head's V chunks are neighbours of its K chunks.  What that saves is a launch;
-// the two do not run faster together (see kKvMeetMax).
+// the two do not run faster together (see kv_in_one_launch_pays).
 template <int DT, int PRE>
 __global__ __launch_bounds__(kThreads, 3) void quant_kv_meet_kernel(const QkvCall c, const PrepParams pp, const HeadSync sk, const HeadSync sv) {
   const int bh = blockIdx.x / (2 * c.nch), item = blockIdx.x - bh * 2 * c.nch;
@@ -2379,14 +2379,23 @@ hipError_t launch_quant_k_fused(const InTensor& k, int B, int H, int L, int nkb,
   return e;
 }
 
-// us, K's and V's launch / one for both, up to here: 12 heads of 9792 tokens 51 / 48, 2 x 24 of 7200 122 / 121, 24 of 27280 (5136
-// workgroups) 251 / 249, and the gap between two launches, 3 us; beyond: 12 heads of 74400 380 / 390, 40 of 32760 413 / 428.
-constexpr int64_t kKvMeetMax = 5200;
+// K with the Wan step and V, a launch each or one for both, by the rounds of the chip that one launch takes (`slots` workgroups at
+// once, 768 where the grid's factors take up to 30 KB of LDS).  One launch has a gap less (3 us) and fills up its last round once
+// and not twice, but V's chunks run three to a compute unit where they would run four.  us per call, a launch each / one, in calls none
+// of whose query rows count (what they do besides is the same), at 12, 24 and 40 heads of one entry and 24 and 40 of two:
+//   under 1.5 rounds     0.7-0.9: 83.6 / 75.7, 80.6 / 72.3, 80.0 / 68.2; 1.3-1.45: 99.4 / 96.0, 94.7 / 91.7, 108.1 / 101.0
+//   1.5 .. 2: slower     112.1 / 116.3, 115.3 / 118.2, 126.1 / 131.0, 120.2 / 130.5, 110.1 / 114.9 (24 of 25 sizes)
+//   2 .. 7 rounds        2.7: 192.3 / 175.6, 193.2 / 180.8, 170.8 / 164.5; 4.5: 308.6 / 299.5, 290.3 / 281.3, 289.2 / 281.8; 6.2-6.5:
+//                        430.4 / 436.7, 393.7 / 389.9, 395.5 / 387.7, 382.8 / 381.0, 387.9 / 381.8; 6.9: +1.2, +2.7, -3.1, -3.2, -4.0
+//   beyond 7: slower     7.1: 462.3 / 464.9, 424.3 / 434.0, 427.9 / 430.4, 413.2 / 414.8, 418.1 / 419.6; up to 14 rounds -1 to +3 %
+static bool kv_in_one_launch_pays(int64_t workgroups, int64_t slots) {
+  return 2 * workgroups < 3 * slots || (workgroups > 2 * slots && workgroups <= 7 * slots);
+}
 
 hipError_t launch_quant_kv_meet(const QkvCall& c, const PrepParams& prep, hipStream_t s, bool* used) {
   *used = false;
   const int64_t grid = 2 * (int64_t)c.B * c.Hkv * c.nch;
-  if (grid > kKvMeetMax || (prep.kind != 1 && prep.kind != 3) || one_read_demoted()) return hipSuccess;
+  if (grid > INT32_MAX || (prep.kind != 1 && prep.kind != 3) || one_read_demoted()) return hipSuccess;
   const QuantSync& y = c.sync;
   const long long ticks = quant_options().wait_ticks;
   int* host = host_word(false).dev;
@@ -2394,7 +2403,8 @@ hipError_t launch_quant_kv_meet(const QkvCall& c, const PrepParams& prep, hipStr
   PrepParams pp = prep;
   const size_t lds = plan_rope_lds(&pp, c.B, kMeanChunk);
   auto go = [&](auto kernel) {
-    if (2 * c.nch > resident_workgroups(kernel, lds)) return;
+    const int slots = resident_workgroups(kernel, lds);
+    if (2 * c.nch > slots || !kv_in_one_launch_pays(grid, slots)) return;
     kernel<<<dim3((unsigned)grid), dim3(kThreads), lds, s>>>(c, pp, sk, sv);
     *used = true;
   };

@@ -116,6 +116,17 @@ def test_the_row_norm_step_in_whole_calls(hip_device, B, Lq, Lk, Hq, Hkv, norm, 
     _compare(hip_device, B, Lq, Lk, Hq, Hkv, 128, torch.bfloat16, True, sage_ops.WanPrep(wq, wk, 1e-6, **kw))
 
 
+# 1140 and 1152, 1536 and 1584, 5376 and 5424 workgroups: one launch for K and V below 1.5 rounds of 768 and from 2 to 7
+@pytest.mark.parametrize("B,Lk,H", [(1, 24300, 6), (1, 24400, 6), (2, 8192, 12), (2, 8200, 12), (1, 28672, 24), (1, 28700, 24)])
+def test_the_row_norm_step_where_one_launch_starts_and_ends(hip_device, B, Lk, H):
+    print(f"case B={B} Lk={Lk} H={H}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(Lk)
+    wq, wk = (1.0 + 0.2 * torch.randn(H * 128, generator=g, device=hip_device) for _ in range(2))
+    ang = torch.rand((1024, 64), generator=g, device=hip_device, dtype=torch.float64) * 6.0
+    prep = sage_ops.WanPrep(wq, wk, 1e-6, freqs=torch.polar(torch.ones_like(ang), ang), grid_sizes=[(2, 4, 5)] * B)
+    _compare(hip_device, B, 40, Lk, H, H, 128, torch.bfloat16, True, prep)
+
+
 def _inputs(hip_device, B, Lk, Hq, Hkv, D, dtype):
     g = torch.Generator(device=hip_device).manual_seed(Lk + D)
     k = torch.randn((B, Lk, Hkv, D), generator=g, device=hip_device) + 2.0 * torch.randn((Hkv, D), generator=g, device=hip_device)
