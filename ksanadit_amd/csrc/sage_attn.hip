@@ -425,19 +425,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         int top = max(s[0][0], s[1][0]);
 #pragma unroll
         for (int r = 1; r < 16; ++r) top = max(max(top, s[0][r]), s[1][r]);
-        const auto sw = __builtin_amdgcn_permlane32_swap(top, top, false, false);
-        top = max((int)sw[0], (int)sw[1]);
         float sc = qs * s_ks[j], mneg = -kMagicVal * sc;
-        const float m_tile = __builtin_fmaf(__int_as_float(top), sc, mneg);
-        const bool nan = m_tile != m_tile;  // a row whose scores are not numbers becomes NaN and goes on with zero scores
-        const float m_new = nan ? 0.0f : (m_tile > x_limit ? m_tile : m_run);
-        const float alpha = fast_exp2((nan ? m_tile : m_run) - m_new);
-        sc = nan ? 0.0f : sc;
-        mneg = nan ? 0.0f : mneg;
-        qs = nan ? 0.0f : qs;
-        m_run = m_new;
-        x_limit = m_new + kLazyMax;
-        x_base = kPShift - m_new;
+        const float alpha = move_point(top, sc, mneg, qs, m_run, x_base, x_limit);
         if (j == j0 ? __any(alpha != alpha) : __any(alpha != 1.0f)) {
 #pragma unroll
           for (int dt = 0; dt < kG; ++dt)
@@ -445,16 +434,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
             for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
           lacc[0] *= alpha;
         }
-        const float xc = x_base + mneg;
-        v8i pf;
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-          float e[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) e[i] = fast_exp2(__builtin_fmaf(__int_as_float(s[w >> 2][4 * (w & 3) + i]), sc, xc));
-          int code = __builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], __float_as_int(e[0]), false);
-          pf[w] = __builtin_amdgcn_cvt_pk_fp8_f32(e[2], e[3], code, true);
-        }
+        v8i pf = tile_probs(s, sc, x_base + mneg);
         if (n_last != 0) blank_probs(pf, hh, n_last);
         fetch_k(min(j + 1, nkb - 1));
         __builtin_amdgcn_sched_barrier(0);
@@ -735,31 +715,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   auto lane_max = [&](const v16i (&blk)[2]) {
     return max(max(max8(blk[0], 0), max8(blk[0], 8)), max(max8(blk[1], 0), max8(blk[1], 8)));
   };
-  constexpr float kShift = kPwlExp ? kPShiftPwl : kPShift, kLazy = kPwlExp ? kLazyMaxPwl : kLazyMax;
-  // Moves query l32's reference point where this tile's maximum asks for it (imax: this lane's maximum, over half the
-  // query's keys) and returns 2^(old point - new point), exactly 1 where the point stays.
-  // A row whose scores are not numbers (an infinity in its q, or in a key) gets the factor NaN, which makes its
-  // accumulators and sums NaN, and goes on with zero scores: its probabilities must stay numbers, see lacc.
-  auto move_point = [&](int imax, float& sc, float& mneg) -> float {
-    {
-      // the other half of query l32's keys lives in lane l32 + 32
-      int other = imax;
-      const auto sw = __builtin_amdgcn_permlane32_swap(imax, other, false, false);
-      imax = max(sw[0], sw[1]);
-    }
-    // the accumulator read as fp32 is magic + dot, so one fma gives sc * dot (mneg = -magic * sc)
-    const float m_tile = __builtin_fmaf(__int_as_float(imax), sc, mneg);
-    const bool nan = m_tile != m_tile;
-    const float m_new = nan ? 0.0f : (m_tile > x_limit ? m_tile : m_run);  // the limit is -inf at the first tile: always taken
-    const float alpha = fast_exp2((nan ? m_tile : m_run) - m_new);
-    sc = nan ? 0.0f : sc;
-    mneg = nan ? 0.0f : mneg;
-    qs = nan ? 0.0f : qs;
-    m_run = m_new;
-    x_limit = m_new + kLazy;
-    x_base = kShift - m_new;
-    return alpha;
-  };
   // p = exp2(sc*dot - m_run + shift); the magic is folded into the constant c, which is off by
   // at most ~1.5 integer steps of the dot product
   auto p_of = [&](int acc_bits, float sc, float c) { return fast_exp2(__builtin_fmaf(__int_as_float(acc_bits), sc, c)); };
@@ -826,7 +781,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       asm volatile("");  // (two branches on purpose: merged into one condition, the second is computed in every step)
       // (a tile this wave's mask row does not ask for, or that is not this loop's, leaves the points alone)
       if (jn < n_tiles && mine_at(jn)) {
-        alpha = move_point(mx, sc, mneg);
+        alpha = move_point<kPwlExp>(mx, sc, mneg, qs, m_run, x_base, x_limit);
         moved = 1;
       }
     }

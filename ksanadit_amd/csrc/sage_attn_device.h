@@ -113,6 +113,47 @@ __device__ __forceinline__ void blank_probs(v8i& pf, int hh, int n) {
   }
 }
 
+// Moves the reference point of a lane's row where this tile's maximum asks for it (imax: the lane's maximum, over half the
+// row's keys; sc, mneg: the tile's scale and -magic * scale) and returns 2^(old point - new point), exactly 1 where the point stays.
+// A row whose scores are not numbers (an infinity in its q, or in a key) gets the factor NaN, which makes its
+// accumulators and sums NaN, and goes on with zero scores: its probabilities must stay numbers, for the 16x16 row sums
+// multiply them by another row's zeros.
+template <bool kPwlExp = false>
+__device__ __forceinline__ float move_point(int imax, float& sc, float& mneg, float& qs, float& m_run, float& x_base, float& x_limit) {
+  {
+    // the other half of the row's keys lives in lane +- 32
+    int other = imax;
+    const auto sw = __builtin_amdgcn_permlane32_swap(imax, other, false, false);
+    imax = max((int)sw[0], (int)sw[1]);
+  }
+  // the accumulator read as fp32 is magic + dot, so one fma gives sc * dot (mneg = -magic * sc)
+  const float m_tile = __builtin_fmaf(__int_as_float(imax), sc, mneg);
+  const bool nan = m_tile != m_tile;
+  const float m_new = nan ? 0.0f : (m_tile > x_limit ? m_tile : m_run);  // the limit is -inf at the first tile: always taken
+  const float alpha = fast_exp2((nan ? m_tile : m_run) - m_new);
+  sc = nan ? 0.0f : sc;
+  mneg = nan ? 0.0f : mneg;
+  qs = nan ? 0.0f : qs;
+  m_run = m_new;
+  x_limit = m_new + (kPwlExp ? kLazyMaxPwl : kLazyMax);
+  x_base = (kPwlExp ? kPShiftPwl : kPShift) - m_new;
+  return alpha;
+}
+
+// the probabilities of a tile as the product with V takes them: 2^(sc * dot + xc - magic * sc), the magic folded into xc, in e4m3
+__device__ __forceinline__ v8i tile_probs(const v16i (&s)[2], float sc, float xc) {
+  v8i pf;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    float e[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) e[i] = fast_exp2(__builtin_fmaf(__int_as_float(s[w >> 2][4 * (w & 3) + i]), sc, xc));
+    int code = __builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], __float_as_int(e[0]), false);  // both halves get written
+    pf[w] = __builtin_amdgcn_cvt_pk_fp8_f32(e[2], e[3], code, true);
+  }
+  return pf;
+}
+
 // S^T tile (64 keys x 32 queries) of one wave: two 32-key sub-tiles, kG 32-channel steps (the channel groups that
 // hold data: 4, or 2 for head size 64, whose upper 64 channels are zeros on both sides).
 template <int kG>

@@ -145,18 +145,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
       const float m_half = __builtin_fmaf(__int_as_float(mx), sc, mneg);
       moved = 0;
       if (__ballot(!(m_half <= x_limit)) != 0 && jn < n_tiles) {
-        const auto sw = __builtin_amdgcn_permlane32_swap(mx, mx, false, false);
-        const int both = max((int)sw[0], (int)sw[1]);
-        const float m_tile = __builtin_fmaf(__int_as_float(both), sc, mneg);
-        const bool nan = m_tile != m_tile;
-        const float m_new = nan ? 0.0f : (m_tile > x_limit ? m_tile : m_run);
-        alpha = fast_exp2((nan ? m_tile : m_run) - m_new);
-        sc = nan ? 0.0f : sc;
-        mneg = nan ? 0.0f : mneg;
-        qs = nan ? 0.0f : qs;
-        m_run = m_new;
-        x_limit = m_new + kLazyMax;
-        x_base = kPShift - m_new;
+        alpha = move_point(mx, sc, mneg, qs, m_run, x_base, x_limit);
         moved = 1;
       }
       xc = x_base + mneg;

@@ -274,31 +274,14 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c,
       // keys [0, allowed) of the tile count for this row
       const int allowed = min(kBlkK, (c.causal ? min(lk, row + 1) : lk) - j * kBlkK);
       const bool whole = __all(allowed == kBlkK);
-      if (!whole) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (32 * u + 8 * (r >> 2) + 4 * hh + (r & 3) >= allowed) s[u][r] = kMagicBits - (1 << 22);  // below every real score
-      }
+      if (!whole) blank_scores<kMagicBits>(s, hh, allowed);
       int top = s[0][0];
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) top = max(top, s[u][r]);
-      const auto sw = __builtin_amdgcn_permlane32_swap(top, top, false, false);
-      top = max((int)sw[0], (int)sw[1]);
       float sc = qs * s_ks[j], mneg = -kMagicVal * sc;
-      const float m_tile = __builtin_fmaf(__int_as_float(top), sc, mneg);
-      const bool nan = m_tile != m_tile;  // a row whose scores are not numbers becomes NaN and goes on with zero scores
-      const float m_new = nan ? 0.0f : (m_tile > x_limit ? m_tile : m_run);
-      const float alpha = fast_exp2((nan ? m_tile : m_run) - m_new);
-      sc = nan ? 0.0f : sc;
-      mneg = nan ? 0.0f : mneg;
-      qs = nan ? 0.0f : qs;
-      m_run = m_new;
-      x_limit = m_new + kLazyMax;
-      x_base = kPShift - m_new;
+      const float alpha = move_point(top, sc, mneg, qs, m_run, x_base, x_limit);
       if (j == 0 ? __any(alpha != alpha) : __any(alpha != 1.0f)) {
 #pragma unroll
         for (int dt = 0; dt < kG; ++dt)
@@ -306,24 +289,8 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c,
           for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
         lacc[0] *= alpha;
       }
-      const float xc = x_base + mneg;
-      v8i pf;
-#pragma unroll
-      for (int w = 0; w < 8; ++w) {
-        float e[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) e[i] = fast_exp2(__builtin_fmaf(__int_as_float(s[w >> 2][4 * (w & 3) + i]), sc, xc));
-        int code = __builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], 0, false);
-        code = __builtin_amdgcn_cvt_pk_fp8_f32(e[2], e[3], code, true);
-        pf[w] = code;
-      }
-      if (!whole) {  // the bytes of keys that do not count are cleared outright (code 0 is +0.0)
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-          const int n = min(max(allowed - (32 * (w >> 2) + 8 * (w & 3) + 4 * hh), 0), 4);
-          pf[w] &= (int)(n >= 4 ? 0xffffffffu : ((1u << (8 * n)) - 1u));
-        }
-      }
+      v8i pf = tile_probs(s, sc, x_base + mneg);
+      if (!whole) blank_probs(pf, hh, allowed);
       const uint8_t* vt = v_tiles + j * kTileBytes;
 #pragma unroll
       for (int dt = 0; dt < kG; ++dt) {
