@@ -1340,9 +1340,7 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   if (p.nkb > kMaxKeyTiles) return hipErrorInvalidValue;
   const bool sparse = p.block_mask != nullptr || p.causal;
   if (sparse && p.nkb > kSparseMaxKeyTiles) return hipErrorInvalidValue;
-  if (!sparse && p.q_rows.ptr != nullptr && p.q_lens == nullptr && p.k_lens == nullptr && p.exact_exp2 && !p.tile_skip && p.wg_waves == 0 &&
-      resident_call_suits(p.B, p.Hq, p.Lq, p.Lk))
-    return launch_resident(p, s);
+  if (p.q_rows.ptr != nullptr && resident_call_suits(p)) return launch_resident(p, s);
   const bool plain_causal = p.causal && p.block_mask == nullptr && p.exact_exp2 && !p.tile_skip;  // no tile list
   int waves = pick_wg_waves(p);
   if (waves == 4 && p.nkb > (sparse ? kSparseMaxKeyTiles4 : kShortMaxKeyTiles)) waves = 8;

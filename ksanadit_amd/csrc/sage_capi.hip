@@ -845,28 +845,12 @@ int ksana_sage_forward_varlen(const void* q, const void* k, const void* v, void*
 }  // extern "C"
 
 namespace {
-// q_rows: nullptr, or Q as the caller has it (validated, of the result's dtype) for the kernel to quantize - with lin, for
-// the linear branch that the kernel then adds
-int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
-              const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags,
-              const ksana_sage::InTensor* q_rows, float q_premul, void* stream, const ksana_sage::AttnLinear* lin) {
-  const StageRange range("ksana_sage.attention");
-  if (int rc = check_shape(s)) return rc;
-  if (int rc = check_mask(s, block_mask, mask_st)) return rc;
-  if (int rc = check_causal(s, causal)) return rc;
-  if (flags & ~(KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES | KSANA_SAGE_FLAG_TILE_SKIP))
-    return fail(KSANA_SAGE_EINVAL, "unknown flag bits 0x%x", flags);
-  if ((flags & KSANA_SAGE_FLAG_TILE_SKIP) && (flags & KSANA_SAGE_FLAG_PWL_EXP2))
-    return fail(KSANA_SAGE_EINVAL, "KSANA_SAGE_FLAG_TILE_SKIP goes with the exact exponential only, not with KSANA_SAGE_FLAG_PWL_EXP2");
-  if (int rc = check_tensor("o", o, dtype, o_st, s->B, s->Lq, s->Hq)) return rc;
-  if (int rc = check_ws(ws)) return rc;
-  if (reinterpret_cast<uintptr_t>(k_lens) & 3) return fail(KSANA_SAGE_EINVAL, "k_lens is not 4-byte aligned");
-  if (reinterpret_cast<uintptr_t>(q_lens) & 3) return fail(KSANA_SAGE_EINVAL, "q_lens is not 4-byte aligned");
+// The attention kernel's view of a call whose arguments have been validated
+ksana_sage::AttnParams attn_params(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
+                                   const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags) {
   ksana_sage_ws_layout l;
   ksana_sage_workspace_layout(s, &l);
   ksana_sage::AttnParams p;
-  if (q_rows != nullptr) p.q_rows = *q_rows, p.q_premul = q_premul;
-  if (lin != nullptr) p.lin = *lin;
   p.q_i8 = ws_at<int8_t>(ws, l.q_i8);
   p.q_scale = ws_at<float>(ws, l.q_scale);
   p.k_tiles = ws_at<int8_t>(ws, l.k_i8);
@@ -889,6 +873,29 @@ int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_s
   p.causal = causal ? 1 : 0;
   p.d_out = s->D;
   p.tile_skip = (flags & KSANA_SAGE_FLAG_TILE_SKIP) ? 1 : 0;
+  return p;
+}
+
+// q_rows: nullptr, or Q as the caller has it (validated, of the result's dtype) for the kernel to quantize - with lin, for
+// the linear branch that the kernel then adds
+int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
+              const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags,
+              const ksana_sage::InTensor* q_rows, float q_premul, void* stream, const ksana_sage::AttnLinear* lin) {
+  const StageRange range("ksana_sage.attention");
+  if (int rc = check_shape(s)) return rc;
+  if (int rc = check_mask(s, block_mask, mask_st)) return rc;
+  if (int rc = check_causal(s, causal)) return rc;
+  if (flags & ~(KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES | KSANA_SAGE_FLAG_TILE_SKIP))
+    return fail(KSANA_SAGE_EINVAL, "unknown flag bits 0x%x", flags);
+  if ((flags & KSANA_SAGE_FLAG_TILE_SKIP) && (flags & KSANA_SAGE_FLAG_PWL_EXP2))
+    return fail(KSANA_SAGE_EINVAL, "KSANA_SAGE_FLAG_TILE_SKIP goes with the exact exponential only, not with KSANA_SAGE_FLAG_PWL_EXP2");
+  if (int rc = check_tensor("o", o, dtype, o_st, s->B, s->Lq, s->Hq)) return rc;
+  if (int rc = check_ws(ws)) return rc;
+  if (reinterpret_cast<uintptr_t>(k_lens) & 3) return fail(KSANA_SAGE_EINVAL, "k_lens is not 4-byte aligned");
+  if (reinterpret_cast<uintptr_t>(q_lens) & 3) return fail(KSANA_SAGE_EINVAL, "q_lens is not 4-byte aligned");
+  ksana_sage::AttnParams p = attn_params(ws, o, dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, flags);
+  if (q_rows != nullptr) p.q_rows = *q_rows, p.q_premul = q_premul;
+  if (lin != nullptr) p.lin = *lin;
   hipError_t e = ksana_sage::launch_attn_fwd(p, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? 0 : hip_fail(e, "attention launch");
 }
@@ -990,9 +997,7 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
   const int n_wg = s->B * s->Hq * ((s->Lq + ksana_sage::kAttnQPerWg - 1) / ksana_sage::kAttnQPerWg);
   const bool own_q = (flags & KSANA_SAGE_FLAG_Q_UNSTORED) && prep == nullptr && block_mask == nullptr && o_dtype == dtype &&
                      (ksana_sage::q_in_attention_pays(n_wg, (s->Lk + ksana_sage::kBlkK - 1) / ksana_sage::kBlkK) ||
-                      (!causal && q_lens == nullptr && k_lens == nullptr &&
-                       !(flags & (KSANA_SAGE_FLAG_PWL_EXP2 | KSANA_SAGE_FLAG_TILE_SKIP | KSANA_SAGE_FLAG_WG_4_WAVES | KSANA_SAGE_FLAG_WG_8_WAVES)) &&
-                       ksana_sage::resident_call_suits(s->B, s->Hq, s->Lq, s->Lk)));
+                      ksana_sage::resident_call_suits(attn_params(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, flags)));
   const bool trim = (flags & KSANA_SAGE_FLAG_WS_UNSTORED) && prep == nullptr;  // what no row or key that takes part needs
   if (int rc = quant_qkv(!own_q, q, k, v, dtype, q_st, k_st, v_st, s, prep, sm_scale, smooth_k, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws,
                          stream, trim ? q_lens : nullptr, trim ? k_lens : nullptr))

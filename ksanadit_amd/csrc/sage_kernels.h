@@ -269,9 +269,10 @@ void plan_key_split(int n_wg, int nkb, int* first_wg, int* runs);
 // Is a call with `n_wg` 256-row query blocks and `nkb` key tiles faster when the attention kernel quantizes Q itself?
 bool q_in_attention_pays(int n_wg, int nkb);
 
-// A dense call with Q as the caller has it, few keys and many query rows (sage_resident.hip): launch_attn_fwd takes it when it
-// suits and the call is plain - p.q_rows set, no mask, no counts, not causal, default variant and shape.
-bool resident_call_suits(int B, int Hq, int Lq, int Lk);
+// A dense call with Q as the caller has it, few keys and many query rows (sage_resident.hip): launch_attn_fwd takes it for calls
+// that suit - no mask, no counts, not causal, default variant and shape - when p.q_rows is set.  (Of p it looks at the sizes and
+// the options.)
+bool resident_call_suits(const AttnParams& p);
 hipError_t launch_resident(const AttnParams& p, hipStream_t s);
 
 // A whole call of at most kMeanChunk keys in one launch (sage_small.hip): q, k and v as the caller has them, o of their type.

@@ -328,9 +328,10 @@ hipError_t launch(const AttnParams& p, hipStream_t s) {
 // 63.6 / 60.2, 2 x 64 of 2700 on 192 78.8 / 68.5; but 40 of 4096 (5120 blocks) on 77 37.7 / 40.2, and beyond 256 keys 40 of 8190
 // on 512 88.6 / 90.1, 100 of 4096 on 320 93.9 / 98.0.  (Not for batches with lengths of their own: 3 x 40 heads of 2776 rows on up to
 // 463 keys 83 / 113.)
-bool resident_call_suits(int B, int Hq, int Lq, int Lk) {
-  const int64_t blocks = (int64_t)B * Hq * ((Lq + kRows - 1) / kRows);
-  return Lk <= kMaxTiles * kBlkK && Lq >= 1024 && blocks >= (Lk <= kMeanChunk ? 4 : 8) * kWaves * kComputeUnits;
+bool resident_call_suits(const AttnParams& p) {
+  if (p.block_mask != nullptr || p.causal || p.q_lens != nullptr || p.k_lens != nullptr || !p.exact_exp2 || p.tile_skip || p.wg_waves != 0) return false;
+  const int64_t blocks = (int64_t)p.B * p.Hq * ((p.Lq + kRows - 1) / kRows);
+  return p.Lk <= kMaxTiles * kBlkK && p.Lq >= 1024 && blocks >= (p.Lk <= kMeanChunk ? 4 : 8) * kWaves * kComputeUnits;
 }
 
 hipError_t launch_resident(const AttnParams& p, hipStream_t s) {
