@@ -48,29 +48,33 @@ def _usable(t: torch.Tensor) -> torch.Tensor:
     return t.contiguous()
 
 
-_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype): (version, converted)}
+_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype): ((version, address), converted)}
 _prep_move_warned = False
 
 
 def _prep_operand(t: torch.Tensor, device, dtype) -> torch.Tensor:
     """A weight or table of the step before attention as the kernels read it: on ``device``, ``dtype``, contiguous.
-    A conversion is remembered per source tensor (and redone once that tensor has been written to), so a caller that
-    keeps its weights in another dtype - or on the host - pays for it once, not in every attention call; a transfer
-    from another device is logged the first time."""
+    A conversion is remembered per source tensor (and redone once that tensor has been written to or has been given other
+    memory, as ``p.data = ...`` does), so a caller that keeps its weights in another dtype - or on the host - pays for it
+    once, not in every attention call; a transfer from another device is logged the first time.  Tensors made in inference
+    mode keep no count of their writes: they are converted in every call."""
     global _prep_move_warned
     device = torch.device(device)
     if t.device == device and t.dtype == dtype and t.is_contiguous():
         return t
     key = (device, dtype)
-    hit = _prep_cache.get(t, {}).get(key)
-    if hit is not None and hit[0] == t._version:
+    state = None if t.is_inference() else (t._version, t.data_ptr())
+    hit = None if state is None else _prep_cache.get(t, {}).get(key)
+    if hit is not None and hit[0] == state:
         return hit[1]
     if t.device != device and not _prep_move_warned:
         _prep_move_warned = True
         log.warning("Sage HIP path: a norm weight / rotary table lives on %s, the tensors on %s; it is copied over once "
                     "per tensor (keep them on the device to avoid even that)", t.device, device)
-    conv = t.detach().to(device=device, dtype=dtype).contiguous()
-    _prep_cache.setdefault(t, {})[key] = (t._version, conv)
+    with torch.inference_mode(False), torch.no_grad():  # (made in inference mode it could not be remembered in turn)
+        conv = t.detach().to(device=device, dtype=dtype).contiguous()
+    if state is not None:
+        _prep_cache.setdefault(t, {})[key] = (state, conv)
     return conv
 
 

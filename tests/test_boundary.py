@@ -340,6 +340,29 @@ def test_prep_operands_are_converted_once_per_source_tensor():
     assert t128.dtype == torch.complex128 and sage_ops._prep_operand(table, "cpu", torch.complex128) is t128
 
 
+def test_prep_operands_given_other_memory_are_converted_anew():
+    """``p.data = ...`` (weights swapped or moved) leaves the count of writes as it was."""
+    p = torch.nn.Parameter(torch.ones(4, dtype=torch.bfloat16))
+    assert torch.equal(sage_ops._prep_operand(p, "cpu", torch.float32), torch.ones(4))
+    other = torch.full((4,), 3.0, dtype=torch.bfloat16)
+    p.data = other
+    assert torch.equal(sage_ops._prep_operand(p, "cpu", torch.float32), torch.full((4,), 3.0))
+
+
+def test_prep_operands_in_inference_mode():
+    """Tensors made in inference mode count no writes; conversions of other tensors made there are remembered."""
+    p = torch.nn.Parameter(torch.ones(4))
+    with torch.inference_mode():
+        w = torch.ones(4, dtype=torch.bfloat16)
+        assert torch.equal(sage_ops._prep_operand(w, "cpu", torch.float32), torch.ones(4))
+        w.fill_(2.0)
+        half = sage_ops._prep_operand(p, "cpu", torch.float16)
+        back = sage_ops._prep_operand(half, "cpu", torch.float32)
+    assert torch.equal(sage_ops._prep_operand(w, "cpu", torch.float32), torch.full((4,), 2.0))
+    assert sage_ops._prep_operand(p, "cpu", torch.float16) is half and sage_ops._prep_operand(half, "cpu", torch.float32) is back
+    assert not half.requires_grad and not back.requires_grad and torch.equal(back, torch.ones(4))
+
+
 def test_one_read_settings_and_the_occupancy_cache_without_gpu():
     """``ksana_sage_configure`` validates and stores its settings without touching a device; the launchers' cache of
     resident-workgroup counts keeps one entry per kernel instantiation (two instantiations of one template have the same
