@@ -29,6 +29,29 @@ static int g_failed = 0;
     }                                                                                             \
   } while (0)
 
+// Every (pair, query block) of a causal launch belongs to one workgroup, and an XCD never starts a longer block of a pair
+// after a shorter one.  `kinds` collects what the grids seen have had: more than one group, an uneven first group, pairs left over,
+// none to an XCD itself.
+static int causal_numbering_is_wrong(int pairs, int n_qwg, unsigned* kinds) {
+  const ksana_sage::CausalGrid c = ksana_sage::causal_grid(pairs, n_qwg);
+  if (c.group < 1) return 1;
+  *kinds |= (c.own >= 2 * c.group ? 1u : 0) | (c.own % c.group != 0 && c.own > c.group ? 2u : 0) | (c.rest != 0 ? 4u : 0) | (c.own == 0 ? 8u : 0);
+  std::vector<char> seen((size_t)pairs * n_qwg, 0);
+  std::vector<int> last(8 * (size_t)pairs, n_qwg);  // the block of the pair that the XCD started last
+  int n = 0;
+  for (int block = 0; block < (pairs * n_qwg + 7) / 8 * 8; ++block) {
+    int pair = -1, qwg = -1;
+    if (!ksana_sage::causal_place(c, block, n_qwg, &pair, &qwg)) continue;
+    if (pair < 0 || pair >= pairs || qwg < 0 || qwg >= n_qwg) return 1;
+    char& here = seen[(size_t)pair * n_qwg + qwg];
+    int& before = last[(size_t)(block & 7) * pairs + pair];
+    if (here++ != 0 || qwg >= before) return 1;
+    before = qwg;
+    ++n;
+  }
+  return n != pairs * n_qwg;
+}
+
 int main() {
   void* const fake = reinterpret_cast<void*>(0x1000);  // aligned and never dereferenced
   ksana_sage_shape s{1, 2, 2, 64, 64, 128};
@@ -99,6 +122,12 @@ int main() {
   EXPECT(ksana_sage_forward(fake, fake, nullptr, fake, KSANA_SAGE_BF16, st, st, st, st, &s, nullptr, 0.1f, 1, 0, 0, fake, nullptr), KSANA_SAGE_EINVAL);
   int first = -1, runs = -1;
   EXPECT(ksana_sage_attn_key_split(&s, &first, nullptr), KSANA_SAGE_EINVAL);
+
+  unsigned kinds = 0;
+  for (int pairs = 1; pairs <= 130; ++pairs)
+    for (int n_qwg : {1, 2, 3, 7, 11, 24, 63, 64, 65, 96, 97, 128, 192, 255, 256, 383, 384, 385, 590, 1024})
+      if (causal_numbering_is_wrong(pairs, n_qwg, &kinds)) ++g_failed, std::printf("causal numbering of %d pairs of %d blocks\n", pairs, n_qwg);
+  if (kinds != 15) ++g_failed, std::printf("causal numbering: kinds of grids seen 0x%x\n", kinds);
 
   // the sparse-linear backend's entry points
   uint64_t bytes = 0;

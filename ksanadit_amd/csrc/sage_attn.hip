@@ -109,32 +109,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   int bh, qwg;  // (batch, head) pair and query block
   const bool is_run = kCanSplit && (int)blockIdx.x >= p.split_first_block;  // uniform
   const int run_id = is_run ? (int)blockIdx.x - p.split_first_block : 0;    // the partial result's place in the workspace
-  if (kCausal && p.causal_group != 0) {
-    // The later a query block, the more key tiles it walks: every XCD starts its long blocks first (causal_grid).
-    const int xcd = blockIdx.x & 7;
-    int at = blockIdx.x >> 3;
-    const int shared = (p.causal_rest * n_qwg - xcd + 7) >> 3;  // this XCD's eighth of the pairs left over
-    if (at < shared) {
-      const int i = at * 8 + xcd, blk = i / p.causal_rest;
-      bh = 8 * p.causal_own + i - blk * p.causal_rest;
-      qwg = n_qwg - 1 - blk;
-    } else {
-      at -= shared;
-      if (at >= p.causal_own * n_qwg) return;
-      // groups of causal_group pairs, the first one with what does not divide evenly
-      const int n_groups = p.causal_own / p.causal_group;
-      int first = 0, size = p.causal_own - (n_groups - 1) * p.causal_group;
-      if (at >= size * n_qwg) {
-        at -= size * n_qwg;
-        const int g = at / (p.causal_group * n_qwg);
-        at -= g * p.causal_group * n_qwg;
-        first = size + g * p.causal_group;
-        size = p.causal_group;
-      }
-      const int blk = at / size;
-      bh = xcd * p.causal_own + first + at - blk * size;
-      qwg = n_qwg - 1 - blk;
-    }
+  if (kCausal && p.causal_grid.group != 0) {
+    if (!causal_place(p.causal_grid, blockIdx.x, n_qwg, &bh, &qwg)) return;
   } else {
     int wg;
     if (is_run) {
@@ -1319,21 +1295,6 @@ static dim3 xcd_grid(AttnParams* p, int n_qwg, int n_wg, int* wg_per_xcd) {
   return dim3(*wg_per_xcd * 8);
 }
 
-// The numbering of a causal launch (the kernel's first lines): every XCD takes B * Hq / 8 (batch, head) pairs of its own and
-// an eighth of the query blocks of the pairs left over - one run of blocks per XCD gives some of them a pair's long half and
-// others its short one.  Blocks go out from the last one down, through a group of pairs together: one pair after the other,
-// the last pair's long blocks start when little is left to run beside them.  A group has six blocks for each of an XCD's
-// workgroup places; larger ones only share the L2 between more heads.  us per call, one run and one pair after the other /
-// groups of 2 / of 6 blocks per place / all pairs together: 8 191 tokens of 32 heads 361 / 356 / 350 / 350, 2 x 3 000 of 64 heads
-// 254 / 240 / 236 / 236, 24 x 2 048 55 / 50 / 50 / 50; without the tile list 40 x 32 760 5 990 in groups of 6, 6 285 all together.
-constexpr int kPlacesPerXcd = 64;  // 4-wave workgroups: two on each of 32 compute units
-static void causal_grid(AttnParams* p, int n_qwg) {
-  const int pairs = p->B * p->Hq;
-  p->causal_own = pairs / 8;
-  p->causal_rest = pairs - 8 * p->causal_own;
-  p->causal_group = min((6 * kPlacesPerXcd + n_qwg - 1) / n_qwg, max(p->causal_own, 1));
-}
-
 hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   AttnParams p = params;
   p.split_first_block = INT32_MAX;
@@ -1349,7 +1310,7 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   const int n_wg = p.B * p.Hq * n_qwg;
   int wg_per_xcd = 0;
   const dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
-  if (p.causal && p.batch_run == 0) causal_grid(&p, n_qwg);  // (the same number of workgroups)
+  if (p.causal && p.batch_run == 0) p.causal_grid = causal_grid(p.B * p.Hq, n_qwg);  // (the same number of workgroups)
   // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
   const size_t lds = (waves == 4 ? WgShape<4>::kRingBytes : WgShape<8>::kRingBytes) + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
   if (p.lin.frag != nullptr) {

@@ -27,6 +27,51 @@ __host__ __device__ constexpr int tiles_counted(int count, int tiles) {
   return (int)(((unsigned)rows_counted(count, tiles * kBlkK) + kBlkK - 1) / kBlkK);
 }
 
+// The numbering of a causal launch's workgroups.  Consecutive ones land on consecutive XCDs.  Every XCD takes pairs / 8 of the
+// (batch, head) pairs for its own and an eighth of the query blocks of the pairs left over - one run of blocks per XCD gives some
+// of them a pair's long half and others its short one.  Blocks go out from the last one down, which walks the most key tiles,
+// through a group of pairs together: one pair after the other, the last pair's long blocks start when little is left to
+// run beside them.  A group has six blocks for each of an XCD's workgroup places; larger ones only share the L2 between
+// more heads.  us per call, one run and one pair after the other / groups of 2 / of 6 blocks per place / all pairs together:
+// 8 191 tokens of 32 heads 361 / 356 / 350 / 350, 2 x 3 000 of 64 heads 254 / 240 / 236 / 236, 24 x 2 048 55 / 50 / 50 / 50; without
+// the tile list 40 x 32 760 5 990 in groups of 6, 6 285 all together.
+struct CausalGrid {
+  int own = 0, rest = 0, group = 0;  // pairs an XCD has to itself, pairs left over, own ones walked together (0: no such launch)
+};
+constexpr int kXcds = 8, kPlacesPerXcd = 64;  // 4-wave workgroups: two on each of 32 compute units
+constexpr CausalGrid causal_grid(int pairs, int n_qwg) {
+  const int own = pairs / kXcds, fill = (6 * kPlacesPerXcd + n_qwg - 1) / n_qwg, most = own > 1 ? own : 1;
+  return CausalGrid{own, pairs - kXcds * own, fill < most ? fill : most};
+}
+// pair and query block of workgroup `block` of the (pairs * n_qwg + 7) / 8 * 8 launched; false: there is none for it
+__host__ __device__ constexpr bool causal_place(const CausalGrid& c, int block, int n_qwg, int* pair, int* qwg) {
+  const int xcd = block & 7;
+  int at = block >> 3;
+  const int shared = (c.rest * n_qwg - xcd + 7) >> 3;  // this XCD's eighth of the pairs left over
+  if (at < shared) {
+    const int i = at * 8 + xcd, blk = i / c.rest;
+    *pair = 8 * c.own + i - blk * c.rest;
+    *qwg = n_qwg - 1 - blk;
+    return true;
+  }
+  at -= shared;
+  if (at >= c.own * n_qwg) return false;
+  // groups of c.group pairs, the first one with what does not divide evenly
+  const int n_groups = c.own / c.group;
+  int first = 0, size = c.own - (n_groups - 1) * c.group;
+  if (at >= size * n_qwg) {
+    at -= size * n_qwg;
+    const int g = at / (c.group * n_qwg);
+    at -= g * c.group * n_qwg;
+    first = size + g * c.group;
+    size = c.group;
+  }
+  const int blk = at / size;
+  *pair = xcd * c.own + first + at - blk * size;
+  *qwg = n_qwg - 1 - blk;
+  return true;
+}
+
 struct InTensor {
   const uint16_t* ptr;
   int64_t sB, sL, sH;  // element strides of [B, L, H, D]; D stride is 1
@@ -251,9 +296,7 @@ struct AttnParams {
   int d_out;     // channels of an output row that exist: 128, or 64 (head size 64 runs zero-padded to 128)
   int tile_skip; // 1: a wave leaves out the exponentials of a key tile whose probabilities would all be the zero code
                  // (same bits; pays on sharply peaked attention, costs 7-13 % where no tile qualifies); 0: every tile in full
-  // filled in by the launcher for causal calls: (batch, head) pairs an XCD has to itself, the pairs left over, and how many
-  // of its own it walks through together (0: not a causal call, or one numbered by batch_run)
-  int causal_own = 0, causal_rest = 0, causal_group = 0;
+  CausalGrid causal_grid{};  // filled in by the launcher for causal calls that batch_run does not number
   // lin.frag != nullptr: that branch is added to every row; q_rows is then Q as the caller has it, for the branch (q_i8 is
   // read as ever).  With a block mask that gives every query block a key block, head size 128, no counts, default variant.
   AttnLinear lin{};

@@ -103,8 +103,8 @@ def test_whole_and_cut_query_blocks_in_one_grid(hip_device, Lk):
 @pytest.mark.parametrize("B,H", [(1, 1), (1, 3), (1, 8), (3, 5), (1, 17), (2, 24)])
 @pytest.mark.parametrize("L", [100, 128, 640, 1300])
 def test_causal_blocks_are_shared_out_over_the_chip(hip_device, B, H, L):
-    """Every (batch, head, query block) is computed once, whether its pair belongs to one XCD or to all of them and
-    whatever group of pairs it is walked through with; one block ahead of the diagonal, on it, and several."""
+    """Every (batch, head, query block) is computed once, whether its pair belongs to one XCD or to all of them; one block
+    ahead of the diagonal, on it, and several.  An XCD's own pairs are one group here."""
     print(f"case B={B} H={H} L={L}", flush=True)
     g = torch.Generator().manual_seed(100 * L + 10 * B + H)
     q, k, v = (torch.randn((B, L, H, 128), generator=g).to(torch.bfloat16) for _ in range(3))
@@ -113,6 +113,19 @@ def test_causal_blocks_are_shared_out_over_the_chip(hip_device, B, H, L):
     sage_ops.quant_q(qd, ws, 128**-0.5), sage_ops.quant_k(kd, ws, True), sage_ops.quant_v(vd, ws)
     out = sage_ops.attn_fwd(ws, torch.full_like(qd, float("nan")), causal=True).cpu()
     _close(out, _emul(ws, L, L, q.dtype, causal=True))
+
+
+def test_causal_pairs_are_walked_in_groups(hip_device):
+    """192 query blocks a head: an XCD walks its five pairs in groups of three and two, and three pairs are left over.  The same
+    bits as eight heads at a time, one to an XCD."""
+    L, H = 24500, 43
+    print(f"case H={H} L={L}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(L)
+    q, k, v = (torch.randn((1, L, H, 128), generator=g, device=hip_device).to(torch.bfloat16) for _ in range(3))
+    out = sage_ops.sageattn(q, k, v, is_causal=True)
+    for h in range(0, H, 8):
+        part = sage_ops.sageattn(q[:, :, h : h + 8], k[:, :, h : h + 8], v[:, :, h : h + 8], is_causal=True)
+        assert torch.equal(out[:, :, h : h + 8], part), h
 
 
 @pytest.mark.parametrize("waves", [4, 8])
