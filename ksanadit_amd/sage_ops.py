@@ -48,7 +48,7 @@ def _usable(t: torch.Tensor) -> torch.Tensor:
     return t.contiguous()
 
 
-_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype): ((version, address), converted)}
+_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype): ((version, address), converted, made on, made)}
 _prep_move_warned = False
 
 
@@ -57,24 +57,34 @@ def _prep_operand(t: torch.Tensor, device, dtype) -> torch.Tensor:
     A conversion is remembered per source tensor (and redone once that tensor has been written to or has been given other
     memory, as ``p.data = ...`` does), so a caller that keeps its weights in another dtype - or on the host - pays for it
     once, not in every attention call; a transfer from another device is logged the first time.  Tensors made in inference
-    mode keep no count of their writes: they are converted in every call."""
+    mode keep no count of their writes: they are converted in every call.  A call on another stream than the conversion's
+    waits for it.  A graph records a conversion of its own: one made before may be gone when it is replayed, and its own has no
+    values before that (a tensor on the host cannot be read by a graph: there the one made before it is taken)."""
     global _prep_move_warned
     device = torch.device(device)
     if t.device == device and t.dtype == dtype and t.is_contiguous():
         return t
     key = (device, dtype)
-    state = None if t.is_inference() else (t._version, t.data_ptr())
+    on_gpu = device.type == "cuda"
+    capturing = on_gpu and torch.cuda.is_current_stream_capturing()
+    state = None if t.is_inference() or (capturing and t.device == device) else (t._version, t.data_ptr())
     hit = None if state is None else _prep_cache.get(t, {}).get(key)
     if hit is not None and hit[0] == state:
-        return hit[1]
+        _, conv, made_on, made = hit
+        if on_gpu and not capturing and made_on != _stream_ptr(device):
+            stream = torch.cuda.current_stream(device)
+            stream.wait_event(made)
+            conv.record_stream(stream)
+        return conv
     if t.device != device and not _prep_move_warned:
         _prep_move_warned = True
         log.warning("Sage HIP path: a norm weight / rotary table lives on %s, the tensors on %s; it is copied over once "
                     "per tensor (keep them on the device to avoid even that)", t.device, device)
     with torch.inference_mode(False), torch.no_grad():  # (made in inference mode it could not be remembered in turn)
         conv = t.detach().to(device=device, dtype=dtype).contiguous()
-    if state is not None:
-        _prep_cache.setdefault(t, {})[key] = (state, conv)
+    if state is not None and not capturing:
+        stream = torch.cuda.current_stream(device) if on_gpu else None
+        _prep_cache.setdefault(t, {})[key] = (state, conv, stream and stream.cuda_stream, stream and stream.record_event())
     return conv
 
 

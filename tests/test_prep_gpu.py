@@ -280,3 +280,41 @@ def test_prep_argument_errors(hip_device):
         sage_ops.quant_q(wide, ws, 0.1, prep=WanPrep(wq, wq, 1e-6, None, None))
     with pytest.raises(ValueError, match="grid_sizes"):
         WanPrep(wq, wq, 1e-6, table, None).to_c(hip_device)
+
+
+def test_a_converted_weight_is_awaited_on_another_stream(hip_device):
+    """The conversion belongs to the stream it was made on; a call on another stream that finds it waits for it."""
+    src = torch.arange(4096, dtype=torch.float64, device=hip_device)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    src.float().clone()  # (kernels are loaded at their first use)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(first):
+        spoiled = torch.full((4096,), float("nan"), device=hip_device)
+        del spoiled  # (the conversion's memory is likely this)
+        torch.cuda._sleep(100_000_000)
+        sage_ops._prep_operand(src, hip_device, torch.float32)
+    with torch.cuda.stream(second):
+        got = sage_ops._prep_operand(src, hip_device, torch.float32).clone()
+    torch.cuda.synchronize()
+    assert torch.equal(got, src.float())
+
+
+@pytest.mark.parametrize("warm", [False, True])
+def test_a_weight_converted_under_capture_is_the_graphs_own(hip_device, warm):
+    """A conversion that a graph records has no values before a replay: calls outside the graph do not find it.  Replays convert
+    what the weight holds then, whatever has become of a conversion made before the capture."""
+    src = torch.full((4096,), 2.0, dtype=torch.float64, device=hip_device)
+    out = torch.zeros(4096, device=hip_device)
+    if warm:
+        sage_ops._prep_operand(src, hip_device, torch.float32)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out.copy_(sage_ops._prep_operand(src, hip_device, torch.float32))
+    assert torch.equal(sage_ops._prep_operand(src, hip_device, torch.float32), src.float())
+    for value in (3.0, 4.0):
+        src.fill_(value)
+        assert torch.equal(sage_ops._prep_operand(src, hip_device, torch.float32), src.float())
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, src.float())
