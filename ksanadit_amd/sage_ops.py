@@ -13,6 +13,7 @@ thousands of calls of one generation.
 from __future__ import annotations
 
 import ctypes as C
+from contextlib import nullcontext
 from dataclasses import dataclass
 
 import torch
@@ -48,12 +49,13 @@ def _usable(t: torch.Tensor) -> torch.Tensor:
     return t.contiguous()
 
 
-_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype): ((version, address), converted, made on, made)}
+_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype, through): ((version, address), converted, made on, made)}
 _prep_move_warned = False
 
 
-def _prep_operand(t: torch.Tensor, device, dtype) -> torch.Tensor:
-    """A weight or table of the step before attention as the kernels read it: on ``device``, ``dtype``, contiguous.
+def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
+    """A weight or table of the step before attention as the kernels read it: on ``device``, ``dtype`` (its values rounded to
+    ``through`` first, if given), contiguous.
     A conversion is remembered per source tensor (and redone once that tensor has been written to or has been given other
     memory, as ``p.data = ...`` does), so a caller that keeps its weights in another dtype - or on the host - pays for it
     once, not in every attention call; a transfer from another device is logged the first time.  Tensors made in inference
@@ -62,13 +64,14 @@ def _prep_operand(t: torch.Tensor, device, dtype) -> torch.Tensor:
     values before that (a tensor on the host cannot be read by a graph: there the one made before it is taken)."""
     global _prep_move_warned
     device = torch.device(device)
-    if t.device == device and t.dtype == dtype and t.is_contiguous():
+    if t.device == device and t.dtype == dtype and through in (None, dtype) and t.is_contiguous():
         return t
-    key = (device, dtype)
+    key = (device, dtype, through)
     on_gpu = device.type == "cuda"
     capturing = on_gpu and torch.cuda.is_current_stream_capturing()
     state = None if t.is_inference() or (capturing and t.device == device) else (t._version, t.data_ptr())
-    hit = None if state is None else _prep_cache.get(t, {}).get(key)
+    made_here = None if state is None else _prep_cache.get(t)
+    hit = None if made_here is None else made_here.get(key)
     if hit is not None and hit[0] == state:
         _, conv, made_on, made = hit
         if on_gpu and not capturing and made_on != _stream_ptr(device):
@@ -80,8 +83,9 @@ def _prep_operand(t: torch.Tensor, device, dtype) -> torch.Tensor:
         _prep_move_warned = True
         log.warning("Sage HIP path: a norm weight / rotary table lives on %s, the tensors on %s; it is copied over once "
                     "per tensor (keep them on the device to avoid even that)", t.device, device)
-    with torch.inference_mode(False), torch.no_grad():  # (made in inference mode it could not be remembered in turn)
-        conv = t.detach().to(device=device, dtype=dtype).contiguous()
+    # (made in inference mode a conversion could not be remembered in turn; entered only there, a context costs 2 us)
+    with torch.inference_mode(False) if torch.is_inference_mode_enabled() else nullcontext():
+        conv = t.detach().to(device=device, dtype=through or dtype).to(dtype).contiguous()
     if state is not None and not capturing:
         stream = torch.cuda.current_stream(device) if on_gpu else None
         _prep_cache.setdefault(t, {})[key] = (state, conv, stream and stream.cuda_stream, stream and stream.record_event())
@@ -512,12 +516,12 @@ def _proj_operands(proj_weight: torch.Tensor, proj_bias: torch.Tensor | None, de
     D = 128
     if tuple(proj_weight.shape) != (D, D):
         raise ValueError(f"proj_weight must be [{D}, {D}]")
-    w = _prep_operand(_prep_operand(proj_weight, device, dtype), device, torch.float32)
+    w = _prep_operand(proj_weight, device, torch.float32, through=dtype)
     if proj_bias is None:
         return w, None
     if proj_bias.numel() != D:
         raise ValueError(f"proj_bias must hold {D} values")
-    return w, _prep_operand(_prep_operand(proj_bias, device, dtype), device, torch.float32)
+    return w, _prep_operand(proj_bias, device, torch.float32, through=dtype)
 
 
 def sla_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, keep: int, proj_weight: torch.Tensor,

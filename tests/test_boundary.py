@@ -363,6 +363,21 @@ def test_prep_operands_in_inference_mode():
     assert not half.requires_grad and not back.requires_grad and torch.equal(back, torch.ones(4))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_the_layers_values_are_rounded_to_the_tensors_dtype_and_remembered(dtype):
+    """The sparse-linear layer's weight and bias, in any dtype: fp32 with the values they have in the tensors' dtype, one look-up
+    and one conversion each."""
+    layer = torch.nn.Linear(128, 128, dtype=dtype)
+    w, b = sage_ops._proj_operands(layer.weight, layer.bias, "cpu", torch.bfloat16)
+    assert w.dtype == b.dtype == torch.float32 and not w.requires_grad
+    assert torch.equal(w, layer.weight.bfloat16().float()) and torch.equal(b, layer.bias.bfloat16().float())
+    again = sage_ops._proj_operands(layer.weight, layer.bias, "cpu", torch.bfloat16)
+    assert again[0] is w and again[1] is b
+    w16 = sage_ops._proj_operands(layer.weight, None, "cpu", torch.float16)[0]  # (the other half type is a conversion of its own)
+    assert torch.equal(w16, layer.weight.half().float())
+    assert all(len(sage_ops._prep_cache[p]) == n for p, n in ((layer.weight, 2), (layer.bias, 1)))
+
+
 def test_one_read_settings_and_the_occupancy_cache_without_gpu():
     """``ksana_sage_configure`` validates and stores its settings without touching a device; the launchers' cache of
     resident-workgroup counts keeps one entry per kernel instantiation (two instantiations of one template have the same
