@@ -9,6 +9,12 @@ from ksanadit_amd import sage_ops
 pytestmark = pytest.mark.gpu
 
 
+def _spoil(q, ws):
+    """What the allocator hands out next, a result and a workspace, holds neither a finished result nor an earlier call's codes."""
+    mem = torch.full_like(q, float("nan")), torch.full((ws.layout.total_bytes,), 0xFF, dtype=torch.uint8, device=q.device)
+    del mem
+
+
 # (B, Hq, Hkv, Lq, Lk): all quantizers in one launch, two stages with one and two tiles a workgroup, K's and V's chunks meeting
 @pytest.mark.parametrize("B,Hq,Hkv,Lq,Lk", [(5, 64, 32, 900, 230), (5, 4, 2, 700, 1500), (5, 24, 24, 300, 3000), (5, 8, 8, 200, 17000)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -23,8 +29,8 @@ def test_same_bits_as_with_everything_quantized(hip_device, B, Hq, Hkv, Lq, Lk, 
         kw = dict(k_lens=torch.tensor(k_lens, dtype=torch.int32, device=hip_device))
         if q_lens is not None:
             kw["q_lens"] = torch.tensor(q_lens, dtype=torch.int32, device=hip_device)
+        _spoil(q, ws)
         got = sage_ops.sageattn(q, k, v, **kw)
-        torch.empty_like(got).fill_(float("nan"))  # what the allocator hands out next is not a finished result
         assert torch.equal(got, sage_ops.attn_fwd(ws, torch.empty_like(q), **kw)), (k_lens, q_lens)
 
 
@@ -46,6 +52,7 @@ def test_counts_of_any_value_are_clamped(hip_device, B, Hq, Hkv, Lq, Lk):
         as_given, clamped = ([torch.tensor(x, dtype=torch.int32, device=hip_device) for x in pair] for pair in ((k_lens, q_lens), within))
         want = sage_ops.attn_fwd(ws, torch.empty_like(q), k_lens=clamped[0], q_lens=clamped[1])
         for lens in (as_given, clamped):
+            _spoil(q, ws)
             assert torch.equal(sage_ops.sageattn(q, k, v, k_lens=lens[0], q_lens=lens[1]), want), (k_lens, q_lens)
         assert torch.equal(sage_ops.attn_fwd(ws, torch.empty_like(q), k_lens=as_given[0], q_lens=as_given[1]), want), (k_lens, q_lens)
         for b, (n_k, n_q) in enumerate(zip(*within)):
