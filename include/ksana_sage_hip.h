@@ -76,10 +76,11 @@ extern "C" {
                                       /* folded into q, where o has its type and the sizes make it pay, the attention      */
                                       /* kernel then quantizes Q itself and the two areas stay unwritten.  Same bits.      */
 
-#define KSANA_SAGE_FLAG_WS_UNSTORED 64 /* ksana_sage_forward* only, with KSANA_SAGE_FLAG_Q_UNSTORED: the caller reads nothing  */
+#define KSANA_SAGE_FLAG_WS_UNSTORED 64 /* ksana_sage_forward* only, with KSANA_SAGE_FLAG_Q_UNSTORED: the caller reads nothing */
                                        /* from the workspace afterwards and o overlaps none of q, k, v.  A call that          */
                                        /* ksana_sage_forward_scratch gives no bytes for then runs in one launch that touches  */
-                                       /* no workspace.  Same bits.                                                           */
+                                       /* no workspace.  In other calls without a folded step, blocks of 128 query rows or    */
+                                       /* 64 keys that q_lens and k_lens leave out may stay unquantized.  Same bits.          */
 
 typedef struct ksana_sage_shape {
   int32_t B;   /* batch                                                     */
@@ -178,13 +179,13 @@ const char* ksana_sage_last_error(void);
  *     one-read kernel when the shape allows ("" = neither).  First value: the environment variable
  *     KSANA_SAGE_ONE_READ, default "v"; the environment is read once, when the first call needs it.  K quantized by a
  *     kernel of its own with a folded norm / rotation step always tries the one-read kernel.
- *     Whole calls (ksana_sage_forward*) without V smoothing and without the Wan step quantize Q, K and V together. Up
+ *     Whole calls (ksana_sage_forward*) without V smoothing and without the Wan step quantize Q, K and V together.  Up
  *     to 64 chunks of 256 keys and 192 MB of K and V two launches read K and V twice whatever is set here, and nobody
  *     waits.  Beyond that, up to 160 chunks and without a folded step, "v" also selects one launch in which K's and
  *     V's chunks meet: both are then read once, with or without a "k".  With the Wan step and its norms of q and k,
- *     "v" also selects one launch for K's and V's one-read kernels where the chip works through the chunks of 256 keys
- *     (K's and V's of all heads) in less than 1.5 or in 2 to 7 rounds, and a launch each otherwise.  Without "v", and for all other whole calls, the letters select the separate
- *     kernels as for the stage-wise entry points.
+ *     "v" also selects one launch for K's and V's one-read kernels where the chip works through the chunks of 256
+ *     keys (K's and V's of all heads) in less than 1.5 or in 2 to 7 rounds, and a launch each otherwise.  Without "v",
+ *     and for all other whole calls, the letters select the separate kernels as for the stage-wise entry points.
  *   wait_ticks: KSANA_SAGE_KEEP = leave as it is; otherwise the bound, in 10 ns ticks, on a workgroup's wait for its
  *     head's statistic.  First value: KSANA_SAGE_WAIT_TICKS, default 200000 (2 ms; the kernels run 0.1 - 0.5 ms).
  *     A positive bound that expires makes the library take the two-pass kernels on that GPU from the next call on (the
@@ -368,15 +369,18 @@ int ksana_sage_attn_fwd_varlen(void* workspace, void* o, int dtype, const int64_
 /* How ksana_sage_attn_fwd cuts `shape` on the current device (dense, non-causal calls): the 256-row query blocks
  * numbered *first_workgroup and up - numbering (b * Hq + h) * ceil(Lq/256) + block - have their key loop cut into
  * *runs runs; *runs == 0 means no cut.  For tools that want to mirror the kernel's rounding exactly (the test
- * emulation does); no counterpart in the reference. */
+ * emulation does); no counterpart in the reference.  Not told here: without a cut, piecewise-linear exp2, tile skip and a
+ * forced shape, calls in 128-row workgroups share out the keys of a head's last block of at most 32 (33 .. 64) rows: 4 (2)
+ * runs of ceil(tiles / 4 (2)) key tiles, where the batch entry counts more than 1024 keys. */
 int ksana_sage_attn_key_split(const ksana_sage_shape* shape, int* first_workgroup, int* runs);
 
 /* The sparse-linear backend's whole call (sage_sla.py:100-292): quantize q, k and v, the block map that keeps the `keep` key
  * blocks of largest pooled score per 128 query rows, attention over the kept blocks, and the linear branch with the block's
- * layer - o = sparse + (phi(q) kv) W^T / (1e-5 + phi(q) . sum phi(k)) + bias - in five launches.  The same results as
- * ksana_sage_quant_qk_pooled, ksana_sage_quant_v, ksana_sage_sla_block_map, ksana_sage_attn_fwd_masked and
- * ksana_sage_sla_linear in turn, the linear branch's row sums up to their order.  Head size 128, Hq == Hkv, Lq == Lk <= 65536, o
- * overlaps none of q, k, v; proj_weight (fp32 [128][128], out x in) and proj_bias (fp32 [128]) may be NULL. */
+ * layer - o = sparse + (phi(q) kv) W^T / (1e-5 + phi(q) . sum phi(k)) + bias - in four launches, five from 64 chunks of 256
+ * keys on, and one more with keep = 0.  The same bits as ksana_sage_quant_qk_pooled, ksana_sage_quant_v,
+ * ksana_sage_sla_block_map, ksana_sage_attn_fwd_masked and ksana_sage_sla_linear in turn.  Head size 128, Hq == Hkv,
+ * Lq == Lk <= 65536, o overlaps none of q, k, v; proj_weight (fp32 [128][128], out x in) and proj_bias (fp32 [128]) may be
+ * NULL. */
 int ksana_sage_sla_forward_bytes(const ksana_sage_shape* shape, uint64_t* bytes);
 int ksana_sage_sla_forward(const void* q, const void* k, const void* v, void* o, int dtype, const int64_t q_strides[4],
                            const int64_t k_strides[4], const int64_t v_strides[4], const int64_t o_strides[4],
