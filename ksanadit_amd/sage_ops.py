@@ -49,7 +49,7 @@ def _usable(t: torch.Tensor) -> torch.Tensor:
     return t.contiguous()
 
 
-_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype, through): ((version, address), converted, made on, made)}
+_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype, through): ((version, address), converted, made on, made, its memory)}
 _prep_move_warned = False
 
 
@@ -58,10 +58,12 @@ def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
     ``through`` first, if given), contiguous.
     A conversion is remembered per source tensor (and redone once that tensor has been written to or has been given other
     memory, as ``p.data = ...`` does), so a caller that keeps its weights in another dtype - or on the host - pays for it
-    once, not in every attention call; a transfer from another device is logged the first time.  Tensors made in inference
-    mode keep no count of their writes: they are converted in every call.  A call on another stream than the conversion's
-    waits for it.  A graph records a conversion of its own: one made before may be gone when it is replayed, and its own has no
-    values before that (a tensor on the host cannot be read by a graph: there the one made before it is taken)."""
+    once, not in every attention call; a transfer from another device is logged the first time.  What was converted is held as
+    long as the conversion is: its address cannot come back with other values.  Writes that autograd does not count
+    (``p.data += ...``) are not noticed.  Tensors made in inference mode keep no count of their writes: they are converted
+    in every call.  A call on another stream than the conversion's waits for it.  A graph records a conversion of its own: one
+    made before may be gone when it is replayed, and its own has no values before that (a tensor on the host cannot be read by
+    a graph: there the one made before it is taken)."""
     global _prep_move_warned
     device = torch.device(device)
     if t.device == device and t.dtype == dtype and through in (None, dtype) and t.is_contiguous():
@@ -73,7 +75,7 @@ def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
     made_here = None if state is None else _prep_cache.get(t)
     hit = None if made_here is None else made_here.get(key)
     if hit is not None and hit[0] == state:
-        _, conv, made_on, made = hit
+        _, conv, made_on, made, _ = hit
         if on_gpu and not capturing and made_on != _stream_ptr(device):
             stream = torch.cuda.current_stream(device)
             stream.wait_event(made)
@@ -88,7 +90,7 @@ def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
         conv = t.detach().to(device=device, dtype=through or dtype).to(dtype).contiguous()
     if state is not None and not capturing:
         stream = torch.cuda.current_stream(device) if on_gpu else None
-        _prep_cache.setdefault(t, {})[key] = (state, conv, stream and stream.cuda_stream, stream and stream.record_event())
+        _prep_cache.setdefault(t, {})[key] = (state, conv, stream and stream.cuda_stream, stream and stream.record_event(), t.detach())
     return conv
 
 

@@ -349,6 +349,34 @@ def test_prep_operands_given_other_memory_are_converted_anew():
     assert torch.equal(sage_ops._prep_operand(p, "cpu", torch.float32), torch.full((4,), 3.0))
 
 
+def test_prep_operands_hold_the_memory_they_were_made_from():
+    """A weight swapped twice between two calls could otherwise get the first swap's memory back from the allocator, with
+    other values at the remembered address.  Held until the conversion is redone, or the weight is gone."""
+    import weakref
+
+    import numpy as np
+
+    from ksanadit_amd import sage_ops
+
+    def memory(value):
+        a = np.full(64, value, dtype=np.float16)
+        return torch.from_numpy(a), weakref.ref(a)
+
+    first, first_alive = memory(2.0)
+    p = torch.nn.Parameter(torch.ones(64, dtype=torch.float16))
+    p.data = first
+    del first
+    sage_ops._prep_operand(p, "cpu", torch.float32)
+    second, second_alive = memory(3.0)
+    p.data = second
+    del second
+    assert first_alive() is not None
+    assert torch.equal(sage_ops._prep_operand(p, "cpu", torch.float32), torch.full((64,), 3.0))
+    assert first_alive() is None and second_alive() is not None
+    del p
+    assert second_alive() is None
+
+
 def test_prep_operands_in_inference_mode():
     """Tensors made in inference mode count no writes; conversions of other tensors made there are remembered."""
     p = torch.nn.Parameter(torch.ones(4))
