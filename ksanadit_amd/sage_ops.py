@@ -49,7 +49,7 @@ def _usable(t: torch.Tensor) -> torch.Tensor:
     return t.contiguous()
 
 
-_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype, through): ((version, address), converted, made on, made, its memory)}
+_prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype, through): ((version, address), {stream: converted}, its memory)}
 _prep_move_warned = False
 
 
@@ -61,9 +61,9 @@ def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
     once, not in every attention call; a transfer from another device is logged the first time.  What was converted is held as
     long as the conversion is: its address cannot come back with other values.  Writes that autograd does not count
     (``p.data += ...``) are not noticed.  Tensors made in inference mode keep no count of their writes: they are converted
-    in every call.  A call on another stream than the conversion's waits for it.  A graph records a conversion of its own: one
-    made before may be gone when it is replayed, and its own has no values before that (a tensor on the host cannot be read by
-    a graph: there the one made before it is taken)."""
+    in every call.  Every stream makes and keeps a conversion of its own, which its other work comes after.  (One for all
+    streams takes an event per conversion, 15-30 us each on the way of the first call.)  So does a graph: one made before may be gone when it is
+    replayed, and its own has no values before that (a tensor on the host cannot be read by a graph: there one made before it is taken)."""
     global _prep_move_warned
     device = torch.device(device)
     if t.device == device and t.dtype == dtype and through in (None, dtype) and t.is_contiguous():
@@ -72,15 +72,15 @@ def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
     on_gpu = device.type == "cuda"
     capturing = on_gpu and torch.cuda.is_current_stream_capturing()
     state = None if t.is_inference() or (capturing and t.device == device) else (t._version, t.data_ptr())
+    stream = _stream_ptr(device) if on_gpu else None
     made_here = None if state is None else _prep_cache.get(t)
     hit = None if made_here is None else made_here.get(key)
     if hit is not None and hit[0] == state:
-        _, conv, made_on, made, _ = hit
-        if on_gpu and not capturing and made_on != _stream_ptr(device):
-            stream = torch.cuda.current_stream(device)
-            stream.wait_event(made)
-            conv.record_stream(stream)
-        return conv
+        conv = hit[1].get(stream)
+        if conv is None and capturing:
+            conv = next(iter(hit[1].values()))
+        if conv is not None:
+            return conv
     if t.device != device and not _prep_move_warned:
         _prep_move_warned = True
         log.warning("Sage HIP path: a norm weight / rotary table lives on %s, the tensors on %s; it is copied over once "
@@ -89,8 +89,10 @@ def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
     with torch.inference_mode(False) if torch.is_inference_mode_enabled() else nullcontext():
         conv = t.detach().to(device=device, dtype=through or dtype).to(dtype).contiguous()
     if state is not None and not capturing:
-        stream = torch.cuda.current_stream(device) if on_gpu else None
-        _prep_cache.setdefault(t, {})[key] = (state, conv, stream and stream.cuda_stream, stream and stream.record_event(), t.detach())
+        if hit is not None and hit[0] == state:
+            hit[1][stream] = conv
+        else:
+            _prep_cache.setdefault(t, {})[key] = (state, {stream: conv}, t.detach())
     return conv
 
 

@@ -283,7 +283,7 @@ def test_prep_argument_errors(hip_device):
 
 
 def test_a_converted_weight_is_awaited_on_another_stream(hip_device):
-    """The conversion belongs to the stream it was made on; a call on another stream that finds it waits for it."""
+    """The conversion belongs to the stream it was made on: a call on another stream reads none that may not have run."""
     src = torch.arange(4096, dtype=torch.float64, device=hip_device)
     first, second = torch.cuda.Stream(), torch.cuda.Stream()
     src.float().clone()  # (kernels are loaded at their first use)
