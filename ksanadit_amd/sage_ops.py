@@ -50,6 +50,7 @@ def _usable(t: torch.Tensor) -> torch.Tensor:
 
 
 _prep_cache = WeakTensorKeyDictionary()  # source tensor -> {(device, dtype, through): ((version, address), {stream: converted}, its memory)}
+_PREP_STREAMS = 8  # conversions kept of one tensor at a time (a program may make streams without end)
 _prep_move_warned = False
 
 
@@ -61,9 +62,10 @@ def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
     once, not in every attention call; a transfer from another device is logged the first time.  What was converted is held as
     long as the conversion is: its address cannot come back with other values.  Writes that autograd does not count
     (``p.data += ...``) are not noticed.  Tensors made in inference mode keep no count of their writes: they are converted
-    in every call.  Every stream makes and keeps a conversion of its own, which its other work comes after.  (One for all
-    streams takes an event per conversion, 15-30 us each on the way of the first call.)  So does a graph: one made before may be gone when it is
-    replayed, and its own has no values before that (a tensor on the host cannot be read by a graph: there one made before it is taken)."""
+    in every call.  Every stream makes and keeps a conversion of its own, which its other work comes after (one for all
+    streams takes an event per conversion, 15-30 us each on the way of the first call).  So does a graph: one made before may be
+    gone when it is replayed, and its own has no values before that (a tensor on the host cannot be read by a graph: there one
+    made before it is taken)."""
     global _prep_move_warned
     device = torch.device(device)
     if t.device == device and t.dtype == dtype and through in (None, dtype) and t.is_contiguous():
@@ -78,7 +80,7 @@ def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
     if hit is not None and hit[0] == state:
         conv = hit[1].get(stream)
         if conv is None and capturing:
-            conv = next(iter(hit[1].values()))
+            conv = list(hit[1].values())[-1]
         if conv is not None:
             return conv
     if t.device != device and not _prep_move_warned:
@@ -90,6 +92,8 @@ def _prep_operand(t: torch.Tensor, device, dtype, through=None) -> torch.Tensor:
         conv = t.detach().to(device=device, dtype=through or dtype).to(dtype).contiguous()
     if state is not None and not capturing:
         if hit is not None and hit[0] == state:
+            if len(hit[1]) >= _PREP_STREAMS:
+                hit[1].pop(list(hit[1])[0], None)
             hit[1][stream] = conv
         else:
             _prep_cache.setdefault(t, {})[key] = (state, {stream: conv}, t.detach())

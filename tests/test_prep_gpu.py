@@ -299,6 +299,24 @@ def test_a_converted_weight_is_awaited_on_another_stream(hip_device):
     assert torch.equal(got, src.float())
 
 
+def test_conversions_of_many_streams_are_bounded(hip_device):
+    """Every stream has its own; the oldest goes when there are more streams than are kept, and all go with the values."""
+    src = torch.arange(4096, dtype=torch.float64, device=hip_device)
+    streams = [torch.cuda.Stream() for _ in range(sage_ops._PREP_STREAMS + 3)]
+    for add in (0.0, 1.0):
+        src += add
+        torch.cuda.synchronize()
+        for stream in streams + streams[:2]:
+            with torch.cuda.stream(stream):
+                got = sage_ops._prep_operand(src, hip_device, torch.float32)
+                assert sage_ops._prep_operand(src, hip_device, torch.float32) is got
+            stream.synchronize()
+            assert torch.equal(got, src.float())
+            (kept,) = sage_ops._prep_cache[src].values()
+            assert len(kept[1]) <= sage_ops._PREP_STREAMS
+    assert len({stream.cuda_stream for stream in streams}) > sage_ops._PREP_STREAMS
+
+
 @pytest.mark.parametrize("warm", [False, True])
 def test_a_weight_converted_under_capture_is_the_graphs_own(hip_device, warm):
     """A conversion that a graph records has no values before a replay: calls outside the graph do not find it.  Replays convert
