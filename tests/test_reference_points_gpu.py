@@ -100,3 +100,21 @@ def test_shapes_and_variants_agree_on_long_rows(hip_device, lifted):
             for kw in ({"wg_waves": 4}, {"wg_waves": 4, "tile_skip": True}, {"block_mask": ones}, {"block_mask": ones, "wg_waves": 8})]
     for other in outs[1:]:
         assert torch.equal(outs[0], other)
+
+
+# points that move by the scores up to the line and across it, and by the codes after calm tiles; calm by the line
+@pytest.mark.parametrize("lifted", [[1, 2, 3, 505, 511, 529, 538], [1, 2, 3, 100, 540]])
+@pytest.mark.parametrize("mode", ["dense4", "dense8", "masked", "causal"])
+def test_very_long_rows_go_over_to_the_codes(hip_device, lifted, mode):
+    """The tile skip's loop looks at the scores in every step: the same points, the same bits."""
+    tiles, tail = 545, 9
+    Lk = 64 * (tiles - 1) + tail
+    Lq, H = (Lk, 1) if mode == "causal" else (256, 136 if mode == "dense8" else 2)  # (136 blocks: nobody's keys are cut)
+    print(f"case {mode} lifted={lifted}", flush=True)
+    q, k, v = (t.to(hip_device).to(torch.bfloat16).expand(1, -1, H, -1).contiguous() for t in _inputs(Lq, Lk, 128, lifted, 6))
+    ws = _quantized(q, k, v, hip_device)
+    kw = {"masked": {"block_mask": torch.ones((2, tiles), dtype=torch.int8)}, "causal": {"causal": True}}.get(mode, {"wg_waves": int(mode[-1]) if mode[-1].isdigit() else 0})
+    if mode == "dense8":
+        assert sage_ops.key_split_plan(ws) is None
+    default, by_scores = (sage_ops.attn_fwd(ws, torch.empty_like(q), tile_skip=skip, **kw) for skip in (False, True))
+    assert torch.isfinite(default).all() and torch.equal(default, by_scores)
