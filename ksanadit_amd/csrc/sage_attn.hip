@@ -64,11 +64,8 @@ constexpr int kMaxKeyTiles = 4096;           // K scales of one head are kept in
 constexpr int kShortKeyTiles = 16;           // with at most this many key tiles (Lk <= 1024) nobody's keys are cut into runs
 // The first kSample tiles of rows that take part in more than kSampleFrom are looked at before the first point is set (see first_point)
 constexpr int kSampleFrom = 32, kSample = 4;
-constexpr float kLightSpread = 2.5f;
+constexpr float kLightSpread = 1.5f;
 constexpr int kLightRows = 8;
-// Waves that look for their points by the scores go over to the codes at a round from tile kCalmFrom on that kCalm tiles without a
-// move lead up to (see look_ahead)
-constexpr int kCalmFrom = 512, kCalm = 16;
 constexpr int kShortMaxKeyTiles = 2048;      // the most key tiles a dense 4-wave workgroup can hold scales for
 
 #pragma clang diagnostic push
@@ -743,7 +740,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // kLightRows of the 32 rows (scores with a standard deviation of 1.44 octaves, one of the exponent: 99 % of the waves; 2.0: 45 %;
   // 2.4: 10 %).  Elsewhere points would go on moving all the same, and small probabilities would lose the octaves.
   // Error against 64 bits over the whole result, from the first tile / like this: flat 0.03916 / 0.03918.
-  float m_first = -INFINITY, m_least = INFINITY, m_tile0 = -INFINITY;
+  float m_first = -INFINITY, m_tile0 = -INFINITY;
   bool sampled = false;  // (wave-uniform)
   // one more tile's scores and K scale
   auto first_point = [&](const v16i (&s)[2], float ks) __attribute__((always_inline)) {
@@ -752,7 +749,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(m_half), __float_as_uint(m_half), false, false);
     const float m_tile = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
     m_tile0 = m_first == -INFINITY ? m_tile : m_tile0;
-    m_least = fminf(m_least, m_tile);
     m_first = fmaxf(m_first, m_tile);  // (scores that are not numbers are left to their tile's step)
   };
   if constexpr (kSparse && kW == 8) {
@@ -786,7 +782,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       }
     }
   }
-  const bool light = sampled && __popcll(__ballot(m_first - m_least > kLightSpread)) <= 2 * kLightRows;  // (a row is in two lanes)
+  const bool light = sampled && __popcll(__ballot(m_first - m_tile0 > kLightSpread)) <= 2 * kLightRows;  // (a row is in two lanes)
   // (with the wait: a bare barrier lets the tile's last reads be on their way still when a wave without rows, which has nothing
   // else to do, requests the tile that goes into their slot)
   if constexpr (kSlotZeroSoon) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -809,17 +805,12 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   //     533, 24 heads of 27280 tokens 4640 / 4400, a radial mask on 40 heads of 37632 5480 / 5170, 51 of 512 tiles kept on 40
   //     heads of 32760 1864 / 1824, causal 8191 tokens of 32 heads 326 / 318; without first points from four tiles 0-1 %
   //     slower than by the scores, and with outliers (points that move in 11 % of the steps) 4 %.
-  // By the codes where points are not expected to move: from the start (light), or once they have become rare.  New maxima of
-  // unordered keys thin out as 1 / tile: with outliers 16 % of a wave's steps over the first 256 tiles, 4.2 % in tiles 256 to 511, 2.3 %
-  // up to 1023, where about 5 % is what the codes' dearer moves can bear.  us per call, by the scores throughout / codes after 16
-  // calm tiles from tile 512 on: 75600 tokens of 40 heads with outliers 50990 / 49980, 32760 (512 tiles) the same; from any tile
-  // on after 32 calm ones 1.02 x at 75600, but 0.995 x at 32760 and 16384.  The row's own decision is move_point's in both, and so are the bits.
+  // By the codes where points are not expected to move (light).  The row's own decision is move_point's in both, and so are the bits.
   float sc = 0.0f, xc = 0.0f;           // scale of the coming tile, its exponent constant
   // factor a tile's point move puts on everything before it, and (wave-uniform) whether there is one: of even tiles and
   // of odd ones (step j applies tile j-1's and then finds tile j+1's)
   float alpha_even = 1.0f, alpha_odd = 1.0f;
   int moved_even = 0, moved_odd = 0;
-  int moved_at = 0;                     // (wave-uniform) by the scores: the last tile that moved a point
   bool nothing = false;                 // (wave-uniform) every probability of the coming tile converts to zero
   // mx: the lane's maximum over the scores of tile jn, the coming one
   auto look_ahead = [&](int jn, int mx, float& alpha, int& moved) __attribute__((always_inline)) {
@@ -837,7 +828,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       if (jn < n_tiles && mine_at(jn)) {
         alpha = move_point<kPwlExp>(mx, sc, mneg, qs, m_run, x_base);
         moved = 1;
-        moved_at = jn;
         xc = x_base + mneg;
       }
     }
@@ -893,11 +883,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   int ks_off = (int)(reinterpret_cast<const uint8_t*>(s_ks) - smem) + 4;
   pin(ks_off);
   constexpr int kHowScores = 0, kHowCodes = 1, kHowEither = 2;
-  int by_scores = 1;  // (wave-uniform) which of the two the steps after the rounds take
   auto tile_step = [&](auto at, auto how, int j, v16i (&s_cur)[2], v16i (&s_nxt)[2], v8i& pf_prev, v8i& pf, float& alpha, int& moved) {
     constexpr int kAt = decltype(at)::value;
-    // by the codes, by the scores, or as by_scores says
-    constexpr bool kCodes = decltype(how)::value != kHowScores, kScores = decltype(how)::value != kHowCodes;
+    // kCodes, or by the scores; kEither: by the codes, and factors left by steps before it
+    constexpr bool kCodes = decltype(how)::value == kHowCodes || decltype(how)::value == kHowEither;
+    constexpr bool kFactors = decltype(how)::value != kHowCodes;
     const uint8_t* kst = k_slot(kAt >= 0 ? kAt + 1 : j + 1);
     const uint8_t* vst = v_slot(kAt >= 0 ? kAt - 1 : j - 1);
     auto k_frag = [&](int i) { return *reinterpret_cast<const v4i*>(kst + (((i & 1) * 4 + (i >> 1)) * 64 + lane) * 16); };
@@ -908,7 +898,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     };
     float sum;
     auto tile_before = [&]() __attribute__((always_inline)) {
-      if constexpr (kScores) {
+      if constexpr (kFactors) {
         if (moved != 0) scale_o(alpha);  // wave-uniform
         moved = 0;
       }
@@ -994,7 +984,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       if (!skip) w = pack4(s_cur[1][4 * dt], s_cur[1][4 * dt + 1], s_cur[1][4 * dt + 2], s_cur[1][4 * dt + 3], scp, cp);
       pin(w);
       pf[4 + dt] = w;
-      if constexpr (kScores) {
+      if constexpr (!kCodes) {
         // one chain over the 32 scores, two per instruction
         const v16i& blk = s_nxt[dt >> 1];
         const int r0 = (dt & 1) * 8;
@@ -1026,9 +1016,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     // exponent of key r: x = sc*dot - m_run + shift, with the magic folded into the constant
     // (which is therefore off by at most ~1.5 integer steps of the dot product)
     xc = x_base - kMagicVal * sc;
-    if constexpr (kScores) {
-      if (!kCodes || by_scores != 0) look_ahead(j + 1, mx, alpha, moved);
-    }
+    if constexpr (!kCodes) look_ahead(j + 1, mx, alpha, moved);
     // after this barrier: K tile j+2 and V^T tile j are visible to every wave, and nobody reads their predecessors any
     // more (after a group's: K tiles up to j+5, V^T tiles up to j+3, the ones the next group reads)
     if constexpr (kAt < 0 || Shape::kGroup == 1) tile_barrier();
@@ -1046,9 +1034,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       };
       auto rounds = [&](auto how) {
         for (; j + kStages <= n_plain; j += kStages) {
-          if constexpr (decltype(how)::value == kHowScores) {
-            if (j >= kCalmFrom && j - moved_at > kCalm) break;  // (no factor is left to be applied, then)
-          }
           two(how, std::integral_constant<int, 0>{});
           two(how, std::integral_constant<int, 2>{});
           if constexpr (kStages == 8) {
@@ -1061,7 +1046,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       // (one after the other, the second with nothing left to do, and not one or the other: joined behind the two, their
       // accumulators cost a hundred spilled registers)
       if (__builtin_amdgcn_readfirstlane(!light) != 0) rounds(std::integral_constant<int, kHowScores>{});
-      by_scores = __builtin_amdgcn_readfirstlane(!light && j + kStages > n_plain);
       rounds(std::integral_constant<int, kHowCodes>{});
     }
     using Last = std::integral_constant<int, kUnrolled ? kHowEither : kHowScores>;
