@@ -62,10 +62,6 @@ struct WgShape {
 constexpr int kSparseMaxKeyTiles4 = 2048;    // 4-wave workgroups keep their tile list as 16-bit entries so that two fit a compute unit
 constexpr int kMaxKeyTiles = 4096;           // K scales of one head are kept in LDS: Lk <= 262144
 constexpr int kShortKeyTiles = 16;           // with at most this many key tiles (Lk <= 1024) nobody's keys are cut into runs
-// The first kSample tiles of rows that take part in more than kSampleFrom are looked at before the first point is set (see first_point)
-constexpr int kSampleFrom = 32, kSample = 4;
-constexpr float kLightSpread = 1.5f;
-constexpr int kLightRows = 8;
 constexpr int kShortMaxKeyTiles = 2048;      // the most key tiles a dense 4-wave workgroup can hold scales for
 
 #pragma clang diagnostic push
@@ -223,7 +219,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         q_raw[2 * s + 1] = *reinterpret_cast<const uint4*>(qrow + 32 * s + 8);
       }
     }
-  } else if (active && !shared) {
+  } else if (active && !(shared && p.q_rows.ptr != nullptr)) {
     const int8_t* qrow = p.q_i8 + ((int64_t)bh * p.lq_pad + q0 + l32) * kD + 16 * hh;
 #pragma unroll
     for (int s = 0; s < kG; ++s) qf[s] = *reinterpret_cast<const v4i*>(qrow + 32 * s);
@@ -236,10 +232,27 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.0f;
   // reference point of query l32 in the log2 domain (its "running maximum"), and what the steps read it as: the
-  // exponent's constant part (base -inf: the probabilities of a row without a point are zeros)
-  float m_run = -INFINITY, x_base = -INFINITY;
-  float l_run = 0.0f;  // the row's sum, see row_sum_ones (no probability may be NaN there: move_point sees to it)
-  const v4i ones = row_sum_ones(lane);
+  // exponent's constant part and the score above which the point has to move
+  // (base -inf: the probabilities of a row without a point are zeros)
+  float m_run = -INFINITY, x_base = -INFINITY, x_limit = -INFINITY;
+  // Row sums come from the matrix pipe too, of the SAME e4m3-rounded P the numerator uses.  The 16x16x128 instruction
+  // takes half the matrix cycles of the 32x32x64 one and a quarter of its accumulators; its B operand is P's register
+  // block read as 16 columns with four groups of 16 lanes stacked along the contraction: groups 0 and 2 hold the two
+  // halves of query (lane % 16)'s keys, groups 1 and 3 those of query 16 + (lane % 16).  A therefore carries ones
+  // (e4m3 1.0 = 0x38) where output row 4 g' .. 4 g' + 3 and group g agree in parity and zeros elsewhere: the lanes of
+  // group g' then find the sum of their own query in all four registers.  Only register 0 is read and rescaled.
+  // A zero of A meets the probabilities of the query 16 further, and zero times NaN is NaN: no probability may be one
+  // (move_point sees to it).
+  v4f lacc = {0.0f, 0.0f, 0.0f, 0.0f};
+  // eight registers on purpose: left as one value the compiler keeps a single copy and rebuilds
+  // the 8-register operand with seven moves in every step
+  v8i ones;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    int one4 = ((lane >> 2) & 1) == ((lane >> 4) & 1) ? 0x38383838 : 0;
+    pin(one4);
+    ones[r] = one4;
+  }
 
   // kept opaque so the 16 registers stay resident instead of being rebuilt from constants
   // (8 moves) at every tile
@@ -347,11 +360,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       // quarter as long.  us per call, whole / shared: 40 heads of 1560 tokens, where eight of the 520 workgroups start when the
       // others end, 67.9 / 56.8.  Errors against 64 bits are those of whole rows or below: 0.0383 / 0.0388 at N(0, 1),
       // 0.0289 / 0.0295 with outliers.
-      // (rows of its own: the main path's would have to be kept for this one, which comes after it, in scratch memory)
-      v4i qf[4];
-      float qs = 0.0f;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) qf[c] = v4i{0, 0, 0, 0};
       if (p.q_rows.ptr != nullptr) {
         uint4 raw[8];
         const uint16_t* qrow = p.q_rows.ptr + b * p.q_rows.sB + (int64_t)min(q0 + l32, p.Lq - 1) * p.q_rows.sL + h * p.q_rows.sH + 16 * hh;
@@ -361,11 +369,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
           if (q0 + l32 >= lq) raw[i] = make_uint4(0, 0, 0, 0);
         }
         quant_q_rows<DT, kG>(raw, p.q_premul, qf, qs);
-      } else if (active) {
-        const int64_t row = (int64_t)bh * p.lq_pad + q0 + l32;
-#pragma unroll
-        for (int c = 0; c < kG; ++c) qf[c] = *reinterpret_cast<const v4i*>(p.q_i8 + row * kD + 16 * hh + 32 * c);
-        qs = p.q_scale[row];
       }
       fill_scales();
       __syncthreads();
@@ -399,13 +402,13 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
         for (int r = 1; r < 16; ++r) top = max(max(top, s[0][r]), s[1][r]);
         float sc = qs * s_ks[j], mneg = -kMagicVal * sc;
-        const float alpha = move_point(top, sc, mneg, qs, m_run, x_base);
+        const float alpha = move_point(top, sc, mneg, qs, m_run, x_base, x_limit);
         if (j == j0 ? __any(alpha != alpha) : __any(alpha != 1.0f)) {
 #pragma unroll
           for (int dt = 0; dt < kG; ++dt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
-          l_run *= alpha;
+          lacc[0] *= alpha;
         }
         v8i pf = tile_probs(s, sc, x_base + mneg);
         if (n_last != 0) blank_probs(pf, hh, n_last);
@@ -413,7 +416,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int dt = 0; dt < kG; ++dt) oacc[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf[dt], pf, oacc[dt], 0, 0, 0, 0, 0, 0);
-        l_run += row_sum(ones, pf);
+        lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, lacc, 0, 0, 0, 0, 0, 0);
       }
       // every wave's accumulators in the ring, points and sums where the K scales were; then the waves of a row group finish a
       // quarter or half of its channels each
@@ -424,7 +427,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       for (int dt = 0; dt < kG; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) s_o[((wave * 4 + dt) * 16 + r) * 64 + lane] = oacc[dt][r];
-      if (hh == 0) s_ml[wave * 32 + l32] = make_float2(m_run, l_run);
+      if (hh == 0) s_ml[wave * 32 + l32] = make_float2(m_run, lacc[0]);
       __syncthreads();
       const int first = wave - run;  // the row group's first wave
       float weight[kW];
@@ -540,7 +543,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 #pragma unroll
     for (int c = 0; c < 8 / kW; ++c) {  // this wave's 1 KiB slices of the tile: slice c * kW + wave
       const int slice = c * kW + wave;
-      lds_copy16(scalar(src + (int64_t)jl * kTileBytes), (unsigned)(slice * 64 + lane) * 16, dst + slice * 1024);
+      lds_copy16(src + (int64_t)jl * kTileBytes, (unsigned)(slice * 64 + lane) * 16, dst + slice * 1024);
     }
   };
   auto copy_half = [&](const uint8_t* src, int tile, uint8_t* dst) {
@@ -559,8 +562,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // The key loop's own copies: descriptors over this workgroup's tiles, the lane's offset in a tile, the offset of the
   // tiles the next copies take (past the last tile it stays there, as above)
   auto tiles_from = [&](const void* base) {
-    const uint64_t a = reinterpret_cast<uint64_t>(scalar(reinterpret_cast<const uint8_t*>(base)));
-    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32) & 0xffff, __builtin_amdgcn_readfirstlane((p.nkb - tile0) * kTileBytes), 0x00020000};
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32) & 0xffff, (p.nkb - tile0) * kTileBytes, 0x00020000};
   };
   const v4i k_buf = tiles_from(k_src), v_buf = tiles_from(v_src);
   const unsigned lane_off = (unsigned)(wave * 64 + lane) * 16;
@@ -578,8 +581,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     using VSlot = std::integral_constant<int, (kStages + ((kTile + kAhead) & (kStages - 1))) * kTileBytes>;
     using KSlot = std::integral_constant<int, ((kTile + Shape::kAheadK) & (kStages - 1)) * kTileBytes>;
     if constexpr (kSparse) {
-      copy_to(VSlot{}, v_buf, __builtin_amdgcn_readfirstlane(ahead[0]) * kTileBytes);
-      copy_to(KSlot{}, k_buf, __builtin_amdgcn_readfirstlane(ahead[kWindow - 1]) * kTileBytes);
+      copy_to(VSlot{}, v_buf, ahead[0] * kTileBytes);
+      copy_to(KSlot{}, k_buf, ahead[kWindow - 1] * kTileBytes);
     } else {
       copy_to(VSlot{}, v_buf, off_v);  // first: it is awaited first
       copy_to(KSlot{}, k_buf, off_k);
@@ -638,26 +641,16 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // rest goes out after the wait as the copies of "steps -2 and -1" and is awaited by the loop's own count (8 key
   // tiles, 32760 queries, 40 heads: -1.2 %).
   constexpr bool kLateCopies = Shape::kGroup == 1;
-  // (unless the first points want K tiles 2 and 3 as well)
-  const bool late_copies = kLateCopies && (kPwlExp || (kSparse && kW == 8) || n_tiles <= kSampleFrom);  // uniform
-  if (!late_copies) {
 #pragma unroll
-    for (int t = 0; t < kAhead; ++t) copy_half(v_src, t, v_slot(t));
-  }
+  for (int t = 0; t < (kLateCopies ? 0 : kAhead); ++t) copy_half(v_src, t, v_slot(t));
 #pragma unroll
-  for (int t = 0; t < 2; ++t) copy_half(k_src, t, k_slot(t));
-  if (!late_copies) {
-#pragma unroll
-    for (int t = 2; t < Shape::kAheadK; ++t) copy_half(k_src, t, k_slot(t));
-  }
+  for (int t = 0; t < (kLateCopies ? 2 : Shape::kAheadK); ++t) copy_half(k_src, t, k_slot(t));
   fill_scales();
   if (__builtin_expect(own_q, 0)) quant_q_rows<DT, kG>(q_raw, p.q_premul, qf, qs);
-#pragma unroll
-  for (int i = 0; i < kG; ++i) pin(qf[i]);  // (one set of registers for the rows, wherever they came from)
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the set-up's loads and, older than some of them, the copies
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  if (late_copies) {
-    static_assert(!kLateCopies || Shape::kAheadK == kAhead + 2, "V^T tiles 0, 1 with K tiles 2, 3");
+  if constexpr (kLateCopies) {
+    static_assert(Shape::kAheadK == kAhead + 2, "V^T tiles 0, 1 with K tiles 2, 3");
 #pragma unroll
     for (int t = 0; t < kAhead; ++t) {
       copy_half(v_src, t, v_slot(t));
@@ -682,11 +675,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 
   auto scale_o = [&](float alpha) {
 #pragma unroll
-    for (int dt = 0; dt < kG; ++dt)
+    for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
-    // (a row that is not a number says so in its accumulators; its sum stays one, see refit)
-    l_run *= alpha != alpha ? 1.0f : alpha;
+    lacc[0] *= alpha;
   };
   // max over the 16 keys one S^T register block holds for query l32, as two independent chains
   auto max8 = [&](const v16i& blk, int r0) {
@@ -734,55 +726,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   auto has_qk = [](int i) { return i >= 0 && i < 8 && (i >> 1) < kG; };
 
   v16i s_a[2], s_b[2];
-  // The first reference point of a wave with many tiles.  Set by 64 keys alone, some row of a wave leaves it behind in 4 % of the
-  // steps on flat data, set by 256 in 0.6 %, for three more products of K and Q in the set-up.  Only where the scores are
-  // flat: where the maximum of kSample tiles is more than kLightSpread octaves above the first tile's in no more than
-  // kLightRows of the 32 rows (scores with a standard deviation of 1.44 octaves, one of the exponent: 99 % of the waves; 2.0: 45 %;
-  // 2.4: 10 %).  Elsewhere points would go on moving all the same, and small probabilities would lose the octaves.
-  // Error against 64 bits over the whole result, from the first tile / like this: flat 0.03916 / 0.03918.
-  float m_first = -INFINITY, m_tile0 = -INFINITY;
-  bool sampled = false;  // (wave-uniform)
-  // one more tile's scores and K scale
-  auto first_point = [&](const v16i (&s)[2], float ks) __attribute__((always_inline)) {
-    const float sct = qs * ks;
-    const float m_half = __builtin_fmaf(__int_as_float(lane_max(s)), sct, -kMagicVal * sct);
-    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(m_half), __float_as_uint(m_half), false, false);
-    const float m_tile = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    m_tile0 = m_first == -INFINITY ? m_tile : m_tile0;
-    m_first = fmaxf(m_first, m_tile);  // (scores that are not numbers are left to their tile's step)
-  };
-  if constexpr (kSparse && kW == 8) {
-    // (the wave's own tiles need not be in the ring)
-    int own[kSample] = {0, 0, 0, 0}, n_own = 0;
-    for (int jj = 0; jj < n_tiles && n_own <= kSampleFrom; ++jj)
-      if (mine_at(jj)) {
-#pragma unroll
-        for (int t = 0; t < kSample; ++t)
-          if (n_own == t) own[t] = jj;
-        ++n_own;
-      }
-    sampled = !kPwlExp && n_own > kSampleFrom;
-    if (sampled) {
-#pragma unroll
-      for (int t = 0; t < kSample; ++t) {
-        qk_tile<kG>(k_src + (int64_t)tile_of(own[t]) * kTileBytes, lane, qf, magic, s_b);
-        first_point(s_b, s_ks[own[t]]);
-      }
-    }
-  }
   qk_tile<kG>(k_slot(0), lane, qf, magic, s_a);
-  if constexpr (!kPwlExp && !(kSparse && kW == 8)) {
-    sampled = n_mine > kSampleFrom;
-    if (sampled) {
-      first_point(s_a, s_ks[0]);
-#pragma unroll
-      for (int t = 1; t < kSample; ++t) {
-        qk_tile<kG>(k_slot(t), lane, qf, magic, s_b);
-        first_point(s_b, s_ks[t]);
-      }
-    }
-  }
-  const bool light = sampled && __popcll(__ballot(m_first - m_tile0 > kLightSpread)) <= 2 * kLightRows;  // (a row is in two lanes)
   // (with the wait: a bare barrier lets the tile's last reads be on their way still when a wave without rows, which has nothing
   // else to do, requests the tile that goes into their slot)
   if constexpr (kSlotZeroSoon) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -791,86 +735,50 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
 
   // What a step needs to know about its tile before the first probability: the scale, the exponent's constant and
   // whether a reference point moves.  Worked out at the end of the step before, so that its chain of dependent
-  // operations runs under that step's last matrix instruction and the wait at the barrier.  Points move in few steps, and
-  // there are two ways to find out:
-  //   by the scores, a tile ahead: a lane compares its own half's maximum with the limit, and only when some lane of the
-  //     wave exceeds it are the halves joined and points, factors and constants formed anew (one wave-uniform branch
-  //     instead of eight vector operations and a transcendental in every step);
-  //   by the codes, a tile behind: a probability that has outgrown e4m3 becomes the NaN code, and the row sum of the tile,
-  //     which the matrix pipe forms at the head of the next step, a NaN - one comparison a step says whether any of the
-  //     wave's 2048 probabilities did.  The tile's scores are still there, so refit moves the points and forms the tile's
-  //     probabilities anew, ahead of their product with V.  That saves the maximum over 32 scores in every step, a
-  //     tenth of its vector instructions, and costs three times as much where a point does move (which the other waves of
-  //     the workgroup wait for).  us per call, by the scores / by the codes: 9001 tokens of 2 x 16 heads of 64 channels 554 /
-  //     533, 24 heads of 27280 tokens 4640 / 4400, a radial mask on 40 heads of 37632 5480 / 5170, 51 of 512 tiles kept on 40
-  //     heads of 32760 1864 / 1824, causal 8191 tokens of 32 heads 326 / 318; without first points from four tiles 0-1 %
-  //     slower than by the scores, and with outliers (points that move in 11 % of the steps) 4 %.
-  // By the codes where points are not expected to move (light).  The row's own decision is move_point's in both, and so are the bits.
+  // operations runs under that step's last matrix instruction and the wait at the barrier.  Points move in few steps
+  // (11 % of a wave's on outlier-ridden scores, 3 % on flat ones): a lane compares its own half's maximum with the
+  // limit, and only when some lane of the wave exceeds it are the halves joined and points, factors and constants
+  // formed anew (one wave-uniform branch instead of eight vector operations and a transcendental in every step).
+  // With the 16x16 row sums, same bits: 10.60 -> 10.35 ms at B=1 H=40 L=32760 with outliers, 11.44 -> 11.05 without
+  // (2045 cycles per step, from 2073, and 1843 with the loop unrolled and grouped; the chip runs at its power limit there,
+  // and fewer operations raise its clock too).
   float sc = 0.0f, xc = 0.0f;           // scale of the coming tile, its exponent constant
   // factor a tile's point move puts on everything before it, and (wave-uniform) whether there is one: of even tiles and
   // of odd ones (step j applies tile j-1's and then finds tile j+1's)
   float alpha_even = 1.0f, alpha_odd = 1.0f;
   int moved_even = 0, moved_odd = 0;
   bool nothing = false;                 // (wave-uniform) every probability of the coming tile converts to zero
-  // mx: the lane's maximum over the scores of tile jn, the coming one
-  auto look_ahead = [&](int jn, int mx, float& alpha, int& moved) __attribute__((always_inline)) {
+  auto look_ahead = [&](int jn, int mx, float ks, float& alpha, int& moved) {
+    sc = qs * ks;
     float mneg = -kMagicVal * sc;
-    bool stays;  // (NaN: no)
-    if constexpr (kPwlExp) {
-      stays = __builtin_fmaf(__int_as_float(mx), sc, mneg) <= m_run;
-    } else {
-      stays = __builtin_fmaf(__int_as_float(mx), sc, xc) <= kXAsk;
-      if constexpr (kSparse && kW == 8) stays = stays && m_run != -INFINITY;  // (whose first tile may be the other half's)
-    }
-    if (__ballot(!stays) != 0) {
+    const float m_half = __builtin_fmaf(__int_as_float(mx), sc, mneg);
+    moved = 0;
+    if (__ballot(!(m_half <= x_limit)) != 0) {  // (NaN counts as above)
       asm volatile("");  // (two branches on purpose: merged into one condition, the second is computed in every step)
       // (a tile this wave's mask row does not ask for, or that is not this loop's, leaves the points alone)
       if (jn < n_tiles && mine_at(jn)) {
-        alpha = move_point<kPwlExp>(mx, sc, mneg, qs, m_run, x_base);
+        alpha = move_point<kPwlExp>(mx, sc, mneg, qs, m_run, x_base, x_limit);
         moved = 1;
-        xc = x_base + mneg;
       }
     }
+    // exponent of key r: x = sc*dot - m_run + shift, with the magic folded into the constant
+    // (which is therefore off by at most ~1.5 integer steps of the dot product)
+    xc = x_base + mneg;
     // Every probability of a row in this tile is below 2^(m_tile - m_run + shift).  Under 2^-10 (half the smallest
     // e4m3 subnormal; a tie goes to the even code, zero) each one converts to the zero code - taken with a margin of
     // one octave for the exponent's few units of rounding.  With every row of the wave that far down, the wave writes
     // the zeros directly and leaves out the 64 exponentials and 32 conversions per lane (every chunk below tests this
     // one scalar); the matrix work that concerns the neighbouring tiles stays.  Same bits either way - the
     // pvthreshold idea of the reference's sparse kernel (sage_sla.py:237-253) with a threshold at which nothing changes.
-    if constexpr (kTileSkip) nothing = __all(__builtin_fmaf(__int_as_float(mx), sc, mneg) < m_run - (kPShift + 11.0f));
+    if constexpr (kTileSkip) nothing = __all(m_half < m_run - (kPShift + 11.0f));
   };
-  sc = qs * s_ks[0];
-  {
-    float mneg = -kMagicVal * sc;
-    if (mine_at(0)) {
-      alpha_even = move_point<kPwlExp>(lane_max(s_a), sc, mneg, qs, m_run, x_base);
-      if (__any(alpha_even != alpha_even)) scale_o(alpha_even);  // nothing has been accumulated yet: only a NaN has anything to say
-    }
-    // (whole octaves above the first tile's maximum: the probabilities' codes are then the ones about that maximum but for the
-    // power of two in front, and that key's is exact)
-    if (light && m_tile0 == m_tile0 && qs != 0.0f) m_run = m_tile0 + rintf(m_first - m_tile0), x_base = kPShift - m_run;
-    xc = x_base + mneg;
-  }
-  // Tile jp is the one before the coming one, s its scores, pf its probabilities, of which some have no code.  Returns the tile's
-  // row sum.  (A row whose scores are not numbers goes on with zero scores, for the tile that is coming too.)
-  auto refit = [&](int jp, const v16i (&s)[2], v8i& pf) __attribute__((always_inline)) -> float {
-    float sc_prev = qs * s_ks[jp], mneg = -kMagicVal * sc_prev;
-    const float alpha = move_point(lane_max(s), sc_prev, mneg, qs, m_run, x_base);
-    scale_o(alpha);
-    pf = tile_probs<true>(s, sc_prev, x_base + mneg);
-    if constexpr (kCausal) {
-      if (diag_at(jp)) blank_probs(pf, hh, n_diag);
-    }
-    if (jp == tail) blank_probs(pf, hh, n_last);
-    if (alpha != alpha) sc = 0.0f;
-    xc = x_base - kMagicVal * sc;
-    return row_sum(ones, pf);
-  };
+  look_ahead(0, lane_max(s_a), s_ks[0], alpha_even, moved_even);
+  moved_even = __any(alpha_even != alpha_even);  // nothing has been accumulated yet: only a NaN has anything to say
 
   // Software pipeline, one key tile per step.  While this tile's probabilities are computed on
   // the VALU, the matrix pipe runs the S^T MFMAs of the NEXT tile and the PV MFMAs of the
   // PREVIOUS tile: every MFMA below is followed by the VALU work that hides it, LDS operands are
-  // requested three MFMAs ahead, and sched_barrier pins that order.  By the scores, the max reduction of the
+  // requested three MFMAs ahead, and sched_barrier pins that order.  The max reduction of the
   // next tile rides in the PV chunks.
   // Because PV lags one tile, so does the rescaling of O:
   //   at step j   O holds tiles <= j-2 relative to point m(j-2); alpha = 2^(m(j-2) - m(j-1)), tile j-1's
@@ -882,12 +790,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // byte offset into LDS of the next tile's K scale (a vector register on purpose: as a scalar it is moved to one at every use)
   int ks_off = (int)(reinterpret_cast<const uint8_t*>(s_ks) - smem) + 4;
   pin(ks_off);
-  constexpr int kHowScores = 0, kHowCodes = 1, kHowEither = 2;
-  auto tile_step = [&](auto at, auto how, int j, v16i (&s_cur)[2], v16i (&s_nxt)[2], v8i& pf_prev, v8i& pf, float& alpha, int& moved) {
+  auto tile_step = [&](auto at, int j, v16i (&s_cur)[2], v16i (&s_nxt)[2], const v8i& pf_prev, v8i& pf, float& alpha, int& moved) {
     constexpr int kAt = decltype(at)::value;
-    // kCodes, or by the scores; kEither: by the codes, and factors left by steps before it
-    constexpr bool kCodes = decltype(how)::value == kHowCodes || decltype(how)::value == kHowEither;
-    constexpr bool kFactors = decltype(how)::value != kHowCodes;
     const uint8_t* kst = k_slot(kAt >= 0 ? kAt + 1 : j + 1);
     const uint8_t* vst = v_slot(kAt >= 0 ? kAt - 1 : j - 1);
     auto k_frag = [&](int i) { return *reinterpret_cast<const v4i*>(kst + (((i & 1) * 4 + (i >> 1)) * 64 + lane) * 16); };
@@ -896,19 +800,6 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       const v4i hi = *reinterpret_cast<const v4i*>(vst + ((dt * 2 + 1) * 64 + lane) * 16);
       return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     };
-    float sum;
-    auto tile_before = [&]() __attribute__((always_inline)) {
-      if constexpr (kFactors) {
-        if (moved != 0) scale_o(alpha);  // wave-uniform
-        moved = 0;
-      }
-      sum = row_sum(ones, pf_prev);
-      if constexpr (kCodes) {
-        if (__builtin_expect(__ballot(sum != sum) != 0, 0)) sum = refit(j - 1, s_nxt, pf_prev);  // wave-uniform
-        l_run += sum;
-      }
-    };
-    if constexpr (kAt < 0) tile_before();  // (ahead of the operands, whose registers refit would have to go without)
     v4i kf[4];
     v8i vf[4];
     // operands of the first three S^T MFMAs and the next tile's K scale
@@ -920,9 +811,9 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if constexpr (kAt < 0) ks_off += 4;
     int entering = 0;  // the list entry the next step's window gains; it arrives with the operands above
     if constexpr (kSparse) entering = s_list[min(j + 1 + Shape::kAheadK, n_tiles - 1)];
+    if (moved != 0) scale_o(alpha);  // wave-uniform
     // row sums of tile j-1: they cover the latency of the operands just requested
-    // row sums of tile j-1: they cover the latency of the operands just requested
-    if constexpr (kAt >= 0) tile_before();
+    lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_prev, lacc, 0, 0, 0, 0, 0, 0);
     const float scp = kPwlExp ? 8.0f * sc : sc;
     const float cp = kPwlExp ? __builtin_fmaf(8.0f, xc, 55.5f) : xc;
     const bool skip = nothing;
@@ -973,7 +864,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       if (j + 1 == tail) blank_scores<kMagicBits>(s_nxt, hh, n_last);
     }
     __builtin_amdgcn_s_setprio(0);
-    // 4 x [PV MFMA of tile j-1 (64 matrix cycles) | 4 probabilities of tile j | (by the scores) a quarter of
+    // 4 x [PV MFMA of tile j-1 (64 matrix cycles) | 4 probabilities of tile j | a quarter of
     // the max reduction of tile j+1, whose S^T MFMAs were issued at least one chunk ago]
     int mx = 0;
 #pragma unroll
@@ -984,16 +875,14 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       if (!skip) w = pack4(s_cur[1][4 * dt], s_cur[1][4 * dt + 1], s_cur[1][4 * dt + 2], s_cur[1][4 * dt + 3], scp, cp);
       pin(w);
       pf[4 + dt] = w;
-      if constexpr (!kCodes) {
-        // one chain over the 32 scores, two per instruction
-        const v16i& blk = s_nxt[dt >> 1];
-        const int r0 = (dt & 1) * 8;
-        mx = dt == 0 ? max(blk[0], blk[1]) : max(max(mx, blk[r0]), blk[r0 + 1]);
-        mx = max(max(mx, blk[r0 + 2]), blk[r0 + 3]);
-        mx = max(max(mx, blk[r0 + 4]), blk[r0 + 5]);
-        mx = max(max(mx, blk[r0 + 6]), blk[r0 + 7]);
-        pin(mx);
-      }
+      // one chain over the 32 scores, two per instruction
+      const v16i& blk = s_nxt[dt >> 1];
+      const int r0 = (dt & 1) * 8;
+      mx = dt == 0 ? max(blk[0], blk[1]) : max(max(mx, blk[r0]), blk[r0 + 1]);
+      mx = max(max(mx, blk[r0 + 2]), blk[r0 + 3]);
+      mx = max(max(mx, blk[r0 + 4]), blk[r0 + 5]);
+      mx = max(max(mx, blk[r0 + 6]), blk[r0 + 7]);
+      pin(mx);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (kSparse) {
@@ -1011,12 +900,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if constexpr (kAt < 0) {
       if (j == tail) blank_probs(pf, hh, n_last);
     }
-    if constexpr (!kCodes) l_run += sum;
-    sc = qs * ks_nxt;
-    // exponent of key r: x = sc*dot - m_run + shift, with the magic folded into the constant
-    // (which is therefore off by at most ~1.5 integer steps of the dot product)
-    xc = x_base - kMagicVal * sc;
-    if constexpr (!kCodes) look_ahead(j + 1, mx, alpha, moved);
+    look_ahead(j + 1, mx, ks_nxt, alpha, moved);
     // after this barrier: K tile j+2 and V^T tile j are visible to every wave, and nobody reads their predecessors any
     // more (after a group's: K tiles up to j+5, V^T tiles up to j+3, the ones the next group reads)
     if constexpr (kAt < 0 || Shape::kGroup == 1) tile_barrier();
@@ -1027,50 +911,39 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     int j = 0;
     using Anywhere = std::integral_constant<int, -1>;
     if constexpr (kUnrolled) {
-      auto two = [&](auto how, auto at) {
+      auto two = [&](auto at) {
         constexpr int kAt = decltype(at)::value;
-        tile_step(std::integral_constant<int, kAt>{}, how, j + kAt, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
-        tile_step(std::integral_constant<int, kAt + 1>{}, how, j + kAt + 1, s_b, s_a, pf_y, pf_x, alpha_even, moved_even);
+        tile_step(std::integral_constant<int, kAt>{}, j + kAt, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
+        tile_step(std::integral_constant<int, kAt + 1>{}, j + kAt + 1, s_b, s_a, pf_y, pf_x, alpha_even, moved_even);
       };
-      auto rounds = [&](auto how) {
-        for (; j + kStages <= n_plain; j += kStages) {
-          two(how, std::integral_constant<int, 0>{});
-          two(how, std::integral_constant<int, 2>{});
-          if constexpr (kStages == 8) {
-            two(how, std::integral_constant<int, 4>{});
-            two(how, std::integral_constant<int, 6>{});
-          }
-          ks_off += 4 * kStages;
+      for (; j + kStages <= n_plain; j += kStages) {
+        two(std::integral_constant<int, 0>{});
+        two(std::integral_constant<int, 2>{});
+        if constexpr (kStages == 8) {
+          two(std::integral_constant<int, 4>{});
+          two(std::integral_constant<int, 6>{});
         }
-      };
-      // (one after the other, the second with nothing left to do, and not one or the other: joined behind the two, their
-      // accumulators cost a hundred spilled registers)
-      if (__builtin_amdgcn_readfirstlane(!light) != 0) rounds(std::integral_constant<int, kHowScores>{});
-      rounds(std::integral_constant<int, kHowCodes>{});
+        ks_off += 4 * kStages;
+      }
     }
-    using Last = std::integral_constant<int, kUnrolled ? kHowEither : kHowScores>;
     for (; j + 2 <= n_tiles; j += 2) {
-      tile_step(Anywhere{}, Last{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
-      tile_step(Anywhere{}, Last{}, j + 1, s_b, s_a, pf_y, pf_x, alpha_even, moved_even);
+      tile_step(Anywhere{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
+      tile_step(Anywhere{}, j + 1, s_b, s_a, pf_y, pf_x, alpha_even, moved_even);
     }
-    if (j < n_tiles) tile_step(Anywhere{}, Last{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
+    if (j < n_tiles) tile_step(Anywhere{}, j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no copy may outlive the workgroup's LDS
   {  // drain: PV of the last tile
-    const bool odd = (n_tiles & 1) != 0;
-    v8i pf_last = odd ? pf_y : pf_x;  // written by the last step
-    if (odd ? moved_even != 0 : moved_odd != 0) scale_o(odd ? alpha_even : alpha_odd);
-    float sum = row_sum(ones, pf_last);
-    if constexpr (kUnrolled) {
-      if (__ballot(sum != sum) != 0) {
-        const v16i s_last[2] = {odd ? s_a[0] : s_b[0], odd ? s_a[1] : s_b[1]};
-        sum = refit(n_tiles - 1, s_last, pf_last);
-      }
+    if ((n_tiles & 1) != 0) {
+      if (moved_even != 0) scale_o(alpha_even);
+    } else {
+      if (moved_odd != 0) scale_o(alpha_odd);
     }
-    l_run += sum;
     const uint8_t* vst = v_slot(n_tiles - 1);
+    const v8i pf_last = (n_tiles & 1) ? pf_y : pf_x;  // written by the last step
 #pragma unroll
     for (int dt = 0; dt < kG; ++dt) pv_slice(vst, dt, pf_last);
+    lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_last, lacc, 0, 0, 0, 0, 0, 0);
   }
 
   if (is_run) {
@@ -1083,7 +956,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       for (int g = 0; g < 4; ++g)
         *reinterpret_cast<float4*>(po + 32 * dt + 8 * g + 4 * hh) =
             make_float4(oacc[dt][4 * g + 0], oacc[dt][4 * g + 1], oacc[dt][4 * g + 2], oacc[dt][4 * g + 3]);
-    if (hh == 0) reinterpret_cast<float2*>(p.split_ml)[(int64_t)run_id * kAttnQPerWg + row] = make_float2(m_run, l_run);
+    if (hh == 0) reinterpret_cast<float2*>(p.split_ml)[(int64_t)run_id * kAttnQPerWg + row] = make_float2(m_run, lacc[0]);
     return;
   }
   // ---- epilogue: O = O^T / rowsum * v_scale (+ the V mean), written [B, Lq, H, D] ---------------
@@ -1091,7 +964,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // touch 32 rows with 16 bytes each.  The rows go through LDS instead (the tile ring is free once every wave is
   // past its last tile) and leave as whole 256-byte rows, 16 bytes per lane.
   // zero for a mask row that allows none of its keys (an empty sum, not 0/0)
-  const float inv_l = !(kSparse || kCausal) || l_run > 0.0f ? 1.0f / l_run : 0.0f;
+  const float inv_l = !(kSparse || kCausal) || lacc[0] > 0.0f ? 1.0f / lacc[0] : 0.0f;
   // the channel means the V quantizer took off come back here (rows of P sum to one); they are zeros without V
   // smoothing, and a row that saw no key stays zero
   const float keep_mean = inv_l != 0.0f ? 1.0f : 0.0f;

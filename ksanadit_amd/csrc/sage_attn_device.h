@@ -23,16 +23,15 @@ constexpr float kMagicF = 12582912.0f;
 constexpr int kMagicI2 = 0x4BC00000;      // bits of 25165824.0f = 1.5 * 2^24
 constexpr float kMagicF2 = 25165824.0f;
 // P is scaled by 2^6 before the e4m3 cast, and the reference point of a row (its "running maximum") is moved only when
-// one of a tile's probabilities no longer has a code: 448 is the largest e4m3 value, up to 464 rounds to it, and beyond that
-// the conversion gives NaN.  A tile's maximum may thus exceed the point by 2.86 octaves, and the accumulators are rescaled in
-// a few per cent of the steps instead of up to half of them (rows of flat attention set a new maximum every few tiles, by small
-// amounts).  An e4m3 rounding does not depend on the power of two in front, so the result differs only where probabilities
-// fall off the subnormal end, 2^-15 of the reference point.
+// a tile's maximum exceeds it by more than kLazyMax octaves: probabilities then reach 2^(6 + 2.7) = 416 < 448, the
+// largest e4m3 value, and the accumulators are rescaled in a few per cent of the steps instead of up to half of them
+// (rows of flat attention set a new maximum every few tiles, by small amounts).  An e4m3 rounding does not depend on
+// the power of two in front, so the result differs only where probabilities fall off the subnormal end, 2^-15 of the
+// reference point.
 // The piecewise-linear path keeps 2^8 and moves the reference point at every new maximum: its code formula is wrong
 // for the subnormal codes (it fades them linearly), which must stay 2^-14 below the true maximum to be harmless.
 constexpr float kPShift = 6.0f, kPShiftPwl = 8.0f;
-constexpr float kPTop = 464.0f, kPMax = 448.0f;
-constexpr float kXAsk = 8.85f;  // exponents up to here give less than kPTop = 2^8.858: move_point need not be asked
+constexpr float kLazyMax = 2.7f, kLazyMaxPwl = 0.0f;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -62,13 +61,6 @@ __device__ __forceinline__ uint2 half4(float a, float b, float c, float d) {
 template <int DT>
 __device__ __forceinline__ void store4(uint16_t* dst, float a, float b, float c, float d) {
   *reinterpret_cast<uint2*>(dst) = half4<DT>(a, b, c, d);
-}
-
-// a wave-uniform address, in scalar registers wherever it was worked out
-__device__ __forceinline__ const uint8_t* scalar(const uint8_t* at) {
-  const uint64_t a = reinterpret_cast<uint64_t>(at);
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
-  return reinterpret_cast<const uint8_t*>((uint64_t)hi << 32 | lo);
 }
 
 // 16 bytes per lane from global memory straight into LDS at `lds_dst + 16 * lane` (lds_dst is
@@ -123,12 +115,11 @@ __device__ __forceinline__ void blank_probs(v8i& pf, int hh, int n) {
 
 // Moves the reference point of a lane's row where this tile's maximum asks for it (imax: the lane's maximum, over half the
 // row's keys; sc, mneg: the tile's scale and -magic * scale) and returns 2^(old point - new point), exactly 1 where the point stays.
-// A row without a point (m_run, x_base: -inf) always gets one.
 // A row whose scores are not numbers (an infinity in its q, or in a key) gets the factor NaN, which makes its
-// accumulators NaN, and goes on with zero scores: its probabilities must stay numbers, for the 16x16 row sums
+// accumulators and sums NaN, and goes on with zero scores: its probabilities must stay numbers, for the 16x16 row sums
 // multiply them by another row's zeros.
 template <bool kPwlExp = false>
-__device__ __forceinline__ float move_point(int imax, float& sc, float& mneg, float& qs, float& m_run, float& x_base) {
+__device__ __forceinline__ float move_point(int imax, float& sc, float& mneg, float& qs, float& m_run, float& x_base, float& x_limit) {
   {
     // the other half of the row's keys lives in lane +- 32
     int other = imax;
@@ -138,67 +129,29 @@ __device__ __forceinline__ float move_point(int imax, float& sc, float& mneg, fl
   // the accumulator read as fp32 is magic + dot, so one fma gives sc * dot (mneg = -magic * sc)
   const float m_tile = __builtin_fmaf(__int_as_float(imax), sc, mneg);
   const bool nan = m_tile != m_tile;
-  bool move;
-  if constexpr (kPwlExp) {
-    move = m_tile > m_run;
-  } else {
-    // the operations that give the probability itself, so that every kernel draws the line at the same scores
-    const float p_max = fast_exp2(__builtin_fmaf(__int_as_float(imax), sc, x_base + mneg));
-    move = m_run == -INFINITY || p_max > kPTop;
-  }
-  const float m_new = nan ? 0.0f : (move ? m_tile : m_run);
+  const float m_new = nan ? 0.0f : (m_tile > x_limit ? m_tile : m_run);  // the limit is -inf at the first tile: always taken
   const float alpha = fast_exp2((nan ? m_tile : m_run) - m_new);
   sc = nan ? 0.0f : sc;
   mneg = nan ? 0.0f : mneg;
   qs = nan ? 0.0f : qs;
   m_run = m_new;
+  x_limit = m_new + (kPwlExp ? kLazyMaxPwl : kLazyMax);
   x_base = (kPwlExp ? kPShiftPwl : kPShift) - m_new;
   return alpha;
 }
 
 // the probabilities of a tile as the product with V takes them: 2^(sc * dot + xc - magic * sc), the magic folded into xc, in e4m3
-// (kCapped: held at the largest code, for where a NaN code would be taken for a point that has yet to move)
-template <bool kCapped = false>
 __device__ __forceinline__ v8i tile_probs(const v16i (&s)[2], float sc, float xc) {
   v8i pf;
 #pragma unroll
   for (int w = 0; w < 8; ++w) {
     float e[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      e[i] = fast_exp2(__builtin_fmaf(__int_as_float(s[w >> 2][4 * (w & 3) + i]), sc, xc));
-      if constexpr (kCapped) e[i] = fminf(e[i], kPMax);
-    }
+    for (int i = 0; i < 4; ++i) e[i] = fast_exp2(__builtin_fmaf(__int_as_float(s[w >> 2][4 * (w & 3) + i]), sc, xc));
     int code = __builtin_amdgcn_cvt_pk_fp8_f32(e[0], e[1], __float_as_int(e[0]), false);  // both halves get written
     pf[w] = __builtin_amdgcn_cvt_pk_fp8_f32(e[2], e[3], code, true);
   }
   return pf;
-}
-
-// Row sums come from the matrix pipe too, of the SAME e4m3-rounded P the numerator uses.  The 16x16x128 instruction takes half
-// the matrix cycles of the 32x32x64 one and a quarter of its accumulators; its B operand is P's register block read as 16
-// columns with four groups of 16 lanes stacked along the contraction: groups 0 and 2 hold the two halves of query
-// (lane % 16)'s keys, groups 1 and 3 those of query 16 + (lane % 16).  A therefore carries ones where output row
-// 4 g' .. 4 g' + 3 and group g agree in parity and zeros elsewhere: the lanes of group g' then find the sum of their own
-// query in all four registers.  As e2m1 (1.0 = 2, four registers instead of eight): a lane's 32 elements are then two runs of
-// 16 along the contraction, whose bytes of B two neighbouring groups hold, an even one and an odd one.
-// A zero of A meets the probabilities of the query 16 further, and zero times NaN is NaN.
-__device__ __forceinline__ v4i row_sum_ones(int lane) {
-  v4i ones;
-  // four registers on purpose: left as two values the compiler rebuilds the operand with moves in every step
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    int one8 = ((lane >> 2) & 1) == (r >> 1) ? 0x22222222 : 0;
-    pin(one8);
-    ones[r] = one8;
-  }
-  return ones;
-}
-// The row sum of one tile's probabilities: of a tile by itself, so that it can be done over.
-__device__ __forceinline__ float row_sum(const v4i& ones, const v8i& pf) {
-  const v8i a = {ones[0], ones[1], ones[2], ones[3], 0, 0, 0, 0};
-  const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, pf, zero, 4 /* A: e2m1 */, 0, 0, 0, 0, 0)[0];
 }
 
 // S^T tile (64 keys x 32 queries) of one wave: two 32-key sub-tiles, kG 32-channel steps (the channel groups that

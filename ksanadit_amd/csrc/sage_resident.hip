@@ -26,6 +26,13 @@ constexpr int kWaves = 8, kMaxTiles = 8, kRows = 32;
 constexpr int kScalesAt = 2 * kMaxTiles * kTileBytes;              // V scales, V means (128 floats each), K scales
 constexpr int kLds = kScalesAt + (2 * kD + kMaxTiles + 4) * 4;     // .. and the next block's number: 132 144 bytes
 
+// a wave-uniform address, in scalar registers wherever it was worked out
+__device__ __forceinline__ const uint8_t* scalar(const uint8_t* at) {
+  const uint64_t a = reinterpret_cast<uint64_t>(at);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  return reinterpret_cast<const uint8_t*>((uint64_t)hi << 32 | lo);
+}
+
 // n_blk: blocks of 32 rows per (batch, head); parts: workgroups per (batch, head)
 template <int DT, int kG>
 __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const AttnParams p, int n_blk, int parts, int n_wg) {
@@ -99,7 +106,13 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
 #pragma unroll
     for (int s = 0; s < 4; ++s) qf[s] = v4i{0, 0, 0, 0};
     quant_q_rows<DT, kG>(raw, p.q_premul, qf, qs);
-    const v4i ones = row_sum_ones(lane);
+    v8i ones;  // the row sums' operand, see the general kernel
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      int one4 = ((lane >> 2) & 1) == ((lane >> 4) & 1) ? 0x38383838 : 0;
+      pin(one4);
+      ones[r] = one4;
+    }
     v16i magic;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -113,32 +126,29 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.0f;
-    float m_run = -INFINITY, x_base = -INFINITY, l_run = 0.0f;
+    v4f lacc = {0.0f, 0.0f, 0.0f, 0.0f};
+    float m_run = -INFINITY, x_base = -INFINITY, x_limit = -INFINITY;
     auto scale_o = [&](float alpha) {
 #pragma unroll
-      for (int dt = 0; dt < kG; ++dt)
+      for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
-      l_run *= alpha != alpha ? 1.0f : alpha;
+      lacc[0] *= alpha;
     };
-    // the coming tile's scale and exponent constant, and the scale of the one before
-    float sc = 0.0f, xc = 0.0f, sc_prev = 0.0f;
-    // Tile jp is the one before the coming one, s its scores, pf its probabilities, of which some have outgrown e4m3 (see the general
-    // kernel's refit).  Returns the tile's row sum.
-    auto refit = [&](int jp, const v16i (&s)[2], v8i& pf) __attribute__((always_inline)) -> float {
-      int mx = s[0][0];
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = max(mx, s[u][r]);
-      float mneg = -kMagicVal * sc_prev;
-      const float alpha = move_point(mx, sc_prev, mneg, qs, m_run, x_base);
-      scale_o(alpha);
-      pf = tile_probs<true>(s, sc_prev, x_base + mneg);
-      if (jp == tail) blank_probs(pf, hh, n_last);
-      if (alpha != alpha) sc = 0.0f;
-      xc = x_base - kMagicVal * sc;
-      return row_sum(ones, pf);
+    // the coming tile's scale and exponent constant; the factors the point moves of even and of odd tiles put on everything
+    // before them, and whether there is one
+    float sc = 0.0f, xc = 0.0f, alpha_even = 1.0f, alpha_odd = 1.0f;
+    int moved_even = 0, moved_odd = 0;
+    auto look_ahead = [&](int jn, int mx, float ks, float& alpha, int& moved) {
+      sc = qs * ks;
+      float mneg = -kMagicVal * sc;
+      const float m_half = __builtin_fmaf(__int_as_float(mx), sc, mneg);
+      moved = 0;
+      if (__ballot(!(m_half <= x_limit)) != 0 && jn < n_tiles) {
+        alpha = move_point(mx, sc, mneg, qs, m_run, x_base, x_limit);
+        moved = 1;
+      }
+      xc = x_base + mneg;
     };
     auto p_of = [&](int acc_bits) { return fast_exp2(__builtin_fmaf(__int_as_float(acc_bits), sc, xc)); };
     auto k_frag = [&](const uint8_t* tile, int i8) { return *reinterpret_cast<const v4i*>(tile + ((i8 & 1) * 4 + (i8 >> 1)) * 1024); };
@@ -151,7 +161,8 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
 
     // One tile per step: its probabilities on the vector unit, under the matrix instructions of the next tile's scores
     // (of some tile's, not used, in the last step) and of the previous tile's values (times no probabilities, in the first).
-    auto step = [&](int j, v16i (&s_cur)[2], v16i (&s_nxt)[2], v8i& pf_prev, v8i& pf) {
+    // alpha, moved: tile j - 1's on the way in, tile j + 1's on the way out.
+    auto step = [&](int j, v16i (&s_cur)[2], v16i (&s_nxt)[2], const v8i& pf_prev, v8i& pf, float& alpha, int& moved) {
       const int nxt = min(j + 1, n_tiles - 1);
       const uint8_t* kst = my_k + nxt * kTileBytes;
       const uint8_t* vst = my_v + max(j - 1, 0) * kTileBytes;
@@ -159,9 +170,8 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
       v8i vf[4];
       kf[0] = k_frag(kst, 0), kf[1] = k_frag(kst, 1), kf[2] = k_frag(kst, 2);
       const float ks_nxt = s_ks[nxt];
-      float sum = row_sum(ones, pf_prev);
-      if (__builtin_expect(__ballot(sum != sum) != 0, 0)) sum = refit(j - 1, s_nxt, pf_prev);  // wave-uniform
-      l_run += sum;
+      if (moved != 0) scale_o(alpha);  // wave-uniform
+      lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_prev, lacc, 0, 0, 0, 0, 0, 0);
       __builtin_amdgcn_s_setprio(1);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -184,6 +194,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
       }
       if (j + 1 == tail) blank_scores<kMagicBits>(s_nxt, hh, n_last);
       __builtin_amdgcn_s_setprio(0);
+      int mx = 0;
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) {
         if (dt == 0 && kG == 4) vf[3] = v_frag(vst, 3);
@@ -194,13 +205,17 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
         w = __builtin_amdgcn_cvt_pk_fp8_f32(e2, e3, w, true);
         pin(w);
         pf[4 + dt] = w;
+        const v16i& blk = s_nxt[dt >> 1];
+        const int r0 = (dt & 1) * 8;
+        mx = dt == 0 ? max(blk[0], blk[1]) : max(max(mx, blk[r0]), blk[r0 + 1]);
+        mx = max(max(mx, blk[r0 + 2]), blk[r0 + 3]);
+        mx = max(max(mx, blk[r0 + 4]), blk[r0 + 5]);
+        mx = max(max(mx, blk[r0 + 6]), blk[r0 + 7]);
+        pin(mx);
         __builtin_amdgcn_sched_barrier(0);
       }
       if (j == tail) blank_probs(pf, hh, n_last);
-      sc_prev = sc;
-      sc = qs * ks_nxt;
-      const float mneg = -kMagicVal * sc;
-      xc = x_base + mneg;
+      look_ahead(j + 1, mx, ks_nxt, alpha, moved);
     };
     v16i s_a[2], s_b[2];
     v8i pf_x = {0, 0, 0, 0, 0, 0, 0, 0}, pf_y = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -212,33 +227,23 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = max(mx, s_a[u][r]);
-      sc = qs * s_ks[0];
-      float mneg = -kMagicVal * sc;
-      const float alpha = move_point(mx, sc, mneg, qs, m_run, x_base);
-      xc = x_base + mneg;
-      if (__any(alpha != alpha)) scale_o(alpha);  // nothing has been accumulated yet: only a NaN has anything to say
+      look_ahead(0, mx, s_ks[0], alpha_even, moved_even);
+      moved_even = __any(alpha_even != alpha_even);  // nothing has been accumulated yet: only a NaN has anything to say
     }
     int j = 0;
 #pragma unroll 1
     for (; j + 2 <= n_tiles; j += 2) {
-      step(j, s_a, s_b, pf_x, pf_y);
-      step(j + 1, s_b, s_a, pf_y, pf_x);
+      step(j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
+      step(j + 1, s_b, s_a, pf_y, pf_x, alpha_even, moved_even);
     }
-    if (j < n_tiles) step(j, s_a, s_b, pf_x, pf_y);
-    v8i pf_last;
-    {  // the last tile's sums
-      const bool odd = (n_tiles & 1) != 0;
-      pf_last = odd ? pf_y : pf_x;
-      float sum = row_sum(ones, pf_last);
-      if (__ballot(sum != sum) != 0) {
-        const v16i s_last[2] = {odd ? s_a[0] : s_b[0], odd ? s_a[1] : s_b[1]};
-        sum = refit(n_tiles - 1, s_last, pf_last);
-      }
-      l_run += sum;
-    }
+    if (j < n_tiles) step(j, s_a, s_b, pf_x, pf_y, alpha_odd, moved_odd);
     request(next);  // (the scores' registers are free by now)
-    {  // .. and its values
+    {  // the last tile's values
+      const bool odd = (n_tiles & 1) != 0;
+      if (odd ? moved_even != 0 : moved_odd != 0) scale_o(odd ? alpha_even : alpha_odd);
+      const v8i pf_last = odd ? pf_y : pf_x;
       const uint8_t* vst = my_v + (n_tiles - 1) * kTileBytes;
+      lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_last, lacc, 0, 0, 0, 0, 0, 0);
 #pragma unroll
       for (int dt = 0; dt < kG; ++dt)
         oacc[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(v_frag(vst, dt), pf_last, oacc[dt], 0, 0, 0, 0, 0, 0);
@@ -247,7 +252,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
     // O = O^T / rowsum * v_scale (+ the V mean).  A lane has channels 32 dt + 8 g + 4 hh .. + 3 of its row; lanes l and l + 32
     // trade every second four, so that each stores eight in a row.  (Staged through LDS for whole 256-byte rows they
     // would need room that the tiles hold; the L2 puts a row's pieces together.)
-    const float inv_l = 1.0f / l_run;
+    const float inv_l = 1.0f / lacc[0];
     const float keep_mean = inv_l != 0.0f ? 1.0f : 0.0f;
     uint16_t* orow = obase + (int64_t)row * p.o.sL;
     auto store = [&](auto with_mean) {

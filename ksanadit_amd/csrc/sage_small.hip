@@ -258,13 +258,15 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c,
   for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[dt][r] = 0.0f;
-  float l_run = 0.0f;
+  v4f lacc = {0.0f, 0.0f, 0.0f, 0.0f};  // row sums, see the general kernel for the operand of ones
   if (active) {
-    const v4i ones = row_sum_ones(lane);
+    v8i ones;
     v16i magic;
 #pragma unroll
+    for (int r = 0; r < 8; ++r) ones[r] = ((lane >> 2) & 1) == ((lane >> 4) & 1) ? 0x38383838 : 0;
+#pragma unroll
     for (int r = 0; r < 16; ++r) magic[r] = kMagicBits;
-    float m_run = -INFINITY, x_base = -INFINITY;
+    float m_run = -INFINITY, x_base = -INFINITY, x_limit = -INFINITY;
     const int n_mine = c.causal ? min(n_tiles, (q0 >> 6) + 1) : n_tiles;
     for (int j = 0; j < n_mine; ++j) {
       v16i s[2];
@@ -279,13 +281,13 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c,
 #pragma unroll
         for (int r = 0; r < 16; ++r) top = max(top, s[u][r]);
       float sc = qs * s_ks[j], mneg = -kMagicVal * sc;
-      const float alpha = move_point(top, sc, mneg, qs, m_run, x_base);
+      const float alpha = move_point(top, sc, mneg, qs, m_run, x_base, x_limit);
       if (j == 0 ? __any(alpha != alpha) : __any(alpha != 1.0f)) {
 #pragma unroll
         for (int dt = 0; dt < kG; ++dt)
 #pragma unroll
           for (int r = 0; r < 16; ++r) oacc[dt][r] *= alpha;
-        l_run *= alpha;
+        lacc[0] *= alpha;
       }
       v8i pf = tile_probs(s, sc, x_base + mneg);
       if (!whole) blank_probs(pf, hh, allowed);
@@ -297,13 +299,13 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c,
         const v8i vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         oacc[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf, pf, oacc[dt], 0, 0, 0, 0, 0, 0);
       }
-      l_run += row_sum(ones, pf);
+      lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, lacc, 0, 0, 0, 0, 0, 0);
     }
   }
 
   // ---- O = O^T / rowsum * v_scale, whole rows out through LDS -----------------------------------------
   // (a dense row always has a sum; causal rows: as the general kernel has it)
-  const float inv_l = !c.causal || l_run > 0.0f ? 1.0f / l_run : 0.0f;
+  const float inv_l = !c.causal || lacc[0] > 0.0f ? 1.0f / lacc[0] : 0.0f;
   float4 s4[16];
 #pragma unroll
   for (int i = 0; i < 4 * kG; ++i) s4[i] = reinterpret_cast<const float4*>(s_vs)[(32 * (i >> 2) + 8 * (i & 3) + 4 * hh) >> 2];

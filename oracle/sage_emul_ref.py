@@ -26,14 +26,9 @@ from .quant_ref import BLKK, BLKQ, FP8_MAX, e4m3fn_decode_table, quant_k_ref, qu
 # P is scaled by 2**P_SHIFT before the fp8 cast so that small probabilities stay above the
 # e4m3 subnormal floor (2**-9); the factor cancels in O = (P V) / rowsum(P).  The online form moves a row's reference
 # point (its "running maximum") only when a tile's maximum exceeds it by more than LAZY_MAX octaves, as the kernel
-# does: probabilities then reach 2**(P_SHIFT + LAZY_MAX) = 464, the largest value that e4m3 rounds to 448 and not to NaN.
+# does: probabilities then reach 2**(P_SHIFT + LAZY_MAX) = 416 < 448.
 P_SHIFT = 6.0
-LAZY_MAX = 2.8579809951275723  # log2(464 / 2**P_SHIFT)
-# 32 rows (the kernel's waves) that take part in more than SAMPLE_FROM key tiles look at SAMPLE of them first: where their maximum
-# is more than LIGHT_SPREAD octaves above the first tile's in at most LIGHT_ROWS of the rows, the points start that many whole
-# octaves (rounded) above the first tile's maximum.
-SAMPLE_FROM, SAMPLE = 32, 4
-LIGHT_SPREAD, LIGHT_ROWS = 1.5, 8
+LAZY_MAX = 2.7
 # The piecewise-linear path keeps 2**8 and follows every new maximum: its code formula fades the subnormal codes
 # linearly, which is harmless only far below the true maximum.
 P_SHIFT_PWL = 8.0
@@ -118,36 +113,12 @@ def sage_emul_from_quant(q_i8, q_scale, k_i8, k_scale, v_fp8, v_scale, out_dtype
 
                 def walk(key_from, key_to):
                     """Online softmax over the tiles of keys [key_from, key_to): (acc, m, l)."""
-                    m = first_point(key_from, key_to)
+                    m = torch.full((Lq, 1), float("-inf"))
                     l = torch.zeros(Lq, 1)
                     acc = torch.zeros(Lq, D)
                     for j0 in range(key_from, key_to, BLKK):
                         m, l, acc = step(j0, min(j0 + BLKK, key_to), m, l, acc)
                     return acc, m, l
-
-                def first_point(key_from, key_to):
-                    starts = list(range(key_from, key_to, BLKK))
-                    take = torch.ones(Lq, len(starts), dtype=torch.bool)
-                    if block_mask is not None:
-                        take &= bm[b, h][:, [j0 // BLKK for j0 in starts]].bool().repeat_interleave(128, dim=0)[:Lq]
-                    if causal:
-                        take &= torch.tensor(starts)[None, :] <= rows // 32 * 32
-                    sampled = take.sum(dim=1, keepdim=True) > SAMPLE_FROM
-                    m, m_0 = (torch.full((Lq, 1), float("-inf")) for _ in range(2))
-                    if not exact_exp2 or not bool(sampled.any()):
-                        return m
-                    take &= sampled & (take.cumsum(dim=1) <= SAMPLE)
-                    for i, j0 in enumerate(starts):
-                        if not bool(take[:, i].any()):
-                            continue
-                        sc = (qs_row[b, h][:, None] * k_scale[b, hk, j0 // BLKK]).to(torch.float32)
-                        top = x_f[:, j0 : min(j0 + BLKK, key_to)].amax(dim=1, keepdim=True)
-                        m_tile = (top.double() * sc.double() - (magic * sc).double()).float()
-                        m_0 = torch.where(take[:, i : i + 1] & torch.isinf(m_0), m_tile, m_0)
-                        m = torch.where(take[:, i : i + 1], torch.maximum(m, m_tile), m)
-                    wide = torch.nn.functional.pad(sampled & (m - m_0 > LIGHT_SPREAD), (0, 0, 0, -Lq % 32)).view(-1, 32).sum(dim=1)
-                    light = sampled & (wide <= LIGHT_ROWS).repeat_interleave(32)[:Lq, None]
-                    return torch.where(light, m_0 + torch.round(m - m_0), torch.full_like(m, float("-inf")))
 
                 def step(j0, j1, m, l, acc):
                     act = None  # rows that take part in this step
