@@ -518,6 +518,15 @@ def _cos(a, b):
     return float((a @ b) / (a.norm() * b.norm()))
 
 
+@pytest.mark.parametrize("kw", [{}, {"causal": True}, {"exact_exp2": False}])
+def test_sage_emul_rows_do_not_hang_on_other_rows(kw):
+    """Flat rows among flat ones and among spread ones, with more key tiles than any of the kernel's special cases for short rows."""
+    L, kept = 64 * 36, torch.arange(64 * 36) % 32 == 5
+    q, k, v = (_rand((1, L, 1, 64), s) for s in (31, 32, 33))
+    outs = [sage_emul_ref(torch.where(kept[:, None, None], q, others * q), k, v, **kw) for others in (1.0, 3.0)]
+    assert torch.equal(outs[0][:, kept], outs[1][:, kept]) and not torch.equal(outs[0], outs[1])
+
+
 def test_sage_emul_close_to_sdpa_and_invariants():
     B, L, H, D = 1, 300, 2, 128
     q, v = _rand((B, L, H, D), 1), _rand((B, L, H, D), 3)
