@@ -34,7 +34,7 @@ namespace {
 // every K/V tile copied serves 256 rows), and 4 waves = 128 query rows with a 4-stage ring, two of which share a
 // compute unit - they run out of step, so one's prologue and epilogue hide under the other's key loop (what short key
 // sequences need), and a workgroup is exactly one row of a block mask.
-template <int kW>
+template <int kW, int kG = 4>
 struct WgShape {
   static_assert(kW == 8 || kW == 4, "workgroups of 8 or 4 waves");
   static constexpr int kThreads = kW * 64;
@@ -44,7 +44,9 @@ struct WgShape {
   // ring of its own K can be requested further ahead.
   static constexpr int kStages = kW == 8 ? 8 : 4;
   static constexpr int kRingBytes = kStages * 2 * kTileBytes;
-  static constexpr int kCopies = 2 * (8 / kW);         // 1 KiB copy instructions per wave and tile (K and V^T halves)
+  // 1 KiB copy instructions per wave and tile, K and V^T: with 64 channels (kG == 2) half of either tile is all that is read,
+  // and the other half is not copied
+  static constexpr int kCopies = 2 * (8 / kW) * kG / 4;
   // How many tiles ahead step j requests the V^T and the K tile.  4 waves: K into the slot of tile j, which every wave
   // has read; a copy then has three steps (about three microseconds) to arrive, which matters where tiles miss the L2
   // (block masks).  8 waves: what the groups of four steps below allow.
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // last tile, 32 lane masks held in scalar registers, the selects that blank a wave's probabilities past its rows)
   // is compiled out of the key loop
   const bool causal = kCausal && (!kSparse || p.causal);
-  using Shape = WgShape<kW>;
+  using Shape = WgShape<kW, kG>;
   constexpr int kThreadsAttn = Shape::kThreads, kRowsWg = Shape::kRows, kStages = Shape::kStages, kAhead = Shape::kAhead;
   constexpr int kListMax = kW == 8 ? kSparseMaxKeyTiles : kSparseMaxKeyTiles4;
   static_assert(!(kTileSkip && kPwlExp), "the piecewise-linear code formula has its own zero point: no tiles are skipped there");
@@ -120,7 +122,21 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       // XCD a contiguous run of (head, query block) pairs so the workgroups that stream the same
       // K/V tiles share one L2.
       const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
-      if (p.batch_run == 0) {
+      if (p.small_last != 0) {
+        // Short last blocks (see launch_attn_fwd) behind the whole ones: an XCD's run of whole blocks, then its share of the
+        // heads' last ones.
+        const int whole = wg_per_xcd - p.small_last, n_pairs = p.B * p.Hq, n_whole = n_pairs * (n_qwg - 1);
+        if (at < whole) {
+          const int w = xcd * whole + at;
+          if (w >= n_whole) return;
+          const int pair = w / (n_qwg - 1);
+          wg = w + pair;
+        } else {
+          const int pair = xcd * p.small_last + (at - whole);
+          if (pair >= n_pairs) return;
+          wg = pair * n_qwg + n_qwg - 1;
+        }
+      } else if (p.batch_run == 0) {
         wg = xcd * wg_per_xcd + at;
         if (wg >= n_wg) return;
       } else {
@@ -147,11 +163,9 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   const int l32 = lane & 31, hh = lane >> 5;
   // query rows [0, lq) of this batch take part: all of them, or the caller's per-batch count; the rows from lq up
   // to Lq exist in the output and are written as zeros
-  int lq = p.Lq;
-  if (p.q_lens != nullptr) lq = rows_counted(p.q_lens[b], p.Lq);  // uniform: a scalar load
   // keys [0, lk) of this batch take part: all of them, or the caller's per-batch count
-  int lk = p.Lk;
-  if (p.k_lens != nullptr) lk = rows_counted(p.k_lens[b], p.Lk);  // uniform: a scalar load
+  int lq = p.Lq, lk = p.Lk;
+  take_counts(p.q_lens, p.k_lens, b, lq, lk);
   // A last block of at most 64 rows has work for one or two waves.  Alone on its unit such a workgroup takes half a microsecond a
   // step, next to another one as long as the whole blocks do; so its four waves share the keys out instead (see below).
   constexpr bool kCanShare = !kSparse && !kCausal && kW == 4 && !kPwlExp && !kTileSkip;
@@ -207,24 +221,12 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   const bool own_q = __builtin_expect(kOwnQ && active && !shared && p.q_rows.ptr != nullptr, 0);  // uniform per wave
 #pragma unroll
   for (int s = 0; s < 4; ++s) qf[s] = v4i{0, 0, 0, 0};
-  if (own_q) {
-    // requested here, quantized once the first tiles are on their way
-    const int row = q0 + l32;
-    const uint16_t* qrow = p.q_rows.ptr + b * p.q_rows.sB + (int64_t)row * p.q_rows.sL + h * p.q_rows.sH + 16 * hh;
-#pragma unroll
-    for (int s = 0; s < kG; ++s) {
-      q_raw[2 * s] = q_raw[2 * s + 1] = make_uint4(0, 0, 0, 0);
-      if (row < p.Lq && 32 * s < p.q_rows.D) {
-        q_raw[2 * s] = *reinterpret_cast<const uint4*>(qrow + 32 * s);
-        q_raw[2 * s + 1] = *reinterpret_cast<const uint4*>(qrow + 32 * s + 8);
-      }
-    }
-  } else if (active && !(shared && p.q_rows.ptr != nullptr)) {
+  auto read_q = [&]() {
     const int8_t* qrow = p.q_i8 + ((int64_t)bh * p.lq_pad + q0 + l32) * kD + 16 * hh;
 #pragma unroll
     for (int s = 0; s < kG; ++s) qf[s] = *reinterpret_cast<const v4i*>(qrow + 32 * s);
     qs = p.q_scale[(int64_t)bh * p.lq_pad + q0 + l32];  // one scale per query row = per lane
-  }
+  };
 
   v16f oacc[4];
 #pragma unroll
@@ -341,22 +343,22 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   }
   // the head's K scales (in loop order: tile order, or the list's) and V scales / means go to LDS, once the first
   // tile copies are on their way, so that the loads' latencies overlap
+  // (copied as the tiles are, with nothing to wait for but the set-up's one wait)
   auto fill_scales = [&]() {
-    // the V value is requested first and stored last: written where it is loaded, its load would only go out after
-    // the K scales' loads had been awaited - a second memory latency in every workgroup's set-up
-    float vsm = 0.0f;
-    if (tid < 2 * kD) vsm = tid < kD ? p.v_scale[(int64_t)bhk * kD + tid] : p.v_mean[(int64_t)bhk * kD + tid - kD];
-    if constexpr (kSparse) {
-      for (int i = tid; i < n_tiles; i += kThreadsAttn) s_ks[i] = ks_ptr[s_list[i] & 0xffff];
-    } else {
-      for (int i = tid; i < n_tiles; i += kThreadsAttn) s_ks[i] = ks_ptr[i];
+    if (wave < 4) lds_copy4((wave < 2 ? p.v_scale : p.v_mean) + (int64_t)bhk * kD, (unsigned)((wave & 1) * 64 + lane) * 4, s_vs + wave * 64);
+    for (int i0 = wave * 64; i0 < n_tiles; i0 += kThreadsAttn) {
+      const int i = i0 + lane;
+      if (i < n_tiles) {
+        unsigned at = (unsigned)i;
+        if constexpr (kSparse) at = (unsigned)(s_list[i] & 0xffff);
+        lds_copy4(ks_ptr, at * 4, s_ks + i0);
+      }
     }
-    if (tid < 2 * kD) s_vs[tid] = vsm;
   };
   if constexpr (kCanShare) {
     if (shared) {
-      // A wave takes a run of ceil(tiles / sharers) key tiles, its operands straight from the L2 into registers (V under
-      // the softmax, the next tile's K under the product with V), with reference points of its own; the four results are put together as the merge kernel does it, through LDS.  Bound by its chain of steps, a
+      // A wave takes a run of ceil(tiles / sharers) key tiles, its operands straight from the L2 into registers (each as soon
+      // as the step before is through with it), with reference points of its own; the four results are put together as the merge kernel does it, through LDS.  Bound by its chain of steps, a
       // quarter as long.  us per call, whole / shared: 40 heads of 1560 tokens, where eight of the 520 workgroups start when the
       // others end, 67.9 / 56.8.  Errors against 64 bits are those of whole rows or below: 0.0383 / 0.0388 at N(0, 1),
       // 0.0289 / 0.0295 with outliers.
@@ -369,9 +371,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
           if (q0 + l32 >= lq) raw[i] = make_uint4(0, 0, 0, 0);
         }
         quant_q_rows<DT, kG>(raw, p.q_premul, qf, qs);
+      } else {
+        read_q();
       }
       fill_scales();
-      __syncthreads();
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
       const int per = (nkb + sharers - 1) / sharers, run = wave & (sharers - 1), j0 = min(run * per, nkb), j1 = min(j0 + per, nkb);
       const uint8_t* kt = k_src + lane * 16;
       const uint8_t* vt = v_src + lane * 16;
@@ -381,7 +385,20 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         for (int i = 0; i < 2 * kG; ++i)
           kf[i] = *reinterpret_cast<const v4i*>(kt + (int64_t)j * kTileBytes + ((i / kG) * 4 + i % kG) * 1024);
       };
-      if (j0 < j1) fetch_k(j0);
+      v8i vf[kG];
+      auto fetch_v = [&](int j) {
+#pragma unroll
+        for (int dt = 0; dt < kG; ++dt) {
+          const v4i lo = *reinterpret_cast<const v4i*>(vt + (int64_t)j * kTileBytes + (2 * dt + 0) * 1024);
+          const v4i hi = *reinterpret_cast<const v4i*>(vt + (int64_t)j * kTileBytes + (2 * dt + 1) * 1024);
+          vf[dt] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        }
+      };
+      if (j0 < j1) {
+        fetch_k(j0);
+        fetch_v(j0);
+      }
+      __builtin_amdgcn_s_setprio(2);  // (a chain with nothing beside it: ahead of the neighbour's waves)
 #pragma unroll 1
       for (int j = j0; j < j1; ++j) {
         v16i s[2] = {magic, magic};
@@ -389,13 +406,9 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         for (int c = 0; c < kG; ++c)
 #pragma unroll
           for (int u = 0; u < 2; ++u) s[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(kf[u * kG + c], qf[c], s[u], 0, 0, 0);
-        v8i vf[kG];
-#pragma unroll
-        for (int dt = 0; dt < kG; ++dt) {
-          const v4i lo = *reinterpret_cast<const v4i*>(vt + (int64_t)j * kTileBytes + (2 * dt + 0) * 1024);
-          const v4i hi = *reinterpret_cast<const v4i*>(vt + (int64_t)j * kTileBytes + (2 * dt + 1) * 1024);
-          vf[dt] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_k(min(j + 1, nkb - 1));
+        __builtin_amdgcn_sched_barrier(0);
         const int n_last = j == nkb - 1 ? lk & (kBlkK - 1) : 0;  // (uniform) keys of a ragged tile
         if (n_last != 0) blank_scores<kMagicBits>(s, hh, n_last);
         int top = max(s[0][0], s[1][0]);
@@ -412,11 +425,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         }
         v8i pf = tile_probs(s, sc, x_base + mneg);
         if (n_last != 0) blank_probs(pf, hh, n_last);
-        fetch_k(min(j + 1, nkb - 1));
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int dt = 0; dt < kG; ++dt) oacc[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf[dt], pf, oacc[dt], 0, 0, 0, 0, 0, 0);
         lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf, lacc, 0, 0, 0, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_v(min(j + 1, nkb - 1));
       }
       // every wave's accumulators in the ring, points and sums where the K scales were; then the waves of a row group finish a
       // quarter or half of its channels each
@@ -539,16 +552,20 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   auto v_slot = [&](int tile) -> uint8_t* { return smem + (kStages + (tile & (kStages - 1))) * kTileBytes; };
   // clamped: past the end the last tile is copied again into a slot nobody reads any more,
   // which keeps the loop free of branches and the outstanding-copy count constant
-  auto copy_tile_half = [&](const uint8_t* src, int jl, uint8_t* dst) {  // jl: key tile number, wave-uniform
+  // This wave's 1 KiB slices of a tile: slice c * kW + wave; with 64 channels the slices that hold any - of K fragments 0, 1
+  // of either half of the keys, of V^T the lower half - are one of each for four waves, and one of either for eight (waves
+  // 0-3 copy K, waves 4-7 V^T).
+  constexpr bool kEither = kG == 2 && kW == 8;
+  const bool copies_k = !kEither || wave < 4, copies_v = !kEither || wave >= 4;
+  const int slice_k = kG == 4 ? wave : (wave & 1) + 2 * (wave & 2), slice_v = kG == 4 ? wave : wave & 3;
+  auto copy_tile_half = [&](bool is_v, int jl, uint8_t* dst) {  // jl: key tile number, wave-uniform
+    if (is_v ? !copies_v : !copies_k) return;
+    const int slice = is_v ? slice_v : slice_k;
 #pragma unroll
-    for (int c = 0; c < 8 / kW; ++c) {  // this wave's 1 KiB slices of the tile: slice c * kW + wave
-      const int slice = c * kW + wave;
-      lds_copy16(src + (int64_t)jl * kTileBytes, (unsigned)(slice * 64 + lane) * 16, dst + slice * 1024);
-    }
+    for (int c = 0; c < (kG == 4 ? 8 / kW : 1); ++c)
+      lds_copy16((is_v ? v_src : k_src) + (int64_t)jl * kTileBytes, (unsigned)((c * kW + slice) * 64 + lane) * 16, dst + (c * kW + slice) * 1024);
   };
-  auto copy_half = [&](const uint8_t* src, int tile, uint8_t* dst) {
-    copy_tile_half(src, tile_of(min(tile, n_tiles - 1)), dst);
-  };
+  auto copy_half = [&](bool is_v, int tile, uint8_t* dst) { copy_tile_half(is_v, tile_of(min(tile, n_tiles - 1)), dst); };
   // With a tile list, the key tiles behind the loop positions whose copies the next steps issue are kept in scalar
   // registers: looked up in the step, a list entry costs an LDS read whose wait also drains the operand reads
   // requested just before it.  ahead[i] = tile at position j + kAhead + i for the step j about to run; a step
@@ -566,26 +583,35 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     return v4i{(int)(uint32_t)a, (int)(uint32_t)(a >> 32) & 0xffff, (p.nkb - tile0) * kTileBytes, 0x00020000};
   };
   const v4i k_buf = tiles_from(k_src), v_buf = tiles_from(v_src);
-  const unsigned lane_off = (unsigned)(wave * 64 + lane) * 16;
-  const unsigned lds_base = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)smem + (unsigned)wave * 1024;
+  const unsigned lds_0 = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)smem;
+  const unsigned lane_off_k = (unsigned)(slice_k * 64 + lane) * 16, lane_off_v = (unsigned)(slice_v * 64 + lane) * 16;
+  const unsigned lds_base_k = lds_0 + (unsigned)slice_k * 1024, lds_base_v = lds_0 + (unsigned)slice_v * 1024;
   const int off_last = (n_tiles - 1) * kTileBytes;
   int off_v = min(kAhead, n_tiles - 1) * kTileBytes, off_k = min(Shape::kAheadK, n_tiles - 1) * kTileBytes;
-  auto copy_to = [&](auto slot, const v4i& buffer, int off) {
+  auto copy_to = [&](auto slot, const v4i& buffer, unsigned lane_off, int off, unsigned lds_base) {
     constexpr int kSlot = decltype(slot)::value;
     lds_copy16_at<kSlot>(buffer, lane_off, off, lds_base);
-    if constexpr (kW == 4) lds_copy16_at<kSlot + 4096>(buffer, lane_off + 4096, off, lds_base);
+    if constexpr (kW == 4 && kG == 4) lds_copy16_at<kSlot + 4096>(buffer, lane_off + 4096, off, lds_base);
   };
+  // (kEither) this wave's tiles
+  const v4i my_buf = copies_k ? k_buf : v_buf;
+  const unsigned my_lane_off = copies_k ? lane_off_k : lane_off_v, my_lds_base = copies_k ? lds_base_k : lds_base_v;
+  int off_mine = copies_k ? off_k : off_v;
   // the V^T and K tile that tile number kTile (modulo kStages) would request in a loop of single steps
   auto copies_of = [&](auto tile) {
     constexpr int kTile = decltype(tile)::value;
     using VSlot = std::integral_constant<int, (kStages + ((kTile + kAhead) & (kStages - 1))) * kTileBytes>;
     using KSlot = std::integral_constant<int, ((kTile + Shape::kAheadK) & (kStages - 1)) * kTileBytes>;
     if constexpr (kSparse) {
-      copy_to(VSlot{}, v_buf, ahead[0] * kTileBytes);
-      copy_to(KSlot{}, k_buf, ahead[kWindow - 1] * kTileBytes);
+      copy_to(VSlot{}, v_buf, lane_off_v, ahead[0] * kTileBytes, lds_base_v);
+      copy_to(KSlot{}, k_buf, lane_off_k, ahead[kWindow - 1] * kTileBytes, lds_base_k);
+    } else if constexpr (kEither) {
+      const unsigned slot = copies_k ? KSlot::value : VSlot::value;
+      lds_copy16_at<0>(my_buf, my_lane_off, off_mine, my_lds_base + slot);
+      off_mine = min(off_mine + kTileBytes, off_last);
     } else {
-      copy_to(VSlot{}, v_buf, off_v);  // first: it is awaited first
-      copy_to(KSlot{}, k_buf, off_k);
+      copy_to(VSlot{}, v_buf, lane_off_v, off_v, lds_base_v);  // first: it is awaited first
+      copy_to(KSlot{}, k_buf, lane_off_k, off_k, lds_base_k);
       off_v = min(off_v + kTileBytes, off_last);
       off_k = min(off_k + kTileBytes, off_last);
     }
@@ -603,11 +629,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // the copies of loop step j (step -1: nothing; the prologue below brings the first tiles in)
   auto issue_copy = [&](int j) {
     if constexpr (kSparse) {
-      copy_tile_half(v_src, ahead[0], v_slot(j + kAhead));
-      copy_tile_half(k_src, ahead[kWindow - 1], k_slot(j + Shape::kAheadK));
+      copy_tile_half(true, ahead[0], v_slot(j + kAhead));
+      copy_tile_half(false, ahead[kWindow - 1], k_slot(j + Shape::kAheadK));
     } else {
-      copy_half(v_src, j + kAhead, v_slot(j + kAhead));  // first: it is awaited first
-      copy_half(k_src, j + Shape::kAheadK, k_slot(j + Shape::kAheadK));
+      copy_half(true, j + kAhead, v_slot(j + kAhead));  // first: it is awaited first
+      copy_half(false, j + Shape::kAheadK, k_slot(j + Shape::kAheadK));
     }
   };
   // wait until every copy except the newest Shape::kInFlight has landed, then meet the other waves.
@@ -642,19 +668,40 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // tiles, 32760 queries, 40 heads: -1.2 %).
   constexpr bool kLateCopies = Shape::kGroup == 1;
 #pragma unroll
-  for (int t = 0; t < (kLateCopies ? 0 : kAhead); ++t) copy_half(v_src, t, v_slot(t));
+  for (int t = 0; t < (kLateCopies ? 0 : kAhead); ++t) copy_half(true, t, v_slot(t));
 #pragma unroll
-  for (int t = 0; t < (kLateCopies ? 2 : Shape::kAheadK); ++t) copy_half(k_src, t, k_slot(t));
+  for (int t = 0; t < (kLateCopies ? 2 : Shape::kAheadK); ++t) copy_half(false, t, k_slot(t));
   fill_scales();
-  if (__builtin_expect(own_q, 0)) quant_q_rows<DT, kG>(q_raw, p.q_premul, qf, qs);
+  if (__builtin_expect(own_q, 0)) {
+    // Requested behind the copies and without a condition: loads return in the order they were issued, and a wait for one issued
+    // before a copy, which the compiler does not count, is a wait for the copy too.  With the loads first and zeros
+    // for what does not exist in their stead, the second pair of loads went out when the first had arrived.
+    const int row = q0 + l32;
+    const bool half = kG == 4 && p.q_rows.D != kD;  // (uniform) 64 channels in the full-width code
+    const uint16_t* qrow = p.q_rows.ptr + b * p.q_rows.sB + (int64_t)min(row, p.Lq - 1) * p.q_rows.sL + h * p.q_rows.sH + 16 * hh;
+#pragma unroll
+    for (int s = 0; s < kG; ++s) {
+      const int at = 32 * (half ? s & 1 : s);
+      q_raw[2 * s] = *reinterpret_cast<const uint4*>(qrow + at);
+      q_raw[2 * s + 1] = *reinterpret_cast<const uint4*>(qrow + at + 8);
+    }
+    if (half || q0 + 32 > p.Lq) {
+#pragma unroll
+      for (int s = 0; s < kG; ++s)
+        if (row >= p.Lq || (half && s >= 2)) q_raw[2 * s] = q_raw[2 * s + 1] = make_uint4(0, 0, 0, 0);
+    }
+    quant_q_rows<DT, kG>(q_raw, p.q_premul, qf, qs);
+  } else if (active) {
+    read_q();
+  }
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the set-up's loads and, older than some of them, the copies
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   if constexpr (kLateCopies) {
     static_assert(Shape::kAheadK == kAhead + 2, "V^T tiles 0, 1 with K tiles 2, 3");
 #pragma unroll
     for (int t = 0; t < kAhead; ++t) {
-      copy_half(v_src, t, v_slot(t));
-      copy_half(k_src, t + 2, k_slot(t + 2));
+      copy_half(true, t, v_slot(t));
+      copy_half(false, t + 2, k_slot(t + 2));
     }
   }
 
@@ -663,8 +710,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     if constexpr (kSlotZeroSoon) __builtin_amdgcn_s_barrier();
     for (int j = 0; j < n_tiles; ++j) {
       // (looks the tiles up where they are needed: a wave without rows has nothing an LDS wait could hold up)
-      copy_half(v_src, j + kAhead, v_slot(j + kAhead));
-      copy_half(k_src, j + Shape::kAheadK, k_slot(j + Shape::kAheadK));
+      copy_half(true, j + kAhead, v_slot(j + kAhead));
+      copy_half(false, j + Shape::kAheadK, k_slot(j + Shape::kAheadK));
       if (j >= n_grouped) tile_barrier();
       else if ((j & (Shape::kGroup - 1)) == Shape::kGroup - 1) group_barrier();
     }
@@ -1309,7 +1356,7 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   const int n_qwg = (p.Lq + rows - 1) / rows;
   const int n_wg = p.B * p.Hq * n_qwg;
   int wg_per_xcd = 0;
-  const dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
+  dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
   if (p.causal && p.batch_run == 0) p.causal_grid = causal_grid(p.B * p.Hq, n_qwg);  // (the same number of workgroups)
   // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
   const size_t lds = (waves == 4 ? WgShape<4>::kRingBytes : WgShape<8>::kRingBytes) + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
@@ -1321,7 +1368,17 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
                ? launch_variant<KSANA_SAGE_BF16, false, true, 4, false, false, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
                : launch_variant<KSANA_SAGE_FP16, false, true, 4, false, false, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s);
   }
+  // Dense calls whose heads end in a short block (at most half a workgroup's rows, which takes a third to half of a whole one's
+  // time): these start last, so that a round they do not fit into is longer by one of them and not by a whole block.
+  auto small_blocks_last = [&]() {
+    const int pairs = p.B * p.Hq;
+    if (sparse || p.batch_run != 0 || n_qwg < 2 || 2 * (p.Lq - (n_qwg - 1) * rows) > rows) return;
+    p.small_last = (pairs + 7) / 8;
+    wg_per_xcd = (pairs * (n_qwg - 1) + 7) / 8 + p.small_last;
+    grid = dim3(wg_per_xcd * 8);
+  };
   if (waves == 4) {
+    small_blocks_last();
     if (plain_causal) return launch_causal(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
     if (sparse)
       return p.causal ? launch_shape<true, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
@@ -1335,7 +1392,10 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   // small kernel merges the runs: 2568 workgroups are then 10 rounds and a bit instead of 11, 280 are 1.1 instead of 2.
   int n_full = n_wg, n_split = 0;
   if (p.split_o != nullptr) plan_key_split(n_wg, p.nkb, &n_full, &n_split);
-  if (n_split == 0) return launch_shape<false, 8>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+  if (n_split == 0) {
+    small_blocks_last();
+    return launch_shape<false, 8>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+  }
   const int rest = n_wg - n_full;
   const dim3 grid_full = n_full > 0 ? xcd_grid(&p, n_qwg, n_full, &wg_per_xcd) : dim3(0);
   p.split_first_block = (int)grid_full.x;

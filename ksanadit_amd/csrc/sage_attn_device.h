@@ -35,6 +35,18 @@ constexpr float kLazyMax = 2.7f, kLazyMaxPwl = 0.0f;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// The counts of batch entry b in place of the lengths lq, lk the tensors have, where the caller gave any: one wait for both
+// scalar loads.  (Left to the compiler they are vector loads, one after the other: two memory latencies before a workgroup
+// knows whether it has anything to do.)
+__device__ __forceinline__ void take_counts(const int32_t* q_lens, const int32_t* k_lens, int b, int& lq, int& lk) {
+  typedef const __attribute__((address_space(4))) int32_t* Constant;
+  if (q_lens == nullptr && k_lens == nullptr) return;
+  const int nq = *reinterpret_cast<Constant>(reinterpret_cast<uintptr_t>((q_lens != nullptr ? q_lens : k_lens) + b));
+  const int nk = *reinterpret_cast<Constant>(reinterpret_cast<uintptr_t>((k_lens != nullptr ? k_lens : q_lens) + b));
+  if (q_lens != nullptr) lq = rows_counted(nq, lq);
+  if (k_lens != nullptr) lk = rows_counted(nk, lk);
+}
+
 // Opaque use+def at this program point: keeps the optimizer from sinking the computation of
 // `x` into a later basic block (it emits no instruction).
 template <typename T>
@@ -76,6 +88,14 @@ __device__ __forceinline__ void store4(uint16_t* dst, float a, float b, float c,
 __device__ __forceinline__ void lds_copy16(const void* gbase, unsigned lane_off, const void* lds_dst) {
   const unsigned lds_off = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)lds_dst;
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds_off), "v"(lane_off), "s"(gbase)
+               : "memory", "m0");
+}
+// ... and 4 bytes per lane, to `lds_dst + 4 * lane`
+__device__ __forceinline__ void lds_copy4(const void* gbase, unsigned lane_off, const void* lds_dst) {
+  const unsigned lds_off = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)lds_dst;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                :
                : "s"(lds_off), "v"(lane_off), "s"(gbase)
                : "memory", "m0");

@@ -63,8 +63,7 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c,
   const bool my_rows = (wave ^ 4) * 32 < rows_wg;
   const int q0 = qwg * rows_wg + (wave ^ 4) * 32, row = q0 + l32;
   int lq = c.Lq, lk = c.Lk;  // rows and keys that take part
-  if (c.q_lens != nullptr) lq = rows_counted(c.q_lens[b], c.Lq);
-  if (c.k_lens != nullptr) lk = rows_counted(c.k_lens[b], c.Lk);
+  take_counts(c.q_lens, c.k_lens, b, lq, lk);
   if (lk == 0 || qwg * rows_wg >= lq) {  // uniform: softmax over no key, or no row that takes part
     if (my_rows && row < c.Lq && 64 * hh < c.d_out) {
       uint4* orow = reinterpret_cast<uint4*>(c.o.ptr + b * c.o.sB + (int64_t)row * c.o.sL + h * c.o.sH + 64 * hh);
