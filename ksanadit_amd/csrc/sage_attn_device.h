@@ -104,10 +104,11 @@ __device__ __forceinline__ void lds_copy4(const void* gbase, unsigned lane_off, 
 
 // Tiles of which a lane's query sees the first n keys only - the one on a wave's diagonal (n depends on the lane) and a
 // head's last one where its keys are no multiple of 64: the scores of the others drop below every real score (hh = lane / 32)
-template <int kMagicBits>
+// (kHalves: 1 where only the tile's first 32 keys are looked at)
+template <int kMagicBits, int kHalves = 2>
 __device__ __forceinline__ void blank_scores(v16i (&blk)[2], int hh, int n) {
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
+  for (int t = 0; t < kHalves; ++t) {
     // (pinned: what follows is the same in every step, and hoisted out of the key loop it would sit in
     // 32 scalar register pairs for a block that runs once per wave)
     int last = n - 1 - 4 * hh;
@@ -121,11 +122,12 @@ __device__ __forceinline__ void blank_scores(v16i (&blk)[2], int hh, int n) {
 }
 // ... and their probability bytes are cleared outright (code 0 is +0.0 in e4m3), so that a row
 // whose scale is zero does not count them either
+template <int kHalves = 2>
 __device__ __forceinline__ void blank_probs(v8i& pf, int hh, int n) {
   int first = n - 4 * hh;
   pin(first);
 #pragma unroll
-  for (int w = 0; w < 8; ++w) {
+  for (int w = 0; w < 4 * kHalves; ++w) {
     // bytes of the first min(max(m, 0), 4) keys of this dword stay
     const int m = min(max(first - (32 * (w >> 2) + 8 * (w & 3)), 0), 4);
     const unsigned keep = m >= 4 ? 0xffffffffu : ((1u << (8 * m)) - 1u);
@@ -161,10 +163,11 @@ __device__ __forceinline__ float move_point(int imax, float& sc, float& mneg, fl
 }
 
 // the probabilities of a tile as the product with V takes them: 2^(sc * dot + xc - magic * sc), the magic folded into xc, in e4m3
+template <int kHalves = 2>
 __device__ __forceinline__ v8i tile_probs(const v16i (&s)[2], float sc, float xc) {
-  v8i pf;
+  v8i pf = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-  for (int w = 0; w < 8; ++w) {
+  for (int w = 0; w < 4 * kHalves; ++w) {
     float e[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) e[i] = fast_exp2(__builtin_fmaf(__int_as_float(s[w >> 2][4 * (w & 3) + i]), sc, xc));

@@ -327,6 +327,8 @@ struct SmallCall {
   float premul;
   int smooth_k, causal, d_out;
   const int32_t *q_lens, *k_lens;  // as in AttnParams
+  int group;             // Hq / Hkv, and the reciprocal that divides by it (launch_small)
+  unsigned group_magic;
 };
 bool small_call_suits(int B, int Hq, int Lq, int Lk);
 hipError_t launch_small(const SmallCall& c, hipStream_t s);

@@ -109,3 +109,16 @@ def test_captured_and_replayed(hip_device):
         torch.cuda.synchronize()
         assert torch.equal(out, want), i
         assert torch.equal(sage_ops.sageattn(q, k, v), want)
+
+
+@pytest.mark.parametrize("pairs,Lq", [((1, 4), 65), ((2, 64), 64), ((2, 64), 65), ((2, 64), 97), ((2, 64), 130), ((2, 64), 257), ((4, 64), 33), ((4, 64), 225)])
+@pytest.mark.parametrize("Lk", [32, 33, 97, 160])
+@pytest.mark.parametrize("D", [64, 128])
+def test_every_size_of_workgroup(hip_device, pairs, Lq, Lk, D):
+    """32, 64, 128 and 256 query rows a workgroup (the fewest that leave a compute unit to each), with row groups that are part
+    full or empty, and last tiles of at most 32 keys, of which the second half is left out."""
+    (B, H), dtype = pairs, torch.float16 if Lk & 1 else torch.bfloat16
+    print(f"case {pairs} Lq={Lq} Lk={Lk} D={D}", flush=True)
+    q, k, v = (t.to(hip_device) for t in _tensors(B, Lq, Lk, H, H // 2, D, dtype, Lq + Lk + D))
+    _same(q, k, v)
+    _same(q, k, v, is_causal=True, k_lens=[Lk - 7 * b for b in range(B)], q_lens=[max(0, Lq - 40 * b) for b in range(B)])
