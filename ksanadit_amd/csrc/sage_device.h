@@ -79,6 +79,63 @@ __device__ __forceinline__ float lane_xor(float v) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(t, 0x1B, 0xF, 0xF, true));
 }
 
+// Reductions over the lanes of a wave without the LDS crossbar: partners meet through DPP and the lane swaps, whose results the
+// next instruction can have, where a shuffle is an LDS round trip - 48 of them stood between a chunk's last row and its sums.  us per
+// call, shuffles / this: 40 heads of 1560 tokens 58.2 / 57.0, joint block of 2 x 774 tokens of 24 heads 50.8 / 49.2, sparse-linear
+// call of 40 heads of 32760 rows 1895 / 1869, of 2 x 40 of 29672 2352 / 2300 (the averages of its blocks), V smoothing 66.0 / 64.2.
+struct Sum {
+  static __device__ __forceinline__ float of(float a, float b) { return a + b; }
+};
+struct Max {
+  static __device__ __forceinline__ float of(float a, float b) { return fmaxf(a, b); }
+};
+// v of this lane and of lane ^ 32
+template <typename Op>
+__device__ __forceinline__ float over_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return Op::of(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// v of this lane and of lane ^ 8, ^ 16, ^ 32 in turn: the adjacent-pair tree over a wave's eight row slots
+template <typename Op>
+__device__ __forceinline__ float over_slots(float v) {
+  v = Op::of(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xF, 0xF, true)));  // row_ror:8
+  const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = Op::of(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
+  return over_halves<Op>(v);
+}
+// The same tree for the sixteen channels of a lane, each result in a quarter of the lanes only: a swap hands over one value
+// while it fetches another, so two channels cost one exchange.  Lane: channels 8 (lane / 16 % 2) + 4 (lane / 32) + 0 .. 3.
+template <typename Op>
+__device__ __forceinline__ float4 over_slots16(const float (&v)[16]) {
+  float x[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) x[e] = Op::of(v[e], __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[e]), 0x128, 0xF, 0xF, true)));
+  float y[8], z[4];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[e]), __float_as_uint(x[e + 8]), false, false);
+    y[e] = Op::of(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[e]), __float_as_uint(y[e + 4]), false, false);
+    z[e] = Op::of(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  }
+  return make_float4(z[0], z[1], z[2], z[3]);
+}
+// .. and where it goes: the wave's 128 channels, 16-byte aligned
+__device__ __forceinline__ void store_slots16(const float4& v, int lane, float* row) {
+  if ((lane & 8) == 0) *reinterpret_cast<float4*>(row + (lane & 7) * 16 + 8 * ((lane >> 4) & 1) + 4 * (lane >> 5)) = v;
+}
+// all 64 lanes, as a tree over adjacent pairs; every lane gets the result
+template <typename Op>
+__device__ __forceinline__ float over_lanes(float v) {
+  v = Op::of(v, lane_xor<1>(v));
+  v = Op::of(v, lane_xor<2>(v));
+  v = Op::of(v, lane_xor<4>(v));
+  return over_slots<Op>(v);
+}
+
 // One butterfly stage across lanes c16 and c16 ^ M: every lane takes `own + sign * other` with sign = -1 on the lane
 // that holds the "b" half of a pair.  That lane ought to take `other - own`: it ends up with the negative of its
 // value, exactly (a sum and its mirror image round alike).  Both lanes of any LATER stage's pair agree in bit M of

@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/ksana_sage_hip.h"
 
@@ -335,8 +336,7 @@ __device__ __forceinline__ float row_inv_rms_of(const uint16_t* base, int n8, fl
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc = acc + v[e] * v[e];
   }
-#pragma unroll
-  for (int m = 1; m <= 32; m <<= 1) acc = acc + __shfl_xor(acc, m);
+  acc = over_lanes<Sum>(acc);
   // sqrtf, not __fsqrt_rn: the latter is the 1-ulp native instruction in this toolchain, the former is
   // correctly rounded (the build passes -fhip-fp32-correctly-rounded-divide-sqrt)
   return __fdiv_rn(1.0f, sqrtf(__fdiv_rn(acc, n_channels) + eps));
@@ -432,21 +432,9 @@ __device__ __forceinline__ void col_partial_chunk(int ch, int h, int b, const ui
       }
     }
   }
-  // slots of one wave differ in lane bits 3..5
-#pragma unroll
-  for (int m = 8; m <= 32; m <<= 1) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const float o = __shfl_xor(acc[e], m);
-      acc[e] = kSum ? acc[e] + o : fmaxf(acc[e], o);
-    }
-  }
-  __shared__ float s_w[4][kD];
+  __shared__ __attribute__((aligned(16))) float s_w[4][kD];
   const int wave = t >> 6, lane = t & 63;
-  if (lane < 8) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) s_w[wave][c16 * 16 + e] = acc[e];
-  }
+  store_slots16(over_slots16<typename std::conditional<kSum, Sum, Max>::type>(acc), lane, s_w[wave]);
   __syncthreads();
   if (t < kD) {
     const float lo = kSum ? s_w[0][t] + s_w[1][t] : fmaxf(s_w[0][t], s_w[1][t]);
@@ -542,8 +530,7 @@ __global__ __launch_bounds__(kFinThreads) void v_scale_finalize_kernel(const flo
 
 // max over the workgroup of a non-negative per-thread value
 __device__ __forceinline__ float block_max(float v, float* s_red) {
-#pragma unroll
-  for (int m = 1; m <= 32; m <<= 1) v = fmaxf(v, __shfl_xor(v, m));
+  v = over_lanes<Max>(v);
   const int wave = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) s_red[wave] = v;
   __syncthreads();
@@ -557,17 +544,8 @@ __device__ __forceinline__ float block_max(float v, float* s_red) {
 template <int DT>
 __device__ __forceinline__ void store_block_mean(float (&acc)[16], int t, float n_rows, uint16_t* __restrict__ out_row,
                                                  float (*s_w)[kD]) {
-  const int c16 = t & 7;
-#pragma unroll
-  for (int m = 8; m <= 32; m <<= 1) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = acc[e] + __shfl_xor(acc[e], m);
-  }
   const int wave = t >> 6, lane = t & 63;
-  if (lane < 8) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) s_w[wave][c16 * 16 + e] = acc[e];
-  }
+  store_slots16(over_slots16<Sum>(acc), lane, s_w[wave]);
   __syncthreads();
   if (t < kD) {
     const float sum = (s_w[0][t] + s_w[1][t]) + (s_w[2][t] + s_w[3][t]);
@@ -652,7 +630,7 @@ __device__ __forceinline__ void quant_q_block(int blk, int h, int b, const uint1
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[e] = ((x[0][e] + x[1][e]) + x[2][e]) + x[3][e];
       static_assert(R == 4, "four rows per slot");
-      __shared__ float s_w[4][kD];
+      __shared__ __attribute__((aligned(16))) float s_w[4][kD];
       store_block_mean<DT>(acc, t, (float)min(kRowsPerWg, L_all - blk * kRowsPerWg),
                            pooled + (bh * (lq_pad / kRowsPerWg) + blk) * kD, s_w);
     }
@@ -730,9 +708,7 @@ __global__ __launch_bounds__(kThreads) void quant_q_rows_kernel(const uint16_t* 
     }
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-      float a = acc[i];
-#pragma unroll
-      for (int m = 1; m <= 32; m <<= 1) a = a + __shfl_xor(a, m);
+      const float a = over_lanes<Sum>(acc[i]);
       const float r = __fdiv_rn(1.0f, sqrtf(__fdiv_rn(a, n_channels) + eps));
       if (lane == 0 && first + i < xL) {
         out[(int64_t)b * xL + first + i] = r;
@@ -876,7 +852,7 @@ __device__ __forceinline__ void quant_k_block(int blk, int h, int b, const uint1
     for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(x[i][e]));
   }
   if constexpr (POOL) {
-    __shared__ float s_w[4][kD];
+    __shared__ __attribute__((aligned(16))) float s_w[4][kD];
     store_block_mean<DT>(pool_acc, t, (float)min(kBlkK, L_all - blk * kBlkK), pooled + (bh * nkb + blk) * kD, s_w);
   }
   __shared__ float s_red[4];
@@ -1147,7 +1123,7 @@ __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __
   const int wave = t >> 6, lane = t & 63;
   const uint16_t* base = k + b * sB + h * sH + c16 * 16;
   const RopeLds rl = maybe_stage_rope<PRE>(pp, b, ch * kMeanChunk, kMeanChunk);
-  __shared__ float s_w[4][kD];
+  __shared__ __attribute__((aligned(16))) float s_w[4][kD];
   __shared__ float s_mean[kD];
   __shared__ float s_red[4][4];
   __shared__ int s_last;
@@ -1183,11 +1159,7 @@ __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __
     for (int e = 0; e < 16; ++e) acc[e] = i == 0 ? x[e] : acc[e] + x[e];
   }
   forget_derived(raw);
-#pragma unroll
-  for (int m = 8; m <= 32; m <<= 1) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = acc[e] + __shfl_xor(acc[e], m);
-  }
+  const float4 sums = over_slots16<Sum>(acc);
   if (!smooth) {  // uniform: nothing is taken off, nothing to wait for
     if (t < kD) {
       s_mean[t] = 0.0f;
@@ -1195,10 +1167,7 @@ __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __
     }
     __syncthreads();
   } else {
-  if (lane < 8) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) s_w[wave][c16 * 16 + e] = acc[e];
-  }
+  store_slots16(sums, lane, s_w[wave]);
   __syncthreads();
   if constexpr (SOLO) {
     if (t < kD) {
@@ -1276,16 +1245,9 @@ __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __
 #pragma unroll
           for (int e = 0; e < 16; ++e) a16[e] = i == 0 ? x[e] : a16[e] + x[e];
         }
-#pragma unroll
-        for (int m = 8; m <= 32; m <<= 1) {
-#pragma unroll
-          for (int e = 0; e < 16; ++e) a16[e] = a16[e] + __shfl_xor(a16[e], m);
-        }
+        const float4 part16 = over_slots16<Sum>(a16);
         __syncthreads();  // s_w of the chunk before has been read
-        if (lane < 8) {
-#pragma unroll
-          for (int e = 0; e < 16; ++e) s_w[wave][c16 * 16 + e] = a16[e];
-        }
+        store_slots16(part16, lane, s_w[wave]);
         __syncthreads();
         if (t < kD) {
           const float pc = (s_w[0][t] + s_w[1][t]) + (s_w[2][t] + s_w[3][t]);
@@ -1316,8 +1278,7 @@ __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __
 #pragma unroll
       for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(x[i][e]));
     }
-#pragma unroll
-    for (int m = 1; m <= 32; m <<= 1) amax = fmaxf(amax, __shfl_xor(amax, m));
+    amax = over_lanes<Max>(amax);
     if (lane == 0) s_red[tt][wave] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(s_red[tt][0], s_red[tt][1]), fmaxf(s_red[tt][2], s_red[tt][3]));
@@ -1364,7 +1325,7 @@ __device__ __forceinline__ void quant_v_chunk(int bh, int ch, const uint16_t* __
   const int L = c16 * 16 < d_in ? L_all : 0;  // channels at or past d_in (head size 64) read as zero padding
   const int wave = t >> 6, lane = t & 63;
   const uint16_t* base = v + b * sB + h * sH + c16 * 16;
-  __shared__ float s_w[4][kD];
+  __shared__ __attribute__((aligned(16))) float s_w[4][kD];
   __shared__ float s_inv[kD];
   __shared__ int s_last;
   constexpr int kStride = kD + 16;  // LDS row pitch in bytes
@@ -1387,15 +1348,7 @@ __device__ __forceinline__ void quant_v_chunk(int bh, int ch, const uint16_t* __
     for (int e = 0; e < 16; ++e) acc[e] = i == 0 ? fabsf(x[e]) : fmaxf(acc[e], fabsf(x[e]));
   }
   forget_derived(raw);
-#pragma unroll
-  for (int m = 8; m <= 32; m <<= 1) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = fmaxf(acc[e], __shfl_xor(acc[e], m));
-  }
-  if (lane < 8) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) s_w[wave][c16 * 16 + e] = acc[e];
-  }
+  store_slots16(over_slots16<Max>(acc), lane, s_w[wave]);
   __syncthreads();
   if constexpr (SOLO) {
     if (t < kD) {
@@ -1464,16 +1417,9 @@ __device__ __forceinline__ void quant_v_chunk(int bh, int ch, const uint16_t* __
 #pragma unroll
         for (int e = 0; e < 16; ++e) m16[e] = fmaxf(m16[e], fabsf(x[e]));
       }
-#pragma unroll
-      for (int m = 8; m <= 32; m <<= 1) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) m16[e] = fmaxf(m16[e], __shfl_xor(m16[e], m));
-      }
+      const float4 top16 = over_slots16<Max>(m16);
       __syncthreads();  // s_w of step 1 has been read
-      if (lane < 8) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) s_w[wave][c16 * 16 + e] = m16[e];
-      }
+      store_slots16(top16, lane, s_w[wave]);
       __syncthreads();
       if (t < kD) {
         const float amax = fmaxf(fmaxf(s_w[0][t], s_w[1][t]), fmaxf(s_w[2][t], s_w[3][t]));
@@ -1719,19 +1665,11 @@ __device__ __forceinline__ void joint_k_sums(int item, const QkvCall& c, const P
   add_row(0, true);
 #pragma unroll 1  // (unrolled, the rows' work is pulled together and spills)
   for (int i = 1; i < kMeanChunk / kSlots; ++i) add_row(i, false);
-  __shared__ float s_w[kJointHeadsK][4][kD];
+  __shared__ __attribute__((aligned(16))) float s_w[kJointHeadsK][4][kD];
   const int wave = t >> 6, lane = t & 63;
 #pragma unroll
   for (int hh = 0; hh < kJointHeadsK; ++hh) {
-#pragma unroll
-    for (int m = 8; m <= 32; m <<= 1) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[hh][e] = acc[hh][e] + __shfl_xor(acc[hh][e], m);
-    }
-    if (lane < 8) {
-#pragma unroll
-      for (int e = 0; e < 16; ++e) s_w[hh][wave][c16 * 16 + e] = acc[hh][e];
-    }
+    store_slots16(over_slots16<Sum>(acc[hh]), lane, s_w[hh][wave]);
   }
   __syncthreads();
   static_assert(kJointHeadsK * kD == kThreads, "a thread per head and channel");
@@ -1793,8 +1731,7 @@ __device__ __forceinline__ void joint_k_item(int item, const QkvCall& c, const P
       for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(x[i][e]));
       __builtin_amdgcn_sched_barrier(0);
     }
-#pragma unroll
-    for (int m = 1; m <= 32; m <<= 1) amax = fmaxf(amax, __shfl_xor(amax, m));
+    amax = over_lanes<Max>(amax);
     if ((t & 63) == 0) s_red[hh][wave] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(s_red[hh][0], s_red[hh][1]), fmaxf(s_red[hh][2], s_red[hh][3]));
@@ -2019,7 +1956,7 @@ __global__ __launch_bounds__(kThreads) void block_mean_kernel(const uint16_t* __
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = i == 0 ? v[e] : acc[e] + v[e];
   }
-  __shared__ float s_w[4][kD];
+  __shared__ __attribute__((aligned(16))) float s_w[4][kD];
   store_block_mean<DT>(acc, t, (float)min(rows, L - blk * rows), out + (bh * gridDim.x + blk) * kD, s_w);
 }
 

@@ -373,7 +373,7 @@ __device__ __forceinline__ float sla_row_exps(const uint4 (&raw)[8], float (&x)[
 #pragma unroll
     for (int e = 0; e < 8; ++e) mx = fmaxf(mx, x[s][e]);
   }
-  mx = fmaxf(mx, __shfl_xor(mx, 32));
+  mx = over_halves<Max>(mx);
   const float c = -mx * kLog2e;
   float sum = 0.0f;
 #pragma unroll
@@ -383,7 +383,7 @@ __device__ __forceinline__ float sla_row_exps(const uint4 (&raw)[8], float (&x)[
       x[s][e] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[s][e], kLog2e, c));
       sum += x[s][e];
     }
-  sum += __shfl_xor(sum, 32);
+  sum = over_halves<Sum>(sum);
   return __builtin_amdgcn_rcpf(sum);
 }
 // the operands fq (phi in the half type) and 1 / (1e-5 + phi . ksum); s_ks: ksum of the head, in LDS
@@ -402,7 +402,7 @@ __device__ __forceinline__ float sla_row_scale(const float (&x)[8][8], float inv
     }
     fq[s] = make_uint4(pw[0], pw[1], pw[2], pw[3]);
   }
-  den += __shfl_xor(den, 32);
+  den = over_halves<Sum>(den);
   return __builtin_amdgcn_rcpf(1e-5f + den);
 }
 // Output channels 32 nt .. + 31 of the lane's row, transposed (out^T = M^T phi(q)^T): register r is channel

@@ -33,42 +33,6 @@ constexpr int kSmallFloats = 8 * kD + 3 * kD + kMaxTiles + 4 * kMaxTiles;
 // LDS: K tiles, V^T tiles; V's codes row by row; Q's operands and scales; small things
 constexpr size_t small_lds(int n, int rows_wg) { return 2 * n * kTileBytes + n * kBlkK * kVPitch + rows_wg * (kD + 4) + kSmallFloats * 4; }
 
-struct Sum {
-  static __device__ __forceinline__ float of(float a, float b) { return a + b; }
-};
-struct Max {
-  static __device__ __forceinline__ float of(float a, float b) { return fmaxf(a, b); }
-};
-// v of this lane and of lane ^ 8, ^ 16, ^ 32 in turn: the adjacent-pair tree over a wave's eight row slots
-template <typename Op>
-__device__ __forceinline__ float over_slots(float v) {
-  v = Op::of(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xF, 0xF, true)));  // row_ror:8
-  const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = Op::of(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
-  const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return Op::of(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
-}
-// The same tree for the sixteen channels of a lane, each result in a quarter of the lanes only: a swap hands over one value
-// while it fetches another, so two channels cost one exchange.  Lane: channels 8 (lane / 16 % 2) + 4 (lane / 32) + 0 .. 3.
-template <typename Op>
-__device__ __forceinline__ float4 over_slots16(const float (&v)[16]) {
-  float x[16];
-#pragma unroll
-  for (int e = 0; e < 16; ++e) x[e] = Op::of(v[e], __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v[e]), 0x128, 0xF, 0xF, true)));
-  float y[8], z[4];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[e]), __float_as_uint(x[e + 8]), false, false);
-    y[e] = Op::of(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(y[e]), __float_as_uint(y[e + 4]), false, false);
-    z[e] = Op::of(__uint_as_float(r[0]), __uint_as_float(r[1]));
-  }
-  return make_float4(z[0], z[1], z[2], z[3]);
-}
-
 // kG: 32-channel groups that hold data, as in the general kernel.  kRows: query rows of a workgroup.
 template <int DT, int kG, int kRows>
 __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c) {
@@ -175,8 +139,7 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c)
       }
       part = over_slots16<Max>(acc);
     }
-    if ((lane & 8) == 0)
-      *reinterpret_cast<float4*>(&(on_k ? s_k : s_v)[w4][c16 * 16 + 8 * ((lane >> 4) & 1) + 4 * hh]) = part;
+    store_slots16(part, lane, (on_k ? s_k : s_v)[w4]);
   }
   __syncthreads();
   if (t < kD) {
@@ -228,10 +191,7 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c)
 #pragma unroll
         for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(x[tt][i][e]));
       }
-      amax = fmaxf(amax, lane_xor<1>(amax));
-      amax = fmaxf(amax, lane_xor<2>(amax));
-      amax = fmaxf(amax, lane_xor<4>(amax));
-      amax = over_slots<Max>(amax);
+      amax = over_lanes<Max>(amax);
       if (lane == 0) s_red[tt][w4] = amax;
     }
   } else {
