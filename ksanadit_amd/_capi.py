@@ -11,7 +11,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "libksana_sage_hip.so"
-ABI_VERSION = 23
+ABI_VERSION = 24
 
 BF16, FP16 = 0, 1
 OK, EINVAL, ENOTSUP, EHIP = 0, -1, -2, -3
@@ -55,6 +55,7 @@ EXPORTS = (
     "ksana_sage_attn_fwd_varlen",
     "ksana_sage_forward_masked",
     "ksana_sage_forward_varlen",
+    "ksana_sage_forward_call",
     "ksana_sage_forward_scratch",
     "ksana_sage_sla_forward_bytes",
     "ksana_sage_sla_forward",
@@ -94,6 +95,13 @@ class Prep(C.Structure):
         ("rope_freqs_img", C.c_void_p),
         ("rope_matrices", C.c_void_p),
     ]
+
+
+class Call(C.Structure):
+    """``ksana_sage_call``: a plain forward call but for its buffers and its stream."""
+
+    _fields_ = [("shape", Shape)] + [(n, C.c_int32) for n in ("dtype", "o_dtype", "smooth_k", "causal", "flags")] + \
+        [("sm_scale", C.c_float)] + [(n, C.c_int64 * 4) for n in ("q_strides", "k_strides", "v_strides", "o_strides")]
 
 
 class SageLibraryError(RuntimeError):
@@ -159,6 +167,7 @@ def _declare(lib):
     # converts in a fraction of the time its pointer objects take)
     lib.ksana_sage_forward_varlen.argtypes = [vp, vp, vp, vp, i, i, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, f, i, i, i, vp, vp]
     lib.ksana_sage_forward_varlen.restype = i
+    lib.ksana_sage_forward_call.argtypes, lib.ksana_sage_forward_call.restype = [vp] * 7, i
 
 
 def library_present() -> bool:

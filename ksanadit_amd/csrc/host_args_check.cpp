@@ -120,6 +120,13 @@ int main() {
   EXPECT(ksana_sage_attn_fwd_masked(fake, fake, KSANA_SAGE_BF16, st, &s, reinterpret_cast<const int8_t*>(fake), neg, nullptr, 0, 0, nullptr),
          KSANA_SAGE_EINVAL);
   EXPECT(ksana_sage_forward(fake, fake, nullptr, fake, KSANA_SAGE_BF16, st, st, st, st, &s, nullptr, 0.1f, 1, 0, 0, fake, nullptr), KSANA_SAGE_EINVAL);
+  ksana_sage_call call{s, KSANA_SAGE_BF16, KSANA_SAGE_BF16, 1, 0, 0, 0.1f, {}, {}, {}, {}};
+  for (int64_t* to : {call.q_strides, call.k_strides, call.v_strides, call.o_strides}) std::memcpy(to, st, sizeof(st));
+  EXPECT(ksana_sage_forward_call(nullptr, fake, fake, fake, fake, fake, nullptr), KSANA_SAGE_EINVAL);
+  EXPECT(ksana_sage_forward_call(&call, fake, fake, fake, nullptr, fake, nullptr), KSANA_SAGE_EINVAL);
+  EXPECT(ksana_sage_forward_call(&call, fake, fake, fake, fake, nullptr, nullptr), KSANA_SAGE_EINVAL);
+  call.flags = 0x4000;
+  EXPECT(ksana_sage_forward_call(&call, fake, fake, fake, fake, fake, nullptr), KSANA_SAGE_EINVAL);
   int first = -1, runs = -1;
   EXPECT(ksana_sage_attn_key_split(&s, &first, nullptr), KSANA_SAGE_EINVAL);
 

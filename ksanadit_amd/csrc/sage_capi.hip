@@ -842,6 +842,12 @@ int ksana_sage_forward_varlen(const void* q, const void* k, const void* v, void*
                       smooth_k, causal, flags, ws, stream);
 }
 
+int ksana_sage_forward_call(const ksana_sage_call* c, const void* q, const void* k, const void* v, void* o, void* ws, void* stream) {
+  if (!c) return fail(KSANA_SAGE_EINVAL, "call is null");
+  return forward_impl(q, k, v, o, c->dtype, c->o_dtype, c->q_strides, c->k_strides, c->v_strides, c->o_strides, &c->shape, nullptr, nullptr,
+                      nullptr, nullptr, nullptr, c->sm_scale, c->smooth_k, c->causal, c->flags, ws, stream);
+}
+
 }  // extern "C"
 
 namespace {

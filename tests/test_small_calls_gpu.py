@@ -122,3 +122,31 @@ def test_every_size_of_workgroup(hip_device, pairs, Lq, Lk, D):
     q, k, v = (t.to(hip_device) for t in _tensors(B, Lq, Lk, H, H // 2, D, dtype, Lq + Lk + D))
     _same(q, k, v)
     _same(q, k, v, is_causal=True, k_lens=[Lk - 7 * b for b in range(B)], q_lens=[max(0, Lq - 40 * b) for b in range(B)])
+
+
+@pytest.mark.parametrize("Lk", [40, 300])
+def test_calls_without_options_and_the_general_call(hip_device, Lk):
+    """A repeated call without options takes a shorter way to the library than one with an option that changes nothing
+    (``out_dtype`` = the inputs' dtype): same result, same layout, whatever the layout and the kinds of its scalars."""
+    print(f"case {Lk}", flush=True)
+    q, k, v = (t.to(hip_device) for t in _tensors(2, 50, Lk, 4, 2, 128, torch.bfloat16, Lk))
+    wide = [torch.cat([t, t], dim=3)[..., :128] for t in (q, k, v)]
+    one = [t[:1] for t in (q, k, v)]
+    odd = [t.as_strided((1, *t.shape[1:]), (8, *t.stride()[1:])) for t in (q, k, v)]  # an entry's stride nobody uses
+    swapped = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v)]
+    for tensors in ([q, k, v], wide, one, odd, swapped, [t.half() for t in (q, k, v)], [torch.nn.Parameter(t) for t in (q, k, v)]):
+        for kw in ({}, {"sm_scale": 0.11}, {"sm_scale": 0.07, "is_causal": True}, {"smooth_k": False}, {"is_causal": 1, "sm_scale": 1}):
+            want = sage_ops.sageattn(*tensors, **kw, out_dtype=tensors[0].dtype)
+            for _ in range(2):
+                out = sage_ops.sageattn(*tensors, **kw)
+                assert torch.equal(out, want) and out.stride() == want.stride() and out.dtype == want.dtype and type(out) is torch.Tensor
+    scale = torch.tensor(0.1)
+    first = sage_ops.sageattn(q, k, v, sm_scale=scale)
+    scale.fill_(0.3)  # a scale that is a tensor is read in every call
+    assert torch.equal(sage_ops.sageattn(q, k, v, sm_scale=scale), sage_ops.sageattn(q, k, v, sm_scale=scale.item()))
+    assert not torch.equal(sage_ops.sageattn(q, k, v, sm_scale=scale), first)
+    for i in range(20):  # more settings than are kept
+        assert torch.equal(sage_ops.sageattn(q, k, v, sm_scale=0.01 * i), sage_ops.sageattn(q, k, v, sm_scale=0.01 * i, out_dtype=q.dtype)), i
+    empty = q[:, :0]
+    for _ in range(2):
+        assert sage_ops.sageattn(empty, k, v).shape == empty.shape
