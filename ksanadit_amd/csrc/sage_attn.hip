@@ -768,9 +768,14 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     const v8i vf = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     oacc[dt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf, pf, oacc[dt], 0, 0, 0, 0, 0, 0);
   };
-  // S^T chunk i of a step is (channel step i / 2, key half i % 2); the chunks of channel steps without data carry only
-  // their share of the probabilities
-  auto has_qk = [](int i) { return i >= 0 && i < 8 && (i >> 1) < kG; };
+  // S^T chunk i of a step: its channel step and half of the keys; the chunks without a product carry only their share of the
+  // probabilities.  Two products in turn share Q's operand; in 8 waves with 64 channels a half is finished before the other.  us
+  // per call, shared / one half after the other: 32760 tokens of 40 heads of 64 channels 8145 / 8046, 9001 of 2 x 16 549.5 /
+  // 544.3; in 4 waves 3000 of 8 40.7 / 41.0, with 128 channels 27280 of 24 4664 / 4676.
+  constexpr bool kByHalves = kG == 2 && kW == 8;
+  auto qk_step = [](int i) { return kByHalves ? i % kG : i >> 1; };
+  auto qk_half = [](int i) { return kByHalves ? i / kG : i & 1; };
+  auto has_qk = [](int i) { return i >= 0 && i < 2 * kG; };
 
   v16i s_a[2], s_b[2];
   qk_tile<kG>(k_slot(0), lane, qf, magic, s_a);
@@ -841,7 +846,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     constexpr int kAt = decltype(at)::value;
     const uint8_t* kst = k_slot(kAt >= 0 ? kAt + 1 : j + 1);
     const uint8_t* vst = v_slot(kAt >= 0 ? kAt - 1 : j - 1);
-    auto k_frag = [&](int i) { return *reinterpret_cast<const v4i*>(kst + (((i & 1) * 4 + (i >> 1)) * 64 + lane) * 16); };
+    auto k_frag = [&](int i) { return *reinterpret_cast<const v4i*>(kst + ((qk_half(i) * 4 + qk_step(i)) * 64 + lane) * 16); };
     auto v_frag = [&](int dt) {
       const v4i lo = *reinterpret_cast<const v4i*>(vst + ((dt * 2 + 0) * 64 + lane) * 16);
       const v4i hi = *reinterpret_cast<const v4i*>(vst + ((dt * 2 + 1) * 64 + lane) * 16);
@@ -871,7 +876,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     // 8 x [S^T MFMA of tile j+1 (32 matrix cycles) | 2 probabilities of tile j]
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int s = i >> 1, t = i & 1;
+      const int s = qk_step(i) & 3, t = qk_half(i) & 1;
       if (i + 3 < 8) {
         if (has_qk(i + 3)) kf[(i + 3) & 3] = k_frag(i + 3);
       } else if (i + 3 - 8 < kG) {
