@@ -80,6 +80,44 @@ __device__ __forceinline__ void lds_copy16_at(const v4i& buffer, unsigned lane_o
 }
 #pragma clang diagnostic pop
 
+// Which workgroup of a batch with counts of its own is number `at` of XCD `xcd`: an eighth of every entry's blocks with rows that
+// take part to every XCD, the entry with the most keys first, then an eighth of every entry's other blocks, which have only zeros
+// to write (-1: no such workgroup); and its entry's counts.  The counts are in device memory, so every workgroup works this out by itself, an entry per lane.
+// In the order of their index, an entry's blocks without rows stand before the next entry's: work waits for a place while they
+// come and go.  us per call, by index / like this, entries falling off to 45 %: 5 x 32 heads of 1500 tokens 140 / 132, 6 x 64 of 2000
+// 373 / 353, 3 x 24 of 3001 on 4099 184.3 / 180.7, 2 x 12 of 6946 on 138 38.1 / 37.1, 3 x 40 of 8000 1340 / 1337, 2 x 40 of 16384
+// 3419 / 3422.  One round of the chip has no order (6 heads of 5000 66.4 / 67.3: the counts come through vector loads).
+template <int kRowsWg>
+__device__ __forceinline__ int packed_place(const AttnParams& p, int xcd, int at, int n_qwg, int& lq, int& lk) {
+  const int lane = threadIdx.x & 63;
+  int rows = 0, keys = -1, blocks = 0;
+  if (lane < p.B) {
+    rows = p.q_lens != nullptr ? rows_counted(p.q_lens[lane], p.Lq) : p.Lq;
+    keys = p.k_lens != nullptr ? rows_counted(p.k_lens[lane], p.Lk) : p.Lk;
+    if (keys > 0) blocks = (rows + kRowsWg - 1) / kRowsWg;
+  }
+  int rank = 0;
+  for (int j = 0; j < p.B; ++j) {
+    const int other = __builtin_amdgcn_readlane(keys, j);
+    rank += other > keys || (other == keys && j < lane);
+  }
+  for (int kind = 0; kind < 2; ++kind)  // blocks with rows, the others
+    for (int r = 0; r < p.B; ++r) {
+      const int b = (int)__ffsll((unsigned long long)__ballot(lane < p.B && rank == r)) - 1;
+      const int with_rows = __builtin_amdgcn_readlane(blocks, b), n = kind == 0 ? with_rows : n_qwg - with_rows;
+      const int per = (p.Hq * n + 7) / 8;
+      if (at < per) {
+        const int i = xcd * per + at;
+        if (i >= p.Hq * n) return -1;
+        const int h = i / n;
+        lq = __builtin_amdgcn_readlane(rows, b), lk = __builtin_amdgcn_readlane(keys, b);
+        return (b * p.Hq + h) * n_qwg + (i - h * n) + (kind == 0 ? 0 : with_rows);
+      }
+      at -= per;
+    }
+  return -1;
+}
+
 // Dense 8-wave calls can hold two kinds of workgroup in one grid: blocks below p.split_first_block walk all key tiles of
 // their (head, query block); each of the blocks from there on takes one of `p.n_split` equal runs of key tiles and leaves
 // unnormalised accumulators, running maxima and row sums in the workspace for sage_attn_merge_kernel.  The runs stand
@@ -109,6 +147,10 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   constexpr int kMagicBits = kG == 4 ? kMagicI : kMagicI2;
   constexpr float kMagicVal = kG == 4 ? kMagicF : kMagicF2;
   int bh, qwg;  // (batch, head) pair and query block
+  // query rows [0, lq) of this batch take part: all of them, or the caller's per-batch count; the rows from lq up
+  // to Lq exist in the output and are written as zeros
+  // keys [0, lk) of this batch take part: all of them, or the caller's per-batch count
+  int lq = p.Lq, lk = p.Lk;
   const bool is_run = kCanSplit && (int)blockIdx.x >= p.split_first_block;  // uniform
   const int run_id = is_run ? (int)blockIdx.x - p.split_first_block : 0;    // the partial result's place in the workspace
   if (kCausal && p.causal_grid.group != 0) {
@@ -136,10 +178,14 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
           if (pair >= n_pairs) return;
           wg = pair * n_qwg + n_qwg - 1;
         }
+      } else if (p.packed) {
+        wg = packed_place<kRowsWg>(p, xcd, at, n_qwg, lq, lk);
+        if (wg < 0) return;
       } else if (p.batch_run == 0) {
         wg = xcd * wg_per_xcd + at;
         if (wg >= n_wg) return;
       } else {
+        // (calls whose last blocks are cut, and batches of more than 64 entries; the others: see packed_place)
         // batch entries of unequal length: an eighth of every entry's workgroups to every XCD.  One run across the entries
         // would leave the XCDs that drew the short ones idle.  The entries run in the order of their index, longest first or
         // not: the order that ends with the longest one costs up to 5-8 % in grids of two rounds, nothing in long ones.  us,
@@ -161,11 +207,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform by construction: keep it scalar
   const int l32 = lane & 31, hh = lane >> 5;
-  // query rows [0, lq) of this batch take part: all of them, or the caller's per-batch count; the rows from lq up
-  // to Lq exist in the output and are written as zeros
-  // keys [0, lk) of this batch take part: all of them, or the caller's per-batch count
-  int lq = p.Lq, lk = p.Lk;
-  take_counts(p.q_lens, p.k_lens, b, lq, lk);
+  if (!p.packed) take_counts(p.q_lens, p.k_lens, b, lq, lk);
   // A last block of at most 64 rows has work for one or two waves.  Alone on its unit such a workgroup takes half a microsecond a
   // step, next to another one as long as the whole blocks do; so its four waves share the keys out instead (see below).
   constexpr bool kCanShare = !kSparse && !kCausal && kW == 4 && !kPwlExp && !kTileSkip;
@@ -1362,6 +1404,11 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   const int n_wg = p.B * p.Hq * n_qwg;
   int wg_per_xcd = 0;
   dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
+  auto pack_batch = [&]() {
+    if (p.batch_run == 0 || sparse || p.B > 64 || n_wg <= (waves == 4 ? 2 : 1) * compute_units()) return;
+    p.packed = 1;
+    grid = dim3(8 * p.B * (p.batch_run + 1));  // (either kind of an entry's blocks is divided by eight)
+  };
   if (p.causal && p.batch_run == 0) p.causal_grid = causal_grid(p.B * p.Hq, n_qwg);  // (the same number of workgroups)
   // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
   const size_t lds = (waves == 4 ? WgShape<4>::kRingBytes : WgShape<8>::kRingBytes) + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
@@ -1384,6 +1431,7 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   };
   if (waves == 4) {
     small_blocks_last();
+    pack_batch();
     if (plain_causal) return launch_causal(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
     if (sparse)
       return p.causal ? launch_shape<true, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
@@ -1399,6 +1447,7 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   if (p.split_o != nullptr) plan_key_split(n_wg, p.nkb, &n_full, &n_split);
   if (n_split == 0) {
     small_blocks_last();
+    pack_batch();
     return launch_shape<false, 8>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
   }
   const int rest = n_wg - n_full;

@@ -292,6 +292,7 @@ struct AttnParams {
   float* split_ml;
   int split_first_block = 0, split_first_wg = 0, n_split = 0;  // filled in by the launcher
   int batch_run = 0;  // filled in by the launcher: 0, or the workgroups of one batch entry that go to one XCD
+  int packed = 0;  // filled in by the launcher: the batch's blocks are numbered by its counts (packed_place)
   int small_last = 0;  // filled in by the launcher: 0, or how many heads' short last blocks each XCD takes behind its whole blocks
   int wg_waves;  // 0: the launcher picks the workgroup shape; 4 or 8: forced (for measurements and tests)
   int d_out;     // channels of an output row that exist: 128, or 64 (head size 64 runs zero-padded to 128)

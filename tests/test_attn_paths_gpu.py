@@ -249,3 +249,29 @@ def test_a_shared_last_block_in_batches_with_lengths(hip_device, k_len, rows):
         out, full = call(q_lens=torch.tensor(q_lens, dtype=torch.int32, device=hip_device)), call()
         for b, n in enumerate(q_lens):
             assert torch.equal(out[b, :n], full[b, :n]) and not out[b, n:].isnan().any() and not out[b, n:].any(), b
+
+
+@pytest.mark.parametrize("B,H,Lq,Lk", [(3, 40, 700, 900), (5, 16, 1000, 300), (64, 2, 700, 130), (65, 2, 700, 130), (2, 40, 2000, 700)])
+@pytest.mark.parametrize("wg_waves", [4, 8])
+def test_batches_are_numbered_by_their_counts(hip_device, B, H, Lq, Lk, wg_waves):
+    """Grids of more than a round whose workgroups work out which block is theirs from the entries' counts - in any order, equal,
+    none, one, all, out of range - against the same operands walked through a mask of ones, whose grid is numbered as the
+    tensor is laid out.  (More than 64 entries are, too.)"""
+    print(f"case B={B} H={H} Lq={Lq} Lk={Lk} waves={wg_waves}", flush=True)
+    g = torch.Generator().manual_seed(B * Lq + Lk)
+    q, k, v = (torch.randn((B, n, H, 128), generator=g).to(torch.bfloat16).to(hip_device) for n in (Lq, Lk, Lk))
+    ws = sage_ops.workspace_for(q, k)
+    sage_ops.sageattn(q, k, v, workspace=ws)
+    ones = torch.ones((-(-Lq // 128), -(-Lk // 64)), dtype=torch.int8, device=hip_device)
+    choice = [0, 1, 63, 64, Lk // 2, Lk - 1, Lk, Lk + 100, -5]
+    lens = [torch.randint(0, n + 1, (B,), generator=g) for n in (Lq, Lk)]
+    some = torch.tensor([choice[i % len(choice)] for i in range(B)])
+    for q_lens, k_lens in ((lens[0], lens[1]), (lens[0].flip(0), some), (None, lens[1].sort()[0]), (lens[0], None), (torch.full((B,), Lq), torch.full((B,), Lk)),
+                           (torch.zeros(B, dtype=torch.int64), lens[1])):
+        got, want = torch.full_like(q, 7.0), torch.full_like(q, 9.0)
+        sage_ops.attn_fwd(ws, got, q_lens=q_lens, k_lens=k_lens, wg_waves=wg_waves)
+        sage_ops.attn_fwd(ws, want, q_lens=q_lens, k_lens=k_lens, wg_waves=4, block_mask=ones)
+        assert torch.equal(got, want)
+        if q_lens is not None:
+            for b in range(B):
+                assert (got[b, int(q_lens[b]) :] == 0).all()
