@@ -175,7 +175,7 @@ __device__ __forceinline__ void prep16_qwen(float* x, const QwenRow& f, float ep
   if (f.w != nullptr) {
     float ss = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) ss = e == 0 ? x[0] * x[0] : ss + x[e] * x[e];  // squares of half values are exact
+    for (int e = 0; e < 16; ++e) ss = __fmaf_rn(x[e], x[e], ss);  // squares of half values are exact: one rounding, the sum's
     ss = ss + lane_xor<1>(ss);
     ss = ss + lane_xor<2>(ss);
     ss = ss + lane_xor<4>(ss);
@@ -334,7 +334,7 @@ __device__ __forceinline__ float row_inv_rms_of(const uint16_t* base, int n8, fl
     float v[8];
     widen8<DT>(*reinterpret_cast<const uint4*>(base + g * 8), v);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc = acc + v[e] * v[e];
+    for (int e = 0; e < 8; ++e) acc = __fmaf_rn(v[e], v[e], acc);
   }
   acc = over_lanes<Sum>(acc);
   // sqrtf, not __fsqrt_rn: the latter is the 1-ulp native instruction in this toolchain, the former is
@@ -572,10 +572,9 @@ __device__ __forceinline__ void quant_q_row(float* x, int c16, float premul_lane
   amax = fmaxf(amax, lane_xor<1>(amax));
   amax = fmaxf(amax, lane_xor<2>(amax));
   amax = fmaxf(amax, lane_xor<4>(amax));
-  const bool nz = amax > 0.0f;
-  const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
-  if (c16 == 0) *scale = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
-  store_out16(codes + c16 * 16, pack_int8x16(x, inv));
+  const Int8Scale r = int8_scale(amax);
+  if (c16 == 0) *scale = r.scale;
+  store_out16(codes + c16 * 16, pack_int8x16(x, r.inv));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -703,7 +702,7 @@ __global__ __launch_bounds__(kThreads) void quant_q_rows_kernel(const uint16_t* 
         float v[8];
         widen8<DT>(raw[i], v);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[i] = acc[i] + v[e] * v[e];
+        for (int e = 0; e < 8; ++e) acc[i] = __fmaf_rn(v[e], v[e], acc[i]);
       }
     }
 #pragma unroll
@@ -782,11 +781,10 @@ __global__ __launch_bounds__(kThreads) void quant_q_rows_kernel(const uint16_t* 
     amax = fmaxf(amax, lane_xor<1>(amax));
     amax = fmaxf(amax, lane_xor<2>(amax));
     amax = fmaxf(amax, lane_xor<4>(amax));
-    const bool nz = amax > 0.0f;
-    const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
+    const Int8Scale r = int8_scale(amax);
     const int64_t bh = (int64_t)b * H + h;
-    if (c16 == 0) q_scale[bh * lq_pad + row] = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
-    store_out16(q_i8 + (bh * lq_pad + row) * kD + c16 * 16, pack_int8x16(xr, inv));
+    if (c16 == 0) q_scale[bh * lq_pad + row] = r.scale;
+    store_out16(q_i8 + (bh * lq_pad + row) * kD + c16 * 16, pack_int8x16(xr, r.inv));
     __builtin_amdgcn_sched_barrier(0);
   }
 }
@@ -857,10 +855,9 @@ __device__ __forceinline__ void quant_k_block(int blk, int h, int b, const uint1
   }
   __shared__ float s_red[4];
   amax = block_max(amax, s_red);
-  const bool nz = amax > 0.0f;
-  const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
-  const float inv_lane = inv * fwht_lane_sign(c16);  // the transform left this lane's values times that sign
-  if (t == 0) k_scale[bh * nkb + blk] = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+  const Int8Scale r = int8_scale(amax);
+  const float inv_lane = r.inv * fwht_lane_sign(c16);  // the transform left this lane's values times that sign
+  if (t == 0) k_scale[bh * nkb + blk] = r.scale;
   int8_t* tile = k_tiles + (bh * nkb + blk) * (int64_t)kTileBytes;
 #pragma unroll
   for (int i = 0; i < R; ++i) {
@@ -1282,10 +1279,9 @@ __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __
     if (lane == 0) s_red[tt][wave] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(s_red[tt][0], s_red[tt][1]), fmaxf(s_red[tt][2], s_red[tt][3]));
-    const bool nz = amax > 0.0f;
-    const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
-    const float inv_lane = inv * fwht_lane_sign(c16);  // the transform left this lane's values times that sign
-    if (t == 0) k_scale[(int64_t)bh * nkb + blk] = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+    const Int8Scale r = int8_scale(amax);
+    const float inv_lane = r.inv * fwht_lane_sign(c16);  // the transform left this lane's values times that sign
+    if (t == 0) k_scale[(int64_t)bh * nkb + blk] = r.scale;
     int8_t* tile = k_tiles + ((int64_t)bh * nkb + blk) * (int64_t)kTileBytes;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -1735,10 +1731,10 @@ __device__ __forceinline__ void joint_k_item(int item, const QkvCall& c, const P
     if ((t & 63) == 0) s_red[hh][wave] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(s_red[hh][0], s_red[hh][1]), fmaxf(s_red[hh][2], s_red[hh][3]));
-    const bool nz = amax > 0.0f;
-    const float inv_lane = (nz ? __fdiv_rn(127.0f, amax) : 0.0f) * fwht_lane_sign(c16);
+    const Int8Scale r = int8_scale(amax);
+    const float inv_lane = r.inv * fwht_lane_sign(c16);
     const int64_t at = ((int64_t)b * c.Hkv + h0 + hh) * c.nkb + blk;
-    if (t == 0) c.k_scale[at] = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+    if (t == 0) c.k_scale[at] = r.scale;
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int frag = i * 4 + (c16 >> 1), ln = (c16 & 1) * 32 + slot;

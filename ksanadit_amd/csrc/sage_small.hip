@@ -231,10 +231,10 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c)
         amax = fmaxf(amax, lane_xor<1>(amax));
         amax = fmaxf(amax, lane_xor<2>(amax));
         amax = fmaxf(amax, lane_xor<4>(amax));
-        const bool nz = amax > 0.0f;
-        const float inv_lane = (nz ? __fdiv_rn(127.0f, amax) : 0.0f) * fwht_lane_sign(c16);
+        const Int8Scale r = int8_scale(amax);
+        const float inv_lane = r.inv * fwht_lane_sign(c16);
         *reinterpret_cast<uint4*>(q_ops + ((g * 4 + (c16 >> 1)) * 64 + (c16 & 1) * 32 + slot) * 16) = pack_int8x16(y, inv_lane);
-        if (c16 == 0) s_qs[g * kSlots + slot] = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+        if (c16 == 0) s_qs[g * kSlots + slot] = r.scale;
       }
     }
   }
@@ -260,9 +260,9 @@ __global__ __launch_bounds__(kThreads) void sage_small_kernel(const SmallCall c)
     for (int tt = 0; tt < kMaxTiles; ++tt) {
       if (tt >= n_tiles) break;
       const float amax = fmaxf(fmaxf(s_red[tt][0], s_red[tt][1]), fmaxf(s_red[tt][2], s_red[tt][3]));
-      const bool nz = amax > 0.0f;
-      const float inv_lane = (nz ? __fdiv_rn(127.0f, amax) : 0.0f) * fwht_lane_sign(c16);
-      if (t == 0) s_ks[tt] = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+      const Int8Scale r = int8_scale(amax);
+      const float inv_lane = r.inv * fwht_lane_sign(c16);
+      if (t == 0) s_ks[tt] = r.scale;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         if ((2 * tt + i) * kSlots >= c.Lk) break;
