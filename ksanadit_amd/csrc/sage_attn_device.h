@@ -202,6 +202,10 @@ __device__ __forceinline__ void qk_tile(const uint8_t* k_stage, int lane, const 
 // SIMD, all at once); what it saves is the quantizer's pass over Q, which is HBM-bound.  Whole calls, us, before / with it:
 // 32760 queries on 512 keys, 40 heads 373 / 336; padded batch (B=3, 24 heads, 3001 x 4099) 210 / 202; causal 8191, 32 heads
 // 352 / 345; 9001 tokens of 64 channels, B=2, 16 heads 563 / 557.  Which calls take it: q_in_attention_pays.
+// The butterflies between the halves move half of the values across the wave and not back: what crosses back are bytes (8 kG and
+// 2 kG swaps a row in place of 16 kG), and one division yields the factor and the scale.  us, before / with it: 32760 queries on
+// 512 keys 312.0 / 306.6, 75600 on 512 693.2 / 685.7, 2 x 20000 of 24 heads on 120 157.4 / 156.3; with channels 2 i and 2 i + 1
+// as pairs, whose bytes have to be woven afterwards, 309.8, 689.3, 156.3.
 template <int DT, int kG>
 __device__ __forceinline__ void quant_q_rows(const uint4 (&raw)[8], float premul, v4i (&qf)[4], float& qs) {
   float x[kG][16];
@@ -218,15 +222,16 @@ __device__ __forceinline__ void quant_q_rows(const uint4 (&raw)[8], float premul
           x[s][i] = a + b;
           x[s][i + st] = a - b;
         }
-    // two values at a time: the first swap gives the lower lanes both ends of the first value's butterfly and the upper
-    // lanes both ends of the second's, the second swap takes the results home
+    // two values at a time, channels i and i + 4: the swap gives the lower lanes both ends of the first's butterfly and the
+    // upper lanes both ends of the second's, and there the results stay until they are bytes: x[s][i] belongs to the lower
+    // sixteen channels, x[s][i + 4] to the upper sixteen
 #pragma unroll
-    for (int i = 0; i < 16; i += 2) {
-      const auto ab = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[s][i]), __float_as_uint(x[s][i + 1]), false, false);
+    for (int j = 0; j < 8; ++j) {
+      const int i = 2 * j - (j & 3);  // 0 .. 3, 8 .. 11
+      const auto ab = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[s][i]), __float_as_uint(x[s][i + 4]), false, false);
       const float a = __uint_as_float(ab[0]), b = __uint_as_float(ab[1]);
-      const auto home = __builtin_amdgcn_permlane32_swap(__float_as_uint(a + b), __float_as_uint(a - b), false, false);
-      x[s][i] = __uint_as_float(home[0]);
-      x[s][i + 1] = __uint_as_float(home[1]);
+      x[s][i] = a + b;
+      x[s][i + 4] = a - b;
     }
   }
 #pragma unroll
@@ -250,11 +255,22 @@ __device__ __forceinline__ void quant_q_rows(const uint4 (&raw)[8], float premul
     }
   const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
   amax = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
-  const bool nz = amax > 0.0f;
-  const float inv = nz ? __fdiv_rn(127.0f, amax) : 0.0f;
-  qs = nz ? __fdiv_rn(amax, 127.0f) : 0.0f;
+  // one division for both quotients (int8_scale): the lower lanes' is the factor, the upper lanes' the scale
+  const bool upper = (threadIdx.x & 32) != 0;
+  float quot = __fdiv_rn(upper ? amax : 127.0f, upper ? 127.0f : amax);
+  quot = amax > 0.0f ? quot : 0.0f;
+  const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(quot), __float_as_uint(quot), false, false);
+  const float inv = __uint_as_float(both[0]);
+  qs = __uint_as_float(both[1]);
 #pragma unroll
-  for (int s = 0; s < kG; ++s) qf[s] = __builtin_bit_cast(v4i, pack_int8x16(x[s], inv));
+  for (int s = 0; s < kG; ++s) {
+    // of the lower sixteen channels codes.x holds 0 .. 3 in the lower lanes and 4 .. 7 in the upper ones, codes.z 8 .. 11 and
+    // 12 .. 15; .y and .w the same of the upper sixteen
+    const uint4 codes = pack_int8x16(x[s], inv);
+    const auto first = __builtin_amdgcn_permlane32_swap(codes.x, codes.y, false, false);
+    const auto second = __builtin_amdgcn_permlane32_swap(codes.z, codes.w, false, false);
+    qf[s] = v4i{(int)first[0], (int)first[1], (int)second[0], (int)second[1]};
+  }
 }
 
 }  // namespace ksana_sage
