@@ -1719,9 +1719,11 @@ __device__ __forceinline__ void joint_k_item(int item, const QkvCall& c, const P
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const bool valid = blk * kBlkK + i * kSlots + slot < c.Lk;
-      if (valid) prep16_qwen<DT>(x[i], f[i], pp.eps);
+      if (valid) {  // (a row that is not there has been read as zeros and stays so)
+        prep16_qwen<DT>(x[i], f[i], pp.eps);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) x[i][e] = valid ? x[i][e] - s_mean[hh][c16 * 16 + e] : 0.0f;
+        for (int e = 0; e < 16; ++e) x[i][e] = x[i][e] - s_mean[hh][c16 * 16 + e];
+      }
       fwht128(x[i], c16);
 #pragma unroll
       for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(x[i][e]));
