@@ -33,6 +33,21 @@ __device__ __forceinline__ const uint8_t* scalar(const uint8_t* at) {
   return reinterpret_cast<const uint8_t*>((uint64_t)hi << 32 | lo);
 }
 
+// A place in LDS of this lane's own as one register, to which only constants are added: in 128 KiB the tiles lie beyond the 64 KiB
+// that an instruction's offset reaches, and left to itself the compiler keeps an address for every constant (39 registers, 18 of
+// them in scratch memory, read back behind the next block's rows, and eight additions per two steps).  us, before / with it: 40
+// heads of 32760 rows on 512 keys 305.1 / 303.5, of 75600 677.9 / 672.2, 2 x 24 of 20000 on 333 203.5 / 201.4.
+typedef const __attribute__((address_space(3))) uint8_t* LdsBytes;
+__device__ __forceinline__ LdsBytes own_place(const uint8_t* at) {
+  LdsBytes lds = (LdsBytes)at;
+  pin(lds);
+  return lds;
+}
+template <typename T>
+__device__ __forceinline__ T lds_read(LdsBytes at) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) T*>(at);
+}
+
 // n_blk: blocks of 32 rows per (batch, head); parts: workgroups per (batch, head)
 template <int DT, int kG>
 __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const AttnParams p, int n_blk, int parts, int n_wg) {
@@ -52,8 +67,8 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
   float* s_vs = reinterpret_cast<float*>(smem + kScalesAt);
   float* s_ks = s_vs + 2 * kD;
   int* s_next = reinterpret_cast<int*>(s_ks + kMaxTiles);
-  const uint8_t* my_k = smem + lane * 16;                             // this lane's pieces of K tile 0 ..
-  const uint8_t* my_v = smem + kMaxTiles * kTileBytes + lane * 16;    // .. and of V^T tile 0
+  const LdsBytes my_k = own_place(smem + lane * 16);                           // this lane's pieces of K tile 0 ..
+  const LdsBytes my_v = own_place(smem + kMaxTiles * kTileBytes + lane * 16);  // .. and of V^T tile 0
 
   const int b = __builtin_amdgcn_readfirstlane(bh / p.Hq), h = bh - b * p.Hq;
   const int bhk = __builtin_amdgcn_readfirstlane(b * p.Hkv + h / (p.Hq / p.Hkv));
@@ -151,10 +166,10 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
       xc = x_base + mneg;
     };
     auto p_of = [&](int acc_bits) { return fast_exp2(__builtin_fmaf(__int_as_float(acc_bits), sc, xc)); };
-    auto k_frag = [&](const uint8_t* tile, int i8) { return *reinterpret_cast<const v4i*>(tile + ((i8 & 1) * 4 + (i8 >> 1)) * 1024); };
-    auto v_frag = [&](const uint8_t* tile, int dt) {
-      const v4i lo = *reinterpret_cast<const v4i*>(tile + dt * 2048);
-      const v4i hi = *reinterpret_cast<const v4i*>(tile + dt * 2048 + 1024);
+    auto k_frag = [&](LdsBytes tile, int i8) { return lds_read<v4i>(tile + ((i8 & 1) * 4 + (i8 >> 1)) * 1024); };
+    auto v_frag = [&](LdsBytes tile, int dt) {
+      const v4i lo = lds_read<v4i>(tile + dt * 2048);
+      const v4i hi = lds_read<v4i>(tile + dt * 2048 + 1024);
       return v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     };
     auto has_qk = [](int i8) { return i8 >= 0 && i8 < 8 && (i8 >> 1) < kG; };
@@ -164,8 +179,8 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
     // alpha, moved: tile j - 1's on the way in, tile j + 1's on the way out.
     auto step = [&](int j, v16i (&s_cur)[2], v16i (&s_nxt)[2], const v8i& pf_prev, v8i& pf, float& alpha, int& moved) {
       const int nxt = min(j + 1, n_tiles - 1);
-      const uint8_t* kst = my_k + nxt * kTileBytes;
-      const uint8_t* vst = my_v + max(j - 1, 0) * kTileBytes;
+      LdsBytes kst = my_k + nxt * kTileBytes, vst = my_v + max(j - 1, 0) * kTileBytes;
+      pin(kst), pin(vst);
       v4i kf[4];
       v8i vf[4];
       kf[0] = k_frag(kst, 0), kf[1] = k_frag(kst, 1), kf[2] = k_frag(kst, 2);
@@ -242,7 +257,8 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
       const bool odd = (n_tiles & 1) != 0;
       if (odd ? moved_even != 0 : moved_odd != 0) scale_o(odd ? alpha_even : alpha_odd);
       const v8i pf_last = odd ? pf_y : pf_x;
-      const uint8_t* vst = my_v + (n_tiles - 1) * kTileBytes;
+      LdsBytes vst = my_v + (n_tiles - 1) * kTileBytes;
+      pin(vst);  // (not an address per piece over the whole loop)
       lacc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ones, pf_last, lacc, 0, 0, 0, 0, 0, 0);
 #pragma unroll
       for (int dt = 0; dt < kG; ++dt)
@@ -255,6 +271,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
     const float inv_l = 1.0f / lacc[0];
     const float keep_mean = inv_l != 0.0f ? 1.0f : 0.0f;
     uint16_t* orow = obase + (int64_t)row * p.o.sL;
+    const LdsBytes scales = own_place(smem + kScalesAt + 16 * hh);
     auto store = [&](auto with_mean) {
 #pragma unroll
       for (int dt = 0; dt < kG; ++dt)
@@ -263,12 +280,13 @@ __global__ __launch_bounds__(kWaves * 64, 1) void sage_resident_kernel(const Att
           uint2 w[2];
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
-            const int r = 4 * (g + e), d = 32 * dt + 8 * (g + e) + 4 * hh;
-            const float4 s4 = *reinterpret_cast<const float4*>(s_vs + d);
-            float o4[4] = {oacc[dt][r] * inv_l * s4.x, oacc[dt][r + 1] * inv_l * s4.y, oacc[dt][r + 2] * inv_l * s4.z, oacc[dt][r + 3] * inv_l * s4.w};
+            const int r = 4 * (g + e), d = 32 * dt + 8 * (g + e);
+            const v4f s4 = lds_read<v4f>(scales + 4 * d);
+            float o4[4] = {oacc[dt][r] * inv_l * s4[0], oacc[dt][r + 1] * inv_l * s4[1], oacc[dt][r + 2] * inv_l * s4[2], oacc[dt][r + 3] * inv_l * s4[3]};
             if constexpr (decltype(with_mean)::value) {
-              const float4 m4 = *reinterpret_cast<const float4*>(s_vs + kD + d);
-              o4[0] += m4.x * keep_mean, o4[1] += m4.y * keep_mean, o4[2] += m4.z * keep_mean, o4[3] += m4.w * keep_mean;
+              const v4f m4 = lds_read<v4f>(scales + 4 * (kD + d));
+#pragma unroll
+              for (int c = 0; c < 4; ++c) o4[c] += m4[c] * keep_mean;
             }
             // (pinned: the last operation and the conversion may otherwise become one fp16 instruction with a single rounding)
 #pragma unroll
