@@ -84,9 +84,10 @@ __device__ __forceinline__ void lds_copy16_at(const v4i& buffer, unsigned lane_o
 // take part to every XCD, the entry with the most keys first, then an eighth of every entry's other blocks, which have only zeros
 // to write (-1: no such workgroup); and its entry's counts.  The counts are in device memory, so every workgroup works this out by itself, an entry per lane.
 // In the order of their index, an entry's blocks without rows stand before the next entry's: work waits for a place while they
-// come and go.  us per call, by index / like this, entries falling off to 45 %: 5 x 32 heads of 1500 tokens 140 / 132, 6 x 64 of 2000
-// 373 / 353, 3 x 24 of 3001 on 4099 184.3 / 180.7, 2 x 12 of 6946 on 138 38.1 / 37.1, 3 x 40 of 8000 1340 / 1337, 2 x 40 of 16384
-// 3419 / 3422.  One round of the chip has no order (6 heads of 5000 66.4 / 67.3: the counts come through vector loads).
+// come and go.  us per call, by index / like this, entries falling off to 45 %: 5 x 32 heads of 1500 tokens 143 / 135.5,
+// 3 x 24 of 3001 on 4099 184.3 / 180.7, 2 x 12 of 6946 on 138 38.1 / 37.1.  Which grids are numbered like this: see launch_attn_fwd.
+constexpr int kPackedMaxEntries = 6;
+static_assert(kPackedMaxEntries <= 64, "an entry per lane");
 template <int kRowsWg>
 __device__ __forceinline__ int packed_place(const AttnParams& p, int xcd, int at, int n_qwg, int& lq, int& lk) {
   const int lane = threadIdx.x & 63;
@@ -185,7 +186,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         wg = xcd * wg_per_xcd + at;
         if (wg >= n_wg) return;
       } else {
-        // (calls whose last blocks are cut, and batches of more than 64 entries; the others: see packed_place)
+        // (grids that launch_attn_fwd does not have numbered by packed_place)
         // batch entries of unequal length: an eighth of every entry's workgroups to every XCD.  One run across the entries
         // would leave the XCDs that drew the short ones idle.  The entries run in the order of their index, longest first or
         // not: the order that ends with the longest one costs up to 5-8 % in grids of two rounds, nothing in long ones.  us,
@@ -1405,7 +1406,14 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   int wg_per_xcd = 0;
   dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
   auto pack_batch = [&]() {
-    if (p.batch_run == 0 || sparse || p.B > 64 || n_wg <= (waves == 4 ? 2 : 1) * compute_units()) return;
+    // One round has no order; beyond four and a half the work of numbering, the same in every workgroup and more with every
+    // entry, is more than the last round's order gives (keys halving over the entries; us, by index / numbered).  2 x 12 heads of 6946
+    // rows (2.6 rounds) on 133 keys 38.7 / 37.7, on 2500 110.5 / 107.7; 3 x 24 of 3001 (3.4) on 600 61.8 / 59.3; 6 x 24 of 2000 (4.5)
+    // on 2000 136 / 133; but 4 x 24 of 3343 (5.1) on 600 80.0 / 80.6, 6 x 24 of 3343 (7.6) on 133 80.5 / 86.1, on 2500 247.7 / 251.3,
+    // 3 x 40 of 8000 (14.8) on 4000 752 / 757; 8 x 8 of 3343 (3.4) on 600 59.0 / 62.2.  (Some long grids gain, 6 x 64 of 2000, 12
+    // rounds, 498 / 480: no rule on sizes was found that has these and not the others.)
+    const int round = (waves == 4 ? 2 : 1) * compute_units();
+    if (p.batch_run == 0 || sparse || p.B > kPackedMaxEntries || n_wg <= round || 2 * n_wg > 9 * round) return;
     p.packed = 1;
     grid = dim3(8 * p.B * (p.batch_run + 1));  // (either kind of an entry's blocks is divided by eight)
   };

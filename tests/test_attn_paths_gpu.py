@@ -256,7 +256,7 @@ def test_a_shared_last_block_in_batches_with_lengths(hip_device, k_len, rows):
 def test_batches_are_numbered_by_their_counts(hip_device, B, H, Lq, Lk, wg_waves):
     """Grids of more than a round whose workgroups work out which block is theirs from the entries' counts - in any order, equal,
     none, one, all, out of range - against the same operands walked through a mask of ones, whose grid is numbered as the
-    tensor is laid out.  (More than 64 entries are, too.)"""
+    tensor is laid out.  (More than six entries and grids of one round are, too.)"""
     print(f"case B={B} H={H} Lq={Lq} Lk={Lk} waves={wg_waves}", flush=True)
     g = torch.Generator().manual_seed(B * Lq + Lk)
     q, k, v = (torch.randn((B, n, H, 128), generator=g).to(torch.bfloat16).to(hip_device) for n in (Lq, Lk, Lk))
