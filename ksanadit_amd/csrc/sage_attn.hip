@@ -262,13 +262,31 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   // calls that do not take it: 12 workgroups of 10 tiles 23.9 us with it in line, 23.0 without)
   constexpr bool kOwnQ = !kSparse || kCausal;
   const bool own_q = __builtin_expect(kOwnQ && active && !shared && p.q_rows.ptr != nullptr, 0);  // uniform per wave
+  // Rows that are quantized already are requested first of all and touched by the set-up's one wait only: their loads run under
+  // the list's mask bytes, the operands' set-up and the tile copies.  us per call, behind the copies / first: dense, 16 heads of
+  // 2600 tokens 59.6 / 58.8, 24 of 2000 53.9 / 53.1, 2 x 24 of 774 36.4 / 35.9, 40 of 420 22.9 / 22.7; causal, 16 of 1500 33.2 / 33.0.
+  // (kPinned: what was loaded is taken over in the branch that has no rows of its own.  Elsewhere the compiler copies the registers
+  // before that branch, and a workgroup with rows of its own waits for its tile copies before it requests them: 24 heads of 4400 on
+  // 700 keys 47.8 / 47.3.  In the causal variants and in 8 waves it costs the calls with stored rows 1 % instead: 16 of 2600 59.3.)
+  constexpr bool kPinned = kW == 4 && !kCausal;
+  v4i q_codes[4];
+  float q_sc = 0.0f;
 #pragma unroll
-  for (int s = 0; s < 4; ++s) qf[s] = v4i{0, 0, 0, 0};
-  auto read_q = [&]() {
+  for (int s = 0; s < 4; ++s) q_codes[s] = v4i{0, 0, 0, 0};
+  if (active && !own_q && !(shared && p.q_rows.ptr != nullptr)) {
     const int8_t* qrow = p.q_i8 + ((int64_t)bh * p.lq_pad + q0 + l32) * kD + 16 * hh;
 #pragma unroll
-    for (int s = 0; s < kG; ++s) qf[s] = *reinterpret_cast<const v4i*>(qrow + 32 * s);
-    qs = p.q_scale[(int64_t)bh * p.lq_pad + q0 + l32];  // one scale per query row = per lane
+    for (int s = 0; s < kG; ++s) q_codes[s] = *reinterpret_cast<const v4i*>(qrow + 32 * s);
+    q_sc = p.q_scale[(int64_t)bh * p.lq_pad + q0 + l32];  // one scale per query row = per lane
+  }
+  auto take_q = [&]() {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      if (kPinned) pin(q_codes[s]);
+      qf[s] = q_codes[s];
+    }
+    if (kPinned) pin(q_sc);
+    qs = q_sc;
   };
 
   v16f oacc[4];
@@ -415,7 +433,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         }
         quant_q_rows<DT, kG>(raw, p.q_premul, qf, qs);
       } else {
-        read_q();
+        take_q();
       }
       fill_scales();
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -716,8 +734,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   for (int t = 0; t < (kLateCopies ? 2 : Shape::kAheadK); ++t) copy_half(false, t, k_slot(t));
   fill_scales();
   if (__builtin_expect(own_q, 0)) {
-    // Requested behind the copies and without a condition: loads return in the order they were issued, and a wait for one issued
-    // before a copy, which the compiler does not count, is a wait for the copy too.  With the loads first and zeros
+    // Requested behind the copies and without a condition (unlike stored rows, these are worked on in the set-up): loads return in
+    // the order they were issued, and a wait for one issued before a copy, which the compiler does not count, is a wait for the copy too.  With the loads first and zeros
     // for what does not exist in their stead, the second pair of loads went out when the first had arrived.
     const int row = q0 + l32;
     const bool half = kG == 4 && p.q_rows.D != kD;  // (uniform) 64 channels in the full-width code
@@ -734,8 +752,8 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
         if (row >= p.Lq || (half && s >= 2)) q_raw[2 * s] = q_raw[2 * s + 1] = make_uint4(0, 0, 0, 0);
     }
     quant_q_rows<DT, kG>(q_raw, p.q_premul, qf, qs);
-  } else if (active) {
-    read_q();
+  } else {
+    take_q();
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the set-up's loads and, older than some of them, the copies
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
