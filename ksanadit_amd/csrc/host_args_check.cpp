@@ -52,6 +52,44 @@ static int causal_numbering_is_wrong(int pairs, int n_qwg, unsigned* kinds) {
   return n != pairs * n_qwg;
 }
 
+// Every block of a batch numbered by its counts belongs to one workgroup of a grid of the launcher's size, and an XCD starts those
+// that have only zeros to write after all others.
+static int batch_numbering_is_wrong(int B, int heads, int n_qwg, const int* with_rows) {
+  int starts[ksana_sage::kBatchStarts], at = 0;
+  for (int i = 0; i < ksana_sage::kBatchStarts; ++i) {
+    starts[i] = i < 2 * B ? at : INT32_MAX;
+    if (i < 2 * B) at += ksana_sage::batch_share(heads, i < B ? with_rows[i] : n_qwg - with_rows[i - B]);
+  }
+  const int per_xcd = B * ((heads * n_qwg + 7) / 8 + 1);
+  if (at > per_xcd) return 1;
+  std::vector<char> seen((size_t)B * heads * n_qwg, 0);
+  int n = 0;
+  for (int xcd = 0; xcd < 8; ++xcd) {
+    bool zeros = false;
+    for (int i = 0; i < per_xcd; ++i) {
+      const ksana_sage::BatchRun run = ksana_sage::batch_run_of(starts, B, i);
+      if (run.b < 0 || run.b >= B) return 1;
+      const ksana_sage::BatchPlace p = ksana_sage::batch_place(run, xcd, i, heads, n_qwg, with_rows[run.b]);
+      if (p.b < 0) continue;
+      if (p.b != run.b || p.h < 0 || p.h >= heads || p.qwg < 0 || p.qwg >= n_qwg) return 1;
+      const bool zero = p.qwg >= with_rows[p.b];
+      if (zero != run.zeros || (zeros && !zero) || seen[((size_t)p.b * heads + p.h) * n_qwg + p.qwg]++ != 0) return 1;
+      zeros = zero;
+      ++n;
+    }
+  }
+  return n != B * heads * n_qwg;
+}
+
+// Which calls are numbered, and with how many rows a workgroup (without a device: 256 compute units)
+static int batch_rows(int B, int heads, int Lq, int Lk, int waves = 0, int causal = 0, bool counts = true) {
+  static const int32_t some[1] = {1};
+  ksana_sage::AttnParams p{};
+  p.B = B, p.Hq = p.Hkv = heads, p.Lq = Lq, p.Lk = Lk, p.nkb = (Lk + 63) / 64, p.causal = causal, p.wg_waves = waves, p.exact_exp2 = 1, p.d_out = 128;
+  p.k_lens = counts ? some : nullptr;
+  return ksana_sage::batch_rows_wg(p);
+}
+
 int main() {
   void* const fake = reinterpret_cast<void*>(0x1000);  // aligned and never dereferenced
   ksana_sage_shape s{1, 2, 2, 64, 64, 128};
@@ -156,6 +194,27 @@ int main() {
   int64_t ticks = 0;
   EXPECT(ksana_sage_one_read_state(&k1, &v1, &ticks, &dem), 0);
   if (!k1 || !v1 || ticks != 123 || dem != 0) ++g_failed, std::printf("settings did not stick\n");
+  unsigned seed = 1;
+  for (int i = 0; i < 4000; ++i) {
+    auto next = [&](int n) { return (int)((seed = seed * 1664525u + 1013904223u) >> 8) % n; };
+    const int B = 2 + next(ksana_sage::kBatchEntries - 1), heads = 1 + next(70), n_qwg = 1 + next(40), kind = next(4);
+    int with_rows[ksana_sage::kBatchEntries];
+    for (int& w : with_rows) w = kind == 0 ? next(n_qwg + 1) : kind == 1 ? n_qwg : kind == 2 ? 0 : next(2) * n_qwg;
+    if (batch_numbering_is_wrong(B, heads, n_qwg, with_rows)) ++g_failed, std::printf("batch numbering: %d entries, %d heads, %d blocks\n", B, heads, n_qwg);
+  }
+  // one round and a block more, four and a half rounds and a block more, entries, options, cut blocks
+  EXPECT(batch_rows(2, 16, 2048, 600), 0);
+  EXPECT(batch_rows(2, 16, 2049, 600), 128);
+  EXPECT(batch_rows(2, 64, 18 * 128, 600), 128);
+  EXPECT(batch_rows(2, 64, 18 * 128 + 1, 600), 0);
+  EXPECT(batch_rows(8, 24, 1000, 600), 128);
+  EXPECT(batch_rows(9, 24, 1000, 600), 0);
+  EXPECT(batch_rows(1, 64, 1500, 600), 0);
+  EXPECT(batch_rows(8, 24, 1000, 600, 0, 1), 0);
+  EXPECT(batch_rows(8, 24, 1000, 600, 0, 0, false), 0);
+  EXPECT(batch_rows(8, 24, 1000, 600, 8), 256);
+  EXPECT(batch_rows(2, 50, 1250, 2560), 256);
+  EXPECT(batch_rows(2, 24, 4352, 4352), 0);
   EXPECT(ksana_sage_selftest(), 0);
   if (ksana_sage_abi_version() != KSANA_SAGE_ABI_VERSION) ++g_failed, std::printf("ABI number differs from the header's\n");
   std::printf("host argument checks: %d failed\n", g_failed);

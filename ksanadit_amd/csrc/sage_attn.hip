@@ -80,45 +80,6 @@ __device__ __forceinline__ void lds_copy16_at(const v4i& buffer, unsigned lane_o
 }
 #pragma clang diagnostic pop
 
-// Which workgroup of a batch with counts of its own is number `at` of XCD `xcd`: an eighth of every entry's blocks with rows that
-// take part to every XCD, the entry with the most keys first, then an eighth of every entry's other blocks, which have only zeros
-// to write (-1: no such workgroup); and its entry's counts.  The counts are in device memory, so every workgroup works this out by itself, an entry per lane.
-// In the order of their index, an entry's blocks without rows stand before the next entry's: work waits for a place while they
-// come and go.  us per call, by index / like this, entries falling off to 45 %: 5 x 32 heads of 1500 tokens 143 / 135.5,
-// 3 x 24 of 3001 on 4099 184.3 / 180.7, 2 x 12 of 6946 on 138 38.1 / 37.1.  Which grids are numbered like this: see launch_attn_fwd.
-constexpr int kPackedMaxEntries = 6;
-static_assert(kPackedMaxEntries <= 64, "an entry per lane");
-template <int kRowsWg>
-__device__ __forceinline__ int packed_place(const AttnParams& p, int xcd, int at, int n_qwg, int& lq, int& lk) {
-  const int lane = threadIdx.x & 63;
-  int rows = 0, keys = -1, blocks = 0;
-  if (lane < p.B) {
-    rows = p.q_lens != nullptr ? rows_counted(p.q_lens[lane], p.Lq) : p.Lq;
-    keys = p.k_lens != nullptr ? rows_counted(p.k_lens[lane], p.Lk) : p.Lk;
-    if (keys > 0) blocks = (rows + kRowsWg - 1) / kRowsWg;
-  }
-  int rank = 0;
-  for (int j = 0; j < p.B; ++j) {
-    const int other = __builtin_amdgcn_readlane(keys, j);
-    rank += other > keys || (other == keys && j < lane);
-  }
-  for (int kind = 0; kind < 2; ++kind)  // blocks with rows, the others
-    for (int r = 0; r < p.B; ++r) {
-      const int b = (int)__ffsll((unsigned long long)__ballot(lane < p.B && rank == r)) - 1;
-      const int with_rows = __builtin_amdgcn_readlane(blocks, b), n = kind == 0 ? with_rows : n_qwg - with_rows;
-      const int per = (p.Hq * n + 7) / 8;
-      if (at < per) {
-        const int i = xcd * per + at;
-        if (i >= p.Hq * n) return -1;
-        const int h = i / n;
-        lq = __builtin_amdgcn_readlane(rows, b), lk = __builtin_amdgcn_readlane(keys, b);
-        return (b * p.Hq + h) * n_qwg + (i - h * n) + (kind == 0 ? 0 : with_rows);
-      }
-      at -= per;
-    }
-  return -1;
-}
-
 // Dense 8-wave calls can hold two kinds of workgroup in one grid: blocks below p.split_first_block walk all key tiles of
 // their (head, query block); each of the blocks from there on takes one of `p.n_split` equal runs of key tiles and leaves
 // unnormalised accumulators, running maxima and row sums in the workspace for sage_attn_merge_kernel.  The runs stand
@@ -132,7 +93,7 @@ template <int DT, bool kPwlExp, bool kSparse, int kW, bool kTileSkip, int kG, bo
 __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel(const AttnParams p, int n_qwg,
                                                                                    int n_wg, int wg_per_xcd) {
   want(p.q_rows.ptr, p.k_tiles, p.o.sH, p.block_mask, n_qwg);
-  constexpr bool kCanSplit = !kSparse && kW == 8;
+  constexpr bool kCanSplit = !kSparse && kW == 8, kDense = !kSparse && !kCausal;
   static_assert(kSparse || !kCausal || (kW == 4 && !kPwlExp && !kTileSkip), "causal without a list: the default variant in 4 waves");
   // kCausal == false: the caller vouches that p.causal is 0, and everything that serves the diagonal (the per-wave
   // last tile, 32 lane masks held in scalar registers, the selects that blank a wave's probabilities past its rows)
@@ -147,14 +108,29 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   constexpr bool kUnrolled = !kPwlExp && !kTileSkip && !(kSparse && kW == 8);  // the variants calls take by default
   constexpr int kMagicBits = kG == 4 ? kMagicI : kMagicI2;
   constexpr float kMagicVal = kG == 4 ? kMagicF : kMagicF2;
-  int bh, qwg;  // (batch, head) pair and query block
+  int bh, b, h, qwg;  // (batch, head) pair, batch entry and head, query block
   // query rows [0, lq) of this batch take part: all of them, or the caller's per-batch count; the rows from lq up
   // to Lq exist in the output and are written as zeros
   // keys [0, lk) of this batch take part: all of them, or the caller's per-batch count
   int lq = p.Lq, lk = p.Lk;
   const bool is_run = kCanSplit && (int)blockIdx.x >= p.split_first_block;  // uniform
   const int run_id = is_run ? (int)blockIdx.x - p.split_first_block : 0;    // the partial result's place in the workspace
-  if (kCausal && p.causal_grid.group != 0) {
+  const bool numbered = kDense && p.numbered != 0;
+  if (numbered) {  // (BatchRun, BatchPlace)
+    typedef const __attribute__((address_space(4))) int32_t* Constant;
+    const Constant at_starts = reinterpret_cast<Constant>(reinterpret_cast<uintptr_t>(p.split_ml));
+    int starts[kBatchStarts];
+#pragma unroll
+    for (int i = 0; i < kBatchStarts; ++i) starts[i] = at_starts[i];  // (scalar loads, together)
+    const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+    const BatchRun run = batch_run_of(starts, p.B, at);
+    b = run.b;
+    take_counts(p.q_lens, p.k_lens, b, lq, lk);
+    const BatchPlace place = batch_place(run, xcd, at, p.Hq, n_qwg, batch_blocks(lq, lk, kRowsWg));
+    if (place.b < 0) return;
+    h = place.h, qwg = place.qwg;
+    bh = b * p.Hq + h;
+  } else if (kCausal && p.causal_grid.group != 0) {
     if (!causal_place(p.causal_grid, blockIdx.x, n_qwg, &bh, &qwg)) return;
   } else {
     int wg;
@@ -179,14 +155,11 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
           if (pair >= n_pairs) return;
           wg = pair * n_qwg + n_qwg - 1;
         }
-      } else if (p.packed) {
-        wg = packed_place<kRowsWg>(p, xcd, at, n_qwg, lq, lk);
-        if (wg < 0) return;
       } else if (p.batch_run == 0) {
         wg = xcd * wg_per_xcd + at;
         if (wg >= n_wg) return;
       } else {
-        // (grids that launch_attn_fwd does not have numbered by packed_place)
+        // (batches that are not numbered by their counts, see batch_rows_wg)
         // batch entries of unequal length: an eighth of every entry's workgroups to every XCD.  One run across the entries
         // would leave the XCDs that drew the short ones idle.  The entries run in the order of their index, longest first or
         // not: the order that ends with the longest one costs up to 5-8 % in grids of two rounds, nothing in long ones.  us,
@@ -202,13 +175,15 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     qwg = wg - bh * n_qwg;
     if (causal) qwg = n_qwg - 1 - qwg;  // the long ones first, as above
   }
-  const int b = bh / p.Hq, h = bh - b * p.Hq;
+  if (!numbered) {
+    b = bh / p.Hq, h = bh - b * p.Hq;
+    take_counts(p.q_lens, p.k_lens, b, lq, lk);
+  }
   const int bhk = b * p.Hkv + h / (p.Hq / p.Hkv);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform by construction: keep it scalar
   const int l32 = lane & 31, hh = lane >> 5;
-  if (!p.packed) take_counts(p.q_lens, p.k_lens, b, lq, lk);
   // A last block of at most 64 rows has work for one or two waves.  Alone on its unit such a workgroup takes half a microsecond a
   // step, next to another one as long as the whole blocks do; so its four waves share the keys out instead (see below).
   constexpr bool kCanShare = !kSparse && !kCausal && kW == 4 && !kPwlExp && !kTileSkip;
@@ -1408,6 +1383,33 @@ static dim3 xcd_grid(AttnParams* p, int n_qwg, int n_wg, int* wg_per_xcd) {
   return dim3(*wg_per_xcd * 8);
 }
 
+// Dense calls, uncut, of more than one round - one round has no order - and up to four and a half.  us, by the tensor's numbering /
+// by the counts:
+//                                        all full      falling to 45 %   rising        half of each    random
+//   2 x 12 heads of 6946 on 138 (2.6)    42.4 / 43.1   38.9 / 37.1       38.7 / 37.3   34.2 / 32.0     37.0 / 35.2
+//   2 x 24 of 3500 (2.6)                 215 / 215.5   150.6 / 152       167 / 150     98.4 / 100.2    140 / 141
+//   3 x 24 of 3001 on 4099 (3.4)         282 / 282.5   185.5 / 181       193 / 182.5   103 / 101       131.5 / 135
+//   5 x 32 of 1500 (3.8)                 183 / 184     142.5 / 131.5     140 / 130     103 / 94        146 / 148.5
+//   6 x 24 of 2000 (4.5)                 243 / 244     174 / 168.5       176 / 170     120 / 119.5     137 / 132
+//   8 x 24 of 1000 on 600 (3.0)          83.5 / 84.2   70.7 / 68.0       71.0 / 67.5   53.6 / 51.9     63.3 / 58.9
+// What all full entries lose, up to 1 us, is the load of the numbers ahead of the counts.  In longer grids the order of the last round is a smaller part,
+// and gains and losses cancel: eight shapes of 5 to 15 rounds in seventeen such sets of counts 0.994 on average, 0.86 to 1.06 each
+// (6 x 64 of 2000, 12 rounds, half of each 334 / 354: blocks that start together keep each other's step).
+int batch_rows_wg(const AttnParams& p) {
+  if (p.B < 2 || p.B > kBatchEntries || (p.q_lens == nullptr && p.k_lens == nullptr) || p.block_mask != nullptr || p.causal || p.nkb > kMaxKeyTiles) return 0;
+  int waves = pick_wg_waves(p);
+  if (waves == 4 && p.nkb > kShortMaxKeyTiles) waves = 8;
+  const int rows = 32 * waves, n_wg = p.B * p.Hq * ((p.Lq + rows - 1) / rows);
+  const int round = (waves == 4 ? 2 : 1) * compute_units();
+  if (n_wg <= round || 2 * n_wg > 9 * round) return 0;
+  if (waves == 8) {
+    int first = n_wg, runs = 0;
+    plan_key_split(n_wg, p.nkb, &first, &runs);
+    if (runs != 0) return 0;
+  }
+  return rows;
+}
+
 hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   AttnParams p = params;
   p.split_first_block = INT32_MAX;
@@ -1423,18 +1425,10 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   const int n_wg = p.B * p.Hq * n_qwg;
   int wg_per_xcd = 0;
   dim3 grid = xcd_grid(&p, n_qwg, n_wg, &wg_per_xcd);
-  auto pack_batch = [&]() {
-    // One round has no order; beyond four and a half the work of numbering, the same in every workgroup and more with every
-    // entry, is more than the last round's order gives (keys halving over the entries; us, by index / numbered).  2 x 12 heads of 6946
-    // rows (2.6 rounds) on 133 keys 38.7 / 37.7, on 2500 110.5 / 107.7; 3 x 24 of 3001 (3.4) on 600 61.8 / 59.3; 6 x 24 of 2000 (4.5)
-    // on 2000 136 / 133; but 4 x 24 of 3343 (5.1) on 600 80.0 / 80.6, 6 x 24 of 3343 (7.6) on 133 80.5 / 86.1, on 2500 247.7 / 251.3,
-    // 3 x 40 of 8000 (14.8) on 4000 752 / 757; 8 x 8 of 3343 (3.4) on 600 59.0 / 62.2.  (Some long grids gain, 6 x 64 of 2000, 12
-    // rounds, 498 / 480: no rule on sizes was found that has these and not the others.)
-    const int round = (waves == 4 ? 2 : 1) * compute_units();
-    if (p.batch_run == 0 || sparse || p.B > kPackedMaxEntries || n_wg <= round || 2 * n_wg > 9 * round) return;
-    p.packed = 1;
+  if (p.numbered != 0) {
+    if (batch_rows_wg(p) != rows) return hipErrorInvalidValue;
     grid = dim3(8 * p.B * (p.batch_run + 1));  // (either kind of an entry's blocks is divided by eight)
-  };
+  }
   if (p.causal && p.batch_run == 0) p.causal_grid = causal_grid(p.B * p.Hq, n_qwg);  // (the same number of workgroups)
   // tile ring + the head's K scales (a multiple of 1 KiB keeps the request tidy)
   const size_t lds = (waves == 4 ? WgShape<4>::kRingBytes : WgShape<8>::kRingBytes) + 1024 + (((size_t)(p.nkb + 1) * 4 + 1023) & ~size_t(1023));
@@ -1457,7 +1451,6 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   };
   if (waves == 4) {
     small_blocks_last();
-    pack_batch();
     if (plain_causal) return launch_causal(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
     if (sparse)
       return p.causal ? launch_shape<true, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
@@ -1473,7 +1466,6 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
   if (p.split_o != nullptr) plan_key_split(n_wg, p.nkb, &n_full, &n_split);
   if (n_split == 0) {
     small_blocks_last();
-    pack_batch();
     return launch_shape<false, 8>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
   }
   const int rest = n_wg - n_full;

@@ -222,7 +222,8 @@ ksana_sage::QkvCall qkv_call(bool with_q, const ksana_sage::InTensor& q, const k
 
 int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
               const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags,
-              const ksana_sage::InTensor* q_rows, float q_premul, void* stream, const ksana_sage::AttnLinear* lin = nullptr);
+              const ksana_sage::InTensor* q_rows, float q_premul, void* stream, const ksana_sage::AttnLinear* lin = nullptr,
+              bool numbered = false);
 
 int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype, int o_dtype, const int64_t q_st[4],
                  const int64_t k_st[4], const int64_t v_st[4], const int64_t o_st[4], const ksana_sage_shape* s,
@@ -886,7 +887,7 @@ ksana_sage::AttnParams attn_params(void* ws, void* o, int dtype, const int64_t o
 // the linear branch that the kernel then adds
 int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
               const int64_t mask_st[2], const int32_t* q_lens, const int32_t* k_lens, int causal, int flags,
-              const ksana_sage::InTensor* q_rows, float q_premul, void* stream, const ksana_sage::AttnLinear* lin) {
+              const ksana_sage::InTensor* q_rows, float q_premul, void* stream, const ksana_sage::AttnLinear* lin, bool numbered) {
   const StageRange range("ksana_sage.attention");
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_mask(s, block_mask, mask_st)) return rc;
@@ -902,15 +903,18 @@ int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_s
   ksana_sage::AttnParams p = attn_params(ws, o, dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, flags);
   if (q_rows != nullptr) p.q_rows = *q_rows, p.q_premul = q_premul;
   if (lin != nullptr) p.lin = *lin;
+  p.numbered = numbered ? 1 : 0;
   hipError_t e = ksana_sage::launch_attn_fwd(p, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? 0 : hip_fail(e, "attention launch");
 }
 
 // The quantizers of a call whose arguments have been validated: of Q, K and V, or (with_q == false, no prep) of K and V.
-// q_lens, k_lens: see QkvCall
+// q_lens, k_lens: see QkvCall; batch_rows: 0, or the attention's rows per workgroup, and *numbered says whether its numbering has been
+// written to split_ml (such calls have no cut blocks)
 int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtype, const int64_t q_st[4], const int64_t k_st[4],
               const int64_t v_st[4], const ksana_sage_shape* s, const ksana_sage_prep* prep, float sm_scale, int smooth_k,
-              int smooth_v, void* ws, void* stream, const int32_t* q_lens, const int32_t* k_lens) {
+              int smooth_v, void* ws, void* stream, const int32_t* q_lens, const int32_t* k_lens, int batch_rows, bool* numbered) {
+  *numbered = false;
   if (!smooth_v) {
     const StageRange range("ksana_sage.quant_qkv");
     ksana_sage_ws_layout l;
@@ -924,10 +928,14 @@ int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtyp
     ksana_sage::QkvCall c = qkv_call(with_q, in_tensor(q, dtype, q_st, s->D), in_tensor(k, dtype, k_st, s->D),
                                      in_tensor(v, dtype, v_st, s->D), s, l, sm_scale, smooth_k, ws);
     c.q_lens = q_lens, c.k_lens = k_lens;
+    if (batch_rows != 0) c.batch_starts = ws_at<int32_t>(ws, l.split_ml), c.rows_wg = batch_rows;
     bool used = false;
     const hipError_t e = ksana_sage::launch_quant_qkv(c, ppq, ppk, static_cast<hipStream_t>(stream), &used);
     if (e != hipSuccess) return hip_fail(e, "q, k, v quantizer launch");
-    if (used) return 0;
+    if (used) {
+      *numbered = batch_rows != 0;
+      return 0;
+    }
   }
   if (with_q && prep != nullptr && !smooth_v && one_read('v')) {
     // a norm over the token row folded in: Q's kernel takes K's row statistic along and clears the counters of K's and V's
@@ -1005,12 +1013,15 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
                      (ksana_sage::q_in_attention_pays(n_wg, (s->Lk + ksana_sage::kBlkK - 1) / ksana_sage::kBlkK) ||
                       ksana_sage::resident_call_suits(attn_params(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, flags)));
   const bool trim = (flags & KSANA_SAGE_FLAG_WS_UNSTORED) && prep == nullptr;  // what no row or key that takes part needs
+  const int attn_flags = flags & ~(KSANA_SAGE_FLAG_SMOOTH_V | KSANA_SAGE_FLAG_Q_UNSTORED | KSANA_SAGE_FLAG_WS_UNSTORED);
+  const int batch_rows =
+      !trim ? 0 : ksana_sage::batch_rows_wg(attn_params(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, attn_flags));
+  bool numbered = false;
   if (int rc = quant_qkv(!own_q, q, k, v, dtype, q_st, k_st, v_st, s, prep, sm_scale, smooth_k, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws,
-                         stream, trim ? q_lens : nullptr, trim ? k_lens : nullptr))
+                         stream, trim ? q_lens : nullptr, trim ? k_lens : nullptr, batch_rows, &numbered))
     return rc;
   const ksana_sage::InTensor q_rows = in_tensor(q, dtype, q_st, s->D);
   return attn_impl(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal,
-                   flags & ~(KSANA_SAGE_FLAG_SMOOTH_V | KSANA_SAGE_FLAG_Q_UNSTORED | KSANA_SAGE_FLAG_WS_UNSTORED), own_q ? &q_rows : nullptr, q_premul_of(sm_scale),
-                   stream);
+                   attn_flags, own_q ? &q_rows : nullptr, q_premul_of(sm_scale), stream, nullptr, numbered);
 }
 }  // namespace

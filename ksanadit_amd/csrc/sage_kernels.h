@@ -27,6 +27,44 @@ __host__ __device__ constexpr int tiles_counted(int count, int tiles) {
   return (int)(((unsigned)rows_counted(count, tiles * kBlkK) + kBlkK - 1) / kBlkK);
 }
 
+// The numbering of a dense launch over a batch with counts of its own.  Every XCD takes an eighth of every entry's blocks with
+// rows that take part, entry after entry, and then an eighth of every entry's other blocks, which have only zeros to write.
+// (Numbered by the tensor alone, an entry's blocks without rows stand before the next entry's, and work waits for a place while they
+// come and go.)  Number `at` of an XCD lies in the last of these 2 B runs that starts at or before it.  The counts are in device
+// memory: the runs' starts, the unused ones INT32_MAX, are written once per call by the quantizers (QkvCall::batch_starts), and a
+// workgroup reads them, a 64-byte line, in one scalar load.  Worked out in every workgroup instead, with the entry with the most keys
+// first, entries of equal counts took 1-5 % longer than by the tensor's numbering and some random ones 8 %.
+constexpr int kBatchEntries = 8, kBatchStarts = 2 * kBatchEntries;
+// blocks of one kind, of an entry, that an XCD takes
+__host__ __device__ constexpr int batch_share(int heads, int blocks) { return (heads * blocks + 7) / 8; }
+// an entry's blocks with rows that take part, of rows_wg rows
+__host__ __device__ constexpr int batch_blocks(int rows, int keys, int rows_wg) { return keys > 0 ? (rows + rows_wg - 1) / rows_wg : 0; }
+// The entry that a number belongs to, and then, when the entry's counts are known, the block
+struct BatchRun {
+  int b, first;  // entry, the run's first number
+  bool zeros;    // a run of blocks without rows
+};
+struct BatchPlace {
+  int b, h, qwg;  // b < 0: no such workgroup
+};
+__host__ __device__ constexpr BatchRun batch_run_of(const int (&starts)[kBatchStarts], int B, int at) {
+  int run = 0, first = 0;
+  for (int i = 1; i < kBatchStarts; ++i) {
+    const bool past = at >= starts[i];
+    run += past ? 1 : 0;
+    first = past ? starts[i] : first;
+  }
+  const bool zeros = run >= B;
+  return BatchRun{zeros ? run - B : run, first, zeros};
+}
+__host__ __device__ constexpr BatchPlace batch_place(const BatchRun& r, int xcd, int at, int heads, int n_qwg, int with_rows) {
+  const int count = r.zeros ? n_qwg - with_rows : with_rows, share = batch_share(heads, count);
+  const int i = xcd * share + (at - r.first);
+  if (at - r.first >= share || i >= heads * count) return BatchPlace{-1, 0, 0};
+  const int h = i / count;
+  return BatchPlace{r.b, h, i - h * count + (r.zeros ? with_rows : 0)};
+}
+
 // The numbering of a causal launch's workgroups.  Consecutive ones land on consecutive XCDs.  Every XCD takes pairs / 8 of the
 // (batch, head) pairs for its own and an eighth of the query blocks of the pairs left over - one run of blocks per XCD gives some
 // of them a pair's long half and others its short one.  Blocks go out from the last one down, which walks the most key tiles,
@@ -205,6 +243,10 @@ struct QkvCall {
   // nullptr, or (no folded step) the counts of the attention that follows and nobody else sees the codes: keys and query
   // rows that take no part count for the statistics as ever, but blocks made of them alone are not quantized
   const int32_t *q_lens, *k_lens;
+  // nullptr, or (no folded step) where the launch that comes first leaves the kBatchStarts numbers of the attention's blocks of
+  // rows_wg rows
+  int32_t* batch_starts;
+  int rows_wg;
 };
 hipError_t launch_quant_qkv(const QkvCall& call, const PrepParams* pq, const PrepParams* pk, hipStream_t s, bool* used);
 
@@ -292,7 +334,7 @@ struct AttnParams {
   float* split_ml;
   int split_first_block = 0, split_first_wg = 0, n_split = 0;  // filled in by the launcher
   int batch_run = 0;  // filled in by the launcher: 0, or the workgroups of one batch entry that go to one XCD
-  int packed = 0;  // filled in by the launcher: the batch's blocks are numbered by its counts (packed_place)
+  int numbered = 0;  // 1: split_ml holds the kBatchStarts numbers of a call whose rows batch_rows_wg has named
   int small_last = 0;  // filled in by the launcher: 0, or how many heads' short last blocks each XCD takes behind its whole blocks
   int wg_waves;  // 0: the launcher picks the workgroup shape; 4 or 8: forced (for measurements and tests)
   int d_out;     // channels of an output row that exist: 128, or 64 (head size 64 runs zero-padded to 128)
@@ -308,6 +350,8 @@ constexpr int kMinTilesPerSplit = 8;    // a run shorter than this does not repa
 constexpr int kMaskBlkQ = 128;           // query rows per mask row (two per workgroup)
 constexpr int kSparseMaxKeyTiles = 2048; // key tiles per head with a block mask or causal masking (tile list lives in LDS)
 hipError_t launch_attn_fwd(const AttnParams& p, hipStream_t s);
+// Rows per workgroup of a call whose blocks are to be numbered by its counts, or 0 (of p it looks at the sizes and the options)
+int batch_rows_wg(const AttnParams& p);
 // Which of `n_wg` dense workgroups the launcher cuts into runs of key tiles on the current device, and into how
 // many: workgroups [*first_wg, n_wg) into *runs each; *runs == 0 means none.
 void plan_key_split(int n_wg, int nkb, int* first_wg, int* runs);

@@ -1582,6 +1582,25 @@ __device__ __forceinline__ int tiles_in_use(const QkvCall& c, int b) {
   return c.k_lens == nullptr ? c.nkb : tiles_counted(c.k_lens[b], c.nkb);
 }
 
+// The numbers of the attention's blocks (kBatchStarts), by one wave of a workgroup of its own, the launch's first: the others'
+// work hides it (as the last one it was 0.2 us of a first stage of 5.8).
+__device__ __forceinline__ int numbers_batch(const QkvCall& c) { return c.batch_starts != nullptr ? 1 : 0; }
+__device__ __forceinline__ void number_batch(const QkvCall& c) {
+  const int lane = threadIdx.x;
+  if (lane >= 64) return;
+  const bool zeros = lane >= c.B;
+  const int b = min(zeros ? lane - c.B : lane, c.B - 1);
+  const int rows = c.q_lens != nullptr ? rows_counted(c.q_lens[b], c.Lq) : c.Lq, keys = c.k_lens != nullptr ? rows_counted(c.k_lens[b], c.Lk) : c.Lk;
+  const int with_rows = batch_blocks(rows, keys, c.rows_wg), all = (c.Lq + c.rows_wg - 1) / c.rows_wg;
+  const int share = lane < 2 * c.B ? batch_share(c.Hq, zeros ? all - with_rows : with_rows) : 0;
+  int start = 0;
+  for (int i = 0; i < 2 * c.B; ++i) {
+    const int n = __builtin_amdgcn_readlane(share, i);
+    start += i < lane ? n : 0;
+  }
+  if (lane < kBatchStarts) c.batch_starts[lane] = lane < 2 * c.B ? start : INT32_MAX;
+}
+
 template <int DT, int KIND>
 __device__ __forceinline__ void quant_q_item(int item, const QkvCall& c, const PrepParams& pp) {
   const int bh = item / c.nqb;
@@ -1750,9 +1769,11 @@ template <int DT, int KIND, bool kHeads>
 __global__ __launch_bounds__(kThreads, KIND == 0 ? 5 : 4) void quant_qkv_stage1_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
   want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   clear_status(c);
+  const int more = KIND == 0 ? numbers_batch(c) : 0;
+  if ((int)blockIdx.x < more) return number_batch(c);
   const int n_v = c.B * c.Hkv * c.nch;
   const int n_k = !c.smooth_k ? 0 : (!kHeads ? n_v : c.B * ((c.Hkv + kJointHeadsK - 1) / kJointHeadsK) * c.nch);
-  int item = blockIdx.x;
+  int item = blockIdx.x - more;
   if (item < n_k) {
     if constexpr (kHeads) {
       joint_k_sums<DT>(item, c, pk);
@@ -1815,10 +1836,12 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 6 : (kHeads ? 4 : 5)) void qu
 // Q blocks (which wait for nobody) and the V chunks work while K's chunks wait for their mean.
 template <int DT>
 __global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCall c, const HeadSync sk, const HeadSync sv) {
+  const int more = numbers_batch(c);
+  if ((int)blockIdx.x < more) return number_batch(c);
   const PrepParams none{};
   const int group = c.Hq / c.Hkv, per_head = 2 * c.nch + group * c.nqb;
-  const int bh = blockIdx.x / per_head;
-  int item = blockIdx.x - bh * per_head;
+  const int block = blockIdx.x - more, bh = block / per_head;
+  int item = block - bh * per_head;
   if (item < c.nch) {
     quant_k_chunk<DT, 0, false>(bh, item, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.nkb, c.nch, c.k_part, c.k_mean,
                                 c.k.dtype, c.smooth_k, c.k_tiles, c.k_scale, none, sk, tiles_in_use(c, bh / c.Hkv));
@@ -1841,8 +1864,10 @@ template <int DT, int KIND>
 __global__ __launch_bounds__(kThreads, 4) void quant_qkv_small_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
   want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   clear_status(c);
+  const int more = KIND == 0 ? numbers_batch(c) : 0;
+  if ((int)blockIdx.x < more) return number_batch(c);
   const int n = c.B * c.Hkv;
-  const int item = blockIdx.x;
+  const int item = blockIdx.x - more;
   const HeadSync nobody{};
   if (item < n)
     quant_k_chunk<DT, KIND, true>(item, 0, c.k.ptr, c.k.sB, c.k.sL, c.k.sH, c.Hkv, c.Lk, c.k.D, c.nkb, 1, c.k_part, c.k_mean, c.k.dtype,
@@ -2400,8 +2425,9 @@ static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepPa
   static_assert(KIND == 0 || KIND == 2, "nothing folded in, or the joint block's step");
   const dim3 block(kThreads);
   const int64_t n_q = (int64_t)c.B * c.Hq * c.nqb, n_chunks = (int64_t)c.B * c.Hkv * c.nch;
+  const int more = KIND == 0 && c.batch_starts != nullptr ? 1 : 0;  // (numbers_batch)
   if (c.nch == 1) {
-    quant_qkv_small_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, pq, pk);
+    quant_qkv_small_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks + more)), block, 0, s>>>(c, pq, pk);
     *used = true;
   } else if (c.nch <= kStageMaxChunks && 4 * (int64_t)c.B * c.Hkv * c.Lk * c.k.D <= kStageMaxBytes) {
     const int64_t tiles = 2 * (int64_t)c.B * c.Hkv * c.nkb;
@@ -2413,7 +2439,7 @@ static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepPa
       quant_qkv_stage1_kernel<DT, 2, true><<<dim3((unsigned)(n_rows + n_chunks + (c.smooth_k ? k_groups * c.nch : 0))), block, 0, s>>>(c, pq, pk);
       quant_qkv_stage2_kernel<DT, 2, true><<<dim3((unsigned)(k_groups * c.nkb + n_v2)), block, 0, s>>>(c, pk);
     } else {
-      quant_qkv_stage1_kernel<DT, KIND, false><<<dim3((unsigned)(n_q + (c.smooth_k ? 2 : 1) * n_chunks)), block, 0, s>>>(c, pq, pk);
+      quant_qkv_stage1_kernel<DT, KIND, false><<<dim3((unsigned)(n_q + (c.smooth_k ? 2 : 1) * n_chunks + more)), block, 0, s>>>(c, pq, pk);
       quant_qkv_stage2_kernel<DT, KIND, false><<<dim3((unsigned)(2 * n_v2)), block, 0, s>>>(c, pk);
     }
     *used = true;
@@ -2428,7 +2454,7 @@ static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepPa
     const hipError_t e = launch_clear_ints(y.k_counter, n_words, s);
     if (e != hipSuccess) return e;
     const HeadSync sk{y.k_counter, y.k_ready, y.k_status, opt.wait_ticks, host}, sv{y.v_counter, y.v_ready, y.v_status, opt.wait_ticks, host};
-    quant_qkv_meet_kernel<DT><<<dim3((unsigned)(n_q + 2 * n_chunks)), block, 0, s>>>(c, sk, sv);
+    quant_qkv_meet_kernel<DT><<<dim3((unsigned)(n_q + 2 * n_chunks + more)), block, 0, s>>>(c, sk, sv);
     *used = true;
   }
   return hipGetLastError();
@@ -2439,7 +2465,7 @@ hipError_t launch_quant_qkv(const QkvCall& call, const PrepParams* pq, const Pre
   QkvCall c = call;
   const int kind = pq != nullptr ? pq->kind : (pk != nullptr ? pk->kind : 0);
   if (kind != 0 && kind != 2) return hipSuccess;
-  if ((int64_t)c.B * c.Hq * c.nqb + 2 * (int64_t)c.B * c.Hkv * c.nkb > INT32_MAX) return hipSuccess;
+  if ((int64_t)c.B * c.Hq * c.nqb + 2 * (int64_t)c.B * c.Hkv * c.nkb >= INT32_MAX) return hipSuccess;
   // (a side without anything to apply runs with every step of its parameters switched off)
   PrepParams off{};
   off.kind = kind;

@@ -253,10 +253,9 @@ def test_a_shared_last_block_in_batches_with_lengths(hip_device, k_len, rows):
 
 @pytest.mark.parametrize("B,H,Lq,Lk", [(3, 40, 700, 900), (5, 16, 1000, 300), (64, 2, 700, 130), (65, 2, 700, 130), (2, 40, 2000, 700)])
 @pytest.mark.parametrize("wg_waves", [4, 8])
-def test_batches_are_numbered_by_their_counts(hip_device, B, H, Lq, Lk, wg_waves):
-    """Grids of more than a round whose workgroups work out which block is theirs from the entries' counts - in any order, equal,
-    none, one, all, out of range - against the same operands walked through a mask of ones, whose grid is numbered as the
-    tensor is laid out.  (More than six entries and grids of one round are, too.)"""
+def test_batches_with_counts(hip_device, B, H, Lq, Lk, wg_waves):
+    """Counts in any order, equal, none, one, all, out of range against the same operands walked through a mask of ones: on a kept
+    workspace, whose grid is numbered entry after entry."""
     print(f"case B={B} H={H} Lq={Lq} Lk={Lk} waves={wg_waves}", flush=True)
     g = torch.Generator().manual_seed(B * Lq + Lk)
     q, k, v = (torch.randn((B, n, H, 128), generator=g).to(torch.bfloat16).to(hip_device) for n in (Lq, Lk, Lk))
@@ -275,3 +274,70 @@ def test_batches_are_numbered_by_their_counts(hip_device, B, H, Lq, Lk, wg_waves
         if q_lens is not None:
             for b in range(B):
                 assert (got[b, int(q_lens[b]) :] == 0).all()
+
+
+# Grids of 1.3 to 4.5 rounds.  The numbers come from the quantizers' first stage, their launch for at most 256 keys or the one that
+# reads K and V once.
+NUMBERED = [
+    (3, 24, 8, 3001, 1100, 128, torch.float16),  # 57 rows in the last block, whose waves share the keys of entries with more than 1024
+    (4, 24, 24, 1300, 1300, 128, torch.bfloat16),  # 20 rows
+    (2, 24, 24, 1500, 300, 64, torch.float16),
+    (8, 24, 24, 1000, 600, 128, torch.bfloat16),  # the most entries
+    (6, 16, 16, 1500, 300, 128, torch.bfloat16),
+    (2, 12, 12, 6946, 138, 128, torch.float16),  # K and V in one launch
+    (3, 40, 40, 1500, 700, 64, torch.bfloat16),
+    (2, 50, 50, 1250, 2560, 128, torch.bfloat16),  # workgroups of 8 waves
+    (2, 50, 10, 1250, 2560, 64, torch.float16),
+    (2, 16, 16, 3500, 16500, 128, torch.bfloat16),  # K and V read once
+    (3, 7, 7, 3200, 600, 128, torch.bfloat16),  # heads that eight does not divide
+]
+
+
+def _counts(B, Lq, Lk):
+    g = torch.Generator().manual_seed(B * Lq + Lk)
+    rand = [torch.randint(0, n + 1, (B,), generator=g) for n in (Lq, Lk)]
+    fall = [torch.tensor([n - n * 55 * b // (100 * max(B - 1, 1)) for b in range(B)]) for n in (Lq, Lk)]
+    odd = torch.tensor([(0, 1, Lq - 1, Lq + 100, -5, 128, 129, Lq)[(b + 2) % 8] for b in range(B)])
+    few = torch.tensor([(0, Lk, 1, Lk + 1, -1, 64, 65, Lk)[b % 8] for b in range(B)])
+    yield from ((fall[0], fall[1]), (fall[0].flip(0), fall[1].flip(0)), (rand[0], rand[1]), (odd, few), (torch.full((B,), Lq), torch.full((B,), Lk)),
+                (torch.full((B,), Lq // 2), torch.full((B,), Lk // 2)), (rand[0], None), (None, few), (torch.zeros(B, dtype=torch.int64), None))
+
+
+@pytest.mark.parametrize("B,H,Hkv,Lq,Lk,D,dtype", NUMBERED)
+def test_batches_numbered_by_their_counts(hip_device, B, H, Hkv, Lq, Lk, D, dtype):
+    """Whole calls, whose blocks are numbered by the entries' counts, against the same calls on a kept workspace, which are not."""
+    print(f"case B={B} H={H}/{Hkv} Lq={Lq} Lk={Lk} D={D} {dtype}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(Lq)
+    q, k, v = (torch.randn((B, n, h, D), generator=g, device=hip_device).to(dtype) for n, h in ((Lq, H), (Lk, Hkv), (Lk, Hkv)))
+    ws = sage_ops.workspace_for(q, k)
+    for q_lens, k_lens in _counts(B, Lq, Lk):
+        kw = {"q_lens": q_lens, "k_lens": k_lens}
+        want = sage_ops.sageattn(q, k, v, workspace=ws, **kw)
+        del_me = torch.full_like(q, float("nan"))  # (memory that the next result may lie in)
+        del del_me
+        got = sage_ops.sageattn(q, k, v, **kw)
+        assert torch.equal(got, want), kw
+        for b in range(B if q_lens is not None else 0):
+            assert not got[b, max(0, int(q_lens[b])) :].any(), (kw, b)
+
+
+def test_numbered_batches_replayed_with_other_counts(hip_device):
+    """A captured call numbers its blocks anew in every replay, by the counts that are there then."""
+    B, H, L = 4, 24, 1300
+    g = torch.Generator(device=hip_device).manual_seed(5)
+    q, k, v = (torch.randn((B, L, H, 128), generator=g, device=hip_device).half() for _ in "qkv")
+    q_lens, k_lens = (torch.full((B,), L, dtype=torch.int32, device=hip_device) for _ in "qk")
+    call = lambda: sage_ops.sageattn(q, k, v, q_lens=q_lens, k_lens=k_lens)  # noqa: E731
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for i, (ql, kl) in enumerate(_counts(B, L, L)):
+        for to, n in ((q_lens, ql), (k_lens, kl)):
+            to.copy_(torch.full((B,), L, dtype=torch.int32) if n is None else n.to(torch.int32))
+        out.fill_(float("nan"))
+        graph.replay()
+        want = call()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), i
