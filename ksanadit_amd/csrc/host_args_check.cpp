@@ -52,20 +52,22 @@ static int causal_numbering_is_wrong(int pairs, int n_qwg, unsigned* kinds) {
   return n != pairs * n_qwg;
 }
 
-// Every block of a batch numbered by its counts belongs to one workgroup of a grid of the launcher's size, and an XCD starts those
-// that have only zeros to write after all others.
-static int batch_numbering_is_wrong(int B, int heads, int n_qwg, const int* with_rows) {
-  int starts[ksana_sage::kBatchStarts], at = 0;
+// Every block of a batch numbered by its counts belongs to one workgroup of a grid of the launcher's size, and an XCD starts the
+// entries in the given order, blocks that have only zeros to write after all others.
+static int batch_numbering_is_wrong(int B, int heads, int n_qwg, const int* with_rows, const int* order) {
+  int starts[ksana_sage::kBatchStarts], at = 0, entries = 0;
   for (int i = 0; i < ksana_sage::kBatchStarts; ++i) {
     starts[i] = i < 2 * B ? at : INT32_MAX;
-    if (i < 2 * B) at += ksana_sage::batch_share(heads, i < B ? with_rows[i] : n_qwg - with_rows[i - B]);
+    if (i < 2 * B) at += ksana_sage::batch_share(heads, i < B ? with_rows[order[i]] : n_qwg - with_rows[order[i - B]]);
+    if (i < B) entries |= order[i] << (4 * i);
   }
+  starts[0] = entries;
   const int per_xcd = B * ((heads * n_qwg + 7) / 8 + 1);
   if (at > per_xcd) return 1;
   std::vector<char> seen((size_t)B * heads * n_qwg, 0);
   int n = 0;
   for (int xcd = 0; xcd < 8; ++xcd) {
-    bool zeros = false;
+    int before = 0;
     for (int i = 0; i < per_xcd; ++i) {
       const ksana_sage::BatchRun run = ksana_sage::batch_run_of(starts, B, i);
       if (run.b < 0 || run.b >= B) return 1;
@@ -73,8 +75,10 @@ static int batch_numbering_is_wrong(int B, int heads, int n_qwg, const int* with
       if (p.b < 0) continue;
       if (p.b != run.b || p.h < 0 || p.h >= heads || p.qwg < 0 || p.qwg >= n_qwg) return 1;
       const bool zero = p.qwg >= with_rows[p.b];
-      if (zero != run.zeros || (zeros && !zero) || seen[((size_t)p.b * heads + p.h) * n_qwg + p.qwg]++ != 0) return 1;
-      zeros = zero;
+      int here = zero ? B : 0;
+      while (order[here % B] != p.b) ++here;
+      if (zero != run.zeros || here < before || seen[((size_t)p.b * heads + p.h) * n_qwg + p.qwg]++ != 0) return 1;
+      before = here;
       ++n;
     }
   }
@@ -200,7 +204,12 @@ int main() {
     const int B = 2 + next(ksana_sage::kBatchEntries - 1), heads = 1 + next(70), n_qwg = 1 + next(40), kind = next(4);
     int with_rows[ksana_sage::kBatchEntries];
     for (int& w : with_rows) w = kind == 0 ? next(n_qwg + 1) : kind == 1 ? n_qwg : kind == 2 ? 0 : next(2) * n_qwg;
-    if (batch_numbering_is_wrong(B, heads, n_qwg, with_rows)) ++g_failed, std::printf("batch numbering: %d entries, %d heads, %d blocks\n", B, heads, n_qwg);
+    int order[ksana_sage::kBatchEntries];
+    for (int e = 0; e < B; ++e) {
+      const int to = next(e + 1);
+      order[e] = order[to], order[to] = e;
+    }
+    if (batch_numbering_is_wrong(B, heads, n_qwg, with_rows, order)) ++g_failed, std::printf("batch numbering: %d entries, %d heads, %d blocks\n", B, heads, n_qwg);
   }
   // one round and a block more, four and a half rounds and a block more, entries, options, cut blocks
   EXPECT(batch_rows(2, 16, 2048, 600), 0);

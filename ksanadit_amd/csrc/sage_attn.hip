@@ -89,11 +89,15 @@ __device__ __forceinline__ void lds_copy16_at(const v4i& buffer, unsigned lane_o
 // 128 channels and the operands keep their layout; see kMagicI2 for what is left out and why nothing is lost; the
 // result equals the full-width code's up to the rounding of one constant in the exponent).
 // kLinear: the sparse-linear backend's linear branch is added to the result in the epilogue.
-template <int DT, bool kPwlExp, bool kSparse, int kW, bool kTileSkip, int kG, bool kCausal, bool kLinear>
+// kNumbered: the blocks of a batch are numbered by its counts (batch_rows_wg).  A variant of its own: with this behind a branch in the
+// dense ones their scalar registers run short and arguments are loaded anew in every workgroup's set-up (16 heads of 2600 tokens
+// 58.7 / 59.3 us, 24 of 2000 53.1 / 54.0).
+template <int DT, bool kPwlExp, bool kSparse, int kW, bool kTileSkip, int kG, bool kCausal, bool kLinear, bool kNumbered>
 __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel(const AttnParams p, int n_qwg,
                                                                                    int n_wg, int wg_per_xcd) {
   want(p.q_rows.ptr, p.k_tiles, p.o.sH, p.block_mask, n_qwg);
-  constexpr bool kCanSplit = !kSparse && kW == 8, kDense = !kSparse && !kCausal;
+  constexpr bool kCanSplit = !kSparse && kW == 8 && !kNumbered;
+  static_assert(!kNumbered || (!kSparse && !kCausal && !kPwlExp && !kTileSkip), "batches with counts: the dense default variant");
   static_assert(kSparse || !kCausal || (kW == 4 && !kPwlExp && !kTileSkip), "causal without a list: the default variant in 4 waves");
   // kCausal == false: the caller vouches that p.causal is 0, and everything that serves the diagonal (the per-wave
   // last tile, 32 lane masks held in scalar registers, the selects that blank a wave's probabilities past its rows)
@@ -115,8 +119,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   int lq = p.Lq, lk = p.Lk;
   const bool is_run = kCanSplit && (int)blockIdx.x >= p.split_first_block;  // uniform
   const int run_id = is_run ? (int)blockIdx.x - p.split_first_block : 0;    // the partial result's place in the workspace
-  const bool numbered = kDense && p.numbered != 0;
-  if (numbered) {  // (BatchRun, BatchPlace)
+  if constexpr (kNumbered) {  // (BatchRun, BatchPlace)
     typedef const __attribute__((address_space(4))) int32_t* Constant;
     const Constant at_starts = reinterpret_cast<Constant>(reinterpret_cast<uintptr_t>(p.split_ml));
     int starts[kBatchStarts];
@@ -175,7 +178,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
     qwg = wg - bh * n_qwg;
     if (causal) qwg = n_qwg - 1 - qwg;  // the long ones first, as above
   }
-  if (!numbered) {
+  if constexpr (!kNumbered) {
     b = bh / p.Hq, h = bh - b * p.Hq;
     take_counts(p.q_lens, p.k_lens, b, lq, lk);
   }
@@ -1238,7 +1241,7 @@ constexpr size_t max_lds() {
                  : WgShape<kW>::kRingBytes + 2048 + (kW == 8 ? kMaxKeyTiles : kShortMaxKeyTiles) * 4;
 }
 
-template <int DT, bool kPwlExp, bool kSparse, int kW, bool kCausal, bool kTileSkip = false, int kG = 4, bool kLinear = false>
+template <int DT, bool kPwlExp, bool kSparse, int kW, bool kCausal, bool kTileSkip = false, int kG = 4, bool kLinear = false, bool kNumbered = false>
 hipError_t launch_variant(const AttnParams& p, dim3 grid, size_t lds, int n_qwg, int n_wg, int wg_per_xcd,
                           hipStream_t s) {
   // more than 64 KiB of dynamic LDS has to be requested per kernel, once per device
@@ -1249,12 +1252,12 @@ hipError_t launch_variant(const AttnParams& p, dim3 grid, size_t lds, int n_qwg,
   if (e != hipSuccess) return e;
   if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
   if (!requested[dev].load(std::memory_order_acquire)) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal, kLinear>),
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal, kLinear, kNumbered>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)max_lds<kSparse, kW>());
     if (e != hipSuccess) return e;
     requested[dev].store(true, std::memory_order_release);
   }
-  sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal, kLinear><<<grid, dim3(kW * 64), lds, s>>>(p, n_qwg, n_wg, wg_per_xcd);
+  sage_attn_fwd_kernel<DT, kPwlExp, kSparse, kW, kTileSkip, kG, kCausal, kLinear, kNumbered><<<grid, dim3(kW * 64), lds, s>>>(p, n_qwg, n_wg, wg_per_xcd);
   return hipGetLastError();
 }
 
@@ -1277,6 +1280,14 @@ hipError_t launch_shape(const AttnParams& p, dim3 grid, size_t lds, int n_qwg, i
   const bool bf16 = p.o.dtype == KSANA_SAGE_BF16;
   // head size 64: the matrix instructions on the zero halves are left out (plain exact-exponential calls; the other
   // variants run the full-width code on the same operands, which gives the same bits)
+  if constexpr (!kSparse && !kCausal)
+    if (p.numbered != 0) {
+      if (p.d_out <= 64)
+        return bf16 ? launch_variant<KSANA_SAGE_BF16, false, false, kW, false, false, 2, false, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
+                    : launch_variant<KSANA_SAGE_FP16, false, false, kW, false, false, 2, false, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+      return bf16 ? launch_variant<KSANA_SAGE_BF16, false, false, kW, false, false, 4, false, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
+                  : launch_variant<KSANA_SAGE_FP16, false, false, kW, false, false, 4, false, true>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
+    }
   if (p.exact_exp2 && !p.tile_skip && p.d_out <= 64)
     return bf16 ? launch_variant<KSANA_SAGE_BF16, false, kSparse, kW, kCausal, false, 2>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s)
                 : launch_variant<KSANA_SAGE_FP16, false, kSparse, kW, kCausal, false, 2>(p, grid, lds, n_qwg, n_wg, wg_per_xcd, s);
@@ -1383,20 +1394,22 @@ static dim3 xcd_grid(AttnParams* p, int n_qwg, int n_wg, int* wg_per_xcd) {
   return dim3(*wg_per_xcd * 8);
 }
 
-// Dense calls, uncut, of more than one round - one round has no order - and up to four and a half.  us, by the tensor's numbering /
-// by the counts:
-//                                        all full      falling to 45 %   rising        half of each    random
-//   2 x 12 heads of 6946 on 138 (2.6)    42.4 / 43.1   38.9 / 37.1       38.7 / 37.3   34.2 / 32.0     37.0 / 35.2
-//   2 x 24 of 3500 (2.6)                 215 / 215.5   150.6 / 152       167 / 150     98.4 / 100.2    140 / 141
-//   3 x 24 of 3001 on 4099 (3.4)         282 / 282.5   185.5 / 181       193 / 182.5   103 / 101       131.5 / 135
-//   5 x 32 of 1500 (3.8)                 183 / 184     142.5 / 131.5     140 / 130     103 / 94        146 / 148.5
-//   6 x 24 of 2000 (4.5)                 243 / 244     174 / 168.5       176 / 170     120 / 119.5     137 / 132
-//   8 x 24 of 1000 on 600 (3.0)          83.5 / 84.2   70.7 / 68.0       71.0 / 67.5   53.6 / 51.9     63.3 / 58.9
-// What all full entries lose, up to 1 us, is the load of the numbers ahead of the counts.  In longer grids the order of the last round is a smaller part,
-// and gains and losses cancel: eight shapes of 5 to 15 rounds in seventeen such sets of counts 0.994 on average, 0.86 to 1.06 each
-// (6 x 64 of 2000, 12 rounds, half of each 334 / 354: blocks that start together keep each other's step).
+// Dense calls in the default variant, uncut, of more than one round - one round has no order - and up to four and a half.  us, by the
+// tensor's numbering / by the counts (entries full, falling to or rising from 45 %, half full, of random counts):
+//                                        full          falling         rising          half          random
+//   2 x 12 heads of 6946 on 138 (2.6)    42.5 / 43.3   38.7 / 37.2     38.5 / 38.1     34.1 / 32.2   37.2 / 35.0
+//   2 x 24 of 3500 (2.6)                 216 / 216     151.4 / 152.9   167.2 / 152.2   98.8 / 100    140.7 / 140.4
+//   3 x 24 of 3001 on 4099 (3.4)         287.5 / 288   187.4 / 183.7   195.7 / 183.4   104 / 102.4   132.6 / 135.8
+//   5 x 32 of 1500 (3.8)                 181 / 181     142 / 129.5     139 / 129.5     103 / 93      147 / 155
+//   6 x 24 of 2000 (4.5)                 246 / 247     175 / 170       177 / 171       120 / 119     137 / 132
+//   8 x 24 of 1000 on 600 (3.0)          82.0 / 82.2   69.5 / 66.0     70.0 / 66.9     53.2 / 51.3   62.6 / 58.0
+// What full entries can lose, up to 0.8 us a call, is the load of the numbers ahead of the counts.  In longer grids the last round's
+// order is a smaller part, and gains and losses cancel: eight shapes of 5 to 15 rounds in eight such sets of counts 0.991 on average, 0.92
+// to 1.05 each (6 x 64 of 2000, 12 rounds, half full 331 / 347: blocks that start together keep in step).
 int batch_rows_wg(const AttnParams& p) {
-  if (p.B < 2 || p.B > kBatchEntries || (p.q_lens == nullptr && p.k_lens == nullptr) || p.block_mask != nullptr || p.causal || p.nkb > kMaxKeyTiles) return 0;
+  if (p.B < 2 || p.B > kBatchEntries || (p.q_lens == nullptr && p.k_lens == nullptr) || p.block_mask != nullptr || p.causal || !p.exact_exp2 || p.tile_skip ||
+      p.nkb > kMaxKeyTiles)
+    return 0;
   int waves = pick_wg_waves(p);
   if (waves == 4 && p.nkb > kShortMaxKeyTiles) waves = 8;
   const int rows = 32 * waves, n_wg = p.B * p.Hq * ((p.Lq + rows - 1) / rows);

@@ -28,13 +28,15 @@ __host__ __device__ constexpr int tiles_counted(int count, int tiles) {
 }
 
 // The numbering of a dense launch over a batch with counts of its own.  Every XCD takes an eighth of every entry's blocks with
-// rows that take part, entry after entry, and then an eighth of every entry's other blocks, which have only zeros to write.
-// (Numbered by the tensor alone, an entry's blocks without rows stand before the next entry's, and work waits for a place while they
-// come and go.)  Number `at` of an XCD lies in the last of these 2 B runs that starts at or before it.  The counts are in device
+// rows that take part, the entry with the most keys first, and then an eighth of every entry's other blocks, which have only zeros to
+// write.  (Numbered by the tensor alone, an entry's blocks without rows stand before the next entry's, and work waits for a place while
+// they come and go.)  Number `at` of an XCD lies in the last of these 2 B runs that starts at or before it.  The counts are in device
 // memory: the runs' starts, the unused ones INT32_MAX, are written once per call by the quantizers (QkvCall::batch_starts), and a
-// workgroup reads them, a 64-byte line, in one scalar load.  Worked out in every workgroup instead, with the entry with the most keys
-// first, entries of equal counts took 1-5 % longer than by the tensor's numbering and some random ones 8 %.
+// workgroup reads them, a 64-byte line, in one scalar load; in the place of the first, which is 0, stand the entries of the runs,
+// four bits each.  60 random calls of 2 to 8 entries, on average (and the worst) of the time by the tensor's numbering: 0.917 (0.99);
+// entry after entry 0.932 (0.99); worked out by every workgroup itself, for up to six entries, 0.952 (1.035).
 constexpr int kBatchEntries = 8, kBatchStarts = 2 * kBatchEntries;
+static_assert(kBatchEntries <= 8, "four bits each, none of them the sign");
 // blocks of one kind, of an entry, that an XCD takes
 __host__ __device__ constexpr int batch_share(int heads, int blocks) { return (heads * blocks + 7) / 8; }
 // an entry's blocks with rows that take part, of rows_wg rows
@@ -55,7 +57,7 @@ __host__ __device__ constexpr BatchRun batch_run_of(const int (&starts)[kBatchSt
     first = past ? starts[i] : first;
   }
   const bool zeros = run >= B;
-  return BatchRun{zeros ? run - B : run, first, zeros};
+  return BatchRun{(starts[0] >> (4 * (zeros ? run - B : run))) & 15, first, zeros};
 }
 __host__ __device__ constexpr BatchPlace batch_place(const BatchRun& r, int xcd, int at, int heads, int n_qwg, int with_rows) {
   const int count = r.zeros ? n_qwg - with_rows : with_rows, share = batch_share(heads, count);

@@ -1593,12 +1593,19 @@ __device__ __forceinline__ void number_batch(const QkvCall& c) {
   const int rows = c.q_lens != nullptr ? rows_counted(c.q_lens[b], c.Lq) : c.Lq, keys = c.k_lens != nullptr ? rows_counted(c.k_lens[b], c.Lk) : c.Lk;
   const int with_rows = batch_blocks(rows, keys, c.rows_wg), all = (c.Lq + c.rows_wg - 1) / c.rows_wg;
   const int share = lane < 2 * c.B ? batch_share(c.Hq, zeros ? all - with_rows : with_rows) : 0;
-  int start = 0;
-  for (int i = 0; i < 2 * c.B; ++i) {
-    const int n = __builtin_amdgcn_readlane(share, i);
-    start += i < lane ? n : 0;
+  int rank = 0;  // of this lane's entry
+  for (int j = 0; j < c.B; ++j) {
+    const int other = __builtin_amdgcn_readlane(keys, j);
+    rank += other > keys || (other == keys && j < b) ? 1 : 0;
   }
-  if (lane < kBatchStarts) c.batch_starts[lane] = lane < 2 * c.B ? start : INT32_MAX;
+  const int run = lane < 2 * c.B ? rank + (zeros ? c.B : 0) : lane;
+  int start = 0, entries = 0;
+  for (int i = 0; i < 2 * c.B; ++i) {
+    const int n = __builtin_amdgcn_readlane(share, i), r = __builtin_amdgcn_readlane(run, i);
+    start += r < run ? n : 0;
+    if (i < c.B) entries |= i << (4 * r);
+  }
+  if (lane < kBatchStarts) c.batch_starts[run] = run == 0 ? entries : (run < 2 * c.B ? start : INT32_MAX);
 }
 
 template <int DT, int KIND>
