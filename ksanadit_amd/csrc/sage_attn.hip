@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
       // XCD a contiguous run of (head, query block) pairs so the workgroups that stream the same
       // K/V tiles share one L2.
       const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
-      if (p.small_last != 0) {
+      if (!kSparse && !kCausal && p.small_last != 0) {
         // Short last blocks (see launch_attn_fwd) behind the whole ones: an XCD's run of whole blocks, then its share of the
         // heads' last ones.
         const int whole = wg_per_xcd - p.small_last, n_pairs = p.B * p.Hq, n_whole = n_pairs * (n_qwg - 1);
@@ -1453,11 +1453,16 @@ hipError_t launch_attn_fwd(const AttnParams& params, hipStream_t s) {
                ? launch_variant<KSANA_SAGE_BF16, false, true, 4, false, false, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s)
                : launch_variant<KSANA_SAGE_FP16, false, true, 4, false, false, 4, true>(p, grid, max_lds<true, 4>(), n_qwg, n_wg, wg_per_xcd, s);
   }
-  // Dense calls whose heads end in a short block (at most half a workgroup's rows, which takes a third to half of a whole one's
-  // time): these start last, so that a round they do not fit into is longer by one of them and not by a whole block.
+  // Dense calls whose heads end in a short block, of at most half a workgroup's rows, and that take a round less without these: the
+  // short ones start last, so that the round they do not fit into is longer by one of them and not by a whole block.  us, in the order
+  // of their index / last, 4 waves: 40 heads of 1560 tokens (1.02 rounds) 56.7 / 54.8, 2 x 32 of 1062 (1.1) 58.7 / 55.5, 4 x 40 of 416
+  // on 2446 (1.25) 107 / 95.5, 4 x 24 of 2110 (3.2, 64 channels) 130 / 123.4, 4 x 40 of 6185 on 819 (15.3) 357 / 359; 8 waves: 4 x 64 of 624
+  // on 4389 (3.0) 359 / 346.5, of 541 on 2302 (3.0) 238 / 241.5; 45 such calls 0.979 on average.  Where the rounds are as many without them
+  // it is no gain: 45 calls 1.003, 64 of 3603 (3.75) 296 / 301, 4 x 16 of 1551 (1.75) 87.5 / 89.1; below a round 12 of 2873 63.1 / 64.3.
   auto small_blocks_last = [&]() {
-    const int pairs = p.B * p.Hq;
+    const int pairs = p.B * p.Hq, round = (waves == 4 ? 2 : 1) * compute_units();
     if (sparse || p.batch_run != 0 || n_qwg < 2 || 2 * (p.Lq - (n_qwg - 1) * rows) > rows) return;
+    if ((n_wg - pairs + round - 1) / round == (n_wg + round - 1) / round) return;
     p.small_last = (pairs + 7) / 8;
     wg_per_xcd = (pairs * (n_qwg - 1) + 7) / 8 + p.small_last;
     grid = dim3(wg_per_xcd * 8);
