@@ -803,7 +803,8 @@ def sageattn(
           and (sm_scale is None or type(sm_scale) is float) and type(is_causal) is bool and type(smooth_k) is bool):
         # The call as models make it, the plan known: nothing left but to find a place for the result.  Host time of a call of
         # 32 tokens through the operator, as below / here: 10.1 / 8.6 us.
-        out = (torch.empty_like(q) if plan.out_like_q and type(q) is torch.Tensor
+        # (empty_like would hand on a subclass and the names of named dimensions)
+        out = (torch.empty_like(q) if plan.out_like_q and type(q) is torch.Tensor and not q.has_names()
                else torch.empty(plan.out_shape, dtype=plan.dtype, device=plan.device))
         blob = None if plan.one_launch else torch.empty(plan.ws_bytes, dtype=torch.uint8, device=plan.device)
         if log.isEnabledFor(10):  # logging.DEBUG

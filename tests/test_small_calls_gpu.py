@@ -147,6 +147,10 @@ def test_calls_without_options_and_the_general_call(hip_device, Lk):
     assert not torch.equal(sage_ops.sageattn(q, k, v, sm_scale=scale), first)
     for i in range(20):  # more settings than are kept
         assert torch.equal(sage_ops.sageattn(q, k, v, sm_scale=0.01 * i), sage_ops.sageattn(q, k, v, sm_scale=0.01 * i, out_dtype=q.dtype)), i
+    named = [t.refine_names("B", "L", "H", "D") for t in (q, k, v)]  # names of the input are no names of the result, in any call
+    for _ in range(2):
+        out = sage_ops.sageattn(*named)
+        assert not out.has_names() and torch.equal(out, sage_ops.sageattn(q, k, v))
     empty = q[:, :0]
     for _ in range(2):
         assert sage_ops.sageattn(empty, k, v).shape == empty.shape
