@@ -82,8 +82,8 @@ __device__ __forceinline__ float lane_xor(float v) {
 // The factor into int8 and the scale back of a largest absolute value that lanes i and i ^ 1 share: 127 / amax and
 // amax / 127, both 0 for 0.  A correctly rounded division is about ten instructions on a wave's every lane, so one is
 // done for the two quotients, the first by the even lanes and the second by the odd ones, and they exchange them.
-// Joint text and image attention, 24 heads x 8 448 tokens, whose quantizers' vector units are busy over half of the time:
-// 361.6 -> 358.1 us together with the squares' fused sums; no case is slower.
+// us, two divisions / one: short calls in one launch, replayed from a graph, 65 tokens of 4 x 24 heads 9.53 / 9.38, 250 of 40 16.50 /
+// 16.32; joint block of 2 x 2577 tokens of 24 heads 164.3 / 163.7; dense calls are the same.
 struct Int8Scale {
   float inv, scale;
 };
@@ -97,8 +97,9 @@ __device__ __forceinline__ Int8Scale int8_scale(float amax) {
 
 // Reductions over the lanes of a wave without the LDS crossbar: partners meet through DPP and the lane swaps, whose results the
 // next instruction can have, where a shuffle is an LDS round trip - 48 of them stood between a chunk's last row and its sums.  us per
-// call, shuffles / this: 40 heads of 1560 tokens 58.2 / 57.0, joint block of 2 x 774 tokens of 24 heads 50.8 / 49.2, sparse-linear
-// call of 40 heads of 32760 rows 1895 / 1869, of 2 x 40 of 29672 2352 / 2300 (the averages of its blocks), V smoothing 66.0 / 64.2.
+// call, shuffles / this, the rest alike: 40 heads of 1560 tokens 57.4 / 55.4, with V smoothing 75.6 / 73.4, 2 x 16 of 3000 114.2 /
+// 112.5, 24 of 4352 172.0 / 171.1, joint block of 2 x 774 tokens of 24 heads 51.5 / 50.8, sparse-linear call of 2 x 40 heads of 29672
+// rows 3170 / 3125 (the averages of its blocks), of 40 of 32760 1858 / 1840.
 struct Sum {
   static __device__ __forceinline__ float of(float a, float b) { return a + b; }
 };

@@ -170,12 +170,16 @@ __device__ __forceinline__ void qwen_row(QwenRow& f, const PrepParams& pp, int r
     for (int j = 0; j < 4; ++j) f.cs[j] = t4[j];
   }
 }
-template <int DT>
+// kFused: the squares of half values are exact (bf16: from 2^-63 up), so a fused multiply-add rounds like the sum alone and is an
+// instruction less.  us, apart / fused: several heads per item, whose vector units are busy over half of the time, 2 x 4352 tokens of
+// 24 heads 345.7 / 344.3, 2 x 1328 73.1 / 72.2; one head per item, bound by the length of its chain, the other way round: 2 x 774
+// 49.4 / 50.3, 2 x 1024 53.2 / 54.1, 1756 61.8 / 62.5.
+template <int DT, bool kFused>
 __device__ __forceinline__ void prep16_qwen(float* x, const QwenRow& f, float eps) {
   if (f.w != nullptr) {
     float ss = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) ss = __fmaf_rn(x[e], x[e], ss);  // squares of half values are exact: one rounding, the sum's
+    for (int e = 0; e < 16; ++e) ss = kFused ? __fmaf_rn(x[e], x[e], ss) : (e == 0 ? x[0] * x[0] : ss + x[e] * x[e]);
     ss = ss + lane_xor<1>(ss);
     ss = ss + lane_xor<2>(ss);
     ss = ss + lane_xor<4>(ss);
@@ -210,7 +214,7 @@ template <int DT>
 __device__ __forceinline__ void prep16_qwen(float* x, const PrepParams& pp, int row, int c16) {
   QwenRow f;
   qwen_row(f, pp, row, c16);
-  prep16_qwen<DT>(x, f, pp.eps);
+  prep16_qwen<DT, false>(x, f, pp.eps);
 }
 
 // The pieces of the Wan step on the 16 channels of a lane.
@@ -1641,7 +1645,7 @@ __device__ __forceinline__ void joint_q_item(int item, const QkvCall& c, const P
     widen8<DT>(next[0], x);
     widen8<DT>(next[1], x + 8);
     if (i + 1 < n) fetch_row16(base + (h0 + i + 1) * c.q.sH, valid, next);
-    if (valid) prep16_qwen<DT>(x, f, pp.eps);
+    if (valid) prep16_qwen<DT, true>(x, f, pp.eps);
     const int64_t at = ((int64_t)b * c.Hq + h0 + i) * c.lq_pad + row;
     quant_q_row(x, c16, premul_lane, c.q_scale + at, c.q_i8 + at * kD);
   }
@@ -1677,7 +1681,7 @@ __device__ __forceinline__ void joint_k_sums(int item, const QkvCall& c, const P
       float x[16];
       widen8<DT>(raw[hh][0], x);
       widen8<DT>(raw[hh][1], x + 8);
-      if (row < c.Lk) prep16_qwen<DT>(x, f, pp.eps);
+      if (row < c.Lk) prep16_qwen<DT, true>(x, f, pp.eps);
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[hh][e] = first ? x[e] : acc[hh][e] + x[e];
       __builtin_amdgcn_sched_barrier(0);
@@ -1746,7 +1750,7 @@ __device__ __forceinline__ void joint_k_item(int item, const QkvCall& c, const P
     for (int i = 0; i < R; ++i) {
       const bool valid = blk * kBlkK + i * kSlots + slot < c.Lk;
       if (valid) {  // (a row that is not there has been read as zeros and stays so)
-        prep16_qwen<DT>(x[i], f[i], pp.eps);
+        prep16_qwen<DT, true>(x[i], f[i], pp.eps);
 #pragma unroll
         for (int e = 0; e < 16; ++e) x[i][e] = x[i][e] - s_mean[hh][c16 * 16 + e];
       }
