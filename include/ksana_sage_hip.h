@@ -114,7 +114,8 @@ typedef struct ksana_sage_ws_layout {
                     /*       dtype; zeros without V smoothing); the attention adds it to its output     */
   uint64_t split_o; /* fp32  [256, 256, D]: scratch of the attention kernel - unnormalised accumulators */
                     /*       of workgroups whose key loop was cut into runs (see ksana_sage_attn_fwd)   */
-  uint64_t split_ml;/* fp32  [256, 256, 2]: their running maxima and row sums                           */
+  uint64_t split_ml;/* fp32  [256, 256, 2]: their running maxima and row sums; or, of a batch with counts, the     */
+                    /*       numbering of its blocks                                                    */
   uint64_t k_sync;  /* int32 [2 * B*Hkv * 32 + 32]: per head a chunk counter and a ready flag (each in a 128-byte */
                     /*       line of its own) through which the workgroups of the one-read K quantizer meet, then */
                     /*       one status word                                                                       */

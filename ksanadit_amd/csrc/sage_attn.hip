@@ -120,15 +120,25 @@ __global__ __launch_bounds__(kW * 64, kW == 8 ? 1 : 2) void sage_attn_fwd_kernel
   const bool is_run = kCanSplit && (int)blockIdx.x >= p.split_first_block;  // uniform
   const int run_id = is_run ? (int)blockIdx.x - p.split_first_block : 0;    // the partial result's place in the workspace
   if constexpr (kNumbered) {  // (BatchRun, BatchPlace)
-    typedef const __attribute__((address_space(4))) int32_t* Constant;
-    const Constant at_starts = reinterpret_cast<Constant>(reinterpret_cast<uintptr_t>(p.split_ml));
-    int starts[kBatchStarts];
-#pragma unroll
-    for (int i = 0; i < kBatchStarts; ++i) starts[i] = at_starts[i];  // (scalar loads, together)
     const int xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
-    const BatchRun run = batch_run_of(starts, p.B, at);
+    int starts[kBatchStarts];
+    BatchRun run;
+    if (p.numbered == 1) {
+      typedef const __attribute__((address_space(4))) int32_t* Constant;
+      const Constant at_starts = reinterpret_cast<Constant>(reinterpret_cast<uintptr_t>(p.split_ml));
+#pragma unroll
+      for (int i = 0; i < kBatchStarts; ++i) starts[i] = at_starts[i];  // (scalar loads, together)
+      run = batch_run_of(starts, p.B, at);
+      take_counts(p.q_lens, p.k_lens, run.b, lq, lk);
+    } else {
+      int rows, keys;
+      const int mine = batch_number(BatchNumbers{nullptr, p.B, p.Hq, p.Lq, p.Lk, kRowsWg, p.q_lens, p.k_lens}, threadIdx.x & 63, rows, keys);
+#pragma unroll
+      for (int i = 0; i < kBatchStarts; ++i) starts[i] = __builtin_amdgcn_readlane(mine, i);
+      run = batch_run_of(starts, p.B, at);
+      lq = __builtin_amdgcn_readlane(rows, run.b), lk = __builtin_amdgcn_readlane(keys, run.b);
+    }
     b = run.b;
-    take_counts(p.q_lens, p.k_lens, b, lq, lk);
     const BatchPlace place = batch_place(run, xcd, at, p.Hq, n_qwg, batch_blocks(lq, lk, kRowsWg));
     if (place.b < 0) return;
     h = place.h, qwg = place.qwg;

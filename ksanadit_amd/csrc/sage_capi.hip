@@ -561,16 +561,16 @@ int ksana_sage_quant_v(const void* v, int dtype, const int64_t st[4], const ksan
 }
 
 static int quant_v_impl(const void* v, int dtype, const int64_t st[4], const ksana_sage_shape* s, int smooth_v,
-                        void* ws, void* stream, bool cleared);
+                        void* ws, void* stream, bool cleared, const ksana_sage::BatchNumbers& numbers = {});
 
 int ksana_sage_quant_v_smooth(const void* v, int dtype, const int64_t st[4], const ksana_sage_shape* s, int smooth_v,
                               void* ws, void* stream) {
   return quant_v_impl(v, dtype, st, s, smooth_v, ws, stream, false);
 }
 
-// `cleared`: the counters are zero
+// `cleared`: the counters are zero; `numbers`: written where V is smoothed
 static int quant_v_impl(const void* v, int dtype, const int64_t st[4], const ksana_sage_shape* s, int smooth_v,
-                        void* ws, void* stream, bool cleared) {
+                        void* ws, void* stream, bool cleared, const ksana_sage::BatchNumbers& numbers) {
   const StageRange range("ksana_sage.quant_v");
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_tensor("v", v, dtype, st, s->B, s->Lk, s->Hkv)) return rc;
@@ -599,7 +599,7 @@ static int quant_v_impl(const void* v, int dtype, const int64_t st[4], const ksa
     e = ksana_sage::launch_col_partial(vt, s->B, s->Hkv, s->Lk, 0, ws_at<float>(ws, l.v_part), l.nch, hs);
     if (e != hipSuccess) return hip_fail(e, "v column sum launch");
     // the same finalisation as for K: the mean rounded to the input dtype
-    e = ksana_sage::launch_k_mean_finalize(ws_at<float>(ws, l.v_part), bhk, l.nch, s->Lk, dtype, 1, v_mean, hs);
+    e = ksana_sage::launch_k_mean_finalize(ws_at<float>(ws, l.v_part), bhk, l.nch, s->Lk, dtype, 1, v_mean, hs, nullptr, numbers);
     if (e != hipSuccess) return hip_fail(e, "v mean finalize launch");
   }
   e = ksana_sage::launch_col_partial(vt, s->B, s->Hkv, s->Lk, smooth_v ? 2 : 1, ws_at<float>(ws, l.v_part), l.nch, hs,
@@ -883,6 +883,14 @@ ksana_sage::AttnParams attn_params(void* ws, void* o, int dtype, const int64_t o
   return p;
 }
 
+// the numbering of the blocks of a call for which batch_rows_wg has named rows; it goes where such calls, which are never cut, have no
+// partial results
+ksana_sage::BatchNumbers batch_numbers(void* ws, const ksana_sage_shape* s, int rows_wg, const int32_t* q_lens, const int32_t* k_lens) {
+  ksana_sage_ws_layout l;
+  ksana_sage_workspace_layout(s, &l);
+  return ksana_sage::BatchNumbers{ws_at<int32_t>(ws, l.split_ml), s->B, s->Hq, s->Lq, s->Lk, rows_wg, q_lens, k_lens};
+}
+
 // q_rows: nullptr, or Q as the caller has it (validated, of the result's dtype) for the kernel to quantize - with lin, for
 // the linear branch that the kernel then adds
 int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_sage_shape* s, const int8_t* block_mask,
@@ -903,17 +911,16 @@ int attn_impl(void* ws, void* o, int dtype, const int64_t o_st[4], const ksana_s
   ksana_sage::AttnParams p = attn_params(ws, o, dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, flags);
   if (q_rows != nullptr) p.q_rows = *q_rows, p.q_premul = q_premul;
   if (lin != nullptr) p.lin = *lin;
-  p.numbered = numbered ? 1 : 0;
-  hipError_t e = ksana_sage::launch_attn_fwd(p, static_cast<hipStream_t>(stream));
+  p.numbered = ksana_sage::batch_rows_wg(p) == 0 ? 0 : (numbered ? 1 : 2);
+  const hipError_t e = ksana_sage::launch_attn_fwd(p, static_cast<hipStream_t>(stream));
   return e == hipSuccess ? 0 : hip_fail(e, "attention launch");
 }
 
 // The quantizers of a call whose arguments have been validated: of Q, K and V, or (with_q == false, no prep) of K and V.
-// q_lens, k_lens: see QkvCall; batch_rows: 0, or the attention's rows per workgroup, and *numbered says whether its numbering has been
-// written to split_ml (such calls have no cut blocks)
+// q_lens, k_lens: see QkvCall; numbers: what the attention would like numbered, and *numbered says whether that has been done
 int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtype, const int64_t q_st[4], const int64_t k_st[4],
               const int64_t v_st[4], const ksana_sage_shape* s, const ksana_sage_prep* prep, float sm_scale, int smooth_k,
-              int smooth_v, void* ws, void* stream, const int32_t* q_lens, const int32_t* k_lens, int batch_rows, bool* numbered) {
+              int smooth_v, void* ws, void* stream, const int32_t* q_lens, const int32_t* k_lens, const ksana_sage::BatchNumbers& numbers, bool* numbered) {
   *numbered = false;
   if (!smooth_v) {
     const StageRange range("ksana_sage.quant_qkv");
@@ -928,12 +935,12 @@ int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtyp
     ksana_sage::QkvCall c = qkv_call(with_q, in_tensor(q, dtype, q_st, s->D), in_tensor(k, dtype, k_st, s->D),
                                      in_tensor(v, dtype, v_st, s->D), s, l, sm_scale, smooth_k, ws);
     c.q_lens = q_lens, c.k_lens = k_lens;
-    if (batch_rows != 0) c.batch_starts = ws_at<int32_t>(ws, l.split_ml), c.rows_wg = batch_rows;
+    if (prep == nullptr) c.numbers = numbers;
     bool used = false;
     const hipError_t e = ksana_sage::launch_quant_qkv(c, ppq, ppk, static_cast<hipStream_t>(stream), &used);
     if (e != hipSuccess) return hip_fail(e, "q, k, v quantizer launch");
     if (used) {
-      *numbered = batch_rows != 0;
+      *numbered = c.numbers.starts != nullptr;
       return 0;
     }
   }
@@ -965,7 +972,8 @@ int quant_qkv(bool with_q, const void* q, const void* k, const void* v, int dtyp
   } else if (int rc = ksana_sage_quant_qk_prep(q, k, dtype, q_st, k_st, s, prep, sm_scale, smooth_k, ws, stream)) {
     return rc;
   }
-  return ksana_sage_quant_v_smooth(v, dtype, v_st, s, smooth_v, ws, stream);
+  *numbered = smooth_v && numbers.starts != nullptr;
+  return quant_v_impl(v, dtype, v_st, s, smooth_v, ws, stream, false, numbers);
 }
 
 int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype, int o_dtype, const int64_t q_st[4],
@@ -1014,11 +1022,11 @@ int forward_impl(const void* q, const void* k, const void* v, void* o, int dtype
                       ksana_sage::resident_call_suits(attn_params(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, flags)));
   const bool trim = (flags & KSANA_SAGE_FLAG_WS_UNSTORED) && prep == nullptr;  // what no row or key that takes part needs
   const int attn_flags = flags & ~(KSANA_SAGE_FLAG_SMOOTH_V | KSANA_SAGE_FLAG_Q_UNSTORED | KSANA_SAGE_FLAG_WS_UNSTORED);
-  const int batch_rows =
-      !trim ? 0 : ksana_sage::batch_rows_wg(attn_params(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, attn_flags));
+  const int rows_wg = ksana_sage::batch_rows_wg(attn_params(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal, attn_flags));
+  const ksana_sage::BatchNumbers numbers = rows_wg == 0 ? ksana_sage::BatchNumbers{} : batch_numbers(ws, s, rows_wg, q_lens, k_lens);
   bool numbered = false;
   if (int rc = quant_qkv(!own_q, q, k, v, dtype, q_st, k_st, v_st, s, prep, sm_scale, smooth_k, flags & KSANA_SAGE_FLAG_SMOOTH_V, ws,
-                         stream, trim ? q_lens : nullptr, trim ? k_lens : nullptr, batch_rows, &numbered))
+                         stream, trim ? q_lens : nullptr, trim ? k_lens : nullptr, numbers, &numbered))
     return rc;
   const ksana_sage::InTensor q_rows = in_tensor(q, dtype, q_st, s->D);
   return attn_impl(ws, o, o_dtype, o_st, s, block_mask, mask_st, q_lens, k_lens, causal,

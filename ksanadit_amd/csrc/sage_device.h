@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "../../include/ksana_sage_hip.h"
+#include "sage_kernels.h"
 
 namespace ksana_sage {
 
@@ -151,6 +152,29 @@ __device__ __forceinline__ float over_lanes(float v) {
   v = Op::of(v, lane_xor<2>(v));
   v = Op::of(v, lane_xor<4>(v));
   return over_slots<Op>(v);
+}
+
+// Number `lane` of the kBatchStarts, by a whole wave; and entry `lane`'s counts (lanes 0 .. B - 1)
+__device__ __forceinline__ int batch_number(const BatchNumbers& n, int lane, int& rows, int& keys) {
+  const bool zeros = lane >= n.B;
+  const int b = min(zeros ? lane - n.B : lane, n.B - 1);
+  rows = n.q_lens != nullptr ? rows_counted(n.q_lens[b], n.Lq) : n.Lq;
+  keys = n.k_lens != nullptr ? rows_counted(n.k_lens[b], n.Lk) : n.Lk;
+  const int with_rows = batch_blocks(rows, keys, n.rows_wg), all = (n.Lq + n.rows_wg - 1) / n.rows_wg;
+  const int share = lane < 2 * n.B ? batch_share(n.Hq, zeros ? all - with_rows : with_rows) : 0;
+  int rank = 0;  // of this lane's entry
+  for (int j = 0; j < n.B; ++j) {
+    const int other = __builtin_amdgcn_readlane(keys, j);
+    rank += other > keys || (other == keys && j < b) ? 1 : 0;
+  }
+  const int run = lane < 2 * n.B ? rank + (zeros ? n.B : 0) : lane;
+  int start = 0, entries = 0;
+  for (int i = 0; i < 2 * n.B; ++i) {
+    const int some = __builtin_amdgcn_readlane(share, i), r = __builtin_amdgcn_readlane(run, i);
+    start += r < run ? some : 0;
+    if (i < n.B) entries |= i << (4 * r);
+  }
+  return __builtin_amdgcn_ds_permute(4 * run, run == 0 ? entries : (run < 2 * n.B ? start : INT32_MAX));
 }
 
 // One butterfly stage across lanes c16 and c16 ^ M: every lane takes `own + sign * other` with sign = -1 on the lane

@@ -31,10 +31,13 @@ __host__ __device__ constexpr int tiles_counted(int count, int tiles) {
 // rows that take part, the entry with the most keys first, and then an eighth of every entry's other blocks, which have only zeros to
 // write.  (Numbered by the tensor alone, an entry's blocks without rows stand before the next entry's, and work waits for a place while
 // they come and go.)  Number `at` of an XCD lies in the last of these 2 B runs that starts at or before it.  The counts are in device
-// memory: the runs' starts, the unused ones INT32_MAX, are written once per call by the quantizers (QkvCall::batch_starts), and a
+// memory: the runs' starts, the unused ones INT32_MAX, are written once per call by the quantizers (BatchNumbers), and a
 // workgroup reads them, a 64-byte line, in one scalar load; in the place of the first, which is 0, stand the entries of the runs,
 // four bits each.  60 random calls of 2 to 8 entries, on average (and the worst) of the time by the tensor's numbering: 0.917 (0.99);
 // entry after entry 0.932 (0.99); worked out by every workgroup itself, for up to six entries, 0.952 (1.035).
+// Attention without a launch of the quantizers that could write them - in stages, behind a folded step or K's and V's separate passes - has
+// every workgroup work them out, a number per lane: 0 to 0.8 us a launch, where a launch of one wave for them is 1 to 2.5 (us of the
+// attention alone, in every workgroup / with such a launch: 2 x 12 heads of 6946 on 138 falling 22.4 / 24.4, 4 x 24 of 1300 42.7 / 44.9).
 constexpr int kBatchEntries = 8, kBatchStarts = 2 * kBatchEntries;
 static_assert(kBatchEntries <= 8, "four bits each, none of them the sign");
 // blocks of one kind, of an entry, that an XCD takes
@@ -158,13 +161,21 @@ struct PrepParams {
 // inv_rms[b, l] from x[b, l, :H*128] (the row must be contiguous: sH == 128)
 hipError_t launch_row_inv_rms(const InTensor& x, int B, int H, int L, float eps, float* inv_rms, hipStream_t s);
 
+// What the numbers of the attention's blocks (kBatchStarts) are worked out from, and where they go; starts == nullptr: they are not
+// asked for.  A launch of the quantizers takes one workgroup more for them.
+struct BatchNumbers {
+  int32_t* starts;
+  int B, Hq, Lq, Lk, rows_wg;
+  const int32_t *q_lens, *k_lens;
+};
+
 // column reductions over the sequence: op 0 = ordered fp32 sum, op 1 = max of |x|
 // op 0: column sums, 1: column max |x|, 2: column max |x - centre[d]| (centre: [B, H, D])
 hipError_t launch_col_partial(const InTensor& x, int B, int H, int L, int op, float* part, int nch, hipStream_t s,
                               const PrepParams* prep = nullptr, const float* centre = nullptr);
 // status: nullptr, or the quantizer's status word to clear (see QuantSync)
 hipError_t launch_k_mean_finalize(const float* part, int BH, int nch, int L, int dtype, int smooth, float* k_mean,
-                                  hipStream_t s, int* status = nullptr);
+                                  hipStream_t s, int* status = nullptr, const BatchNumbers& numbers = {});
 // zero_mean: nullptr, or the [BH, D] mean slot to clear (V quantized without smoothing)
 hipError_t launch_v_scale_finalize(const float* part, int BH, int nch, float* v_scale, float* v_inv, float* zero_mean,
                                    hipStream_t s, int* status = nullptr);
@@ -245,10 +256,7 @@ struct QkvCall {
   // nullptr, or (no folded step) the counts of the attention that follows and nobody else sees the codes: keys and query
   // rows that take no part count for the statistics as ever, but blocks made of them alone are not quantized
   const int32_t *q_lens, *k_lens;
-  // nullptr, or (no folded step) where the launch that comes first leaves the kBatchStarts numbers of the attention's blocks of
-  // rows_wg rows
-  int32_t* batch_starts;
-  int rows_wg;
+  BatchNumbers numbers;  // (no folded step) the launch that comes first writes them
 };
 hipError_t launch_quant_qkv(const QkvCall& call, const PrepParams* pq, const PrepParams* pk, hipStream_t s, bool* used);
 
@@ -336,7 +344,7 @@ struct AttnParams {
   float* split_ml;
   int split_first_block = 0, split_first_wg = 0, n_split = 0;  // filled in by the launcher
   int batch_run = 0;  // filled in by the launcher: 0, or the workgroups of one batch entry that go to one XCD
-  int numbered = 0;  // 1: split_ml holds the kBatchStarts numbers of a call whose rows batch_rows_wg has named
+  int numbered = 0;  // 0, or (batch_rows_wg has named rows) 1: split_ml holds the kBatchStarts numbers, 2: every workgroup works them out
   int small_last = 0;  // filled in by the launcher: 0, or how many heads' short last blocks each XCD takes behind its whole blocks
   int wg_waves;  // 0: the launcher picks the workgroup shape; 4 or 8: forced (for measurements and tests)
   int d_out;     // channels of an output row that exist: 128, or 64 (head size 64 runs zero-padded to 128)

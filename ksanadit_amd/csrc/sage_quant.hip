@@ -501,12 +501,24 @@ __device__ __forceinline__ float combine_partials(const float* __restrict__ part
   return acc;
 }
 
+// The numbers of the attention's blocks (kBatchStarts), by one wave of a workgroup of its own, the launch's first: the others'
+// work hides it (as the last one it was 0.2 us of a first stage of 5.8).
+__host__ __device__ __forceinline__ int numbers_batch(const BatchNumbers& n) { return n.starts != nullptr ? 1 : 0; }
+__device__ __forceinline__ void number_batch(const BatchNumbers& n) {
+  if (threadIdx.x >= 64) return;
+  int rows, keys;
+  const int mine = batch_number(n, threadIdx.x, rows, keys);
+  if (threadIdx.x < kBatchStarts) n.starts[threadIdx.x] = mine;
+}
+
 // chunk sums -> mean rounded to the input dtype, stored widened
 __global__ __launch_bounds__(kFinThreads) void k_mean_finalize_kernel(const float* __restrict__ part, int nch, int L,
                                                                       int dtype, int smooth,
-                                                                      float* __restrict__ k_mean, int* status) {
+                                                                      float* __restrict__ k_mean, int* status, const BatchNumbers numbers) {
   __shared__ float s_part[kFinMaxChunks * kD];
-  const int bh = blockIdx.x;
+  const int more = numbers_batch(numbers);
+  if ((int)blockIdx.x < more) return number_batch(numbers);
+  const int bh = blockIdx.x - more;
   if (status != nullptr && bh == 0 && threadIdx.x == 0) *status = 0;  // this path has no wait that could expire
   const float tot = combine_partials<0>(part + (int64_t)bh * nch * kD, nch, s_part);
   if (threadIdx.x < kD) {
@@ -1586,32 +1598,6 @@ __device__ __forceinline__ int tiles_in_use(const QkvCall& c, int b) {
   return c.k_lens == nullptr ? c.nkb : tiles_counted(c.k_lens[b], c.nkb);
 }
 
-// The numbers of the attention's blocks (kBatchStarts), by one wave of a workgroup of its own, the launch's first: the others'
-// work hides it (as the last one it was 0.2 us of a first stage of 5.8).
-__device__ __forceinline__ int numbers_batch(const QkvCall& c) { return c.batch_starts != nullptr ? 1 : 0; }
-__device__ __forceinline__ void number_batch(const QkvCall& c) {
-  const int lane = threadIdx.x;
-  if (lane >= 64) return;
-  const bool zeros = lane >= c.B;
-  const int b = min(zeros ? lane - c.B : lane, c.B - 1);
-  const int rows = c.q_lens != nullptr ? rows_counted(c.q_lens[b], c.Lq) : c.Lq, keys = c.k_lens != nullptr ? rows_counted(c.k_lens[b], c.Lk) : c.Lk;
-  const int with_rows = batch_blocks(rows, keys, c.rows_wg), all = (c.Lq + c.rows_wg - 1) / c.rows_wg;
-  const int share = lane < 2 * c.B ? batch_share(c.Hq, zeros ? all - with_rows : with_rows) : 0;
-  int rank = 0;  // of this lane's entry
-  for (int j = 0; j < c.B; ++j) {
-    const int other = __builtin_amdgcn_readlane(keys, j);
-    rank += other > keys || (other == keys && j < b) ? 1 : 0;
-  }
-  const int run = lane < 2 * c.B ? rank + (zeros ? c.B : 0) : lane;
-  int start = 0, entries = 0;
-  for (int i = 0; i < 2 * c.B; ++i) {
-    const int n = __builtin_amdgcn_readlane(share, i), r = __builtin_amdgcn_readlane(run, i);
-    start += r < run ? n : 0;
-    if (i < c.B) entries |= i << (4 * r);
-  }
-  if (lane < kBatchStarts) c.batch_starts[run] = run == 0 ? entries : (run < 2 * c.B ? start : INT32_MAX);
-}
-
 template <int DT, int KIND>
 __device__ __forceinline__ void quant_q_item(int item, const QkvCall& c, const PrepParams& pp) {
   const int bh = item / c.nqb;
@@ -1780,8 +1766,8 @@ template <int DT, int KIND, bool kHeads>
 __global__ __launch_bounds__(kThreads, KIND == 0 ? 5 : 4) void quant_qkv_stage1_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
   want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   clear_status(c);
-  const int more = KIND == 0 ? numbers_batch(c) : 0;
-  if ((int)blockIdx.x < more) return number_batch(c);
+  const int more = KIND == 0 ? numbers_batch(c.numbers) : 0;
+  if ((int)blockIdx.x < more) return number_batch(c.numbers);
   const int n_v = c.B * c.Hkv * c.nch;
   const int n_k = !c.smooth_k ? 0 : (!kHeads ? n_v : c.B * ((c.Hkv + kJointHeadsK - 1) / kJointHeadsK) * c.nch);
   int item = blockIdx.x - more;
@@ -1847,8 +1833,8 @@ __global__ __launch_bounds__(kThreads, KIND == 0 ? 6 : (kHeads ? 4 : 5)) void qu
 // Q blocks (which wait for nobody) and the V chunks work while K's chunks wait for their mean.
 template <int DT>
 __global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCall c, const HeadSync sk, const HeadSync sv) {
-  const int more = numbers_batch(c);
-  if ((int)blockIdx.x < more) return number_batch(c);
+  const int more = numbers_batch(c.numbers);
+  if ((int)blockIdx.x < more) return number_batch(c.numbers);
   const PrepParams none{};
   const int group = c.Hq / c.Hkv, per_head = 2 * c.nch + group * c.nqb;
   const int block = blockIdx.x - more, bh = block / per_head;
@@ -1875,8 +1861,8 @@ template <int DT, int KIND>
 __global__ __launch_bounds__(kThreads, 4) void quant_qkv_small_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
   want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   clear_status(c);
-  const int more = KIND == 0 ? numbers_batch(c) : 0;
-  if ((int)blockIdx.x < more) return number_batch(c);
+  const int more = KIND == 0 ? numbers_batch(c.numbers) : 0;
+  if ((int)blockIdx.x < more) return number_batch(c.numbers);
   const int n = c.B * c.Hkv;
   const int item = blockIdx.x - more;
   const HeadSync nobody{};
@@ -2074,8 +2060,8 @@ hipError_t launch_col_partial(const InTensor& x, int B, int H, int L, int op, fl
 }
 
 hipError_t launch_k_mean_finalize(const float* part, int BH, int nch, int L, int dtype, int smooth, float* k_mean,
-                                  hipStream_t s, int* status) {
-  k_mean_finalize_kernel<<<dim3(BH), dim3(kFinThreads), 0, s>>>(part, nch, L, dtype, smooth, k_mean, status);
+                                  hipStream_t s, int* status, const BatchNumbers& numbers) {
+  k_mean_finalize_kernel<<<dim3(BH + numbers_batch(numbers)), dim3(kFinThreads), 0, s>>>(part, nch, L, dtype, smooth, k_mean, status, numbers);
   return hipGetLastError();
 }
 
@@ -2436,7 +2422,7 @@ static hipError_t launch_qkv_kind(QkvCall& c, const PrepParams& pq, const PrepPa
   static_assert(KIND == 0 || KIND == 2, "nothing folded in, or the joint block's step");
   const dim3 block(kThreads);
   const int64_t n_q = (int64_t)c.B * c.Hq * c.nqb, n_chunks = (int64_t)c.B * c.Hkv * c.nch;
-  const int more = KIND == 0 && c.batch_starts != nullptr ? 1 : 0;  // (numbers_batch)
+  const int more = KIND == 0 ? numbers_batch(c.numbers) : 0;
   if (c.nch == 1) {
     quant_qkv_small_kernel<DT, KIND><<<dim3((unsigned)(n_q + 2 * n_chunks + more)), block, 0, s>>>(c, pq, pk);
     *used = true;

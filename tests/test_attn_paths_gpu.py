@@ -254,8 +254,8 @@ def test_a_shared_last_block_in_batches_with_lengths(hip_device, k_len, rows):
 @pytest.mark.parametrize("B,H,Lq,Lk", [(3, 40, 700, 900), (5, 16, 1000, 300), (64, 2, 700, 130), (65, 2, 700, 130), (2, 40, 2000, 700)])
 @pytest.mark.parametrize("wg_waves", [4, 8])
 def test_batches_with_counts(hip_device, B, H, Lq, Lk, wg_waves):
-    """Counts in any order, equal, none, one, all, out of range against the same operands walked through a mask of ones: on a kept
-    workspace, whose grid is numbered entry after entry."""
+    """Counts in any order, equal, none, one, all, out of range against the same operands walked through a mask of ones: grids
+    numbered by the counts and (64 and 65 entries, three rounds of 8 waves and more) entry after entry."""
     print(f"case B={B} H={H} Lq={Lq} Lk={Lk} waves={wg_waves}", flush=True)
     g = torch.Generator().manual_seed(B * Lq + Lk)
     q, k, v = (torch.randn((B, n, H, 128), generator=g).to(torch.bfloat16).to(hip_device) for n in (Lq, Lk, Lk))
@@ -279,11 +279,11 @@ def test_batches_with_counts(hip_device, B, H, Lq, Lk, wg_waves):
 @pytest.mark.parametrize("B,H,Lq,Lk,D", [(2, 32, 1062, 1062, 128), (2, 30, 1034, 300, 64), (4, 64, 541, 2302, 128), (4, 64, 624, 1500, 64), (3, 11, 1932, 700, 128)])
 def test_short_last_blocks_that_start_last(hip_device, B, H, Lq, Lk, D):
     """Grids that take a round less without the heads' short last blocks, which are numbered behind all others, in 4 and 8 waves,
-    against the same call with counts that leave nothing out on a kept workspace, whose blocks are in the order of their index."""
+    against the same call with counts that leave nothing out, whose blocks are numbered by these or in the order of their index."""
     print(f"case B={B} H={H} Lq={Lq} Lk={Lk} D={D}", flush=True)
     g = torch.Generator(device=hip_device).manual_seed(Lq)
     q, k, v = (torch.randn((B, n, H, D), generator=g, device=hip_device).half() for n in (Lq, Lk, Lk))
-    want = sage_ops.sageattn(q, k, v, workspace=sage_ops.workspace_for(q, k), k_lens=torch.full((B,), Lk))
+    want = sage_ops.sageattn(q, k, v, k_lens=torch.full((B,), Lk))
     del_me = torch.full_like(q, float("nan"))  # (memory that the next result may lie in)
     del del_me
     assert torch.equal(sage_ops.sageattn(q, k, v), want)
@@ -316,22 +316,79 @@ def _counts(B, Lq, Lk):
                 (torch.full((B,), Lq // 2), torch.full((B,), Lk // 2)), (rand[0], None), (None, few), (torch.zeros(B, dtype=torch.int64), None))
 
 
+def _by_index(q, k, v, q_lens, k_lens, **kw):
+    """The same call with empty entries up to nine, whose blocks are not numbered by the counts; none of NUMBERED is cut with these,
+    and those whose last blocks share their keys stay in workgroups of 4 waves."""
+    B = q.shape[0]
+    q, k, v = (torch.cat([x, x.new_zeros((9 - B, *x.shape[1:]))]) for x in (q, k, v))
+    assert sage_ops.key_split_plan(sage_ops.workspace_for(q, k)) is None
+    more = lambda n: None if n is None else torch.cat([n, n.new_zeros(9 - B)])  # noqa: E731
+    return sage_ops.sageattn(q, k, v, q_lens=more(q_lens), k_lens=more(k_lens), **kw)[:B]
+
+
 @pytest.mark.parametrize("B,H,Hkv,Lq,Lk,D,dtype", NUMBERED)
 def test_batches_numbered_by_their_counts(hip_device, B, H, Hkv, Lq, Lk, D, dtype):
-    """Whole calls, whose blocks are numbered by the entries' counts, against the same calls on a kept workspace, which are not."""
+    """Calls whose blocks are numbered by the entries' counts - in one piece, on a kept workspace, in stages on its operands, with V
+    smoothed - against the same calls numbered entry after entry."""
     print(f"case B={B} H={H}/{Hkv} Lq={Lq} Lk={Lk} D={D} {dtype}", flush=True)
     g = torch.Generator(device=hip_device).manual_seed(Lq)
     q, k, v = (torch.randn((B, n, h, D), generator=g, device=hip_device).to(dtype) for n, h in ((Lq, H), (Lk, Hkv), (Lk, Hkv)))
     ws = sage_ops.workspace_for(q, k)
-    for q_lens, k_lens in _counts(B, Lq, Lk):
+    for i, (q_lens, k_lens) in enumerate(_counts(B, Lq, Lk)):
         kw = {"q_lens": q_lens, "k_lens": k_lens}
-        want = sage_ops.sageattn(q, k, v, workspace=ws, **kw)
-        del_me = torch.full_like(q, float("nan"))  # (memory that the next result may lie in)
-        del del_me
-        got = sage_ops.sageattn(q, k, v, **kw)
-        assert torch.equal(got, want), kw
-        for b in range(B if q_lens is not None else 0):
-            assert not got[b, max(0, int(q_lens[b])) :].any(), (kw, b)
+        want = _by_index(q, k, v, **kw)
+        calls = [lambda: sage_ops.sageattn(q, k, v, **kw)]
+        if i < 4:
+            calls += [lambda: sage_ops.sageattn(q, k, v, workspace=ws, **kw), lambda: sage_ops.attn_fwd(ws, torch.empty_like(q), **kw)]
+        if i in (2, 3):
+            calls += [lambda: sage_ops.sageattn(q, k, v, smooth_v=True, **kw)]
+        for c, call in enumerate(calls):
+            if c == 3:
+                want = _by_index(q, k, v, smooth_v=True, **kw)
+            del_me = torch.full_like(q, float("nan"))  # (memory that the next result may lie in)
+            del del_me
+            got = call()
+            assert torch.equal(got, want), (kw, c)
+            for b in range(B if q_lens is not None else 0):
+                assert not got[b, max(0, int(q_lens[b])) :].any(), (kw, b)
+
+
+@pytest.mark.parametrize("B,H,Lq,Lk,rows", [(3, 24, 3001, 1100, 128), (2, 12, 6946, 138, 128), (2, 50, 1250, 2560, 256), (2, 16, 3500, 16500, 256)])
+@pytest.mark.parametrize("smooth_v", [False, True])
+def test_the_quantizers_number_every_whole_call(hip_device, B, H, Lq, Lk, rows, smooth_v):
+    """A kept workspace and smoothed V too: the numbers that the attention kernel has read are those that the counts make."""
+    print(f"case B={B} H={H} Lq={Lq} Lk={Lk} smooth_v={smooth_v}", flush=True)
+    g = torch.Generator(device=hip_device).manual_seed(Lq)
+    q, k, v = (torch.randn((B, n, H, 128), generator=g, device=hip_device).half() for n in (Lq, Lk, Lk))
+    ws = sage_ops.workspace_for(q, k)
+    blocks = -(-Lq // rows)
+    for q_lens, k_lens in _counts(B, Lq, Lk):
+        sage_ops.sageattn(q, k, v, workspace=ws, q_lens=q_lens, k_lens=k_lens, smooth_v=smooth_v)
+        ql, kl = ([min(max(int(x), 0), n) for x in (lens if lens is not None else [n] * B)] for lens, n in ((q_lens, Lq), (k_lens, Lk)))
+        order = sorted(range(B), key=lambda b: -kl[b])
+        some = [-(-ql[b] // rows) if kl[b] else 0 for b in order]
+        starts = [0]
+        for n in some + [blocks - n for n in some]:
+            starts.append(starts[-1] + (H * n + 7) // 8)
+        want = [sum(b << (4 * i) for i, b in enumerate(order)), *starts[1 : 2 * B]] + [2**31 - 1] * (16 - 2 * B)
+        assert ws.blob[ws.layout.split_ml :][:64].view(torch.int32).tolist() == want, (q_lens, k_lens)
+
+
+@pytest.mark.parametrize("H,Lq,Lk,step", [(16, 3500, 16500, False), (24, 1500, 1500, True)])
+def test_batches_numbered_in_the_attention_kernel(hip_device, quant_settings, H, Lq, Lk, step):
+    """.. where no launch of the quantizers can take the numbering along: K and V in passes of their own, or a step folded in."""
+    print(f"case H={H} Lq={Lq} Lk={Lk} step={step}", flush=True)
+    B = 2
+    if not step:
+        quant_settings(one_read="")
+    g = torch.Generator(device=hip_device).manual_seed(3)
+    q, k, v = (torch.randn((B, n, H, 128), generator=g, device=hip_device).to(torch.bfloat16) for n in (Lq, Lk, Lk))
+    w = torch.rand((4, 128), generator=g, device=hip_device).to(torch.bfloat16) + 0.5
+    prep = sage_ops.QwenPrep(100, *w, 1e-6) if step else None
+    for q_lens, k_lens in list(_counts(B, Lq, Lk))[:4]:
+        kw = {"q_lens": q_lens, "k_lens": k_lens, "prep": prep}
+        want = _by_index(q, k, v, **kw)
+        assert torch.equal(sage_ops.sageattn(q, k, v, **kw), want), kw
 
 
 def test_numbered_batches_replayed_with_other_counts(hip_device):
