@@ -1376,14 +1376,21 @@ void plan_key_split(int n_wg, int nkb, int* first_wg, int* runs) {
 }
 
 // Quantized in the attention kernel, Q is read once (2 bytes per channel where the quantizer's pass moves 4 with its reading
-// back), for about 800 vector instructions per wave that its set-up then waits for, 2-3 us.  That pays
+// back), for its transform in every workgroup's set-up.  us replayed from a graph, through memory / in the kernel, by blocks of 256
+// rows and on 300, 600, 1024, 2048, 4096 keys:
+//    32 blocks   17.8 / 18.6   21.1 / 21.9   25.4 / 26.0   36.6 / 37.5     46.8 / 47.1
+//    96          20.2 / 19.9   24.5 / 24.1   29.0 / 28.8   43.4 / 42.4     70.1 / 69.5
+//   160          24.5 / 23.8   31.5 / 30.2   37.9 / 36.8   56.9 / 56.3     96.3 / 95.5
+//   256          30.5 / 27.5   38.8 / 35.5   49.3 / 46.2   80.1 / 77.1    145.6 / 143.2
+//   320          38.2 / 34.9   50.0 / 45.9   62.9 / 60.6  102.4 / 99.1    181.6 / 179.1
+// That pays
 //   from one full round of the chip: below it every workgroup's set-up is exposed, and the quantizer's Q blocks ride in
-//     the launches of K and V (us through memory / in the kernel: 256 blocks, 32 tiles 58.3 / 56.6; 128 blocks 41.0 / 42.1;
-//     16 blocks 32.2 / 34.8);
-//   beyond 256 keys: up to there all quantizers are one launch (256 blocks, 2 tiles 23.0 / 24.1; 8 tiles 33.1 / 30.0);
-//   up to 256 tiles: there the gain is half a per cent (2560 blocks: 8 tiles 195 / 178, 32 tiles 452 / 438, 128 tiles
-//     1477 / 1455, 256 tiles 2801 / 2786), and on chips at their power limit the instructions cost the key loop as much
-//     (512 tiles: 10337 / 10365).
+//     the launches of K and V.  (The line is older than the present set-up, whose break-even is near 96 blocks; between the
+//     two 1-7 % are left.)
+//   beyond 256 keys: up to there all quantizers are one launch (256 blocks, 2 tiles 23.0 / 24.1 and 8 tiles 33.1 / 30.0 with an
+//     earlier set-up; calls of one round on so few keys are one launch altogether, see small_call_suits);
+//   up to 256 tiles: there the gain is half a per cent (40 heads of 16384 rows on 2048 keys 447.5 / 426.7, 8192 1439 / 1413, 16384
+//     2726 / 2715), and on chips at their power limit the instructions cost the key loop as much (24000 keys 3962 / 3969).
 bool q_in_attention_pays(int n_wg, int nkb) { return n_wg >= compute_units() && nkb * kBlkK > kMeanChunk && nkb <= 256; }
 
 // Workgroup shape for a call: 4-wave workgroups (two per compute unit) when a block mask or causal masking is

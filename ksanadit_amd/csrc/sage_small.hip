@@ -401,7 +401,10 @@ hipError_t launch_rows(const SmallCall& c, hipStream_t s) {
 }  // namespace
 
 // One round of the chip: every workgroup quantizes its head's K and V by itself, and beyond that the general path, which does
-// it once, is ahead (us, two launches / this: 280 workgroups of 256 keys 34 / 42, 504 of 250 keys 45 / 46; 256 of 200 keys 34 / 24).
+// it once, is ahead.  us replayed from a graph, general / one launch, on 64, 128, 256 keys: 256 workgroups (64 heads of 1000 rows)
+// 18.5 / 15.0, 22.2 / 18.5, 30.0 / 26.8; 264 22.6 / 25.2, 26.2 / 30.8, 34.5 / 44.1; 384 (96 of 1000) 25.1 / 26.3, 28.7 / 33.1, 37.3 / 46.5.
+// Two kinds of call beyond the line would still gain, and take the general path: entries of one block each (8 x 64 heads of 250
+// rows, 512 workgroups, 35.8 / 29.7, 41.4 / 36.8, 56.0 / 54.9) and 64 channels on few keys (264: 19.3 / 16.9, 21.5 / 21.6, 27.8 / 33.2).
 bool small_call_suits(int B, int Hq, int Lq, int Lk) { return Lk <= kMeanChunk && (int64_t)B * Hq * ((Lq + 255) / 256) <= kComputeUnits; }
 
 hipError_t launch_small(const SmallCall& call, hipStream_t s) {
