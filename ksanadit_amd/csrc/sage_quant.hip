@@ -173,7 +173,8 @@ __device__ __forceinline__ void qwen_row(QwenRow& f, const PrepParams& pp, int r
 // kFused: the squares of half values are exact (bf16: from 2^-63 up), so a fused multiply-add rounds like the sum alone and is an
 // instruction less.  us, apart / fused: several heads per item, whose vector units are busy over half of the time, 2 x 4352 tokens of
 // 24 heads 345.7 / 344.3, 2 x 1328 73.1 / 72.2; one head per item, bound by the length of its chain, the other way round: 2 x 774
-// 49.4 / 50.3, 2 x 1024 53.2 / 54.1, 1756 61.8 / 62.5.
+// 49.4 / 50.3, 2 x 1024 53.2 / 54.1, 1756 61.8 / 62.5.  K's only chunk (at most 256 tokens) takes it fused: 256 of 24 heads 27.8 / 27.6,
+// two of them 28.8 / 28.5.
 template <int DT, bool kFused>
 __device__ __forceinline__ void prep16_qwen(float* x, const QwenRow& f, float eps) {
   if (f.w != nullptr) {
@@ -210,11 +211,11 @@ __device__ __forceinline__ void prep16_qwen(float* x, const QwenRow& f, float ep
   }
 }
 
-template <int DT>
+template <int DT, bool kFused>
 __device__ __forceinline__ void prep16_qwen(float* x, const PrepParams& pp, int row, int c16) {
   QwenRow f;
   qwen_row(f, pp, row, c16);
-  prep16_qwen<DT, false>(x, f, pp.eps);
+  prep16_qwen<DT, kFused>(x, f, pp.eps);
 }
 
 // The pieces of the Wan step on the 16 channels of a lane.
@@ -271,11 +272,11 @@ __device__ __forceinline__ RopeLaneIndex rope_lane_index(int c16, int base_f, in
 
 // KIND: PrepParams::kind, a template argument so that every kernel instantiation carries the registers of its own
 // variant only (with a run-time switch the three variants' table reads add up).
-template <int DT, int KIND>
+template <int DT, int KIND, bool kFused = false>
 __device__ __forceinline__ void prep16(float* x, const PrepParams& pp, const RopeLds& rl, int b, int row, int h,
                                        int c16, bool staged = true, const float* row_rms = nullptr) {
   if constexpr (KIND == 2) {
-    prep16_qwen<DT>(x, pp, row, c16);
+    prep16_qwen<DT, kFused>(x, pp, row, c16);
     return;
   }
   if (pp.inv_rms != nullptr) {
@@ -1163,7 +1164,7 @@ __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __
     widen8<DT>(raw[i][0], x);
     widen8<DT>(raw[i][1], x + 8);
     if constexpr (PRE) {
-      if (row < L) prep16<DT, PRE>(x, pp, rl, b, row, h, c16);
+      if (row < L) prep16<DT, PRE, SOLO>(x, pp, rl, b, row, h, c16);
       raw[i][0] = narrow8<DT>(x);
       raw[i][1] = narrow8<DT>(x + 8);
       __builtin_amdgcn_sched_barrier(0);
@@ -1253,7 +1254,7 @@ __device__ __forceinline__ void quant_k_chunk(int bh, int ch, const uint16_t* __
           widen8<DT>(r[0], x);
           widen8<DT>(r[1], x + 8);
           if constexpr (PRE) {
-            if (row < L) prep16<DT, PRE>(x, pp, rl, b, row, h, c16, false);
+            if (row < L) prep16<DT, PRE, SOLO>(x, pp, rl, b, row, h, c16, false);
           }
 #pragma unroll
           for (int e = 0; e < 16; ++e) a16[e] = i == 0 ? x[e] : a16[e] + x[e];
@@ -1857,8 +1858,12 @@ __global__ __launch_bounds__(kThreads, 4) void quant_qkv_meet_kernel(const QkvCa
 }
 
 // at most 256 keys: one launch
+// (The joint step's K chunk holds its rows in 163 registers.  With the 128 that four workgroups a unit have, up to 69 went through
+// memory, how many depending on the kernel's arguments; three a unit are enough for the grids of this launch.  us per call of 24 heads,
+// four / three: 84 tokens 20.0 / 17.4, 256 30.6 / 27.6, 4 x 256 35.8 / 31.5; beside the four with 50 in memory 8 x 120 27.1 / 21.9, 8 x 256
+// 44.0 / 39.3, 12 x 256 53.7 / 46.6, 16 x 256, four rounds in place of three, 57.3 / 56.9, 24 x 256 79.9 / 78.9.)
 template <int DT, int KIND>
-__global__ __launch_bounds__(kThreads, 4) void quant_qkv_small_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
+__global__ __launch_bounds__(kThreads, KIND == 2 ? 3 : 4) void quant_qkv_small_kernel(const QkvCall c, const PrepParams pq, const PrepParams pk) {
   want(c.q.ptr, c.v.ptr, c.B, c.k_part, c.v_tiles);
   clear_status(c);
   const int more = KIND == 0 ? numbers_batch(c.numbers) : 0;
